@@ -1,14 +1,17 @@
 """ctypes loaders for the native libraries.  There is no fallback: a missing library raises."""
 import ctypes
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(_HERE, "lib")
 KERNELS_SO = os.path.join(LIB_DIR, "libnnf_hip_kernels.so")
+TORCH_SO = os.path.join(LIB_DIR, "nnf_torch.so")
 HOST_SO = os.path.join(LIB_DIR, "libnnf_host.so")
 
 _kernels = None
 _host = None
+_torch_front = None
 
 _c_int = ctypes.c_int
 _c_vp = ctypes.c_void_p
@@ -76,6 +79,23 @@ def kernels():
             fn.argtypes = args
         _kernels = lib
     return _kernels
+
+
+def torch_front():
+    """nnf_torch.so: the native front of ops.py (torch tensors -> the C ABI)."""
+    global _torch_front
+    if _torch_front is None:
+        kernels()
+        if not os.path.exists(TORCH_SO):
+            raise NativeLibraryMissing(
+                f"{TORCH_SO} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
+                "(or `make -C nnfusion_amd/csrc/torch_front`).")
+        import torch  # noqa: F401  (its libraries first)
+
+        spec = importlib.util.spec_from_file_location("nnf_torch", TORCH_SO)
+        _torch_front = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_torch_front)
+    return _torch_front
 
 
 def host():

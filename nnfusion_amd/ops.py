@@ -48,6 +48,23 @@ class NnfError(RuntimeError):
         super().__init__(f"{where}: status {status} ({msg})")
 
 
+class _Native:
+    """The functions of the native front (csrc/torch_front/nnf_torch.cpp), loaded at the first use of one: they take the
+    tensors and plain values in the order of the calls below, check them, allocate an output or workspace that was not
+    given and call the C ABI on the current stream."""
+
+    def __getattr__(self, name):
+        module = _lib.torch_front()
+        module.set_error(NnfError)
+        for f in dir(module):
+            if not f.startswith("_"):
+                setattr(self, f, getattr(module, f))
+        return getattr(module, name)
+
+
+_native = _Native()
+
+
 def _stream():
     return torch.cuda.current_stream().cuda_stream
 
@@ -68,20 +85,7 @@ def _p(t):
 
 def w4a16_gemm(a, wq, scales, group=128, zp=8, out=None, workspace=None):
     """Y[M,N] = A[M,K] . ((Wq - zp) * scales)^T ; a fp16 [M,K], wq u8 [N,K/2], scales fp16 [N,K/group]."""
-    lib = _lib.kernels()
-    m, k = a.shape
-    n = wq.shape[0]
-    assert a.dtype == torch.float16 and wq.dtype == torch.uint8 and scales.dtype == torch.float16
-    assert a.is_contiguous() and wq.is_contiguous() and scales.is_contiguous()
-    assert wq.shape[1] * 2 == k and tuple(scales.shape) == (n, k // group)
-    if out is None:
-        out = torch.empty((m, n), dtype=torch.float16, device=a.device)
-    need = lib.nnf_w4a16_gemm_workspace_bytes(m, n, k, group)
-    if workspace is None:
-        workspace = _ws(need, a.device)
-    _check(lib.nnf_w4a16_gemm(_stream(), a.data_ptr(), wq.data_ptr(), scales.data_ptr(), out.data_ptr(),
-                              m, n, k, group, zp, workspace.data_ptr(), workspace.numel()), "nnf_w4a16_gemm")
-    return out
+    return _native.w4a16_gemm(a, wq, scales, group, zp, out, workspace)
 
 
 class NnfQuant(ctypes.Structure):
@@ -110,28 +114,7 @@ def wna16_gemm(a, wq, scales, bits=4, group=128, zp=8, zero_points=None, out=Non
     """Y[M,N] = A[M,K] . ((Wq - z) * scales)^T with 4- or 8-bit weights (wq u8 [N, K*bits/8]), groups of 32 / 64 / 128
     and either a scalar zero point or zero_points u8 [N, ceil(K/group*bits/8)] (4-bit: two per byte, even group low).
     sync: synchronisation words (sync_flags()) for the one-launch form of the tile GEMM: nnf_wna16_gemm_planned."""
-    lib = _lib.kernels()
-    m, k = a.shape
-    n = wq.shape[0]
-    assert a.dtype == torch.float16 and wq.dtype == torch.uint8 and scales.dtype == torch.float16
-    assert a.is_contiguous() and wq.is_contiguous() and scales.is_contiguous()
-    assert wq.shape[1] * 8 == k * bits and tuple(scales.shape) == (n, k // group)
-    if zero_points is not None:
-        assert zero_points.dtype == torch.uint8 and zero_points.is_contiguous()
-        assert tuple(zero_points.shape) == (n, (k // group * bits + 7) // 8)
-    if out is None:
-        out = torch.empty((m, n), dtype=torch.float16, device=a.device)
-    keep, qp = _quant_arg(bits, group, zp, zero_points)
-    if workspace is None:
-        workspace = _ws(lib.nnf_wna16_gemm_workspace_bytes(m, n, k, qp), a.device)
-    if sync is not None:
-        keep_plan, plan_ptr = _plan_arg(None, sync, spin_limit)
-        _check(lib.nnf_wna16_gemm_planned(_stream(), a.data_ptr(), wq.data_ptr(), scales.data_ptr(), out.data_ptr(), m, n, k, qp,
-                                          plan_ptr, workspace.data_ptr(), workspace.numel()), "nnf_wna16_gemm_planned")
-        return out
-    _check(lib.nnf_wna16_gemm(_stream(), a.data_ptr(), wq.data_ptr(), scales.data_ptr(), out.data_ptr(), m, n, k, qp,
-                              workspace.data_ptr(), workspace.numel()), "nnf_wna16_gemm")
-    return out
+    return _native.wna16_gemm(a, wq, scales, bits, group, zp, zero_points, out, workspace, sync, spin_limit)
 
 
 VARIANTS = {"auto": 0, "gemv_valu": 1, "gemv_mfma": 2, "gemm_mfma": 3, "gemv_rows": 4}
@@ -166,28 +149,23 @@ def w4a16_gemm_fused(a, wq, scales, group=128, zp=8, rms_gamma=None, rms_eps=1e-
                      act=0, out=None, workspace=None, variant="auto", plan=None, sync=None, spin_limit=0):
     """GEMM with the fused RMSNorm prologue / bias, residual, SiLU-gate epilogues (see the C header); variant
     "gemm_mfma" and a plan (tile_rows, k_parts) go through nnf_w4a16_gemm_fused_variant."""
+    if variant == "auto" and plan is None:
+        return _native.w4a16_gemm_fused(a, wq, scales, group, zp, rms_gamma, rms_eps, bias, residual, act, out, workspace, sync,
+                                        spin_limit)
     lib = _lib.kernels()
     m, k = a.shape
     n = wq.shape[0] // (2 if act == 1 else 1)
     if out is None:
         out = torch.empty((m, n), dtype=torch.float16, device=a.device)
-    need = lib.nnf_w4a16_gemm_fused_workspace_bytes(m, n, k, group, act)
-    if variant != "auto" or plan is not None or sync is not None:
-        keep, plan_ptr = _plan_arg(plan, sync, spin_limit)
-        v = VARIANTS[variant]
-        if workspace is None:
-            workspace = _ws(need + lib.nnf_w4a16_gemm_variant_workspace_bytes(m, wq.shape[0], k, group, v, plan_ptr),
-                            a.device)
-        _check(lib.nnf_w4a16_gemm_fused_variant(_stream(), a.data_ptr(), wq.data_ptr(), scales.data_ptr(),
-                                                out.data_ptr(), m, n, k, group, zp, _p(rms_gamma), float(rms_eps),
-                                                _p(bias), _p(residual), int(act), v, plan_ptr, workspace.data_ptr(),
-                                                workspace.numel()), "nnf_w4a16_gemm_fused_variant")
-        return out
+    keep, plan_ptr = _plan_arg(plan, sync, spin_limit)
+    v = VARIANTS[variant]
     if workspace is None:
-        workspace = _ws(need, a.device)
-    _check(lib.nnf_w4a16_gemm_fused(_stream(), a.data_ptr(), wq.data_ptr(), scales.data_ptr(), out.data_ptr(),
-                                    m, n, k, group, zp, _p(rms_gamma), float(rms_eps), _p(bias), _p(residual),
-                                    int(act), workspace.data_ptr(), workspace.numel()), "nnf_w4a16_gemm_fused")
+        need = lib.nnf_w4a16_gemm_fused_workspace_bytes(m, n, k, group, act)
+        workspace = _ws(need + lib.nnf_w4a16_gemm_variant_workspace_bytes(m, wq.shape[0], k, group, v, plan_ptr), a.device)
+    _check(lib.nnf_w4a16_gemm_fused_variant(_stream(), a.data_ptr(), wq.data_ptr(), scales.data_ptr(),
+                                            out.data_ptr(), m, n, k, group, zp, _p(rms_gamma), float(rms_eps),
+                                            _p(bias), _p(residual), int(act), v, plan_ptr, workspace.data_ptr(),
+                                            workspace.numel()), "nnf_w4a16_gemm_fused_variant")
     return out
 
 
@@ -214,40 +192,24 @@ def w8a8_gemm(a, s_tok, w, s_ch, out=None, workspace=None, variant="auto", plan=
     """Y fp16 [M,N] = fp16((float)(A . W^T) * s_tok[m] * s_ch[n]) ; a i8 [M,K], w i8 [N,K].  A variant (a key of
     W8A8_VARIANTS), a plan (tile_rows, k_parts) or `sync` (see sync_flags: a few rows with a long K then run over
     two ranges of K in one launch) goes through nnf_w8a8_gemm_variant."""
-    lib = _lib.kernels()
-    m, k = a.shape
-    n = w.shape[0]
+    if variant == "auto" and plan is None:
+        return _native.w8a8_gemm(a, s_tok, w, s_ch, out, workspace, sync)
     assert a.dtype == torch.int8 and w.dtype == torch.int8
     assert s_tok.dtype == torch.float32 and s_ch.dtype == torch.float32
     if out is None:
-        out = torch.empty((m, n), dtype=torch.float16, device=a.device)
-    if variant != "auto" or plan is not None or sync is not None:
-        _w8a8_variant(a, s_tok, w, s_ch, out, None, variant, plan, workspace, sync)
-        return out
-    need = lib.nnf_w8a8_gemm_workspace_bytes(m, n, k)
-    if workspace is None:
-        workspace = _ws(need, a.device)
-    _check(lib.nnf_w8a8_gemm(_stream(), a.data_ptr(), s_tok.data_ptr(), w.data_ptr(), s_ch.data_ptr(),
-                             out.data_ptr(), m, n, k, workspace.data_ptr(), workspace.numel()), "nnf_w8a8_gemm")
+        out = torch.empty((a.shape[0], w.shape[0]), dtype=torch.float16, device=a.device)
+    _w8a8_variant(a, s_tok, w, s_ch, out, None, variant, plan, workspace, sync)
     return out
 
 
 def w8a8_gemm_acc(a, w, out=None, workspace=None, variant="auto", plan=None, sync=None):
     """acc i32 [M,N] = A . W^T, exact."""
-    lib = _lib.kernels()
-    m, k = a.shape
-    n = w.shape[0]
+    if variant == "auto" and plan is None:
+        return _native.w8a8_gemm(a, None, w, None, out, workspace, sync)
     assert a.dtype == torch.int8 and w.dtype == torch.int8
     if out is None:
-        out = torch.empty((m, n), dtype=torch.int32, device=a.device)
-    if variant != "auto" or plan is not None or sync is not None:
-        _w8a8_variant(a, None, w, None, None, out, variant, plan, workspace, sync)
-        return out
-    need = lib.nnf_w8a8_gemm_workspace_bytes(m, n, k)
-    if workspace is None:
-        workspace = _ws(need, a.device)
-    _check(lib.nnf_w8a8_gemm_acc(_stream(), a.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k,
-                                 workspace.data_ptr(), workspace.numel()), "nnf_w8a8_gemm_acc")
+        out = torch.empty((a.shape[0], w.shape[0]), dtype=torch.int32, device=a.device)
+    _w8a8_variant(a, None, w, None, None, out, variant, plan, workspace, sync)
     return out
 
 
@@ -255,30 +217,25 @@ def fused_mlp_w4a16(x, gamma, wgu, sgu, wd, sd, eps=1e-6, group=128, zp=8, out=N
                     spin_limit=0, gate_up_plan=None, down_plan=None):
     """out = x + Wd . (SiLU(Wg . n) * (Wu . n)), n = RMSNorm(x, gamma, eps).  `sync` (see sync_flags) or a plan for
     either product goes through nnf_fused_mlp_w4a16_planned."""
+    if gate_up_plan is None and down_plan is None:
+        return _native.fused_mlp_w4a16(x, gamma, wgu, sgu, wd, sd, eps, group, zp, out, workspace, sync, spin_limit)
     lib = _lib.kernels()
     m, h = x.shape
     i = wgu.shape[0] // 2
     if out is None:
         out = torch.empty((m, h), dtype=torch.float16, device=x.device)
-    need = lib.nnf_fused_mlp_w4a16_workspace_bytes(m, h, i, group)
-    if sync is not None or gate_up_plan is not None or down_plan is not None:
-        keep_a, plan_a = _plan_arg(gate_up_plan, sync, spin_limit)
-        keep_b, plan_b = _plan_arg(down_plan, sync, spin_limit)
-        if workspace is None:
-            v = VARIANTS["gemm_mfma"]
-            extra = (lib.nnf_w4a16_gemm_variant_workspace_bytes(m, 2 * i, h, group, v, plan_a) if gate_up_plan is not None else 0) + \
-                    (lib.nnf_w4a16_gemm_variant_workspace_bytes(m, h, i, group, v, plan_b) if down_plan is not None else 0)
-            workspace = _ws(need + extra, x.device)
-        _check(lib.nnf_fused_mlp_w4a16_planned(_stream(), x.data_ptr(), gamma.data_ptr(), float(eps), wgu.data_ptr(),
-                                               sgu.data_ptr(), wd.data_ptr(), sd.data_ptr(), out.data_ptr(), m, h, i, group,
-                                               zp, plan_a, plan_b, workspace.data_ptr(), workspace.numel()),
-               "nnf_fused_mlp_w4a16_planned")
-        return out
+    keep_a, plan_a = _plan_arg(gate_up_plan, sync, spin_limit)
+    keep_b, plan_b = _plan_arg(down_plan, sync, spin_limit)
     if workspace is None:
-        workspace = _ws(need, x.device)
-    _check(lib.nnf_fused_mlp_w4a16(_stream(), x.data_ptr(), gamma.data_ptr(), float(eps), wgu.data_ptr(),
-                                   sgu.data_ptr(), wd.data_ptr(), sd.data_ptr(), out.data_ptr(), m, h, i, group, zp,
-                                   workspace.data_ptr(), workspace.numel()), "nnf_fused_mlp_w4a16")
+        v = VARIANTS["gemm_mfma"]
+        need = lib.nnf_fused_mlp_w4a16_workspace_bytes(m, h, i, group)
+        extra = (lib.nnf_w4a16_gemm_variant_workspace_bytes(m, 2 * i, h, group, v, plan_a) if gate_up_plan is not None else 0) + \
+                (lib.nnf_w4a16_gemm_variant_workspace_bytes(m, h, i, group, v, plan_b) if down_plan is not None else 0)
+        workspace = _ws(need + extra, x.device)
+    _check(lib.nnf_fused_mlp_w4a16_planned(_stream(), x.data_ptr(), gamma.data_ptr(), float(eps), wgu.data_ptr(),
+                                           sgu.data_ptr(), wd.data_ptr(), sd.data_ptr(), out.data_ptr(), m, h, i, group,
+                                           zp, plan_a, plan_b, workspace.data_ptr(), workspace.numel()),
+           "nnf_fused_mlp_w4a16_planned")
     return out
 
 
@@ -287,72 +244,25 @@ EW_OPS = {"add": 0, "multiply": 1, "sigmoid": 2, "swish": 3}
 
 def elementwise(op, a, b=None, out=None):
     """y = op(a, b) over fp16 tensors (b of a's shape, or a row [cols] broadcast over a's leading axes)."""
-    lib = _lib.kernels()
-    assert a.dtype == torch.float16 and a.is_contiguous()
-    cols = a.shape[-1]
-    rows = a.numel() // cols
-    b_is_row = 0
-    if b is not None:
-        assert b.dtype == torch.float16 and b.is_contiguous()
-        b_is_row = 1 if (b.dim() == 1 and a.dim() > 1) else 0
-        assert b_is_row or b.shape == a.shape
-    if out is None:
-        out = torch.empty_like(a)
-    _check(lib.nnf_elementwise_f16(_stream(), EW_OPS[op], a.data_ptr(), _p(b), out.data_ptr(), rows, cols, b_is_row),
-           "nnf_elementwise_f16")
-    return out
+    return _native.elementwise(EW_OPS[op], a, b, out)
 
 
 def rms_norm(x, gamma, eps=1e-6, out=None):
-    lib = _lib.kernels()
-    m, k = x.shape
-    if out is None:
-        out = torch.empty_like(x)
-    _check(lib.nnf_rms_norm_f16(_stream(), x.data_ptr(), gamma.data_ptr(), out.data_ptr(), m, k, float(eps)), "nnf_rms_norm_f16")
-    return out
+    return _native.rms_norm(x, gamma, eps, out)
 
 
 def dequantize(wq, scales, bits=4, group=128, zp=8, zero_points=None, out=None):
     """W fp16 [N, K] = (q - z) * s per block of `group` weights."""
-    lib = _lib.kernels()
-    n = wq.shape[0]
-    k = wq.shape[1] * 8 // bits
-    if out is None:
-        out = torch.empty((n, k), dtype=torch.float16, device=wq.device)
-    keep, qp = _quant_arg(bits, group, zp, zero_points)
-    _check(lib.nnf_dequantize_f16(_stream(), wq.data_ptr(), scales.data_ptr(), out.data_ptr(), n, k, qp), "nnf_dequantize_f16")
-    return out
+    return _native.dequantize(wq, scales, bits, group, zp, zero_points, out)
 
 
 def wna16_gemm_fused(a, wq, scales, bits=4, group=128, zp=8, zero_points=None, rms_gamma=None, rms_eps=1e-6, bias=None,
                      residual=None, act=0, out=None, workspace=None):
     """nnf_wna16_gemm_fused: the fused product for every block parameter."""
-    lib = _lib.kernels()
-    m, k = a.shape
-    n = wq.shape[0] // (2 if act == 1 else 1)
-    if out is None:
-        out = torch.empty((m, n), dtype=torch.float16, device=a.device)
-    keep, qp = _quant_arg(bits, group, zp, zero_points)
-    if workspace is None:
-        workspace = _ws(lib.nnf_wna16_gemm_fused_workspace_bytes(m, n, k, qp, int(act)), a.device)
-    _check(lib.nnf_wna16_gemm_fused(_stream(), a.data_ptr(), wq.data_ptr(), scales.data_ptr(), out.data_ptr(), m, n, k, qp,
-                                    _p(rms_gamma), float(rms_eps), _p(bias), _p(residual), int(act), workspace.data_ptr(),
-                                    workspace.numel()), "nnf_wna16_gemm_fused")
-    return out
+    return _native.wna16_gemm_fused(a, wq, scales, bits, group, zp, zero_points, rms_gamma, rms_eps, bias, residual, act, out,
+                                    workspace)
 
 
 def fused_mlp_wna16(x, gamma, wgu, sgu, wd, sd, bits=4, group=128, zp=8, zgu=None, zd=None, eps=1e-6, out=None, workspace=None):
     """The MLP block for every block parameter (zgu / zd: zero-point tensors of the two weight matrices, or None)."""
-    lib = _lib.kernels()
-    m, h = x.shape
-    i = wgu.shape[0] // 2
-    if out is None:
-        out = torch.empty((m, h), dtype=torch.float16, device=x.device)
-    keep_a, qa = _quant_arg(bits, group, zp, zgu)
-    keep_b, qb = _quant_arg(bits, group, zp, zd)
-    if workspace is None:
-        workspace = _ws(lib.nnf_fused_mlp_wna16_workspace_bytes(m, h, i, qa, qb), x.device)
-    _check(lib.nnf_fused_mlp_wna16(_stream(), x.data_ptr(), gamma.data_ptr(), float(eps), wgu.data_ptr(), sgu.data_ptr(),
-                                   wd.data_ptr(), sd.data_ptr(), out.data_ptr(), m, h, i, qa, qb, workspace.data_ptr(),
-                                   workspace.numel()), "nnf_fused_mlp_wna16")
-    return out
+    return _native.fused_mlp_wna16(x, gamma, wgu, sgu, wd, sd, bits, group, zp, zgu, zd, eps, out, workspace)

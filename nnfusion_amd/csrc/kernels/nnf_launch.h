@@ -86,9 +86,12 @@ namespace nnf
     // 2 <= M <= 16, K = 1024 / 2048 / 4096 / 8192: weights streamed through LDS rings, activations in registers
     // (N: outputs; gate / fusion.gate: from 2 N weight rows)
     // the same kernel for groups of 2^group_shift = 32 / 64 / 128 and a scalar zero point or (zero_points != null) one per
-    // (row, group): 2 <= M <= 16, K = 2048 / 4096 / 8192, no fused parts
+    // (row, group): 2 <= M <= 16, K = 2048 / 4096 / 8192.  fusion: gamma (normalised inside the kernel; no rstd), bias /
+    // residual or gate, where w4a16_mrows_q_fused_supported
     hipError_t launch_w4a16_mrows_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
-                                    int K, int group_shift, int zp, const void* zero_points, int num_cu);
+                                    int K, int group_shift, int zp, const void* zero_points, int num_cu,
+                                    const GemvFusion& fusion = GemvFusion());
+    bool w4a16_mrows_q_fused_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool gate);
     bool w4a16_mrows_q_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu);
     // ... for 8-bit weights (u8 [N, K]; zero points u8 [N, K / group]): 2 <= M <= 16 (32 up to K = 4096), K = 2048 (groups of 32 / 64) / 4096 /
     // 8192
@@ -99,9 +102,13 @@ namespace nnf
     // more: fp32 sums of each range of K to partial[ranges][M][N], Y is not written (launch_wna16_reduce adds them up)
     int w4a16_mrows_q_any_ranges(int M, int N, int K, int group_shift, bool zero_points, int num_cu);
     hipError_t launch_w4a16_mrows_q_any(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, float* partial,
-                                        int M, int N, int K, int group_shift, int zp, const void* zero_points, int num_cu);
-    // Y [M, N] = fp16(sum over the ranges of partial[ranges][M][N])
-    hipError_t launch_wna16_reduce(hipStream_t stream, const float* partial, int ranges, void* Y, int M, int N);
+                                        int M, int N, int K, int group_shift, int zp, const void* zero_points, int num_cu,
+                                        const GemvFusion& fusion = GemvFusion());
+    bool w4a16_mrows_q_any_fused_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool gate);
+    // Y [M, N] = fp16(sum over the ranges of partial[ranges][M][N]) + bias + residual (or null); gate: SiLU-gate of
+    // partial[ranges][M][2N]
+    hipError_t launch_wna16_reduce(hipStream_t stream, const float* partial, int ranges, void* Y, int M, int N, const void* bias = nullptr,
+                                   const void* residual = nullptr, bool gate = false);
     hipError_t launch_w4a16_mrows(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                   int K, int zp, int num_cu, const GemvFusion& fusion = GemvFusion());
     bool w4a16_mrows_supported(int M, int N, int K, int num_cu, bool gate = false);

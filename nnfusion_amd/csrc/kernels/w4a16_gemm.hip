@@ -453,20 +453,21 @@ namespace nnf
         return hipGetLastError();
     }
 
-    hipError_t launch_wna16_reduce(hipStream_t stream, const float* partial, int ranges, void* Y, int M, int N)
+    hipError_t launch_wna16_reduce(hipStream_t stream, const float* partial, int ranges, void* Y, int M, int N, const void* bias,
+                                   const void* residual, bool gate)
     {
         GemmParams p;
         p.Y = (half_t*)Y;
         p.M = M;
         p.N = N;
         p.ldy = N;
-        p.bias = nullptr;
-        p.residual = nullptr;
+        p.bias = (const half_t*)bias;
+        p.residual = (const half_t*)residual;
         p.rstd = nullptr;
         p.partial = const_cast<float*>(partial);
         p.splits = ranges;
-        p.ld_partial = N;
-        return launch_reduce_any(stream, p, false, false, false);
+        p.ld_partial = gate ? 2 * N : N;
+        return launch_reduce_any(stream, p, gate, bias != nullptr, residual != nullptr);
     }
 
     // ---- the tile GEMM with other block parameters ----------------------------------------------------------------------

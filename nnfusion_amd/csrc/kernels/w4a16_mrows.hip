@@ -76,6 +76,77 @@ namespace nnf
         }
     }
 
+    // RMSNorm of the activations in registers as rms_norm_kernel computes it: fp16(x * rstd * gamma), in fp32, one rounding.
+    // Lane (m = col, kq) holds 64 bytes of each of its wavefront's GA groups; counts(g): whether this wavefront is the one
+    // that counts group g into its row's sum of squares; gsrc(g): the 64 bytes of gamma that pair with group g.
+    // sum_sq: [8 wavefronts][MB x 16 rows] of LDS of its own.  (Unlike mrows_scale_a, where rstd joins the sums at the end:
+    // these kernels have no per-group sums to scale, and x * gamma alone may leave the range of fp16.)
+    template <int MB, int GA, class Counts, class F>
+    __device__ __forceinline__ void mrows_rms_norm(uintx4 (&areg)[MB][GA][4], float* sum_sq, int K, float eps, int wave, int col, int kq,
+                                                   Counts&& counts, F&& gsrc)
+    {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+        {
+            float ss = 0.f;
+#pragma unroll
+            for (int g = 0; g < GA; ++g)
+            {
+                float sg = 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    const uint32_t rr[4] = {areg[mb][g][j].x, areg[mb][g][j].y, areg[mb][g][j].z, areg[mb][g][j].w};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                    {
+                        const half2_t h = as_half2(rr[i]);
+                        sg = __builtin_fmaf((float)h.x, (float)h.x, sg);
+                        sg = __builtin_fmaf((float)h.y, (float)h.y, sg);
+                    }
+                }
+                ss += counts(g) ? sg : 0.f;
+            }
+            ss += __shfl_xor(ss, 16, 64);
+            ss += __shfl_xor(ss, 32, 64);
+            if (kq == 0)
+                sum_sq[wave * (MB * 16) + mb * 16 + col] = ss;
+        }
+        __syncthreads();
+        float rs[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+        {
+            float total = 0.f;
+#pragma unroll
+            for (int w = 0; w < MR_WAVES; ++w)
+                total += sum_sq[w * (MB * 16) + mb * 16 + col];
+            rs[mb] = 1.0f / __builtin_sqrtf(total / (float)K + eps);
+        }
+#pragma unroll
+        for (int g = 0; g < GA; ++g)
+        {
+            const uintx4* gp = reinterpret_cast<const uintx4*>(gsrc(g));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                const uintx4 gm = gp[j];
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                {
+                    auto norm = [&](uint32_t a, uint32_t w) {
+                        const half2_t x = as_half2(a), g2 = as_half2(w);
+                        return as_u32(half2_t{(half_t)((float)x.x * rs[mb] * (float)g2.x), (half_t)((float)x.y * rs[mb] * (float)g2.y)});
+                    };
+                    uintx4 a = areg[mb][g][j];
+                    // (opaque: the compiler would keep the fp32 values of the sums of squares for this, twice the registers)
+                    asm volatile("" : "+v"(a));
+                    areg[mb][g][j] = uintx4{norm(a.x, gm.x), norm(a.y, gm.y), norm(a.z, gm.z), norm(a.w, gm.w)};
+                }
+            }
+        }
+    }
+
     // The workgroup's parked sums -> Y.  Plain: fp16 of the sum.  Fused (see GemvFusion in nnf_launch.h): the sums of
     // row m times rstd[m]; gate: tiles 2 i and 2 i + 1 of the workgroup are the gate and the up rows of its output tile
     // i; bias and residual.  t0: the workgroup's first output tile, T_out of them; N: output columns.
@@ -489,13 +560,17 @@ namespace nnf
     // loads, NSL of them) and, ZPT, their zero points (one byte per lane, NZL loads; a byte load lands in a lane's four
     // bytes of LDS).
     // LDS (bytes): weights [8 wavefronts][2 slots][GW KiB] | scales and zero points [8][2][(NSL + NZL) x 256] |
-    //              partial tiles [2][8][MB KiB] | parked sums [tiles of the workgroup][M][16] fp32
-    // pack = M | zp << 8.
-    template <int GW, int GSHIFT, bool ZPT, int MB>
+    //              (FUSED: sums of squares [8][MB x 16] fp32) | partial tiles [2][8][MB KiB] |
+    //              parked sums [tiles of the workgroup][M][16] fp32
+    // pack = M | zp << 8 | gate << 16.
+    // FUSED: RMSNorm ahead of the product (f.gamma), bias / residual or SiLU-gate behind it, as the nodes of their own
+    // would compute them.  They were launches of their own (2 - 4 us each at 8 rows, 19 of the 56 us of a decoder layer
+    // with groups of 64 and zero points); inside, the prologue runs while the first weights are on their way.
+    template <int GW, int GSHIFT, bool ZPT, int MB, bool FUSED>
     __global__ __launch_bounds__(512) void w4a16_mrows_q_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                                 const half_t* __restrict__ S, half_t* __restrict__ Y,
                                                                 const uint8_t* __restrict__ zps, int N, int tiles_q,
-                                                                int tiles_r, int pack)
+                                                                int tiles_r, int pack, GemvFusionArgs f)
     {
         static_assert(GW == 1 || GW == 2 || GW == 4, "K = 2048, 4096, 8192");
         static_assert(GSHIFT >= 5 && GSHIFT <= 7 && ((GW << (7 - GSHIFT)) & 1) == 0, "whole words of scales, whole bytes of zero points");
@@ -503,6 +578,7 @@ namespace nnf
         constexpr int STEPS = 2;
         constexpr int K = GW * STEPS * 1024, G = K >> GSHIFT;
         constexpr int GA = GW * STEPS;         // groups of 128 of a wavefront
+        constexpr int GAMMA_LOADS = (GA + 3) / 4; // of the RMSNorm weight into LDS: 1 KiB, four groups, each
         constexpr int ROW_BYTES = K / 2;       // a weight row
         constexpr int SLICE = GW * 64;         // a wavefront's bytes of a weight row per step
         constexpr int SPAN = 8 * SLICE;        // bytes of a weight row that the workgroup covers per step
@@ -525,15 +601,21 @@ namespace nnf
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int col = lane & 15; // n within the tile (B operand / D column), m for the A operand
         const int kq = lane >> 4;  // K quarter of the MFMA operands, row quad of D
-        const int M = pack & 0xff, zp = (pack >> 8) & 0xff;
+        const int M = pack & 0xff, zp = (pack >> 8) & 0xff, gate = FUSED ? (pack >> 16) & 1 : 0;
         const int b = blockIdx.x;
         const int t0 = b * tiles_q + min(b, tiles_r);
-        const int T = tiles_q + (b < tiles_r ? 1 : 0);
-        auto row0_of = [&](int i) { return __builtin_amdgcn_readfirstlane(min((t0 + i) * 16, N - 16)); };
+        const int T_out = tiles_q + (b < tiles_r ? 1 : 0);
+        const int T = gate ? 2 * T_out : T_out; // weight tiles this workgroup walks
+        auto row0_of = [&](int i) {
+            if (gate)
+                return __builtin_amdgcn_readfirstlane(((i & 1) ? N : 0) + min((t0 + (i >> 1)) * 16, N - 16));
+            return __builtin_amdgcn_readfirstlane(min((t0 + i) * 16, N - 16));
+        };
 
         uint8_t* ring = smem + wave * (2 * TILE_BYTES);
         uint8_t* aux = smem + MR_WAVES * 2 * TILE_BYTES + wave * (2 * AUX);
-        uint8_t* red = smem + MR_WAVES * 2 * TILE_BYTES + MR_WAVES * 2 * AUX; // [2][8][1024]
+        float* sum_sq = reinterpret_cast<float*>(smem + MR_WAVES * 2 * TILE_BYTES + MR_WAVES * 2 * AUX);
+        uint8_t* red = reinterpret_cast<uint8_t*>(sum_sq + (FUSED ? MR_WAVES * MB * 16 : 0)); // [2][8][MB KiB]
         float* parked = reinterpret_cast<float*>(red + 2 * MR_WAVES * MB * 1024);
 
         // weights: as in w4a16_mrows_kernel
@@ -594,6 +676,10 @@ namespace nnf
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     areg[0][g][j] = *reinterpret_cast<const uintx4*>(a_bytes + (size_t)(a_off + (g / GW) * (SPAN * 4) + (g % GW) * 256 + j * 16));
+            if (FUSED && f.gamma)
+                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [](int) { return true; }, [&](int g) {
+                    return reinterpret_cast<const uint8_t*>(f.gamma) + wave * (GW * 256) + kq * 64 + (g / GW) * (SPAN * 4) + (g % GW) * 256;
+                });
         }
         else
         {
@@ -614,11 +700,33 @@ namespace nnf
                     fetch(p + 1);
                     __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
                 }
+                else if (FUSED && f.gamma)
+                {
+                    // gamma of the wavefront's k positions into the free half, as in w4a16_mrows_kernel
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                    for (int i = 0; i < GAMMA_LOADS; ++i)
+                    {
+                        const int g = min(4 * i + (lane >> 4), GA - 1);
+                        const uint8_t* src = reinterpret_cast<const uint8_t*>(f.gamma) + wave * (GW * 256) + (g / GW) * (SPAN * 4) +
+                                             (g % GW) * 256 + (lane & 15) * 16;
+                        __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(stage + (NP & 1) * ROW_BLOCK_BYTES + i * 1024),
+                                                         16, 0, 0);
+                    }
+                    __builtin_amdgcn_s_waitcnt(vmcnt_only(GAMMA_LOADS));
+                }
                 else
                     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     areg[p / GA][p % GA][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
+            }
+            if (FUSED && f.gamma)
+            {
+                const uint8_t* gamma_block = stage + (NP & 1) * ROW_BLOCK_BYTES;
+                __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [](int) { return true; },
+                                       [&](int g) { return gamma_block + g * 256 + kq * 64; });
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __syncthreads();
@@ -709,7 +817,7 @@ namespace nnf
         }
         __builtin_amdgcn_s_waitcnt(mr_vmcnt(0)); // the reloads past the end, before the LDS goes away
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        mrows_flush<false, MB>(parked, Y, t0, T, M, N, tid, GemvFusionArgs{nullptr, nullptr, nullptr, nullptr, 0.f}, 0);
+        mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate);
     }
 
     // ---- 8-bit weights -------------------------------------------------------------------------------------------------
@@ -945,16 +1053,18 @@ namespace nnf
     // A block of 128 weights has SPC = 128 / group scales; with groups of 128 a wavefront's first block may be an odd one:
     // its scales are fetched from the 4-byte word, its zero points from the byte, at or below it (`skip` = 1), and
     // one word / byte more per row comes along.
-    template <int GW, int GSHIFT, bool ZPT>
+    // FUSED (one range of K): as in w4a16_mrows_q_kernel; over ranges the rest of the epilogue belongs to the reduction pass.
+    template <int GW, int GSHIFT, bool ZPT, bool FUSED>
     __global__ __launch_bounds__(512) void w4a16_mrows_q_any_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                                     const half_t* __restrict__ S, half_t* __restrict__ Y,
                                                                     const uint8_t* __restrict__ zps, float* __restrict__ partial,
                                                                     int N, int K, int range_blocks, int tiles_q, int tiles_r,
-                                                                    int pack)
+                                                                    int pack, GemvFusionArgs f)
     {
         static_assert(GW >= 2 && GW <= 4 && GSHIFT >= 5 && GSHIFT <= 7, "blocks per wavefront and step; groups of 32 / 64 / 128");
         constexpr int STEPS = 2, MB = 1;
         constexpr int GA = GW * STEPS;
+        constexpr int GAMMA_LOADS = (GA + 3) / 4;
         constexpr int SLICE = GW * 64;
         constexpr int TILE_BYTES = 16 * SLICE;
         constexpr int SPC = 1 << (7 - GSHIFT);                     // scales per block of 128 weights
@@ -975,21 +1085,27 @@ namespace nnf
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int col = lane & 15;
         const int kq = lane >> 4;
-        const int M = pack & 0xff, zp = (pack >> 8) & 0xff;
+        const int M = pack & 0xff, zp = (pack >> 8) & 0xff, gate = FUSED ? (pack >> 16) & 1 : 0;
         const int B = K >> 7, ROW_BYTES = K >> 1; // blocks of 128 weights in a row
         const int SROW = (K >> GSHIFT) * 2;       // bytes of a row of scales
         const int ZROW = K >> (GSHIFT + 1);       // bytes of a row of zero points
         const int b = blockIdx.x;
         const int t0 = b * tiles_q + min(b, tiles_r);
-        const int T = tiles_q + (b < tiles_r ? 1 : 0);
-        auto row0_of = [&](int i) { return __builtin_amdgcn_readfirstlane(min((t0 + i) * 16, N - 16)); };
+        const int T_out = tiles_q + (b < tiles_r ? 1 : 0);
+        const int T = gate ? 2 * T_out : T_out; // weight tiles this workgroup walks
+        auto row0_of = [&](int i) {
+            if (gate)
+                return __builtin_amdgcn_readfirstlane(((i & 1) ? N : 0) + min((t0 + (i >> 1)) * 16, N - 16));
+            return __builtin_amdgcn_readfirstlane(min((t0 + i) * 16, N - 16));
+        };
         const int b_lo = (int)blockIdx.y * range_blocks, b_hi = min(B, b_lo + range_blocks); // this workgroup's part of K
         auto own_block = [&](int st) { return b_lo + st * (8 * GW) + wave * GW; };
         auto fetch_block = [&](int st) { return min(own_block(st), b_hi - GW); };
 
         uint8_t* ring = smem + wave * (2 * TILE_BYTES);
         uint8_t* aux = smem + MR_WAVES * 2 * TILE_BYTES + wave * (2 * AUX);
-        uint8_t* red = smem + MR_WAVES * 2 * TILE_BYTES + MR_WAVES * 2 * AUX; // [2][8][1024]
+        float* sum_sq = reinterpret_cast<float*>(smem + MR_WAVES * 2 * TILE_BYTES + MR_WAVES * 2 * AUX); // (FUSED) [8][16]
+        uint8_t* red = reinterpret_cast<uint8_t*>(sum_sq + (FUSED ? MR_WAVES * MB * 16 : 0)); // [2][8][1024]
         float* parked = reinterpret_cast<float*>(red + 2 * MR_WAVES * MB * 1024);
 
         auto swz = [](int r) { return GW % 4 == 0 ? (r & 15) : GW % 2 == 0 ? (r >> 1) & 7 : (r >> 2) & 3; };
@@ -1047,7 +1163,9 @@ namespace nnf
         const uint32_t parked_addr = lds_address(parked);
         // activations: into the MFMA operand registers (through LDS as whole lines from a few rows on, see
         // workspace::mrows_stages_activations), then in the pair order of the nibble trick
-        uintx4 areg[GA][4];
+        uintx4 areg[MB][GA][4];
+        // (a group that another wavefront covers as well: counted there)
+        auto counts = [&](int p) { return p % GW >= own_block(p / GW) - fetch_block(p / GW); };
         {
             if (!workspace::mrows_stages_activations(M, K))
             {
@@ -1060,8 +1178,12 @@ namespace nnf
                     for (int g = 0; g < GW; ++g)
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
-                            areg[st * GW + g][j] = *reinterpret_cast<const uintx4*>(a_src + g * 256 + j * 16);
+                            areg[0][st * GW + g][j] = *reinterpret_cast<const uintx4*>(a_src + g * 256 + j * 16);
                 }
+                if (FUSED && f.gamma)
+                    mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, counts, [&](int p) {
+                        return reinterpret_cast<const uint8_t*>(f.gamma) + (fetch_block(p / GW) + p % GW) * 256 + kq * 64;
+                    });
             }
             else
             {
@@ -1080,11 +1202,31 @@ namespace nnf
                         fetch(p + 1);
                         __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
                     }
+                    else if (FUSED && f.gamma)
+                    {
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                        for (int i = 0; i < GAMMA_LOADS; ++i)
+                        {
+                            const int g = min(4 * i + (lane >> 4), GA - 1);
+                            const uint8_t* src = reinterpret_cast<const uint8_t*>(f.gamma) + (fetch_block(g / GW) + g % GW) * 256 + (lane & 15) * 16;
+                            __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(stage + (GA & 1) * ROW_BLOCK_BYTES + i * 1024),
+                                                             16, 0, 0);
+                        }
+                        __builtin_amdgcn_s_waitcnt(vmcnt_only(GAMMA_LOADS));
+                    }
                     else
                         __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        areg[p][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
+                        areg[0][p][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
+                }
+                if (FUSED && f.gamma)
+                {
+                    const uint8_t* gamma_block = stage + (GA & 1) * ROW_BLOCK_BYTES;
+                    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+                    mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, counts,
+                                           [&](int g) { return gamma_block + g * 256 + kq * 64; });
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 __syncthreads();
@@ -1093,7 +1235,7 @@ namespace nnf
             for (int g = 0; g < GA; ++g)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    areg[g][j] = permute_a8(areg[g][j]);
+                    areg[0][g][j] = permute_a8(areg[0][g][j]);
         }
         const uint32_t zp16 = (uint32_t)zp | ((uint32_t)zp << 16);
         const int sub = (kq * 32) >> GSHIFT; // the lane's scale within a block
@@ -1150,7 +1292,7 @@ namespace nnf
                         bq.y = as_u32((as_half2((w & MASK_HI) | MAGIC_HI) + hi_add) * sc);
                         bq.z = as_u32((as_half2((w8 & MASK_LO) | MAGIC) + lo_add) * sc);
                         bq.w = as_u32((as_half2((w8 & MASK_HI) | MAGIC_HI) + hi_add) * sc);
-                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[st * GW + g][j]),
+                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[0][st * GW + g][j]),
                                                                         __builtin_bit_cast(half8_t, bq), acc[0], 0, 0, 0);
                     }
                 }
@@ -1170,7 +1312,7 @@ namespace nnf
             }
         }
         else
-            mrows_flush<false, MB>(parked, Y, t0, T, M, N, tid, GemvFusionArgs{nullptr, nullptr, nullptr, nullptr, 0.f}, 0);
+            mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate);
     }
 
     // The same kernel with K as a run-time value: any multiple of 256 up to 8 * GW * STEPS groups (2 <= M <= 16).
@@ -1612,9 +1754,9 @@ namespace nnf
 
     namespace
     {
-        template <int GW, int GSHIFT, bool ZPT, int MB>
+        template <int GW, int GSHIFT, bool ZPT, int MB, bool FUSED>
         hipError_t launch_mrows_q_mb(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
-                                     const void* zps, int num_cu)
+                                     const void* zps, int num_cu, const GemvFusion& fusion)
         {
             if constexpr (((GW << (7 - GSHIFT)) & 1) != 0 || (MB == 2 && GW > 2))
                 return hipErrorInvalidValue;
@@ -1623,10 +1765,11 @@ namespace nnf
                 const int n_tiles = (N + 15) / 16;
                 const int grid = n_tiles < num_cu ? n_tiles : num_cu;
                 const int tiles_q = n_tiles / grid, tiles_r = n_tiles % grid;
-                const size_t lds = workspace::w4a16_mrows_q_lds_bytes(GW * 2048, M, tiles_q + (tiles_r ? 1 : 0), GSHIFT, ZPT);
+                const size_t lds = workspace::w4a16_mrows_q_lds_bytes(GW * 2048, M, (tiles_q + (tiles_r ? 1 : 0)) * (fusion.gate ? 2 : 1),
+                                                                      GSHIFT, ZPT, FUSED);
                 if (lds > MAX_LDS_BYTES)
                     return hipErrorInvalidValue;
-                auto kernel = &w4a16_mrows_q_kernel<GW, GSHIFT, ZPT, MB>;
+                auto kernel = &w4a16_mrows_q_kernel<GW, GSHIFT, ZPT, MB, FUSED>;
                 if (lds > 64 * 1024)
                 {
                     static LdsGrant granted;
@@ -1635,48 +1778,59 @@ namespace nnf
                         return e;
                 }
                 hipLaunchKernelGGL(kernel, dim3(grid), dim3(MR_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
-                                   (const half_t*)S, (half_t*)Y, (const uint8_t*)zps, N, tiles_q, tiles_r, M | (zp << 8));
+                                   (const half_t*)S, (half_t*)Y, (const uint8_t*)zps, N, tiles_q, tiles_r,
+                                   M | (zp << 8) | ((fusion.gate ? 1 : 0) << 16), fusion_args(fusion));
                 return hipGetLastError();
             }
         }
         template <int GW, int GSHIFT, bool ZPT>
         hipError_t launch_mrows_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
-                                  const void* zps, int num_cu)
+                                  const void* zps, int num_cu, const GemvFusion& f)
         {
-            return M <= 16 ? launch_mrows_q_mb<GW, GSHIFT, ZPT, 1>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu)
-                           : launch_mrows_q_mb<GW, GSHIFT, ZPT, 2>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu);
+            if (f.any())
+                return M <= 16 ? launch_mrows_q_mb<GW, GSHIFT, ZPT, 1, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f)
+                               : launch_mrows_q_mb<GW, GSHIFT, ZPT, 2, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            return M <= 16 ? launch_mrows_q_mb<GW, GSHIFT, ZPT, 1, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f)
+                           : launch_mrows_q_mb<GW, GSHIFT, ZPT, 2, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
         }
         template <int GW>
         hipError_t launch_mrows_q_gw(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
-                                     int group_shift, int zp, const void* zps, int num_cu)
+                                     int group_shift, int zp, const void* zps, int num_cu, const GemvFusion& f)
         {
             switch (group_shift * 2 + (zps ? 1 : 0))
             {
-            case 10: return launch_mrows_q<GW, 5, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu);
-            case 11: return launch_mrows_q<GW, 5, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu);
-            case 12: return launch_mrows_q<GW, 6, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu);
-            case 13: return launch_mrows_q<GW, 6, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu);
-            case 15: return launch_mrows_q<GW, 7, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu);
+            case 10: return launch_mrows_q<GW, 5, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            case 11: return launch_mrows_q<GW, 5, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            case 12: return launch_mrows_q<GW, 6, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            case 13: return launch_mrows_q<GW, 6, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            case 15: return launch_mrows_q<GW, 7, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
             default: return hipErrorInvalidValue; // groups of 128 with a scalar zero point: w4a16_mrows_kernel
             }
         }
     } // namespace
 
+    // the kernel with the nodes around the product inside it (gate: N outputs from 2 N weight rows)
+    bool w4a16_mrows_q_fused_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool gate)
+    {
+        return !(group_shift == 7 && !zero_points) && workspace::w4a16_mrows_q_fits(M, N, K, group_shift, zero_points, num_cu, true, gate);
+    }
     bool w4a16_mrows_q_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu)
     {
         return !(group_shift == 7 && !zero_points) && workspace::w4a16_mrows_q_fits(M, N, K, group_shift, zero_points, num_cu);
     }
 
     hipError_t launch_w4a16_mrows_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
-                                    int K, int group_shift, int zp, const void* zero_points, int num_cu)
+                                    int K, int group_shift, int zp, const void* zero_points, int num_cu, const GemvFusion& fusion)
     {
-        if (!w4a16_mrows_q_supported(M, N, K, group_shift, zero_points != nullptr, num_cu))
+        if (fusion.any() ? fusion.rstd || (fusion.gate && (fusion.bias || fusion.residual)) ||
+                               !w4a16_mrows_q_fused_supported(M, N, K, group_shift, zero_points != nullptr, num_cu, fusion.gate)
+                         : !w4a16_mrows_q_supported(M, N, K, group_shift, zero_points != nullptr, num_cu))
             return hipErrorInvalidValue;
         switch (K >> 11)
         {
-        case 1: return launch_mrows_q_gw<1>(stream, A, Wq, S, Y, M, N, group_shift, zp, zero_points, num_cu);
-        case 2: return launch_mrows_q_gw<2>(stream, A, Wq, S, Y, M, N, group_shift, zp, zero_points, num_cu);
-        default: return launch_mrows_q_gw<4>(stream, A, Wq, S, Y, M, N, group_shift, zp, zero_points, num_cu);
+        case 1: return launch_mrows_q_gw<1>(stream, A, Wq, S, Y, M, N, group_shift, zp, zero_points, num_cu, fusion);
+        case 2: return launch_mrows_q_gw<2>(stream, A, Wq, S, Y, M, N, group_shift, zp, zero_points, num_cu, fusion);
+        default: return launch_mrows_q_gw<4>(stream, A, Wq, S, Y, M, N, group_shift, zp, zero_points, num_cu, fusion);
         }
     }
 
@@ -1753,18 +1907,20 @@ namespace nnf
 
     namespace
     {
-        template <int GW, int GSHIFT, bool ZPT>
-        hipError_t launch_mrows_q_any(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
-                                      int zp, const void* zps, float* partial, int ranges, int range_blocks, int num_cu)
+        template <int GW, int GSHIFT, bool ZPT, bool FUSED>
+        hipError_t launch_mrows_q_any_f(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
+                                        int zp, const void* zps, float* partial, int ranges, int range_blocks, int num_cu,
+                                        const GemvFusion& fusion)
         {
             const int n_tiles = (N + 15) / 16;
             const int per_range = num_cu / ranges > 0 ? num_cu / ranges : 1;
             const int grid = n_tiles < per_range ? n_tiles : per_range;
             const int tiles_q = n_tiles / grid, tiles_r = n_tiles % grid;
-            const size_t lds = workspace::w4a16_mrows_q_any_lds_bytes(GW, M, tiles_q + (tiles_r ? 1 : 0), GSHIFT, ZPT);
+            const size_t lds = workspace::w4a16_mrows_q_any_lds_bytes(GW, M, (tiles_q + (tiles_r ? 1 : 0)) * (fusion.gate ? 2 : 1), GSHIFT,
+                                                                      ZPT, FUSED);
             if (lds > MAX_LDS_BYTES)
                 return hipErrorInvalidValue;
-            auto kernel = &w4a16_mrows_q_any_kernel<GW, GSHIFT, ZPT>;
+            auto kernel = &w4a16_mrows_q_any_kernel<GW, GSHIFT, ZPT, FUSED>;
             if (lds > 64 * 1024)
             {
                 static LdsGrant granted;
@@ -1774,18 +1930,28 @@ namespace nnf
             }
             hipLaunchKernelGGL(kernel, dim3(grid, ranges), dim3(MR_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
                                (const half_t*)S, (half_t*)Y, (const uint8_t*)zps, ranges > 1 ? partial : nullptr, N, K, range_blocks,
-                               tiles_q, tiles_r, M | (zp << 8));
+                               tiles_q, tiles_r, M | (zp << 8) | ((fusion.gate ? 1 : 0) << 16), fusion_args(fusion));
             return hipGetLastError();
+        }
+        template <int GW, int GSHIFT, bool ZPT>
+        hipError_t launch_mrows_q_any(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
+                                      int zp, const void* zps, float* partial, int ranges, int range_blocks, int num_cu,
+                                      const GemvFusion& fusion)
+        {
+            return fusion.any() ? launch_mrows_q_any_f<GW, GSHIFT, ZPT, true>(stream, A, Wq, S, Y, M, N, K, zp, zps, partial, ranges,
+                                                                              range_blocks, num_cu, fusion)
+                                : launch_mrows_q_any_f<GW, GSHIFT, ZPT, false>(stream, A, Wq, S, Y, M, N, K, zp, zps, partial, ranges,
+                                                                               range_blocks, num_cu, fusion);
         }
         template <int GW>
         hipError_t launch_mrows_q_any_gw(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                          int K, int group_shift, int zp, const void* zps, float* partial, int ranges,
-                                         int range_blocks, int num_cu)
+                                         int range_blocks, int num_cu, const GemvFusion& fusion)
         {
             switch (group_shift * 2 + (zps ? 1 : 0))
             {
 #define NNF_Q_ANY(GS, Z)                                                                                                          \
-    return launch_mrows_q_any<GW, GS, Z>(stream, A, Wq, S, Y, M, N, K, zp, zps, partial, ranges, range_blocks, num_cu)
+    return launch_mrows_q_any<GW, GS, Z>(stream, A, Wq, S, Y, M, N, K, zp, zps, partial, ranges, range_blocks, num_cu, fusion)
             case 10: NNF_Q_ANY(5, false);
             case 11: NNF_Q_ANY(5, true);
             case 12: NNF_Q_ANY(6, false);
@@ -1806,17 +1972,28 @@ namespace nnf
         return workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points, num_cu).ranges;
     }
 
-    hipError_t launch_w4a16_mrows_q_any(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, float* partial,
-                                        int M, int N, int K, int group_shift, int zp, const void* zero_points, int num_cu)
+    // one range of K with the nodes around the product inside the kernel (gate: N outputs from 2 N weight rows)
+    bool w4a16_mrows_q_any_fused_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool gate)
     {
-        const workspace::MrowsQAny pl = workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points != nullptr, num_cu);
+        return !(group_shift == 7 && !zero_points) &&
+               workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points, num_cu, true, gate).ranges == 1;
+    }
+
+    hipError_t launch_w4a16_mrows_q_any(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, float* partial,
+                                        int M, int N, int K, int group_shift, int zp, const void* zero_points, int num_cu,
+                                        const GemvFusion& fusion)
+    {
+        const workspace::MrowsQAny pl =
+            workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points != nullptr, num_cu, fusion.any(), fusion.gate);
+        if (fusion.any() && (pl.ranges != 1 || fusion.rstd || (fusion.gate && (fusion.bias || fusion.residual))))
+            return hipErrorInvalidValue;
         if (pl.ranges < 1 || (pl.ranges > 1 && !partial) || (group_shift == 7 && !zero_points))
             return hipErrorInvalidValue;
         switch (pl.gw)
         {
-        case 2: return launch_mrows_q_any_gw<2>(stream, A, Wq, S, Y, M, N, K, group_shift, zp, zero_points, partial, pl.ranges, pl.range_blocks, num_cu);
-        case 3: return launch_mrows_q_any_gw<3>(stream, A, Wq, S, Y, M, N, K, group_shift, zp, zero_points, partial, pl.ranges, pl.range_blocks, num_cu);
-        default: return launch_mrows_q_any_gw<4>(stream, A, Wq, S, Y, M, N, K, group_shift, zp, zero_points, partial, pl.ranges, pl.range_blocks, num_cu);
+        case 2: return launch_mrows_q_any_gw<2>(stream, A, Wq, S, Y, M, N, K, group_shift, zp, zero_points, partial, pl.ranges, pl.range_blocks, num_cu, fusion);
+        case 3: return launch_mrows_q_any_gw<3>(stream, A, Wq, S, Y, M, N, K, group_shift, zp, zero_points, partial, pl.ranges, pl.range_blocks, num_cu, fusion);
+        default: return launch_mrows_q_any_gw<4>(stream, A, Wq, S, Y, M, N, K, group_shift, zp, zero_points, partial, pl.ranges, pl.range_blocks, num_cu, fusion);
         }
     }
 

@@ -359,8 +359,68 @@ int nnf_dequantize_f16(nnf_stream_t stream, const void* Wq, const void* scales, 
                                        q->zero_point);
 }
 
-// The fused product with other block parameters: the plain product between the kernels of the nodes around it, as the
-// unfused graph would run them.  workspace = [ RMSNorm(A): M x K fp16 ][ product: M x rows fp16 ][ the product's own ]
+} // extern "C"
+
+namespace
+{
+    bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes)
+    {
+        const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+        return x < y + b_bytes && y < x + a_bytes;
+    }
+
+    // A fused product of 4-bit weights on a few rows (other block parameters than the plain kernels'): where the plain product
+    // runs on a row-streaming kernel, the nodes around it move into that kernel, or, over ranges of K, into the reduction
+    // pass behind it (RMSNorm stays a launch there: a range does not see a whole row).  Same arithmetic as the nodes'
+    // own kernels, 2 - 4 us each at 8 rows.  fusion.gate: N outputs from 2 N weight rows.  xn: M x K fp16, for RMSNorm;
+    // own: the product's scratch memory.  taken = false: the nodes have to run one by one, nothing was launched.
+    int wna16_fused_rows(hipStream_t s, const void* A, const void* Wq, const void* scales, void* Y, int M, int N, int K,
+                         const nnf_quant* q, const nnf::GemvFusion& fusion, void* xn, void* own, size_t own_bytes, int num_cu, bool& taken)
+    {
+        taken = false;
+        // (workgroups still read A when others write Y: an output over the input goes through the pre-pass's copy)
+        if (q->bits != 4 || M < 2 || M > 32 || !fusion.any() || overlap(A, (size_t)M * K * 2, Y, (size_t)M * N * 2))
+            return NNF_OK;
+        const int gs = group_shift_of(q->group), rows = fusion.gate ? 2 * N : N;
+        const bool zpt = q->zero_points != nullptr;
+        if (nnf::w4a16_mrows_q_supported(M, rows, K, gs, zpt, num_cu))
+        {
+            taken = nnf::w4a16_mrows_q_fused_supported(M, N, K, gs, zpt, num_cu, fusion.gate);
+            return taken ? (int)nnf::launch_w4a16_mrows_q(s, A, Wq, scales, Y, M, N, K, gs, q->zero_point, q->zero_points, num_cu, fusion)
+                         : NNF_OK;
+        }
+        const int ranges = M <= 16 ? nnf::w4a16_mrows_q_any_ranges(M, rows, K, gs, zpt, num_cu) : 0;
+        if (ranges == 1)
+        {
+            taken = nnf::w4a16_mrows_q_any_fused_supported(M, N, K, gs, zpt, num_cu, fusion.gate);
+            return taken ? (int)nnf::launch_w4a16_mrows_q_any(s, A, Wq, scales, Y, nullptr, M, N, K, gs, q->zero_point, q->zero_points,
+                                                              num_cu, fusion)
+                         : NNF_OK;
+        }
+        if (ranges > 1 && own && aligned16(own) && own_bytes >= (size_t)ranges * M * rows * sizeof(float))
+        {
+            taken = true;
+            hipError_t e = hipSuccess;
+            if (fusion.gamma)
+            {
+                e = nnf::launch_rms_norm(s, A, fusion.gamma, xn, M, K, fusion.rms_eps);
+                A = xn;
+            }
+            if (e == hipSuccess)
+                e = nnf::launch_w4a16_mrows_q_any(s, A, Wq, scales, nullptr, (float*)own, M, rows, K, gs, q->zero_point, q->zero_points, num_cu);
+            if (e == hipSuccess)
+                e = nnf::launch_wna16_reduce(s, (const float*)own, ranges, Y, M, N, fusion.bias, fusion.residual, fusion.gate);
+            return (int)e;
+        }
+        return NNF_OK;
+    }
+} // namespace
+
+extern "C" {
+
+// The fused product with other block parameters: on a few rows the row-streaming kernels with the nodes inside
+// (wna16_fused_rows), otherwise the plain product between the kernels of the nodes around it, as the unfused graph would
+// run them.  workspace = [ RMSNorm(A): M x K fp16 ][ product: M x rows fp16 ][ the product's own ]
 size_t nnf_wna16_gemm_fused_workspace_bytes(int M, int N, int K, const nnf_quant* q, int act)
 {
     if (!q || M <= 0 || N <= 0 || K <= 0)
@@ -395,6 +455,20 @@ int nnf_wna16_gemm_fused(nnf_stream_t stream, const void* A, const void* Wq, con
         return NNF_ERR_WORKSPACE_TOO_SMALL;
     uint8_t* ws = (uint8_t*)workspace;
     const hipStream_t s = (hipStream_t)stream;
+    DeviceInfo dev;
+    int st = current_device_info(dev);
+    if (st != NNF_OK)
+        return st;
+    nnf::GemvFusion fusion;
+    fusion.gamma = rms_gamma;
+    fusion.rms_eps = rms_eps;
+    fusion.bias = bias;
+    fusion.residual = residual;
+    fusion.gate = gate;
+    bool taken;
+    st = wna16_fused_rows(s, A, Wq, scales, Y, M, N, K, q, fusion, ws, l.gemm ? ws + l.xn + l.product : nullptr, l.gemm, dev.num_cu, taken);
+    if (taken || st != NNF_OK)
+        return st;
     if (rms)
     {
         const hipError_t e = nnf::launch_rms_norm(s, A, rms_gamma, ws, M, K, rms_eps);
@@ -403,7 +477,7 @@ int nnf_wna16_gemm_fused(nnf_stream_t stream, const void* A, const void* Wq, con
         A = ws;
     }
     void* product = l.product ? (void*)(ws + l.xn) : Y;
-    const int st = nnf_wna16_gemm(stream, A, Wq, scales, product, M, rows, K, q, l.gemm ? ws + l.xn + l.product : nullptr, l.gemm);
+    st = nnf_wna16_gemm(stream, A, Wq, scales, product, M, rows, K, q, l.gemm ? ws + l.xn + l.product : nullptr, l.gemm);
     if (st != NNF_OK)
         return st;
     if (gate)
@@ -675,16 +749,35 @@ int nnf_fused_mlp_wna16(nnf_stream_t stream, const void* x, const void* gamma, f
     uint8_t* own = h + nnf::workspace::align256((size_t)M * I * 2);
     const size_t own_bytes = workspace_bytes - (size_t)(own - xn);
     const hipStream_t s = (hipStream_t)stream;
-    // the nodes of the block, one after the other, fp16 tensors between them
-    hipError_t e = nnf::launch_rms_norm(s, x, gamma, xn, M, H, eps);
-    if (e != hipSuccess)
-        return (int)e;
-    int st = nnf_wna16_gemm(stream, xn, Wgu, Sgu, product, M, 2 * I, H, q_gate_up, own, own_bytes);
+    DeviceInfo dev;
+    int st = current_device_info(dev);
     if (st != NNF_OK)
         return st;
-    e = nnf::launch_silu_gate(s, product, h, M, I);
-    if (e != hipSuccess)
-        return (int)e;
+    // two fused products, or the nodes of the block one after the other; fp16 tensors between them either way
+    nnf::GemvFusion gate_up, down;
+    gate_up.gamma = gamma;
+    gate_up.rms_eps = eps;
+    gate_up.gate = true;
+    down.residual = x;
+    bool taken;
+    st = wna16_fused_rows(s, x, Wgu, Sgu, h, M, I, H, q_gate_up, gate_up, xn, own, own_bytes, dev.num_cu, taken);
+    if (st != NNF_OK)
+        return st;
+    if (!taken)
+    {
+        hipError_t e = nnf::launch_rms_norm(s, x, gamma, xn, M, H, eps);
+        if (e != hipSuccess)
+            return (int)e;
+        st = nnf_wna16_gemm(stream, xn, Wgu, Sgu, product, M, 2 * I, H, q_gate_up, own, own_bytes);
+        if (st != NNF_OK)
+            return st;
+        e = nnf::launch_silu_gate(s, product, h, M, I);
+        if (e != hipSuccess)
+            return (int)e;
+    }
+    st = wna16_fused_rows(s, h, Wd, Sd, out, M, H, I, q_down, down, nullptr, own, own_bytes, dev.num_cu, taken); // out may be x
+    if (taken || st != NNF_OK)
+        return st;
     st = nnf_wna16_gemm(stream, h, Wd, Sd, product, M, H, I, q_down, own, own_bytes);
     if (st != NNF_OK)
         return st;

@@ -566,17 +566,19 @@ namespace nnf
         // The same kernel for groups of 32 / 64 / 128 and zero points per (row, group) (w4a16_mrows_q_kernel): 2 .. 16 rows
         // (.. 32 up to K = 4096), K = 2048, 4096, 8192 (GW = K / 2048 groups of 128 per wavefront and step); per wavefront and ring slot 256 bytes
         // per 64 4-byte words of scales (GW x 128 / group scales for each of 16 rows) and as much again for zero points.
-        inline size_t w4a16_mrows_q_lds_bytes(int K, int M, int tiles, int group_shift, bool zero_points)
+        // (fused: the wavefronts' sums of squares per row for RMSNorm inside the kernel)
+        inline size_t w4a16_mrows_q_lds_bytes(int K, int M, int tiles, int group_shift, bool zero_points, bool fused = false)
         {
             const int gw = K >> 11;
             const int words = (gw << (7 - group_shift)) / 2; // of scales per row, step and wavefront
             const int loads = (16 * words + 63) / 64;
             const size_t aux = (size_t)(zero_points ? 2 : 1) * loads * 256;
             const size_t mb = M <= 16 ? 1 : 2; // blocks of 16 rows
-            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + mrows_tail_bytes((size_t)2 * 8 * mb * 1024 + (size_t)tiles * M * 64);
+            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (fused ? 8 * mb * 64 : 0) + mrows_tail_bytes((size_t)2 * 8 * mb * 1024 + (size_t)tiles * M * 64);
         }
         // (17 .. 32 rows: two blocks of rows in registers, up to K = 4096)
-        inline bool w4a16_mrows_q_fits(int M, int N, int K, int group_shift, bool zero_points, int num_cu)
+        // fused, gate: with the nodes around the product inside the kernel, N outputs from 2 N weight rows
+        inline bool w4a16_mrows_q_fits(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool fused = false, bool gate = false)
         {
             if (M < 2 || M > 32 || (M > 16 && K > 4096) || N < 16 || num_cu < 1 || (K != 2048 && K != 4096 && K != 8192) ||
                 group_shift < 5 || group_shift > 7)
@@ -585,7 +587,7 @@ namespace nnf
                 return false;
             const int n_tiles = (N + 15) / 16;
             const int grid = n_tiles < num_cu ? n_tiles : num_cu;
-            return w4a16_mrows_q_lds_bytes(K, M, (n_tiles + grid - 1) / grid, group_shift, zero_points) <= LDS_BYTES_PER_CU;
+            return w4a16_mrows_q_lds_bytes(K, M, (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid), group_shift, zero_points, fused) <= LDS_BYTES_PER_CU;
         }
         // 8-bit weights, 2 .. 16 rows, up to 32 at K <= 4096 (w8a16_mrows_q_kernel): K = 4096 / 8192 (four 64-byte pieces of a weight row per
         // wavefront and step, two / four steps), K = 2048 with groups of 32 / 64 (two pieces, two steps)
@@ -615,15 +617,16 @@ namespace nnf
         {
             int ranges = 0, range_blocks = 0, gw = 0; // ranges 0: not applicable; 1: no workspace
         };
-        inline size_t w4a16_mrows_q_any_lds_bytes(int gw, int M, int tiles, int group_shift, bool zero_points)
+        inline size_t w4a16_mrows_q_any_lds_bytes(int gw, int M, int tiles, int group_shift, bool zero_points, bool fused = false)
         {
             const int spc = 1 << (7 - group_shift);
             const int words = spc == 1 ? gw / 2 + 1 : gw * spc / 2;
             const int loads = (16 * words + 63) / 64;
             const size_t aux = (size_t)(zero_points ? 2 : 1) * loads * 256;
-            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + mrows_tail_bytes((size_t)2 * 8 * 1024 + (size_t)tiles * M * 64);
+            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (fused ? 8 * 64 : 0) + mrows_tail_bytes((size_t)2 * 8 * 1024 + (size_t)tiles * M * 64);
         }
-        inline MrowsQAny w4a16_mrows_q_any_plan(int M, int N, int K, int group_shift, bool zero_points, int num_cu)
+        inline MrowsQAny w4a16_mrows_q_any_plan(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool fused = false,
+                                                bool gate = false)
         {
             MrowsQAny p;
             if (M < 2 || M > 16 || N < 16 || K < 1024 || K > 65536 || (K & 255) || num_cu < 16 || group_shift < 5 || group_shift > 7)
@@ -646,7 +649,7 @@ namespace nnf
             }
             const int n_tiles = (N + 15) / 16, per_range = num_cu / ranges;
             const int grid = n_tiles < per_range ? n_tiles : per_range;
-            if (w4a16_mrows_q_any_lds_bytes(gw, M, (n_tiles + grid - 1) / grid, group_shift, zero_points) > LDS_BYTES_PER_CU)
+            if (w4a16_mrows_q_any_lds_bytes(gw, M, (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid), group_shift, zero_points, fused) > LDS_BYTES_PER_CU)
                 return p;
             p.ranges = ranges;
             p.range_blocks = rb;

@@ -243,3 +243,74 @@ def test_wna16_argument_errors(gpu):
     assert call(NnfQuant(8, 128, 0, None), k=192) == -2  # K % group
     assert call(NnfQuant(8, 64, 255, None)) == 0
     torch.cuda.synchronize()
+
+
+# fixed K (one, two, four blocks per wavefront and step; one and two blocks of rows; activations straight in and through
+# LDS), run-time K (two, three, four blocks; wavefronts past the end of K), ranges of K; fewer tiles than CUs, ragged N,
+# several tiles per workgroup
+FUSED_SHAPES = [(2, 40, 2048), (16, 1000, 2048), (32, 4111, 2048), (3, 520, 4096), (8, 4111, 4096), (17, 300, 4096), (32, 5000, 4096),
+                (2, 1000, 8192), (16, 4111, 8192), (2, 300, 3584), (16, 1000, 3584), (9, 520, 5120), (16, 4111, 7168), (6, 33, 2560),
+                (5, 520, 11008), (16, 1000, 14336)]
+
+
+@pytest.mark.parametrize("m,n,k", FUSED_SHAPES)
+@pytest.mark.parametrize("group,zp_tensor", [(32, True), (64, False), (64, True), (128, True)])
+def test_fused_rows_equal_the_nodes(gpu, m, n, k, group, zp_tensor):
+    """The nodes around a product inside the row-streaming kernels against the same nodes as calls of their own.  Without
+    RMSNorm bit for bit.  With it the sum of squares is added in another order, so a normalised activation may round the
+    other way now and then (2^-11 of its value): on a sum of K independent terms that is at most 2^-11 of its RMS (five
+    sigma: 2.5e-3), plus the rounding of y itself (2^-11 of up to five RMS)."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    a, wq, s, zps = _case(m * 17 + n + k + group, m, 2 * n, k, 4, group, zp_tensor)
+    t = [torch.from_numpy(x).to(gpu) for x in (a, wq, s)]
+    tz = torch.from_numpy(zps).to(gpu) if zp_tensor else None
+    gen = torch.Generator(device="cpu").manual_seed(m + n)
+    gamma = torch.randn(k, generator=gen).mul(0.1).add(1).half().to(gpu)
+    bias = torch.randn(n, generator=gen).half().to(gpu)
+    res = torch.randn(m, n, generator=gen).half().to(gpu)
+    q = dict(bits=4, group=group, zp=5)
+    half = lambda x: None if x is None else x[:n].contiguous()
+    w1, s1, z1 = half(t[1]), half(t[2]), half(tz)
+    plain = ops.wna16_gemm(t[0], w1, s1, zero_points=z1, **q)
+    y = ops.wna16_gemm_fused(t[0], w1, s1, zero_points=z1, bias=bias, residual=res, **q)
+    assert torch.equal(y, ops.elementwise("add", ops.elementwise("add", plain, bias), res))
+    inplace = res.clone()
+    ops.wna16_gemm_fused(t[0], w1, s1, zero_points=z1, residual=inplace, out=inplace, **q)
+    assert torch.equal(inplace, ops.elementwise("add", plain, res))
+
+    def gated(x):
+        p = ops.wna16_gemm(x, t[1], t[2], zero_points=tz, **q).float()
+        g = p[:, :n]
+        return (g / (1 + torch.exp(-g)) * p[:, n:])
+
+    def close(y, ref, tol):
+        rms = float(ref.float().pow(2).mean().sqrt())
+        assert torch.isfinite(y).all()
+        assert float((y.float() - ref.float()).abs().max()) <= tol * rms
+
+    # (fp16 results of values up to some ten RMS, the device's exp)
+    close(ops.wna16_gemm_fused(t[0], t[1], t[2], zero_points=tz, act=1, **q), gated(t[0]), 1e-2)
+    # activations times gamma beyond the range of fp16 are still normalised
+    x = (t[0] * 12000).clamp(-6e4, 6e4)
+    normed = ops.rms_norm(x, gamma, 1e-5)
+    close(ops.wna16_gemm_fused(x, w1, s1, zero_points=z1, rms_gamma=gamma, rms_eps=1e-5, **q),
+          ops.wna16_gemm(normed, w1, s1, zero_points=z1, **q), 5e-3)
+    close(ops.wna16_gemm_fused(x, t[1], t[2], zero_points=tz, rms_gamma=gamma, rms_eps=1e-5, act=1, **q), gated(normed), 2e-2)
+
+
+def test_fused_rows_with_the_output_over_the_input(gpu):
+    """x = product(RMSNorm(x)) written over x: workgroups that finish must not change what others still read."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    m, k = 8, 4096
+    a, wq, s, zps = _case(77, m, k, k, 4, 64, True)
+    t = [torch.from_numpy(x).to(gpu) for x in (a, wq, s, zps)]
+    gamma = torch.ones(k, dtype=torch.float16, device=gpu)
+    ref = ops.wna16_gemm(ops.rms_norm(t[0], gamma), t[1], t[2], group=64, zero_points=t[3])
+    ops.wna16_gemm_fused(t[0], t[1], t[2], group=64, zero_points=t[3], rms_gamma=gamma, out=t[0])
+    assert torch.equal(t[0], ref)

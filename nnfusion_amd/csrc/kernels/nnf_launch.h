@@ -123,8 +123,9 @@ namespace nnf
                                         int M, int N, int K, int zp, int num_cu, const void* gamma = nullptr, void* Y = nullptr,
                                         const GemvFusion* epilogue = nullptr, uint32_t* sync = nullptr);
 
+    // (bias, residual: added behind the product, each or null; the residual may be Y)
     hipError_t launch_w4a16_skinny(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M,
-                                   int N, int K, int zp, int num_cu);
+                                   int N, int K, int zp, int num_cu, const void* bias = nullptr, const void* residual = nullptr);
     // true when one workgroup can hold the activations (M <= 16 rows of K) in LDS
     bool w4a16_skinny_supported(int M, int N, int K);
 

@@ -16,6 +16,7 @@
 #include "../nnf_workspace.h"
 
 #include <algorithm>
+#include <initializer_list>
 
 namespace nnf
 {
@@ -209,32 +210,74 @@ namespace nnf
         }
     }
 
-    // Epilogues for the M <= 16 path, whose GEMV kernel writes plain fp16 products.
+    // Epilogues behind kernels that write plain fp16 products: bound by memory.  Eight columns per thread, 16 bytes per
+    // access, where N is a multiple of eight (the rows of T and Y then start on 16-byte boundaries: the buffers do);
+    // otherwise one column.  grid: x over the columns of a row, y = row (several rows per workgroup row above 65535).
     // T [M, 2N] = (gate | up) products  ->  Y [M, N] = SiLU(gate) * up
-    __global__ __launch_bounds__(256) void skinny_silu_gate_kernel(const half_t* __restrict__ T, half_t* __restrict__ Y,
-                                                                   int M, int N)
+    __device__ __forceinline__ half_t silu_gate_of(half_t gate, half_t up)
     {
-        const int i = blockIdx.x * 256 + threadIdx.x;
-        if (i >= M * N)
+        const float g = (float)gate, u = (float)up;
+        return (half_t)(g * (1.0f / (1.0f + __expf(-g))) * u);
+    }
+    template <bool VEC>
+    __global__ __launch_bounds__(256) void silu_gate_kernel(const half_t* __restrict__ T, half_t* __restrict__ Y, int M, int N)
+    {
+        constexpr int W = VEC ? 8 : 1;
+        const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * W;
+        if (n >= N)
             return;
-        const int m = i / N, n = i - m * N;
-        const float g = (float)T[(size_t)m * 2 * N + n];
-        const float u = (float)T[(size_t)m * 2 * N + N + n];
-        Y[i] = (half_t)(g * (1.0f / (1.0f + __expf(-g))) * u);
+        for (int m = blockIdx.y; m < M; m += gridDim.y)
+        {
+            const half_t* g = T + (size_t)m * 2 * N + n;
+            half_t* y = Y + (size_t)m * N + n;
+            if constexpr (VEC)
+            {
+                const half8_t gv = *reinterpret_cast<const half8_t*>(g), uv = *reinterpret_cast<const half8_t*>(g + N);
+                half8_t o;
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    o[i] = silu_gate_of(gv[i], uv[i]);
+                *reinterpret_cast<half8_t*>(y) = o;
+            }
+            else
+                *y = silu_gate_of(*g, g[N]);
+        }
     }
     // Y [M, N] = T [M, N] + bias [N] (rounded to fp16), then + residual [M, N]; T may be Y, residual may be Y
-    __global__ __launch_bounds__(256) void skinny_bias_residual_kernel(const half_t* T, half_t* Y, const half_t* bias,
-                                                                       const half_t* residual, int M, int N)
+    template <bool VEC>
+    __global__ __launch_bounds__(256) void bias_residual_kernel(const half_t* T, half_t* Y, const half_t* bias, const half_t* residual,
+                                                                int M, int N)
     {
-        const int i = blockIdx.x * 256 + threadIdx.x;
-        if (i >= M * N)
+        constexpr int W = VEC ? 8 : 1;
+        const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * W;
+        if (n >= N)
             return;
-        float v = (float)T[i];
-        if (bias)
-            v = (float)(half_t)(v + (float)bias[i % N]);
-        if (residual)
-            v = v + (float)residual[i];
-        Y[i] = (half_t)v;
+        auto finish = [&](half_t t, half_t b, half_t r) {
+            float v = (float)t;
+            if (bias)
+                v = (float)(half_t)(v + (float)b);
+            if (residual)
+                v = v + (float)r;
+            return (half_t)v;
+        };
+        for (int m = blockIdx.y; m < M; m += gridDim.y)
+        {
+            const size_t at = (size_t)m * N + n;
+            if constexpr (VEC)
+            {
+                half8_t t = *reinterpret_cast<const half8_t*>(T + at), b = t, r = t;
+                if (bias)
+                    b = *reinterpret_cast<const half8_t*>(bias + n);
+                if (residual)
+                    r = *reinterpret_cast<const half8_t*>(residual + at);
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    t[i] = finish(t[i], b[i], r[i]);
+                *reinterpret_cast<half8_t*>(Y + at) = t;
+            }
+            else
+                Y[at] = finish(T[at], bias ? bias[n] : (half_t)0.f, residual ? residual[at] : (half_t)0.f);
+        }
     }
 
     namespace
@@ -339,22 +382,14 @@ namespace nnf
             return route.kind == W4A16Route::ROWS ? launch_w4a16_gemv_rows(stream, A, Wq, S, Y, N, K, zp, num_cu, fusion)
                                                   : launch_w4a16_mrows(stream, A, Wq, S, Y, M, N, K, zp, num_cu, fusion);
         }
-        // ---- the MFMA GEMV kernel on the (normalised) activations, then a small element-wise kernel for whatever
-        // epilogue is asked for ----------------------------------------------------------------------------------
+        // ---- the MFMA GEMV kernel on the (normalised) activations, bias and residual inside, SiLU-gate as an element-wise
+        // kernel behind it ----------------------------------------------------------------------------------------
         if (route.kind == W4A16Route::SKINNY)
         {
-            void* y_gemv = route.via_scratch ? partial_ws : Y;
-            hipError_t e = launch_w4a16_skinny(stream, A, Wq, S, y_gemv, M, n_rows, K, zp, num_cu);
-            if (e != hipSuccess || (!gate && !hb && !hr))
-                return e;
-            const int blocks = (M * N + 255) / 256;
-            if (gate)
-                hipLaunchKernelGGL(skinny_silu_gate_kernel, dim3(blocks), dim3(256), 0, stream, (const half_t*)y_gemv,
-                                   (half_t*)Y, M, N);
-            else
-                hipLaunchKernelGGL(skinny_bias_residual_kernel, dim3(blocks), dim3(256), 0, stream, (const half_t*)y_gemv,
-                                   (half_t*)Y, (const half_t*)bias, (const half_t*)residual, M, N);
-            return hipGetLastError();
+            if (!gate)
+                return launch_w4a16_skinny(stream, A, Wq, S, Y, M, N, K, zp, num_cu, bias, residual);
+            const hipError_t e = launch_w4a16_skinny(stream, A, Wq, S, partial_ws, M, n_rows, K, zp, num_cu);
+            return e != hipSuccess ? e : launch_silu_gate(stream, partial_ws, Y, M, N);
         }
         // ---- more activations than one workgroup holds: a GEMV kernel over ranges of K, then the reduction pass
         // (which applies rstd and the epilogue) ------------------------------------------------------------------
@@ -441,15 +476,30 @@ namespace nnf
         hipLaunchKernelGGL(rms_norm_kernel, dim3(M), dim3(256), 0, stream, (const half_t*)X, (const half_t*)gamma, (half_t*)Xn, M, K, eps);
         return hipGetLastError();
     }
+    namespace
+    {
+        // (every pointer: aligned to 16 bytes where N is a multiple of eight, or one column at a time)
+        bool rows_of_whole_pieces(int N, std::initializer_list<const void*> pointers)
+        {
+            uintptr_t bits = (uintptr_t)(N % 8) * 2;
+            for (const void* p : pointers)
+                bits |= reinterpret_cast<uintptr_t>(p);
+            return (bits & 15) == 0;
+        }
+        dim3 row_grid(int M, int N, bool vec) { return dim3((unsigned)((N + (vec ? 2047 : 255)) / (vec ? 2048 : 256)), (unsigned)std::min(M, 65535)); }
+    } // namespace
     hipError_t launch_silu_gate(hipStream_t stream, const void* T, void* Y, int M, int N)
     {
-        hipLaunchKernelGGL(skinny_silu_gate_kernel, dim3((M * N + 255) / 256), dim3(256), 0, stream, (const half_t*)T, (half_t*)Y, M, N);
+        const bool vec = rows_of_whole_pieces(N, {T, Y});
+        hipLaunchKernelGGL(vec ? silu_gate_kernel<true> : silu_gate_kernel<false>, row_grid(M, N, vec), dim3(256), 0, stream,
+                           (const half_t*)T, (half_t*)Y, M, N);
         return hipGetLastError();
     }
     hipError_t launch_bias_residual(hipStream_t stream, const void* T, void* Y, const void* bias, const void* residual, int M, int N)
     {
-        hipLaunchKernelGGL(skinny_bias_residual_kernel, dim3((M * N + 255) / 256), dim3(256), 0, stream, (const half_t*)T, (half_t*)Y,
-                           (const half_t*)bias, (const half_t*)residual, M, N);
+        const bool vec = rows_of_whole_pieces(N, {T, Y, bias, residual});
+        hipLaunchKernelGGL(vec ? bias_residual_kernel<true> : bias_residual_kernel<false>, row_grid(M, N, vec), dim3(256), 0, stream,
+                           (const half_t*)T, (half_t*)Y, (const half_t*)bias, (const half_t*)residual, M, N);
         return hipGetLastError();
     }
 

@@ -62,6 +62,10 @@ namespace nnf
         int s_row_groups;  // row stride of S (elements) = full K / 128
         int k_last;        // length of the last range (the kernel's K is the length of the others)
         float* partial;    // [ksplits][M][N]
+        // without KSPLIT, each or null: Y = fp16(fp16(product + bias[n]) + residual[m, n]); the residual may be Y itself.
+        // (An element-wise kernel of its own took 1.9 us and a gap of 1 - 2: down projection of a shard at 6 rows, K = 5504.)
+        const half_t* bias;
+        const half_t* residual;
     };
 
     // rows of activations from which a wavefront loads its own operand instead of staging all rows in LDS
@@ -384,6 +388,14 @@ namespace nnf
         // scalar operand, so the masks live in scalar registers and the magic number in a vector register
         // (MAGIC is set at the top of the kernel, with every lane active)
 
+        // (columns of a last tile that was moved back belong to the tile before it: written once, so that a residual that is
+        // the output buffer is added once)
+        auto store = [&](int m, int n, int tile, float v) {
+            if (n < tile * 16)
+                return;
+            const size_t at = (size_t)m * N + n;
+            Y[at] = finish_bias_residual(v, sp.bias, n, sp.residual, at);
+        };
         int local_tile = 0;
         // MFMAs of one pass h of a tile from register set wt, scales from LDS copy `par`, added to acc
         auto compute = [&](floatx4 acc, const uintx4* wt, auto hh, int par) -> floatx4 {
@@ -476,7 +488,7 @@ namespace nnf
                         if (KSPLIT)
                             sp.partial[((size_t)k_range * M + (o >> 4)) * N + n] = v;
                         else
-                            Y[(size_t)(o >> 4) * N + n] = (half_t)v;
+                            store(o >> 4, n, tile_cur, v);
                     }
                 }
                 else if (q == 0)
@@ -496,7 +508,7 @@ namespace nnf
                     if (KSPLIT)
                         sp.partial[((size_t)k_range * M + (r >> 4)) * N + n] = outb[i];
                     else
-                        Y[(size_t)(r >> 4) * N + n] = (half_t)outb[i];
+                        store(r >> 4, n, tile0 + lt * stride, outb[i]);
                 }
             }
             ++local_tile;
@@ -619,17 +631,20 @@ namespace nnf
     }
 
     hipError_t launch_w4a16_skinny(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M,
-                                   int N, int K, int zp, int num_cu)
+                                   int N, int K, int zp, int num_cu, const void* bias, const void* residual)
     {
         SkinnyPlan p = plan_skinny(M, K);
+        SkinnySplit sp = SkinnySplit();
+        sp.bias = (const half_t*)bias;
+        sp.residual = (const half_t*)residual;
         switch (p.cps * 10 + p.h)
         {
-        case 11: return launch_cps<1, true, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu);
-        case 21: return launch_cps<2, true, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu);
-        case 31: return launch_cps<3, false, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu);
-        case 41: return launch_cps<4, false, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu);
-        case 32: return launch_cps<3, false, 2>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu);
-        case 42: return launch_cps<4, false, 2>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu);
+        case 11: return launch_cps<1, true, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu, sp);
+        case 21: return launch_cps<2, true, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu, sp);
+        case 31: return launch_cps<3, false, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu, sp);
+        case 41: return launch_cps<4, false, 1>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu, sp);
+        case 32: return launch_cps<3, false, 2>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu, sp);
+        case 42: return launch_cps<4, false, 2>(stream, A, Wq, S, Y, M, N, K, zp, p, num_cu, sp);
         default: return hipErrorInvalidValue;
         }
     }
@@ -646,7 +661,7 @@ namespace nnf
         if (k_range <= 0 || (K + k_range - 1) / k_range != ksplits)
             return hipErrorInvalidValue;
         SkinnyPlan p = workspace::plan_w4a16_skinny(M, k_range);
-        SkinnySplit sp;
+        SkinnySplit sp = SkinnySplit();
         sp.ksplits = ksplits;
         sp.lda = K;
         sp.w_row_bytes = K >> 1;

@@ -184,3 +184,27 @@ def test_every_kernel_variant_that_accepts_a_shape_matches_the_oracle(gpu, m, n,
     assert "auto" in served and "gemm_mfma" in served
     assert ("gemv_rows" in served) == (m == 1 or (m <= 32 and k % 256 == 0 and k >= 1024))
     assert ("gemv_valu" in served) == (m <= 16)
+
+
+# K no multiple of 256: the MFMA GEMV kernel with one, two and three groups per wavefront, and three / four in two passes;
+# N whole tiles, a last tile moved back over its neighbour's columns, fewer tiles than workgroups
+@pytest.mark.parametrize("m,n,k", [(2, 64, 384), (16, 1000, 1920), (6, 4111, 3968), (16, 520, 2944), (6, 4096, 5504), (3, 1001, 5504),
+                                   (2, 4111, 11136), (1, 1000, 15488)])
+def test_mfma_gemv_adds_bias_and_residual_as_the_nodes_do(gpu, m, n, k):
+    """Bias and residual behind the product inside the kernel: bit for bit what the nodes of their own make of the plain
+    product, also with the residual in the output buffer (columns of the moved-back tile must be added once)."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    a, wq, s = datagen.w4a16_case(m + n + k, m, n, k)
+    t = [torch.from_numpy(x).to(gpu) for x in (a, wq, s)]
+    gen = torch.Generator(device="cpu").manual_seed(k)
+    bias = torch.randn(n, generator=gen).half().to(gpu)
+    res = torch.randn(m, n, generator=gen).half().to(gpu)
+    plain = ops.w4a16_gemm(*t)
+    both = ops.elementwise("add", ops.elementwise("add", plain, bias), res)
+    assert torch.equal(ops.w4a16_gemm_fused(*t, bias=bias, residual=res), both)
+    y = res.clone()
+    ops.w4a16_gemm_fused(*t, residual=y, out=y)
+    assert torch.equal(y, ops.elementwise("add", plain, res))

@@ -250,7 +250,9 @@ def test_wna16_argument_errors(gpu):
 # several tiles per workgroup
 FUSED_SHAPES = [(2, 40, 2048), (16, 1000, 2048), (32, 4111, 2048), (3, 520, 4096), (8, 4111, 4096), (17, 300, 4096), (32, 5000, 4096),
                 (2, 1000, 8192), (16, 4111, 8192), (2, 300, 3584), (16, 1000, 3584), (9, 520, 5120), (16, 4111, 7168), (6, 33, 2560),
-                (5, 520, 11008), (16, 1000, 14336)]
+                (5, 520, 11008), (16, 1000, 14336),
+                # the nodes one by one behind the tile kernels: whole 16-byte pieces of a row, and one column at a time
+                (40, 1000, 1024), (37, 1001, 640)]
 
 
 @pytest.mark.parametrize("m,n,k", FUSED_SHAPES)

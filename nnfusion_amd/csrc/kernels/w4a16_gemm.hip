@@ -10,7 +10,7 @@
 //   * epilogues: bias, residual add, SiLU(gate) * up with the gate and up projections as two halves of
 //     the N tile -- in the tile GEMM's epilogue, in the reduction pass, or in an element-wise kernel
 //     behind a GEMV kernel.
-//   * tile height and split of the work over the CUs follow nnf::workspace::plan_w4a16_sk.
+//   * tile height and split of the work over the CUs follow nnf::workspace::plan_w4a16_tiles.
 #include "w4a16_gemm_sk_launch.h"
 
 #include "../nnf_workspace.h"
@@ -327,7 +327,8 @@ namespace nnf
         // RMSNorm's rstd[] can be left to the GEMM launch itself: the caller gave (zeroed) synchronisation words
         bool rstd_inside_tile_gemm(const workspace::SkPlan& plan, const LaunchChoice& choice, int num_cu)
         {
-            return plan.grid <= num_cu && choice.sync_flags && choice.sync_bytes >= plan.sync_bytes(true);
+            // (two words for it alone where no tile is shared)
+            return plan.grid <= num_cu && choice.sync_flags && choice.sync_bytes >= (plan.slots ? plan.sync_bytes(true) : 2 * sizeof(unsigned));
         }
     } // namespace
 
@@ -343,7 +344,8 @@ namespace nnf
             return hipErrorInvalidValue;
         const int n_rows = gate ? 2 * N : N; // weight rows
         const W4A16Route route =
-            workspace::route_w4a16(M, N, K, gate, rms, hr && residual == Y, num_cu, choice.path, choice.tile_rows, choice.k_parts, choice.tile_cols);
+            workspace::route_w4a16(M, N, K, gate, rms, hr && residual == Y, num_cu, choice.path, choice.tile_rows, choice.k_parts,
+                                   choice.tile_cols, choice.sync_flags ? choice.sync_bytes : 0);
         if (route.kind == W4A16Route::NONE || (route.partial_bytes > 0 && !partial_ws) || (route.rms_bytes > 0 && !rms_ws))
             return hipErrorInvalidValue;
         // ---- RMSNorm pre-pass: rstd[m] for the kernels that multiply the weight in themselves, the normalised
@@ -528,7 +530,7 @@ namespace nnf
     {
         if (!w4a16_gemm_q_supported(M, N, K, group_shift))
             return hipErrorInvalidValue;
-        const workspace::SkPlan plan = workspace::plan_w4a16_sk(M, N, K, false, num_cu);
+        const workspace::SkPlan plan = workspace::plan_w4a16_tiles(M, N, K, false, false, num_cu, choice.sync_flags ? choice.sync_bytes : 0);
         if (plan.slots && !partial_ws)
             return hipErrorInvalidValue;
         SkGemmParams p;

@@ -1309,6 +1309,33 @@ int main(int argc, char** argv)
             EXPECT(ws::plan_w4a16_sk(4096, 8192, 8192, false, 256, 0, 0, 128).tile_weight_rows == 256);  // width alone: the plan's
             // K = 128 * odd: the last superstep of a tile holds one group
             EXPECT(ws::plan_w4a16_sk(64, 512, 384, false, 256).supersteps == 2);
+            // the library's own plan: never more scratch memory than the even split (workspaces are sized for that), workgroups
+            // that share a tile all resident, equal parts of a tile, tiles the kernels are built for
+            unsigned seed = 12345;
+            auto draw = [&](int low, int high) {
+                seed = seed * 1664525u + 1013904223u;
+                return low + (int)((seed >> 8) % (unsigned)(high - low + 1));
+            };
+            for (int i = 0; i < 4000; ++i)
+            {
+                const int m = 17 + draw(0, 1 << draw(1, 12)), n = draw(1, 1 << draw(1, 14)), k = 128 * draw(1, 1 << draw(0, 7));
+                const bool gate = draw(0, 2) == 0;
+                const int cus = i % 5 == 0 ? draw(1, 304) : 256;
+                const auto even = ws::plan_w4a16_sk(m, n, k, gate, cus), p = ws::plan_w4a16_tiles(m, n, k, gate, draw(0, 1) != 0, cus);
+                EXPECT(p.bytes() <= even.bytes() && p.supersteps == even.supersteps);
+                EXPECT(p.units == (long long)p.tiles_m * p.tiles_n * p.supersteps && p.grid >= 1 && p.grid <= p.units);
+                EXPECT(p.tiles_m * p.tile_rows >= m && (p.tiles_m - 1) * p.tile_rows < m);
+                EXPECT(p.tiles_n == ws::ceil_div(n, (gate || p.tile_weight_rows == 128) ? 128 : 256));
+                EXPECT(p.slots == 0 || p.grid <= cus);
+                const bool narrow = p.tile_weight_rows == 128;
+                EXPECT(p.tile_rows == 256 || p.tile_rows == 128 || (p.tile_rows == 64 && (gate || narrow)) || (p.tile_rows == 32 && !narrow));
+                EXPECT(!(gate && narrow));
+                const size_t words = (size_t)draw(1, 200) * 8;
+                const auto few = ws::plan_w4a16_tiles(m, n, k, gate, false, cus, words);
+                EXPECT(few.slots == 0 || few.sync_bytes() <= words || few.grid == even.grid);
+                const auto r = ws::route_w4a16(m, n, k, gate, false, false, cus, 3);
+                EXPECT(r.partial_bytes == even.bytes());
+            }
         }
     });
 

@@ -455,3 +455,34 @@ def test_fused_parts_in_the_workspace_the_query_asks_for(gpu, m, n, k):
     assert ops.w4a16_gemm_fused(ta, tw, ts, act=1).shape == (m, n)
     assert ops.w4a16_gemm_fused(ta, tw, ts, act=1, rms_gamma=tg, rms_eps=1e-6).shape == (m, n)
     torch.cuda.synchronize()
+
+
+# the library's own plan: whole tiles of each shape (fewer than CUs, more than CUs), tiles in 2 .. 16 equal parts, the even
+# split; ragged M and N, K with a last superstep of one group
+@pytest.mark.parametrize("m,n,k", [(20, 1160, 640), (33, 300, 16256), (64, 4096, 2304), (73, 12288, 1536), (160, 1792, 5504), (200, 257, 11008),
+                                   (250, 4111, 640), (315, 9216, 2304), (450, 448, 640), (450, 1800, 7168), (700, 10000, 512), (1000, 256, 5504),
+                                   (1800, 2500, 1408), (2500, 16384, 384), (3000, 700, 3072)])
+def test_own_plan_matches_whole_tiles(gpu, m, n, k):
+    """The plan the library picks against whole tiles of 128 x 128, one workgroup each (the order in which a tile's K is
+    added differs: fp32 sums of K terms, then one rounding to fp16; 2e-3 of the RMS is four times that rounding at the
+    RMS), with and without synchronisation words (bit for bit), plain, with RMSNorm and residual, with SiLU-gate."""
+    import torch
+
+    from nnfusion_amd import datagen, ops
+
+    a, wq, s = datagen.w4a16_case(m + n + k, m, 2 * n, k)
+    a, wq, s = (torch.from_numpy(x).to(gpu) for x in (a, wq, s))
+    w1, s1 = wq[:n].contiguous(), s[:n].contiguous()
+    gen = torch.Generator(device="cpu").manual_seed(n)
+    gamma = torch.randn(k, generator=gen).mul(0.1).add(1).half().to(gpu)
+    res = torch.randn(m, n, generator=gen).half().to(gpu)
+    sync = ops.sync_flags(gpu)
+    for w, sc, parts in ((w1, s1, {}), (w1, s1, dict(rms_gamma=gamma, residual=res)), (wq, s, dict(act=1, rms_gamma=gamma))):
+        ref = ops.w4a16_gemm_fused(a, w, sc, variant="gemm_mfma", plan=(128, 1, 256 if "act" in parts else 128), **parts).float()
+        one = ops.w4a16_gemm_fused(a, w, sc, variant="gemm_mfma", sync=sync, plan=(0, 0, 0), **parts)
+        two = ops.w4a16_gemm_fused(a, w, sc, variant="gemm_mfma", plan=(0, 0, 0), **parts)
+        assert torch.equal(one, two)
+        err = float((one.float() - ref).abs().max())
+        assert err <= (2e-2 if "act" in parts else 1e-2) * float(ref.pow(2).mean().sqrt()), err
+        assert float((one.float() - ref).pow(2).mean().sqrt()) <= 2e-3 * float(ref.pow(2).mean().sqrt())
+        assert not sync.any()

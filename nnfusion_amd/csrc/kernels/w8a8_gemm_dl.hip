@@ -498,16 +498,29 @@ namespace nnf
             }
         }
         const float st = RAW ? 0.f : p.s_tok[m];
-        for (int j = 0; j < 4 && n + j < p.N; ++j)
+        const size_t at = (size_t)m * p.N + n;
+        if (RAW)
         {
-            if (RAW)
-                p.acc[(size_t)m * p.N + n + j] = a[j];
+            if (vec)
+                *reinterpret_cast<intx4*>(p.acc + at) = intx4{a[0], a[1], a[2], a[3]};
             else
-            {
-                float v = (float)a[j] * st;
-                p.Y[(size_t)m * p.N + n + j] = f32_to_f16_two_step(v * p.s_ch[n + j]);
-            }
+                for (int j = 0; j < 4 && n + j < p.N; ++j)
+                    p.acc[at + j] = a[j];
+            return;
         }
+        half4_t y;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            const float v = (float)a[j] * st;
+            y[j] = f32_to_f16_two_step(v * p.s_ch[min(n + j, p.N - 1)]);
+        }
+        // (whole quads of a row as one 8-byte store)
+        if (vec)
+            *reinterpret_cast<half4_t*>(p.Y + at) = y;
+        else
+            for (int j = 0; j < 4 && n + j < p.N; ++j)
+                p.Y[at + j] = y[j];
     }
 
     namespace
@@ -567,7 +580,9 @@ namespace nnf
                     return launch_tile<2, 4, 2, 1, 3, RAW, false, 4>(stream, p);
                 e = launch_tile<2, 4, 2, 1, 3, RAW, true, 4>(stream, p);
                 break;
-            default: // 64 x 256, always through the partial sums: three stages of 128, one workgroup per CU
+            default: // 64 x 256, three stages of 128, one workgroup per CU
+                if (!plan.reduce_pass)
+                    return launch_tile<1, 8, 2, 1, 3, RAW, false, 2, 128>(stream, p);
                 e = launch_tile<1, 8, 2, 1, 3, RAW, true, 2, 128>(stream, p);
                 break;
             }
@@ -584,7 +599,7 @@ namespace nnf
                                 void* Y, void* acc, int M, int N, int K, void* partial_ws, const LaunchChoice& choice)
     {
         const int tile = workspace::w8a8_forced_tile(choice.tile_rows, choice.tile_cols);
-        const workspace::GemmPlan plan = workspace::plan_w8a8_gemm(M, N, K, tile, choice.k_parts);
+        const workspace::GemmPlan plan = workspace::plan_w8a8_launch(M, N, K, tile, choice.k_parts);
         if (plan.reduce_pass && !partial_ws)
             return hipErrorInvalidValue;
         Q8GemmParams p;

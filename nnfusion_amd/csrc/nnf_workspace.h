@@ -98,6 +98,33 @@ namespace nnf
         {
             return plan_gemm(M, N, K, false, true, forced_tile, forced_splits);
         }
+        // What the launch runs: that plan, but for 64 x 256 tiles, which write their results themselves where K is in one range
+        // and whose ranges (never more than the plan's, whose scratch memory is what callers bring) follow a fit of measured
+        // times: per round of tiles 3.6 us, per 128 of K 0.47 and up to 0.64 with the CUs busy; ranges 2 us, 0.28 each and their
+        // sums at 10 TB/s (1482 timings, 17 .. 64 rows, 64 %: within 3 %).  33 .. 64 rows: 7 % faster in the geometric mean of
+        // 66 products, 58 x 12672 x 512 10.1 -> 7.9 us.
+        inline GemmPlan plan_w8a8_launch(int M, int N, int K, int forced_tile, int forced_splits)
+        {
+            GemmPlan p = plan_w8a8_gemm(M, N, K, forced_tile, forced_splits);
+            if (p.tile != GEMM_TILE_SMALL)
+                return p;
+            static const int split_options[] = {1, 2, 3, 4, 6, 8, 12, 16};
+            double best = -1.0;
+            const int planned = p.splits;
+            for (int s : split_options)
+            {
+                if (forced_splits > 0 || s > planned)
+                    break;
+                const long long grid = (long long)ceil_div(M, 64) * ceil_div(N, 256) * s, rounds = (grid + PLAN_CUS - 1) / PLAN_CUS;
+                const double last = (double)(grid - (rounds - 1) * PLAN_CUS) / PLAN_CUS, steps = ceil_div(K / 128, s);
+                const double t = 3.6 * rounds + steps * (0.47 * rounds + 0.64 * (rounds - 1 + last)) +
+                                 (s > 1 ? 2.0 + 0.28 * s + (double)s * M * N * 8.0 / 1e7 : 0.0);
+                if (best < 0.0 || t < best)
+                    best = t, p.splits = s;
+            }
+            p.reduce_pass = p.splits > 1;
+            return p;
+        }
         // a caller's tile_rows / tile_cols as a forced tile of plan_w8a8_gemm (-1: none; -2: 256-row tiles of the
         // plan's own width)
         inline int w8a8_forced_tile(int tile_rows, int tile_cols)

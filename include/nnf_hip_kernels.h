@@ -205,6 +205,10 @@ typedef struct nnf_quant
 /* 1 when nnf_wna16_gemm serves the shape with these parameters (zero_points is not read), else 0. */
 NNF_API int nnf_wna16_supported(int M, int N, int K, const nnf_quant* q);
 NNF_API size_t nnf_wna16_gemm_workspace_bytes(int M, int N, int K, const nnf_quant* q);
+/* At least that: the bytes with which nnf_wna16_gemm runs fastest.  More where the tile kernel behind products without a
+ * specialised one (8-bit weights, K no multiple of 256; above 16 rows) leaves CUs idle and can work on ranges of K instead,
+ * whose fp32 sums it keeps there; given less it runs as many ranges as fit, or one. */
+NNF_API size_t nnf_wna16_gemm_preferred_workspace_bytes(int M, int N, int K, const nnf_quant* q);
 NNF_API int nnf_wna16_gemm(nnf_stream_t stream,
                    const void* A, const void* Wq, const void* scales, void* Y,
                    int M, int N, int K, const nnf_quant* q,

@@ -167,9 +167,11 @@ namespace nnf
 
     // fp16 activations x 4- or 8-bit weights, groups of 32 / 64 / 128, a scalar zero point or one per (row, group)
     // (zero_points: u8 [N, ceil(K/group * bits / 8)], 4-bit ones two to a byte, even group low): wna16_generic.hip
+    // ws (or none): the tile kernel's fp32 sums of ranges of K, as many as fit (workspace::plan_wna16_tile)
     bool wna16_supported(int M, int N, int K, int bits, int group);
     hipError_t launch_wna16_generic(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
-                                    int K, int bits, int group, int zp, const void* zero_points, int num_cu);
+                                    int K, int bits, int group, int zp, const void* zero_points, int num_cu,
+                                    void* ws = nullptr, size_t ws_bytes = 0);
 
     // W8A8: acc != nullptr writes the raw int32 accumulators, otherwise Y = fp16(acc * s_tok * s_ch).
     // partial_ws: w8a8_partial_bytes(...) bytes

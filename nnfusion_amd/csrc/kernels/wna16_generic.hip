@@ -20,6 +20,8 @@
 #include "nnf_device.h"
 #include "nnf_launch.h"
 
+#include "../nnf_workspace.h"
+
 namespace nnf
 {
     namespace
@@ -308,10 +310,15 @@ namespace nnf
     // for every load in flight at the top of the loop.  Tiles are numbered in groups of four tile rows, tile row fastest,
     // and dealt to the eight XCDs in contiguous runs, so that the workgroups in flight together share activations and
     // weights in one L2 (groups of 2, 8 or 16 tile rows measure the same).
-    template <int BITS, int WM, int WN, bool TAIL, int WAVES_M, int WAVES_N>
+    // Ranges of K (blockIdx.y; range_k values each, a multiple of 256, the last range what is left): fp32 sums of a range to
+    // partial[range][M][N], added up by the reduction pass.  (An instantiation of its own: the choice at run time
+    // cost the product of one range 2 %.)  For products whose
+    // tiles leave CUs idle: 249 x 256 x 15232 with 8-bit weights took 80 us on 16 workgroups.
+    template <int BITS, int WM, int WN, bool TAIL, int WAVES_M, int WAVES_N, bool RANGES>
     __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void wna16_tile_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                              const half_t* __restrict__ S, half_t* __restrict__ Y, int M, int N,
-                                                             int K, int tiles_m, int tiles_n, QuantArgs qa)
+                                                             int K_row, int tiles_m, int tiles_n, QuantArgs qa,
+                                                             float* __restrict__ partial, int range_k)
     {
         constexpr int NW = WAVES_M * WAVES_N, THREADS = 64 * NW; // wavefronts: WAVES_M x WAVES_N
         constexpr int TM = 32 * WAVES_M * WM, TN = 32 * WAVES_N * WN; // rows and columns of the output tile
@@ -349,8 +356,21 @@ namespace nnf
             tn = rr / gm;
         }
         const int m0 = tm * TM, n0 = tn * TN;
-        const int G = K >> qa.group_shift;
-        const size_t row_bytes = (size_t)K * BITS / 8;
+        // this workgroup's range of K: the operands from its first value on, K its length (a multiple of 256 values ahead:
+        // whole groups, whole bytes of zero points, 16-byte pieces); rows are K_row values long
+        const int G = K_row >> qa.group_shift;
+        const size_t row_bytes = (size_t)K_row * BITS / 8;
+        int K = K_row;
+        if constexpr (RANGES)
+        {
+            const int k_first = (int)blockIdx.y * range_k;
+            K = min(range_k, K_row - k_first);
+            A += k_first;
+            Wq += (size_t)k_first * BITS / 8;
+            S += k_first >> qa.group_shift;
+            if (qa.zps)
+                qa.zps += ((k_first >> qa.group_shift) * BITS) >> 3;
+        }
         const int steps = (K + KS - 1) / KS;
         const int a_row = tid >> 3, a_k = (tid & 7) * 8;
         // fragments: wavefront (wm, wn) owns rows [32 WM wm, +32 WM) x columns [32 WN wn, +32 WN)
@@ -383,7 +403,7 @@ namespace nnf
             for (int i = 0; i < A_PER; ++i)
             {
                 const int row = min(m0 + a_row + A_ROWS * i, M - 1), k = min(step * KS + a_k, K - 8);
-                r.a[i] = *reinterpret_cast<const uintx4*>(A + (size_t)row * K + k);
+                r.a[i] = *reinterpret_cast<const uintx4*>(A + (size_t)row * K_row + k);
             }
         };
         auto fetch_w = [&](int step_raw, Staged& r) {
@@ -553,16 +573,21 @@ namespace nnf
                 {
                     const int m = m0 + (wm * WM + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
                     if (m < M && n < N)
-                        Y[(size_t)m * N + n] = (half_t)acc[i][j][e];
+                    {
+                        if constexpr (RANGES)
+                            partial[((size_t)blockIdx.y * M + m) * N + n] = acc[i][j][e];
+                        else
+                            Y[(size_t)m * N + n] = (half_t)acc[i][j][e];
+                    }
                 }
             }
     }
 
     namespace
     {
-        template <int BITS, int WM, int WN, bool TAIL, int WAVES_M = 2, int WAVES_N = 2>
+        template <int BITS, int WM, int WN, bool TAIL, int WAVES_M, int WAVES_N, bool RANGES>
         hipError_t launch_wna16_tile_k(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
-                                     const QuantArgs& qa)
+                                     const QuantArgs& qa, float* partial, int range_k)
         {
             constexpr int NW = WAVES_M * WAVES_N;
             constexpr int TM = 32 * WAVES_M * WM, TN = 32 * WAVES_N * WN;
@@ -570,7 +595,7 @@ namespace nnf
             const int tiles_m = (M + TM - 1) / TM, tiles_n = (N + TN - 1) / TN;
             if ((long long)tiles_m * tiles_n > 0x7fffff00ll)
                 return hipErrorInvalidValue;
-            auto kernel = &wna16_tile_kernel<BITS, WM, WN, TAIL, WAVES_M, WAVES_N>;
+            auto kernel = &wna16_tile_kernel<BITS, WM, WN, TAIL, WAVES_M, WAVES_N, RANGES>;
             if (LDS > 64 * 1024)
             {
                 static LdsGrant granted;
@@ -579,8 +604,9 @@ namespace nnf
                     return e;
             }
             const int grid = (tiles_m * tiles_n + 7) / 8 * 8; // whole rounds of the XCDs
-            hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * NW), LDS, stream, (const half_t*)A, (const uint8_t*)Wq,
-                               (const half_t*)S, (half_t*)Y, M, N, K, tiles_m, tiles_n, qa);
+            const int ranges = RANGES ? (K + range_k - 1) / range_k : 1;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)grid, (unsigned)ranges), dim3(64 * NW), LDS, stream, (const half_t*)A,
+                               (const uint8_t*)Wq, (const half_t*)S, (half_t*)Y, M, N, K, tiles_m, tiles_n, qa, partial, range_k);
             return hipGetLastError();
         }
     } // namespace
@@ -590,10 +616,13 @@ namespace nnf
         // (K is a multiple of 32; the kernel walks K in pairs of steps of 64)
         template <int BITS, int WM, int WN, int WAVES_M, int WAVES_N>
         hipError_t launch_wna16_tile(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
-                                     const QuantArgs& qa)
+                                     const QuantArgs& qa, float* partial, int range_k)
         {
-            return K % 128 ? launch_wna16_tile_k<BITS, WM, WN, true, WAVES_M, WAVES_N>(stream, A, Wq, S, Y, M, N, K, qa)
-                           : launch_wna16_tile_k<BITS, WM, WN, false, WAVES_M, WAVES_N>(stream, A, Wq, S, Y, M, N, K, qa);
+            if (partial)
+                return K % 128 ? launch_wna16_tile_k<BITS, WM, WN, true, WAVES_M, WAVES_N, true>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k)
+                               : launch_wna16_tile_k<BITS, WM, WN, false, WAVES_M, WAVES_N, true>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k);
+            return K % 128 ? launch_wna16_tile_k<BITS, WM, WN, true, WAVES_M, WAVES_N, false>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k)
+                           : launch_wna16_tile_k<BITS, WM, WN, false, WAVES_M, WAVES_N, false>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k);
         }
     } // namespace
 
@@ -603,7 +632,7 @@ namespace nnf
     }
 
     hipError_t launch_wna16_generic(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
-                                    int bits, int group, int zp, const void* zero_points, int num_cu)
+                                    int bits, int group, int zp, const void* zero_points, int num_cu, void* ws, size_t ws_bytes)
     {
         if (!wna16_supported(M, N, K, bits, group))
             return hipErrorInvalidValue;
@@ -666,29 +695,36 @@ namespace nnf
                                    (const uint8_t*)Wq, (const half_t*)S, (half_t*)Y, M, N, K, qa);
             return hipGetLastError();
         }
-        // 256 x 256 (eight wavefronts, 2 x 4, of 128 x 64), 256 x 128 (eight, 4 x 2, of 64 x 64), 128 x 128 or 64 x 64
-        // tiles (four wavefronts): the shape with the lowest estimate, in thousandths of the time of one round of
-        // 256 x 256 tiles (one tile per CU).  Measured at K = 8192 and 4096 on 256 CUs: a round of 256 x 128 tiles takes
-        // 0.60 of that, 128 x 128 tiles 0.45 while every tile has a CU to itself and 0.73 per round of two tiles per CU,
-        // 64 x 64 tiles 0.135 + 0.143 per tile and CU (twelve products between 200 and 4096 rows: the estimate picks
-        // the fastest of the four measured shapes in each).
-        const auto rounds = [&](int tm, int tn, int per_cu) {
-            const long long t = (long long)((M + tm - 1) / tm) * ((N + tn - 1) / tn);
-            return (t + (long long)num_cu * per_cu - 1) / ((long long)num_cu * per_cu);
-        };
-        const long long c256 = 1000 * rounds(256, 256, 1), c256n = 600 * rounds(256, 128, 1);
-        const long long c128 = rounds(128, 128, 1) == 1 ? 450 : 730 * rounds(128, 128, 2);
-        const long long c64 = 135 + 143 * rounds(64, 64, 1);
-        if (c256 <= c256n && c256 <= c128 && c256 <= c64)
-            return bits == 4 ? launch_wna16_tile<4, 4, 2, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa)
-                             : launch_wna16_tile<8, 4, 2, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa);
-        if (c256n <= c128 && c256n <= c64)
-            return bits == 4 ? launch_wna16_tile<4, 2, 2, 4, 2>(stream, A, Wq, S, Y, M, N, K, qa)
-                             : launch_wna16_tile<8, 2, 2, 4, 2>(stream, A, Wq, S, Y, M, N, K, qa);
-        if (c128 <= c64)
-            return bits == 4 ? launch_wna16_tile<4, 2, 2, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa)
-                             : launch_wna16_tile<8, 2, 2, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa);
-        return bits == 4 ? launch_wna16_tile<4, 1, 1, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa)
-                         : launch_wna16_tile<8, 1, 1, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa);
+        // 256 x 256 (eight wavefronts, 2 x 4, of 128 x 64), 256 x 128 (eight, 4 x 2, of 64 x 64), 192 x 128 (eight, 2 x 4, of
+        // 96 x 32), 128 x 128 or 64 x 64
+        // tiles (four wavefronts), over as many ranges of K as the plan says and the workspace holds
+        const workspace::Wna16TilePlan plan =
+            workspace::plan_wna16_tile(M, N, K, num_cu, ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 ? ws_bytes : 0);
+        float* partial = plan.ranges > 1 ? (float*)ws : nullptr;
+        hipError_t e;
+        switch (plan.tile)
+        {
+        case 0:
+            e = bits == 4 ? launch_wna16_tile<4, 4, 2, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
+                          : launch_wna16_tile<8, 4, 2, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
+            break;
+        case 1:
+            e = bits == 4 ? launch_wna16_tile<4, 2, 2, 4, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
+                          : launch_wna16_tile<8, 2, 2, 4, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
+            break;
+        case 2:
+            e = bits == 4 ? launch_wna16_tile<4, 2, 2, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
+                          : launch_wna16_tile<8, 2, 2, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
+            break;
+        case 4:
+            e = bits == 4 ? launch_wna16_tile<4, 3, 1, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
+                          : launch_wna16_tile<8, 3, 1, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
+            break;
+        default:
+            e = bits == 4 ? launch_wna16_tile<4, 1, 1, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
+                          : launch_wna16_tile<8, 1, 1, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
+            break;
+        }
+        return e != hipSuccess || !partial ? e : launch_wna16_reduce(stream, partial, plan.ranges, Y, M, N);
     }
 } // namespace nnf

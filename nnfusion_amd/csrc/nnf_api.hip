@@ -263,6 +263,15 @@ size_t nnf_wna16_gemm_workspace_bytes(int M, int N, int K, const nnf_quant* q)
     return nnf_wna16_supported(M, N, K, q) ? nnf::workspace::wna16_gemm(M, N, K, q->bits, q->group) : 0;
 }
 
+size_t nnf_wna16_gemm_preferred_workspace_bytes(int M, int N, int K, const nnf_quant* q)
+{
+    const size_t needed = nnf_wna16_gemm_workspace_bytes(M, N, K, q);
+    if (!q || is_plain_w4a16(q) || !nnf_wna16_supported(M, N, K, q))
+        return needed;
+    const size_t preferred = nnf::workspace::wna16_gemm_preferred(M, N, K, q->bits, q->group);
+    return preferred > needed ? preferred : needed;
+}
+
 int nnf_wna16_gemm(nnf_stream_t stream, const void* A, const void* Wq, const void* scales, void* Y, int M, int N, int K,
                    const nnf_quant* q, void* workspace, size_t workspace_bytes)
 {
@@ -323,7 +332,7 @@ int nnf_wna16_gemm_planned(nnf_stream_t stream, const void* A, const void* Wq, c
                                                  q->zero_point, q->zero_points, workspace, dev.num_cu, choice);
     }
     return (int)nnf::launch_wna16_generic((hipStream_t)stream, A, Wq, scales, Y, M, N, K, q->bits, q->group, q->zero_point,
-                                          q->zero_points, dev.num_cu);
+                                          q->zero_points, dev.num_cu, workspace, workspace_bytes);
 }
 
 // ---- the nodes around a product as calls of their own ------------------------------------------------------------------
@@ -427,7 +436,7 @@ size_t nnf_wna16_gemm_fused_workspace_bytes(int M, int N, int K, const nnf_quant
         return 0;
     if (is_plain_w4a16(q))
         return nnf::workspace::w4a16_gemm_fused(M, N, K, q->group, act);
-    return nnf::workspace::wna16_fused_layout(M, N, K, q->bits, q->group, true, act == NNF_ACT_SILU_GATE, true).total();
+    return nnf::workspace::wna16_fused_layout(M, N, K, q->bits, q->group, true, act == NNF_ACT_SILU_GATE, true, false).total();
 }
 
 int nnf_wna16_gemm_fused(nnf_stream_t stream, const void* A, const void* Wq, const void* scales, void* Y, int M, int N, int K,
@@ -466,7 +475,11 @@ int nnf_wna16_gemm_fused(nnf_stream_t stream, const void* A, const void* Wq, con
     fusion.residual = residual;
     fusion.gate = gate;
     bool taken;
-    st = wna16_fused_rows(s, A, Wq, scales, Y, M, N, K, q, fusion, ws, l.gemm ? ws + l.xn + l.product : nullptr, l.gemm, dev.num_cu, taken);
+    // the product's own: what the workspace holds behind the tensors
+    const size_t tensors = l.xn + l.product;
+    const size_t own_bytes = workspace && workspace_bytes > tensors ? workspace_bytes - tensors : 0;
+    uint8_t* own = own_bytes ? ws + tensors : nullptr;
+    st = wna16_fused_rows(s, A, Wq, scales, Y, M, N, K, q, fusion, ws, own, own_bytes, dev.num_cu, taken);
     if (taken || st != NNF_OK)
         return st;
     if (rms)
@@ -477,7 +490,7 @@ int nnf_wna16_gemm_fused(nnf_stream_t stream, const void* A, const void* Wq, con
         A = ws;
     }
     void* product = l.product ? (void*)(ws + l.xn) : Y;
-    st = nnf_wna16_gemm(stream, A, Wq, scales, product, M, rows, K, q, l.gemm ? ws + l.xn + l.product : nullptr, l.gemm);
+    st = nnf_wna16_gemm(stream, A, Wq, scales, product, M, rows, K, q, own, own_bytes);
     if (st != NNF_OK)
         return st;
     if (gate)
@@ -721,7 +734,7 @@ size_t nnf_fused_mlp_wna16_workspace_bytes(int M, int H, int I, const nnf_quant*
     if (is_plain_w4a16(q_gate_up) && is_plain_w4a16(q_down) && q_gate_up->zero_point == q_down->zero_point)
         return nnf::workspace::fused_mlp_w4a16(M, H, I, 128);
     const int bits = q_gate_up->bits, group = q_gate_up->group;
-    return nnf::workspace::fused_mlp_wna16(M, H, I, bits, group);
+    return nnf::workspace::fused_mlp_wna16(M, H, I, bits, group, false);
 }
 
 int nnf_fused_mlp_wna16(nnf_stream_t stream, const void* x, const void* gamma, float eps, const void* Wgu, const void* Sgu,
@@ -740,7 +753,7 @@ int nnf_fused_mlp_wna16(nnf_stream_t stream, const void* x, const void* gamma, f
     if (H % 8 != 0 || q_gate_up->bits != q_down->bits || q_gate_up->group != q_down->group ||
         !nnf_wna16_supported(M, 2 * I, H, q_gate_up) || !nnf_wna16_supported(M, H, I, q_down))
         return NNF_ERR_UNSUPPORTED_SHAPE;
-    if (!workspace || workspace_bytes < nnf_fused_mlp_wna16_workspace_bytes(M, H, I, q_gate_up, q_down))
+    if (!workspace || workspace_bytes < nnf::workspace::fused_mlp_wna16(M, H, I, q_gate_up->bits, q_gate_up->group))
         return NNF_ERR_WORKSPACE_TOO_SMALL;
     const size_t wide = (size_t)(2 * I > H ? 2 * I : H);
     uint8_t* xn = (uint8_t*)workspace;

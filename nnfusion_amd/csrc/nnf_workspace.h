@@ -6,6 +6,8 @@
 #include <math.h>
 #include <stddef.h>
 
+#include <initializer_list>
+
 namespace nnf
 {
     namespace workspace
@@ -769,6 +771,73 @@ namespace nnf
             return M > 16 && N >= 1 && K >= 256 && !(K & 255) && group_shift >= 5 && group_shift <= 7 &&
                    (size_t)M * K * 2 + 8192 < ((size_t)1 << 32) && (size_t)N * (K >> 1) < ((size_t)1 << 32);
         }
+        // ---- the plain tile kernel (wna16_generic.hip): tile shape and ranges of K ------------------------------------------
+        // One range: the tile shape with the lowest time of a K step of 64 on a busy chip: 256 x 256 (0) 2.0 us a round of
+        // tiles over the CUs, 256 x 128 (1) 1.2, 192 x 128 (4) 0.95, 128 x 128 (2) 0.9 while every tile has a CU to itself and 1.46 per round of
+        // two tiles per CU, 64 x 64 (3) 0.27 + 0.286 per tile and CU (measured at K = 8192 and 4096, 256 CUs; twelve products
+        // between 200 and 4096 rows: it picks the fastest of the four).
+        // Ranges of K: steps are faster while CUs are idle (busy: their share that works; 64 x 64 tiles 0.3 us), every round of
+        // workgroups costs 2.5 us, the reduction pass 3 us, 0.3 a range and its sums at 2.5 TB/s; taken where the estimate is 7 % lower and
+        // ws_bytes hold the sums.  Sixty products of 17 .. 2500 rows, one range -> the plan's: 21 x 512 x 16256 81 -> 16 us,
+        // 249 x 256 x 15232 80 -> 20, 126 x 1472 x 11648 86 -> 25, 1707 x 896 x 15872 156 -> 82, 261 x 3840 x 8320 88 -> 53.
+        struct Wna16TilePlan
+        {
+            int tile = 3, ranges = 1, range_k = 0;
+            size_t bytes = 0; // of fp32 sums [ranges][M][N]
+        };
+        inline Wna16TilePlan plan_wna16_tile(int M, int N, int K, int num_cu, size_t ws_bytes)
+        {
+            static const int rows[] = {256, 256, 128, 64, 192}, cols[] = {256, 128, 128, 64, 128};
+            static const int ranges_tried[] = {2, 3, 4, 6, 8, 12, 16, 24};
+            static const double step_idle[] = {0.9, 0.5, 0.35, 0.3, 0.42}, step_busy[] = {2.0, 1.2, 0.9, 0.44, 0.95};
+            const auto tiles = [&](int tile) { return (long long)ceil_div(M, rows[tile]) * ceil_div(N, cols[tile]); };
+            const auto rounds = [&](long long grid, int per_cu) { return (grid + (long long)num_cu * per_cu - 1) / ((long long)num_cu * per_cu); };
+            const auto step_full = [&](int tile, long long grid) {
+                const long long r = rounds(grid, 1);
+                return tile == 0 ? 2.0 * r : tile == 1 ? 1.2 * r : tile == 4 ? 0.95 * r : tile == 2 ? (r == 1 ? 0.9 : 1.46 * rounds(grid, 2)) : 0.27 + 0.286 * r;
+            };
+            const auto estimate = [&](int tile, int ranges, int range_k) {
+                const long long grid = tiles(tile) * ranges, r = rounds(grid, 1);
+                const double busy = (double)grid / num_cu;
+                // (64 x 64 tiles of one range: up to four a CU at once, no rounds)
+                const bool together = tile == 3 && (r == 1 || ranges == 1);
+                const double step = tile == 3 && together ? (busy <= 2.0 ? 0.30 + 0.14 * busy : 0.27 + 0.286 * busy)
+                                    : r > 1              ? step_full(tile, grid)
+                                                         : step_idle[tile] + busy * (step_busy[tile] - step_idle[tile]);
+                return (together ? 4.5 : 2.0 + 2.5 * r) + step * ceil_div(range_k, 64) +
+                       (ranges > 1 ? 3.0 + 0.3 * ranges + (double)ranges * M * N * sizeof(float) / 2.5e6 : 0.0);
+            };
+            Wna16TilePlan best;
+            best.range_k = K;
+            for (int tile : {2, 4, 1, 0}) // (ties: the larger tile)
+                if (step_full(tile, tiles(tile)) <= step_full(best.tile, tiles(best.tile)))
+                    best.tile = tile;
+            double best_t = 0.93 * estimate(best.tile, 1, K);
+            for (int tile = 0; tile < 5; ++tile)
+                for (int want : ranges_tried)
+                {
+                    // (a range: whole groups and bytes of zero points, at least eight steps)
+                    const int range_k = (K / want + 255) / 256 * 256, ranges = ceil_div(K, range_k);
+                    const size_t bytes = (size_t)ranges * M * N * sizeof(float);
+                    if (range_k < 512 || ranges < 2 || bytes > ws_bytes)
+                        break;
+                    const double t = estimate(tile, ranges, range_k);
+                    if (t < best_t)
+                        best_t = t, best.tile = tile, best.ranges = ranges, best.range_k = range_k, best.bytes = bytes;
+                }
+            return best;
+        }
+        // whether launch_wna16_generic runs a product on that kernel
+        inline bool wna16_on_tile_kernel(int M, int N, int K, int bits, int group_shift, int num_cu)
+        {
+            if (M <= 16)
+                return false;
+            if (bits == 4)
+                return !w4a16_mrows_q_fits(M, N, K, group_shift, true, num_cu);
+            const int block = K == 8192 ? 16 : 32, blocks = ceil_div(M, block);
+            return !w8a16_mrows_q_fits(M, N, K, group_shift, true, num_cu) &&
+                   !(blocks <= (N <= 8192 ? 3 : 2) && w8a16_mrows_q_fits(block, N, K, group_shift, true, num_cu));
+        }
         // nnf_wna16_gemm with parameters other than 4 bits / groups of 128 / scalar zero point, 4-bit weights: [ parked tiles ]
         // on the tile GEMM, [ fp32 sums per range of K ] for 2 .. 16 rows with K above 8192; nothing otherwise
         inline size_t wna16_gemm(int M, int N, int K, int bits, int group, int num_cu = PLAN_CUS)
@@ -785,12 +854,23 @@ namespace nnf
                 return 0;
             return plan_w4a16_sk(M, N, K, false, num_cu).bytes();
         }
+        // ... and what the plain tile kernel can use for ranges of K (it runs without)
+        inline size_t wna16_gemm_preferred(int M, int N, int K, int bits, int group, int num_cu = PLAN_CUS)
+        {
+            const size_t needed = wna16_gemm(M, N, K, bits, group, num_cu);
+            const int gs = group == 32 ? 5 : group == 64 ? 6 : group == 128 ? 7 : 0;
+            if (gs == 0 || (bits != 4 && bits != 8) || (bits == 4 && w4a16_gemm_q_fits(M, N, K, gs)) ||
+                !wna16_on_tile_kernel(M, N, K, bits, gs, num_cu))
+                return needed;
+            return align256(plan_wna16_tile(M, N, K, num_cu, (size_t)64 << 20).bytes);
+        }
         // ---- the fused product / MLP block for block parameters that run the nodes one after the other ----------------------
         inline size_t w4a16_gemm(int M, int N, int K, int, int num_cu = PLAN_CUS);
         // nnf_wna16_gemm's own scratch memory, whichever form the zero point takes
-        inline size_t wna16_gemm_any(int M, int N, int K, int bits, int group, int num_cu = PLAN_CUS)
+        // (needed: without what it can use but runs without)
+        inline size_t wna16_gemm_any(int M, int N, int K, int bits, int group, bool needed, int num_cu = PLAN_CUS)
         {
-            size_t a = wna16_gemm(M, N, K, bits, group, num_cu);
+            size_t a = needed ? wna16_gemm(M, N, K, bits, group, num_cu) : wna16_gemm_preferred(M, N, K, bits, group, num_cu);
             if (bits == 4 && group == 128)
             {
                 const size_t b = w4a16_gemm(M, N, K, group, num_cu);
@@ -805,20 +885,21 @@ namespace nnf
             size_t xn = 0, product = 0, gemm = 0;
             size_t total() const { return xn + product + gemm; }
         };
-        inline QFusedLayout wna16_fused_layout(int M, int N, int K, int bits, int group, bool rms, bool gate, bool through_scratch)
+        inline QFusedLayout wna16_fused_layout(int M, int N, int K, int bits, int group, bool rms, bool gate, bool through_scratch,
+                                               bool needed = true)
         {
             QFusedLayout l;
             const int rows = gate ? 2 * N : N;
             l.xn = rms ? align256((size_t)M * K * 2) : 0;
             l.product = (gate || through_scratch) ? align256((size_t)M * rows * 2) : 0;
-            l.gemm = wna16_gemm_any(M, rows, K, bits, group);
+            l.gemm = wna16_gemm_any(M, rows, K, bits, group, needed);
             return l;
         }
         // nnf_fused_mlp_wna16: [ RMSNorm(x): M x H fp16 ][ gate | up products M x 2I fp16, then the down product M x H fp16 ]
         //                      [ h: M x I fp16 ][ the products' own ]
-        inline size_t fused_mlp_wna16(int M, int H, int I, int bits, int group)
+        inline size_t fused_mlp_wna16(int M, int H, int I, int bits, int group, bool needed = true)
         {
-            const size_t a = wna16_gemm_any(M, 2 * I, H, bits, group), b = wna16_gemm_any(M, H, I, bits, group);
+            const size_t a = wna16_gemm_any(M, 2 * I, H, bits, group, needed), b = wna16_gemm_any(M, H, I, bits, group, needed);
             const size_t wide = (size_t)(2 * I > H ? 2 * I : H);
             return align256((size_t)M * H * 2) + align256((size_t)M * wide * 2) + align256((size_t)M * I * 2) + (a > b ? a : b);
         }

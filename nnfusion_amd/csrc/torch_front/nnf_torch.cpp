@@ -185,7 +185,7 @@ namespace
             require(z.dim() == 2 && z.size(0) == n && z.size(1) == (k / q.group * q.bits + 7) / 8, "shape of the zero points");
         }
         Output y(v[7], m, n, at::kHalf, a);
-        Workspace w(v[8], a, [&] { return nnf_wna16_gemm_workspace_bytes(m, n, k, &q); });
+        Workspace w(v[8], a, [&] { return nnf_wna16_gemm_preferred_workspace_bytes(m, n, k, &q); });
         const SyncPlan plan(v[9], integer(v[10]));
         call(plan.ptr ? "nnf_wna16_gemm_planned" : "nnf_wna16_gemm", nnf_wna16_gemm_planned, stream(), a.data_ptr(), wq.data_ptr(),
              s.data_ptr(), y.data, m, n, k, &q, plan.ptr, w.data, w.bytes);

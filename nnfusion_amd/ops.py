@@ -107,7 +107,7 @@ def wna16_supported(m, n, k, bits, group, zp=8):
 def wna16_workspace_bytes(m, n, k, bits, group, zero_points=None):
     """Bytes of workspace nnf_wna16_gemm wants for this product (0: none)."""
     _, qp = _quant_arg(bits, group, 0, zero_points)
-    return int(_lib.kernels().nnf_wna16_gemm_workspace_bytes(m, n, k, qp))
+    return int(_lib.kernels().nnf_wna16_gemm_preferred_workspace_bytes(m, n, k, qp))
 
 
 def wna16_gemm(a, wq, scales, bits=4, group=128, zp=8, zero_points=None, out=None, workspace=None, sync=None, spin_limit=0):

@@ -316,3 +316,29 @@ def test_fused_rows_with_the_output_over_the_input(gpu):
     ref = ops.wna16_gemm(ops.rms_norm(t[0], gamma), t[1], t[2], group=64, zero_points=t[3])
     ops.wna16_gemm_fused(t[0], t[1], t[2], group=64, zero_points=t[3], rms_gamma=gamma, out=t[0])
     assert torch.equal(t[0], ref)
+
+
+# the plain tile kernel over ranges of K: every tile shape, a last range shorter than the others (and one that is no multiple of
+# 128), ragged M and N; 4-bit zero points that start at any byte of a row
+@pytest.mark.parametrize("m,n,k", [(40, 300, 4000), (100, 257, 15232), (130, 1030, 8192), (249, 256, 11008), (257, 520, 6304), (300, 3000, 5504),
+                                   (600, 448, 14336), (1000, 256, 2080)])
+@pytest.mark.parametrize("bits,group,zp_tensor", [(8, 32, True), (8, 128, False), (4, 32, True), (4, 64, False)])
+def test_tile_kernel_over_ranges_of_k(gpu, m, n, k, bits, group, zp_tensor):
+    """With the workspace it prefers against the oracle, and with any smaller one (fewer ranges, or one)."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    if k % group:
+        pytest.skip("K is not a multiple of the group")
+    a, wq, s, zps = _case(m + n + k + bits, m, n, k, bits, group, zp_tensor)
+    zp = 7 if bits == 4 else 131
+    ref = oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True)
+    t = [torch.from_numpy(x).to(gpu) for x in (a, wq, s)]
+    tz = None if zps is None else torch.from_numpy(zps).to(gpu)
+    want = ops.wna16_workspace_bytes(m, n, k, bits, group, tz)
+    for nbytes in {want, want // 2, 16}:
+        y = ops.wna16_gemm(*t, bits=bits, group=group, zp=zp, zero_points=tz,
+                           workspace=torch.empty(max(16, nbytes), dtype=torch.uint8, device=gpu))
+        torch.cuda.synchronize()
+        _check(y.cpu().numpy(), ref)

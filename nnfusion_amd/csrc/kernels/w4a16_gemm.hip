@@ -352,7 +352,7 @@ namespace nnf
         // activations for the MFMA GEMV kernel -------------------------------------------------------------------
         // (the row-streaming kernels add up the squares of the activations they hold themselves: no pre-pass; the form
         // with a run-time K keeps it)
-        const bool normalised_copy = route.kind == W4A16Route::SKINNY || route.kind == W4A16Route::SKINNY_SPLIT;
+        const bool normalised_copy = route.normalised_copy;
         const bool rstd_in_tile_gemm = rms && route.kind == W4A16Route::TILE && rstd_inside_tile_gemm(route.plan, choice, num_cu);
         const bool rstd_in_kernel = route.kind == W4A16Route::ROWS ||
                                     (route.kind == W4A16Route::MROWS && workspace::w4a16_mrows_fixed_k(M, K)) || rstd_in_tile_gemm;
@@ -375,7 +375,7 @@ namespace nnf
         if (route.kind == W4A16Route::ROWS || route.kind == W4A16Route::MROWS)
         {
             GemvFusion fusion;
-            fusion.gamma = rms_gamma;
+            fusion.gamma = normalised_copy ? nullptr : rms_gamma;
             fusion.rstd = rstd;
             fusion.rms_eps = rms_eps;
             fusion.bias = bias;

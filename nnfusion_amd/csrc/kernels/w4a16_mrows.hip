@@ -1389,10 +1389,12 @@ namespace nnf
             const int r = pos / SLICE, q = (pos % SLICE) >> 4;
             w_off[c] = (uint32_t)r * (uint32_t)ROW_BYTES + (uint32_t)((q ^ swz(r)) << 4);
         }
-        // scales: lane l fetches 4 bytes of row l / SC_LANES, counted from the 4-byte boundary at or below the first
-        // fetched group (never past the end of the row: the last word is fetched twice instead)
-        const uint32_t s_lane_row = (uint32_t)min(lane / SC_LANES, 15) * (uint32_t)(G * 2);
-        const int s_lane_word = lane % SC_LANES;
+        // scales: lane l fetches 4 bytes of row l / SC_LANES, counted from the 4-byte boundary at or below the row's first
+        // fetched group -- with an odd number of groups per row that boundary differs from row to row -- (never past the end
+        // of the matrix, which holds whole words: the last one again instead)
+        const uint32_t s_lane_row = (uint32_t)min(lane / SC_LANES, 15) * (uint32_t)G;
+        const uint32_t s_lane_word = (uint32_t)(lane % SC_LANES);
+        const uint32_t s_last_word = ((uint32_t)((FUSED && gate) ? 2 * N : N) * (uint32_t)G >> 1) - 1u;
 
         auto issue = [&](int tile, int st, int slot) {
             const uint32_t row0 = (uint32_t)row0_of(tile);
@@ -1402,10 +1404,8 @@ namespace nnf
             for (int c = 0; c < GW; ++c)
                 __builtin_amdgcn_global_load_lds((mr_global_ptr_t)(wsrc + w_off[c]),
                                                  (mr_lds_ptr_t)(ring + slot * TILE_BYTES + c * 1024), 16, 0, 0);
-            const int first = (gs * 2) & ~3;                  // byte offset of the first word within the row's scales
-            const int last_word = ((G * 2 - first) >> 2) - 1; // of this window that is still inside the row
-            const uint32_t s_off = s_lane_row + (uint32_t)(first + 4 * min(s_lane_word, last_word));
-            __builtin_amdgcn_global_load_lds((mr_global_ptr_t)(reinterpret_cast<const uint8_t*>(S) + (size_t)row0 * (G * 2) + s_off),
+            const uint32_t s_word = min(((row0 * (uint32_t)G + (uint32_t)gs + s_lane_row) >> 1) + s_lane_word, s_last_word);
+            __builtin_amdgcn_global_load_lds((mr_global_ptr_t)(reinterpret_cast<const uint8_t*>(S) + s_word * 4u),
                                              (mr_lds_ptr_t)(sc_ring + slot * 256), 4, 0, 0);
         };
         issue(0, 0, 0);
@@ -1459,6 +1459,8 @@ namespace nnf
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 __syncthreads();
             }
+            // (RMSNorm: gamma here, rstd from a pass of its own.  The sum of squares and gamma inside the kernel -- spills at eight
+            // groups or two blocks of rows, gamma straight from memory -- took longer than that pass: 7168 / 12 rows 0.7 x)
             if (FUSED && f.gamma)
                 mrows_scale_a<MB, GA>(areg, [&](int g) {
                     return reinterpret_cast<const uint8_t*>(f.gamma) + kq * 64 + (size_t)fetch_group(g / GW) * 256 + (g % GW) * 256;
@@ -1476,7 +1478,7 @@ namespace nnf
                     // the groups of this step that no other wavefront covers: from `fresh` on
                     const int gs = fetch_group(st);
                     const int fresh = own_group(st) - gs;
-                    const int sc_skip = gs & 1;
+                    const int sc_skip = (gs + ((row0_of(it) + col) & G)) & 1; // (an even G: gs & 1)
                     // this step has landed when at most the next step's loads are outstanding
                     __builtin_amdgcn_s_waitcnt(mr_vmcnt(LT));
                     uintx4 wv[GW];
@@ -1726,12 +1728,13 @@ namespace nnf
     hipError_t launch_w4a16_mrows(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                   int K, int zp, int num_cu, const GemvFusion& fusion)
     {
-        if (!w4a16_mrows_supported(M, N, K, num_cu, fusion.gate) || (fusion.gate && (fusion.bias || fusion.residual)))
+        if (!workspace::w4a16_mrows_fits(M, N, K, num_cu, fusion.gate, true) || (fusion.gate && (fusion.bias || fusion.residual)))
             return hipErrorInvalidValue;
         if (!workspace::w4a16_mrows_fixed_k(M, K))
         {
             switch (workspace::w4a16_mrows_step_groups(M, K))
             {
+            case 1: return launch_mrows_any<1, 2>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, fusion);
             case 2: return launch_mrows_any<2, 2>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, fusion);
             case 3: return launch_mrows_any<3, 2>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, fusion);
             default: return launch_mrows_any<4, 2>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, fusion);

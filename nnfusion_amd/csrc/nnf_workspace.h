@@ -637,7 +637,7 @@ namespace nnf
             const int kw = K >> 10, G = K >> 7;
             if (w4a16_mrows_fixed_k(M, K))
                 return (kw & 1) ? kw : kw / 2; // even K / 1024: two steps per tile
-            return G <= 32 ? 2 : G <= 48 ? 3 : 4;
+            return G <= 16 ? 1 : G <= 32 ? 2 : G <= 48 ? 3 : 4;
         }
         // Whether the kernel brings its activations in through LDS as whole lines or straight into the registers.  Straight
         // in, a load touches two lines of every row for 32 bytes each, four times over; through LDS every line is touched
@@ -661,9 +661,12 @@ namespace nnf
             return w4a16_mrows_lds_bytes_gw(w4a16_mrows_step_groups(M, K), M, tiles);
         }
         // N: output columns; gate: from 2 N weight rows (a workgroup walks the gate and the up tile of each output tile)
-        inline bool w4a16_mrows_fits(int M, int N, int K, int num_cu, bool gate = false)
+        // odd_groups: K may be an odd multiple of 128 (the run-time-K form fetches the scales of each row from its own word;
+        // an even number of weight rows, so that the scales are whole words)
+        inline bool w4a16_mrows_fits(int M, int N, int K, int num_cu, bool gate = false, bool odd_groups = false)
         {
-            if (M < 2 || M > 32 || N < 16 || num_cu < 1 || K < 1024 || K > 8192 || (K & 255))
+            if (M < 2 || M > 32 || N < 16 || num_cu < 1 || K < 1024 || K > 8192 || (K & 127) ||
+                ((K & 128) && (!odd_groups || (!gate && (N & 1)) || (size_t)(gate ? 2 : 1) * N * (K >> 7) >= ((size_t)1 << 30))))
                 return false;
             if (!w4a16_mrows_fixed_k(M, K) && M > 16 && K > 4096) // two blocks of rows: at most four groups per wavefront
                 return false;
@@ -966,14 +969,21 @@ namespace nnf
         // least three quarters of the fetched groups count.
         inline bool w4a16_mrows_preferred(int M, int N, int K, int num_cu, bool gate = false)
         {
-            if (!w4a16_mrows_fits(M, N, K, num_cu, gate))
+            if (!w4a16_mrows_fits(M, N, K, num_cu, gate, true))
                 return false;
             if (w4a16_mrows_fixed_k(M, K))
                 return true;
             const int gw = w4a16_mrows_step_groups(M, K);
             if (gw == 4 && M < 8) // K = 6400 .. 7936: N = K = 7168 takes 10.7 us at M = 2 against 9.0 (level from M = 6 on)
                 return false;
-            return 4 * (K >> 7) >= 3 * 16 * gw;
+            // Odd numbers of groups, and up to sixteen of them (one group per wavefront and step), from eight rows on (N = 1152 /
+            // 4096 / 12288 against the MFMA GEMV, 2 / 6 rows: 0.91 - 1.1 x; 12 / 16 rows: K = 3200 1.15 - 1.4 x, 5504 1.6 - 1.75,
+            // 8064 1.2 - 1.45, 1920 1.1 - 1.25).  17 .. 32 rows, whose other kernel is the tile GEMM, whatever part of what is fetched
+            // counts (K = 1664 .. 1920 1.8 - 2.9 x, 3200 1.7 - 2.5, 3968 1.8 - 2.2).
+            if (((K & 128) || gw == 1) && M < 8)
+                return false;
+            // (up to 16 rows K = 1536 on one group per wavefront is level: left where it was)
+            return M > 16 || 4 * (K >> 7) >= (gw == 1 ? 52 : 3 * 16 * gw);
         }
         // ---- W8A8, one activation row: the row-streaming GEMV (w8a8_gemv_rows.hip) ----
         struct Q8RowsPlan
@@ -1037,6 +1047,8 @@ namespace nnf
             // NONE: the kernel family asked for cannot serve the shape
             enum Kind { NONE, ROWS, MROWS, SKINNY, MROWS_SPLIT, SKINNY_SPLIT, TILE } kind = NONE;
             int ksplits = 0;          // *_SPLIT: ranges of K (fp32 partial sums, then the reduction pass)
+            bool normalised_copy = false; // RMSNorm as a pass that writes the normalised activations (MFMA GEMV kernels; an odd
+                                          // number of groups on the row-streaming kernel, which took those products over)
             bool via_scratch = false; // SKINNY: products to scratch first, an element-wise epilogue kernel reads them
             SkPlan plan;              // TILE
             size_t partial_bytes = 0; // partial sums / parked tiles / the products ahead of an element-wise epilogue
@@ -1067,12 +1079,18 @@ namespace nnf
                 const bool two_ranges = !gate && !rms && K == 8192 && M >= 8 && M <= 16 && w4a16_mrows_split(M, n_rows, K, num_cu).ranges > 1;
                 if (rows_family && M > 1 && !two_ranges &&
                     (any ? w4a16_mrows_preferred(M, N, K, num_cu, gate) : w4a16_mrows_fits(M, N, K, num_cu, gate)))
-                    return r.kind = W4A16Route::MROWS, r.rms_bytes = rstd_bytes, r;
+                {
+                    r.kind = W4A16Route::MROWS;
+                    r.normalised_copy = (K & 128) != 0;
+                    r.rms_bytes = r.normalised_copy ? xn_bytes : rstd_bytes;
+                    return r;
+                }
                 // the MFMA GEMV kernel writes plain products: an epilogue that cannot work in place (the [M, 2N] gate | up
                 // pair, a residual that is the output buffer) reads them from scratch memory
                 if (skinny_family && M <= 16 && w4a16_skinny_fits(M, n_rows, K))
                 {
                     r.kind = W4A16Route::SKINNY;
+                    r.normalised_copy = true;
                     r.via_scratch = gate || in_place_residual;
                     r.partial_bytes = r.via_scratch ? align256((size_t)M * n_rows * 2) : 0;
                     r.rms_bytes = xn_bytes;
@@ -1090,6 +1108,7 @@ namespace nnf
                 if (skinny_family && (r.ksplits = w4a16_skinny_ksplits(M, n_rows, K)) > 0)
                 {
                     r.kind = W4A16Route::SKINNY_SPLIT;
+                    r.normalised_copy = true;
                     r.partial_bytes = align256((size_t)r.ksplits * M * n_rows * sizeof(float));
                     r.rms_bytes = xn_bytes;
                     return r;

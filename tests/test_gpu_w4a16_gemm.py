@@ -486,3 +486,43 @@ def test_own_plan_matches_whole_tiles(gpu, m, n, k):
         assert err <= (2e-2 if "act" in parts else 1e-2) * float(ref.pow(2).mean().sqrt()), err
         assert float((one.float() - ref).pow(2).mean().sqrt()) <= 2e-3 * float(ref.pow(2).mean().sqrt())
         assert not sync.any()
+
+
+# the row-streaming kernel with K as a run-time value: an odd number of groups per row (scales of odd rows start in the middle
+# of a word), one to four groups per wavefront and step, one and two blocks of rows, activations straight in and through
+# LDS; fewer tiles than CUs, a last tile moved back by an odd number of rows, several tiles per workgroup
+@pytest.mark.parametrize("m,n,k", [(2, 40, 1664), (16, 1002, 1920), (9, 4110, 1920), (20, 300, 1920), (32, 4110, 3968), (3, 520, 3200), (16, 4110, 3968),
+                                   (6, 4096, 5504), (16, 30, 4992), (8, 1002, 8064), (13, 9000, 6784), (5, 520, 5120), (31, 1000, 3584)])
+def test_run_time_k_with_any_number_of_groups(gpu, m, n, k):
+    """Plain, with bias and residual, with RMSNorm (activations times gamma beyond fp16 among them) and SiLU-gate, against
+    the oracle's product of the same tensors; RMSNorm against the node as a call of its own."""
+    import torch
+
+    from nnfusion_amd import datagen, ops
+
+    a, wq, s = datagen.w4a16_case(m + n + k, m, 2 * n, k)
+    ref = oracle.wna16_gemm(a, wq, s, 4, 128, zp=8, f32_out=True)
+    t = [torch.from_numpy(x).to(gpu) for x in (a, wq, s)]
+    w1, s1 = t[1][:n].contiguous(), t[2][:n].contiguous()
+    rms = float(np.sqrt((ref.astype(np.float64) ** 2).mean()))
+    plain = ops.w4a16_gemm(t[0], w1, s1)
+    assert np.abs(plain.float().cpu().numpy() - ref[:, :n]).max() <= 1e-2 * rms
+    gen = torch.Generator(device="cpu").manual_seed(k)
+    gamma = torch.randn(k, generator=gen).mul(0.1).add(1).half().to(gpu)
+    bias, res = torch.randn(n, generator=gen).half().to(gpu), torch.randn(m, n, generator=gen).half().to(gpu)
+    y = res.clone()
+    ops.w4a16_gemm_fused(t[0], w1, s1, bias=bias, residual=y, out=y)
+    assert torch.equal(y, ops.elementwise("add", ops.elementwise("add", plain, bias), res))
+    x = (t[0] * 12000).clamp(-6e4, 6e4)
+    normed = ops.rms_norm(x, gamma, 1e-5)
+    one = ops.w4a16_gemm_fused(x, w1, s1, rms_gamma=gamma, rms_eps=1e-5)
+    if k % 256:  # (elsewhere gamma alone joins the activations, rstd the sums: another rounding, and other limits)
+        want = ops.w4a16_gemm(normed, w1, s1).float()
+        # (one rounding the other way now and then in the activations, then y's own: 2^-11 of up to five RMS each)
+        assert float((one.float() - want).abs().max()) <= 5e-3 * float(want.pow(2).mean().sqrt())
+    x = x if k % 256 else t[0]
+    p = ops.w4a16_gemm(ops.rms_norm(x, gamma, 1e-5), t[1], t[2]).float()
+    g = p[:, :n]
+    want = g / (1 + torch.exp(-g)) * p[:, n:]
+    y = ops.w4a16_gemm_fused(x, t[1], t[2], rms_gamma=gamma, rms_eps=1e-5, act=1).float()
+    assert float((y - want).abs().max()) <= 2e-2 * float(want.pow(2).mean().sqrt())

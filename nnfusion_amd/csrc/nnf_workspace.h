@@ -630,7 +630,7 @@ namespace nnf
         inline bool w4a16_mrows_fixed_k(int M, int K)
         {
             const int kw = K >> 10;
-            return !(K & 1023) && kw >= 1 && kw <= 8 && kw != 5 && kw != 7 && (M <= 16 || kw <= 4);
+            return !(K & 1023) && kw >= 1 && kw <= 8 && kw != 5 && kw != 7 && (M <= 16 || kw <= 4) && M <= 32;
         }
         inline int w4a16_mrows_step_groups(int M, int K) // GW
         {
@@ -665,7 +665,7 @@ namespace nnf
         // an even number of weight rows, so that the scales are whole words)
         inline bool w4a16_mrows_fits(int M, int N, int K, int num_cu, bool gate = false, bool odd_groups = false)
         {
-            if (M < 2 || M > 32 || N < 16 || num_cu < 1 || K < 1024 || K > 8192 || (K & 127) ||
+            if (M < 2 || M > (odd_groups && K <= 2048 ? 64 : 32) || N < 16 || num_cu < 1 || K < 1024 || K > 8192 || (K & 127) ||
                 ((K & 128) && (!odd_groups || (!gate && (N & 1)) || (size_t)(gate ? 2 : 1) * N * (K >> 7) >= ((size_t)1 << 30))))
                 return false;
             if (!w4a16_mrows_fixed_k(M, K) && M > 16 && K > 4096) // two blocks of rows: at most four groups per wavefront
@@ -982,6 +982,10 @@ namespace nnf
             // counts (K = 1664 .. 1920 1.8 - 2.9 x, 3200 1.7 - 2.5, 3968 1.8 - 2.2).
             if (((K & 128) || gw == 1) && M < 8)
                 return false;
+            // 33 .. 64 rows, up to sixteen groups: four blocks of rows against the tile GEMM, 1152 / 4096 / 12288 / 22016 weight rows: K = 1280
+            // 1.45 / 1.3 / 0.9 - 1.0 / 0.7 x, 1664 .. 2048 1.5 / 1.4 / 1.1 - 1.3 / 0.8 - 1.0; RMSNorm and SiLU-gate 1.5 / 1.5 / 1.2 - 1.4 / 1.0 - 1.3
+            if (M > 32)
+                return gate ? 2 * N <= (K >= 1280 ? 22016 : 12288) : N <= (K >= 1408 ? 12288 : 8192);
             // (up to 16 rows K = 1536 on one group per wavefront is level: left where it was)
             return M > 16 || 4 * (K >> 7) >= (gw == 1 ? 52 : 3 * 16 * gw);
         }
@@ -1047,8 +1051,8 @@ namespace nnf
             // NONE: the kernel family asked for cannot serve the shape
             enum Kind { NONE, ROWS, MROWS, SKINNY, MROWS_SPLIT, SKINNY_SPLIT, TILE } kind = NONE;
             int ksplits = 0;          // *_SPLIT: ranges of K (fp32 partial sums, then the reduction pass)
-            bool normalised_copy = false; // RMSNorm as a pass that writes the normalised activations (MFMA GEMV kernels; an odd
-                                          // number of groups on the row-streaming kernel, which took those products over)
+            bool normalised_copy = false; // RMSNorm as a pass that writes the normalised activations (MFMA GEMV kernels, and what
+                                          // the row-streaming kernel took over from other kernels)
             bool via_scratch = false; // SKINNY: products to scratch first, an element-wise epilogue kernel reads them
             SkPlan plan;              // TILE
             size_t partial_bytes = 0; // partial sums / parked tiles / the products ahead of an element-wise epilogue
@@ -1081,7 +1085,8 @@ namespace nnf
                     (any ? w4a16_mrows_preferred(M, N, K, num_cu, gate) : w4a16_mrows_fits(M, N, K, num_cu, gate)))
                 {
                     r.kind = W4A16Route::MROWS;
-                    r.normalised_copy = (K & 128) != 0;
+                    // (the products that once ran elsewhere: gamma times the activations alone may leave the range of fp16)
+                    r.normalised_copy = !w4a16_mrows_fixed_k(M, K) && ((K & 128) || M > 32 || 4 * (K >> 7) < 3 * 16 * (K <= 4096 ? 2 : 3));
                     r.rms_bytes = r.normalised_copy ? xn_bytes : rstd_bytes;
                     return r;
                 }

@@ -492,7 +492,8 @@ def test_own_plan_matches_whole_tiles(gpu, m, n, k):
 # of a word), one to four groups per wavefront and step, one and two blocks of rows, activations straight in and through
 # LDS; fewer tiles than CUs, a last tile moved back by an odd number of rows, several tiles per workgroup
 @pytest.mark.parametrize("m,n,k", [(2, 40, 1664), (16, 1002, 1920), (9, 4110, 1920), (20, 300, 1920), (32, 4110, 3968), (3, 520, 3200), (16, 4110, 3968),
-                                   (6, 4096, 5504), (16, 30, 4992), (8, 1002, 8064), (13, 9000, 6784), (5, 520, 5120), (31, 1000, 3584)])
+                                   (6, 4096, 5504), (16, 30, 4992), (8, 1002, 8064), (13, 9000, 6784), (5, 520, 5120), (31, 1000, 3584),
+                                   (33, 300, 1152), (64, 4110, 2048), (45, 1000, 1664), (50, 5000, 1280)])
 def test_run_time_k_with_any_number_of_groups(gpu, m, n, k):
     """Plain, with bias and residual, with RMSNorm (activations times gamma beyond fp16 among them) and SiLU-gate, against
     the oracle's product of the same tensors; RMSNorm against the node as a call of its own."""

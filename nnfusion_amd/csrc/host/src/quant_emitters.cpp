@@ -54,7 +54,8 @@ namespace nnfusion
                     if (route.kind != nnf::workspace::W4A16Route::TILE && !split)
                         return "";
                     return declare_sync_words(name, split ? nnf::workspace::mrows_split_sync_bytes(nnf::workspace::PLAN_CUS)
-                                                          : route.plan.sync_bytes(rms));
+                                                          : nnf::workspace::w4a16_launch_plan(route, M, N, K, gate, rms, nnf::workspace::PLAN_CUS)
+                                                                .sync_bytes(rms));
                 }
                 // `name` as an nnf_plan over a persistent, zero-initialised tensor of (at least) `need` bytes; "": none needed
                 std::string declare_sync_words(const std::string& name, size_t need)

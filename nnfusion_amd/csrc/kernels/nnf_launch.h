@@ -9,6 +9,11 @@
 
 namespace nnf
 {
+    namespace workspace
+    {
+        struct W4A16Route;
+    }
+
     // largest dynamic LDS a workgroup may ask for on gfx950 (160 KiB per CU)
     constexpr size_t MAX_LDS_BYTES = 160 * 1024;
 
@@ -135,19 +140,20 @@ namespace nnf
     hipError_t launch_w4a16_skinny_split(hipStream_t stream, const void* A, const void* Wq, const void* S, float* partial,
                                          int M, int N, int K, int zp, int ksplits, int num_cu);
 
-    // Y = epilogue(prologue(A) . W^T) through the kernel that nnf::workspace::route_w4a16 names for the shape, the fused
-    // parts and choice: the RMSNorm prologue and the bias / residual / SiLU-gate epilogues inside the row-streaming
-    // kernels and the tile GEMM, in the reduction pass behind a GEMV kernel over ranges of K, or (MFMA GEMV kernel) as a
-    // pre-pass and an element-wise kernel.  rms_ws / partial_ws: the route's rms_bytes / partial_bytes (null when 0).
     // the tile GEMM for groups of 2^group_shift = 32 / 64 / 128 and a scalar zero point or (zero_points != null) one per
     // (row, group): M > 16, K a multiple of 256; partial_ws: workspace::wna16_gemm bytes (0: not needed)
     bool w4a16_gemm_q_supported(int M, int N, int K, int group_shift);
     hipError_t launch_w4a16_gemm_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                    int K, int group_shift, int zp, const void* zero_points, void* partial_ws, int num_cu,
                                    const LaunchChoice& choice = LaunchChoice());
-    hipError_t launch_w4a16_gemm(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M,
-                                 int N, int K, int zp, const void* rms_gamma, float rms_eps, const void* bias,
-                                 const void* residual, int act, void* rms_ws, void* partial_ws, int num_cu,
+    // Y = epilogue(prologue(A) . W^T) through the kernel that `route` (nnf::workspace::route_w4a16 of the same product, fused
+    // parts and choice: made once, by the entry point that checks the workspace with it) names: the RMSNorm prologue and the
+    // bias / residual / SiLU-gate epilogues inside the row-streaming kernels and the tile GEMM, in the reduction pass behind a
+    // GEMV kernel over ranges of K, or (MFMA GEMV kernel) RMSNorm as a pre-pass, bias and residual inside and SiLU-gate as an
+    // element-wise kernel.  rms_ws / partial_ws: the route's rms_bytes / partial_bytes (null when 0).
+    hipError_t launch_w4a16_gemm(hipStream_t stream, const workspace::W4A16Route& route, const void* A, const void* Wq,
+                                 const void* S, void* Y, int M, int N, int K, int zp, const void* rms_gamma, float rms_eps,
+                                 const void* bias, const void* residual, int act, void* rms_ws, void* partial_ws, int num_cu,
                                  const LaunchChoice& choice = LaunchChoice());
 
     // ---- the nodes around a product as kernels of their own (elementwise.hip, w4a16_gemm.hip) --------------------------

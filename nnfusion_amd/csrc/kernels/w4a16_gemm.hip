@@ -332,8 +332,8 @@ namespace nnf
         }
     } // namespace
 
-    hipError_t launch_w4a16_gemm(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M,
-                                 int N, int K, int zp, const void* rms_gamma, float rms_eps, const void* bias,
+    hipError_t launch_w4a16_gemm(hipStream_t stream, const workspace::W4A16Route& route, const void* A, const void* Wq,
+                                 const void* S, void* Y, int M, int N, int K, int zp, const void* rms_gamma, float rms_eps, const void* bias,
                                  const void* residual, int act, void* rms_ws, void* partial_ws, int num_cu,
                                  const LaunchChoice& choice)
     {
@@ -343,9 +343,6 @@ namespace nnf
         if (gate && (hb || hr))
             return hipErrorInvalidValue;
         const int n_rows = gate ? 2 * N : N; // weight rows
-        const W4A16Route route =
-            workspace::route_w4a16(M, N, K, gate, rms, hr && residual == Y, num_cu, choice.path, choice.tile_rows, choice.k_parts,
-                                   choice.tile_cols, choice.sync_flags ? choice.sync_bytes : 0);
         if (route.kind == W4A16Route::NONE || (route.partial_bytes > 0 && !partial_ws) || (route.rms_bytes > 0 && !rms_ws))
             return hipErrorInvalidValue;
         // ---- RMSNorm pre-pass: rstd[m] for the kernels that multiply the weight in themselves, the normalised
@@ -353,7 +350,11 @@ namespace nnf
         // (the row-streaming kernels add up the squares of the activations they hold themselves: no pre-pass; the form
         // with a run-time K keeps it)
         const bool normalised_copy = route.normalised_copy;
-        const bool rstd_in_tile_gemm = rms && route.kind == W4A16Route::TILE && rstd_inside_tile_gemm(route.plan, choice, num_cu);
+        const workspace::SkPlan plan = route.kind == W4A16Route::TILE
+                                           ? workspace::w4a16_launch_plan(route, M, N, K, gate, rms, num_cu,
+                                                                          choice.sync_flags ? choice.sync_bytes : 0)
+                                           : workspace::SkPlan();
+        const bool rstd_in_tile_gemm = rms && route.kind == W4A16Route::TILE && rstd_inside_tile_gemm(plan, choice, num_cu);
         const bool rstd_in_kernel = route.kind == W4A16Route::ROWS ||
                                     (route.kind == W4A16Route::MROWS && workspace::w4a16_mrows_fixed_k(M, K)) || rstd_in_tile_gemm;
         if (rms && !rstd_in_kernel)
@@ -429,7 +430,6 @@ namespace nnf
             return launch_reduce_any(stream, p, gate, hb, hr);
         }
         // ---- the tile GEMM ------------------------------------------------------------------------------------
-        const workspace::SkPlan& plan = route.plan;
         if ((size_t)M * K * 2 + 8192 >= ((size_t)1 << 32) || (size_t)n_rows * (K >> 1) >= ((size_t)1 << 32))
             return hipErrorInvalidValue; // the kernel addresses its operands with 32-bit byte offsets
         SkGemmParams p;

@@ -197,7 +197,7 @@ namespace
         // what this launch writes on this device
         if (!workspace_ok(route.partial_bytes, workspace, workspace_bytes))
             return NNF_ERR_WORKSPACE_TOO_SMALL;
-        return (int)nnf::launch_w4a16_gemm(s, A, Wq, scales, Y, M, N, K, zp, nullptr, 0.f, nullptr, nullptr, NNF_ACT_NONE,
+        return (int)nnf::launch_w4a16_gemm(s, route, A, Wq, scales, Y, M, N, K, zp, nullptr, 0.f, nullptr, nullptr, NNF_ACT_NONE,
                                            nullptr, workspace, dev.num_cu, choice);
     }
 } // namespace
@@ -242,8 +242,8 @@ int nnf_w4a16_gemm_static_scratch(nnf_stream_t stream, const void* A, const void
     nnf::LaunchChoice choice;
     choice.sync_flags = sync;
     choice.sync_bytes = NNF_SYNC_FLAGS_BYTES;
-    st = w4a16_gemm_checked(stream, A, Wq, scales, Y, M, N, K, group, zp, choice, buffer, STATIC_SCRATCH_BYTES);
-    return st == NNF_ERR_WORKSPACE_TOO_SMALL ? NNF_ERR_STATIC_SCRATCH_LIMIT : st;
+    return (int)nnf::launch_w4a16_gemm((hipStream_t)stream, route, A, Wq, scales, Y, M, N, K, zp, nullptr, 0.f, nullptr, nullptr,
+                                       NNF_ACT_NONE, nullptr, buffer, dev.num_cu, choice);
 }
 
 int nnf_wna16_supported(int M, int N, int K, const nnf_quant* q)
@@ -562,7 +562,7 @@ int nnf_w4a16_gemm_fused_variant(nnf_stream_t stream, const void* A, const void*
     if (!workspace_ok(route.rms_bytes + route.partial_bytes, workspace, workspace_bytes))
         return NNF_ERR_WORKSPACE_TOO_SMALL;
     uint8_t* ws = (uint8_t*)workspace;
-    return (int)nnf::launch_w4a16_gemm((hipStream_t)stream, A, Wq, scales, Y, M, N, K, zp, rms_gamma, rms_eps, bias,
+    return (int)nnf::launch_w4a16_gemm((hipStream_t)stream, route, A, Wq, scales, Y, M, N, K, zp, rms_gamma, rms_eps, bias,
                                        residual, act, route.rms_bytes ? ws : nullptr,
                                        route.partial_bytes ? ws + route.rms_bytes : nullptr, dev.num_cu, choice);
 }
@@ -715,12 +715,12 @@ int nnf_fused_mlp_w4a16_planned(nnf_stream_t stream, const void* x, const void* 
     void* partial = ws + partial_offset;
     // h = SiLU(gate) * up, gate|up = RMSNorm(x) . Wgu^T : one GEMM with the gate and up projections as the two halves
     // of every N tile, the RMSNorm weight and rstd inside it
-    hipError_t e = nnf::launch_w4a16_gemm((hipStream_t)stream, x, Wgu, Sgu, h, M, I, H, zp, gamma, eps, nullptr,
+    hipError_t e = nnf::launch_w4a16_gemm((hipStream_t)stream, route_gu, x, Wgu, Sgu, h, M, I, H, zp, gamma, eps, nullptr,
                                           nullptr, NNF_ACT_SILU_GATE, ws, partial, dev.num_cu, choice_gu);
     if (e != hipSuccess)
         return (int)e;
     // out = h . Wd^T + x
-    e = nnf::launch_w4a16_gemm((hipStream_t)stream, h, Wd, Sd, out, M, H, I, zp, nullptr, 0.f, nullptr, x, NNF_ACT_NONE,
+    e = nnf::launch_w4a16_gemm((hipStream_t)stream, route_d, h, Wd, Sd, out, M, H, I, zp, nullptr, 0.f, nullptr, x, NNF_ACT_NONE,
                                nullptr, partial, dev.num_cu, choice_d);
     return (int)e;
 }

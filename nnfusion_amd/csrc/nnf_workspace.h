@@ -234,18 +234,20 @@ namespace nnf
             if (forced_grid > 0)
                 grid = forced_grid < p.units ? forced_grid : p.units;
             p.grid = (int)grid;
-            bool first_used = false, later_used = false;
-            for (int v = 0; v < p.grid && !later_used; ++v)
+            // Share v is the units [v * units / grid, (v + 1) * units / grid), rounded down.  In lowest terms a share is T / W tiles (W:
+            // grid, T: tiles, over their common factor).  Share boundaries that are not tile boundaries exist unless W = 1 (or a
+            // tile is one unit): then the first segment of some share is a part of a tile.  The first boundary behind a tile's
+            // begin lies G * j / W units from it, j = 0 .. T - 1 all occurring; a share reaches over that begin and stops short of
+            // the tile's end where 1 <= G * j / W < G for some j, and the largest j below W (and T) comes closest to that.  (No
+            // walk over the shares: this is made on the host for every call, and again for every size query; 256 shares took 2 us.)
+            long long common = p.grid, rest = tiles;
+            while (rest)
             {
-                const long long u0 = ((long long)v * p.units) / p.grid, u1 = ((long long)(v + 1) * p.units) / p.grid;
-                if (u1 <= u0)
-                    continue;
-                if (u0 % G != 0 || u1 - u0 < G - u0 % G) // the first segment is not a whole tile
-                    first_used = true;
-                const long long last_tile_begin = ((u1 - 1) / G) * G;
-                if (last_tile_begin > u0 && u1 % G != 0) // a later segment that stops short of its tile's end
-                    later_used = true;
+                const long long r = common % rest;
+                common = rest, rest = r;
             }
+            const long long W = p.grid / common, T = tiles / common;
+            const bool first_used = W > 1 && G > 1, later_used = G * ((W < T ? W : T) - 1) >= W;
             p.slots = later_used ? 2 * p.grid : first_used ? p.grid : 0;
             return p;
         }
@@ -304,7 +306,8 @@ namespace nnf
         // than CUs leaves to a pass of its own.  Never parks more than the even split does: scratch memory sized for that
         // is enough, and is what the *_workspace_bytes queries keep asking for.  sync_bytes: of synchronisation words the caller
         // has (a generated program: what it reserved); tiles that need more are not shared.  0: none, or as many as wanted.
-        inline SkPlan plan_w4a16_tiles(int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = 0)
+        // even: plan_w4a16_sk of the same product.
+        inline SkPlan plan_w4a16_tiles(const SkPlan& even, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes)
         {
             static const SkCost costs[] = {
                 {32, 256, 4.26, 1.70, 0.33, 4.65, 0.46, 2.98, 4.69, 8.0, 2.13, 0.0, 5.5},
@@ -316,7 +319,6 @@ namespace nnf
                 {256, 256, 13.40, 3.67, 2.07, 2.60, 9.29, 1.77, 3.53, 20.8, 0.0, 7.17, 10.7},
             };
             static const int parts_tried[] = {1, 2, 3, 4, 6, 8, 12, 16};
-            const SkPlan even = plan_w4a16_sk(M, N, K, gate, num_cu);
             if (even.grid < 1)
                 return even;
             const int weight_rows = gate ? 2 * N : N, G = even.supersteps;
@@ -329,7 +331,8 @@ namespace nnf
                                       : sk_cost_parts(c, (long long)even.tiles_m * even.tiles_n, G, 1, num_cu);
                 }
             best *= 0.97; // (another plan for a gain the estimates can tell from nothing)
-            int rows = 0, cols = 0, parts = 0;
+            int rows = 0, cols = 0;
+            long long best_grid = 0;
             for (const SkCost& c : costs)
             {
                 // (64 x 256 is the SiLU-gate products' small tile; the others pad M to more than twice itself, or would
@@ -348,10 +351,14 @@ namespace nnf
                         continue;
                     const double t = sk_cost_parts(c, tiles, G, n, num_cu) + (rms && grid > num_cu ? 4.0 : 0.0);
                     if (t < best)
-                        best = t, rows = c.rows, cols = c.cols, parts = n;
+                        best = t, rows = c.rows, cols = c.cols, best_grid = grid;
                 }
             }
-            return parts ? plan_w4a16_sk_with(M, N, K, gate, num_cu, rows, parts, cols) : even;
+            return best_grid ? plan_w4a16_sk(M, N, K, gate, num_cu, rows, best_grid, cols) : even;
+        }
+        inline SkPlan plan_w4a16_tiles(int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = 0)
+        {
+            return plan_w4a16_tiles(plan_w4a16_sk(M, N, K, gate, num_cu), M, N, K, gate, rms, num_cu, sync_bytes);
         }
 
         // ---- plan of the skinny (M <= 16) MFMA GEMV kernel ---------------------------------------------
@@ -1054,17 +1061,17 @@ namespace nnf
             bool normalised_copy = false; // RMSNorm as a pass that writes the normalised activations (MFMA GEMV kernels, and what
                                           // the row-streaming kernel took over from other kernels)
             bool via_scratch = false; // SKINNY: products to scratch first, an element-wise epilogue kernel reads them
-            SkPlan plan;              // TILE
+            SkPlan plan;              // TILE: what the caller fixed, or (own_plan) the even split, in whose scratch memory the launch fits
+            bool own_plan = false;    // TILE: the launch follows plan_w4a16_tiles (w4a16_launch_plan)
             size_t partial_bytes = 0; // partial sums / parked tiles / the products ahead of an element-wise epilogue
             size_t rms_bytes = 0;     // RMSNorm prologue: rstd, fp32 [M] (the kernels multiply the RMSNorm weight in
                                       // themselves), or for the MFMA GEMV kernel the normalised activations, fp16 [M, K]
         };
         // N: output columns (gate: from 2 N weight rows); rms: with the RMSNorm prologue; in_place_residual: the residual
         // is the output buffer itself.  path: 0 the library's order of preference, 2 / 4 one family of GEMV kernels only
-        // (values of nnf_w4a16_variant), 3 the tile GEMM with tile_rows / k_parts (0: its own plan, for sync_bytes of
-        // synchronisation words).
+        // (values of nnf_w4a16_variant), 3 the tile GEMM with tile_rows / k_parts (0: its own plan).
         inline W4A16Route route_w4a16(int M, int N, int K, bool gate, bool rms, bool in_place_residual, int num_cu, int path = 0,
-                                      int tile_rows = 0, int k_parts = 0, int tile_cols = 0, size_t sync_bytes = 0)
+                                      int tile_rows = 0, int k_parts = 0, int tile_cols = 0)
         {
             W4A16Route r;
             if (M <= 0 || N <= 0 || K < 128 || (K & 127) || num_cu < 1)
@@ -1124,11 +1131,18 @@ namespace nnf
             }
             r.kind = W4A16Route::TILE;
             // (the workspace: for the even split, of which the library's own plan never needs more)
-            const SkPlan split = plan_w4a16_sk_with(M, N, K, gate, num_cu, tile_rows, k_parts, tile_cols);
-            r.plan = tile_rows == 0 && k_parts == 0 && tile_cols == 0 ? plan_w4a16_tiles(M, N, K, gate, rms, num_cu, sync_bytes) : split;
-            r.partial_bytes = split.bytes();
+            r.plan = plan_w4a16_sk_with(M, N, K, gate, num_cu, tile_rows, k_parts, tile_cols);
+            r.own_plan = tile_rows == 0 && k_parts == 0 && tile_cols == 0;
+            r.partial_bytes = r.plan.bytes();
             r.rms_bytes = rstd_bytes;
             return r;
+        }
+
+        // the tiles a TILE route's launch runs: the estimates are compared once, there, and not by the size queries and checks.
+        // sync_bytes: of synchronisation words (0: none, or as many as wanted)
+        inline SkPlan w4a16_launch_plan(const W4A16Route& r, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = 0)
+        {
+            return r.own_plan ? plan_w4a16_tiles(r.plan, M, N, K, gate, rms, num_cu, sync_bytes) : r.plan;
         }
 
         inline bool w4a16_variant_fits(int M, int N, int K, int variant, int num_cu)

@@ -13,6 +13,7 @@
 #include "nnfusion/frontend/onnx_import/onnx.hpp"
 
 #include <algorithm>
+#include <chrono>
 
 #include "../../nnfusion_amd/csrc/nnf_workspace.h"
 
@@ -20,6 +21,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <fstream>
+#include <functional>
 #include <iterator>
 
 using namespace nnfusion;
@@ -1335,6 +1337,63 @@ int main(int argc, char** argv)
                 EXPECT(few.slots == 0 || few.sync_bytes() <= words || few.grid == even.grid);
                 const auto r = ws::route_w4a16(m, n, k, gate, false, false, cus, 3);
                 EXPECT(r.partial_bytes == even.bytes());
+            }
+            // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
+            const auto walk_slots = [](const ws::SkPlan& p) {
+                const long long G = p.supersteps;
+                bool first_used = false, later_used = false;
+                for (int v = 0; v < p.grid && !later_used; ++v)
+                {
+                    const long long u0 = ((long long)v * p.units) / p.grid, u1 = ((long long)(v + 1) * p.units) / p.grid;
+                    if (u1 <= u0)
+                        continue;
+                    if (u0 % G != 0 || u1 - u0 < G - u0 % G) // the first segment is not a whole tile
+                        first_used = true;
+                    if (((u1 - 1) / G) * G > u0 && u1 % G != 0) // a later segment that stops short of its tile's end
+                        later_used = true;
+                }
+                return later_used ? 2 * p.grid : first_used ? p.grid : 0;
+            };
+            for (int tiles = 1; tiles <= 24; ++tiles)
+                for (int per_tile = 1; per_tile <= 12; ++per_tile)
+                    for (int grid = 1; grid <= tiles * per_tile; ++grid)
+                    {
+                        const auto p = ws::plan_sk(1, tiles, per_tile, 2, 256, 256, grid);
+                        EXPECT(p.grid == grid && p.slots == walk_slots(p));
+                    }
+            for (int i = 0; i < 4000; ++i)
+            {
+                const int m = 17 + draw(0, 1 << draw(1, 12)), n = draw(1, 1 << draw(1, 14)), k = 128 * draw(1, 1 << draw(0, 7));
+                const int cus = i % 3 == 0 ? draw(1, 304) : 256;
+                const auto p = ws::plan_w4a16_sk_with(m, n, k, draw(0, 2) == 0, cus, 32 << draw(0, 3), draw(0, 64));
+                EXPECT(p.slots == walk_slots(p));
+                const auto e = ws::plan_w4a16_sk(m, n, k, draw(0, 2) == 0, cus);
+                EXPECT(e.slots == walk_slots(e));
+            }
+            // a call plans on the host, ahead of kernels of a few microseconds: a size query or check no more than one walk over 256
+            // shares, the fused query (four routes) no more than four, a launch's choice of tiles one (each the quickest of 40 runs)
+            const auto quickest = [](const std::function<size_t()>& f) {
+                double best = 1e9;
+                volatile size_t sink = 0;
+                for (int run = 0; run < 40; ++run)
+                {
+                    const auto t0 = std::chrono::steady_clock::now();
+                    for (int i = 0; i < 50; ++i)
+                        sink = sink + f();
+                    best = std::min(best, std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+                }
+                return best;
+            };
+            const int planned[][3] = {{45, 4096, 4096}, {100, 4096, 4096}, {256, 4096, 4096}, {1000, 4096, 11008}};
+            const auto walked = ws::plan_sk(1, 64, 16, 2, 256, 256, 256); // (equal parts: walked to the end)
+            const double walk = quickest([&] { return (size_t)walk_slots(walked); });
+            for (const auto& s : planned)
+            {
+                const int m = s[0], n = s[1], k = s[2];
+                EXPECT(quickest([&] { return ws::w4a16_gemm(m, n, k, 128); }) <= walk);
+                EXPECT(quickest([&] { return ws::w4a16_gemm_fused(m, n, k, 128, 0); }) <= 4 * walk);
+                const auto r = ws::route_w4a16(m, n, k, false, false, false, 256);
+                EXPECT(quickest([&] { return (size_t)ws::w4a16_launch_plan(r, m, n, k, false, false, 256).grid; }) <= walk);
             }
         }
     });

@@ -554,8 +554,8 @@ int nnf_w4a16_gemm_fused_variant(nnf_stream_t stream, const void* A, const void*
     if (st != NNF_OK)
         return st;
     const nnf::workspace::W4A16Route route =
-        nnf::workspace::route_w4a16(M, N, K, act == NNF_ACT_SILU_GATE, rms_gamma != nullptr, residual == Y, dev.num_cu,
-                                    choice.path, choice.tile_rows, choice.k_parts, choice.tile_cols);
+        nnf::workspace::route_w4a16_within(workspace ? workspace_bytes : 0, M, N, K, act == NNF_ACT_SILU_GATE, rms_gamma != nullptr,
+                                           residual == Y, dev.num_cu, choice.path, choice.tile_rows, choice.k_parts, choice.tile_cols);
     if (route.kind == nnf::workspace::W4A16Route::NONE)
         return NNF_ERR_UNSUPPORTED_SHAPE;
     // [ RMSNorm scratch ][ what this launch parks, on this device ]
@@ -699,28 +699,25 @@ int nnf_fused_mlp_w4a16_planned(nnf_stream_t stream, const void* x, const void* 
         return st;
     // workspace = [ rstd of the first product ][ h: M x I fp16 ][ what either launch parks, on this device ] (the down
     // projection's residual is x: in place when the caller passes out == x)
-    const nnf::workspace::W4A16Route route_gu = nnf::workspace::route_w4a16(
-        M, I, H, true, true, false, dev.num_cu, choice_gu.path, choice_gu.tile_rows, choice_gu.k_parts, choice_gu.tile_cols);
-    const nnf::workspace::W4A16Route route_d = nnf::workspace::route_w4a16(
-        M, H, I, false, false, out == x, dev.num_cu, choice_d.path, choice_d.tile_rows, choice_d.k_parts, choice_d.tile_cols);
-    if (route_gu.kind == nnf::workspace::W4A16Route::NONE || route_d.kind == nnf::workspace::W4A16Route::NONE)
+    const nnf::workspace::FusedMlpRoutes routes = nnf::workspace::fused_mlp_routes(
+        M, H, I, out == x, dev.num_cu, workspace_bytes,
+        {choice_gu.path, choice_gu.tile_rows, choice_gu.k_parts, choice_gu.tile_cols},
+        {choice_d.path, choice_d.tile_rows, choice_d.k_parts, choice_d.tile_cols});
+    if (routes.gate_up.kind == nnf::workspace::W4A16Route::NONE || routes.down.kind == nnf::workspace::W4A16Route::NONE)
         return NNF_ERR_UNSUPPORTED_SHAPE;
-    const size_t h_offset = route_gu.rms_bytes;
-    const size_t partial_offset = h_offset + nnf::workspace::align256((size_t)M * I * 2);
-    const size_t parked = route_gu.partial_bytes > route_d.partial_bytes ? route_gu.partial_bytes : route_d.partial_bytes;
-    if (!workspace || workspace_bytes < partial_offset + parked)
+    if (!workspace || workspace_bytes < routes.total)
         return NNF_ERR_WORKSPACE_TOO_SMALL;
     uint8_t* ws = (uint8_t*)workspace;
-    void* h = ws + h_offset;
-    void* partial = ws + partial_offset;
+    void* h = ws + routes.h_offset;
+    void* partial = ws + routes.partial_offset;
     // h = SiLU(gate) * up, gate|up = RMSNorm(x) . Wgu^T : one GEMM with the gate and up projections as the two halves
     // of every N tile, the RMSNorm weight and rstd inside it
-    hipError_t e = nnf::launch_w4a16_gemm((hipStream_t)stream, route_gu, x, Wgu, Sgu, h, M, I, H, zp, gamma, eps, nullptr,
+    hipError_t e = nnf::launch_w4a16_gemm((hipStream_t)stream, routes.gate_up, x, Wgu, Sgu, h, M, I, H, zp, gamma, eps, nullptr,
                                           nullptr, NNF_ACT_SILU_GATE, ws, partial, dev.num_cu, choice_gu);
     if (e != hipSuccess)
         return (int)e;
     // out = h . Wd^T + x
-    e = nnf::launch_w4a16_gemm((hipStream_t)stream, route_d, h, Wd, Sd, out, M, H, I, zp, nullptr, 0.f, nullptr, x, NNF_ACT_NONE,
+    e = nnf::launch_w4a16_gemm((hipStream_t)stream, routes.down, h, Wd, Sd, out, M, H, I, zp, nullptr, 0.f, nullptr, x, NNF_ACT_NONE,
                                nullptr, partial, dev.num_cu, choice_d);
     return (int)e;
 }

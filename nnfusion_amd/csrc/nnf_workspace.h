@@ -5,6 +5,7 @@
 
 #include <math.h>
 #include <stddef.h>
+#include <stdint.h>
 
 #include <initializer_list>
 
@@ -1070,8 +1071,10 @@ namespace nnf
         // N: output columns (gate: from 2 N weight rows); rms: with the RMSNorm prologue; in_place_residual: the residual
         // is the output buffer itself.  path: 0 the library's order of preference, 2 / 4 one family of GEMV kernels only
         // (values of nnf_w4a16_variant), 3 the tile GEMM with tile_rows / k_parts (0: its own plan).
+        // room_for_copy = false: the caller's scratch memory does not hold the normalised activations of the products that the
+        // row-streaming kernel took over from others: they run where they ran (see route_w4a16_within).
         inline W4A16Route route_w4a16(int M, int N, int K, bool gate, bool rms, bool in_place_residual, int num_cu, int path = 0,
-                                      int tile_rows = 0, int k_parts = 0, int tile_cols = 0)
+                                      int tile_rows = 0, int k_parts = 0, int tile_cols = 0, bool room_for_copy = true)
         {
             W4A16Route r;
             if (M <= 0 || N <= 0 || K < 128 || (K & 127) || num_cu < 1)
@@ -1088,12 +1091,13 @@ namespace nnf
                 // (K = 8192 at 8 .. 16 rows: over two ranges of K, see w4a16_mrows_split -- not with SiLU-gate, whose two halves
                 // the reduction would have to pair, nor with RMSNorm, which the single launch folds in without a pre-pass)
                 const bool two_ranges = !gate && !rms && K == 8192 && M >= 8 && M <= 16 && w4a16_mrows_split(M, n_rows, K, num_cu).ranges > 1;
-                if (rows_family && M > 1 && !two_ranges &&
+                // (the products that once ran elsewhere: gamma times the activations alone may leave the range of fp16)
+                const bool taken_over = rms && !w4a16_mrows_fixed_k(M, K) && ((K & 128) || M > 32 || 4 * (K >> 7) < 3 * 16 * (K <= 4096 ? 2 : 3));
+                if (rows_family && M > 1 && !two_ranges && !(any && taken_over && !room_for_copy) &&
                     (any ? w4a16_mrows_preferred(M, N, K, num_cu, gate) : w4a16_mrows_fits(M, N, K, num_cu, gate)))
                 {
                     r.kind = W4A16Route::MROWS;
-                    // (the products that once ran elsewhere: gamma times the activations alone may leave the range of fp16)
-                    r.normalised_copy = !w4a16_mrows_fixed_k(M, K) && ((K & 128) || M > 32 || 4 * (K >> 7) < 3 * 16 * (K <= 4096 ? 2 : 3));
+                    r.normalised_copy = taken_over && room_for_copy;
                     r.rms_bytes = r.normalised_copy ? xn_bytes : rstd_bytes;
                     return r;
                 }
@@ -1138,6 +1142,19 @@ namespace nnf
             return r;
         }
 
+        // The route of a call that brings `bytes` of scratch memory.  What the size queries ask for covers the normalised activations
+        // (M x K x 2 bytes) of the products that the row-streaming kernel took over, most of them from the tile GEMM, which asks for
+        // rstd [M] and its parked tiles.  A caller that sized its scratch memory for those -- a generated program carries the
+        // byte count as a literal -- keeps the kernel it had.
+        inline W4A16Route route_w4a16_within(size_t bytes, int M, int N, int K, bool gate, bool rms, bool in_place_residual, int num_cu,
+                                             int path = 0, int tile_rows = 0, int k_parts = 0, int tile_cols = 0)
+        {
+            const W4A16Route r = route_w4a16(M, N, K, gate, rms, in_place_residual, num_cu, path, tile_rows, k_parts, tile_cols);
+            if (r.kind != W4A16Route::MROWS || !r.normalised_copy || r.rms_bytes + r.partial_bytes <= bytes)
+                return r;
+            return route_w4a16(M, N, K, gate, rms, in_place_residual, num_cu, path, tile_rows, k_parts, tile_cols, false);
+        }
+
         // the tiles a TILE route's launch runs: the estimates are compared once, there, and not by the size queries and checks.
         // sync_bytes: of synchronisation words (0: none, or as many as wanted)
         inline SkPlan w4a16_launch_plan(const W4A16Route& r, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = 0)
@@ -1174,25 +1191,42 @@ namespace nnf
                 }
             return most;
         }
-        // nnf_fused_mlp_w4a16: [ RMSNorm scratch of the first product ][ h: M x I fp16 ][ partial sums of either product ]
-        inline size_t fused_mlp_h_offset(int M, int H, int I, int num_cu = PLAN_CUS)
+        // nnf_fused_mlp_w4a16: [ RMSNorm scratch of the first product ][ h: M x I fp16 ][ partial sums of either product ].
+        // Of either product what a caller may fix (path: 0, or 3 with a plan's tiles); the down projection's residual is x, in
+        // place where the caller passes it as the output too.  bytes: of scratch memory at hand (see route_w4a16_within)
+        struct W4A16Choice
         {
-            return route_w4a16(M, I, H, true, true, false, num_cu).rms_bytes;
-        }
-        inline size_t fused_mlp_partial_offset(int M, int H, int I, int num_cu = PLAN_CUS)
+            int path = 0, tile_rows = 0, k_parts = 0, tile_cols = 0;
+        };
+        struct FusedMlpRoutes
         {
-            return fused_mlp_h_offset(M, H, I, num_cu) + align256((size_t)M * I * 2);
+            W4A16Route gate_up, down;
+            size_t h_offset = 0, partial_offset = 0, total = 0;
+        };
+        inline FusedMlpRoutes fused_mlp_routes(int M, int H, int I, bool in_place, int num_cu, size_t bytes = SIZE_MAX,
+                                               const W4A16Choice& gate_up = W4A16Choice(), const W4A16Choice& down = W4A16Choice())
+        {
+            FusedMlpRoutes f;
+            f.down = route_w4a16(M, H, I, false, false, in_place, num_cu, down.path, down.tile_rows, down.k_parts, down.tile_cols);
+            for (int room_for_copy = 1; room_for_copy >= 0; --room_for_copy)
+            {
+                f.gate_up = route_w4a16(M, I, H, true, true, false, num_cu, gate_up.path, gate_up.tile_rows, gate_up.k_parts,
+                                        gate_up.tile_cols, room_for_copy != 0);
+                f.h_offset = f.gate_up.rms_bytes;
+                f.partial_offset = f.h_offset + align256((size_t)M * I * 2);
+                f.total = f.partial_offset +
+                          (f.gate_up.partial_bytes > f.down.partial_bytes ? f.gate_up.partial_bytes : f.down.partial_bytes);
+                if (f.total <= bytes || f.gate_up.kind != W4A16Route::MROWS || !f.gate_up.normalised_copy)
+                    break;
+            }
+            return f;
         }
         inline size_t fused_mlp_w4a16(int M, int H, int I, int, int num_cu = PLAN_CUS)
         {
             if (M <= 0 || I <= 0 || H < 128 || I < 128)
                 return 0;
-            const size_t a = route_w4a16(M, I, H, true, true, false, num_cu).partial_bytes;
-            // (the second product's residual x may be the output buffer itself)
-            const size_t b = route_w4a16(M, H, I, false, false, false, num_cu).partial_bytes;
-            const size_t c = route_w4a16(M, H, I, false, false, true, num_cu).partial_bytes;
-            const size_t bc = b > c ? b : c;
-            return fused_mlp_partial_offset(M, H, I, num_cu) + (a > bc ? a : bc);
+            const size_t a = fused_mlp_routes(M, H, I, false, num_cu).total, b = fused_mlp_routes(M, H, I, true, num_cu).total;
+            return a > b ? a : b;
         }
     } // namespace workspace
 } // namespace nnf

@@ -1246,6 +1246,43 @@ int main(int argc, char** argv)
             EXPECT(ws::route_w4a16(4, 4096, 11008, false, false, true, 256).kind == ws::W4A16Route::SKINNY &&
                    ws::route_w4a16(4, 4096, 11008, false, false, true, 256).partial_bytes == (size_t)4 * 4096 * 2 &&
                    ws::route_w4a16(4, 4096, 11008, false, false, false, 256).partial_bytes == 0);
+            // what the row-streaming kernel took over from the tile GEMM asks for the normalised activations; scratch memory sized for the
+            // tile GEMM (rstd and its parked tiles) is still accepted, and the product runs there
+            const size_t blocks[][4] = {{64, 2048, 6400, 13926656}, {48, 1024, 2304, 2580736}, {32, 3968, 17664, 3670272}};
+            for (const auto& b : blocks)
+            {
+                const int m = (int)b[0], h = (int)b[1], i = (int)b[2];
+                const auto roomy = ws::fused_mlp_routes(m, h, i, true, 256), tight = ws::fused_mlp_routes(m, h, i, true, 256, b[3]);
+                EXPECT(roomy.gate_up.kind == ws::W4A16Route::MROWS && roomy.gate_up.normalised_copy && roomy.total > b[3]);
+                EXPECT(tight.gate_up.kind == ws::W4A16Route::TILE && tight.total <= b[3] && ws::fused_mlp_w4a16(m, h, i, 128) == roomy.total);
+                EXPECT(tight.partial_offset == tight.h_offset + ws::align256((size_t)m * i * 2) && tight.h_offset == tight.gate_up.rms_bytes);
+                EXPECT(ws::fused_mlp_routes(m, h, i, true, 256, roomy.total).gate_up.kind == ws::W4A16Route::MROWS);
+            }
+            int refused_before = 0;
+            for (int m = 2; m <= 64; m += m < 18 ? 3 : 7)
+                for (int n : {40, 126, 1152, 4096, 9216, 12288})
+                    for (int k = 1024; k <= 4096; k += 128)
+                        for (int gate = 0; gate < 2; ++gate)
+                            for (int path : {0, 4})
+                            {
+                                const auto r = ws::route_w4a16(m, n, k, gate != 0, true, false, 256, path);
+                                if (r.kind != ws::W4A16Route::MROWS || !r.normalised_copy)
+                                    continue;
+                                // without the copy: rstd alone on the kernel that was asked for by name, else the MFMA GEMV up to 16 rows where it
+                                // takes the product (it writes the copy too), else the tile GEMM
+                                auto old = ws::route_w4a16(m, n, k, gate != 0, true, false, 256, 2);
+                                if (old.kind == ws::W4A16Route::NONE)
+                                    old = ws::route_w4a16(m, n, k, gate != 0, true, false, 256, 3);
+                                const size_t was = path == 4 ? ws::align256((size_t)m * 4) : old.rms_bytes + old.partial_bytes;
+                                if (was >= r.rms_bytes + r.partial_bytes)
+                                    continue;
+                                ++refused_before;
+                                const auto t = ws::route_w4a16_within(was, m, n, k, gate != 0, true, false, 256, path);
+                                EXPECT(t.kind == (path == 4 ? ws::W4A16Route::MROWS : old.kind) && t.rms_bytes + t.partial_bytes <= was &&
+                                       (path != 4 || !t.normalised_copy));
+                                EXPECT(ws::route_w4a16_within(r.rms_bytes, m, n, k, gate != 0, true, false, 256, path).normalised_copy);
+                            }
+            EXPECT(refused_before > 100);
             // one family of kernels only: the MFMA GEMV kernel reads normalised activations and leaves gate | up in scratch
             {
                 const auto r = ws::route_w4a16(8, 11008, 4096, true, true, false, 256, 2);

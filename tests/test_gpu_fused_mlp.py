@@ -93,3 +93,23 @@ def test_mlp_workspace_contract(gpu):
     with pytest.raises(ops.NnfError) as e:
         ops.fused_mlp_w4a16(*tens, workspace=small)
     assert e.value.status == -3
+
+
+# bytes a block needs with its gate | up product on the tile GEMM: less than with it on the row-streaming kernel
+@pytest.mark.parametrize("m,h,i,need", [(64, 2048, 6400, 13926656), (48, 1024, 2304, 2580736), (32, 3968, 17664, 3670272)])
+def test_mlp_in_scratch_memory_sized_for_the_tile_gemm(gpu, m, h, i, need):
+    import torch
+
+    from nnfusion_amd import _lib, ops
+
+    assert _lib.kernels().nnf_fused_mlp_w4a16_workspace_bytes(m, h, i, 128) > need
+    tens = _t(gpu, *datagen.mlp_case(3, m, h, i))
+    want = ops.fused_mlp_w4a16(*tens).float()
+    sync = ops.sync_flags(gpu)
+    for words in (None, sync):
+        buf = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=gpu)
+        x = tens[0].clone()
+        got = ops.fused_mlp_w4a16(x, *tens[1:], out=x, workspace=buf[:need], sync=words).float()
+        # (another kernel: gamma and the scales rounded into fp16 weights there; the block's own tolerance)
+        assert float((got - want).abs().max()) <= 1e-2 * float(want.pow(2).mean().sqrt())
+        assert bool((buf[need:] == 0x5A).all()) and not sync.any()

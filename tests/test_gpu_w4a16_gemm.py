@@ -527,3 +527,39 @@ def test_run_time_k_with_any_number_of_groups(gpu, m, n, k):
     want = g / (1 + torch.exp(-g)) * p[:, n:]
     y = ops.w4a16_gemm_fused(x, t[1], t[2], rms_gamma=gamma, rms_eps=1e-5, act=1).float()
     assert float((y - want).abs().max()) <= 2e-2 * float(want.pow(2).mean().sqrt())
+
+
+# shapes whose RMSNorm form on the row-streaming kernel writes M x K normalised activations to scratch memory: 33 .. 64 rows, K no
+# multiple of 256, 17 .. 32 rows; few weight rows, so that the tile GEMM needs less
+@pytest.mark.parametrize("m,n,k", [(50, 107, 1536), (64, 23, 2048), (58, 109, 1792), (32, 126, 3200), (31, 16, 3712), (27, 33, 1280)])
+def test_scratch_memory_sized_for_the_tile_gemm_is_accepted(gpu, m, n, k):
+    """A program that sized its scratch memory for the tile GEMM (rstd and the parked tiles, a literal in generated code)
+    is served there: same results, nothing written beyond; without room for that either the call is refused."""
+    import torch
+
+    from nnfusion_amd import _lib, ops
+
+    a, wq, s = datagen.w4a16_case(m + n, m, n, k)
+    gamma = datagen.normal_f16(5, datagen.S_GAMMA, (k,), 1.0, 0.1)
+    res = datagen.normal_f16(5, datagen.S_RES, (m, n))
+    ta, tw, ts, tg, tr = _t(gpu, a, wq, s, gamma, res)
+    lib = _lib.kernels()
+    sync = ops.sync_flags(gpu)
+    parked = lib.nnf_w4a16_gemm_variant_workspace_bytes(m, n, k, 128, ops.VARIANTS["gemm_mfma"], None)
+    need = 256 + parked
+    assert need < m * k * 2  # (what the row-streaming kernel asks for)
+    ref = oracle.add_f16(oracle.w4a16_gemm(oracle.rmsnorm_f16(a, gamma, 1e-6), wq, s), res)
+    for words in (None, sync):
+        buf = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=gpu)
+        y = ops.w4a16_gemm_fused(ta, tw, ts, rms_gamma=tg, rms_eps=1e-6, residual=tr, workspace=buf[:need], sync=words)
+        _check(y.cpu().numpy(), ref)
+        assert bool((buf[need:] == 0x5A).all()) and not sync.any()
+        if parked:
+            with pytest.raises(ops.NnfError) as e:
+                ops.w4a16_gemm_fused(ta, tw, ts, rms_gamma=tg, rms_eps=1e-6, residual=tr, workspace=buf[:need - 16], sync=words)
+            assert e.value.status == -3
+    # the same kernel by name, given rstd alone
+    if k % 256 == 0 and m <= 32:
+        y = ops.w4a16_gemm_fused(ta, tw, ts, rms_gamma=tg, rms_eps=1e-6, residual=tr, workspace=buf[:256], variant="gemv_rows")
+        _check(y.cpu().numpy(), ref)
+        assert bool((buf[need:] == 0x5A).all())

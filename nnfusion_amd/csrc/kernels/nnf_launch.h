@@ -16,6 +16,8 @@ namespace nnf
 
     // largest dynamic LDS a workgroup may ask for on gfx950 (160 KiB per CU)
     constexpr size_t MAX_LDS_BYTES = 160 * 1024;
+    // workgroups of a grid in y
+    constexpr int MAX_GRID_Y = 65535;
 
     // Lifts a kernel's dynamic-LDS limit to `bytes`, once per (kernel, device): `granted` is a static of the calling
     // template instantiation (one per kernel).  Racing first calls at worst set the attribute twice.

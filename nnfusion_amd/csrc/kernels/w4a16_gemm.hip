@@ -286,10 +286,19 @@ namespace nnf
         hipError_t launch_reduce(hipStream_t stream, const GemmParams& p)
         {
             const int quads = (p.N + 3) >> 2;
-            hipLaunchKernelGGL((splitk_reduce_kernel<GATE, BIAS, RESID>), dim3((unsigned)((quads + 255) / 256), (unsigned)p.M), dim3(256), 0,
-                               stream, (const float*)p.partial, p.splits, p.M, p.N, p.ld_partial, p.bias, p.residual, p.Y,
-                               p.ldy, p.rstd);
-            return hipGetLastError();
+            // (a launch for every 65535 rows: what a grid is limited to in y)
+            for (int m0 = 0; m0 < p.M; m0 += MAX_GRID_Y)
+            {
+                const size_t at = (size_t)m0 * p.ldy;
+                hipLaunchKernelGGL((splitk_reduce_kernel<GATE, BIAS, RESID>),
+                                   dim3((unsigned)((quads + 255) / 256), (unsigned)std::min(p.M - m0, MAX_GRID_Y)), dim3(256), 0, stream,
+                                   (const float*)p.partial + (size_t)m0 * p.ld_partial, p.splits, p.M, p.N, p.ld_partial, p.bias,
+                                   RESID ? p.residual + at : nullptr, p.Y + at, p.ldy, p.rstd ? p.rstd + m0 : nullptr);
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess)
+                    return e;
+            }
+            return hipSuccess;
         }
 
         hipError_t launch_reduce_any(hipStream_t stream, const GemmParams& p, bool gate, bool hb, bool hr)
@@ -488,7 +497,7 @@ namespace nnf
                 bits |= reinterpret_cast<uintptr_t>(p);
             return (bits & 15) == 0;
         }
-        dim3 row_grid(int M, int N, bool vec) { return dim3((unsigned)((N + (vec ? 2047 : 255)) / (vec ? 2048 : 256)), (unsigned)std::min(M, 65535)); }
+        dim3 row_grid(int M, int N, bool vec) { return dim3((unsigned)((N + (vec ? 2047 : 255)) / (vec ? 2048 : 256)), (unsigned)std::min(M, MAX_GRID_Y)); }
     } // namespace
     hipError_t launch_silu_gate(hipStream_t stream, const void* T, void* Y, int M, int N)
     {

@@ -17,6 +17,8 @@
 
 #include "../nnf_workspace.h"
 
+#include <algorithm>
+
 namespace nnf
 {
     struct Q8GemmParams
@@ -589,9 +591,21 @@ namespace nnf
             if (e != hipSuccess)
                 return e;
             const int quads = (p.N + 3) >> 2;
-            hipLaunchKernelGGL((w8a8_splitk_reduce_kernel<RAW>), dim3((unsigned)((quads + 255) / 256), (unsigned)p.M), dim3(256), 0,
-                               stream, p);
-            return hipGetLastError();
+            // (a launch for every 65535 rows: what a grid is limited to in y; p.M stays the distance between the ranges' sums)
+            Q8GemmParams rows = p;
+            for (int m0 = 0; m0 < p.M && e == hipSuccess; m0 += MAX_GRID_Y)
+            {
+                const size_t at = (size_t)m0 * p.N;
+                rows.partial = p.partial + at;
+                if (RAW)
+                    rows.acc = p.acc + at;
+                else
+                    rows.s_tok = p.s_tok + m0, rows.Y = p.Y + at;
+                hipLaunchKernelGGL((w8a8_splitk_reduce_kernel<RAW>),
+                                   dim3((unsigned)((quads + 255) / 256), (unsigned)std::min(p.M - m0, MAX_GRID_Y)), dim3(256), 0, stream, rows);
+                e = hipGetLastError();
+            }
+            return e;
         }
     } // namespace
 

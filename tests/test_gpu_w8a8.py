@@ -132,3 +132,21 @@ def test_full_size_sampled(gpu, m):
     assert np.array_equal(acc[:, cols], oracle.w8a8_acc(a, w[cols]))
     wsum = w.astype(np.int64).sum(axis=0)
     assert np.array_equal(acc.astype(np.int64).sum(axis=1), a.astype(np.int64) @ wsum)
+
+
+def test_reduction_pass_over_more_rows_than_a_grid_has(gpu):
+    """Two ranges of K asked for: the pass that adds them up above 65535 rows (what other launches limit a grid to in y)."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    m, n, k = 65537, 20, 512
+    a, s_tok, w, s_ch = datagen.w8a8_case(0, m, n, k)
+    ta, tw, tst, tsc = _t(gpu, a, w, s_tok, s_ch)
+    kw = {"variant": "gemm_mfma", "plan": (256, 2, 128)}
+    acc = ops.w8a8_gemm_acc(ta, tw, **kw).cpu().numpy()
+    y = ops.w8a8_gemm(ta, tst, tw, tsc, **kw).cpu().numpy()
+    torch.cuda.synchronize()
+    ref = oracle.w8a8_acc(a, w)
+    assert np.array_equal(acc, ref)
+    assert np.array_equal(y.view(np.uint16), oracle.w8a8_epilogue(ref, s_tok, s_ch).view(np.uint16))

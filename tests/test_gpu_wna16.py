@@ -342,3 +342,21 @@ def test_tile_kernel_over_ranges_of_k(gpu, m, n, k, bits, group, zp_tensor):
                            workspace=torch.empty(max(16, nbytes), dtype=torch.uint8, device=gpu))
         torch.cuda.synchronize()
         _check(y.cpu().numpy(), ref)
+
+
+def test_reduction_pass_over_more_rows_than_a_grid_has(gpu):
+    """A tall, narrow product whose plan takes two ranges of K: the pass that adds them up, above 65535 rows (what other
+    launches limit a grid to in y)."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    m, n, k, group = 65600, 100, 8192, 128
+    assert ops.wna16_workspace_bytes(m, n, k, 8, group) >= 2 * m * n * 4
+    gen = torch.Generator(device=gpu).manual_seed(m)
+    a = torch.randn((m, k), generator=gen, device=gpu, dtype=torch.float16)
+    _, wq, s, _ = _case(17, 1, n, k, 8, group, False)
+    y = ops.wna16_gemm(a, torch.from_numpy(wq).to(gpu), torch.from_numpy(s).to(gpu), bits=8, group=group, zp=128)
+    rows = [0, 1, 64, 4095, 65533, 65534, 65535, 65536, m - 1]
+    _check(y[rows].cpu().numpy(), oracle.wna16_gemm(a[rows].cpu().numpy(), wq, s, 8, group, zp=128, f32_out=True))
+    torch.cuda.synchronize()

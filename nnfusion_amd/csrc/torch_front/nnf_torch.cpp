@@ -254,26 +254,29 @@ namespace
         return y.release();
     }
 
-    // (a, s_tok, w, s_ch, out, workspace, sync); s_tok and s_ch None: the raw int32 accumulators
-    PyObject* w8a8_gemm(Args v)
+    // the raw int32 accumulators (no scales) or the fp16 product
+    PyObject* w8a8(const Tensor& a, const Tensor& b, const Tensor* s_tok, const Tensor* s_ch, PyObject* out, PyObject* workspace, PyObject* sync)
     {
-        const Tensor &a = tensor(v[0]), &b = tensor(v[2]);
         matrix(a), matrix(b);
         const int m = (int)a.size(0), k = (int)a.size(1), n = (int)b.size(0);
-        const bool raw = v[1] == Py_None;
+        const bool raw = !s_tok;
         require(a.scalar_type() == at::kChar && b.scalar_type() == at::kChar, "int8 operands");
         if (!raw)
-            require(tensor(v[1]).scalar_type() == at::kFloat && tensor(v[3]).scalar_type() == at::kFloat, "fp32 scales");
-        Output y(v[4], m, n, raw ? at::kInt : at::kHalf, a);
-        const SyncPlan plan(v[6]);
-        Workspace w(v[5], a, [&] {
+            require(s_tok->scalar_type() == at::kFloat && s_ch->scalar_type() == at::kFloat, "fp32 scales");
+        Output y(out, m, n, raw ? at::kInt : at::kHalf, a);
+        const SyncPlan plan(sync);
+        Workspace w(workspace, a, [&] {
             return plan.ptr ? nnf_w8a8_gemm_variant_workspace_bytes(m, n, k, NNF_W8A8_AUTO, plan.ptr) : nnf_w8a8_gemm_workspace_bytes(m, n, k);
         });
         call(plan.ptr ? "nnf_w8a8_gemm_variant" : raw ? "nnf_w8a8_gemm_acc" : "nnf_w8a8_gemm", nnf_w8a8_gemm_variant, stream(),
-             a.data_ptr(), address(v[1]), b.data_ptr(), address(v[3]), raw ? nullptr : y.data, raw ? y.data : nullptr, m, n, k,
-             NNF_W8A8_AUTO, plan.ptr, w.data, w.bytes);
+             a.data_ptr(), raw ? nullptr : s_tok->data_ptr(), b.data_ptr(), raw ? nullptr : s_ch->data_ptr(), raw ? nullptr : y.data,
+             raw ? y.data : nullptr, m, n, k, NNF_W8A8_AUTO, plan.ptr, w.data, w.bytes);
         return y.release();
     }
+    // (a, s_tok, w, s_ch, out, workspace, sync)
+    PyObject* w8a8_gemm(Args v) { return w8a8(tensor(v[0]), tensor(v[2]), &tensor(v[1]), &tensor(v[3]), v[4], v[5], v[6]); }
+    // (a, w, out, workspace, sync)
+    PyObject* w8a8_gemm_acc(Args v) { return w8a8(tensor(v[0]), tensor(v[1]), nullptr, nullptr, v[2], v[3], v[4]); }
 
     // (op, a, b, out)
     PyObject* elementwise(Args v)
@@ -368,8 +371,9 @@ namespace
 
 #define NNF_ENTRY(f, n) {#f, (PyCFunction)(void (*)(void))entry<f, n>, METH_FASTCALL, nullptr}
     PyMethodDef methods[] = {NNF_ENTRY(w4a16_gemm, 7),       NNF_ENTRY(wna16_gemm, 11),      NNF_ENTRY(w4a16_gemm_fused, 14), NNF_ENTRY(fused_mlp_w4a16, 13),
-                             NNF_ENTRY(wna16_gemm_fused, 14), NNF_ENTRY(fused_mlp_wna16, 14), NNF_ENTRY(w8a8_gemm, 7),         NNF_ENTRY(elementwise, 4),
-                             NNF_ENTRY(rms_norm, 4),          NNF_ENTRY(dequantize, 7),       {"set_error", set_error, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
+                             NNF_ENTRY(wna16_gemm_fused, 14), NNF_ENTRY(fused_mlp_wna16, 14), NNF_ENTRY(w8a8_gemm, 7),         NNF_ENTRY(w8a8_gemm_acc, 5),
+                             NNF_ENTRY(elementwise, 4),       NNF_ENTRY(rms_norm, 4),         NNF_ENTRY(dequantize, 7),        {"set_error", set_error, METH_O, nullptr},
+                             {nullptr, nullptr, 0, nullptr}};
     PyModuleDef module = {PyModuleDef_HEAD_INIT, "nnf_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 } // namespace
 

@@ -205,7 +205,7 @@ def w8a8_gemm(a, s_tok, w, s_ch, out=None, workspace=None, variant="auto", plan=
 def w8a8_gemm_acc(a, w, out=None, workspace=None, variant="auto", plan=None, sync=None):
     """acc i32 [M,N] = A . W^T, exact."""
     if variant == "auto" and plan is None:
-        return _native.w8a8_gemm(a, None, w, None, out, workspace, sync)
+        return _native.w8a8_gemm_acc(a, w, out, workspace, sync)
     assert a.dtype == torch.int8 and w.dtype == torch.int8
     if out is None:
         out = torch.empty((a.shape[0], w.shape[0]), dtype=torch.int32, device=a.device)

@@ -150,3 +150,30 @@ def test_reduction_pass_over_more_rows_than_a_grid_has(gpu):
     ref = oracle.w8a8_acc(a, w)
     assert np.array_equal(acc, ref)
     assert np.array_equal(y.view(np.uint16), oracle.w8a8_epilogue(ref, s_tok, s_ch).view(np.uint16))
+
+
+@pytest.mark.parametrize("m,n,k", [
+    # one range of K, the 64-row tile writes its results itself: every remainder of rows and of columns by 2, 4, 8 (stores of 16
+    # bytes and single ones), a single column, fewer columns than a wavefront's part of the tile, the shortest K
+    (33, 12801, 128), (64, 12802, 256), (47, 12804, 512), (58, 12680, 512), (63, 12672, 384), (34, 1, 128), (40, 31, 128), (64, 257, 256),
+    # ranges of K and the reduction pass: whole quads of columns, 1 .. 3 left over, fewer than four
+    (33, 1001, 8192), (64, 1002, 8192), (45, 1003, 4096), (50, 1000, 8192), (64, 3, 8192), (60, 4, 8192)])
+def test_64_row_tiles_at_ragged_columns(gpu, m, n, k):
+    """Bit exact, nothing written beyond the outputs or the workspace the query asks for."""
+    import torch
+
+    from nnfusion_amd import _lib, ops
+
+    a, s_tok, w, s_ch = datagen.w8a8_case(2, m, n, k)
+    ta, tw, tst, tsc = _t(gpu, a, w, s_tok, s_ch)
+    need = _lib.kernels().nnf_w8a8_gemm_workspace_bytes(m, n, k)
+    ref = oracle.w8a8_acc(a, w)
+    y_ref = oracle.w8a8_epilogue(ref, s_tok, s_ch)
+    for dtype, run, want in ((torch.int32, lambda **kw: ops.w8a8_gemm_acc(ta, tw, **kw), ref),
+                             (torch.float16, lambda **kw: ops.w8a8_gemm(ta, tst, tw, tsc, **kw), y_ref)):
+        out = torch.full((m * n + 512,), 77, dtype=dtype, device=gpu)
+        ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=gpu)
+        run(out=out, workspace=ws[:need])
+        torch.cuda.synchronize()
+        assert np.array_equal(out[:m * n].cpu().numpy().reshape(m, n), want)
+        assert bool((out[m * n:] == 77).all()) and bool((ws[need:] == 0x5A).all())

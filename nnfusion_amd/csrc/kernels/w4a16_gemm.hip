@@ -539,7 +539,7 @@ namespace nnf
     {
         if (!w4a16_gemm_q_supported(M, N, K, group_shift))
             return hipErrorInvalidValue;
-        const workspace::SkPlan plan = workspace::plan_w4a16_tiles(M, N, K, false, false, num_cu, choice.sync_flags ? choice.sync_bytes : 0);
+        const workspace::SkPlan plan = workspace::plan_w4a16_tiles_q(M, N, K, num_cu, choice.sync_flags ? choice.sync_bytes : 0);
         if (plan.slots && !partial_ws)
             return hipErrorInvalidValue;
         SkGemmParams p;

@@ -306,9 +306,10 @@ namespace nnf
         // N: output columns (gate: from 2 N weight rows).  rms: with the RMSNorm prologue, which a launch of more workgroups
         // than CUs leaves to a pass of its own.  Never parks more than the even split does: scratch memory sized for that
         // is enough, and is what the *_workspace_bytes queries keep asking for.  sync_bytes: of synchronisation words the caller
-        // has (a generated program: what it reserved); tiles that need more are not shared.  0: none, or as many as wanted.
-        // even: plan_w4a16_sk of the same product.
-        inline SkPlan plan_w4a16_tiles(const SkPlan& even, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes)
+        // has (a generated program: what it reserved); tiles that need more are not shared.  0: none, parts are added up by a second launch.
+        // even: plan_w4a16_sk of the same product.  blocks: other block parameters than groups of 128 and a scalar zero point
+        inline SkPlan plan_w4a16_tiles(const SkPlan& even, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes,
+                                       bool blocks = false)
         {
             static const SkCost costs[] = {
                 {32, 256, 4.26, 1.70, 0.33, 4.65, 0.46, 2.98, 4.69, 8.0, 2.13, 0.0, 5.5},
@@ -323,13 +324,30 @@ namespace nnf
             if (even.grid < 1)
                 return even;
             const int weight_rows = gate ? 2 * N : N, G = even.supersteps;
+            const long long even_tiles = (long long)even.tiles_m * even.tiles_n;
+            // Where the fit is off by more than its spread, and a plan picked by it was slower than the even split (even split, the plan
+            // without and with the correction timed in turns, the 160 of 60 000 drawn products whose plan they change):
+            // whole 128 x 128 tiles on more than half of the CUs over K from 8192 on take 12 % longer than fitted (700 x 4096 x 8192
+            // 67.4 us in the even split, 74.5 on them; 315 x 8192 x 11008 97.8 / 106.9): parts of larger tiles instead are 8 % faster in
+            // the geometric mean, 2 % with the weights in the last-level cache; without synchronisation words (a second launch adds
+            // the parts up) 3 % faster and 2 % slower: left on whole tiles, than which the even split is 10 % slower there;
+            // SiLU-gate products of four supersteps on few whole tiles 3 % (1300 rows, 128 outputs, K = 896: halves of tiles 14.9 us in two
+            // launches, whole ones 17.1): 3.5 % and 12 %.
+            // (neither with other block parameters: 1000 x 4096 x 11008, groups of 32 with zero points, is faster on whole tiles)
+            const auto estimate = [&](const SkCost& c, long long tiles, int parts) {
+                const double t = sk_cost_parts(c, tiles, G, parts, num_cu);
+                if (blocks || parts > 1 || c.rows != 128)
+                    return t;
+                return c.cols == 128 ? (sync_bytes && G >= 32 && tiles <= num_cu && 2 * tiles > num_cu ? 1.12 * t : t)
+                                     : (gate && G == 4 && 16 * tiles <= num_cu ? 1.03 * t : t);
+            };
             double best = -1.0;
             for (const SkCost& c : costs)
                 if (c.rows == even.tile_rows && c.cols == even.tile_weight_rows)
                 {
                     const double busy = (double)even.grid / num_cu, longest = (double)((even.units + even.grid - 1) / even.grid);
                     best = even.slots ? c.even_start + longest * (c.even_step + busy * c.even_step_load) + busy * c.even_load
-                                      : sk_cost_parts(c, (long long)even.tiles_m * even.tiles_n, G, 1, num_cu);
+                                      : estimate(c, even_tiles, 1);
                 }
             best *= 0.97; // (another plan for a gain the estimates can tell from nothing)
             int rows = 0, cols = 0;
@@ -342,6 +360,11 @@ namespace nnf
                     (c.rows == 64 && M > 256) || (c.rows == 128 && M > 2048))
                     continue;
                 const long long tiles = (long long)ceil_div(M, c.rows) * ceil_div(weight_rows, c.cols);
+                // (whole tiles that a workgroup walks one behind the other start their pipeline once, where the estimate has a start a
+                // round: K = 384 .. 1280 on one round of 256 x 256 tiles is 7 - 18 % slower, 1000 x 16384 x 512 27.0 / 29.2 us;
+                // level at 2048, 7 % faster above 4096; level for SiLU-gate)
+                if (!gate && c.rows == 256 && c.cols == 256 && even.slots == 0 && even_tiles > num_cu && tiles <= num_cu && G >= 2 && G <= 6)
+                    continue;
                 for (int n : parts_tried)
                 {
                     const long long grid = tiles * n;
@@ -350,16 +373,21 @@ namespace nnf
                     if (n > 1 && ((size_t)grid * c.rows * c.cols * sizeof(float) > even.bytes() ||
                                   (sync_bytes && (size_t)(tiles + 1) * 2 * sizeof(unsigned) > sync_bytes)))
                         continue;
-                    const double t = sk_cost_parts(c, tiles, G, n, num_cu) + (rms && grid > num_cu ? 4.0 : 0.0);
+                    const double t = estimate(c, tiles, n) + (rms && grid > num_cu ? 4.0 : 0.0);
                     if (t < best)
                         best = t, rows = c.rows, cols = c.cols, best_grid = grid;
                 }
             }
             return best_grid ? plan_w4a16_sk(M, N, K, gate, num_cu, rows, best_grid, cols) : even;
         }
-        inline SkPlan plan_w4a16_tiles(int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = 0)
+        inline SkPlan plan_w4a16_tiles(int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = SIZE_MAX)
         {
             return plan_w4a16_tiles(plan_w4a16_sk(M, N, K, gate, num_cu), M, N, K, gate, rms, num_cu, sync_bytes);
+        }
+        // ... of the plain product with other block parameters
+        inline SkPlan plan_w4a16_tiles_q(int M, int N, int K, int num_cu, size_t sync_bytes = SIZE_MAX)
+        {
+            return plan_w4a16_tiles(plan_w4a16_sk(M, N, K, false, num_cu), M, N, K, false, false, num_cu, sync_bytes, true);
         }
 
         // ---- plan of the skinny (M <= 16) MFMA GEMV kernel ---------------------------------------------
@@ -1156,8 +1184,8 @@ namespace nnf
         }
 
         // the tiles a TILE route's launch runs: the estimates are compared once, there, and not by the size queries and checks.
-        // sync_bytes: of synchronisation words (0: none, or as many as wanted)
-        inline SkPlan w4a16_launch_plan(const W4A16Route& r, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = 0)
+        // sync_bytes: of synchronisation words (0: none)
+        inline SkPlan w4a16_launch_plan(const W4A16Route& r, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = SIZE_MAX)
         {
             return r.own_plan ? plan_w4a16_tiles(r.plan, M, N, K, gate, rms, num_cu, sync_bytes) : r.plan;
         }

@@ -1375,6 +1375,19 @@ int main(int argc, char** argv)
                 const auto r = ws::route_w4a16(m, n, k, gate, false, false, cus, 3);
                 EXPECT(r.partial_bytes == even.bytes());
             }
+            // products on which the estimates alone picked plans slower than the even split: whole 128 x 128 tiles on most CUs over a long
+            // K, one round of 256 x 256 tiles over a short one, few whole SiLU-gate tiles of four supersteps
+            const auto whole_128 = [](const ws::SkPlan& p) { return p.tile_rows == 128 && p.tile_weight_rows == 128 && p.slots == 0; };
+            const int long_k[][3] = {{700, 4096, 8192}, {315, 8192, 11008}, {160, 16384, 11008}, {450, 8192, 11008}, {512, 8192, 11008}};
+            for (const auto& s : long_k)
+                EXPECT(!whole_128(ws::plan_w4a16_tiles(s[0], s[1], s[2], false, false, 256)));
+            EXPECT(whole_128(ws::plan_w4a16_tiles_q(1000, 4096, 11008, 256)) && ws::plan_w4a16_tiles_q(1000, 16384, 512, 256).tile_weight_rows == 128 &&
+                   whole_128(ws::plan_w4a16_tiles(700, 4096, 8192, false, false, 256, 0)));
+            EXPECT(whole_128(ws::plan_w4a16_tiles(1000, 4096, 5504, false, false, 256)) && whole_128(ws::plan_w4a16_tiles(896, 4096, 7168, false, false, 256)));
+            for (int k : {384, 512, 896, 1280})
+                EXPECT(ws::plan_w4a16_tiles(1000, 16384, k, false, false, 256).tile_weight_rows == 128);
+            EXPECT(ws::plan_w4a16_tiles(1000, 16384, 7168, false, false, 256).tile_weight_rows == 256);
+            EXPECT(ws::plan_w4a16_tiles(1300, 128, 896, true, false, 256).slots > 0 && ws::plan_w4a16_tiles(1300, 128, 640, true, false, 256).slots == 0);
             // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
             const auto walk_slots = [](const ws::SkPlan& p) {
                 const long long G = p.supersteps;

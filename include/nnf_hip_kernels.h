@@ -73,10 +73,10 @@ NNF_API const char* nnf_status_string(int status);
  * fp16 x int4 (group-scaled) GEMM / GEMV:  Y[M,N] = A[M,K] . ((Wq - zp) * scales)^T
  * Replaces the cublasHgemm / cublasSgemm call of cuda::Dot (cuda_gpu/kernels/dot.cpp:128-205,
  * :271-363) for a weight-quantized Dot node with transpose_B = true.  By shape: M = 1 the row-streaming
- * GEMV kernel; 2 <= M <= 32 (40 for long K) the row-streaming MFMA kernel, over ranges of K (partial sums in
+ * GEMV kernel; 2 <= M <= 32 (40 up to K = 4096, 64 up to K = 2048) the row-streaming MFMA kernel, over ranges of K (partial sums in
  * `workspace`, then a reduction pass) where the activations exceed one workgroup's registers; other M <= 16
- * shapes the MFMA GEMV kernel over K ranges; everything else the MFMA tile GEMM, whose work is split evenly
- * over the CUs (tiles shared by several workgroups are summed through `workspace` by a second launch).
+ * shapes the MFMA GEMV kernel over K ranges; everything else the MFMA tile GEMM, whose tiles are cut into equal parts of K or
+ * whose work is split evenly over the CUs (tiles shared by several workgroups are summed through `workspace` by a second launch).
  * ------------------------------------------------------------------------------------------- */
 NNF_API size_t nnf_w4a16_gemm_workspace_bytes(int M, int N, int K, int group);
 
@@ -137,7 +137,7 @@ typedef struct nnf_plan
                       256 weight rows of a full tile); ignored elsewhere */
     /* fp16 x int4 products in one launch (any variant that ends up on one of the kernels below; ignored by every other
      * kernel; W8A8: see the last sentence).
-     * The work of the GEMM is split evenly over the CUs, so most output tiles of a mid-sized product are shared by
+     * Where a product has fewer tiles than the device has CUs, most of its output tiles are shared by
      * several workgroups.  Without sync_flags their parts are added up by a second launch.  With sync_flags the
      * workgroups count themselves in at their tiles there, and each adds up and finishes its share of a tile's rows
      * once all that hold a part have arrived -- same summation order, bit-identical results, one launch less.
@@ -194,7 +194,8 @@ NNF_API int nnf_w4a16_gemm_variant(nnf_stream_t stream,
  * 4-byte aligned.  The ranges of K and the tile GEMM want nnf_wna16_gemm_workspace_bytes of workspace; called with
  * less (or NULL) the product runs on a plain kernel instead, at about half the rate.
  * Everything else runs on plain kernels that need no workspace: a row-per-wavefront GEMV for M = 1, an MFMA kernel
- * with the operands fetched straight into registers for 2 <= M <= 16, MFMA tiles through LDS above. */
+ * with the operands fetched straight into registers for 2 <= M <= 16, MFMA tiles through LDS above (over ranges of K where
+ * nnf_wna16_gemm_preferred_workspace_bytes says so and the caller brings them). */
 typedef struct nnf_quant
 {
     int bits;                /* 4 or 8 */
@@ -259,13 +260,15 @@ enum nnf_activation
 };
 
 /* Same GEMM with prologue / epilogue in one call.  They run inside the kernel that serves the shape: the
- * row-streaming kernels (M = 1; M <= 32) and the tile GEMM multiply gamma in on the way in, rstd[m] and the
+ * row-streaming kernels (M = 1; M <= 64) and the tile GEMM multiply gamma in on the way in, rstd[m] and the
  * epilogue at their end.  The row-streaming kernels add up the squares of the activations they hold themselves
  * (K a multiple of 1024 up to 8192; M = 1: any K they take): one launch in all; the tile GEMM and the other
  * forms take rstd from a small pre-pass over A (fp32 [M] in `workspace`); a GEMV kernel over ranges of K
- * leaves rstd and the epilogue to its reduction pass.  Only the MFMA GEMV kernel (M <= 16 with K not a
- * multiple of 256) reads normalised activations written to `workspace` by a pre-pass and leaves its
- * products to one element-wise kernel.
+ * leaves rstd and the epilogue to its reduction pass.  The MFMA GEMV kernel (M <= 16, other K) and the
+ * row-streaming kernel where K is an odd multiple of 128, up to sixteen groups or above 32 rows read normalised
+ * activations written to `workspace` by a pre-pass (M x K x 2 bytes; a workspace that holds rstd and the tile
+ * GEMM's parked tiles but not these is accepted too, and the product runs there).  The MFMA GEMV kernel adds bias
+ * and residual itself and leaves SiLU-gate to one element-wise kernel.
  *   rms_gamma != NULL : A is replaced by RMSNorm(A) = A * rsqrt(mean_k(A^2) + rms_eps) * gamma[k]
  *                       (rsqrt(x + eps) as in LayerNorm, cuda_gpu/cuda_langunit.cpp:618)
  *   bias      != NULL : fp16 [N], added to every row (MatMulAdd precedent,

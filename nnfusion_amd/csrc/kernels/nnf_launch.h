@@ -90,10 +90,10 @@ namespace nnf
                                         int K, int group_shift, int zp, const void* zero_points, int num_cu, int bits = 4);
     bool w4a16_gemv_rows_q_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu, int bits = 4);
 
-    // 2 <= M <= 16, K = 1024 / 2048 / 4096 / 8192: weights streamed through LDS rings, activations in registers
+    // a few rows (workspace::w4a16_mrows_fits): weights streamed through LDS rings, activations in registers
     // (N: outputs; gate / fusion.gate: from 2 N weight rows)
     // the same kernel for groups of 2^group_shift = 32 / 64 / 128 and a scalar zero point or (zero_points != null) one per
-    // (row, group): 2 <= M <= 16, K = 2048 / 4096 / 8192.  fusion: gamma (normalised inside the kernel; no rstd), bias /
+    // (row, group): 2 <= M <= 16 (32 up to K = 4096), K = 2048 / 4096 / 8192.  fusion: gamma (normalised inside the kernel; no rstd), bias /
     // residual or gate, where w4a16_mrows_q_fused_supported
     hipError_t launch_w4a16_mrows_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                     int K, int group_shift, int zp, const void* zero_points, int num_cu,

@@ -1,15 +1,15 @@
 // fp16 x int4 (g128) products beyond one activation row: the dispatcher between the row-streaming /
-// split-K GEMV kernels (up to 40 rows) and the tile GEMM (w4a16_gemm_sk.h), the RMSNorm pre-passes, the
-// reduction pass behind the GEMV kernels that run over ranges of K, and their element-wise epilogues.
+// split-K GEMV kernels (up to 64 rows) and the tile GEMM (w4a16_gemm_sk.h), the RMSNorm pre-passes, the
+// reduction pass behind the GEMV kernels that run over ranges of K, and the element-wise kernels.
 //
 //   Y[M,N] = epilogue( prologue(A)[M,K] . ((Wq - zp) * S)^T )
 //
-//   * prologue: RMSNorm.  The tile GEMM folds it in (a pre-pass computes rstd[m] only); the GEMV
-//     kernels read normalised activations, fp16(x * rsqrt(mean(x^2) + eps) * gamma) written to scratch
-//     memory by a pre-pass (the tensor of the unfused graph, at most 40 rows of it).
+//   * prologue: RMSNorm.  The tile GEMM and the row-streaming kernels fold it in (rstd[m] computed by the launch or a
+//     pre-pass); the MFMA GEMV kernel, and the row-streaming kernel on the products it took over from others, read
+//     normalised activations, fp16(x * rsqrt(mean(x^2) + eps) * gamma) written to scratch memory by a pre-pass (the tensor of
+//     the unfused graph, at most 64 rows of it).
 //   * epilogues: bias, residual add, SiLU(gate) * up with the gate and up projections as two halves of
-//     the N tile -- in the tile GEMM's epilogue, in the reduction pass, or in an element-wise kernel
-//     behind a GEMV kernel.
+//     the N tile -- inside the kernels, in the reduction pass, or (SiLU-gate of the MFMA GEMV) in an element-wise kernel.
 //   * tile height and split of the work over the CUs follow nnf::workspace::plan_w4a16_tiles.
 #include "w4a16_gemm_sk_launch.h"
 

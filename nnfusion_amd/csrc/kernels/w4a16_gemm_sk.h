@@ -1,5 +1,5 @@
-// fp16 x int4 (g128) MFMA tile GEMM for gfx950: four wavefronts side by side along N, work split evenly
-// over the CUs.
+// fp16 x int4 (g128) MFMA tile GEMM for gfx950: four wavefronts side by side along N, tiles cut into
+// equal parts of K, or the work of all tiles split evenly over the CUs.
 //
 //   Y[M,N] = epilogue( prologue(A)[M,K] . ((Wq - zp) * S)^T )
 //

@@ -1,5 +1,5 @@
-// fp16 x int4 (g128) for 2 <= M <= 16 activation rows and K = 1024, 2048, ... 8192 (M <= 32 up to K = 4096): the
-// memory pipeline of the
+// fp16 x int4 (g128) for 2 <= M <= 16 activation rows and K up to 8192 (M <= 32 up to K = 4096, M <= 64 up to K = 2048; K a
+// compile-time constant at multiples of 1024, a run-time value otherwise): the memory pipeline of the
 // row-streaming GEMV (w4a16_gemv_rows.hip) under the arithmetic of the M <= 16 MFMA kernel
 // (w4a16_skinny.hip).
 //
@@ -1315,7 +1315,7 @@ namespace nnf
             mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate);
     }
 
-    // The same kernel with K as a run-time value: any multiple of 256 up to 8 * GW * STEPS groups (2 <= M <= 16).
+    // The same kernel with K as a run-time value: any multiple of 128 up to 8 * GW * STEPS groups (2 <= M <= 16 MB).
     // A wavefront whose GW groups of a step would reach past the end of K fetches the last GW groups of the row
     // instead (the loads of every wavefront and step stay the same in number, which the hand-written wait counts
     // need) and multiplies what another wavefront already covers by a scale of zero.
@@ -2000,7 +2000,7 @@ namespace nnf
         }
     }
 
-    // K above 8192 (a multiple of 256, 2 <= M <= 16): the run-time-K kernel over ranges of K, fp32 sums to
+    // K beyond one launch (a multiple of 256; up to 40 rows): the run-time-K kernel over ranges of K, fp32 sums to
     // partial[ranges][M][N] (the caller runs the reduction pass).  Returns the number of ranges; 0: does not apply.
     int w4a16_mrows_ksplits(int M, int N, int K, int num_cu) { return workspace::w4a16_mrows_split(M, N, K, num_cu).ranges; }
 

@@ -144,7 +144,8 @@ namespace nnf
         // ---- plan of the fp16 x int4 tile GEMM (w4a16_gemm_sk.h) ----------------------------------------------
         // Tiles of tile_rows x 256 weight rows (SiLU-gate: 128 gate + 128 up rows, i.e. 128 output columns) or, for
         // the products without SiLU-gate, tile_rows x 128; the
-        // (tile, superstep of 256 k) units of the whole product are split evenly over `grid` workgroups, one per CU.
+        // (tile, superstep of 256 k) units of the whole product are split evenly over `grid` workgroups, at most one per CU (or
+        // one per tile: plan_w4a16_tiles chooses between numbers of workgroups and tile shapes).
         // A tile whose units belong to more than one workgroup is summed through the workspace: slots of
         // tile_rows x 256 fp32; workgroup v parks the first segment of its range in slot v and a later one in slot
         // grid + v; a second launch adds them up.
@@ -1089,10 +1090,12 @@ namespace nnf
             int ksplits = 0;          // *_SPLIT: ranges of K (fp32 partial sums, then the reduction pass)
             bool normalised_copy = false; // RMSNorm as a pass that writes the normalised activations (MFMA GEMV kernels, and what
                                           // the row-streaming kernel took over from other kernels)
-            bool via_scratch = false; // SKINNY: products to scratch first, an element-wise epilogue kernel reads them
+            // SKINNY with SiLU-gate: the products go to scratch memory, where the element-wise kernel reads them.  Also set for a
+            // residual in place, which the kernel adds itself now: the scratch memory is still asked for, not written.
+            bool via_scratch = false;
             SkPlan plan;              // TILE: what the caller fixed, or (own_plan) the even split, in whose scratch memory the launch fits
             bool own_plan = false;    // TILE: the launch follows plan_w4a16_tiles (w4a16_launch_plan)
-            size_t partial_bytes = 0; // partial sums / parked tiles / the products ahead of an element-wise epilogue
+            size_t partial_bytes = 0; // partial sums / parked tiles / the products ahead of SiLU-gate
             size_t rms_bytes = 0;     // RMSNorm prologue: rstd, fp32 [M] (the kernels multiply the RMSNorm weight in
                                       // themselves), or for the MFMA GEMV kernel the normalised activations, fp16 [M, K]
         };
@@ -1129,8 +1132,8 @@ namespace nnf
                     r.rms_bytes = r.normalised_copy ? xn_bytes : rstd_bytes;
                     return r;
                 }
-                // the MFMA GEMV kernel writes plain products: an epilogue that cannot work in place (the [M, 2N] gate | up
-                // pair, a residual that is the output buffer) reads them from scratch memory
+                // the MFMA GEMV kernel writes the [M, 2N] gate | up pair to scratch memory (and once wrote the products ahead of a
+                // residual in place there: what callers reserve for them stays what it was)
                 if (skinny_family && M <= 16 && w4a16_skinny_fits(M, n_rows, K))
                 {
                     r.kind = W4A16Route::SKINNY;

@@ -6,7 +6,10 @@
                                                                                       > counters per row and kernel
     python3 -m nnfusion_amd.profile_summary kernels  <dir of a --pmc run> <last n> [name part ...]
                                                        > counters per kernel: means over its last n dispatches
+    python3 -m nnfusion_amd.profile_summary pass     <case> [passes]     runs a case of perf/cases.py for a profile to be taken
+    python3 -m nnfusion_amd.profile_summary cases    <passes> <dir of a --stats run of `pass`>...   > kernels of each case
 
+A case is the name of one that perf/cases.py lists, or linear:MxNxK, a 4-bit linear layer of that size.
 `bench.py --pmc-probe` launches every configuration row eagerly with a marker launch (probe_read_kernel) ahead of each
 and prints the order of the rows as one JSON line ({"pmc_probe": ...}): the probe log is the file that line went to.  The
 dispatches between two markers are a row's; their counters are summed over the row's kernels and divided by its launches.
@@ -37,7 +40,7 @@ def short(name, width=64):
     name = demangle(name)
     name = re.sub(r"\b(nnf|gemm_sk)::", "", name)
     # (a name the demangler at hand does not know -- the _Float16 mangling -- : the kernel's name and its literal arguments)
-    m = re.match(r"_ZN3nnf\d+([a-z0-9_]+?_kernel)(?:I((?:L[ib]\d+E)+)E)?", name)
+    m = re.match(r"_ZN3nnf(?:12_GLOBAL__N_1)?\d+([a-z0-9_]+?_kernel)(?:I((?:L[ib]\d+E)+)E)?", name)
     if m:
         args = [("true" if v == "1" else "false") if t == "b" else v for t, v in re.findall(r"L([ib])(\d+)E", m.group(2) or "")]
         name = m.group(1) + (f"<{', '.join(args)}>" if args else "")
@@ -206,6 +209,41 @@ def kernels(directory, last, parts):
     return out
 
 
+def run_passes(name, count):
+    """`count` passes of a case, as a program would run them, after the input is prepared."""
+    import torch
+
+    from perf import cases
+
+    if name.startswith("linear:"):
+        case = cases._linear(name, *(int(x) for x in name[7:].split("x")))
+    else:
+        case = next(c for c in cases.listed() if c["name"] == name)
+    state = cases.prepare(case, 0)
+    torch.cuda.synchronize()
+    for _ in range(count):
+        cases.run(state)
+    torch.cuda.synchronize()
+    return [f"{count} passes of {name}"]
+
+
+def cases_table(passes, directories):
+    """Per case (the directory's name): this library's kernels, launches per pass and mean duration."""
+    out = ["rocprofv3 kernel statistics: kernels of one pass of every case of perf/cases.py", "",
+           "Commands (one run a case; on the MI355X box, from /tmp with TMPDIR=/tmp and PYTHONPATH=<this repository>):",
+           f"  rocprofv3 --kernel-trace --stats --output-format csv -d <dir>/<case> -o case -- python3 -m nnfusion_amd.profile_summary pass <case> {passes}",
+           f"  python3 -m nnfusion_amd.profile_summary cases {passes} <dir>/<case>...", "",
+           "Launches per pass and mean duration of each (passes follow one another; the inputs of a pass stay the same, so that what fits",
+           "the 256 MB cache may be read from it; a case in a captured graph runs one pass more, eagerly, when it is prepared).", ""]
+    for d in directories:
+        rows = [r for r in csv_rows(d, "kernel_stats.csv") if "nnf" in r["Name"]]
+        total = sum(float(r["AverageNs"]) * int(r["Calls"]) for r in rows) / 1e3 / passes
+        out.append(f"{os.path.basename(os.path.normpath(d))}: {total:.1f} us of kernels a pass")
+        for r in rows:
+            out.append(f"    {short(r['Name'], 78):<78} x {int(r['Calls']) / passes:<4.4g} {float(r['AverageNs']) / 1e3:>8.2f} us")
+    return out
+
+
 def main(argv):
     if len(argv) >= 2 and argv[0] == "stats":
         lines = stats(argv[1])
@@ -215,6 +253,10 @@ def main(argv):
         lines = counters(argv[1], argv[2], argv[3:])
     elif len(argv) >= 3 and argv[0] == "kernels":
         lines = kernels(argv[1], int(argv[2]), argv[3:])
+    elif len(argv) in (2, 3) and argv[0] == "pass":
+        lines = run_passes(argv[1], int(argv[2]) if len(argv) == 3 else 20)
+    elif len(argv) >= 3 and argv[0] == "cases":
+        lines = cases_table(int(argv[1]), argv[2:])
     else:
         raise SystemExit(__doc__)
     print("\n".join(lines))

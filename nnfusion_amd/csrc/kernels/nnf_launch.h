@@ -93,8 +93,8 @@ namespace nnf
     // a few rows (workspace::w4a16_mrows_fits): weights streamed through LDS rings, activations in registers
     // (N: outputs; gate / fusion.gate: from 2 N weight rows)
     // the same kernel for groups of 2^group_shift = 32 / 64 / 128 and a scalar zero point or (zero_points != null) one per
-    // (row, group): 2 <= M <= 16 (32 up to K = 4096), K = 2048 / 4096 / 8192.  fusion: gamma (normalised inside the kernel; no rstd), bias /
-    // residual or gate, where w4a16_mrows_q_fused_supported
+    // (row, group): 2 <= M <= 16 (32 up to K = 4096), K = 2048 / 4096 / 8192.  fusion: gamma (normalised inside the kernel; no rstd; where
+    // workspace::mrows_q_norm_inside), bias / residual or gate, where w4a16_mrows_q_fused_supported
     hipError_t launch_w4a16_mrows_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                     int K, int group_shift, int zp, const void* zero_points, int num_cu,
                                     const GemvFusion& fusion = GemvFusion());
@@ -106,7 +106,8 @@ namespace nnf
                                     int K, int group_shift, int zp, const void* zero_points, int num_cu);
     bool w8a16_mrows_q_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu);
     // ... with K any other multiple of 256 (2 <= M <= 16).  w4a16_mrows_q_any_ranges: 0 does not apply; 1: results to Y;
-    // more: fp32 sums of each range of K to partial[ranges][M][N], Y is not written (launch_wna16_reduce adds them up)
+    // more: fp32 sums of each range of K to partial[ranges][M][N], Y is not written (launch_wna16_reduce adds them up).
+    // fusion (one range): bias / residual or gate; no RMSNorm
     int w4a16_mrows_q_any_ranges(int M, int N, int K, int group_shift, bool zero_points, int num_cu);
     hipError_t launch_w4a16_mrows_q_any(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, float* partial,
                                         int M, int N, int K, int group_shift, int zp, const void* zero_points, int num_cu,

@@ -77,13 +77,12 @@ namespace nnf
     }
 
     // RMSNorm of the activations in registers as rms_norm_kernel computes it: fp16(x * rstd * gamma), in fp32, one rounding.
-    // Lane (m = col, kq) holds 64 bytes of each of its wavefront's GA groups; counts(g): whether this wavefront is the one
-    // that counts group g into its row's sum of squares; gsrc(g): the 64 bytes of gamma that pair with group g.
-    // sum_sq: [8 wavefronts][MB x 16 rows] of LDS of its own.  (Unlike mrows_scale_a, where rstd joins the sums at the end:
+    // Lane (m = col, kq) holds 64 bytes of each of its wavefront's GA groups; gsrc(g): the 64 bytes of gamma that pair with
+    // group g.  sum_sq: [8 wavefronts][MB x 16 rows] of LDS of its own.  (Unlike mrows_scale_a, where rstd joins the sums at the end:
     // these kernels have no per-group sums to scale, and x * gamma alone may leave the range of fp16.)
-    template <int MB, int GA, class Counts, class F>
+    template <int MB, int GA, class F>
     __device__ __forceinline__ void mrows_rms_norm(uintx4 (&areg)[MB][GA][4], float* sum_sq, int K, float eps, int wave, int col, int kq,
-                                                   Counts&& counts, F&& gsrc)
+                                                   F&& gsrc)
     {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -105,7 +104,7 @@ namespace nnf
                         sg = __builtin_fmaf((float)h.y, (float)h.y, sg);
                     }
                 }
-                ss += counts(g) ? sg : 0.f;
+                ss += sg;
             }
             ss += __shfl_xor(ss, 16, 64);
             ss += __shfl_xor(ss, 32, 64);
@@ -560,12 +559,14 @@ namespace nnf
     // loads, NSL of them) and, ZPT, their zero points (one byte per lane, NZL loads; a byte load lands in a lane's four
     // bytes of LDS).
     // LDS (bytes): weights [8 wavefronts][2 slots][GW KiB] | scales and zero points [8][2][(NSL + NZL) x 256] |
-    //              (FUSED: sums of squares [8][MB x 16] fp32) | partial tiles [2][8][MB KiB] |
+    //              (FUSED where RMSNorm may be inside: sums of squares [8][16] fp32) | partial tiles [2][8][MB KiB] |
     //              parked sums [tiles of the workgroup][M][16] fp32
     // pack = M | zp << 8 | gate << 16.
     // FUSED: RMSNorm ahead of the product (f.gamma), bias / residual or SiLU-gate behind it, as the nodes of their own
     // would compute them.  They were launches of their own (2 - 4 us each at 8 rows, 19 of the 56 us of a decoder layer
-    // with groups of 64 and zero points); inside, the prologue runs while the first weights are on their way.
+    // with groups of 64 and zero points); inside, the prologue runs while the first weights are on their way.  RMSNorm only
+    // where workspace::mrows_q_norm_inside says so (every workgroup normalises all the rows for itself: with more groups per
+    // wavefront that takes longer than the pass of its own).
     template <int GW, int GSHIFT, bool ZPT, int MB, bool FUSED>
     __global__ __launch_bounds__(512) void w4a16_mrows_q_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                                 const half_t* __restrict__ S, half_t* __restrict__ Y,
@@ -577,6 +578,7 @@ namespace nnf
         static_assert(MB == 1 || (MB == 2 && GW <= 2), "two blocks of rows: 32 VGPRs per group");
         constexpr int STEPS = 2;
         constexpr int K = GW * STEPS * 1024, G = K >> GSHIFT;
+        constexpr bool NORM = FUSED && MB == 1 && GW <= 2;
         constexpr int GA = GW * STEPS;         // groups of 128 of a wavefront
         constexpr int GAMMA_LOADS = (GA + 3) / 4; // of the RMSNorm weight into LDS: 1 KiB, four groups, each
         constexpr int ROW_BYTES = K / 2;       // a weight row
@@ -615,7 +617,7 @@ namespace nnf
         uint8_t* ring = smem + wave * (2 * TILE_BYTES);
         uint8_t* aux = smem + MR_WAVES * 2 * TILE_BYTES + wave * (2 * AUX);
         float* sum_sq = reinterpret_cast<float*>(smem + MR_WAVES * 2 * TILE_BYTES + MR_WAVES * 2 * AUX);
-        uint8_t* red = reinterpret_cast<uint8_t*>(sum_sq + (FUSED ? MR_WAVES * MB * 16 : 0)); // [2][8][MB KiB]
+        uint8_t* red = reinterpret_cast<uint8_t*>(sum_sq + (NORM ? MR_WAVES * 16 : 0)); // [2][8][MB KiB]
         float* parked = reinterpret_cast<float*>(red + 2 * MR_WAVES * MB * 1024);
 
         // weights: as in w4a16_mrows_kernel
@@ -676,8 +678,8 @@ namespace nnf
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     areg[0][g][j] = *reinterpret_cast<const uintx4*>(a_bytes + (size_t)(a_off + (g / GW) * (SPAN * 4) + (g % GW) * 256 + j * 16));
-            if (FUSED && f.gamma)
-                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [](int) { return true; }, [&](int g) {
+            if (NORM && f.gamma)
+                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [&](int g) {
                     return reinterpret_cast<const uint8_t*>(f.gamma) + wave * (GW * 256) + kq * 64 + (g / GW) * (SPAN * 4) + (g % GW) * 256;
                 });
         }
@@ -700,7 +702,7 @@ namespace nnf
                     fetch(p + 1);
                     __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
                 }
-                else if (FUSED && f.gamma)
+                else if (NORM && f.gamma)
                 {
                     // gamma of the wavefront's k positions into the free half, as in w4a16_mrows_kernel
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -721,12 +723,11 @@ namespace nnf
                 for (int j = 0; j < 4; ++j)
                     areg[p / GA][p % GA][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
             }
-            if (FUSED && f.gamma)
+            if (NORM && f.gamma)
             {
                 const uint8_t* gamma_block = stage + (NP & 1) * ROW_BLOCK_BYTES;
                 __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [](int) { return true; },
-                                       [&](int g) { return gamma_block + g * 256 + kq * 64; });
+                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [&](int g) { return gamma_block + g * 256 + kq * 64; });
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __syncthreads();
@@ -1053,7 +1054,9 @@ namespace nnf
     // A block of 128 weights has SPC = 128 / group scales; with groups of 128 a wavefront's first block may be an odd one:
     // its scales are fetched from the 4-byte word, its zero points from the byte, at or below it (`skip` = 1), and
     // one word / byte more per row comes along.
-    // FUSED (one range of K): as in w4a16_mrows_q_kernel; over ranges the rest of the epilogue belongs to the reduction pass.
+    // FUSED (one range of K): bias / residual or SiLU-gate as in w4a16_mrows_q_kernel; over ranges they belong to the reduction
+    // pass.  RMSNorm is a launch of its own either way: inside, it took longer at every K that this kernel serves
+    // (workspace::mrows_q_norm_inside).
     template <int GW, int GSHIFT, bool ZPT, bool FUSED>
     __global__ __launch_bounds__(512) void w4a16_mrows_q_any_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                                     const half_t* __restrict__ S, half_t* __restrict__ Y,
@@ -1064,7 +1067,6 @@ namespace nnf
         static_assert(GW >= 2 && GW <= 4 && GSHIFT >= 5 && GSHIFT <= 7, "blocks per wavefront and step; groups of 32 / 64 / 128");
         constexpr int STEPS = 2, MB = 1;
         constexpr int GA = GW * STEPS;
-        constexpr int GAMMA_LOADS = (GA + 3) / 4;
         constexpr int SLICE = GW * 64;
         constexpr int TILE_BYTES = 16 * SLICE;
         constexpr int SPC = 1 << (7 - GSHIFT);                     // scales per block of 128 weights
@@ -1104,8 +1106,7 @@ namespace nnf
 
         uint8_t* ring = smem + wave * (2 * TILE_BYTES);
         uint8_t* aux = smem + MR_WAVES * 2 * TILE_BYTES + wave * (2 * AUX);
-        float* sum_sq = reinterpret_cast<float*>(smem + MR_WAVES * 2 * TILE_BYTES + MR_WAVES * 2 * AUX); // (FUSED) [8][16]
-        uint8_t* red = reinterpret_cast<uint8_t*>(sum_sq + (FUSED ? MR_WAVES * MB * 16 : 0)); // [2][8][1024]
+        uint8_t* red = smem + MR_WAVES * 2 * TILE_BYTES + MR_WAVES * 2 * AUX; // [2][8][1024]
         float* parked = reinterpret_cast<float*>(red + 2 * MR_WAVES * MB * 1024);
 
         auto swz = [](int r) { return GW % 4 == 0 ? (r & 15) : GW % 2 == 0 ? (r >> 1) & 7 : (r >> 2) & 3; };
@@ -1164,8 +1165,6 @@ namespace nnf
         // activations: into the MFMA operand registers (through LDS as whole lines from a few rows on, see
         // workspace::mrows_stages_activations), then in the pair order of the nibble trick
         uintx4 areg[MB][GA][4];
-        // (a group that another wavefront covers as well: counted there)
-        auto counts = [&](int p) { return p % GW >= own_block(p / GW) - fetch_block(p / GW); };
         {
             if (!workspace::mrows_stages_activations(M, K))
             {
@@ -1180,10 +1179,6 @@ namespace nnf
                         for (int j = 0; j < 4; ++j)
                             areg[0][st * GW + g][j] = *reinterpret_cast<const uintx4*>(a_src + g * 256 + j * 16);
                 }
-                if (FUSED && f.gamma)
-                    mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, counts, [&](int p) {
-                        return reinterpret_cast<const uint8_t*>(f.gamma) + (fetch_block(p / GW) + p % GW) * 256 + kq * 64;
-                    });
             }
             else
             {
@@ -1202,31 +1197,11 @@ namespace nnf
                         fetch(p + 1);
                         __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
                     }
-                    else if (FUSED && f.gamma)
-                    {
-                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-                        for (int i = 0; i < GAMMA_LOADS; ++i)
-                        {
-                            const int g = min(4 * i + (lane >> 4), GA - 1);
-                            const uint8_t* src = reinterpret_cast<const uint8_t*>(f.gamma) + (fetch_block(g / GW) + g % GW) * 256 + (lane & 15) * 16;
-                            __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(stage + (GA & 1) * ROW_BLOCK_BYTES + i * 1024),
-                                                             16, 0, 0);
-                        }
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(GAMMA_LOADS));
-                    }
                     else
                         __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         areg[0][p][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
-                }
-                if (FUSED && f.gamma)
-                {
-                    const uint8_t* gamma_block = stage + (GA & 1) * ROW_BLOCK_BYTES;
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-                    mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, counts,
-                                           [&](int g) { return gamma_block + g * 256 + kq * 64; });
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 __syncthreads();
@@ -1826,6 +1801,7 @@ namespace nnf
                                     int K, int group_shift, int zp, const void* zero_points, int num_cu, const GemvFusion& fusion)
     {
         if (fusion.any() ? fusion.rstd || (fusion.gate && (fusion.bias || fusion.residual)) ||
+                               (fusion.gamma && !workspace::mrows_q_norm_inside(M, K)) ||
                                !w4a16_mrows_q_fused_supported(M, N, K, group_shift, zero_points != nullptr, num_cu, fusion.gate)
                          : !w4a16_mrows_q_supported(M, N, K, group_shift, zero_points != nullptr, num_cu))
             return hipErrorInvalidValue;
@@ -1920,7 +1896,7 @@ namespace nnf
             const int grid = n_tiles < per_range ? n_tiles : per_range;
             const int tiles_q = n_tiles / grid, tiles_r = n_tiles % grid;
             const size_t lds = workspace::w4a16_mrows_q_any_lds_bytes(GW, M, (tiles_q + (tiles_r ? 1 : 0)) * (fusion.gate ? 2 : 1), GSHIFT,
-                                                                      ZPT, FUSED);
+                                                                      ZPT);
             if (lds > MAX_LDS_BYTES)
                 return hipErrorInvalidValue;
             auto kernel = &w4a16_mrows_q_any_kernel<GW, GSHIFT, ZPT, FUSED>;
@@ -1979,7 +1955,7 @@ namespace nnf
     bool w4a16_mrows_q_any_fused_supported(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool gate)
     {
         return !(group_shift == 7 && !zero_points) &&
-               workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points, num_cu, true, gate).ranges == 1;
+               workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points, num_cu, gate).ranges == 1;
     }
 
     hipError_t launch_w4a16_mrows_q_any(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, float* partial,
@@ -1987,8 +1963,8 @@ namespace nnf
                                         const GemvFusion& fusion)
     {
         const workspace::MrowsQAny pl =
-            workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points != nullptr, num_cu, fusion.any(), fusion.gate);
-        if (fusion.any() && (pl.ranges != 1 || fusion.rstd || (fusion.gate && (fusion.bias || fusion.residual))))
+            workspace::w4a16_mrows_q_any_plan(M, N, K, group_shift, zero_points != nullptr, num_cu, fusion.gate);
+        if (fusion.any() && (pl.ranges != 1 || fusion.gamma || fusion.rstd || (fusion.gate && (fusion.bias || fusion.residual))))
             return hipErrorInvalidValue;
         if (pl.ranges < 1 || (pl.ranges > 1 && !partial) || (group_shift == 7 && !zero_points))
             return hipErrorInvalidValue;

@@ -380,7 +380,8 @@ namespace
 
     // A fused product of 4-bit weights on a few rows (other block parameters than the plain kernels'): where the plain product
     // runs on a row-streaming kernel, the nodes around it move into that kernel, or, over ranges of K, into the reduction
-    // pass behind it (RMSNorm stays a launch there: a range does not see a whole row).  Same arithmetic as the nodes'
+    // pass behind it (RMSNorm stays a launch there: a range does not see a whole row).  In the kernel, RMSNorm is a launch
+    // ahead of it where that is faster (workspace::mrows_q_norm_inside).  Same arithmetic as the nodes'
     // own kernels, 2 - 4 us each at 8 rows.  fusion.gate: N outputs from 2 N weight rows.  xn: M x K fp16, for RMSNorm;
     // own: the product's scratch memory.  taken = false: the nodes have to run one by one, nothing was launched.
     int wna16_fused_rows(hipStream_t s, const void* A, const void* Wq, const void* scales, void* Y, int M, int N, int K,
@@ -392,29 +393,38 @@ namespace
             return NNF_OK;
         const int gs = group_shift_of(q->group), rows = fusion.gate ? 2 * N : N;
         const bool zpt = q->zero_points != nullptr;
+        nnf::GemvFusion inside = fusion; // what the kernel does
+        if (!nnf::workspace::mrows_q_norm_inside(M, K))
+            inside.gamma = nullptr;
+        const auto norm_ahead = [&]() -> hipError_t {
+            if (!fusion.gamma || inside.gamma)
+                return hipSuccess;
+            const hipError_t e = nnf::launch_rms_norm(s, A, fusion.gamma, xn, M, K, fusion.rms_eps);
+            A = xn;
+            return e;
+        };
         if (nnf::w4a16_mrows_q_supported(M, rows, K, gs, zpt, num_cu))
         {
-            taken = nnf::w4a16_mrows_q_fused_supported(M, N, K, gs, zpt, num_cu, fusion.gate);
-            return taken ? (int)nnf::launch_w4a16_mrows_q(s, A, Wq, scales, Y, M, N, K, gs, q->zero_point, q->zero_points, num_cu, fusion)
-                         : NNF_OK;
+            taken = !inside.any() || nnf::w4a16_mrows_q_fused_supported(M, N, K, gs, zpt, num_cu, fusion.gate);
+            if (!taken)
+                return NNF_OK;
+            const hipError_t e = norm_ahead();
+            return (int)(e != hipSuccess ? e : nnf::launch_w4a16_mrows_q(s, A, Wq, scales, Y, M, N, K, gs, q->zero_point, q->zero_points, num_cu, inside));
         }
         const int ranges = M <= 16 ? nnf::w4a16_mrows_q_any_ranges(M, rows, K, gs, zpt, num_cu) : 0;
         if (ranges == 1)
         {
-            taken = nnf::w4a16_mrows_q_any_fused_supported(M, N, K, gs, zpt, num_cu, fusion.gate);
-            return taken ? (int)nnf::launch_w4a16_mrows_q_any(s, A, Wq, scales, Y, nullptr, M, N, K, gs, q->zero_point, q->zero_points,
-                                                              num_cu, fusion)
-                         : NNF_OK;
+            taken = !inside.any() || nnf::w4a16_mrows_q_any_fused_supported(M, N, K, gs, zpt, num_cu, fusion.gate);
+            if (!taken)
+                return NNF_OK;
+            const hipError_t e = norm_ahead();
+            return (int)(e != hipSuccess ? e : nnf::launch_w4a16_mrows_q_any(s, A, Wq, scales, Y, nullptr, M, N, K, gs, q->zero_point,
+                                                                            q->zero_points, num_cu, inside));
         }
         if (ranges > 1 && own && aligned16(own) && own_bytes >= (size_t)ranges * M * rows * sizeof(float))
         {
             taken = true;
-            hipError_t e = hipSuccess;
-            if (fusion.gamma)
-            {
-                e = nnf::launch_rms_norm(s, A, fusion.gamma, xn, M, K, fusion.rms_eps);
-                A = xn;
-            }
+            hipError_t e = norm_ahead();
             if (e == hipSuccess)
                 e = nnf::launch_w4a16_mrows_q_any(s, A, Wq, scales, nullptr, (float*)own, M, rows, K, gs, q->zero_point, q->zero_points, num_cu);
             if (e == hipSuccess)

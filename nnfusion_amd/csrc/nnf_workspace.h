@@ -714,7 +714,15 @@ namespace nnf
         // The same kernel for groups of 32 / 64 / 128 and zero points per (row, group) (w4a16_mrows_q_kernel): 2 .. 16 rows
         // (.. 32 up to K = 4096), K = 2048, 4096, 8192 (GW = K / 2048 groups of 128 per wavefront and step); per wavefront and ring slot 256 bytes
         // per 64 4-byte words of scales (GW x 128 / group scales for each of 16 rows) and as much again for zero points.
-        // (fused: the wavefronts' sums of squares per row for RMSNorm inside the kernel)
+        // RMSNorm in front of such a product: inside the kernel, or a pass of its own ahead of it.  Inside, every workgroup
+        // normalises all the rows for itself before its first product, twice over once a second block of rows is there; the
+        // pass takes 2 us and a launch.  Measured (N = 2304 .. 11008, groups of 32 / 64 / 128, with and without zero points,
+        // time with the pass / time inside; alone, with SiLU-gate behind): K = 2048, 2 .. 16 rows 1.01 - 1.16, 1.03 - 1.17;
+        // 17 .. 32 rows 0.93 - 0.98, 0.97 - 1.02; K = 4096, 2 .. 7 rows 0.87 - 0.93, 0.92 - 0.99 (8 rows and up bring their
+        // activations in as whole lines), 8 .. 16 rows 0.95 - 1.02, 0.97 - 1.03, 17 .. 32 rows 0.82 - 0.89, 0.83 - 0.93;
+        // K = 3072 / 3584 0.88 - 1.00, 0.92 - 1.01; K = 4608 / 5120 0.76 - 0.96, 0.80 - 0.97; K = 8192 0.70 - 0.91, 0.78 - 0.95.
+        constexpr bool mrows_q_norm_inside(int M, int K) { return M <= 16 && (K == 2048 || (K == 4096 && mrows_stages_activations(M, K))); }
+        // (fused: with room for the wavefronts' sums of squares per row, at the sizes that may have RMSNorm inside)
         inline size_t w4a16_mrows_q_lds_bytes(int K, int M, int tiles, int group_shift, bool zero_points, bool fused = false)
         {
             const int gw = K >> 11;
@@ -722,7 +730,7 @@ namespace nnf
             const int loads = (16 * words + 63) / 64;
             const size_t aux = (size_t)(zero_points ? 2 : 1) * loads * 256;
             const size_t mb = M <= 16 ? 1 : 2; // blocks of 16 rows
-            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (fused ? 8 * mb * 64 : 0) + mrows_tail_bytes((size_t)2 * 8 * mb * 1024 + (size_t)tiles * M * 64);
+            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (fused && M <= 16 && K <= 4096 ? 8 * 64 : 0) + mrows_tail_bytes((size_t)2 * 8 * mb * 1024 + (size_t)tiles * M * 64);
         }
         // (17 .. 32 rows: two blocks of rows in registers, up to K = 4096)
         // fused, gate: with the nodes around the product inside the kernel, N outputs from 2 N weight rows
@@ -765,16 +773,15 @@ namespace nnf
         {
             int ranges = 0, range_blocks = 0, gw = 0; // ranges 0: not applicable; 1: no workspace
         };
-        inline size_t w4a16_mrows_q_any_lds_bytes(int gw, int M, int tiles, int group_shift, bool zero_points, bool fused = false)
+        inline size_t w4a16_mrows_q_any_lds_bytes(int gw, int M, int tiles, int group_shift, bool zero_points)
         {
             const int spc = 1 << (7 - group_shift);
             const int words = spc == 1 ? gw / 2 + 1 : gw * spc / 2;
             const int loads = (16 * words + 63) / 64;
             const size_t aux = (size_t)(zero_points ? 2 : 1) * loads * 256;
-            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (fused ? 8 * 64 : 0) + mrows_tail_bytes((size_t)2 * 8 * 1024 + (size_t)tiles * M * 64);
+            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + mrows_tail_bytes((size_t)2 * 8 * 1024 + (size_t)tiles * M * 64);
         }
-        inline MrowsQAny w4a16_mrows_q_any_plan(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool fused = false,
-                                                bool gate = false)
+        inline MrowsQAny w4a16_mrows_q_any_plan(int M, int N, int K, int group_shift, bool zero_points, int num_cu, bool gate = false)
         {
             MrowsQAny p;
             if (M < 2 || M > 16 || N < 16 || K < 1024 || K > 65536 || (K & 255) || num_cu < 16 || group_shift < 5 || group_shift > 7)
@@ -797,7 +804,7 @@ namespace nnf
             }
             const int n_tiles = (N + 15) / 16, per_range = num_cu / ranges;
             const int grid = n_tiles < per_range ? n_tiles : per_range;
-            if (w4a16_mrows_q_any_lds_bytes(gw, M, (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid), group_shift, zero_points, fused) > LDS_BYTES_PER_CU)
+            if (w4a16_mrows_q_any_lds_bytes(gw, M, (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid), group_shift, zero_points) > LDS_BYTES_PER_CU)
                 return p;
             p.ranges = ranges;
             p.range_blocks = rb;

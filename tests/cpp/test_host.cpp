@@ -1184,6 +1184,13 @@ int main(int argc, char** argv)
             EXPECT(ws::w4a16_mrows_q_lds_bytes(8192, 16, 2, 5, true) == 65536 + 16384 + 65536);
             EXPECT(ws::w4a16_mrows_q_lds_bytes(4096, 16, 1, 6, false) == 32768 + 4096 + 65536);
             EXPECT(!ws::w4a16_mrows_q_fits(16, 1000000, 8192, 5, true, 256)); // the parked sums do not fit
+            // RMSNorm inside the kernel where it is faster than its own pass, with room for the sums of squares only there
+            for (int k = 1024; k <= 16384; k += 256)
+                for (int m = 1; m <= 32; ++m)
+                    EXPECT(ws::mrows_q_norm_inside(m, k) == (m <= 16 && (k == 2048 || (k == 4096 && m >= 8))));
+            EXPECT(ws::w4a16_mrows_q_lds_bytes(4096, 16, 1, 6, false, true) == 32768 + 4096 + 512 + 65536);
+            EXPECT(ws::w4a16_mrows_q_lds_bytes(4096, 32, 1, 6, false, true) == 32768 + 4096 + 65536);
+            EXPECT(ws::w4a16_mrows_q_lds_bytes(8192, 16, 2, 5, true, true) == 65536 + 16384 + 65536);
         }
         // ... with a run-time K: one piece up to 8192 where most of what is fetched counts, ranges of at most 32 blocks above
         {

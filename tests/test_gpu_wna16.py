@@ -303,6 +303,30 @@ def test_fused_rows_equal_the_nodes(gpu, m, n, k, group, zp_tensor):
     close(ops.wna16_gemm_fused(x, t[1], t[2], zero_points=tz, rms_gamma=gamma, rms_eps=1e-5, act=1, **q), gated(normed), 2e-2)
 
 
+# both sides of the line between RMSNorm ahead of the row-streaming kernels and inside them: rows at K = 4096 (8 and up
+# inside) and at K = 2048 (17 and up ahead); every other K ahead
+@pytest.mark.parametrize("m,n,k", [(7, 1000, 4096), (17, 520, 4096), (32, 4111, 4096), (17, 520, 2048), (2, 1000, 8192), (16, 4111, 8192),
+                                   (4, 520, 3072), (16, 1000, 5120), (9, 300, 6400)])
+@pytest.mark.parametrize("group,zp_tensor", [(32, True), (64, False)])
+def test_fused_rows_with_rms_norm_ahead(gpu, m, n, k, group, zp_tensor):
+    """Where RMSNorm is a pass of its own in front of the kernel, the fused product is the nodes' own arithmetic, bit for bit
+    (inside, the sum of squares is added in another order: some rounding of some activation differs)."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    a, wq, s, zps = _case(m * 13 + n + k + group, m, n, k, 4, group, zp_tensor)
+    a, wq, s = [torch.from_numpy(x).to(gpu) for x in (a, wq, s)]
+    q = dict(bits=4, group=group, zp=5, zero_points=torch.from_numpy(zps).to(gpu) if zp_tensor else None)
+    gen = torch.Generator(device="cpu").manual_seed(m + k)
+    gamma = torch.randn(k, generator=gen).mul(0.1).add(1).half().to(gpu)
+    res = torch.randn(m, n, generator=gen).half().to(gpu)
+    ref = ops.wna16_gemm(ops.rms_norm(a, gamma, 1e-5), wq, s, **q)
+    assert torch.equal(ops.wna16_gemm_fused(a, wq, s, rms_gamma=gamma, rms_eps=1e-5, **q), ref)
+    y = ops.wna16_gemm_fused(a, wq, s, rms_gamma=gamma, rms_eps=1e-5, residual=res, out=res.clone(), **q)
+    assert torch.equal(y, ops.elementwise("add", ref, res))
+
+
 def test_fused_rows_with_the_output_over_the_input(gpu):
     """x = product(RMSNorm(x)) written over x: workgroups that finish must not change what others still read."""
     import torch

@@ -287,6 +287,8 @@ namespace nnf
         // measured time for nine in ten plans, and the plans they pick 15 % (SiLU-gate: 9 %) faster than the even split in the
         // geometric mean, within 1 - 2 % of the fastest one tried.  450 x 448 x 640: 17.1 -> 8.8 us; 110 x 12288 x 1536: 20.8 -> 13.4;
         // 128 x 9216 x 2304: 23.0 -> 16.0; 250 x 16384 x 4096: 47.0 -> 38.9; 450 x 9216 x 11008: 140 -> 106.
+        // One in fifty of the plans picked is more than 1 % slower than the even split, by up to 13 % (77 x 5824 x 10624: 28.6 -> 29.2 us);
+        // a wider margin than 3 % gives up more than it saves (the plans estimated 3 - 5 % ahead are 7 % faster in the geometric mean).
         // Microseconds: rounds of workgroups x start; the longest share's supersteps (256 k) x (step + load x busy CUs);
         // parts that meet: share + load, more of it from five and nine parts a tile on.
         struct SkCost
@@ -1033,6 +1035,19 @@ namespace nnf
             // (up to 16 rows K = 1536 on one group per wavefront is level: left where it was)
             return M > 16 || 4 * (K >> 7) >= (gw == 1 ? 52 : 3 * 16 * gw);
         }
+        // ... except where the MFMA GEMV, which needs no scratch memory but RMSNorm's either, is faster: odd numbers of groups and up
+        // to sixteen of them, of which less than seven eighths of what is fetched counts, at eight rows (up to sixteen groups) or
+        // until the activations arrive as whole lines (eight to ten).  Time on the MFMA GEMV / here, N = 512 .. 4096, plain and with
+        // RMSNorm: K = 3200, 8 .. 10 rows 0.94 - 0.98 (4096 columns at 8 rows 5.7 / 6.0 us), 3456, 8 and 9 rows 0.96 - 1.01, 1664, 8 rows
+        // 0.94 - 0.97; with 9152 columns 0.98 - 1.06; K = 3712, 3968, 1792, and 1664 at nine rows: 0.98 - 1.2.
+        // (Not with SiLU-gate, 1.05 - 1.2 x here, nor with the residual in place, for which that route asks for scratch memory.)
+        inline bool w4a16_skinny_ahead_of_mrows(int M, int N, int K)
+        {
+            const int gw = w4a16_mrows_step_groups(M, K);
+            if (M < 8 || M > 16 || N > 8192 || w4a16_mrows_fixed_k(M, K) || 8 * (K >> 7) >= 7 * 16 * gw || !w4a16_skinny_fits(M, N, K))
+                return false;
+            return gw == 1 ? M == 8 && 4 * (K >> 7) >= 52 : (K & 128) && !mrows_stages_activations(M, K);
+        }
         // ---- W8A8, one activation row: the row-streaming GEMV (w8a8_gemv_rows.hip) ----
         struct Q8RowsPlan
         {
@@ -1131,7 +1146,8 @@ namespace nnf
                 const bool two_ranges = !gate && !rms && K == 8192 && M >= 8 && M <= 16 && w4a16_mrows_split(M, n_rows, K, num_cu).ranges > 1;
                 // (the products that once ran elsewhere: gamma times the activations alone may leave the range of fp16)
                 const bool taken_over = rms && !w4a16_mrows_fixed_k(M, K) && ((K & 128) || M > 32 || 4 * (K >> 7) < 3 * 16 * (K <= 4096 ? 2 : 3));
-                if (rows_family && M > 1 && !two_ranges && !(any && taken_over && !room_for_copy) &&
+                const bool gemv_ahead = any && !gate && !in_place_residual && w4a16_skinny_ahead_of_mrows(M, n_rows, K);
+                if (rows_family && M > 1 && !two_ranges && !gemv_ahead && !(any && taken_over && !room_for_copy) &&
                     (any ? w4a16_mrows_preferred(M, N, K, num_cu, gate) : w4a16_mrows_fits(M, N, K, num_cu, gate)))
                 {
                     r.kind = W4A16Route::MROWS;

@@ -103,7 +103,7 @@ def traffic(fetch_dir, write_dir, log):
         scale[counter] = (kib / (sum(cal) / len(cal)), sum(cal) / len(cal))
         per[counter] = [(row, sum(d.get(counter, 0.0) for d in ds) / row["launches"], kernels_of(row, ds)) for row, ds in segs]
     out = ["rocprofv3 hardware counters: HBM traffic per launch of every benchmark configuration (FETCH_SIZE, WRITE_SIZE)", "",
-           "Commands (two runs, one counter each; on the MI355X box, from /tmp with TMPDIR=/tmp):",
+           "Commands (two runs, one counter each; on an MI355X, from /tmp with TMPDIR=/tmp):",
            "  rocprofv3 --pmc FETCH_SIZE --kernel-trace --output-format csv -d <FETCH dir> -o fetch -- python3 bench.py --pmc-probe",
            "  rocprofv3 --pmc WRITE_SIZE --kernel-trace --output-format csv -d <WRITE dir> -o write -- python3 bench.py --pmc-probe",
            "  python3 -m nnfusion_amd.profile_summary traffic <FETCH dir> <WRITE dir> <stdout of the first run>", "",
@@ -128,7 +128,7 @@ def traffic(fetch_dir, write_dir, log):
 def stats(directory):
     rows = csv_rows(directory, "kernel_stats.csv")
     out = ["rocprofv3 kernel statistics: bench.py, decode sweep (M=1 fp16 x int4 g128) + the extra configurations", "",
-           "Commands (on the MI355X box, from /tmp with TMPDIR=/tmp):",
+           "Commands (on an MI355X, from /tmp with TMPDIR=/tmp):",
            "  rocprofv3 --kernel-trace --stats --output-format csv -d <dir> -o bench -- python3 bench.py --no-cpu-baseline",
            "  python3 -m nnfusion_amd.profile_summary stats <dir>", "",
            "Source: bench_kernel_stats.csv (all kernels of the process, parity gate and probes included; durations in ns).", "",
@@ -230,7 +230,7 @@ def run_passes(name, count):
 def cases_table(passes, directories):
     """Per case (the directory's name): this library's kernels, launches per pass and mean duration."""
     out = ["rocprofv3 kernel statistics: kernels of one pass of every case of perf/cases.py", "",
-           "Commands (one run a case; on the MI355X box, from /tmp with TMPDIR=/tmp and PYTHONPATH=<this repository>):",
+           "Commands (one run a case; on an MI355X, from /tmp with TMPDIR=/tmp and PYTHONPATH=<this repository>):",
            f"  rocprofv3 --kernel-trace --stats --output-format csv -d <dir>/<case> -o case -- python3 -m nnfusion_amd.profile_summary pass <case> {passes}",
            f"  python3 -m nnfusion_amd.profile_summary cases {passes} <dir>/<case>...", "",
            "Launches per pass and mean duration of each (passes follow one another; the inputs of a pass stay the same, so that what fits",

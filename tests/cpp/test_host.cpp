@@ -1184,6 +1184,23 @@ int main(int argc, char** argv)
             EXPECT(ws::w4a16_mrows_q_lds_bytes(8192, 16, 2, 5, true) == 65536 + 16384 + 65536);
             EXPECT(ws::w4a16_mrows_q_lds_bytes(4096, 16, 1, 6, false) == 32768 + 4096 + 65536);
             EXPECT(!ws::w4a16_mrows_q_fits(16, 1000000, 8192, 5, true, 256)); // the parked sums do not fit
+            // the MFMA GEMV keeps a few products that the row-streaming kernel could take: no other scratch memory than there
+            for (int k = 128; k <= 16384; k += 128)
+                for (int m = 1; m <= 64; ++m)
+                {
+                    const bool keeps = (k == 3200 && m >= 8 && m <= 10) || (k == 3456 && (m == 8 || m == 9)) || (k == 1664 && m == 8);
+                    EXPECT((ws::w4a16_skinny_ahead_of_mrows(m, 4096, k) && ws::w4a16_mrows_preferred(m, 4096, k, 256)) == keeps);
+                    if (!keeps)
+                        continue;
+                    for (int rms = 0; rms < 2; ++rms)
+                    {
+                        const auto gemv = ws::route_w4a16(m, 4096, k, false, rms, false, 256), rows = ws::route_w4a16(m, 4096, k, false, rms, true, 256);
+                        EXPECT(gemv.kind == ws::W4A16Route::SKINNY && rows.kind == ws::W4A16Route::MROWS);
+                        EXPECT(gemv.partial_bytes == 0 && rows.partial_bytes == 0 && gemv.rms_bytes == rows.rms_bytes);
+                    }
+                    EXPECT(ws::route_w4a16(m, 2048, k, true, false, false, 256).kind == ws::W4A16Route::MROWS);
+                    EXPECT(ws::route_w4a16(m, 9152, k, false, false, false, 256).kind == ws::W4A16Route::MROWS);
+                }
             // RMSNorm inside the kernel where it is faster than its own pass, with room for the sums of squares only there
             for (int k = 1024; k <= 16384; k += 256)
                 for (int m = 1; m <= 32; ++m)

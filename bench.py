@@ -51,14 +51,14 @@ PROBES_SO = os.path.join(ROOT, "nnfusion_amd", "lib", "libnnf_bench_probes.so")
 PROFILES_DIR = os.path.join(ROOT, "profiles")
 
 GEMM_NK = 8192
-GEMM_MS = (16, 128, 1024, 4096)       # configs[2]
-W8A8_MS = (1, 32, 512, 4096)          # configs[3]
+GEMM_MS = (16, 128, 1024, 4096)       # fp16 x int4, N = K = 8192
+W8A8_MS = (1, 32, 512, 4096)          # W8A8, N = K = 8192
 SMALL_BATCHES = (2, 4, 8, 16)         # the sweep's shapes with a few rows
 # the fp16 x int-N product with other block parameters (bits, group, zero point per (row, group)?) than the benchmark's,
 # on the two plain kernels that serve them, at N = K = GEMM_NK
 WNA16_CASES = ((8, 128, False), (4, 64, True))
 WNA16_MS = (1, 16, 4096)
-MLP_HI = (4096, 11008)                # configs[4]: hidden and intermediate size
+MLP_HI = (4096, 11008)                # the fused MLP block: hidden and intermediate size
 MLP_MS = (1, 16, 256)                 # ... at M = 256; the same block at decode sizes beside it
 
 def load_row_kernels():

@@ -12,6 +12,7 @@ namespace nnf
     namespace workspace
     {
         struct W4A16Route;
+        struct KstreamPlan;
     }
 
     // largest dynamic LDS a workgroup may ask for on gfx950 (160 KiB per CU)
@@ -130,6 +131,12 @@ namespace nnf
     hipError_t launch_w4a16_mrows_split(hipStream_t stream, const void* A, const void* Wq, const void* S, float* partial,
                                         int M, int N, int K, int zp, int num_cu, const void* gamma = nullptr, void* Y = nullptr,
                                         const GemvFusion* epilogue = nullptr, uint32_t* sync = nullptr);
+
+    // 33 .. 64 rows: the K-streaming kernel, as `plan` (workspace::kstream_plan) says.  fusion: gamma (rstd computed inside), bias /
+    // residual or gate; over ranges of K neither gamma nor gate, the ranges' sums in `partial` (plan.partial_bytes) and one zeroed
+    // word per workgroup of a range in `sync` (zero again afterwards)
+    hipError_t launch_w4a16_kstream(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
+                                    void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync);
 
     // (bias, residual: added behind the product, each or null; the residual may be Y)
     hipError_t launch_w4a16_skinny(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M,

@@ -354,6 +354,19 @@ namespace nnf
         const int n_rows = gate ? 2 * N : N; // weight rows
         if (route.kind == W4A16Route::NONE || (route.partial_bytes > 0 && !partial_ws) || (route.rms_bytes > 0 && !rms_ws))
             return hipErrorInvalidValue;
+        // ---- the K-streaming kernel: prologue and epilogue inside, ranges of K added up in the launch ---------------------------
+        const workspace::KstreamPlan kstream =
+            workspace::w4a16_launch_kstream(route, M, N, K, gate, rms, num_cu, choice.sync_flags ? choice.sync_bytes : 0);
+        if (kstream.tiles > 0)
+        {
+            GemvFusion fusion;
+            fusion.gamma = rms_gamma;
+            fusion.rms_eps = rms_eps;
+            fusion.bias = bias;
+            fusion.residual = residual;
+            fusion.gate = gate;
+            return launch_w4a16_kstream(stream, kstream, A, Wq, S, Y, M, N, K, zp, fusion, (float*)partial_ws, (uint32_t*)choice.sync_flags);
+        }
         // ---- RMSNorm pre-pass: rstd[m] for the kernels that multiply the weight in themselves, the normalised
         // activations for the MFMA GEMV kernel -------------------------------------------------------------------
         // (the row-streaming kernels add up the squares of the activations they hold themselves: no pre-pass; the form

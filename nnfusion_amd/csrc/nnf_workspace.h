@@ -1048,6 +1048,82 @@ namespace nnf
                 return false;
             return gw == 1 ? M == 8 && 4 * (K >> 7) >= 52 : (K & 128) && !mrows_stages_activations(M, K);
         }
+        // ---- 33 .. 64 activation rows: the K-streaming kernel (w4a16_kstream.hip) ----
+        // One workgroup per CU with up to KSTREAM_MAX_TILES 16-row weight tiles, their sums in registers; K in chunks of eight groups.
+        constexpr int KSTREAM_WAVES = 8, KSTREAM_MAX_TILES = 6, KSTREAM_MAX_GROUPS = 64;
+        // blocks of 16 rows x 256 bytes of activations in a wavefront's ring; its bytes of LDS
+        constexpr int kstream_ring(int mb) { return mb < 4 ? mb : 3; }
+        constexpr int kstream_wave_bytes(int tiles, int mb, bool rms) { return kstream_ring(mb) * 4096 + tiles * 1024 + (rms ? 256 : 0); }
+        // tiles whose eight partial sums are in LDS at a time (an even number where there is more than one round)
+        constexpr int kstream_round(int tiles, int mb) { return mb == 4 && tiles > 4 ? 4 : tiles; }
+        constexpr size_t kstream_lds_bytes(int tiles, int mb, bool rms)
+        {
+            const size_t stream = (size_t)KSTREAM_WAVES * kstream_wave_bytes(tiles, mb, rms) + (size_t)tiles * 2048;
+            const size_t sums = (size_t)4096 + (size_t)KSTREAM_WAVES * kstream_round(tiles, mb) * mb * 1024;
+            return stream > sums ? stream : sums;
+        }
+        struct KstreamPlan
+        {
+            int tiles = 0; // weight tiles of a workgroup, at most; 0: does not apply
+            int tiles_q = 0, tiles_r = 0, grid = 0, ranges = 0, range_groups = 0;
+            size_t partial_bytes = 0; // more than one range of K: their fp32 sums
+        };
+        // N: output columns (gate: from 2 N weight rows); more than one range of K: not with RMSNorm or SiLU-gate
+        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges)
+        {
+            KstreamPlan p;
+            const int mb = (M + 15) / 16, G = K >> 7;
+            if (M < 17 || mb > 4 || N < 16 || K < 1024 || (K & 127) || ranges < 1 || num_cu < ranges || (ranges > 1 && (gate || rms)))
+                return p;
+            const int rg = (G + ranges - 1) / ranges, n_tiles = (N + 15) / 16, per_range = num_cu / ranges;
+            const int grid = n_tiles < per_range ? n_tiles : per_range;
+            const int tiles = (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid);
+            // (a range's scales: rows of 32 words, from a half word where rows or ranges start in the middle of one)
+            if (rg > ((G & 1) || ranges > 1 ? KSTREAM_MAX_GROUPS - 2 : KSTREAM_MAX_GROUPS) || (ranges - 1) * rg >= G ||
+                ((G & 1) && ((N & 1) || (size_t)(gate ? 2 : 1) * N * G >= ((size_t)1 << 31))) || tiles > KSTREAM_MAX_TILES ||
+                kstream_lds_bytes(tiles, mb, rms) > LDS_BYTES_PER_CU)
+                return p;
+            p.tiles = tiles;
+            p.grid = grid;
+            p.tiles_q = n_tiles / grid;
+            p.tiles_r = n_tiles % grid;
+            p.ranges = ranges;
+            p.range_groups = rg;
+            p.partial_bytes = ranges > 1 ? (size_t)ranges * n_tiles * 16 * ((M + 3) & ~3) * sizeof(float) : 0;
+            return p;
+        }
+        // Microseconds x 100 of a launch, a fit of 245 measured products (20 .. 64 rows, N = 512 .. 16384, K = 1152 .. 11008, one to four ranges;
+        // the number of ranges it picks is within 3 % of the fastest but for six of them, 13 % at most): a chunk of eight groups takes what
+        // its loads and its unpacking take, a little less where fewer CUs fetch the activations; ranges of K pay for the sums' way through memory.
+        inline int kstream_estimate(const KstreamPlan& p, int mb)
+        {
+            const int chunks = (p.range_groups + KSTREAM_WAVES - 1) / KSTREAM_WAVES, workgroups = p.grid * p.ranges;
+            return chunks * (32 + 21 * mb + 33 * p.tiles) * (180 + (workgroups < 256 ? workgroups : 256)) / 436 + 187 + 29 * p.tiles +
+                   (p.ranges > 1 ? 46 + 12 * p.ranges + 63 * p.tiles : 0);
+        }
+        // What the library runs on it by itself, from measurements against the kernels that served these products before: 33 .. 64 rows
+        // everything that fits (against the tile GEMM: N = K = 4096 at 48 rows 13.8 -> 9.0 us, 12288 x 4096 21.0 -> 15.0, 4096 x 11008 20.5 -> 16.6,
+        // RMSNorm and SiLU-gate at 11008 x 4096 35.2 -> 22.4; against the row-streaming kernel up to K = 2048 1.2 - 1.9 x), 17 .. 32 rows all but more
+        // than four tiles a workgroup where the row-streaming kernel runs K as a compile-time constant (11008 x 4096 with both: 18.6 us
+        // there, 19.9 here) or over ranges (12288 x 11008: 25.1 us there, 26.8 here); with up to four 1.02 - 1.3 x, K = 5504 2.0 - 2.4 x.
+        // partial_bytes, sync_bytes: of scratch memory and synchronisation words (one per workgroup of a range) at hand
+        inline KstreamPlan kstream_choice(int M, int N, int K, int num_cu, bool gate, bool rms, size_t partial_bytes, size_t sync_bytes)
+        {
+            KstreamPlan best;
+            // (17 .. 32 rows: N = 320 .. 600 at K = 1024 takes 3.3 us there, 3.5 here; N = 256 .. 2400 at K = 11776 .. 12288 0.92 - 0.97 x, 4480 and more
+            // 1.06 - 1.16)
+            if (M < 17 || M > 64 || (M <= 32 && (K <= 1024 || (K > 11264 && N < 4096))))
+                return best;
+            for (int ranges = 1; ranges <= (gate || rms ? 1 : 4); ++ranges)
+            {
+                const KstreamPlan p = kstream_plan(M, N, K, num_cu, gate, rms, ranges);
+                if (p.tiles == 0 || (ranges > 1 && (p.partial_bytes > partial_bytes || p.grid * sizeof(unsigned) > sync_bytes)) || (M <= 32 && p.tiles > 4 && (ranges > 1 || w4a16_mrows_fixed_k(M, K))))
+                    continue;
+                if (best.tiles == 0 || kstream_estimate(p, (M + 15) / 16) < kstream_estimate(best, (M + 15) / 16))
+                    best = p;
+            }
+            return best;
+        }
         // ---- W8A8, one activation row: the row-streaming GEMV (w8a8_gemv_rows.hip) ----
         struct Q8RowsPlan
         {
@@ -1109,6 +1185,9 @@ namespace nnf
         {
             // NONE: the kernel family asked for cannot serve the shape
             enum Kind { NONE, ROWS, MROWS, SKINNY, MROWS_SPLIT, SKINNY_SPLIT, TILE } kind = NONE;
+            // the caller fixed nothing: the launch may run on the K-streaming kernel instead, within the scratch memory that `kind` asks for
+            // (w4a16_launch_kstream; the size queries and checks stay those of `kind`)
+            bool free_choice = false;
             int ksplits = 0;          // *_SPLIT: ranges of K (fp32 partial sums, then the reduction pass)
             bool normalised_copy = false; // RMSNorm as a pass that writes the normalised activations (MFMA GEMV kernels, and what
                                           // the row-streaming kernel took over from other kernels)
@@ -1126,8 +1205,8 @@ namespace nnf
         // (values of nnf_w4a16_variant), 3 the tile GEMM with tile_rows / k_parts (0: its own plan).
         // room_for_copy = false: the caller's scratch memory does not hold the normalised activations of the products that the
         // row-streaming kernel took over from others: they run where they ran (see route_w4a16_within).
-        inline W4A16Route route_w4a16(int M, int N, int K, bool gate, bool rms, bool in_place_residual, int num_cu, int path = 0,
-                                      int tile_rows = 0, int k_parts = 0, int tile_cols = 0, bool room_for_copy = true)
+        inline W4A16Route route_w4a16_other(int M, int N, int K, bool gate, bool rms, bool in_place_residual, int num_cu, int path,
+                                            int tile_rows, int k_parts, int tile_cols, bool room_for_copy)
         {
             W4A16Route r;
             if (M <= 0 || N <= 0 || K < 128 || (K & 127) || num_cu < 1)
@@ -1194,6 +1273,20 @@ namespace nnf
             r.partial_bytes = r.plan.bytes();
             r.rms_bytes = rstd_bytes;
             return r;
+        }
+
+        inline W4A16Route route_w4a16(int M, int N, int K, bool gate, bool rms, bool in_place_residual, int num_cu, int path = 0,
+                                      int tile_rows = 0, int k_parts = 0, int tile_cols = 0, bool room_for_copy = true)
+        {
+            W4A16Route r =
+                route_w4a16_other(M, N, K, gate, rms, in_place_residual, num_cu, path, tile_rows, k_parts, tile_cols, room_for_copy);
+            r.free_choice = path == 0 && tile_rows == 0 && k_parts == 0 && tile_cols == 0;
+            return r;
+        }
+        // the plan of the launch on the K-streaming kernel, or one of no tiles: not there.  sync_bytes: of synchronisation words (0: none)
+        inline KstreamPlan w4a16_launch_kstream(const W4A16Route& r, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes)
+        {
+            return r.free_choice && r.kind != W4A16Route::NONE ? kstream_choice(M, N, K, num_cu, gate, rms, r.partial_bytes, sync_bytes) : KstreamPlan();
         }
 
         // The route of a call that brings `bytes` of scratch memory.  What the size queries ask for covers the normalised activations

@@ -1,0 +1,107 @@
+"""The K-streaming MFMA kernel: fp16 x int4 products of 17 .. 64 rows (w4a16_kstream.hip).
+
+Sizes at its edges: rows around the blocks of 16, one column tile up to six a workgroup, columns that are no multiple of 16 (the
+last tile is moved back), a single group for the last chunk, an odd number of groups (scale rows that start in the middle of
+a word), all 64 groups of the longest range, ranges of K that end unevenly.  Every product also runs without
+synchronisation words (one range of K, or the kernel that served it before).
+Tolerance: fp16 results of fp32 sums, 1e-2 of the result's RMS as for the other kernels (measured: 2e-3 at most).
+"""
+import numpy as np
+import pytest
+
+import oracle
+from nnfusion_amd import datagen
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-2
+
+
+def _t(gpu, *arrays):
+    import torch
+
+    return [None if a is None else torch.from_numpy(np.ascontiguousarray(a)).to(gpu) for a in arrays]
+
+
+def _check(y, ref, tol=TOL):
+    y = y.cpu().numpy().astype(np.float32)
+    assert np.isfinite(y).all()
+    err = float(np.abs(y - ref.astype(np.float32)).max())
+    rms = float(np.sqrt(np.mean(np.asarray(ref, np.float64) ** 2)))
+    assert err <= tol * max(rms, 1e-6), (err, rms)
+
+
+def _ws(gpu, nbytes=64 << 20):
+    import torch
+
+    return torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (17, 16, 1152), (32, 48, 2176), (33, 40, 1152), (48, 4096, 1024), (49, 520, 4096), (64, 4112, 1280), (64, 24576, 1024), (63, 300, 8192),
+    (45, 8200, 2048), (20, 12288, 1280), (40, 640, 11008), (33, 4096, 11008), (64, 1030, 9984), (29, 256, 8448), (50, 2048, 1664)])
+@pytest.mark.parametrize("with_sync", [True, False], ids=["sync", "no-sync"])
+def test_products(gpu, m, n, k, with_sync):
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case kstream M={m} N={n} K={k} sync={with_sync}", flush=True)
+    a, wq, s = datagen.w4a16_case(3, m, n, k)
+    ta, tw, ts = _t(gpu, a, wq, s)
+    sync = ops.sync_flags(gpu) if with_sync else None
+    ws = _ws(gpu)
+    ref = oracle.w4a16_gemm(a, wq, s, f32_out=True)
+    y = ops.wna16_gemm(ta, tw, ts, workspace=ws, sync=sync)
+    _check(y, ref)
+    again = ops.wna16_gemm(ta, tw, ts, workspace=ws, sync=sync)
+    torch.cuda.synchronize()
+    assert torch.equal(y, again)
+    assert sync is None or int(sync.count_nonzero()) == 0
+
+
+@pytest.mark.parametrize("zp", [0, 15])
+def test_zero_points(gpu, zp):
+    from nnfusion_amd import ops
+
+    a, wq, s = datagen.w4a16_case(5, 45, 200, 2304)
+    ta, tw, ts = _t(gpu, a, wq, s)
+    _check(ops.w4a16_gemm(ta, tw, ts, zp=zp, workspace=_ws(gpu)), oracle.w4a16_gemm(a, wq, s, zp=zp, f32_out=True))
+
+
+@pytest.mark.parametrize("m,n,k", [(45, 200, 1152), (64, 4128, 2048), (31, 72, 4096), (48, 1024, 9216)])
+def test_bias_and_residual_in_place(gpu, m, n, k):
+    from nnfusion_amd import ops
+
+    a, wq, s = datagen.w4a16_case(7, m, n, k)
+    rng = np.random.default_rng(1)
+    bias = rng.standard_normal(n).astype(np.float16)
+    resid = rng.standard_normal((m, n)).astype(np.float16)
+    ta, tw, ts, tb, out = _t(gpu, a, wq, s, bias, resid)
+    ops.w4a16_gemm_fused(ta, tw, ts, bias=tb, residual=out, out=out, workspace=_ws(gpu), sync=ops.sync_flags(gpu))
+    ref = oracle.add_f16(oracle.add_f16(oracle.w4a16_gemm(a, wq, s), np.broadcast_to(bias, (m, n))), resid)
+    _check(out, ref)
+
+
+@pytest.mark.parametrize("gate", [False, True], ids=["plain", "silu-gate"])
+@pytest.mark.parametrize("m,n,k,spread", [(45, 300, 1152, 1.0), (64, 8200, 1024, 1.0), (33, 2048, 8192, 1.0), (20, 40, 2176, 1.0), (48, 512, 2048, 3000.0)])
+def test_rms_norm(gpu, m, n, k, spread, gate):
+    """spread: of the RMSNorm weight.  At 3000 neither gamma times an activation (up to 80) nor gamma times a weight of 15 is an fp16 number."""
+    from nnfusion_amd import ops
+
+    a, wq, s = datagen.w4a16_case(9, m, 2 * n if gate else n, k)
+    if spread > 1:
+        a, s = (a.astype(np.float32) * 20).astype(np.float16), (s.astype(np.float32) / spread).astype(np.float16)
+    gamma = (spread * (1.0 + 0.1 * np.random.default_rng(2).standard_normal(k))).astype(np.float16)
+    ta, tw, ts, tg = _t(gpu, a, wq, s, gamma)
+    y = ops.w4a16_gemm_fused(ta, tw, ts, rms_gamma=tg, act=1 if gate else 0, workspace=_ws(gpu), sync=ops.sync_flags(gpu))
+    x = a.astype(np.float64)
+    x = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * gamma.astype(np.float64)
+    ref = x @ oracle.dequantize_w4(wq, s).astype(np.float64).T
+    if gate:
+        g, u = ref[:, :n], ref[:, n:]
+        ref = g / (1.0 + np.exp(-g)) * u
+        # the gate and up products are rounded to fp16 and multiplied: twice the relative error of one, on a result with heavier tails
+        _check(y, ref, 2 * TOL)
+    else:
+        _check(y, ref)

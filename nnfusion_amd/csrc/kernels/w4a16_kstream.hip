@@ -1,20 +1,24 @@
-// fp16 x int4 (g128) for 33 .. 64 activation rows: all tiles of a workgroup side by side, K in chunks.
+// fp16 x int4 (g128) for 2 .. 64 activation rows: all tiles of a workgroup side by side, K in chunks.
 //
 //   Y[M,N] = A[M,K] . ((Wq - zp) * S)^T
 //
 // Replaces the cublasHgemm call of cuda::Dot (src/nnfusion/core/kernels/cuda_gpu/kernels/dot.cpp:271-363) for a
-// weight-quantized Dot node with more activation rows than the row-streaming kernels (w4a16_mrows.hip) keep in registers
-// and fewer than fill the tiles of the tile GEMM (w4a16_gemm_sk.h).
+// weight-quantized Dot node with a few activation rows, where it is ahead of the row-streaming kernels (w4a16_mrows.hip), which keep
+// the activations of all of K in registers, and of the tile GEMM (w4a16_gemm_sk.h): workspace::kstream_choice.
 //
 //   * One workgroup of eight wavefronts per CU owns up to T 16-row weight tiles and keeps the fp32 sums of all of them in
 //     registers (T x MB accumulators of 16 x 16, MB blocks of 16 activation rows).  K is walked in chunks of eight groups
 //     of 128, wavefront w the group w of each: a wavefront sums its own groups, nothing but its own loads feeds its MFMAs,
 //     and there is no barrier between the first load and the last.  The eight wavefronts' sums meet in LDS once, at the end.
-//   * What bounds it is the activations: every CU fetches all M x K of them from its L2 (48 x 4096: 384 KiB against 96 KiB of
-//     weights with three tiles), so they are asked for as whole 128-byte lines, global -> LDS without registers, through a
-//     ring of RB blocks (16 rows x 256 bytes) per wavefront that is refilled block by block as the blocks are copied into
-//     operand registers: 96 KiB of them in flight per CU next to T KiB of weights per wavefront.  The unpacking and the
-//     MFMAs of a chunk run below that.
+//   * With 33 .. 64 rows what bounds it is the activations: every CU fetches all M x K of them from its L2 (48 x 4096: 384 KiB against
+//     96 KiB of weights with three tiles), and of the 3500 cycles of a chunk (1.9 GHz) the load issue, the way of the activations through
+//     LDS and the unpacking take about 2000 each.  They are asked for as whole 128-byte lines, global -> LDS without registers, through a
+//     ring of RB blocks (16 rows x 256 bytes) per wavefront that is refilled block by block as the blocks are copied into operand
+//     registers.  45 x 12288 x 4096: 14.1 us (21.6 on the tile GEMM); with up to 16 rows HBM and the latency of the first chunk bound it:
+//     16 x 12288 x 2560 7.4 us (10.4 on the row-streaming kernel), 8 x 4096 x 2560 3.9 (5.2).
+//     Measured level or slower: the chunks in another order on each CU of an XCD (14.9 at 45 rows); the weights through registers and an
+//     LDS write (14.5); the next chunk's loads one at a time between the MFMAs (14.5); two or three chunks ahead
+//     (8 - 15 % slower with two and more tiles; with one tile and up to 16 rows two chunks are 4 - 10 % faster: D).
 //   * The weights of a lane (32 of one row and group) are unpacked to the exact integers q - zp in fp16 (the nibble in the
 //     mantissa of 1024.0 or 64.0, minus 1024 + zp or 64 + zp) once per chunk and meet MB blocks of rows; the group's sum times its scale
 //     joins the accumulator in fp32.
@@ -55,10 +59,12 @@ namespace nnf
                                                                           int K, int tiles, int pack, float* __restrict__ partial,
                                                                           uint32_t* sync, GemvFusionArgs f)
     {
-        static_assert(T >= 1 && MB >= 2 && MB <= 4, "");
-        constexpr int RB = workspace::kstream_ring(MB); // blocks of activations in a wavefront's ring
-        static_assert(RB <= MB, "");
-        constexpr int NG = RMS ? 1 : 0;
+        static_assert(T >= 1 && MB >= 1 && MB <= 4, "");
+        constexpr int D = workspace::kstream_depth(T, MB); // chunks asked for ahead
+        constexpr int RB = workspace::kstream_ring(MB);    // blocks of activations in a slot of a wavefront's ring
+        static_assert(RB == MB || (RB < MB && D == 1), "");
+        constexpr int NG = RMS ? 1 : 0, L = NG + 4 * MB + T; // loads of a chunk
+        constexpr int SLOT = RB * ROW_BLOCK_BYTES + T * 1024 + NG * 256;
         constexpr int WAVE_BYTES = workspace::kstream_wave_bytes(T, MB, RMS);
         constexpr int RT = workspace::kstream_round(T, MB); // tiles whose sums are in LDS at a time
         extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -91,9 +97,7 @@ namespace nnf
         const int g_lo = (int)blockIdx.y * range_groups, g_hi = min(G, g_lo + range_groups); // this workgroup's part of K
         const int Gr = g_hi - g_lo;
 
-        uint8_t* a_ring = smem + wave * WAVE_BYTES;
-        uint8_t* w_slots = a_ring + RB * ROW_BLOCK_BYTES;
-        uint8_t* g_slot = w_slots + T * 1024;
+        uint8_t* ring = smem + wave * WAVE_BYTES;
         uint8_t* sc = smem + KS_WAVES * WAVE_BYTES;
 
         // ---- the scales of the range: asked for first, into LDS as rows of 32 words ---------------------------------------
@@ -120,8 +124,8 @@ namespace nnf
 #pragma unroll
         for (int t = 0; t < T; ++t)
             w_row[t] = Wq + (size_t)row0_of(t) * (size_t)ROW_BYTES;
-        auto fetch_w = [&](int g, int t) {
-            __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(w_row[t] + (uint32_t)g * 64u + w_off), (ks_lds_ptr_t)(w_slots + t * 1024), 16,
+        auto fetch_w = [&](int g, int t, uint8_t* to) {
+            __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(w_row[t] + (uint32_t)g * 64u + w_off), (ks_lds_ptr_t)(to + RB * ROW_BLOCK_BYTES + t * 1024), 16,
                                              0, 0);
         };
         // activations: as row_block_fetch (nnf_device.h); rows past M (in the last block only): the last row again
@@ -134,30 +138,34 @@ namespace nnf
             a_off[c] = (uint32_t)r * (uint32_t)(K * 2) + piece;
             a_off_last[c] = (uint32_t)min(r, M - 1 - (MB - 1) * 16) * (uint32_t)(K * 2) + piece;
         }
-        auto fetch_a = [&](int g, int mb, int slot) {
+        auto fetch_a = [&](int g, int mb, uint8_t* to) {
             const uint8_t* base = reinterpret_cast<const uint8_t*>(A) + (size_t)(mb * 16) * (size_t)(K * 2) + (size_t)g * 256;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
                 __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(base + (mb == MB - 1 ? a_off_last[c] : a_off[c])),
-                                                 (ks_lds_ptr_t)(a_ring + slot * ROW_BLOCK_BYTES + c * 1024), 16, 0, 0);
+                                                 (ks_lds_ptr_t)(to + c * 1024), 16, 0, 0);
         };
-        auto fetch_gamma = [&](int g) {
+        auto fetch_gamma = [&](int g, uint8_t* to) {
             if constexpr (RMS)
                 __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(reinterpret_cast<const uint8_t*>(f.gamma) + (size_t)g * 256 + lane * 4),
-                                                 (ks_lds_ptr_t)g_slot, 4, 0, 0);
+                                                 (ks_lds_ptr_t)(to + RB * ROW_BLOCK_BYTES + T * 1024), 4, 0, 0);
         };
 
         // groups of this wavefront: g_lo + wave + 8 c
         const int chunks = (Gr - wave + KS_WAVES - 1) / KS_WAVES;
         auto group_of = [&](int c) { return min(g_lo + wave + c * KS_WAVES, g_hi - 1); };
-        fetch_gamma(group_of(0));
 #pragma unroll
-        for (int p = 0; p < RB; ++p)
-            fetch_a(group_of(0), p, p);
+        for (int d = 0; d < D; ++d)
+        {
+            fetch_gamma(group_of(d), ring + d * SLOT);
 #pragma unroll
-        for (int t = 0; t < T; ++t)
-            fetch_w(group_of(0), t);
-        wait_loads<NG + 4 * RB + T>(); // the scales
+            for (int p = 0; p < RB; ++p)
+                fetch_a(group_of(d), p, ring + d * SLOT + p * ROW_BLOCK_BYTES);
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                fetch_w(group_of(d), t, ring + d * SLOT);
+        }
+        wait_loads<D*(NG + 4 * RB + T)>(); // the scales
         lds_barrier();
 
         const half_t clo = (half_t)(-(1024.0f + (float)zp)), chi = (half_t)(-(64.0f + (float)zp)); // exact
@@ -181,51 +189,56 @@ namespace nnf
         const uint32_t w_rd = (uint32_t)(col * 64 + ((kq ^ (col >> 2)) << 4));
         const int sc_first = ((col * G + g_lo) & 1) + wave; // place of the wavefront's first scale in row col (row0_of() * G is even)
 
-        // Loads of a wavefront in order: chunk by chunk [gamma] [MB blocks of activations] [T tiles of weights]; gamma, the
-        // first RB blocks and the weights of a chunk are asked for during the chunk before it, each where its slot has just been
-        // read.  Loads come back in order: the wait counts below are the loads that follow the one waited for (LAST: nothing of a
-        // next chunk is asked for).  Weights asked for ahead of the chunk's last activations (RB < MB) need no wait of their own.
-        int slot = 0; // of the ring: block p sits in slot p % RB
-        auto chunk = [&](int c, auto last) {
-            constexpr bool LAST = decltype(last)::value;
-            const int g = group_of(c), gn = group_of(c + 1);
+        // Loads of a wavefront in order: chunk by chunk [gamma] [MB blocks of activations] [T tiles of weights]; those of chunk c + D
+        // (RB < MB: of the activations, the first RB blocks) are asked for during chunk c, each where its slot has just been
+        // read.  Loads come back in order: the wait counts below are the loads that follow the one waited for.  AHEAD: the chunks still to come,
+        // as far as they matter: below D nothing more is asked for.  Weights asked for ahead of the chunk's last activations
+        // (RB < MB) need no wait of their own.
+        int block = 0;                 // RB < MB: block p of the activations sits in place p % RB
+        uint8_t* at_slot = ring;       // chunk c: slot c % D
+        auto chunk = [&](int c, auto ahead) {
+            constexpr int AHEAD = decltype(ahead)::value;
+            constexpr bool FULL = AHEAD == D;
+            constexpr int LATER = FULL ? (D - 1) * L : AHEAD * L; // of later chunks, asked for before this one began
+            const int g = group_of(c), gn = group_of(c + D);
+            const uint8_t* slot = at_slot;
             uintx4 gm[4];
             if constexpr (RMS)
             {
-                wait_loads<4 * RB + T>();
+                wait_loads<LATER + 4 * RB + T>();
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
                     const half2_t sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
-                    const uintx4 g8 = permute_a8(*reinterpret_cast<const uintx4*>(g_slot + kq * 64 + j * 16));
+                    const uintx4 g8 = permute_a8(*reinterpret_cast<const uintx4*>(slot + RB * ROW_BLOCK_BYTES + T * 1024 + kq * 64 + j * 16));
                     gm[j] = uintx4{as_u32(as_half2(g8.x) * sixteenth), as_u32(as_half2(g8.y) * sixteenth), as_u32(as_half2(g8.z) * sixteenth),
                                    as_u32(as_half2(g8.w) * sixteenth)};
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                if constexpr (!LAST)
-                    fetch_gamma(gn);
+                if constexpr (FULL)
+                    fetch_gamma(gn, at_slot);
             }
             uintx4 areg[MB][4];
             unroll_for<0, MB>([&](auto p_c) {
                 constexpr int p = decltype(p_c)::value;
-                if constexpr (LAST)
-                {
-                    constexpr int fetched = p < MB - RB ? p : MB - RB; // blocks asked for in this chunk so far
-                    wait_loads<(p < RB ? 4 * (RB - 1 - p) + T + 4 * fetched : 4 * (p - 1 + RB < MB ? RB - 1 : MB - 1 - p))>();
-                }
+                if constexpr (FULL)
+                    wait_loads<LATER + 4 * (RB - 1) + (p < RB ? T + NG : 0)>();
                 else
-                    wait_loads<4 * (RB - 1) + (p < RB ? T + NG : 0)>();
-                const int at = RB == MB ? p : slot;
+                {
+                    constexpr int fetched = p < MB - RB ? p : MB - RB; // RB < MB: blocks asked for in this chunk so far
+                    wait_loads<(p < RB ? LATER + 4 * (RB - 1 - p) + T + 4 * fetched : 4 * (p - 1 + RB < MB ? RB - 1 : MB - 1 - p))>();
+                }
+                uint8_t* at = at_slot + (RB == MB ? p : block) * ROW_BLOCK_BYTES;
                 uintx4 a[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    a[j] = *reinterpret_cast<const uintx4*>(a_ring + at * ROW_BLOCK_BYTES + a_rd[j]);
+                    a[j] = *reinterpret_cast<const uintx4*>(at + a_rd[j]);
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the slot has been read before it is refilled
                 if constexpr (p + RB < MB)
                     fetch_a(g, p + RB, at);
-                else if constexpr (!LAST)
+                else if constexpr (FULL)
                     fetch_a(gn, p + RB - MB, at);
-                slot = slot + 1 == RB ? 0 : slot + 1;
+                block = block + 1 == RB ? 0 : block + 1;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
@@ -247,8 +260,8 @@ namespace nnf
             auto read_w = [&](auto t_c) {
                 constexpr int t = decltype(t_c)::value;
                 if constexpr (RB == MB)
-                    wait_loads<LAST ? T - 1 - t : T - 1 + 4 * MB + NG>();
-                wnext = *reinterpret_cast<const uintx4*>(w_slots + t * 1024 + w_rd);
+                    wait_loads<FULL ? D * L - 1 : LATER + T - 1 - t>();
+                wnext = *reinterpret_cast<const uintx4*>(slot + RB * ROW_BLOCK_BYTES + t * 1024 + w_rd);
                 snext = *reinterpret_cast<const half_t*>(sc_rd + t * 2048);
             };
             read_w(std::integral_constant<int, 0>());
@@ -258,8 +271,8 @@ namespace nnf
                 __builtin_amdgcn_sched_barrier(0);
                 const uintx4 wv = wnext;
                 const float scale = (float)snext;
-                if constexpr (!LAST)
-                    fetch_w(gn, t);
+                if constexpr (FULL)
+                    fetch_w(gn, t, at_slot);
                 if constexpr (t + 1 < T)
                     read_w(std::integral_constant<int, (t + 1 < T ? t + 1 : 0)>());
                 floatx4 sum[MB];
@@ -297,11 +310,17 @@ namespace nnf
                     acc[t][mb].w = __builtin_fmaf(sum[mb].w, scale, acc[t][mb].w);
                 }
             });
+            if constexpr (D > 1)
+                at_slot = at_slot == ring + (D - 1) * SLOT ? ring : at_slot + SLOT;
         };
-        for (int c = 0; c < chunks - 1; ++c)
-            chunk(c, std::false_type());
-        if (chunks > 0)
-            chunk(chunks - 1, std::true_type());
+        int c = 0;
+        for (; c < chunks - D; ++c)
+            chunk(c, std::integral_constant<int, D>());
+        unroll_for<0, D>([&](auto i) { // the last D chunks, of which the last one has none ahead (fewer in all: nothing is waited for too little)
+            constexpr int AHEAD = D - 1 - decltype(i)::value;
+            if (c + AHEAD < chunks)
+                chunk(c++, std::integral_constant<int, AHEAD>());
+        });
         wait_loads<0>(); // (a wavefront without a group of its own has asked for one all the same)
         __syncthreads();
 
@@ -503,6 +522,7 @@ namespace nnf
             return hipErrorInvalidValue;
         switch ((M + 15) / 16)
         {
+        case 1: return launch_kstream_t<1>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
         case 2: return launch_kstream_t<2>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
         case 3: return launch_kstream_t<3>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
         case 4: return launch_kstream_t<4>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);

@@ -1051,9 +1051,13 @@ namespace nnf
         // ---- 33 .. 64 activation rows: the K-streaming kernel (w4a16_kstream.hip) ----
         // One workgroup per CU with up to KSTREAM_MAX_TILES 16-row weight tiles, their sums in registers; K in chunks of eight groups.
         constexpr int KSTREAM_WAVES = 8, KSTREAM_MAX_TILES = 6, KSTREAM_MAX_GROUPS = 64;
-        // blocks of 16 rows x 256 bytes of activations in a wavefront's ring; its bytes of LDS
+        // chunks asked for ahead; blocks of 16 rows x 256 bytes of activations in a slot of a wavefront's ring; its bytes of LDS
+        constexpr int kstream_depth(int tiles, int mb) { return tiles == 1 && mb == 1 ? 2 : 1; }
         constexpr int kstream_ring(int mb) { return mb < 4 ? mb : 3; }
-        constexpr int kstream_wave_bytes(int tiles, int mb, bool rms) { return kstream_ring(mb) * 4096 + tiles * 1024 + (rms ? 256 : 0); }
+        constexpr int kstream_wave_bytes(int tiles, int mb, bool rms)
+        {
+            return kstream_depth(tiles, mb) * (kstream_ring(mb) * 4096 + tiles * 1024 + (rms ? 256 : 0));
+        }
         // tiles whose eight partial sums are in LDS at a time (an even number where there is more than one round)
         constexpr int kstream_round(int tiles, int mb) { return mb == 4 && tiles > 4 ? 4 : tiles; }
         constexpr size_t kstream_lds_bytes(int tiles, int mb, bool rms)
@@ -1073,7 +1077,7 @@ namespace nnf
         {
             KstreamPlan p;
             const int mb = (M + 15) / 16, G = K >> 7;
-            if (M < 17 || mb > 4 || N < 16 || K < 1024 || (K & 127) || ranges < 1 || num_cu < ranges || (ranges > 1 && (gate || rms)))
+            if (M < 2 || mb > 4 || N < 16 || K < 1024 || (K & 127) || ranges < 1 || num_cu < ranges || (ranges > 1 && (gate || rms)))
                 return p;
             const int rg = (G + ranges - 1) / ranges, n_tiles = (N + 15) / 16, per_range = num_cu / ranges;
             const int grid = n_tiles < per_range ? n_tiles : per_range;
@@ -1110,14 +1114,21 @@ namespace nnf
         inline KstreamPlan kstream_choice(int M, int N, int K, int num_cu, bool gate, bool rms, size_t partial_bytes, size_t sync_bytes)
         {
             KstreamPlan best;
+            const bool fixed_k = w4a16_mrows_fixed_k(M, K);
             // (17 .. 32 rows: N = 320 .. 600 at K = 1024 takes 3.3 us there, 3.5 here; N = 256 .. 2400 at K = 11776 .. 12288 0.92 - 0.97 x, 4480 and more
             // 1.06 - 1.16)
-            if (M < 17 || M > 64 || (M <= 32 && (K <= 1024 || (K > 11264 && N < 4096))))
+            if (M < 2 || M > 64 || (M > 16 && M <= 32 && (K <= 1024 || (K > 11264 && N < 4096))))
+                return best;
+            // 2 .. 16 rows, against the row-streaming kernel and the MFMA GEMV (time there / here, 1320 products).  K that is a compile-time constant
+            // of the row-streaming kernel stays there (SiLU-gate 0.85 - 1.08, others 0.91 - 1.25, most within 8 %); with any other K RMSNorm and SiLU-gate,
+            // which cost passes of their own there, 1.03 - 2.4; plain products from eight rows on 1.0 - 1.6 (0.94 - 1.0 for K = 1152 .. 1536 at 8 and 9 rows in
+            // one tile a workgroup), of fewer rows 0.94 - 1.3: left where they are, like K above 8192, 0.9 - 1.1 over ranges.
+            if (M <= 16 && (fixed_k || K > 8192 || (!gate && !rms && (M < 8 || (K < 1664 && M <= 9 && N <= 4096)))))
                 return best;
             for (int ranges = 1; ranges <= (gate || rms ? 1 : 4); ++ranges)
             {
                 const KstreamPlan p = kstream_plan(M, N, K, num_cu, gate, rms, ranges);
-                if (p.tiles == 0 || (ranges > 1 && (p.partial_bytes > partial_bytes || p.grid * sizeof(unsigned) > sync_bytes)) || (M <= 32 && p.tiles > 4 && (ranges > 1 || w4a16_mrows_fixed_k(M, K))))
+                if (p.tiles == 0 || (ranges > 1 && (p.partial_bytes > partial_bytes || p.grid * sizeof(unsigned) > sync_bytes)) || (M <= 32 && p.tiles > 4 && (ranges > 1 || fixed_k)) || (M <= 16 && ranges > 1))
                     continue;
                 if (best.tiles == 0 || kstream_estimate(p, (M + 15) / 16) < kstream_estimate(best, (M + 15) / 16))
                     best = p;

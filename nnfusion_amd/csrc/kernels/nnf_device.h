@@ -95,7 +95,7 @@ namespace nnf
     // f(integral_constant<int, I>) for I = BEGIN .. END-1: for bodies that need I as a compile-time constant
     // (instruction offsets, wait counts)
     template <int BEGIN, int END, class F>
-    __device__ __forceinline__ void unroll_for(F&& f)
+    __host__ __device__ __forceinline__ void unroll_for(F&& f)
     {
         if constexpr (BEGIN < END)
         {

@@ -48,8 +48,9 @@ namespace nnf
         }
     } // namespace
 
-    // pack = M | zp << 8 | gate << 16 | range_groups << 17; tiles = tiles_q | tiles_r << 16: output tiles of a workgroup, one
-    // more for the first tiles_r (gate: twice as many weight tiles, the gate and the up tile of each in turn).  M > 16 (MB - 1).
+    // blockIdx.z: blocks of 16 MB activation rows.
+    // pack = M | zp << 13 | gate << 17 | range_groups << 18; tiles = tiles_q | tiles_r << 16: output tiles of a workgroup, one
+    // more for the first tiles_r (gate: twice as many weight tiles, the gate and the up tile of each in turn).
     // LDS (bytes): per wavefront [RB][4096] activations | [T][1024] weights | (RMS) 256 gamma; then the scales of the
     //              workgroup's range of K, [T][16][32] words.  At the end, over all of it: (RMS) the wavefronts' sums of squares
     //              [8][16 MB] and rstd[16 MB] | from byte 4096 on the wavefronts' sums [8][tiles of a round][MB KiB].
@@ -79,9 +80,15 @@ namespace nnf
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int col = lane & 15; // n within the tile (B operand / D column), m for the A operand
         const int kq = lane >> 4;  // K quarter of the MFMA operands, row quad of D
-        const int M = pack & 0xff, zp = (pack >> 8) & 0xff, gate = (pack >> 16) & 1, range_groups = (int)((unsigned)pack >> 17);
+        const int M_all = pack & 0x1fff, zp = (pack >> 13) & 0xf, gate = (pack >> 17) & 1, range_groups = (int)((unsigned)pack >> 18);
         const int tiles_q = tiles & 0xffff, tiles_r = (int)((unsigned)tiles >> 16);
         const int G = K >> 7, ROW_BYTES = K >> 1;
+        // rows first_row .. first_row + M - 1 of the activations, as a product of its own
+        const int first_row = (int)blockIdx.z * (MB * 16), M = min(M_all - first_row, MB * 16);
+        A += (size_t)first_row * K;
+        Y += (size_t)first_row * N;
+        if (f.residual)
+            f.residual += (size_t)first_row * N;
         const int b = blockIdx.x;
         const int t0 = b * tiles_q + min(b, tiles_r);
         const int T_out = tiles_q + (b < tiles_r ? 1 : 0);
@@ -128,7 +135,8 @@ namespace nnf
             __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(w_row[t] + (uint32_t)g * 64u + w_off), (ks_lds_ptr_t)(to + RB * ROW_BLOCK_BYTES + t * 1024), 16,
                                              0, 0);
         };
-        // activations: as row_block_fetch (nnf_device.h); rows past M (in the last block only): the last row again
+        // activations: as row_block_fetch (nnf_device.h); rows past M: the last row again, blocks past its block: that block again
+        const int last_block = (M - 1) >> 4;
         uint32_t a_off[4], a_off_last[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c)
@@ -136,13 +144,13 @@ namespace nnf
             const int r = c * 4 + (lane >> 4);
             const uint32_t piece = (uint32_t)(((lane & 15) ^ r) * 16);
             a_off[c] = (uint32_t)r * (uint32_t)(K * 2) + piece;
-            a_off_last[c] = (uint32_t)min(r, M - 1 - (MB - 1) * 16) * (uint32_t)(K * 2) + piece;
+            a_off_last[c] = (uint32_t)min(r, M - 1 - last_block * 16) * (uint32_t)(K * 2) + piece;
         }
         auto fetch_a = [&](int g, int mb, uint8_t* to) {
-            const uint8_t* base = reinterpret_cast<const uint8_t*>(A) + (size_t)(mb * 16) * (size_t)(K * 2) + (size_t)g * 256;
+            const uint8_t* base = reinterpret_cast<const uint8_t*>(A) + (size_t)(min(mb, last_block) * 16) * (size_t)(K * 2) + (size_t)g * 256;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(base + (mb == MB - 1 ? a_off_last[c] : a_off[c])),
+                __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(base + (mb >= last_block ? a_off_last[c] : a_off[c])),
                                                  (ks_lds_ptr_t)(to + c * 1024), 16, 0, 0);
         };
         auto fetch_gamma = [&](int g, uint8_t* to) {
@@ -218,8 +226,10 @@ namespace nnf
                 if constexpr (FULL)
                     fetch_gamma(gn, at_slot);
             }
-            uintx4 areg[MB][4];
-            unroll_for<0, MB>([&](auto p_c) {
+            const int sc_place = sc_first + c * KS_WAVES;
+            const uint8_t* sc_rd = sc + (uint32_t)(col * 128 + ((((sc_place >> 1) ^ (2 * col)) & 31) << 2) + (sc_place & 1) * 2);
+            // block p of the chunk's activations from its place in the ring, in operand order; the place is refilled
+            auto read_a = [&](auto p_c, uintx4(&a)[4]) {
                 constexpr int p = decltype(p_c)::value;
                 if constexpr (FULL)
                     wait_loads<LATER + 4 * (RB - 1) + (p < RB ? T + NG : 0)>();
@@ -229,7 +239,6 @@ namespace nnf
                     wait_loads<(p < RB ? LATER + 4 * (RB - 1 - p) + T + 4 * fetched : 4 * (p - 1 + RB < MB ? RB - 1 : MB - 1 - p))>();
                 }
                 uint8_t* at = at_slot + (RB == MB ? p : block) * ROW_BLOCK_BYTES;
-                uintx4 a[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     a[j] = *reinterpret_cast<const uintx4*>(at + a_rd[j]);
@@ -243,7 +252,6 @@ namespace nnf
                 for (int j = 0; j < 4; ++j)
                 {
                     a[j] = permute_a8(a[j]);
-                    areg[p][j] = a[j];
                     if constexpr (RMS)
                     {
                         ss[p] = dot2(as_half2(a[j].x), as_half2(a[j].x), ss[p]);
@@ -252,15 +260,41 @@ namespace nnf
                         ss[p] = dot2(as_half2(a[j].w), as_half2(a[j].w), ss[p]);
                     }
                 }
-            });
-            const int sc_place = sc_first + c * KS_WAVES;
-            const uint8_t* sc_rd = sc + (uint32_t)(col * 128 + ((((sc_place >> 1) ^ (2 * col)) & 31) << 2) + (sc_place & 1) * 2);
+            };
+            auto wait_w = [&](auto t_c) {
+                constexpr int t = decltype(t_c)::value;
+                if constexpr (RB == MB)
+                    wait_loads<FULL ? D * L - 1 : LATER + T - 1 - t>();
+            };
+            // weights 8 j .. 8 j + 7 of a lane's 32: exact integers q - zp (times gamma / 16)
+            auto unpack = [&](uint32_t w4, int j) {
+                const uint32_t w8 = w4 >> 8;
+                half2_t q0 = as_half2((w4 & MASK_LO) | MAGIC) + c_lo;    // (q0, q4) - zp
+                half2_t q1 = as_half2((w4 & MASK_HI) | MAGIC_HI) + c_hi; // (q1, q5) - zp
+                half2_t q2 = as_half2((w8 & MASK_LO) | MAGIC) + c_lo;    // (q2, q6) - zp
+                half2_t q3 = as_half2((w8 & MASK_HI) | MAGIC_HI) + c_hi; // (q3, q7) - zp
+                if constexpr (RMS)
+                {
+                    q0 *= as_half2(gm[j].x);
+                    q1 *= as_half2(gm[j].y);
+                    q2 *= as_half2(gm[j].z);
+                    q3 *= as_half2(gm[j].w);
+                }
+                return uintx4{as_u32(q0), as_u32(q1), as_u32(q2), as_u32(q3)};
+            };
+            auto add_scaled = [](floatx4& to, const floatx4& sum, float scale) {
+                to.x = __builtin_fmaf(sum.x, scale, to.x);
+                to.y = __builtin_fmaf(sum.y, scale, to.y);
+                to.z = __builtin_fmaf(sum.z, scale, to.z);
+                to.w = __builtin_fmaf(sum.w, scale, to.w);
+            };
+            uintx4 areg[MB][4];
+            unroll_for<0, MB>([&](auto p_c) { read_a(p_c, areg[decltype(p_c)::value]); });
             uintx4 wnext;
             half_t snext;
             auto read_w = [&](auto t_c) {
                 constexpr int t = decltype(t_c)::value;
-                if constexpr (RB == MB)
-                    wait_loads<FULL ? D * L - 1 : LATER + T - 1 - t>();
+                wait_w(t_c);
                 wnext = *reinterpret_cast<const uintx4*>(slot + RB * ROW_BLOCK_BYTES + t * 1024 + w_rd);
                 snext = *reinterpret_cast<const half_t*>(sc_rd + t * 2048);
             };
@@ -283,19 +317,7 @@ namespace nnf
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
-                    const uint32_t w4 = ww[j], w8 = w4 >> 8;
-                    half2_t q0 = as_half2((w4 & MASK_LO) | MAGIC) + c_lo;    // (q0, q4) - zp
-                    half2_t q1 = as_half2((w4 & MASK_HI) | MAGIC_HI) + c_hi; // (q1, q5) - zp
-                    half2_t q2 = as_half2((w8 & MASK_LO) | MAGIC) + c_lo;    // (q2, q6) - zp
-                    half2_t q3 = as_half2((w8 & MASK_HI) | MAGIC_HI) + c_hi; // (q3, q7) - zp
-                    if constexpr (RMS)
-                    {
-                        q0 *= as_half2(gm[j].x);
-                        q1 *= as_half2(gm[j].y);
-                        q2 *= as_half2(gm[j].z);
-                        q3 *= as_half2(gm[j].w);
-                    }
-                    const uintx4 bq = {as_u32(q0), as_u32(q1), as_u32(q2), as_u32(q3)};
+                    const uintx4 bq = unpack(ww[j], j);
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb)
                         sum[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[mb][j]),
@@ -303,12 +325,7 @@ namespace nnf
                 }
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
-                {
-                    acc[t][mb].x = __builtin_fmaf(sum[mb].x, scale, acc[t][mb].x);
-                    acc[t][mb].y = __builtin_fmaf(sum[mb].y, scale, acc[t][mb].y);
-                    acc[t][mb].z = __builtin_fmaf(sum[mb].z, scale, acc[t][mb].z);
-                    acc[t][mb].w = __builtin_fmaf(sum[mb].w, scale, acc[t][mb].w);
-                }
+                    add_scaled(acc[t][mb], sum[mb], scale);
             });
             if constexpr (D > 1)
                 at_slot = at_slot == ring + (D - 1) * SLOT ? ring : at_slot + SLOT;
@@ -352,10 +369,10 @@ namespace nnf
         const int n_tiles = (N + 15) / 16;
         // the sums of output tile `it`, block mb, lane `l` (rows 16 mb + 4 (l / 16) .. + 3, below M rounded up to a multiple of four) of a
         // range: where the ranges of K meet in scratch memory
-        const int quads = (M + 3) >> 2;
+        const int quads = gridDim.z == 1 ? (M + 3) >> 2 : MB * 4;
         auto partial_at = [&](int range, int it, int mb, int l) {
             return reinterpret_cast<unsigned long long*>(partial) +
-                   ((((size_t)range * n_tiles + t0 + it) * quads + mb * 4 + (l >> 4)) * 16 + (l & 15)) * 2;
+                   (((((size_t)blockIdx.z * gridDim.y + range) * n_tiles + t0 + it) * quads + mb * 4 + (l >> 4)) * 16 + (l & 15)) * 2;
         };
         auto write_out = [&](int it, int mb, int l, const floatx4& s) {
             const int nn = min((t0 + it) * 16, N - 16) + (l & 15);
@@ -435,7 +452,7 @@ namespace nnf
             volatile uint32_t* arrived_before = reinterpret_cast<volatile uint32_t*>(smem);
             __syncthreads();
             if (tid == 0)
-                *arrived_before = atomicAdd(sync + blockIdx.x, 1u);
+                *arrived_before = atomicAdd(sync + blockIdx.z * gridDim.x + blockIdx.x, 1u);
             __syncthreads();
             if (*arrived_before != gridDim.y - 1)
                 return;
@@ -464,7 +481,7 @@ namespace nnf
                 write_out(it, mb, lane, s);
             }
             if (tid == 0)
-                atomicExch(sync + blockIdx.x, 0u);
+                atomicExch(sync + blockIdx.z * gridDim.x + blockIdx.x, 0u);
         }
     }
 
@@ -484,33 +501,23 @@ namespace nnf
                 return e;
             const GemvFusionArgs args{(const half_t*)fusion.gamma, nullptr, (const half_t*)fusion.bias, (const half_t*)fusion.residual,
                                       fusion.rms_eps};
-            hipLaunchKernelGGL(kernel, dim3(plan.grid, plan.ranges), dim3(KS_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
+            hipLaunchKernelGGL(kernel, dim3(plan.grid, plan.ranges, plan.row_blocks), dim3(KS_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
                                (const half_t*)S, (half_t*)Y, N, K, plan.tiles_q | (plan.tiles_r << 16),
-                               M | (zp << 8) | (fusion.gate ? 1 << 16 : 0) | (plan.range_groups << 17), plan.ranges > 1 ? partial : nullptr,
+                               M | (zp << 13) | (fusion.gate ? 1 << 17 : 0) | (plan.range_groups << 18), plan.ranges > 1 ? partial : nullptr,
                                plan.ranges > 1 ? sync : nullptr, args);
             return hipGetLastError();
-        }
-        template <int T, int MB>
-        hipError_t launch_kstream_f(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
-                                    void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync)
-        {
-            return fusion.gamma ? launch_kstream<T, MB, true>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync)
-                                : launch_kstream<T, MB, false>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
         }
         template <int MB>
         hipError_t launch_kstream_t(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                     void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync)
         {
-            switch (plan.tiles)
-            {
-            case 1: return launch_kstream_f<1, MB>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-            case 2: return launch_kstream_f<2, MB>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-            case 3: return launch_kstream_f<3, MB>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-            case 4: return launch_kstream_f<4, MB>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-            case 5: return launch_kstream_f<5, MB>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-            case 6: return launch_kstream_f<6, MB>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-            default: return hipErrorInvalidValue;
-            }
+            hipError_t e = hipErrorInvalidValue;
+            unroll_for<1, workspace::KSTREAM_MAX_TILES + 1>([&](auto t) {
+                if (plan.tiles == t.value)
+                    e = fusion.gamma ? launch_kstream<t.value, MB, true>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync)
+                                     : launch_kstream<t.value, MB, false>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
+            });
+            return e;
         }
     } // namespace
 
@@ -520,13 +527,11 @@ namespace nnf
         if (plan.tiles < 1 || (plan.ranges > 1 && (!partial || !sync || fusion.gate || fusion.gamma)) || fusion.rstd ||
             (fusion.gate && (fusion.bias || fusion.residual)))
             return hipErrorInvalidValue;
-        switch ((M + 15) / 16)
-        {
-        case 1: return launch_kstream_t<1>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-        case 2: return launch_kstream_t<2>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-        case 3: return launch_kstream_t<3>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-        case 4: return launch_kstream_t<4>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
-        default: return hipErrorInvalidValue;
-        }
+        hipError_t e = hipErrorInvalidValue;
+        unroll_for<1, 5>([&](auto mb) {
+            if (plan.row_tiles == mb.value)
+                e = launch_kstream_t<mb.value>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync);
+        });
+        return e;
     }
 } // namespace nnf

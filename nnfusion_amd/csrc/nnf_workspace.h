@@ -1069,17 +1069,19 @@ namespace nnf
         struct KstreamPlan
         {
             int tiles = 0; // weight tiles of a workgroup, at most; 0: does not apply
+            int row_tiles = 0, row_blocks = 0; // blocks of row_tiles x 16 activation rows
             int tiles_q = 0, tiles_r = 0, grid = 0, ranges = 0, range_groups = 0;
             size_t partial_bytes = 0; // more than one range of K: their fp32 sums
         };
         // N: output columns (gate: from 2 N weight rows); more than one range of K: not with RMSNorm or SiLU-gate
-        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges)
+        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges, int row_blocks = 1)
         {
             KstreamPlan p;
-            const int mb = (M + 15) / 16, G = K >> 7;
-            if (M < 2 || mb > 4 || N < 16 || K < 1024 || (K & 127) || ranges < 1 || num_cu < ranges || (ranges > 1 && (gate || rms)))
+            const int mb = ((M + row_blocks - 1) / row_blocks + 15) / 16, G = K >> 7;
+            if (M < 2 || M > 4096 || mb > 4 || N < 16 || K < 1024 || (K & 127) || ranges < 1 || num_cu < ranges * row_blocks ||
+                (ranges > 1 && (gate || rms)) || (row_blocks - 1) * mb * 16 >= M)
                 return p;
-            const int rg = (G + ranges - 1) / ranges, n_tiles = (N + 15) / 16, per_range = num_cu / ranges;
+            const int rg = (G + ranges - 1) / ranges, n_tiles = (N + 15) / 16, per_range = num_cu / (ranges * row_blocks);
             const int grid = n_tiles < per_range ? n_tiles : per_range;
             const int tiles = (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid);
             // (a range's scales: rows of 32 words, from a half word where rows or ranges start in the middle of one)
@@ -1088,28 +1090,49 @@ namespace nnf
                 kstream_lds_bytes(tiles, mb, rms) > LDS_BYTES_PER_CU)
                 return p;
             p.tiles = tiles;
+            p.row_tiles = mb;
+            p.row_blocks = row_blocks;
             p.grid = grid;
             p.tiles_q = n_tiles / grid;
             p.tiles_r = n_tiles % grid;
             p.ranges = ranges;
             p.range_groups = rg;
-            p.partial_bytes = ranges > 1 ? (size_t)ranges * n_tiles * 16 * ((M + 3) & ~3) * sizeof(float) : 0;
+            p.partial_bytes =
+                ranges > 1 ? (size_t)row_blocks * ranges * n_tiles * 16 * (row_blocks > 1 ? mb * 16 : (M + 3) & ~3) * sizeof(float) : 0;
             return p;
         }
-        // Microseconds x 100 of a launch, a fit of 245 measured products (20 .. 64 rows, N = 512 .. 16384, K = 1152 .. 11008, one to four ranges;
-        // the number of ranges it picks is within 3 % of the fastest but for six of them, 13 % at most): a chunk of eight groups takes what
-        // its loads and its unpacking take, a little less where fewer CUs fetch the activations; ranges of K pay for the sums' way through memory.
-        inline int kstream_estimate(const KstreamPlan& p, int mb)
+        // Microseconds x 100 of a launch, a fit of 841 measured products (20 .. 512 rows, N = 512 .. 16384, K = 1152 .. 11008, with all numbers of ranges
+        // and blocks of rows that apply; 11 % rms, and what it picks is within 4 % of the fastest but for 15 of them, 19 % at most): a chunk of eight
+        // groups takes what its loads and its unpacking take, a little less where fewer CUs fetch the activations; ranges of K pay for
+        // the sums' way through memory.
+        inline int kstream_estimate(const KstreamPlan& p)
         {
-            const int chunks = (p.range_groups + KSTREAM_WAVES - 1) / KSTREAM_WAVES, workgroups = p.grid * p.ranges;
-            return chunks * (32 + 21 * mb + 33 * p.tiles) * (180 + (workgroups < 256 ? workgroups : 256)) / 436 + 187 + 29 * p.tiles +
-                   (p.ranges > 1 ? 46 + 12 * p.ranges + 63 * p.tiles : 0);
+            const int chunks = (p.range_groups + KSTREAM_WAVES - 1) / KSTREAM_WAVES, workgroups = p.grid * p.ranges * p.row_blocks;
+            const int mb = p.row_tiles, t = p.tiles;
+            return chunks * (17 + 27 * mb + 16 * t + 9 * mb * t) * (358 + (workgroups < 256 ? workgroups : 256)) / 614 + 200 + 6 * t + 15 * mb * t +
+                   (p.ranges > 1 ? 84 + 20 * p.ranges + 60 * t : 0);
         }
-        // What the library runs on it by itself, from measurements against the kernels that served these products before: 33 .. 64 rows
+        // What the library runs on it by itself, from measurements against the kernels that served these products before.  33 .. 64 rows:
         // everything that fits (against the tile GEMM: N = K = 4096 at 48 rows 13.8 -> 9.0 us, 12288 x 4096 21.0 -> 15.0, 4096 x 11008 20.5 -> 16.6,
-        // RMSNorm and SiLU-gate at 11008 x 4096 35.2 -> 22.4; against the row-streaming kernel up to K = 2048 1.2 - 1.9 x), 17 .. 32 rows all but more
+        // RMSNorm and SiLU-gate at 11008 x 4096 35.2 -> 22.4; against the row-streaming kernel up to K = 2048 1.2 - 1.9 x).  17 .. 32 rows: all but more
         // than four tiles a workgroup where the row-streaming kernel runs K as a compile-time constant (11008 x 4096 with both: 18.6 us
         // there, 19.9 here) or over ranges (12288 x 11008: 25.1 us there, 26.8 here); with up to four 1.02 - 1.3 x, K = 5504 2.0 - 2.4 x.
+        // More than 64 rows (blocks of at most 64 rows, each on its share of the CUs): the tile GEMM leaves CUs idle or shares tiles through
+        // memory where a product has few tiles.  72 .. 512 rows, N = 1024 .. 12288: 1.05 - 2.3 x, with RMSNorm and SiLU-gate 1.1 - 3.0 (128 rows of N = K = 4096
+        // 14.9 -> 11.0 us, 256 of 4096 x 6144 28.2 -> 22.9); not at six tiles of four blocks of 16 rows with RMSNorm or SiLU-gate beyond K = 2560
+        // (0.84 - 1.1), five or six below K = 2048 (0.89 - 0.98), nor over ranges of K above 256 rows (0.87 - 1.1).
+        inline bool kstream_ahead_of_tiles(const KstreamPlan& p, int M, int N, int K, bool gate, bool rms)
+        {
+            // (the longer K, the less there is to gain, down to nothing where the last tile of many workgroups is missing: 116 x 3200 x 8064 at 78 %
+            // of the workgroups' tiles 0.91 x, 117 x 2240 x 8064 at 73 % 0.96, 804 x 1280 x 3456 at 84 % 0.95)
+            // (256 x 1600 x 7424 0.92, 921 x 256 x 5504 0.84)
+            if ((M > 224 && K > 6144) || (M > 512 && K > 4096))
+                return false;
+            const int used = 100 * (gate ? 2 : 1) * ((N + 15) / 16) / (p.tiles * p.grid);
+            if (used < (K > 6144 || (M > 512 && K > 2048) ? 86 : K > 3072 ? 60 : 0))
+                return false;
+            return p.tiles * p.row_tiles < 20 || (K >= 2048 && (p.tiles * p.row_tiles < 24 || K <= 2560 || (!gate && !rms)));
+        }
         // partial_bytes, sync_bytes: of scratch memory and synchronisation words (one per workgroup of a range) at hand
         inline KstreamPlan kstream_choice(int M, int N, int K, int num_cu, bool gate, bool rms, size_t partial_bytes, size_t sync_bytes)
         {
@@ -1117,7 +1140,7 @@ namespace nnf
             const bool fixed_k = w4a16_mrows_fixed_k(M, K);
             // (17 .. 32 rows: N = 320 .. 600 at K = 1024 takes 3.3 us there, 3.5 here; N = 256 .. 2400 at K = 11776 .. 12288 0.92 - 0.97 x, 4480 and more
             // 1.06 - 1.16)
-            if (M < 2 || M > 64 || (M > 16 && M <= 32 && (K <= 1024 || (K > 11264 && N < 4096))))
+            if (M < 2 || M > 1024 || (M > 16 && M <= 32 && (K <= 1024 || (K > 11264 && N < 4096))))
                 return best;
             // 2 .. 16 rows, against the row-streaming kernel and the MFMA GEMV (time there / here, 1320 products).  K that is a compile-time constant
             // of the row-streaming kernel stays there (SiLU-gate 0.85 - 1.08, others 0.91 - 1.25, most within 8 %); with any other K RMSNorm and SiLU-gate,
@@ -1125,14 +1148,18 @@ namespace nnf
             // one tile a workgroup), of fewer rows 0.94 - 1.3: left where they are, like K above 8192, 0.9 - 1.1 over ranges.
             if (M <= 16 && (fixed_k || K > 8192 || (!gate && !rms && (M < 8 || (K < 1664 && M <= 9 && N <= 4096)))))
                 return best;
-            for (int ranges = 1; ranges <= (gate || rms ? 1 : 4); ++ranges)
-            {
-                const KstreamPlan p = kstream_plan(M, N, K, num_cu, gate, rms, ranges);
-                if (p.tiles == 0 || (ranges > 1 && (p.partial_bytes > partial_bytes || p.grid * sizeof(unsigned) > sync_bytes)) || (M <= 32 && p.tiles > 4 && (ranges > 1 || fixed_k)) || (M <= 16 && ranges > 1))
-                    continue;
-                if (best.tiles == 0 || kstream_estimate(p, (M + 15) / 16) < kstream_estimate(best, (M + 15) / 16))
-                    best = p;
-            }
+            const int fewest = (M + 63) / 64, most = M <= 32 ? 1 : fewest + 2;
+            for (int row_blocks = fewest; row_blocks <= most; ++row_blocks)
+                for (int ranges = 1; ranges <= (gate || rms || M <= 16 || M > 256 ? 1 : 4); ++ranges)
+                {
+                    const KstreamPlan p = kstream_plan(M, N, K, num_cu, gate, rms, ranges, row_blocks);
+                    if (p.tiles == 0 || (ranges > 1 && (p.partial_bytes > partial_bytes || (size_t)p.grid * row_blocks * sizeof(unsigned) > sync_bytes)) ||
+                        (M <= 32 && p.tiles > 4 && (ranges > 1 || fixed_k)) ||
+                        (M > 64 && !kstream_ahead_of_tiles(p, M, N, K, gate, rms)))
+                        continue;
+                    if (best.tiles == 0 || kstream_estimate(p) < kstream_estimate(best))
+                        best = p;
+                }
             return best;
         }
         // ---- W8A8, one activation row: the row-streaming GEMV (w8a8_gemv_rows.hip) ----

@@ -1,4 +1,4 @@
-"""The K-streaming MFMA kernel: fp16 x int4 products of 2 .. 64 rows (w4a16_kstream.hip).
+"""The K-streaming MFMA kernel: fp16 x int4 products of 2 .. 64 rows and of blocks of up to 64 (w4a16_kstream.hip).
 
 Sizes at its edges: rows around the blocks of 16, one column tile up to six a workgroup, columns that are no multiple of 16 (the
 last tile is moved back), a single group for the last chunk, an odd number of groups (scale rows that start in the middle of
@@ -40,7 +40,7 @@ def _ws(gpu, nbytes=64 << 20):
 @pytest.mark.parametrize("m,n,k", [
     (17, 16, 1152), (32, 48, 2176), (33, 40, 1152), (48, 4096, 1024), (49, 520, 4096), (64, 4112, 1280), (64, 24576, 1024), (63, 300, 8192),
     (8, 40, 1792), (11, 4096, 1152), (16, 4112, 1408), (13, 2064, 7936), (10, 4096, 3968), (16, 12288, 3712), (8, 24576, 1792),
-    (45, 8200, 2048), (20, 12288, 1280), (40, 640, 11008), (33, 4096, 11008), (64, 1030, 9984), (29, 256, 8448), (50, 2048, 1664)])
+    (65, 520, 2048), (128, 4104, 1408), (130, 1000, 4096), (257, 1040, 1152), (1000, 272, 1280), (90, 2048, 8448), (200, 1024, 9216), (45, 8200, 2048), (20, 12288, 1280), (40, 640, 11008), (33, 4096, 11008), (64, 1030, 9984), (29, 256, 8448), (50, 2048, 1664)])
 @pytest.mark.parametrize("with_sync", [True, False], ids=["sync", "no-sync"])
 def test_products(gpu, m, n, k, with_sync):
     import torch
@@ -70,7 +70,7 @@ def test_zero_points(gpu, zp):
     _check(ops.w4a16_gemm(ta, tw, ts, zp=zp, workspace=_ws(gpu)), oracle.w4a16_gemm(a, wq, s, zp=zp, f32_out=True))
 
 
-@pytest.mark.parametrize("m,n,k", [(45, 200, 1152), (64, 4128, 2048), (31, 72, 4096), (48, 1024, 9216), (9, 1000, 2688), (16, 4096, 7936)])
+@pytest.mark.parametrize("m,n,k", [(45, 200, 1152), (64, 4128, 2048), (31, 72, 4096), (48, 1024, 9216), (9, 1000, 2688), (16, 4096, 7936), (100, 1032, 2048), (150, 1024, 8704)])
 def test_bias_and_residual_in_place(gpu, m, n, k):
     from nnfusion_amd import ops
 
@@ -86,7 +86,7 @@ def test_bias_and_residual_in_place(gpu, m, n, k):
 
 @pytest.mark.parametrize("gate", [False, True], ids=["plain", "silu-gate"])
 @pytest.mark.parametrize("m,n,k,spread", [(45, 300, 1152, 1.0), (64, 8200, 1024, 1.0), (33, 2048, 8192, 1.0), (20, 40, 2176, 1.0), (48, 512, 2048, 3000.0),
-                                              (4, 40, 1152, 1.0), (16, 2050, 2560, 1.0), (9, 8192, 1280, 1.0), (16, 512, 1280, 3000.0)])
+                                              (4, 40, 1152, 1.0), (16, 2050, 2560, 1.0), (9, 8192, 1280, 1.0), (16, 512, 1280, 3000.0), (70, 1030, 1152, 1.0), (200, 512, 2048, 1.0)])
 def test_rms_norm(gpu, m, n, k, spread, gate):
     """spread: of the RMSNorm weight.  At 3000 neither gamma times an activation (up to 80) nor gamma times a weight of 15 is an fp16 number."""
     from nnfusion_amd import ops

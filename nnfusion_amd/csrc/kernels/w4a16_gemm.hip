@@ -357,7 +357,9 @@ namespace nnf
         // ---- the K-streaming kernel: prologue and epilogue inside, ranges of K added up in the launch ---------------------------
         const workspace::KstreamPlan kstream =
             workspace::w4a16_launch_kstream(route, M, N, K, gate, rms, num_cu, choice.sync_flags ? choice.sync_bytes : 0);
-        if (kstream.tiles > 0)
+        // (workgroups still read A when others write Y: an output over the input may rely on a pre-pass's copy of it)
+        const bool apart = (uintptr_t)A + (size_t)M * K * 2 <= (uintptr_t)Y || (uintptr_t)Y + (size_t)M * N * 2 <= (uintptr_t)A;
+        if (kstream.tiles > 0 && apart)
         {
             GemvFusion fusion;
             fusion.gamma = rms_gamma;

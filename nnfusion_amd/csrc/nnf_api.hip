@@ -162,6 +162,29 @@ namespace
     bool is_plain_w4a16(const nnf_quant* q) { return q->bits == 4 && q->group == 128 && !q->zero_points; }
     int group_shift_of(int group) { return group == 32 ? 5 : group == 64 ? 6 : 7; }
 
+    bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes)
+    {
+        const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+        return x < y + b_bytes && y < x + a_bytes;
+    }
+
+    // 4-bit weights with other block parameters on the K-streaming kernel, the nodes around the product inside it; taken = false: not one of
+    // its products (workspace::kstream_choice_q), nothing was launched.  (Workgroups still read A when others write Y: not there.)
+    int wna16_kstream(hipStream_t s, const void* A, const void* Wq, const void* scales, void* Y, int M, int N, int K, const nnf_quant* q,
+                      const nnf::GemvFusion& fusion, int num_cu, bool& taken)
+    {
+        taken = false;
+        if (q->bits != 4 || overlap(A, (size_t)M * K * 2, Y, (size_t)M * N * 2))
+            return NNF_OK;
+        const int gs = group_shift_of(q->group);
+        const nnf::workspace::KstreamPlan plan = nnf::workspace::kstream_choice_q(M, N, K, gs, num_cu, fusion.gate, fusion.gamma != nullptr);
+        if (plan.tiles == 0)
+            return NNF_OK;
+        taken = true;
+        const auto launch = gs == 5 ? nnf::launch_w4a16_kstream_q5 : gs == 6 ? nnf::launch_w4a16_kstream_q6 : nnf::launch_w4a16_kstream_q7;
+        return (int)launch(s, plan, A, Wq, scales, Y, M, N, K, q->zero_point, q->zero_points, fusion);
+    }
+
     // nnf_w8a8_variant -> the launchers' numbering of kernel families (that of nnf_w4a16_variant)
     int w8a8_path(int variant) { return variant == NNF_W8A8_AUTO ? 0 : variant + 1; }
 
@@ -302,6 +325,10 @@ int nnf_wna16_gemm_planned(nnf_stream_t stream, const void* A, const void* Wq, c
     const int st = current_device_info(dev);
     if (st != NNF_OK)
         return st;
+    bool taken;
+    const int streamed = wna16_kstream((hipStream_t)stream, A, Wq, scales, Y, M, N, K, q, nnf::GemvFusion(), dev.num_cu, taken);
+    if (taken)
+        return streamed;
     // 4-bit weights, 2 .. 16 rows, a K the fixed-K row-streaming kernel does not take: its run-time-K form, above K = 8192
     // over ranges of K with the reduction pass (given the workspace for the sums of the ranges)
     const int gs = group_shift_of(q->group);
@@ -372,12 +399,6 @@ int nnf_dequantize_f16(nnf_stream_t stream, const void* Wq, const void* scales, 
 
 namespace
 {
-    bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes)
-    {
-        const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-        return x < y + b_bytes && y < x + a_bytes;
-    }
-
     // A fused product of 4-bit weights on a few rows (other block parameters than the plain kernels'): where the plain product
     // runs on a row-streaming kernel, the nodes around it move into that kernel, or, over ranges of K, into the reduction
     // pass behind it (RMSNorm stays a launch there: a range does not see a whole row).  In the kernel, RMSNorm is a launch
@@ -388,6 +409,26 @@ namespace
                          const nnf_quant* q, const nnf::GemvFusion& fusion, void* xn, void* own, size_t own_bytes, int num_cu, bool& taken)
     {
         taken = false;
+        // (RMSNorm of a few rows inside that kernel where it is inside the row-streaming kernels as well or SiLU-gate follows; otherwise a
+        // launch ahead of it, so that the fused product stays the nodes' own arithmetic, bit for bit)
+        if (fusion.gamma && !fusion.gate && M <= 32 && !nnf::workspace::mrows_q_norm_inside(M, K))
+        {
+            if (q->bits == 4 && nnf::workspace::kstream_choice_q(M, N, K, group_shift_of(q->group), num_cu, false, false).tiles > 0)
+            {
+                nnf::GemvFusion behind = fusion;
+                behind.gamma = nullptr;
+                const hipError_t e = nnf::launch_rms_norm(s, A, fusion.gamma, xn, M, K, fusion.rms_eps);
+                taken = true;
+                bool streamed;
+                return e != hipSuccess ? (int)e : wna16_kstream(s, xn, Wq, scales, Y, M, N, K, q, behind, num_cu, streamed);
+            }
+        }
+        else
+        {
+            const int status = wna16_kstream(s, A, Wq, scales, Y, M, N, K, q, fusion, num_cu, taken);
+            if (taken)
+                return status;
+        }
         // (workgroups still read A when others write Y: an output over the input goes through the pre-pass's copy)
         if (q->bits != 4 || M < 2 || M > 32 || !fusion.any() || overlap(A, (size_t)M * K * 2, Y, (size_t)M * N * 2))
             return NNF_OK;

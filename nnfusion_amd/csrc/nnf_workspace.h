@@ -1054,15 +1054,19 @@ namespace nnf
         // chunks asked for ahead; blocks of 16 rows x 256 bytes of activations in a slot of a wavefront's ring; its bytes of LDS
         constexpr int kstream_depth(int tiles, int mb) { return tiles == 1 && mb == 1 ? 2 : 1; }
         constexpr int kstream_ring(int mb) { return mb < 4 ? mb : 3; }
-        constexpr int kstream_wave_bytes(int tiles, int mb, bool rms)
+        // qg: 0, or log2 of the group of other block parameters, whose scales and zero points come chunk by chunk: words of 16 rows, two of
+        // them a group of 128 for groups of 32, 64 a load, and as many loads of zero points
+        constexpr int kstream_scale_loads(int tiles, int qg) { return (tiles * 16 * (qg == 5 ? 2 : 1) + 63) / 64; }
+        constexpr int kstream_wave_bytes(int tiles, int mb, bool rms, int qg = 0)
         {
-            return kstream_depth(tiles, mb) * (kstream_ring(mb) * 4096 + tiles * 1024 + (rms ? 256 : 0));
+            return kstream_depth(tiles, mb) *
+                   (kstream_ring(mb) * 4096 + tiles * 1024 + (rms ? 256 : 0) + (qg ? 2 * kstream_scale_loads(tiles, qg) * 256 : 0));
         }
         // tiles whose eight partial sums are in LDS at a time (an even number where there is more than one round)
         constexpr int kstream_round(int tiles, int mb) { return mb == 4 && tiles > 4 ? 4 : tiles; }
-        constexpr size_t kstream_lds_bytes(int tiles, int mb, bool rms)
+        constexpr size_t kstream_lds_bytes(int tiles, int mb, bool rms, int qg = 0)
         {
-            const size_t stream = (size_t)KSTREAM_WAVES * kstream_wave_bytes(tiles, mb, rms) + (size_t)tiles * 2048;
+            const size_t stream = (size_t)KSTREAM_WAVES * kstream_wave_bytes(tiles, mb, rms, qg) + (qg ? 0 : (size_t)tiles * 2048);
             const size_t sums = (size_t)4096 + (size_t)KSTREAM_WAVES * kstream_round(tiles, mb) * mb * 1024;
             return stream > sums ? stream : sums;
         }
@@ -1074,7 +1078,7 @@ namespace nnf
             size_t partial_bytes = 0; // more than one range of K: their fp32 sums
         };
         // N: output columns (gate: from 2 N weight rows); more than one range of K: not with RMSNorm or SiLU-gate
-        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges, int row_blocks = 1)
+        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges, int row_blocks = 1, int qg = 0)
         {
             KstreamPlan p;
             const int mb = ((M + row_blocks - 1) / row_blocks + 15) / 16, G = K >> 7;
@@ -1085,9 +1089,12 @@ namespace nnf
             const int grid = n_tiles < per_range ? n_tiles : per_range;
             const int tiles = (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid);
             // (a range's scales: rows of 32 words, from a half word where rows or ranges start in the middle of one)
-            if (rg > ((G & 1) || ranges > 1 ? KSTREAM_MAX_GROUPS - 2 : KSTREAM_MAX_GROUPS) || (ranges - 1) * rg >= G ||
+            if (qg ? ranges > 1 || (K & 255) || (size_t)(gate ? 2 : 1) * N * (K >> qg) >= ((size_t)1 << 31)
+                   : rg > ((G & 1) || ranges > 1 ? KSTREAM_MAX_GROUPS - 2 : KSTREAM_MAX_GROUPS))
+                return p;
+            if ((ranges - 1) * rg >= G ||
                 ((G & 1) && ((N & 1) || (size_t)(gate ? 2 : 1) * N * G >= ((size_t)1 << 31))) || tiles > KSTREAM_MAX_TILES ||
-                kstream_lds_bytes(tiles, mb, rms) > LDS_BYTES_PER_CU)
+                kstream_lds_bytes(tiles, mb, rms, qg) > LDS_BYTES_PER_CU)
                 return p;
             p.tiles = tiles;
             p.row_tiles = mb;
@@ -1160,6 +1167,41 @@ namespace nnf
                     if (best.tiles == 0 || kstream_estimate(p) < kstream_estimate(best))
                         best = p;
                 }
+            return best;
+        }
+        // The same kernel for 4-bit weights in groups of 2^qg with a scalar zero point or one per (row, group): what the library runs on it, from
+        // measurements of 560 products against the row-streaming kernels of these parameters and the tile GEMM (time there / here).  Up to 16 rows:
+        // K = 2048 / 4096 / 8192 0.85 - 1.1, with RMSNorm 1.01 - 1.9 (SiLU-gate beyond four tiles a workgroup 0.84 - 1.07); other K 1.05 - 2.2, above 8192 from
+        // 4096 columns on 1.06 - 1.28 up to two tiles (0.89 - 1.1 outside).  17 .. 32 rows 0.98 - 2.7, 33 .. 64 1.02 - 2.4 (two tiles and more of
+        // four blocks of rows beyond K = 8192 0.91 - 1.0), more rows up to K = 6144 1.02 - 2.2 (0.85 - 1.3 beyond).
+        inline KstreamPlan kstream_choice_q(int M, int N, int K, int qg, int num_cu, bool gate, bool rms)
+        {
+            KstreamPlan best;
+            if (M < 2 || M > 512 || qg < 5 || qg > 7 || (M > 64 && K > 6144))
+                return best;
+            const int fewest = (M + 63) / 64, most = M <= 32 ? 1 : fewest + 2;
+            for (int row_blocks = fewest; row_blocks <= most; ++row_blocks)
+            {
+                const KstreamPlan p = kstream_plan(M, N, K, num_cu, gate, rms, 1, row_blocks, qg);
+                // (four blocks of rows and six tiles with RMSNorm do not fit the registers: 51 x 9408 x 3328 0.79)
+                if (p.tiles == 0 || (rms && p.tiles * p.row_tiles == 24))
+                    continue;
+                if (M <= 16)
+                {
+                    const bool fixed_k = K == 2048 || K == 4096 || K == 8192;
+                    if (fixed_k ? !rms || (gate && p.tiles > (K == 2048 ? 6 : 4)) : K > 8192 && (N < 4096 || p.tiles > 2))
+                        continue;
+                }
+                else if (M <= 64)
+                {
+                    if (K > 8192 && p.tiles * p.row_tiles >= 8)
+                        continue;
+                }
+                else if (!kstream_ahead_of_tiles(p, M, N, K, gate, rms))
+                    continue;
+                if (best.tiles == 0 || kstream_estimate(p) < kstream_estimate(best))
+                    best = p;
+            }
             return best;
         }
         // ---- W8A8, one activation row: the row-streaming GEMV (w8a8_gemv_rows.hip) ----

@@ -223,6 +223,9 @@ namespace nnf
     hipError_t launch_w8a8_mrows(hipStream_t stream, const void* A, const void* s_tok, const void* W, const void* s_ch,
                                  void* Y, void* acc, int M, int N, int K, int num_cu, void* partial_ws = nullptr,
                                  size_t partial_bytes = 0, uint32_t* sync = nullptr, size_t sync_bytes = 0);
+    // a few rows, or blocks of rows: the K-streaming kernel, as `plan` (workspace::w8a8_kstream_plan) says
+    hipError_t launch_w8a8_kstream(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* s_tok, const void* W,
+                                   const void* s_ch, void* Y, void* acc, int M, int N, int K);
     bool w8a8_mrows_supported(int M, int N, int K, int num_cu);
     bool w8a8_mrows_preferred(int M, int N, int K, int num_cu); // where the library picks it without being told
 

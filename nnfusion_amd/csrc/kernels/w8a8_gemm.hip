@@ -325,6 +325,13 @@ namespace nnf
         p.N = N;
         p.K = K;
         const bool raw = acc != nullptr;
+        // (the caller fixed nothing: the K-streaming kernel where it is ahead; scratch memory is asked for as for the kernel it replaces)
+        if (choice.path == 0 && choice.tile_rows == 0 && choice.tile_cols == 0 && choice.k_parts == 0)
+        {
+            const workspace::KstreamPlan plan = workspace::w8a8_kstream_choice(M, N, K, num_cu);
+            if (plan.tiles > 0)
+                return launch_w8a8_kstream(stream, plan, A, s_tok, W, s_ch, Y, acc, M, N, K);
+        }
         switch (pick_w8a8(M, N, K, num_cu, choice.path))
         {
         case Q8_ROWS: return launch_w8a8_gemv_rows(stream, A, s_tok, W, s_ch, Y, acc, N, K, num_cu);

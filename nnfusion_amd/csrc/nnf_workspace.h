@@ -1070,6 +1070,9 @@ namespace nnf
             const size_t sums = (size_t)4096 + (size_t)KSTREAM_WAVES * kstream_round(tiles, mb) * mb * 1024;
             return stream > sums ? stream : sums;
         }
+        // CUs of a block of rows: a multiple of eight, so that the workgroups of all blocks that read the same weights are on one XCD (they
+        // are dealt out to the eight XCDs in turn)
+        constexpr int kstream_cus(int share, int row_blocks) { return row_blocks > 1 && share >= 8 ? share & ~7 : share; }
         struct KstreamPlan
         {
             int tiles = 0; // weight tiles of a workgroup, at most; 0: does not apply
@@ -1085,7 +1088,7 @@ namespace nnf
             if (M < 2 || M > 4096 || mb > 4 || N < 16 || K < 1024 || (K & 127) || ranges < 1 || num_cu < ranges * row_blocks ||
                 (ranges > 1 && (gate || rms)) || (row_blocks - 1) * mb * 16 >= M)
                 return p;
-            const int rg = (G + ranges - 1) / ranges, n_tiles = (N + 15) / 16, per_range = num_cu / (ranges * row_blocks);
+            const int rg = (G + ranges - 1) / ranges, n_tiles = (N + 15) / 16, per_range = kstream_cus(num_cu / (ranges * row_blocks), row_blocks);
             const int grid = n_tiles < per_range ? n_tiles : per_range;
             const int tiles = (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid);
             // (a range's scales: rows of 32 words, from a half word where rows or ranges start in the middle of one)
@@ -1132,8 +1135,8 @@ namespace nnf
         {
             // (the longer K, the less there is to gain, down to nothing where the last tile of many workgroups is missing: 116 x 3200 x 8064 at 78 %
             // of the workgroups' tiles 0.91 x, 117 x 2240 x 8064 at 73 % 0.96, 804 x 1280 x 3456 at 84 % 0.95)
-            // (256 x 1600 x 7424 0.92, 921 x 256 x 5504 0.84)
-            if ((M > 224 && K > 6144) || (M > 512 && K > 4096))
+            // (256 x 1600 x 7424 0.92, 218 x 5376 x 7936 0.93, 921 x 256 x 5504 0.84)
+            if ((M > 192 && K > 6144) || (M > 512 && K > 4096))
                 return false;
             const int used = 100 * (gate ? 2 : 1) * ((N + 15) / 16) / (p.tiles * p.grid);
             if (used < (K > 6144 || (M > 512 && K > 2048) ? 86 : K > 3072 ? 60 : 0))
@@ -1200,6 +1203,65 @@ namespace nnf
                 else if (!kstream_ahead_of_tiles(p, M, N, K, gate, rms))
                     continue;
                 if (best.tiles == 0 || kstream_estimate(p) < kstream_estimate(best))
+                    best = p;
+            }
+            return best;
+        }
+        // ---- W8A8: the K-streaming kernel (w8a8_kstream.hip) ----
+        // bytes of K of a wavefront's part of a chunk: two lines of a row where the LDS has room for them and K is a multiple of that
+        constexpr size_t w8a8_kstream_lds_bytes(int tiles, int mb, int unit)
+        {
+            const size_t stream = (size_t)KSTREAM_WAVES * (tiles + mb) * 16 * unit, sums = (size_t)KSTREAM_WAVES * kstream_round(tiles, mb) * mb * 1024;
+            return stream > sums ? stream : sums;
+        }
+        constexpr int w8a8_kstream_unit(int tiles, int mb, int K)
+        {
+            return !(K & 255) && w8a8_kstream_lds_bytes(tiles, mb, 256) <= LDS_BYTES_PER_CU ? 256 : 128;
+        }
+        inline KstreamPlan w8a8_kstream_plan(int M, int N, int K, int num_cu, int row_blocks)
+        {
+            KstreamPlan p;
+            const int mb = ((M + row_blocks - 1) / row_blocks + 15) / 16;
+            if (M < 2 || mb > 4 || N < 16 || K < 1024 || (K & 127) || num_cu < row_blocks || (row_blocks - 1) * mb * 16 >= M ||
+                (size_t)16 * K >= ((size_t)1 << 31))
+                return p;
+            const int n_tiles = (N + 15) / 16, per_block = kstream_cus(num_cu / row_blocks, row_blocks);
+            const int grid = n_tiles < per_block ? n_tiles : per_block, tiles = (n_tiles + grid - 1) / grid;
+            if (tiles > KSTREAM_MAX_TILES || w8a8_kstream_lds_bytes(tiles, mb, w8a8_kstream_unit(tiles, mb, K)) > LDS_BYTES_PER_CU)
+                return p;
+            p.tiles = tiles;
+            p.row_tiles = mb;
+            p.row_blocks = row_blocks;
+            p.grid = grid;
+            p.tiles_q = n_tiles / grid;
+            p.tiles_r = n_tiles % grid;
+            p.ranges = 1;
+            return p;
+        }
+        // Microseconds x 100, a fit of 471 measured launches (2 .. 1000 rows, N = 512 .. 16384, K = 1152 .. 14336; 23 % rms, and the number of blocks of rows it
+        // picks is within 6 % of the fastest everywhere)
+        inline int w8a8_kstream_estimate(const KstreamPlan& p, int K)
+        {
+            const int unit = w8a8_kstream_unit(p.tiles, p.row_tiles, K), chunks = (K / unit + KSTREAM_WAVES - 1) / KSTREAM_WAVES;
+            const int workgroups = p.grid * p.row_blocks;
+            return chunks * (3 + unit / 128 * (23 * p.row_tiles + 40 * p.tiles)) * (363 + (workgroups < 256 ? workgroups : 256)) / 619 + 190 +
+                   10 * p.tiles + 3 * p.row_tiles * p.tiles;
+        }
+        // What the library runs on it by itself (against the row-streaming kernel up to 32 rows and the tile GEMM, time there / here): 2 .. 32 rows
+        // 1.0 - 2.8, but four tiles a workgroup of rows of 8 KiB up to 16 rows 0.81 - 0.85 (all workgroups in the same memory channels); 33 .. 64 rows
+        // 1.04 - 2.9 (K = 14336 from 8192 columns on 0.96 - 1.03); more rows up to K = 8192 1.1 - 3.8 (14336: 0.9 - 1.7).
+        inline KstreamPlan w8a8_kstream_choice(int M, int N, int K, int num_cu)
+        {
+            KstreamPlan best;
+            if (M < 2 || M > 1024 || num_cu < 8 || (M > 32 && M <= 64 && K > 12288 && N >= 8192) || (M > 64 && K > 8192))
+                return best;
+            const int fewest = (M + 63) / 64, most = M <= 32 ? 1 : fewest + 2;
+            for (int row_blocks = fewest; row_blocks <= most; ++row_blocks)
+            {
+                const KstreamPlan p = w8a8_kstream_plan(M, N, K, num_cu, row_blocks);
+                if (p.tiles == 0 || (M <= 16 && p.tiles == 4 && K % 8192 == 0))
+                    continue;
+                if (best.tiles == 0 || w8a8_kstream_estimate(p, K) < w8a8_kstream_estimate(best, K))
                     best = p;
             }
             return best;

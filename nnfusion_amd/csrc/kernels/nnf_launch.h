@@ -137,13 +137,20 @@ namespace nnf
     // word per workgroup of a range in `sync` (zero again afterwards)
     hipError_t launch_w4a16_kstream(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                     void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync);
-    // ... for groups of 32 / 64 / 128 (q5 / q6 / q7) and a scalar zero point or (zero_points != null) one per (row, group): one range of K, K a
-    // multiple of 256, the zero points of a row in K / group / 2 bytes
+    // ... for groups of 32 / 64 / 128 (q5 / q6 / q7) and a scalar zero point or (zero_points != null) one per (row, group): one range of K; the zero
+    // points of a row in (K / group + 1) / 2 bytes
     hipError_t launch_w4a16_kstream_q5(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                        void* Y, int M, int N, int K, int zp, const void* zero_points, const GemvFusion& fusion);
     hipError_t launch_w4a16_kstream_q6(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                        void* Y, int M, int N, int K, int zp, const void* zero_points, const GemvFusion& fusion);
     hipError_t launch_w4a16_kstream_q7(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
+                                       void* Y, int M, int N, int K, int zp, const void* zero_points, const GemvFusion& fusion);
+    // ... and 8-bit weights, a byte each; the zero points of a row in K / group bytes
+    hipError_t launch_w8a16_kstream_q5(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
+                                       void* Y, int M, int N, int K, int zp, const void* zero_points, const GemvFusion& fusion);
+    hipError_t launch_w8a16_kstream_q6(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
+                                       void* Y, int M, int N, int K, int zp, const void* zero_points, const GemvFusion& fusion);
+    hipError_t launch_w8a16_kstream_q7(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                        void* Y, int M, int N, int K, int zp, const void* zero_points, const GemvFusion& fusion);
 
     // (bias, residual: added behind the product, each or null; the residual may be Y)

@@ -1,4 +1,4 @@
-// fp16 x int4 (g128) for 2 .. 64 activation rows: all tiles of a workgroup side by side, K in chunks.
+// fp16 x int4 / int8 for blocks of 2 .. 64 activation rows: all tiles of a workgroup side by side, K in chunks.
 //
 //   Y[M,N] = A[M,K] . ((Wq - zp) * S)^T
 //
@@ -22,6 +22,10 @@
 //   * The weights of a lane (32 of one row and group) are unpacked to the exact integers q - zp in fp16 (the nibble in the
 //     mantissa of 1024.0 or 64.0, minus 1024 + zp or 64 + zp) once per chunk and meet MB blocks of rows; the group's sum times its scale
 //     joins the accumulator in fp32.
+//   * BITS 8 (groups of 32 / 64 / 128 with their scales in the weights, as QG of 4 bits): a byte b behind 0x64 is 1024 + b in fp16, less 1024 + zp
+//     exact; lanes read 32 bytes of a row's 128, pieces 2 kq and 2 kq + 1 swizzled over eight places: no bank conflicts.  Against the
+//     row-streaming kernel on bytes, the tile kernel and the passes of the nodes around them: 45 x 12288 x 4096 28.3 -> 18.2 us
+//     (16.0 at 32 rows, where the weights alone bound it), 16 x 4096 x 4096 with RMSNorm and SiLU-gate 17.0 -> 12.9, 5 x 1000 x 1280 5.4 -> 3.9.
 //   * RMS: rstd from the squares of the activations as they pass (fp32), applied to the sums; gamma[k] multiplies the
 //     unpacked weights, as in the tile GEMM: gamma times an activation alone may leave the range of fp16 (gamma / 16 times
 //     q - zp, of at most 15, does not).
@@ -51,12 +55,12 @@ namespace nnf
     } // namespace
 
     // blockIdx.z: blocks of 16 MB activation rows.
-    // pack = M | zp << 13 | gate << 17 | range_groups << 18; tiles = tiles_q | tiles_r << 16: output tiles of a workgroup, one
+    // pack = M | zp << 13 | gate << 21 | range_groups << 22 (ten bits: one range where K / 128 takes more); tiles = tiles_q | tiles_r << 16: output tiles of a workgroup, one
     // more for the first tiles_r (gate: twice as many weight tiles, the gate and the up tile of each in turn).
     // LDS (bytes): per wavefront [RB][4096] activations | [T][1024] weights | (RMS) 256 gamma; then the scales of the
     //              workgroup's range of K, [T][16][32] words.  At the end, over all of it: (RMS) the wavefronts' sums of squares
     //              [8][16 MB] and rstd[16 MB] | from byte 4096 on the wavefronts' sums [8][tiles of a round][MB KiB].
-    template <int T, int MB, bool RMS, int QG>
+    template <int T, int MB, bool RMS, int QG, int BITS>
     __global__ __launch_bounds__(KS_WAVES * 64) void w4a16_kstream_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                                           const half_t* __restrict__ S, half_t* __restrict__ Y, int N,
                                                                           int K, int tiles, int pack, float* __restrict__ partial,
@@ -67,12 +71,16 @@ namespace nnf
         constexpr int D = workspace::kstream_depth(T, MB); // chunks asked for ahead
         constexpr int RB = workspace::kstream_ring(MB);    // blocks of activations in a slot of a wavefront's ring
         static_assert(RB == MB || (RB < MB && D == 1), "");
-        // QG: scales of a tile's row and group of 128 as words, 64 words a load; as many loads of bytes with their zero points
-        constexpr int SPW = QG == 5 ? 2 : 1, NSL = QG ? workspace::kstream_scale_loads(T, QG) : 0, NS = 2 * NSL;
-        constexpr int NG = RMS ? 1 : 0, L = NG + 4 * MB + NS + T; // loads of a chunk
-        constexpr int SLOT = RB * ROW_BLOCK_BYTES + T * 1024 + NG * 256 + NS * 256;
-        constexpr int W_AT = RB * ROW_BLOCK_BYTES, G_AT = W_AT + T * 1024, S_AT = G_AT + NG * 256; // parts of a slot
-        constexpr int WAVE_BYTES = workspace::kstream_wave_bytes(T, MB, RMS, QG);
+        // QG: scales of a tile's row and group of 128 as words, 64 words a load; then loads of bytes with their zero points
+        static_assert(BITS == 4 || (BITS == 8 && QG != 0), "");
+        constexpr int SPW = QG == 5 ? 2 : 1, NSL = QG ? workspace::kstream_scale_loads(T, QG) : 0;
+        constexpr int ZPB = BITS == 8 ? 1 << (7 - QG) : QG == 5 ? 2 : 1, NZL = QG ? workspace::kstream_zero_loads(T, QG, BITS) : 0;
+        constexpr int NS = NSL + NZL;
+        constexpr int NW = BITS / 4, WB = NW * 1024, LW = NW * T;      // of a tile's weights: loads, bytes; loads of all of them
+        constexpr int NG = RMS ? 1 : 0, L = NG + 4 * MB + NS + LW; // loads of a chunk
+        constexpr int SLOT = RB * ROW_BLOCK_BYTES + T * WB + NG * 256 + NS * 256;
+        constexpr int W_AT = RB * ROW_BLOCK_BYTES, G_AT = W_AT + T * WB, S_AT = G_AT + NG * 256; // parts of a slot
+        constexpr int WAVE_BYTES = workspace::kstream_wave_bytes(T, MB, RMS, QG, BITS);
         constexpr int RT = workspace::kstream_round(T, MB); // tiles whose sums are in LDS at a time
         extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
         uint32_t MAGIC, MAGIC_HI, MASK_LO, MASK_HI;
@@ -86,9 +94,9 @@ namespace nnf
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int col = lane & 15; // n within the tile (B operand / D column), m for the A operand
         const int kq = lane >> 4;  // K quarter of the MFMA operands, row quad of D
-        const int M_all = pack & 0x1fff, zp = (pack >> 13) & 0xf, gate = (pack >> 17) & 1, range_groups = (int)((unsigned)pack >> 18);
+        const int M_all = pack & 0x1fff, zp = (pack >> 13) & 0xff, gate = (pack >> 21) & 1, range_groups = (int)((unsigned)pack >> 22);
         const int tiles_q = tiles & 0xffff, tiles_r = (int)((unsigned)tiles >> 16);
-        const int G = K >> 7, ROW_BYTES = K >> 1;
+        const int G = K >> 7, ROW_BYTES = BITS == 8 ? K : K >> 1;
         // rows first_row .. first_row + M - 1 of the activations, as a product of its own
         const int first_row = (int)blockIdx.z * (MB * 16), M = min(M_all - first_row, MB * 16);
         A += (size_t)first_row * K;
@@ -133,14 +141,25 @@ namespace nnf
 
         // ---- what each lane fetches -------------------------------------------------------------------------------------
         // weights: lane l the 16-byte piece (l & 3) ^ (r >> 2) of row r = l >> 2 of a tile's group
-        const uint32_t w_off = (uint32_t)(lane >> 2) * (uint32_t)ROW_BYTES + (uint32_t)(((lane & 3) ^ (lane >> 4)) << 4);
+        // (8 bits: piece (l & 7) ^ (r >> 1) & 7 of row r = 8 c + l / 8 in load c)
+        uint32_t w_off[NW];
+        if constexpr (BITS == 8)
+        {
+#pragma unroll
+            for (int c = 0; c < NW; ++c)
+                w_off[c] = (uint32_t)(c * 8 + (lane >> 3)) * (uint32_t)ROW_BYTES + (uint32_t)(((lane & 7) ^ (((c * 8 + (lane >> 3)) >> 1) & 7)) << 4);
+        }
+        else
+            w_off[0] = (uint32_t)(lane >> 2) * (uint32_t)ROW_BYTES + (uint32_t)(((lane & 3) ^ (lane >> 4)) << 4);
         const uint8_t* w_row[T];
 #pragma unroll
         for (int t = 0; t < T; ++t)
             w_row[t] = Wq + (size_t)row0_of(t) * (size_t)ROW_BYTES;
         auto fetch_w = [&](int g, int t, uint8_t* to) {
-            __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(w_row[t] + (uint32_t)g * 64u + w_off), (ks_lds_ptr_t)(to + W_AT + t * 1024), 16,
-                                             0, 0);
+#pragma unroll
+            for (int c = 0; c < NW; ++c)
+                __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(w_row[t] + (uint32_t)g * (uint32_t)(16 * BITS) + w_off[c]),
+                                                 (ks_lds_ptr_t)(to + W_AT + t * WB + c * 1024), 16, 0, 0);
         };
         // activations: as row_block_fetch (nnf_device.h); rows past M: the last row again, blocks past its block: that block again
         const int last_block = (M - 1) >> 4;
@@ -166,31 +185,34 @@ namespace nnf
                                                  (ks_lds_ptr_t)(to + G_AT), 4, 0, 0);
         };
 
-        // QG: lane l of load i fetches word (64 i + l) % SPW of a group of 128 in row (64 i + l) / SPW of the tiles, and the byte that
-        // holds the same weights' zero points (one byte load: lands in the lane's four bytes; without a tensor the scales again, unused)
-        const int GQ = QG ? K >> QG : 0; // scales of a row, an even number
-        uint32_t s_at[NSL ? NSL : 1], z_at[NSL ? NSL : 1];
+        // QG: lane l of load i fetches word (64 i + l) % SPW of a group of 128's scales in row (64 i + l) / SPW of the tiles; of the zero points
+        // likewise one of ZPB bytes (a byte load lands in the lane's four bytes; without a tensor the scales again, unused)
+        // (128: an odd number of groups starts every other row in the middle of a word; N is even then, and the tiles' first rows start in none)
+        const int GQ = QG ? K >> QG : 0; // scales of a row
+        uint32_t s_at[NSL ? NSL : 1], z_at[NZL ? NZL : 1];
         if constexpr (QG != 0)
         {
+            auto weight_row = [&](int at) { // row at % 16 of tile at / 16
+                const int it = min(at >> 4, TW - 1);
+                return (gate ? ((it & 1) ? N : 0) + min((t0 + (it >> 1)) * 16, N - 16) : min((t0 + it) * 16, N - 16)) + (at & 15);
+            };
 #pragma unroll
             for (int i = 0; i < NSL; ++i)
-            {
-                const int at = (i * 64 + lane) / SPW, it = min(at >> 4, TW - 1), word = (i * 64 + lane) % SPW;
-                const int row = (gate ? ((it & 1) ? N : 0) + min((t0 + (it >> 1)) * 16, N - 16) : min((t0 + it) * 16, N - 16)) + (at & 15);
-                s_at[i] = (uint32_t)row * (uint32_t)GQ + (uint32_t)word * 2u;
-                z_at[i] = (uint32_t)row * (uint32_t)(GQ >> 1) + (uint32_t)word;
-            }
+                s_at[i] = (uint32_t)weight_row((i * 64 + lane) / SPW) * (uint32_t)GQ + (uint32_t)((i * 64 + lane) % SPW) * 2u;
+#pragma unroll
+            for (int i = 0; i < NZL; ++i)
+                z_at[i] = (uint32_t)weight_row((i * 64 + lane) / ZPB) * (uint32_t)(BITS == 8 ? GQ : (GQ + 1) >> 1) + (uint32_t)((i * 64 + lane) % ZPB);
         }
         auto fetch_s = [&](int g, uint8_t* to) {
             if constexpr (QG != 0)
             {
-                const uint32_t s0 = (uint32_t)((g << (7 - QG)) & ~1), z0 = (uint32_t)((g << (7 - QG)) >> 1);
+                const uint32_t s0 = (uint32_t)(g << (7 - QG)), z0 = (uint32_t)(BITS == 8 ? g << (7 - QG) : (g << (7 - QG)) >> 1);
 #pragma unroll
                 for (int i = 0; i < NSL; ++i)
-                    __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(reinterpret_cast<const uint8_t*>(S) + (size_t)(s_at[i] + s0) * 2),
+                    __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(reinterpret_cast<const uint8_t*>(S) + (size_t)((s_at[i] + s0) & ~1u) * 2),
                                                      (ks_lds_ptr_t)(to + S_AT + i * 256), 4, 0, 0);
 #pragma unroll
-                for (int i = 0; i < NSL; ++i)
+                for (int i = 0; i < NZL; ++i)
                     __builtin_amdgcn_global_load_lds((ks_global_ptr_t)(zps ? zps + (z_at[i] + z0) : reinterpret_cast<const uint8_t*>(S)),
                                                      (ks_lds_ptr_t)(to + S_AT + (NSL + i) * 256), 1, 0, 0);
             }
@@ -211,7 +233,7 @@ namespace nnf
                 fetch_w(group_of(d), t, ring + d * SLOT);
         }
         if constexpr (QG == 0)
-            wait_loads<D*(NG + 4 * RB + T)>(); // the scales
+            wait_loads<D*(NG + 4 * RB + LW)>(); // the scales
         lds_barrier();
 
         const half_t clo = (half_t)(-(1024.0f + (float)zp)), chi = (half_t)(-(64.0f + (float)zp)); // exact
@@ -232,9 +254,19 @@ namespace nnf
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             a_rd[j] = (uint32_t)(col * 256 + (((kq * 4 + j) ^ col) << 4));
-        const uint32_t w_rd = (uint32_t)(col * 64 + ((kq ^ (col >> 2)) << 4));
+        uint32_t w_rd[NW];
+        if constexpr (BITS == 8)
+        {
+#pragma unroll
+            for (int c = 0; c < NW; ++c)
+                w_rd[c] = (uint32_t)(col * 128 + (((2 * kq + c) ^ ((col >> 1) & 7)) << 4));
+        }
+        else
+            w_rd[0] = (uint32_t)(col * 64 + ((kq ^ (col >> 2)) << 4));
         const int sc_first = ((col * G + g_lo) & 1) + wave; // place of the wavefront's first scale in row col (row0_of() * G is even)
 
+        // activations and gamma in the order in which the weights are unpacked: the pairs of the nibble trick, 8 bits memory order
+        auto operand_order = [](uintx4 v) { return BITS == 8 ? v : permute_a8(v); };
         // Loads of a wavefront in order: chunk by chunk [gamma] [MB blocks of activations] [QG: scales, zero points] [T tiles of weights]; those of chunk c + D
         // (RB < MB: of the activations, the first RB blocks) are asked for during chunk c, each where its slot has just been
         // read.  Loads come back in order: the wait counts below are the loads that follow the one waited for.  AHEAD: the chunks still to come,
@@ -251,13 +283,13 @@ namespace nnf
             uintx4 gm[4];
             if constexpr (RMS)
             {
-                wait_loads<LATER + 4 * RB + NS + T>();
+                wait_loads<LATER + 4 * RB + NS + LW>();
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
                     // (QG: q - zp carries its scale already)
                     const half2_t sixteenth = {(half_t)(QG ? 1.f : 0.0625f), (half_t)(QG ? 1.f : 0.0625f)};
-                    const uintx4 g8 = permute_a8(*reinterpret_cast<const uintx4*>(slot + G_AT + kq * 64 + j * 16));
+                    const uintx4 g8 = operand_order(*reinterpret_cast<const uintx4*>(slot + G_AT + kq * 64 + j * 16));
                     gm[j] = uintx4{as_u32(as_half2(g8.x) * sixteenth), as_u32(as_half2(g8.y) * sixteenth), as_u32(as_half2(g8.z) * sixteenth),
                                    as_u32(as_half2(g8.w) * sixteenth)};
                 }
@@ -271,11 +303,11 @@ namespace nnf
             auto read_a = [&](auto p_c, uintx4(&a)[4]) {
                 constexpr int p = decltype(p_c)::value;
                 if constexpr (FULL)
-                    wait_loads<LATER + 4 * (RB - 1) + (p < RB ? NS + T + NG : 0)>();
+                    wait_loads<LATER + 4 * (RB - 1) + (p < RB ? NS + LW + NG : 0)>();
                 else
                 {
                     constexpr int fetched = p < MB - RB ? p : MB - RB; // RB < MB: blocks asked for in this chunk so far
-                    wait_loads<(p < RB ? LATER + 4 * (RB - 1 - p) + NS + T + 4 * fetched : 4 * (p - 1 + RB < MB ? RB - 1 : MB - 1 - p))>();
+                    wait_loads<(p < RB ? LATER + 4 * (RB - 1 - p) + NS + LW + 4 * fetched : 4 * (p - 1 + RB < MB ? RB - 1 : MB - 1 - p))>();
                 }
                 uint8_t* at = at_slot + (RB == MB ? p : block) * ROW_BLOCK_BYTES;
 #pragma unroll
@@ -290,7 +322,7 @@ namespace nnf
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
-                    a[j] = permute_a8(a[j]);
+                    a[j] = operand_order(a[j]);
                     if constexpr (RMS)
                     {
                         ss[p] = dot2(as_half2(a[j].x), as_half2(a[j].x), ss[p]);
@@ -303,11 +335,30 @@ namespace nnf
             auto wait_w = [&](auto t_c) {
                 constexpr int t = decltype(t_c)::value;
                 if constexpr (RB == MB)
-                    wait_loads<FULL ? D * L - 1 : LATER + T - 1 - t>();
+                    wait_loads<FULL ? D * L - NW : LATER + NW * (T - 1 - t)>();
             };
             // weights 8 j .. 8 j + 7 of a lane's 32: exact integers q - zp (QG: times their scale, rounded once), times gamma
             // lo, hi: -(1024 + zp) and -(64 + zp) in both halves
-            auto unpack = [&](uint32_t w4, int j, half2_t lo, half2_t hi, half2_t scale2) {
+            // (8 bits: w4, w5 the eight bytes; a byte behind 0x64 is 1024 + b)
+            auto unpack = [&](uint32_t w4, uint32_t w5, int j, half2_t lo, half2_t hi, half2_t scale2) {
+                if constexpr (BITS == 8)
+                {
+                    half2_t b[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                    {
+                        b[i] = as_half2(__builtin_amdgcn_perm(MAGIC, i < 2 ? w4 : w5, i & 1 ? 0x07030702u : 0x07010700u)) + lo;
+                        b[i] *= scale2;
+                    }
+                    if constexpr (RMS)
+                    {
+                        b[0] *= as_half2(gm[j].x);
+                        b[1] *= as_half2(gm[j].y);
+                        b[2] *= as_half2(gm[j].z);
+                        b[3] *= as_half2(gm[j].w);
+                    }
+                    return uintx4{as_u32(b[0]), as_u32(b[1]), as_u32(b[2]), as_u32(b[3])};
+                }
                 const uint32_t w8 = w4 >> 8;
                 half2_t q0 = as_half2((w4 & MASK_LO) | MAGIC) + lo;    // (q0, q4) - zp
                 half2_t q1 = as_half2((w4 & MASK_HI) | MAGIC_HI) + hi; // (q1, q5) - zp
@@ -342,26 +393,30 @@ namespace nnf
             if constexpr (QG != 0)
             {
                 if constexpr (RB == MB)
-                    wait_loads<FULL ? (D - 1) * L + T + NG + 4 * MB : LATER + T>();
-                const int sub = QG == 5 ? kq : QG == 6 ? kq >> 1 : g & 1; // of the group of 128
+                    wait_loads<FULL ? (D - 1) * L + LW + NG + 4 * MB : LATER + LW>();
+                const int sub = QG == 5 ? kq : QG == 6 ? kq >> 1 : g & 1;     // of the group of 128 (128: of the byte)
+                const int half = QG == 7 ? (col * GQ + g) & 1 : sub & 1; // of the word
 #pragma unroll
                 for (int t = 0; t < T; ++t)
                 {
                     const uint8_t* at = slot + S_AT + (((t * 16 + col) * SPW + (SPW == 2 ? sub >> 1 : 0)) << 2);
-                    const uint32_t zb = at[NSL * 256];
-                    const uint32_t z = zps ? (zb >> ((sub & 1) * 4)) & 0xfu : (uint32_t)zp;
-                    scale_zero[t] = *reinterpret_cast<const uint16_t*>(at + (sub & 1) * 2) | (z << 16);
+                    const int byte = BITS == 8 ? (QG == 7 ? 0 : sub) : QG == 5 ? sub >> 1 : 0;
+                    const uint32_t zb = slot[S_AT + NSL * 256 + (((t * 16 + col) * ZPB + byte) << 2)];
+                    const uint32_t z = !zps ? (uint32_t)zp : BITS == 8 ? zb : (zb >> ((sub & 1) * 4)) & 0xfu;
+                    scale_zero[t] = *reinterpret_cast<const uint16_t*>(at + half * 2) | (z << 16);
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if constexpr (FULL)
                     fetch_s(gn, at_slot);
             }
-            uintx4 wnext;
+            uintx4 wnext[NW];
             half_t snext = (half_t)0.f;
             auto read_w = [&](auto t_c) {
                 constexpr int t = decltype(t_c)::value;
                 wait_w(t_c);
-                wnext = *reinterpret_cast<const uintx4*>(slot + W_AT + t * 1024 + w_rd);
+#pragma unroll
+                for (int c = 0; c < NW; ++c)
+                    wnext[c] = *reinterpret_cast<const uintx4*>(slot + W_AT + t * WB + w_rd[c]);
                 if constexpr (QG == 0)
                     snext = *reinterpret_cast<const half_t*>(sc_rd + t * 2048);
             };
@@ -370,7 +425,15 @@ namespace nnf
                 constexpr int t = decltype(t_c)::value;
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);
-                const uintx4 wv = wnext;
+                uint32_t ww[4 * NW];
+#pragma unroll
+                for (int c = 0; c < NW; ++c)
+                {
+                    ww[4 * c] = wnext[c].x;
+                    ww[4 * c + 1] = wnext[c].y;
+                    ww[4 * c + 2] = wnext[c].z;
+                    ww[4 * c + 3] = wnext[c].w;
+                }
                 const float scale = (float)snext;
                 if constexpr (FULL)
                     fetch_w(gn, t, at_slot);
@@ -389,11 +452,10 @@ namespace nnf
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
                     sum[mb] = QG ? acc[t][mb] : floatx4{0.f, 0.f, 0.f, 0.f};
-                const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
-                    const uintx4 bq = unpack(ww[j], j, lo, hi, scale2);
+                    const uintx4 bq = unpack(ww[NW * j], ww[NW * j + NW - 1], j, lo, hi, scale2);
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb)
                         sum[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[mb][j]),
@@ -566,12 +628,12 @@ namespace nnf
 
     namespace
     {
-        template <int T, int MB, bool RMS, int QG>
+        template <int T, int MB, bool RMS, int QG, int BITS>
         hipError_t launch_kstream(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                   void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync, const void* zps)
         {
-            auto kernel = &w4a16_kstream_kernel<T, MB, RMS, QG>;
-            const size_t lds = workspace::kstream_lds_bytes(T, MB, RMS, QG);
+            auto kernel = &w4a16_kstream_kernel<T, MB, RMS, QG, BITS>;
+            const size_t lds = workspace::kstream_lds_bytes(T, MB, RMS, QG, BITS);
             if (lds > MAX_LDS_BYTES)
                 return hipErrorInvalidValue;
             static LdsGrant granted;
@@ -582,26 +644,27 @@ namespace nnf
                                       fusion.rms_eps};
             hipLaunchKernelGGL(kernel, dim3(plan.grid, plan.ranges, plan.row_blocks), dim3(KS_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
                                (const half_t*)S, (half_t*)Y, N, K, plan.tiles_q | (plan.tiles_r << 16),
-                               M | (zp << 13) | (fusion.gate ? 1 << 17 : 0) | (plan.range_groups << 18), plan.ranges > 1 ? partial : nullptr,
+                               (int)((unsigned)(M | (zp << 13) | (fusion.gate ? 1 << 21 : 0)) | ((unsigned)(plan.ranges > 1 ? plan.range_groups : 1023) << 22)), plan.ranges > 1 ? partial : nullptr,
                                plan.ranges > 1 ? sync : nullptr, args, (const uint8_t*)zps);
             return hipGetLastError();
         }
-        template <int MB, int QG>
+        template <int MB, int QG, int BITS>
         hipError_t launch_kstream_t(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                     void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync, const void* zps)
         {
             hipError_t e = hipErrorInvalidValue;
             unroll_for<1, workspace::KSTREAM_MAX_TILES + 1>([&](auto t) {
-                if (plan.tiles == t.value)
-                    e = fusion.gamma ? launch_kstream<t.value, MB, true, QG>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps)
-                                     : launch_kstream<t.value, MB, false, QG>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps);
+                if constexpr (workspace::kstream_lds_bytes(t.value, MB, false, QG, BITS) <= MAX_LDS_BYTES)
+                    if (plan.tiles == t.value)
+                        e = fusion.gamma ? launch_kstream<t.value, MB, true, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps)
+                                         : launch_kstream<t.value, MB, false, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps);
             });
             return e;
         }
     } // namespace
 
     // QG: 0 groups of 128 and a scalar zero point, else the group's log2, with zero points from `zps` (or null: zp)
-    template <int QG>
+    template <int QG, int BITS = 4>
     hipError_t launch_w4a16_kstream_g(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                       void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync,
                                       const void* zps)
@@ -612,7 +675,7 @@ namespace nnf
         hipError_t e = hipErrorInvalidValue;
         unroll_for<1, 5>([&](auto mb) {
             if (plan.row_tiles == mb.value)
-                e = launch_kstream_t<mb.value, QG>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps);
+                e = launch_kstream_t<mb.value, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps);
         });
         return e;
     }

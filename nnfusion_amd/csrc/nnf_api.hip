@@ -168,20 +168,28 @@ namespace
         return x < y + b_bytes && y < x + a_bytes;
     }
 
-    // 4-bit weights with other block parameters on the K-streaming kernel, the nodes around the product inside it; taken = false: not one of
+    // 4-bit weights with other block parameters and 8-bit weights on the K-streaming kernel, the nodes around the product inside it; taken = false: not one of
     // its products (workspace::kstream_choice_q), nothing was launched.  (Workgroups still read A when others write Y: not there.)
     int wna16_kstream(hipStream_t s, const void* A, const void* Wq, const void* scales, void* Y, int M, int N, int K, const nnf_quant* q,
                       const nnf::GemvFusion& fusion, int num_cu, bool& taken)
     {
         taken = false;
-        if (q->bits != 4 || overlap(A, (size_t)M * K * 2, Y, (size_t)M * N * 2))
+        if (overlap(A, (size_t)M * K * 2, Y, (size_t)M * N * 2))
             return NNF_OK;
         const int gs = group_shift_of(q->group);
-        const nnf::workspace::KstreamPlan plan = nnf::workspace::kstream_choice_q(M, N, K, gs, num_cu, fusion.gate, fusion.gamma != nullptr);
+        const nnf::workspace::KstreamPlan plan =
+            q->bits == 8 ? nnf::workspace::kstream_choice_b8(M, N, K, gs, num_cu, fusion.gate, fusion.gamma != nullptr, fusion.any(),
+                                                                             q->zero_points != nullptr)
+                         : nnf::workspace::kstream_choice_q(M, N, K, gs, num_cu, fusion.gate, fusion.gamma != nullptr);
         if (plan.tiles == 0)
             return NNF_OK;
         taken = true;
-        const auto launch = gs == 5 ? nnf::launch_w4a16_kstream_q5 : gs == 6 ? nnf::launch_w4a16_kstream_q6 : nnf::launch_w4a16_kstream_q7;
+        const auto launch = q->bits == 8 ? (gs == 5   ? nnf::launch_w8a16_kstream_q5
+                                            : gs == 6 ? nnf::launch_w8a16_kstream_q6
+                                                      : nnf::launch_w8a16_kstream_q7)
+                            : gs == 5 ? nnf::launch_w4a16_kstream_q5
+                            : gs == 6 ? nnf::launch_w4a16_kstream_q6
+                                      : nnf::launch_w4a16_kstream_q7;
         return (int)launch(s, plan, A, Wq, scales, Y, M, N, K, q->zero_point, q->zero_points, fusion);
     }
 
@@ -411,9 +419,9 @@ namespace
         taken = false;
         // (RMSNorm of a few rows inside that kernel where it is inside the row-streaming kernels as well or SiLU-gate follows; otherwise a
         // launch ahead of it, so that the fused product stays the nodes' own arithmetic, bit for bit)
-        if (fusion.gamma && !fusion.gate && M <= 32 && !nnf::workspace::mrows_q_norm_inside(M, K))
+        if (q->bits == 4 && fusion.gamma && !fusion.gate && M <= 32 && !nnf::workspace::mrows_q_norm_inside(M, K))
         {
-            if (q->bits == 4 && nnf::workspace::kstream_choice_q(M, N, K, group_shift_of(q->group), num_cu, false, false).tiles > 0)
+            if (nnf::workspace::kstream_choice_q(M, N, K, group_shift_of(q->group), num_cu, false, false).tiles > 0)
             {
                 nnf::GemvFusion behind = fusion;
                 behind.gamma = nullptr;

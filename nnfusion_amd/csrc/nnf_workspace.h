@@ -1055,18 +1055,19 @@ namespace nnf
         constexpr int kstream_depth(int tiles, int mb) { return tiles == 1 && mb == 1 ? 2 : 1; }
         constexpr int kstream_ring(int mb) { return mb < 4 ? mb : 3; }
         // qg: 0, or log2 of the group of other block parameters, whose scales and zero points come chunk by chunk: words of 16 rows, two of
-        // them a group of 128 for groups of 32, 64 a load, and as many loads of zero points
+        // them a group of 128 for groups of 32, 64 a load; of zero points as many bytes, a lane each
         constexpr int kstream_scale_loads(int tiles, int qg) { return (tiles * 16 * (qg == 5 ? 2 : 1) + 63) / 64; }
-        constexpr int kstream_wave_bytes(int tiles, int mb, bool rms, int qg = 0)
+        constexpr int kstream_zero_loads(int tiles, int qg, int bits) { return (tiles * 16 * (bits == 8 ? 1 << (7 - qg) : qg == 5 ? 2 : 1) + 63) / 64; }
+        constexpr int kstream_wave_bytes(int tiles, int mb, bool rms, int qg = 0, int bits = 4)
         {
-            return kstream_depth(tiles, mb) *
-                   (kstream_ring(mb) * 4096 + tiles * 1024 + (rms ? 256 : 0) + (qg ? 2 * kstream_scale_loads(tiles, qg) * 256 : 0));
+            return kstream_depth(tiles, mb) * (kstream_ring(mb) * 4096 + tiles * 256 * bits + (rms ? 256 : 0) +
+                                               (qg ? (kstream_scale_loads(tiles, qg) + kstream_zero_loads(tiles, qg, bits)) * 256 : 0));
         }
         // tiles whose eight partial sums are in LDS at a time (an even number where there is more than one round)
         constexpr int kstream_round(int tiles, int mb) { return mb == 4 && tiles > 4 ? 4 : tiles; }
-        constexpr size_t kstream_lds_bytes(int tiles, int mb, bool rms, int qg = 0)
+        constexpr size_t kstream_lds_bytes(int tiles, int mb, bool rms, int qg = 0, int bits = 4)
         {
-            const size_t stream = (size_t)KSTREAM_WAVES * kstream_wave_bytes(tiles, mb, rms, qg) + (qg ? 0 : (size_t)tiles * 2048);
+            const size_t stream = (size_t)KSTREAM_WAVES * kstream_wave_bytes(tiles, mb, rms, qg, bits) + (qg ? 0 : (size_t)tiles * 2048);
             const size_t sums = (size_t)4096 + (size_t)KSTREAM_WAVES * kstream_round(tiles, mb) * mb * 1024;
             return stream > sums ? stream : sums;
         }
@@ -1081,7 +1082,7 @@ namespace nnf
             size_t partial_bytes = 0; // more than one range of K: their fp32 sums
         };
         // N: output columns (gate: from 2 N weight rows); more than one range of K: not with RMSNorm or SiLU-gate
-        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges, int row_blocks = 1, int qg = 0)
+        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges, int row_blocks = 1, int qg = 0, int bits = 4)
         {
             KstreamPlan p;
             const int mb = ((M + row_blocks - 1) / row_blocks + 15) / 16, G = K >> 7;
@@ -1092,12 +1093,12 @@ namespace nnf
             const int grid = n_tiles < per_range ? n_tiles : per_range;
             const int tiles = (gate ? 2 : 1) * ((n_tiles + grid - 1) / grid);
             // (a range's scales: rows of 32 words, from a half word where rows or ranges start in the middle of one)
-            if (qg ? ranges > 1 || (K & 255) || (size_t)(gate ? 2 : 1) * N * (K >> qg) >= ((size_t)1 << 31)
+            if (qg ? ranges > 1 || G > 1023 || (size_t)(gate ? 2 : 1) * N * (K >> qg) >= ((size_t)1 << 31)
                    : rg > ((G & 1) || ranges > 1 ? KSTREAM_MAX_GROUPS - 2 : KSTREAM_MAX_GROUPS))
                 return p;
             if ((ranges - 1) * rg >= G ||
-                ((G & 1) && ((N & 1) || (size_t)(gate ? 2 : 1) * N * G >= ((size_t)1 << 31))) || tiles > KSTREAM_MAX_TILES ||
-                kstream_lds_bytes(tiles, mb, rms, qg) > LDS_BYTES_PER_CU)
+                ((G & 1) && (qg == 0 || qg == 7) && ((N & 1) || (size_t)(gate ? 2 : 1) * N * G >= ((size_t)1 << 31))) || tiles > KSTREAM_MAX_TILES ||
+                kstream_lds_bytes(tiles, mb, rms, qg, bits) > LDS_BYTES_PER_CU)
                 return p;
             p.tiles = tiles;
             p.row_tiles = mb;
@@ -1115,11 +1116,11 @@ namespace nnf
         // and blocks of rows that apply; 11 % rms, and what it picks is within 4 % of the fastest but for 15 of them, 19 % at most): a chunk of eight
         // groups takes what its loads and its unpacking take, a little less where fewer CUs fetch the activations; ranges of K pay for
         // the sums' way through memory.
-        inline int kstream_estimate(const KstreamPlan& p)
+        inline int kstream_estimate(const KstreamPlan& p, int bits = 4)
         {
             const int chunks = (p.range_groups + KSTREAM_WAVES - 1) / KSTREAM_WAVES, workgroups = p.grid * p.ranges * p.row_blocks;
             const int mb = p.row_tiles, t = p.tiles;
-            return chunks * (17 + 27 * mb + 16 * t + 9 * mb * t) * (358 + (workgroups < 256 ? workgroups : 256)) / 614 + 200 + 6 * t + 15 * mb * t +
+            return chunks * (17 + 27 * mb + (bits == 8 ? 24 : 16) * t + 9 * mb * t) * (358 + (workgroups < 256 ? workgroups : 256)) / 614 + 200 + 6 * t + 15 * mb * t +
                    (p.ranges > 1 ? 84 + 20 * p.ranges + 60 * t : 0);
         }
         // What the library runs on it by itself, from measurements against the kernels that served these products before.  33 .. 64 rows:
@@ -1173,7 +1174,7 @@ namespace nnf
             return best;
         }
         // The same kernel for 4-bit weights in groups of 2^qg with a scalar zero point or one per (row, group): what the library runs on it, from
-        // measurements of 560 products against the row-streaming kernels of these parameters and the tile GEMM (time there / here).  Up to 16 rows:
+        // measurements of 1050 products against the row-streaming kernels of these parameters and the tile GEMM (time there / here).  Up to 16 rows:
         // K = 2048 / 4096 / 8192 0.85 - 1.1, with RMSNorm 1.01 - 1.9 (SiLU-gate beyond four tiles a workgroup 0.84 - 1.07); other K 1.05 - 2.2, above 8192 from
         // 4096 columns on 1.06 - 1.28 up to two tiles (0.89 - 1.1 outside).  17 .. 32 rows 0.98 - 2.7, 33 .. 64 1.02 - 2.4 (two tiles and more of
         // four blocks of rows beyond K = 8192 0.91 - 1.0), more rows up to K = 6144 1.02 - 2.2 (0.85 - 1.3 beyond).
@@ -1203,6 +1204,26 @@ namespace nnf
                 else if (!kstream_ahead_of_tiles(p, M, N, K, gate, rms))
                     continue;
                 if (best.tiles == 0 || kstream_estimate(p) < kstream_estimate(best))
+                    best = p;
+            }
+            return best;
+        }
+        // The same kernel for 8-bit weights in groups of 2^qg (fused: nodes around the product, which take passes of their own elsewhere), from
+        // measurements of 1140 products against the row-streaming kernel and the tile kernel (time there / here): 2 .. 16 rows 0.96 - 2.9, but
+        // plain products that the row-streaming kernel takes with a compile-time K 0.85 - 1.1: left there; 17 .. 64 rows 0.98 - 2.6
+        // (45 x 12288 x 4096 28.3 -> 18.2 us, with RMSNorm 31.5 -> 19.4), more rows 0.97 - 2.3 up to K = 8192 (0.82 - 1.1 beyond).
+        inline KstreamPlan kstream_choice_b8(int M, int N, int K, int qg, int num_cu, bool gate, bool rms, bool fused, bool zero_points)
+        {
+            KstreamPlan best;
+            if (M < 2 || M > 512 || qg < 5 || qg > 7 || (M > 64 && K > 8192) || (M <= 16 && !fused && w8a16_mrows_q_fits(M, N, K, qg, zero_points, num_cu)))
+                return best;
+            const int fewest = (M + 63) / 64, most = M <= 32 ? 1 : fewest + 2;
+            for (int row_blocks = fewest; row_blocks <= most; ++row_blocks)
+            {
+                const KstreamPlan p = kstream_plan(M, N, K, num_cu, gate, rms, 1, row_blocks, qg, 8);
+                if (p.tiles == 0)
+                    continue;
+                if (best.tiles == 0 || kstream_estimate(p, 8) < kstream_estimate(best, 8))
                     best = p;
             }
             return best;

@@ -1,0 +1,74 @@
+"""The K-streaming MFMA kernel on 8-bit weights in groups of 32 / 64 / 128 (w8a16_kstream_q{5,6,7}.hip), and on 4-bit weights whose rows hold an odd
+number of groups of 128 (scales of every other row start in the middle of a word).
+
+Sizes at the kernel's edges: rows around the blocks of 16 and blocks of rows, columns that are no multiple of 16, one to six tiles a workgroup
+(bytes of zero points come 64 a load, four a tile row with groups of 32), chunks with a single group, long K, odd numbers of columns (groups of
+128 in odd numbers go elsewhere then).  Tolerance: weights rounded to fp16 ahead of fp32 sums, 1e-2 of the result's RMS as for the other
+kernels of these parameters (SiLU-gate: two rounded products multiplied, twice that).
+"""
+import numpy as np
+import pytest
+
+import oracle
+from nnfusion_amd import datagen
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-2
+
+
+def _t(gpu, *arrays):
+    import torch
+
+    return [None if a is None else torch.from_numpy(np.ascontiguousarray(a)).to(gpu) for a in arrays]
+
+
+def _check(y, ref, tol):
+    y = y.cpu().numpy().astype(np.float32)
+    assert np.isfinite(y).all()
+    err = float(np.abs(y - ref.astype(np.float32)).max())
+    rms = float(np.sqrt(np.mean(np.asarray(ref, np.float64) ** 2)))
+    assert err <= tol * max(rms, 1e-6), (err, rms)
+
+
+@pytest.mark.parametrize("zero_points", [True, False], ids=["zero-points", "scalar"])
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("bits,m,n,k,form", [
+    (8, 2, 40, 1280, "plain"), (8, 16, 4112, 1536, "plain"), (8, 7, 8200, 2816, "residual"), (8, 12, 4096, 11008, "residual"),
+    (8, 17, 16, 1024, "plain"), (8, 33, 528, 2048, "residual"), (8, 49, 12288, 1024, "plain"), (8, 16, 24576, 1280, "plain"),
+    (8, 100, 1032, 2304, "plain"), (8, 300, 272, 1280, "residual"), (8, 5, 300, 1152, "rms"), (8, 9, 6144, 4096, "rms"), (8, 31, 72, 2432, "rms"),
+    (8, 64, 4128, 1280, "rms"), (8, 3, 2056, 1664, "gate"), (8, 16, 300, 8192, "gate"), (8, 45, 4100, 1024, "gate"), (8, 9, 301, 1152, "plain"),
+    (4, 5, 300, 1152, "plain"), (4, 20, 4130, 1664, "residual"), (4, 64, 272, 11136, "rms"), (4, 9, 302, 2432, "gate"), (4, 9, 301, 1152, "plain")])
+def test_products(gpu, bits, m, n, k, form, group, zero_points):
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case kstream_q bits={bits} M={m} N={n} K={k} {form} group={group} zero_points={zero_points}", flush=True)
+    zp = 7 if bits == 4 else 119
+    gate, rms = form == "gate", form in ("rms", "gate")
+    rows = 2 * n if gate else n
+    a, wq, s, z = datagen.wna16_case(5, m, rows, k, bits, group, zero_points)
+    rng = np.random.default_rng(3)
+    gamma = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float16) if rms else None
+    resid = rng.standard_normal((m, n)).astype(np.float16) if form == "residual" else None
+    ta, tw, ts, tz, tg, tr = _t(gpu, a, wq, s, z, gamma, resid)
+    w = oracle.dequantize_wn(wq, s, bits, group, zp, z).astype(np.float64)
+    x = a.astype(np.float64)
+    if rms:
+        x = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * gamma.astype(np.float64)
+    ref = x @ w.T
+    if gate:
+        ref = ref[:, :n] / (1.0 + np.exp(-ref[:, :n])) * ref[:, n:]
+    if resid is not None:
+        ref = ref + resid.astype(np.float64)
+    if form == "plain":
+        y = ops.wna16_gemm(ta, tw, ts, bits, group, zp, tz)
+        again = ops.wna16_gemm(ta, tw, ts, bits, group, zp, tz)
+    else:
+        y = ops.wna16_gemm_fused(ta, tw, ts, bits, group, zp, tz, rms_gamma=tg, residual=tr, act=1 if gate else 0)
+        out = tr.clone() if tr is not None else None  # the residual in place
+        again = ops.wna16_gemm_fused(ta, tw, ts, bits, group, zp, tz, rms_gamma=tg, residual=out, act=1 if gate else 0, out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(y, again)
+    _check(y, ref, 2 * TOL if gate else TOL)

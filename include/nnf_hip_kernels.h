@@ -73,9 +73,10 @@ NNF_API const char* nnf_status_string(int status);
  * fp16 x int4 (group-scaled) GEMM / GEMV:  Y[M,N] = A[M,K] . ((Wq - zp) * scales)^T
  * Replaces the cublasHgemm / cublasSgemm call of cuda::Dot (cuda_gpu/kernels/dot.cpp:128-205,
  * :271-363) for a weight-quantized Dot node with transpose_B = true.  By shape: M = 1 the row-streaming
- * GEMV kernel; 2 <= M <= 32 (40 up to K = 4096, 64 up to K = 2048) the row-streaming MFMA kernel, over ranges of K (partial sums in
- * `workspace`, then a reduction pass) where the activations exceed one workgroup's registers; other M <= 16
- * shapes the MFMA GEMV kernel over K ranges; everything else the MFMA tile GEMM, whose tiles are cut into equal parts of K or
+ * GEMV kernel; 2 <= M <= 16 the row-streaming MFMA kernel where K is one of its compile-time constants (most multiples of 1024 up
+ * to 8192); 17 <= M <= 64, and from 2 rows up to 1024 where it was measured ahead, the K-streaming MFMA kernel (over ranges of K only
+ * with synchronisation words: nnf_plan); other M <= 16 shapes the row-streaming kernel over ranges of K (partial sums in `workspace`, then a reduction
+ * pass) or the MFMA GEMV kernel; everything else the MFMA tile GEMM, whose tiles are cut into equal parts of K or
  * whose work is split evenly over the CUs (tiles shared by several workgroups are summed through `workspace` by a second launch).
  * ------------------------------------------------------------------------------------------- */
 NNF_API size_t nnf_w4a16_gemm_workspace_bytes(int M, int N, int K, int group);
@@ -146,7 +147,8 @@ typedef struct nnf_plan
      * Two more launches go the same way: a fused RMSNorm's rstd[] is computed by the GEMM launch itself (every
      * workgroup a few rows before its first tile; no pass of its own), and the row-streaming kernel for a few
      * activation rows and K above 8192, which works on ranges of K, adds the ranges up itself (the last workgroup to
-     * arrive at a group of columns, in the order of the ranges; no reduction pass).  W8A8 with 8 .. 32 rows and K from
+     * arrive at a group of columns, in the order of the ranges; no reduction pass).  Products of 17 .. 256 rows may run on the K-streaming
+     * kernel over ranges of K then, which they do not without (another order of sums: equal to rounding, not bit for bit).  W8A8 with 8 .. 32 rows and K from
      * 8192 runs its row-streaming kernel over two ranges of K the same way (int32 sums: exact), given sync_flags and
      * nnf_w8a8_gemm_variant_workspace_bytes of workspace; without either, in one pass over K (same bits, ~1 us more).
      *   sync_flags: device memory, 16-byte aligned, ALL ZERO before the first call that uses it; every call leaves it
@@ -188,7 +190,8 @@ NNF_API int nnf_w4a16_gemm_variant(nnf_stream_t stream,
  *                         the groups of a row, even group in the low nibble
  * bits 4, group 128 and no zero-point tensor is nnf_w4a16_gemm itself (same kernels, same workspace).  For every other
  * combination (group 32 / 64 / 128, K a multiple of group) 4-bit weights run on the kernels of nnf_w4a16_gemm where
- * those apply: the row-streaming kernels for M = 1 with K a multiple of 256 from 1024 to 16384 and for 2 <= M <= 16
+ * those apply: the K-streaming kernel for 2 .. 512 rows where it was measured ahead (no workspace; 8-bit weights too), else
+ * the row-streaming kernels for M = 1 with K a multiple of 256 from 1024 to 16384 and for 2 <= M <= 16
  * with K a multiple of 256 from about 2560 on (2048 / 4096 also up to 32 rows; above K = 8192 over ranges of K with a
  * reduction pass), and the tile GEMM for the other shapes above 16 rows with K a multiple of 256 and zero_points
  * 4-byte aligned.  The ranges of K and the tile GEMM want nnf_wna16_gemm_workspace_bytes of workspace; called with
@@ -260,9 +263,9 @@ enum nnf_activation
 };
 
 /* Same GEMM with prologue / epilogue in one call.  They run inside the kernel that serves the shape: the
- * row-streaming kernels (M = 1; M <= 64) and the tile GEMM multiply gamma in on the way in, rstd[m] and the
- * epilogue at their end.  The row-streaming kernels add up the squares of the activations they hold themselves
- * (K a multiple of 1024 up to 8192; M = 1: any K they take): one launch in all; the tile GEMM and the other
+ * K-streaming kernel (2 rows and more), the row-streaming kernels (M = 1; M <= 64) and the tile GEMM multiply gamma in on the way in, rstd[m] and the
+ * epilogue at their end.  The K-streaming kernel and the row-streaming kernels add up the squares of the activations they hold themselves
+ * (row-streaming: K a multiple of 1024 up to 8192; M = 1: any K they take): one launch in all; the tile GEMM and the other
  * forms take rstd from a small pre-pass over A (fp32 [M] in `workspace`); a GEMV kernel over ranges of K
  * leaves rstd and the epilogue to its reduction pass.  The MFMA GEMV kernel (M <= 16, other K) and the
  * row-streaming kernel where K is an odd multiple of 128, up to sixteen groups or above 32 rows read normalised

@@ -55,9 +55,9 @@ namespace nnf
     } // namespace
 
     // blockIdx.z: blocks of 16 MB activation rows.
-    // pack = M | zp << 13 | gate << 21 | range_groups << 22 (ten bits: one range where K / 128 takes more); tiles = tiles_q | tiles_r << 16: output tiles of a workgroup, one
-    // more for the first tiles_r (gate: twice as many weight tiles, the gate and the up tile of each in turn).
-    // LDS (bytes): per wavefront [RB][4096] activations | [T][1024] weights | (RMS) 256 gamma; then the scales of the
+    // pack = M | zp << 13 | gate << 21 | range_groups << 22 (ten bits, all set for one range); tiles = tiles_q | tiles_r << 16: output
+    // tiles of a workgroup, one more for the first tiles_r (gate: twice as many weight tiles, the gate and the up tile of each in turn).
+    // LDS (bytes): per wavefront [RB][4096] activations | [T][256 BITS] weights | (RMS) 256 gamma; then the scales of the
     //              workgroup's range of K, [T][16][32] words.  At the end, over all of it: (RMS) the wavefronts' sums of squares
     //              [8][16 MB] and rstd[16 MB] | from byte 4096 on the wavefronts' sums [8][tiles of a round][MB KiB].
     template <int T, int MB, bool RMS, int QG, int BITS>
@@ -267,8 +267,8 @@ namespace nnf
 
         // activations and gamma in the order in which the weights are unpacked: the pairs of the nibble trick, 8 bits memory order
         auto operand_order = [](uintx4 v) { return BITS == 8 ? v : permute_a8(v); };
-        // Loads of a wavefront in order: chunk by chunk [gamma] [MB blocks of activations] [QG: scales, zero points] [T tiles of weights]; those of chunk c + D
-        // (RB < MB: of the activations, the first RB blocks) are asked for during chunk c, each where its slot has just been
+        // Loads of a wavefront in order: chunk by chunk [gamma] [MB blocks of activations] [QG: scales, zero points] [T tiles of weights];
+        // those of chunk c + D (RB < MB: of the activations, the first RB blocks) are asked for during chunk c, each where its slot has just been
         // read.  Loads come back in order: the wait counts below are the loads that follow the one waited for.  AHEAD: the chunks still to come,
         // as far as they matter: below D nothing more is asked for.  Weights asked for ahead of the chunk's last activations
         // (RB < MB) need no wait of their own.
@@ -642,10 +642,12 @@ namespace nnf
                 return e;
             const GemvFusionArgs args{(const half_t*)fusion.gamma, nullptr, (const half_t*)fusion.bias, (const half_t*)fusion.residual,
                                       fusion.rms_eps};
-            hipLaunchKernelGGL(kernel, dim3(plan.grid, plan.ranges, plan.row_blocks), dim3(KS_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
-                               (const half_t*)S, (half_t*)Y, N, K, plan.tiles_q | (plan.tiles_r << 16),
-                               (int)((unsigned)(M | (zp << 13) | (fusion.gate ? 1 << 21 : 0)) | ((unsigned)(plan.ranges > 1 ? plan.range_groups : 1023) << 22)), plan.ranges > 1 ? partial : nullptr,
-                               plan.ranges > 1 ? sync : nullptr, args, (const uint8_t*)zps);
+            const unsigned pack = (unsigned)(M | (zp << 13) | (fusion.gate ? 1 << 21 : 0)) |
+                                  ((unsigned)(plan.ranges > 1 ? plan.range_groups : 1023) << 22);
+            hipLaunchKernelGGL(kernel, dim3(plan.grid, plan.ranges, plan.row_blocks), dim3(KS_WAVES * 64), lds, stream,
+                               (const half_t*)A, (const uint8_t*)Wq, (const half_t*)S, (half_t*)Y, N, K, plan.tiles_q | (plan.tiles_r << 16),
+                               (int)pack, plan.ranges > 1 ? partial : nullptr, plan.ranges > 1 ? sync : nullptr, args,
+                               (const uint8_t*)zps);
             return hipGetLastError();
         }
         template <int MB, int QG, int BITS>
@@ -656,8 +658,10 @@ namespace nnf
             unroll_for<1, workspace::KSTREAM_MAX_TILES + 1>([&](auto t) {
                 if constexpr (workspace::kstream_lds_bytes(t.value, MB, false, QG, BITS) <= MAX_LDS_BYTES)
                     if (plan.tiles == t.value)
-                        e = fusion.gamma ? launch_kstream<t.value, MB, true, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps)
-                                         : launch_kstream<t.value, MB, false, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps);
+                        e = fusion.gamma ? launch_kstream<t.value, MB, true, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial,
+                                                                                       sync, zps)
+                                         : launch_kstream<t.value, MB, false, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial,
+                                                                                        sync, zps);
             });
             return e;
         }

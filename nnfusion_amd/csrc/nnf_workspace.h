@@ -965,7 +965,8 @@ namespace nnf
         inline MrowsSplit w4a16_mrows_split(int M, int N, int K, int num_cu)
         {
             MrowsSplit sp;
-            // (33 .. 64 rows run on the kernel, but against the tile GEMM, measured alternately: 33 / 40 rows take 25.9 / 27.4 us
+            // (What follows decides scratch sizes and the forms without the K-streaming kernel, which serves most of these products:
+            // kstream_choice.)  (33 .. 64 rows run on the kernel, but against the tile GEMM, measured alternately: 33 / 40 rows take 25.9 / 27.4 us
             // against 29.1 / 29.3 at N = 22016, K = 4096 and 12.2 / 12.9 against 14.8 / 15.3 at N = K = 4096, are level at K = 8192 and
             // 11008, 8-10 % slower at K = 5120, and slower everywhere from about 48 rows on: taken up to 40 rows and K = 4096)
             // (8 .. 16 rows at K = 8192, up to 8192 weight rows: in one launch every workgroup fetches all M x 8192 activations
@@ -1028,7 +1029,8 @@ namespace nnf
             // counts (K = 1664 .. 1920 1.8 - 2.9 x, 3200 1.7 - 2.5, 3968 1.8 - 2.2).
             if (((K & 128) || gw == 1) && M < 8)
                 return false;
-            // 33 .. 64 rows, up to sixteen groups: four blocks of rows against the tile GEMM, 1152 / 4096 / 12288 / 22016 weight rows: K = 1280
+            // 33 .. 64 rows (the library's own choice is the K-streaming kernel there, 1.2 - 1.9 x; scratch sizes follow this rule), up to
+            // sixteen groups: four blocks of rows against the tile GEMM, 1152 / 4096 / 12288 / 22016 weight rows: K = 1280
             // 1.45 / 1.3 / 0.9 - 1.0 / 0.7 x, 1664 .. 2048 1.5 / 1.4 / 1.1 - 1.3 / 0.8 - 1.0; RMSNorm and SiLU-gate 1.5 / 1.5 / 1.2 - 1.4 / 1.0 - 1.3
             if (M > 32)
                 return gate ? 2 * N <= (K >= 1280 ? 22016 : 12288) : N <= (K >= 1408 ? 12288 : 8192);
@@ -1048,7 +1050,7 @@ namespace nnf
                 return false;
             return gw == 1 ? M == 8 && 4 * (K >> 7) >= 52 : (K & 128) && !mrows_stages_activations(M, K);
         }
-        // ---- 33 .. 64 activation rows: the K-streaming kernel (w4a16_kstream.hip) ----
+        // ---- 2 .. 1024 activation rows in blocks of up to 64: the K-streaming kernel (w4a16_kstream.h) ----
         // One workgroup per CU with up to KSTREAM_MAX_TILES 16-row weight tiles, their sums in registers; K in chunks of eight groups.
         constexpr int KSTREAM_WAVES = 8, KSTREAM_MAX_TILES = 6, KSTREAM_MAX_GROUPS = 64;
         // chunks asked for ahead; blocks of 16 rows x 256 bytes of activations in a slot of a wavefront's ring; its bytes of LDS
@@ -1057,7 +1059,10 @@ namespace nnf
         // qg: 0, or log2 of the group of other block parameters, whose scales and zero points come chunk by chunk: words of 16 rows, two of
         // them a group of 128 for groups of 32, 64 a load; of zero points as many bytes, a lane each
         constexpr int kstream_scale_loads(int tiles, int qg) { return (tiles * 16 * (qg == 5 ? 2 : 1) + 63) / 64; }
-        constexpr int kstream_zero_loads(int tiles, int qg, int bits) { return (tiles * 16 * (bits == 8 ? 1 << (7 - qg) : qg == 5 ? 2 : 1) + 63) / 64; }
+        constexpr int kstream_zero_loads(int tiles, int qg, int bits)
+        {
+            return (tiles * 16 * (bits == 8 ? 1 << (7 - qg) : qg == 5 ? 2 : 1) + 63) / 64;
+        }
         constexpr int kstream_wave_bytes(int tiles, int mb, bool rms, int qg = 0, int bits = 4)
         {
             return kstream_depth(tiles, mb) * (kstream_ring(mb) * 4096 + tiles * 256 * bits + (rms ? 256 : 0) +
@@ -1082,7 +1087,8 @@ namespace nnf
             size_t partial_bytes = 0; // more than one range of K: their fp32 sums
         };
         // N: output columns (gate: from 2 N weight rows); more than one range of K: not with RMSNorm or SiLU-gate
-        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges, int row_blocks = 1, int qg = 0, int bits = 4)
+        inline KstreamPlan kstream_plan(int M, int N, int K, int num_cu, bool gate, bool rms, int ranges, int row_blocks = 1, int qg = 0,
+                                        int bits = 4)
         {
             KstreamPlan p;
             const int mb = ((M + row_blocks - 1) / row_blocks + 15) / 16, G = K >> 7;

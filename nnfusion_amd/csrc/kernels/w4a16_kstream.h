@@ -29,6 +29,9 @@
 //   * RMS: rstd from the squares of the activations as they pass (fp32), applied to the sums; gamma[k] multiplies the
 //     unpacked weights, as in the tile GEMM: gamma times an activation alone may leave the range of fp16 (gamma / 16 times
 //     q - zp, of at most 15, does not).
+//     QG: scale times gamma is rounded to fp16 with the weight, and a small product of the two has few bits left there (5e-7: 1 %
+//     off); 16 times the scale, exact, moves that to products of 4e-8, and a weight times gamma reaches the end of
+//     fp16 at 4094, where sums of K >= 1024 of them are beyond fp16 as well.
 //   * Ranges of K (blockIdx.y): fp32 sums to scratch memory, added up in range order by the workgroup that arrives last,
 //     as in w4a16_mrows_any_kernel.
 #pragma once
@@ -287,7 +290,7 @@ namespace nnf
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
-                    // (QG: q - zp carries its scale already)
+                    // (QG: as it is, the factor 16 is on the scales)
                     const half2_t sixteenth = {(half_t)(QG ? 1.f : 0.0625f), (half_t)(QG ? 1.f : 0.0625f)};
                     const uintx4 g8 = operand_order(*reinterpret_cast<const uintx4*>(slot + G_AT + kq * 64 + j * 16));
                     gm[j] = uintx4{as_u32(as_half2(g8.x) * sixteenth), as_u32(as_half2(g8.y) * sixteenth), as_u32(as_half2(g8.z) * sixteenth),
@@ -447,6 +450,8 @@ namespace nnf
                     lo = as_half2(0xE400E400u | z2);
                     hi = as_half2(0xD400D400u | (z2 << 4));
                     scale2 = as_half2(s1 | (s1 << 16));
+                    if constexpr (RMS)
+                        scale2 *= half2_t{(half_t)16.f, (half_t)16.f};
                 }
                 floatx4 sum[MB];
 #pragma unroll
@@ -504,7 +509,7 @@ namespace nnf
 #pragma unroll
                 for (int w = 0; w < KS_WAVES; ++w)
                     total += sum_sq[w * (MB * 16) + tid];
-                rstd[tid] = (QG ? 1.0f : 16.0f) / __builtin_sqrtf(total / (float)K + f.rms_eps); // (gamma / 16, above)
+                rstd[tid] = (QG ? 0.0625f : 16.0f) / __builtin_sqrtf(total / (float)K + f.rms_eps); // (gamma / 16, or 16 times the scales, above)
             }
         }
         const int n_tiles = (N + 15) / 16;

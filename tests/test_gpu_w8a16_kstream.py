@@ -72,3 +72,29 @@ def test_products(gpu, bits, m, n, k, form, group, zero_points):
     torch.cuda.synchronize()
     assert torch.equal(y, again)
     _check(y, ref, 2 * TOL if gate else TOL)
+
+
+@pytest.mark.parametrize("bits,group,m,n,k,gate", [(4, 32, 40, 72, 4096, False), (4, 64, 64, 40, 1280, True), (4, 128, 16, 300, 2304, True),
+                                                   (8, 32, 5, 300, 1152, False), (8, 128, 45, 72, 4096, False), (8, 64, 9, 302, 2560, True)])
+def test_small_rms_norm_weight(gpu, bits, group, m, n, k, gate):
+    """A weight's scale times gamma of 7.7e-7 (8 bits: 4.8e-8), where fp16 keeps a few bits of a weight.  The 2-norm of the error: the roundings of
+    the weight times its scale and of that times gamma (16 times as large), 2^-11 / sqrt(3) each, and of the output: 1e-3 (3.9e-4 in this
+    arithmetic on the CPU, 3.2e-3 without the factor 16), and the output's own spacing of 2^-24 where it is a subnormal number."""
+    from nnfusion_amd import ops
+
+    print(f"case small gamma bits={bits} group={group} M={m} N={n} K={k} gate={gate}", flush=True)
+    zp = 7 if bits == 4 else 119
+    a, wq, s, z = datagen.wna16_case(6, m, 2 * n if gate else n, k, bits, group, True)
+    s = (s.astype(np.float32) / 16).astype(np.float16)
+    if gate: # (the product of the two within the range of fp16)
+        s[n:] = (s[n:].astype(np.float32) * 512).astype(np.float16)
+    gamma = ((1.0 + 0.1 * np.random.default_rng(4).standard_normal(k)) / 1024).astype(np.float16)
+    ta, tw, ts, tz, tg = _t(gpu, a, wq, s, z, gamma)
+    x = a.astype(np.float64)
+    x = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * gamma.astype(np.float64)
+    q = oracle.dequantize_wn(wq, np.ones_like(s), bits, group, zp, z).astype(np.float64)
+    ref = x @ (q * np.repeat(s.astype(np.float64), group, axis=1)).T
+    if gate:
+        ref = ref[:, :n] / (1.0 + np.exp(-ref[:, :n])) * ref[:, n:]
+    y = ops.wna16_gemm_fused(ta, tw, ts, bits, group, zp, tz, rms_gamma=tg, act=1 if gate else 0).cpu().numpy().astype(np.float64)
+    assert np.linalg.norm(y - ref) <= (1e-3 + 2.0 ** -24 / np.sqrt(12 * np.mean(ref ** 2))) * np.linalg.norm(ref)

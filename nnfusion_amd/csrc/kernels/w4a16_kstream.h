@@ -27,8 +27,8 @@
 //     row-streaming kernel on bytes, the tile kernel and the passes of the nodes around them: 45 x 12288 x 4096 28.3 -> 18.2 us
 //     (16.0 at 32 rows, where the weights alone bound it), 16 x 4096 x 4096 with RMSNorm and SiLU-gate 17.0 -> 12.9, 5 x 1000 x 1280 5.4 -> 3.9.
 //   * RMS: rstd from the squares of the activations as they pass (fp32), applied to the sums; gamma[k] multiplies the
-//     unpacked weights, as in the tile GEMM: gamma times an activation alone may leave the range of fp16 (gamma / 16 times
-//     q - zp, of at most 15, does not).
+//     unpacked weights, as in the tile GEMM: gamma times an activation alone may leave the range of fp16.  The weights are unpacked to
+//     (q - zp) / 16 there, by other exponents of the same trick: at most 15 / 16 of gamma, and rounded once where gamma is small.
 //     QG: scale times gamma is rounded to fp16 with the weight, and a small product of the two has few bits left there (5e-7: 1 %
 //     off); 16 times the scale, exact, moves that to products of 4e-8, and a weight times gamma reaches the end of
 //     fp16 at 4094, where sums of K >= 1024 of them are beyond fp16 as well.
@@ -87,8 +87,17 @@ namespace nnf
         constexpr int RT = workspace::kstream_round(T, MB); // tiles whose sums are in LDS at a time
         extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
         uint32_t MAGIC, MAGIC_HI, MASK_LO, MASK_HI;
-        asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(MAGIC));
-        asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(MAGIC_HI));
+        constexpr bool SIXTEENTHS = RMS && QG == 0; // (q - zp) / 16: in the mantissas of 64.0 and 4.0
+        if constexpr (SIXTEENTHS)
+        {
+            asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(MAGIC));
+            asm volatile("v_mov_b32 %0, 0x44004400" : "=v"(MAGIC_HI));
+        }
+        else
+        {
+            asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(MAGIC));
+            asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(MAGIC_HI));
+        }
         asm volatile("s_mov_b32 %0, 0x000F000F" : "=s"(MASK_LO));
         asm volatile("s_mov_b32 %0, 0x00F000F0" : "=s"(MASK_HI));
 
@@ -239,7 +248,8 @@ namespace nnf
             wait_loads<D*(NG + 4 * RB + LW)>(); // the scales
         lds_barrier();
 
-        const half_t clo = (half_t)(-(1024.0f + (float)zp)), chi = (half_t)(-(64.0f + (float)zp)); // exact
+        const half_t clo = (half_t)(SIXTEENTHS ? -(64.0f + (float)zp * 0.0625f) : -(1024.0f + (float)zp)),
+                     chi = (half_t)(SIXTEENTHS ? -(4.0f + (float)zp * 0.0625f) : -(64.0f + (float)zp)); // exact
         const half2_t c_lo = {clo, clo}, c_hi = {chi, chi};
         floatx4 acc[T][MB];
 #pragma unroll
@@ -289,13 +299,7 @@ namespace nnf
                 wait_loads<LATER + 4 * RB + NS + LW>();
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                {
-                    // (QG: as it is, the factor 16 is on the scales)
-                    const half2_t sixteenth = {(half_t)(QG ? 1.f : 0.0625f), (half_t)(QG ? 1.f : 0.0625f)};
-                    const uintx4 g8 = operand_order(*reinterpret_cast<const uintx4*>(slot + G_AT + kq * 64 + j * 16));
-                    gm[j] = uintx4{as_u32(as_half2(g8.x) * sixteenth), as_u32(as_half2(g8.y) * sixteenth), as_u32(as_half2(g8.z) * sixteenth),
-                                   as_u32(as_half2(g8.w) * sixteenth)};
-                }
+                    gm[j] = operand_order(*reinterpret_cast<const uintx4*>(slot + G_AT + kq * 64 + j * 16));
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if constexpr (FULL)
                     fetch_gamma(gn, at_slot);
@@ -509,7 +513,7 @@ namespace nnf
 #pragma unroll
                 for (int w = 0; w < KS_WAVES; ++w)
                     total += sum_sq[w * (MB * 16) + tid];
-                rstd[tid] = (QG ? 0.0625f : 16.0f) / __builtin_sqrtf(total / (float)K + f.rms_eps); // (gamma / 16, or 16 times the scales, above)
+                rstd[tid] = (QG ? 0.0625f : 16.0f) / __builtin_sqrtf(total / (float)K + f.rms_eps); // (sixteenths of weights, or 16 times the scales, above)
             }
         }
         const int n_tiles = (N + 15) / 16;

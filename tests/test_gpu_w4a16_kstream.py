@@ -107,3 +107,20 @@ def test_rms_norm(gpu, m, n, k, spread, gate):
         _check(y, ref, 2 * TOL)
     else:
         _check(y, ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(4, 40, 1152), (16, 2050, 2560), (45, 300, 1152)])
+def test_small_rms_norm_weight(gpu, m, n, k):
+    """gamma of about 2^-14: a sixteenth of it alone has six bits in fp16 (4e-3 of the 2-norm), of weights times it the largest ten.  Bound: the
+    products of gamma and a sixteenth of a weight, 4.6 / 16 of gamma in the root mean square and 2^-24 apart, 1e-3; the output, 2^-24 apart below 2^-14."""
+    from nnfusion_amd import ops
+
+    a, wq, s = datagen.w4a16_case(9, m, n, k)
+    gamma = ((1.0 + 0.1 * np.random.default_rng(2).standard_normal(k)) / 16384).astype(np.float16)
+    ta, tw, ts, tg = _t(gpu, a, wq, s, gamma)
+    y = ops.w4a16_gemm_fused(ta, tw, ts, rms_gamma=tg, workspace=_ws(gpu), sync=ops.sync_flags(gpu)).cpu().numpy().astype(np.float64)
+    x = a.astype(np.float64)
+    x = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * gamma.astype(np.float64)
+    q = oracle.dequantize_w4(wq, np.ones_like(s)).astype(np.float64)
+    ref = x @ (q * np.repeat(s.astype(np.float64), 128, axis=1)).T
+    assert np.linalg.norm(y - ref) <= (1.3e-3 + 2.0 ** -24 / np.sqrt(12 * np.mean(ref ** 2))) * np.linalg.norm(ref)

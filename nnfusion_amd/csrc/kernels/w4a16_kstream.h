@@ -27,8 +27,9 @@
 //     row-streaming kernel on bytes, the tile kernel and the passes of the nodes around them: 45 x 12288 x 4096 28.3 -> 18.2 us
 //     (16.0 at 32 rows, where the weights alone bound it), 16 x 4096 x 4096 with RMSNorm and SiLU-gate 17.0 -> 12.9, 5 x 1000 x 1280 5.4 -> 3.9.
 //   * RMS: rstd from the squares of the activations as they pass (fp32), applied to the sums; gamma[k] multiplies the
-//     unpacked weights, as in the tile GEMM: gamma times an activation alone may leave the range of fp16.  The weights are unpacked to
-//     (q - zp) / 16 there, by other exponents of the same trick: at most 15 / 16 of gamma, and rounded once where gamma is small.
+//     unpacked weights, as in the tile GEMM: gamma times an activation alone may leave the range of fp16.  (q - zp) times gamma is rounded
+//     to eleven bits, as a normalised activation is in a pass of its own: at most 15 gamma, and a multiple of 2^-24 like gamma, so exact where it
+//     is a subnormal number.  Gamma is used as it is, a sixteenth of it where a group has one of 4096 and more (16 on that group's sum).
 //     QG: scale times gamma is rounded to fp16 with the weight, and a small product of the two has few bits left there (5e-7: 1 %
 //     off); 16 times the scale, exact, moves that to products of 4e-8, and a weight times gamma reaches the end of
 //     fp16 at 4094, where sums of K >= 1024 of them are beyond fp16 as well.
@@ -87,17 +88,8 @@ namespace nnf
         constexpr int RT = workspace::kstream_round(T, MB); // tiles whose sums are in LDS at a time
         extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
         uint32_t MAGIC, MAGIC_HI, MASK_LO, MASK_HI;
-        constexpr bool SIXTEENTHS = RMS && QG == 0; // (q - zp) / 16: in the mantissas of 64.0 and 4.0
-        if constexpr (SIXTEENTHS)
-        {
-            asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(MAGIC));
-            asm volatile("v_mov_b32 %0, 0x44004400" : "=v"(MAGIC_HI));
-        }
-        else
-        {
-            asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(MAGIC));
-            asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(MAGIC_HI));
-        }
+        asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(MAGIC));
+        asm volatile("v_mov_b32 %0, 0x54005400" : "=v"(MAGIC_HI));
         asm volatile("s_mov_b32 %0, 0x000F000F" : "=s"(MASK_LO));
         asm volatile("s_mov_b32 %0, 0x00F000F0" : "=s"(MASK_HI));
 
@@ -248,8 +240,7 @@ namespace nnf
             wait_loads<D*(NG + 4 * RB + LW)>(); // the scales
         lds_barrier();
 
-        const half_t clo = (half_t)(SIXTEENTHS ? -(64.0f + (float)zp * 0.0625f) : -(1024.0f + (float)zp)),
-                     chi = (half_t)(SIXTEENTHS ? -(4.0f + (float)zp * 0.0625f) : -(64.0f + (float)zp)); // exact
+        const half_t clo = (half_t)(-(1024.0f + (float)zp)), chi = (half_t)(-(64.0f + (float)zp)); // exact
         const half2_t c_lo = {clo, clo}, c_hi = {chi, chi};
         floatx4 acc[T][MB];
 #pragma unroll
@@ -294,12 +285,14 @@ namespace nnf
             const int g = group_of(c), gn = group_of(c + D);
             const uint8_t* slot = at_slot;
             uintx4 gm[4];
+            uint32_t gamma_own = 0; // two of the group's 128, without their signs
             if constexpr (RMS)
             {
                 wait_loads<LATER + 4 * RB + NS + LW>();
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     gm[j] = operand_order(*reinterpret_cast<const uintx4*>(slot + G_AT + kq * 64 + j * 16));
+                gamma_own = *reinterpret_cast<const uint32_t*>(slot + G_AT + lane * 4) & 0x7fff7fffu;
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if constexpr (FULL)
                     fetch_gamma(gn, at_slot);
@@ -395,6 +388,12 @@ namespace nnf
             };
             uintx4 areg[MB][4];
             unroll_for<0, MB>([&](auto p_c) { read_a(p_c, areg[decltype(p_c)::value]); });
+            bool large = false;
+            if constexpr (RMS && QG == 0)
+            {
+                const uint32_t own_largest = max(gamma_own & 0xffffu, gamma_own >> 16);
+                large = __builtin_amdgcn_ballot_w64(own_largest >= 0x6c00u) != 0; // 4096.0 and more: 15 times it may leave fp16
+            }
             // QG: scale (low half) and zero point of the lane's 32 weights of every tile: group (128 g + 32 kq) >> QG of row col
             uint32_t scale_zero[QG ? T : 1];
             if constexpr (QG != 0)
@@ -428,6 +427,17 @@ namespace nnf
                     snext = *reinterpret_cast<const half_t*>(sc_rd + t * 2048);
             };
             read_w(std::integral_constant<int, 0>());
+            float sum_factor = 1.0f; // (RMS, scales on the sums) the reciprocal of what gamma is multiplied by
+            if constexpr (RMS && QG == 0)
+                if (large)
+                {
+                    sum_factor = 16.0f;
+                    const half2_t sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        gm[j] = uintx4{as_u32(as_half2(gm[j].x) * sixteenth), as_u32(as_half2(gm[j].y) * sixteenth),
+                                       as_u32(as_half2(gm[j].z) * sixteenth), as_u32(as_half2(gm[j].w) * sixteenth)};
+                }
             unroll_for<0, T>([&](auto t_c) {
                 constexpr int t = decltype(t_c)::value;
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -441,7 +451,7 @@ namespace nnf
                     ww[4 * c + 2] = wnext[c].z;
                     ww[4 * c + 3] = wnext[c].w;
                 }
-                const float scale = (float)snext;
+                const float scale = RMS ? (float)snext * sum_factor : (float)snext;
                 if constexpr (FULL)
                     fetch_w(gn, t, at_slot);
                 if constexpr (t + 1 < T)
@@ -513,7 +523,7 @@ namespace nnf
 #pragma unroll
                 for (int w = 0; w < KS_WAVES; ++w)
                     total += sum_sq[w * (MB * 16) + tid];
-                rstd[tid] = (QG ? 0.0625f : 16.0f) / __builtin_sqrtf(total / (float)K + f.rms_eps); // (sixteenths of weights, or 16 times the scales, above)
+                rstd[tid] = (QG ? 0.0625f : 1.0f) / __builtin_sqrtf(total / (float)K + f.rms_eps);
             }
         }
         const int n_tiles = (N + 15) / 16;

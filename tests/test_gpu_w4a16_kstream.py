@@ -124,3 +124,32 @@ def test_small_rms_norm_weight(gpu, m, n, k):
     q = oracle.dequantize_w4(wq, np.ones_like(s)).astype(np.float64)
     ref = x @ (q * np.repeat(s.astype(np.float64), 128, axis=1)).T
     assert np.linalg.norm(y - ref) <= (1.3e-3 + 2.0 ** -24 / np.sqrt(12 * np.mean(ref ** 2))) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(4, 40, 1152), (16, 2050, 2560), (45, 300, 1152), (70, 72, 1024)])
+@pytest.mark.parametrize("form", ["outliers", "small"])
+def test_rms_norm_weights_of_any_size(gpu, form, m, n, k):
+    """Weights times gamma on both sides of fp16's range.  outliers: one gamma in 64 of 30000 (up to 15 times that a weight), in every other group of
+    128 only; small: gamma of 6e-5.  2-norm of the error: a weight times gamma and the output are rounded to eleven bits each, 2^-11 / sqrt(3) at
+    most; the output's own spacing of 2^-24 where it is a subnormal number."""
+    from nnfusion_amd import ops
+
+    print(f"case gamma {form} M={m} N={n} K={k}", flush=True)
+    a, wq, s = datagen.w4a16_case(9, m, n, k)
+    rng = np.random.default_rng(6)
+    gamma = 6e-5 * (1.0 + 0.1 * rng.standard_normal(k))
+    if form == "outliers":
+        gamma = gamma / 6e-2
+        gamma.reshape(-1, 128)[::2, 5::64] *= 3e7
+        s = (s.astype(np.float32) / 16).astype(np.float16)
+    gamma = gamma.astype(np.float16)
+    ta, tw, ts, tg = _t(gpu, a, wq, s, gamma)
+    y = ops.w4a16_gemm_fused(ta, tw, ts, rms_gamma=tg, workspace=_ws(gpu), sync=ops.sync_flags(gpu)).cpu().numpy().astype(np.float64)
+    x = a.astype(np.float64)
+    x = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * gamma.astype(np.float64)
+    q = oracle.dequantize_w4(wq, np.ones_like(s)).astype(np.float64)
+    ref = x @ (q * np.repeat(s.astype(np.float64), 128, axis=1)).T
+    assert np.abs(ref).max() < 60000.0
+    assert np.isfinite(y).all()
+    subnormal = 2.0 ** -24 / np.sqrt(12 * np.mean(ref ** 2))
+    assert np.linalg.norm(y - ref) <= (np.sqrt(2 / 3) * 2.0 ** -11 + subnormal) * np.linalg.norm(ref)

@@ -30,9 +30,11 @@
 //     unpacked weights, as in the tile GEMM: gamma times an activation alone may leave the range of fp16.  (q - zp) times gamma is rounded
 //     to eleven bits, as a normalised activation is in a pass of its own: at most 15 gamma, and a multiple of 2^-24 like gamma, so exact where it
 //     is a subnormal number.  Gamma is used as it is, a sixteenth of it where a group has one of 4096 and more (16 on that group's sum).
-//     QG: scale times gamma is rounded to fp16 with the weight, and a small product of the two has few bits left there (5e-7: 1 %
-//     off); 16 times the scale, exact, moves that to products of 4e-8, and a weight times gamma reaches the end of
-//     fp16 at 4094, where sums of K >= 1024 of them are beyond fp16 as well.
+//     QG: a weight is (q - zp) times its scale, rounded, and that times gamma, rounded, as a weight and a normalised activation are rounded
+//     once each elsewhere.  The scales of a row's group of 128 are multiplied by a power of two, which the group's sum takes back in fp32: with
+//     the exponent e of the largest of them by 2^(18 - BITS - e), a weight stays below 2^4, times gamma below 2^16 (where the group has a gamma of 4096
+//     and more a sixteenth of that, where all are below 1 256 times that), and only products 2^15 below the largest possible lose bits.
+//     Costs 4 % (45 x 11008 x 4096, groups of 64 with zero points 16.9 -> 17.5 us); RMSNorm as a launch ahead takes 2.8 us.
 //   * Ranges of K (blockIdx.y): fp32 sums to scratch memory, added up in range order by the workgroup that arrives last,
 //     as in w4a16_mrows_any_kernel.
 #pragma once
@@ -389,12 +391,16 @@ namespace nnf
             uintx4 areg[MB][4];
             unroll_for<0, MB>([&](auto p_c) { read_a(p_c, areg[decltype(p_c)::value]); });
             bool large = false;
-            if constexpr (RMS && QG == 0)
+            int x_first = 0; // (QG) 2^(x_first - e) goes onto scales below 2^(e - 14)
+            if constexpr (RMS)
             {
                 const uint32_t own_largest = max(gamma_own & 0xffffu, gamma_own >> 16);
                 large = __builtin_amdgcn_ballot_w64(own_largest >= 0x6c00u) != 0; // 4096.0 and more: 15 times it may leave fp16
+                const bool below_one = __builtin_amdgcn_ballot_w64(own_largest >= 0x3c00u) == 0;
+                x_first = (large ? 14 : below_one ? 26 : 18) - BITS;
             }
-            // QG: scale (low half) and zero point of the lane's 32 weights of every tile: group (128 g + 32 kq) >> QG of row col
+            // QG: scale (low half) and zero point (eight bits) of the lane's 32 weights of every tile: group (128 g + 32 kq) >> QG of row col;
+            // RMS: and e in the upper eight bits
             uint32_t scale_zero[QG ? T : 1];
             if constexpr (QG != 0)
             {
@@ -409,7 +415,22 @@ namespace nnf
                     const int byte = BITS == 8 ? (QG == 7 ? 0 : sub) : QG == 5 ? sub >> 1 : 0;
                     const uint32_t zb = slot[S_AT + NSL * 256 + (((t * 16 + col) * ZPB + byte) << 2)];
                     const uint32_t z = !zps ? (uint32_t)zp : BITS == 8 ? zb : (zb >> ((sub & 1) * 4)) & 0xfu;
-                    scale_zero[t] = *reinterpret_cast<const uint16_t*>(at + half * 2) | (z << 16);
+                    if constexpr (RMS)
+                    {
+                        // the row's scales of this group of 128: 2, or 4 in two words, or one half of a word
+                        const uint32_t own = *reinterpret_cast<const uint32_t*>(at);
+                        uint32_t all = own;
+                        if constexpr (QG == 5)
+                        {
+                            const uint32_t other = *reinterpret_cast<const uint32_t*>(slot + S_AT + (((t * 16 + col) * SPW + 1 - (sub >> 1)) << 2));
+                            all = max((own >> 16) & 0x7fffu, (other >> 16) & 0x7fffu) << 16 | max(own & 0x7fffu, other & 0x7fffu);
+                        }
+                        const uint32_t scale = half ? own >> 16 : own & 0xffffu;
+                        const uint32_t largest = QG == 7 ? scale & 0x7fffu : max((all >> 16) & 0x7fffu, all & 0x7fffu);
+                        scale_zero[t] = scale | (z << 16) | ((largest >> 10) << 24);
+                    }
+                    else
+                        scale_zero[t] = *reinterpret_cast<const uint16_t*>(at + half * 2) | (z << 16);
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if constexpr (FULL)
@@ -451,7 +472,7 @@ namespace nnf
                     ww[4 * c + 2] = wnext[c].z;
                     ww[4 * c + 3] = wnext[c].w;
                 }
-                const float scale = RMS ? (float)snext * sum_factor : (float)snext;
+                float scale = RMS ? (float)snext * sum_factor : (float)snext;
                 if constexpr (FULL)
                     fetch_w(gn, t, at_slot);
                 if constexpr (t + 1 < T)
@@ -460,17 +481,22 @@ namespace nnf
                 half2_t lo = c_lo, hi = c_hi, scale2 = {};
                 if constexpr (QG != 0)
                 {
-                    const uint32_t z2 = (scale_zero[t] >> 16) * 0x10001u, s1 = scale_zero[t] & 0xffffu;
+                    const uint32_t z2 = ((scale_zero[t] >> 16) & 0xffu) * 0x10001u, e = scale_zero[t] >> 24;
+                    uint32_t s1 = scale_zero[t] & 0xffffu;
+                    if constexpr (RMS)
+                    {
+                        s1 = __builtin_bit_cast(uint16_t, __builtin_amdgcn_ldexph(__builtin_bit_cast(half_t, (uint16_t)s1), x_first - (int)e));
+                        scale = __builtin_bit_cast(float, ((uint32_t)(127 - x_first) + e) << 23); // 2^(e - x_first)
+                    }
                     lo = as_half2(0xE400E400u | z2);
                     hi = as_half2(0xD400D400u | (z2 << 4));
                     scale2 = as_half2(s1 | (s1 << 16));
-                    if constexpr (RMS)
-                        scale2 *= half2_t{(half_t)16.f, (half_t)16.f};
                 }
+                constexpr bool OWN_SUM = QG == 0 || RMS; // the group's sum, which meets a factor, or the accumulators themselves
                 floatx4 sum[MB];
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
-                    sum[mb] = QG ? acc[t][mb] : floatx4{0.f, 0.f, 0.f, 0.f};
+                    sum[mb] = OWN_SUM ? floatx4{0.f, 0.f, 0.f, 0.f} : acc[t][mb];
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                 {
@@ -482,10 +508,10 @@ namespace nnf
                 }
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
-                    if constexpr (QG != 0)
-                        acc[t][mb] = sum[mb];
-                    else
+                    if constexpr (OWN_SUM)
                         add_scaled(acc[t][mb], sum[mb], scale);
+                    else
+                        acc[t][mb] = sum[mb];
             });
             if constexpr (D > 1)
                 at_slot = at_slot == ring + (D - 1) * SLOT ? ring : at_slot + SLOT;
@@ -523,7 +549,7 @@ namespace nnf
 #pragma unroll
                 for (int w = 0; w < KS_WAVES; ++w)
                     total += sum_sq[w * (MB * 16) + tid];
-                rstd[tid] = (QG ? 0.0625f : 1.0f) / __builtin_sqrtf(total / (float)K + f.rms_eps);
+                rstd[tid] = 1.0f / __builtin_sqrtf(total / (float)K + f.rms_eps);
             }
         }
         const int n_tiles = (N + 15) / 16;
@@ -652,9 +678,8 @@ namespace nnf
                                   void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync, const void* zps)
         {
             auto kernel = &w4a16_kstream_kernel<T, MB, RMS, QG, BITS>;
-            const size_t lds = workspace::kstream_lds_bytes(T, MB, RMS, QG, BITS);
-            if (lds > MAX_LDS_BYTES)
-                return hipErrorInvalidValue;
+            constexpr size_t lds = workspace::kstream_lds_bytes(T, MB, RMS, QG, BITS);
+            static_assert(lds <= MAX_LDS_BYTES, "");
             static LdsGrant granted;
             const hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), granted, (int)MAX_LDS_BYTES);
             if (e != hipSuccess)
@@ -675,12 +700,14 @@ namespace nnf
         {
             hipError_t e = hipErrorInvalidValue;
             unroll_for<1, workspace::KSTREAM_MAX_TILES + 1>([&](auto t) {
-                if constexpr (workspace::kstream_lds_bytes(t.value, MB, false, QG, BITS) <= MAX_LDS_BYTES)
-                    if (plan.tiles == t.value)
-                        e = fusion.gamma ? launch_kstream<t.value, MB, true, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial,
-                                                                                       sync, zps)
-                                         : launch_kstream<t.value, MB, false, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial,
-                                                                                        sync, zps);
+                if (plan.tiles != t.value)
+                    return;
+                if constexpr (workspace::kstream_built(t.value, MB, true, QG, BITS))
+                    if (fusion.gamma)
+                        e = launch_kstream<t.value, MB, true, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps);
+                if constexpr (workspace::kstream_built(t.value, MB, false, QG, BITS))
+                    if (!fusion.gamma)
+                        e = launch_kstream<t.value, MB, false, QG, BITS>(stream, plan, A, Wq, S, Y, M, N, K, zp, fusion, partial, sync, zps);
             });
             return e;
         }

@@ -1076,6 +1076,12 @@ namespace nnf
             const size_t sums = (size_t)4096 + (size_t)KSTREAM_WAVES * kstream_round(tiles, mb) * mb * 1024;
             return stream > sums ? stream : sums;
         }
+        // built and used: what the LDS holds.  qg with RMSNorm needs registers for a group's own sums beside the accumulators: four blocks
+        // of rows and five or six tiles spill 14 - 47 of 256
+        constexpr bool kstream_built(int tiles, int mb, bool rms, int qg, int bits)
+        {
+            return kstream_lds_bytes(tiles, mb, rms, qg, bits) <= LDS_BYTES_PER_CU && !(qg && rms && tiles * mb >= 20);
+        }
         // CUs of a block of rows: a multiple of eight, so that the workgroups of all blocks that read the same weights are on one XCD (they
         // are dealt out to the eight XCDs in turn)
         constexpr int kstream_cus(int share, int row_blocks) { return row_blocks > 1 && share >= 8 ? share & ~7 : share; }
@@ -1104,7 +1110,7 @@ namespace nnf
                 return p;
             if ((ranges - 1) * rg >= G ||
                 ((G & 1) && (qg == 0 || qg == 7) && ((N & 1) || (size_t)(gate ? 2 : 1) * N * G >= ((size_t)1 << 31))) || tiles > KSTREAM_MAX_TILES ||
-                kstream_lds_bytes(tiles, mb, rms, qg, bits) > LDS_BYTES_PER_CU)
+                !kstream_built(tiles, mb, rms, qg, bits))
                 return p;
             p.tiles = tiles;
             p.row_tiles = mb;
@@ -1193,8 +1199,7 @@ namespace nnf
             for (int row_blocks = fewest; row_blocks <= most; ++row_blocks)
             {
                 const KstreamPlan p = kstream_plan(M, N, K, num_cu, gate, rms, 1, row_blocks, qg);
-                // (four blocks of rows and six tiles with RMSNorm do not fit the registers: 51 x 9408 x 3328 0.79)
-                if (p.tiles == 0 || (rms && p.tiles * p.row_tiles == 24))
+                if (p.tiles == 0)
                     continue;
                 if (M <= 16)
                 {

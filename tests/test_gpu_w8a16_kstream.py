@@ -98,3 +98,39 @@ def test_small_rms_norm_weight(gpu, bits, group, m, n, k, gate):
         ref = ref[:, :n] / (1.0 + np.exp(-ref[:, :n])) * ref[:, n:]
     y = ops.wna16_gemm_fused(ta, tw, ts, bits, group, zp, tz, rms_gamma=tg, act=1 if gate else 0).cpu().numpy().astype(np.float64)
     assert np.linalg.norm(y - ref) <= (1e-3 + 2.0 ** -24 / np.sqrt(12 * np.mean(ref ** 2))) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("bits,group,m,n,k,gate", [(4, 32, 40, 72, 1024, False), (4, 64, 45, 40, 1280, True), (4, 128, 64, 300, 1152, False),
+                                                   (8, 32, 5, 300, 1152, True), (8, 64, 40, 72, 2304, False), (8, 128, 9, 302, 1024, False)])
+@pytest.mark.parametrize("form", ["outliers", "scales", "small"])
+def test_rms_norm_weights_and_scales_of_any_size(gpu, form, bits, group, m, n, k, gate):
+    """Weights times gamma on both sides of fp16's range (scales: of 4 bits, 1 / 16 of them with 8).  outliers: one gamma in 64 of 3000, scales up
+    to 0.1; scales of 150 .. 300 with gamma of 1e-2; scales of 2e-3 .. 4e-3 with gamma of 6e-5.  2-norm of the error: a weight, that times gamma and
+    the output are rounded to eleven bits each, 2^-11 / sqrt(3) at most, 2^-11 in all; a gate: of two products multiplied, twice that; the output's
+    own spacing of 2^-24 where it is a subnormal number."""
+    from nnfusion_amd import ops
+
+    print(f"case gamma {form} bits={bits} group={group} M={m} N={n} K={k} gate={gate}", flush=True)
+    zp = 7 if bits == 4 else 119
+    a, wq, _, z = datagen.wna16_case(8, m, 2 * n if gate else n, k, bits, group, True)
+    rng = np.random.default_rng(5)
+    low, high, gamma = {"outliers": (0.05, 0.1, 1.0), "scales": (150.0, 300.0, 1e-2), "small": (2e-3, 4e-3, 6e-5)}[form]
+    s = (rng.uniform(low, high, (wq.shape[0], k // group)) / (1 if bits == 4 else 16)).astype(np.float16)
+    gamma = gamma * (1.0 + 0.1 * rng.standard_normal(k))
+    if form == "outliers":
+        gamma[5::64] *= 3000.0
+    gamma = gamma.astype(np.float16)
+    if gate: # (products of a gate of about one and up: within the range of fp16)
+        s[:n] = (s[:n].astype(np.float32) * {"outliers": 2.0 ** -14, "scales": 2.0 ** -8, "small": 2.0 ** 14}[form]).astype(np.float16)
+    ta, tw, ts, tz, tg = _t(gpu, a, wq, s, z, gamma)
+    x = a.astype(np.float64)
+    x = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * gamma.astype(np.float64)
+    q = oracle.dequantize_wn(wq, np.ones_like(s), bits, group, zp, z).astype(np.float64)
+    ref = x @ (q * np.repeat(s.astype(np.float64), group, axis=1)).T
+    if gate:
+        ref = ref[:, :n] / (1.0 + np.exp(-ref[:, :n])) * ref[:, n:]
+    assert np.abs(ref).max() < 60000.0
+    y = ops.wna16_gemm_fused(ta, tw, ts, bits, group, zp, tz, rms_gamma=tg, act=1 if gate else 0).cpu().numpy().astype(np.float64)
+    assert np.isfinite(y).all()
+    subnormal = 2.0 ** -24 / np.sqrt(12 * np.mean(ref ** 2))
+    assert np.linalg.norm(y - ref) <= ((2 if gate else 1) * 2.0 ** -11 + subnormal) * np.linalg.norm(ref)

@@ -417,6 +417,10 @@ namespace
                          const nnf_quant* q, const nnf::GemvFusion& fusion, void* xn, void* own, size_t own_bytes, int num_cu, bool& taken)
     {
         taken = false;
+        // (these kernels fetch 16 bytes at a time: an input that RMSNorm copies, or an output behind a product in scratch memory, may lie
+        // elsewhere; the callers refuse other tensors that do)
+        if (!aligned16(A) || !aligned16(Y))
+            return NNF_OK;
         // (RMSNorm of a few rows inside that kernel where it is inside the row-streaming kernels as well or SiLU-gate follows; otherwise a
         // launch ahead of it, so that the fused product stays the nodes' own arithmetic, bit for bit)
         if (q->bits == 4 && fusion.gamma && !fusion.gate && M <= 32 && !nnf::workspace::mrows_q_norm_inside(M, K))
@@ -521,6 +525,9 @@ int nnf_wna16_gemm_fused(nnf_stream_t stream, const void* A, const void* Wq, con
     const nnf::workspace::QFusedLayout l = nnf::workspace::wna16_fused_layout(M, N, K, q->bits, q->group, rms, gate, residual == Y);
     if (l.total() > 0 && (!workspace || !aligned16(workspace) || workspace_bytes < l.total()))
         return NNF_ERR_WORKSPACE_TOO_SMALL;
+    // the tensors that the product itself takes, as nnf_wna16_gemm refuses them
+    if (!aligned16(Wq) || !aligned16(scales) || (!rms && !aligned16(A)) || (l.product == 0 && !aligned16(Y)))
+        return NNF_ERR_INVALID_ARGUMENT;
     uint8_t* ws = (uint8_t*)workspace;
     const hipStream_t s = (hipStream_t)stream;
     DeviceInfo dev;
@@ -811,6 +818,8 @@ int nnf_fused_mlp_wna16(nnf_stream_t stream, const void* x, const void* gamma, f
         return NNF_ERR_UNSUPPORTED_SHAPE;
     if (!workspace || workspace_bytes < nnf::workspace::fused_mlp_wna16(M, H, I, q_gate_up->bits, q_gate_up->group))
         return NNF_ERR_WORKSPACE_TOO_SMALL;
+    if (!aligned16(Wgu) || !aligned16(Sgu) || !aligned16(Wd) || !aligned16(Sd))
+        return NNF_ERR_INVALID_ARGUMENT;
     const size_t wide = (size_t)(2 * I > H ? 2 * I : H);
     uint8_t* xn = (uint8_t*)workspace;
     uint8_t* product = xn + nnf::workspace::align256((size_t)M * H * 2);

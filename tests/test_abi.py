@@ -99,3 +99,49 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_kernels", None)
     with pytest.raises(_lib.NativeLibraryMissing):
         _lib.kernels()
+
+
+def _fused_calls(gate, rms, in_place, bits, group, m):
+    """status of nnf_wna16_gemm_fused and nnf_fused_mlp_wna16 with made-up tensors of which the named one lies 8 bytes off; no device: nothing runs"""
+    from nnfusion_amd.ops import NnfQuant
+
+    lib = _lib.kernels()
+    q = NnfQuant(bits, group, 7, None)
+    qp = ctypes.cast(ctypes.pointer(q), ctypes.c_void_p)
+    n, k = 256, 1024
+    sizes = dict(a=1 << 32, wq=2 << 32, s=3 << 32, y=4 << 32, gamma=5 << 32, x=6 << 32, wgu=7 << 32, sgu=8 << 32, wd=9 << 32, sd=10 << 32)
+
+    def fused(off):
+        at = {name: p + (8 if name == off else 0) for name, p in sizes.items()}
+        return lib.nnf_wna16_gemm_fused(None, at["a"], at["wq"], at["s"], at["y"], m, n, k, qp, at["gamma"] if rms else None, 1e-6, None,
+                                        at["y"] if in_place else None, 1 if gate else 0, 11 << 32, 1 << 40)
+
+    def mlp(off):
+        at = {name: p + (8 if name == off else 0) for name, p in sizes.items()}
+        return lib.nnf_fused_mlp_wna16(None, at["x"], at["gamma"], 1e-6, at["wgu"], at["sgu"], at["wd"], at["sd"], at["y"], m, k, 512, qp, qp,
+                                       11 << 32, 1 << 40)
+
+    return fused, mlp
+
+
+def test_fused_products_refuse_tensors_off_their_alignment():
+    """Weights and scales always; activations where RMSNorm makes no copy of them; the output where no product in scratch memory lies ahead of it."""
+    import pytest
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("made-up addresses: where there is a device, a call that is let through would run")
+    no_device = -4
+    for bits, group, m in ((4, 64, 4), (4, 64, 45), (4, 32, 300), (4, 128, 1000), (8, 32, 1), (8, 128, 8), (8, 64, 200)):
+        if bits == 4 and group == 128:
+            bits = 8
+        for gate, rms, in_place in ((0, 0, 0), (0, 1, 0), (1, 1, 0), (1, 0, 0), (0, 0, 1)):
+            fused, mlp = _fused_calls(gate, rms, in_place, bits, group, m)
+            assert fused(None) == no_device and mlp(None) == no_device
+            for off in ("wq", "s"):
+                assert fused(off) == -1, (off, bits, group, m, gate, rms, in_place)
+            assert fused("a") == (no_device if rms else -1)
+            if not in_place:
+                assert fused("y") == (no_device if gate else -1)
+            for off in ("x", "gamma", "wgu", "sgu", "wd", "sd", "y"):
+                assert mlp(off) == -1, (off, bits, group, m)

@@ -1338,6 +1338,102 @@ int main(int argc, char** argv)
         EXPECT(ws::w8a8_mrows_ranges(7, 4096, 8192, 256) == 1 && ws::w8a8_mrows_ranges(32, 8192, 4096, 256) == 1 &&
                ws::w8a8_mrows_ranges(32, 8208, 8192, 256) == 1 && ws::w8a8_mrows_ranges(16, 4096, 11008, 256) == 1);
         EXPECT(ws::w8a8_mrows_ranges_bytes(8, 4096, 8192, 256) == (size_t)2 * 8 * 4096 * 4 && ws::w8a8_gemm(8, 4096, 8192) >= (size_t)2 * 8 * 4096 * 4);
+        // the K-streaming kernels: every plan of the library's own choice covers the product, and nothing beyond it, within the LDS and
+        // the CUs; over ranges of K within the scratch memory and synchronisation words it was offered
+        {
+            const auto covers = [](const ws::KstreamPlan& p, int m, int n, int k, bool gate, int cus) {
+                const int n_tiles = (n + 15) / 16, groups = k / 128;
+                return p.grid >= 1 && p.grid * p.ranges * p.row_blocks <= cus && p.tiles_q * p.grid + p.tiles_r == n_tiles && p.tiles_q >= 1 &&
+                       p.tiles_r < p.grid && p.tiles == (gate ? 2 : 1) * (p.tiles_q + (p.tiles_r ? 1 : 0)) && p.tiles <= ws::KSTREAM_MAX_TILES &&
+                       p.row_tiles >= 1 && p.row_tiles <= 4 && p.row_blocks * p.row_tiles * 16 >= m && (p.row_blocks - 1) * p.row_tiles * 16 < m &&
+                       (p.range_groups == 0 || (p.ranges * p.range_groups >= groups && (p.ranges - 1) * p.range_groups < groups));
+            };
+            uint32_t state = 12345;
+            const auto draw = [&](int lo, int hi) {
+                state = state * 1664525u + 1013904223u;
+                return lo + (int)((state >> 8) % (unsigned)(hi - lo + 1));
+            };
+            int taken[4] = {0, 0, 0, 0};
+            for (int i = 0; i < 200000; ++i)
+            {
+                const int m = draw(2, 1 << draw(2, 10)), n = draw(16, 1 << draw(5, 15)), k = 128 * draw(8, 1 << draw(3, 7)), cus = i % 3 ? 256 : draw(1, 304);
+                const bool gate = draw(0, 3) == 0, rms = draw(0, 1) != 0;
+                const size_t partial = (size_t)draw(0, 64) << 20, sync = draw(0, 1) ? 65536 : draw(0, 1024);
+                const auto p = ws::kstream_choice(m, n, k, cus, gate, rms, partial, sync);
+                if (p.tiles > 0)
+                {
+                    ++taken[0];
+                    EXPECT(covers(p, m, n, k, gate, cus) && ws::kstream_lds_bytes(p.tiles, p.row_tiles, rms) <= ws::LDS_BYTES_PER_CU);
+                    EXPECT(p.ranges == 1 || (!gate && !rms && p.partial_bytes <= partial && (size_t)p.grid * p.row_blocks * 4 <= sync &&
+                                             p.partial_bytes >= (size_t)p.ranges * ((n + 15) / 16) * 16 * m * sizeof(float)));
+                }
+                const int qg = draw(5, 7);
+                const auto q = ws::kstream_choice_q(m, n, k, qg, cus, gate, rms);
+                if (q.tiles > 0)
+                {
+                    ++taken[1];
+                    EXPECT(covers(q, m, n, k, gate, cus) && q.ranges == 1 && ws::kstream_built(q.tiles, q.row_tiles, rms, qg, 4) &&
+                           (rms ? q.tiles * q.row_tiles < 20 : true));
+                }
+                const auto b = ws::kstream_choice_b8(m, n, k, qg, cus, gate, rms, true, draw(0, 1) != 0);
+                if (b.tiles > 0)
+                {
+                    ++taken[2];
+                    EXPECT(covers(b, m, n, k, gate, cus) && b.ranges == 1 && ws::kstream_built(b.tiles, b.row_tiles, rms, qg, 8));
+                }
+                const auto w = ws::w8a8_kstream_choice(m, n, k, cus);
+                if (w.tiles > 0)
+                {
+                    ++taken[3];
+                    const int unit = ws::w8a8_kstream_unit(w.tiles, w.row_tiles, k);
+                    EXPECT(covers(w, m, n, k, false, cus) && k % unit == 0 && ws::w8a8_kstream_lds_bytes(w.tiles, w.row_tiles, unit) <= ws::LDS_BYTES_PER_CU);
+                }
+            }
+            for (int t : taken)
+                EXPECT(t > 10000);
+            // which kernel the GPU tests' sizes get.  The K-streaming kernels' own tests, by (tiles, blocks of 16 rows):
+            const auto own = [](const ws::KstreamPlan& p, int tiles, int mb) { return p.tiles == tiles && p.row_tiles == mb; };
+            EXPECT(own(ws::kstream_choice(17, 16, 1152, 256, false, false, 0, 0), 1, 2));
+            EXPECT(own(ws::kstream_choice(48, 4096, 1024, 256, false, false, 0, 0), 1, 3));
+            EXPECT(own(ws::kstream_choice(64, 24576, 1024, 256, false, false, 0, 0), 6, 4));
+            EXPECT(own(ws::kstream_choice(8, 24576, 1792, 256, false, false, 0, 0), 6, 1));
+            EXPECT(own(ws::kstream_choice(16, 2050, 2560, 256, false, true, 0, 0), 1, 1));
+            EXPECT(own(ws::kstream_choice(64, 8200, 1024, 256, false, true, 0, 0), 5, 2) && own(ws::kstream_choice(64, 8200, 1024, 256, true, true, 0, 0), 6, 4));
+            EXPECT(ws::kstream_choice(33, 4096, 11008, 256, false, false, 64 << 20, 65536).ranges == 4 &&
+                   ws::kstream_choice(150, 1024, 8704, 256, false, false, 64 << 20, 65536).ranges == 3);
+            EXPECT(own(ws::kstream_choice_q(2, 40, 1280, 5, 256, false, false), 1, 1));
+            EXPECT(own(ws::kstream_choice_q(64, 24576, 1280, 7, 256, false, false), 6, 4));
+            EXPECT(own(ws::kstream_choice_q(45, 40, 1280, 6, 256, true, true), 2, 1));
+            EXPECT(own(ws::kstream_choice_q(64, 16380, 1152, 5, 256, false, true), 4, 4) && own(ws::kstream_choice_q(48, 24560, 1024, 6, 256, false, true), 6, 3) &&
+                   own(ws::kstream_choice_q(40, 12280, 1152, 7, 256, true, true), 6, 3));
+            EXPECT(ws::kstream_choice_q(64, 20480, 1280, 6, 256, false, true).tiles == 0 && ws::kstream_choice_q(64, 20480, 1280, 6, 256, false, false).tiles == 5);
+            EXPECT(own(ws::kstream_choice_b8(16, 24576, 1280, 5, 256, false, false, false, true), 6, 1));
+            EXPECT(own(ws::kstream_choice_b8(5, 300, 1152, 5, 256, true, true, true, true), 2, 1));
+            EXPECT(own(ws::kstream_choice_b8(49, 12288, 1024, 6, 256, false, false, false, true), 3, 4));
+            EXPECT(own(ws::w8a8_kstream_choice(100, 8208, 1024, 256), 5, 4) && own(ws::w8a8_kstream_choice(128, 12288, 1152, 256), 6, 4) &&
+                   own(ws::w8a8_kstream_choice(64, 24560, 1024, 256), 6, 4) && own(ws::w8a8_kstream_choice(16, 24560, 1152, 256), 6, 1) &&
+                   own(ws::w8a8_kstream_choice(30, 20000, 1024, 256), 5, 2) && own(ws::w8a8_kstream_choice(33, 24576, 1024, 256), 6, 3));
+            // tests of the tile GEMM with other block parameters: tiles shared between workgroups, not on the K-streaming kernel
+            const int shared[][3] = {{600, 520, 2048}, {130, 1024, 8192}, {256, 1040, 7168}, {70, 300, 6400}, {520, 128, 1536}, {1000, 300, 4096}};
+            for (const auto& s : shared)
+                for (int gs = 5; gs <= 7; ++gs)
+                    EXPECT(ws::kstream_choice_q(s[0], s[1], s[2], gs, 256, false, false).tiles == 0 && ws::w4a16_gemm_q_fits(s[0], s[1], s[2], gs) &&
+                           ws::wna16_gemm(s[0], s[1], s[2], 4, 1 << gs) > 0);
+            // ... of what is too wide, too long or has too many rows for the K-streaming kernel: two blocks of rows on the row-streaming kernels, tiles
+            const int beyond[][3] = {{17, 24592, 2048}, {32, 24610, 4096}, {20, 24600, 1024}, {60, 24592, 1280}, {520, 300, 1024}, {600, 1100, 1536}, {70, 520, 6400}};
+            for (const auto& s : beyond)
+            {
+                EXPECT(ws::kstream_choice_q(s[0], s[1], s[2], 5, 256, false, false).tiles == 0);
+                EXPECT(ws::w4a16_mrows_q_fits(s[0], s[1], s[2], 5, true, 256) == (s[0] <= 32 && s[2] >= 2048));
+                EXPECT((s[0] == 70) == (ws::kstream_choice_b8(s[0], s[1], s[2], 5, 256, false, false, false, true).tiles > 0));
+            }
+            // by itself the library runs no W8A8 product over two ranges of K on the row-streaming kernel: the K-streaming kernel takes them all
+            for (int m = 2; m <= 32; ++m)
+                for (int k = 8192; k <= 16384; k += 512)
+                    for (int n = 16; n <= 8192; n += 16)
+                        if (ws::w8a8_mrows_preferred(m, n, k, 256) && ws::w8a8_mrows_ranges(m, n, k, 256) > 1)
+                            EXPECT(ws::w8a8_kstream_choice(m, n, k, 256).tiles > 0);
+        }
         // fp16 x int4 tile GEMM: the (tile, superstep) units are split evenly over at most one workgroup per CU; a
         // workgroup parks at most two partial tiles; whole tiles need no workspace
         {

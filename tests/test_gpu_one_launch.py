@@ -220,13 +220,16 @@ def test_ranges_of_k_added_up_inside_the_launch(gpu, m, n, k, fused):
 
 
 @pytest.mark.parametrize("bits,group,zpt", [(4, 32, True), (4, 64, False), (4, 128, True)])
-@pytest.mark.parametrize("m,n,k", [(200, 300, 1024), (64, 520, 2048), (130, 128, 1536), (256, 1024, 4096)])
+@pytest.mark.parametrize("m,n,k", [(200, 300, 1024), (64, 520, 2048), (130, 128, 1536), (256, 1024, 4096), (600, 520, 2048), (130, 1024, 8192),
+                                   (256, 1040, 7168), (70, 300, 6400), (520, 128, 1536), (1000, 300, 4096)])
 def test_one_launch_with_other_block_parameters(gpu, m, n, k, bits, group, zpt):
-    """nnf_wna16_gemm_planned: the tile GEMM for groups of 32 / 64 / 128 and zero-point tensors in one launch."""
+    """nnf_wna16_gemm_planned: the tile GEMM for groups of 32 / 64 / 128 and zero-point tensors in one launch (the first four sizes run on the
+    K-streaming kernel, which has one launch either way; the others share tiles on the tile GEMM: tests/cpp/test_host.cpp)."""
     import torch
 
     from nnfusion_amd import ops
 
+    print(f"case one launch M={m} N={n} K={k} group={group} zero_points={zpt}", flush=True)
     a, wq, s, z = datagen.wna16_case(m + k, m, n, k, bits, group, zpt)
     ta, tw, ts, tz = _t(gpu, a, wq, s, z if zpt else None)
     two = ops.wna16_gemm(ta, tw, ts, bits=bits, group=group, zp=8, zero_points=tz)

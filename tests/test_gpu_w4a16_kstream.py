@@ -4,7 +4,9 @@ Sizes at its edges: rows around the blocks of 16, one column tile up to six a wo
 last tile is moved back), a single group for the last chunk, an odd number of groups (scale rows that start in the middle of
 a word), all 64 groups of the longest range, ranges of K that end unevenly.  Every product also runs without
 synchronisation words (one range of K, or the kernel that served it before).
-Tolerance: fp16 results of fp32 sums, 1e-2 of the result's RMS as for the other kernels (measured: 2e-3 at most).
+Tolerance, of the result's RMS: the output's rounding, 2^-11 of up to 5.5 RMS, 2.7e-3, and a bias's and a residual's once more; with
+RMSNorm weights times gamma rounded to eleven bits, 2^-11 / sqrt(3) in the 2-norm at most and 5.5 of that, 1.6e-3: 5e-3 (SiLU-gate: two rounded
+products multiplied, values up to some ten RMS, 2e-2).
 """
 import numpy as np
 import pytest
@@ -14,7 +16,7 @@ from nnfusion_amd import datagen
 
 pytestmark = pytest.mark.gpu
 
-TOL = 1e-2
+TOL = 5e-3
 
 
 def _t(gpu, *arrays):
@@ -104,7 +106,7 @@ def test_rms_norm(gpu, m, n, k, spread, gate):
         g, u = ref[:, :n], ref[:, n:]
         ref = g / (1.0 + np.exp(-g)) * u
         # the gate and up products are rounded to fp16 and multiplied: twice the relative error of one, on a result with heavier tails
-        _check(y, ref, 2 * TOL)
+        _check(y, ref, 4 * TOL)
     else:
         _check(y, ref)
 

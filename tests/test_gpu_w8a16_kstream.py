@@ -3,8 +3,9 @@ number of groups of 128 (scales of every other row start in the middle of a word
 
 Sizes at the kernel's edges: rows around the blocks of 16 and blocks of rows, columns that are no multiple of 16, one to six tiles a workgroup
 (bytes of zero points come 64 a load, four a tile row with groups of 32), chunks with a single group, long K, odd numbers of columns (groups of
-128 in odd numbers go elsewhere then).  Tolerance: weights rounded to fp16 ahead of fp32 sums, 1e-2 of the result's RMS as for the other
-kernels of these parameters (SiLU-gate: two rounded products multiplied, twice that).
+128 in odd numbers go elsewhere then).  Tolerance, of the result's RMS: the output's rounding, 2^-11 of up to 5.5 RMS, 2.7e-3, and a residual's
+once more; weights, and weights times gamma, rounded to eleven bits each, 2^-11 / sqrt(3) in the 2-norm at most and 5.5 of that, 2.2e-3: 5e-3
+(SiLU-gate: two rounded products multiplied, values up to some ten RMS, 2e-2).
 """
 import numpy as np
 import pytest
@@ -14,7 +15,7 @@ from nnfusion_amd import datagen
 
 pytestmark = pytest.mark.gpu
 
-TOL = 1e-2
+TOL = 5e-3
 
 
 def _t(gpu, *arrays):
@@ -71,7 +72,7 @@ def test_products(gpu, bits, m, n, k, form, group, zero_points):
         again = ops.wna16_gemm_fused(ta, tw, ts, bits, group, zp, tz, rms_gamma=tg, residual=out, act=1 if gate else 0, out=out)
     torch.cuda.synchronize()
     assert torch.equal(y, again)
-    _check(y, ref, 2 * TOL if gate else TOL)
+    _check(y, ref, 4 * TOL if gate else TOL)
 
 
 @pytest.mark.parametrize("bits,group,m,n,k,gate", [(4, 32, 40, 72, 4096, False), (4, 64, 64, 40, 1280, True), (4, 128, 16, 300, 2304, True),

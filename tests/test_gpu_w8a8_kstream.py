@@ -1,7 +1,7 @@
 """The K-streaming W8A8 kernel (w8a8_kstream.hip): 2 .. 64 rows and blocks of up to 64.
 
 Sizes at its edges: rows around the blocks of 16, columns that are no multiple of 16 (the last tile is moved back), one to six tiles a
-workgroup, K that is no multiple of 256 (half the bytes a wavefront and chunk), a single wavefront in the last chunk, chunks that wrap around.
+workgroup (five and six with four blocks of rows: their sums meet in two rounds), K that is no multiple of 256 (half the bytes a wavefront and chunk), a single wavefront in the last chunk, chunks that wrap around.
 The int32 accumulators are exact; the fp16 results follow from them by the oracle's formula, bit for bit.
 """
 import numpy as np
@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("m,n,k", [
     (2, 16, 1024), (16, 4112, 1152), (7, 40, 8192), (9, 8200, 2048), (17, 528, 2176), (32, 8192, 4096), (33, 24576, 1024), (48, 300, 5504), (64, 4100, 1280),
-    (65, 520, 2048), (130, 1000, 1152), (200, 2056, 1024), (300, 272, 4096), (1000, 144, 1152), (45, 12296, 1408), (64, 16384, 1024)])
+    (65, 520, 2048), (130, 1000, 1152), (200, 2056, 1024), (300, 272, 4096), (1000, 144, 1152), (45, 12296, 1408), (64, 16384, 1024),
+    (100, 8208, 1024), (128, 12288, 1152), (64, 24560, 1024), (16, 24560, 1152), (30, 20000, 1024)])
 def test_products(gpu, m, n, k):
     import torch
 

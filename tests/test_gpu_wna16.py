@@ -179,14 +179,15 @@ def test_wna16_random_shapes(gpu, m, n, k, bits, group, zp_tensor, zp):
     _check(_run(gpu, a, wq, s, bits, group, zp, zps), ref)
 
 
-def test_tile_gemm_without_its_workspace_runs_on_the_plain_kernel(gpu):
+@pytest.mark.parametrize("k", [4096, 8192])
+def test_tile_gemm_without_its_workspace_runs_on_the_plain_kernel(gpu, k):
     """Above 16 rows 4-bit weights want the stream-K tile GEMM's workspace; a caller that brings none (or too little)
-    gets the same product from the plain tile kernel."""
+    gets the same product from the plain tile kernel (K = 8192; at 4096 the K-streaming kernel needs none)."""
     import torch
 
     from nnfusion_amd import ops
 
-    m, n, k, group = 130, 1024, 4096, 64
+    m, n, group = 130, 1024, 64
     a, wq, s, zps = _case(21, m, n, k, 4, group, True)
     need = ops.wna16_workspace_bytes(m, n, k, 4, group)
     assert need > 0
@@ -197,6 +198,18 @@ def test_tile_gemm_without_its_workspace_runs_on_the_plain_kernel(gpu):
                            workspace=torch.empty(ws_bytes, dtype=torch.uint8, device=gpu))
         torch.cuda.synchronize()
         _check(y.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("bits,group,zp_tensor", [(4, 32, True), (4, 64, False), (4, 128, True), (8, 32, True), (8, 128, False)])
+@pytest.mark.parametrize("m,n,k", [(17, 24592, 2048), (32, 24610, 4096), (20, 24600, 1024), (60, 24592, 1280), (520, 300, 1024), (600, 1100, 1536),
+                                   (70, 520, 6400)])
+def test_products_beyond_the_k_streaming_kernel(gpu, m, n, k, bits, group, zp_tensor):
+    """More columns than six tiles a workgroup hold, more rows, longer K: two blocks of rows on the row-streaming kernels (17 .. 32 rows, K = 2048
+    and 4096), the tile GEMM of 4-bit weights, the plain tile kernel of 8-bit ones (which sizes go where: tests/cpp/test_host.cpp)."""
+    print(f"case beyond kstream bits={bits} M={m} N={n} K={k} group={group} zero_points={zp_tensor}", flush=True)
+    a, wq, s, zps = _case(m + n + k + group, m, n, k, bits, group, zp_tensor)
+    zp = 5 if bits == 4 else 83
+    _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
 
 
 def test_default_parameters_are_the_specialised_kernels(gpu):

@@ -1135,6 +1135,13 @@ namespace nnf
             return chunks * (17 + 27 * mb + (bits == 8 ? 24 : 16) * t + 9 * mb * t) * (358 + (workgroups < 256 ? workgroups : 256)) / 614 + 200 + 6 * t + 15 * mb * t +
                    (p.ranges > 1 ? 84 + 20 * p.ranges + 60 * t : 0);
         }
+        // 17 .. 32 rows, K = 2048 in fewer than 112 tiles, without RMSNorm and SiLU-gate: the row-streaming kernels, which have K as a compile-time
+        // constant, are 2 - 6 % faster (17 x 512 x 2048 4.0 us there, 4.25 here; groups of 32 / 64 up to 8 %; at
+        // 1920 columns level, at 2560 1 - 7 % slower; K = 4096 level at all widths)
+        constexpr bool kstream_behind_mrows(int M, int N, int K, bool gate, bool rms)
+        {
+            return M > 16 && M <= 32 && K == 2048 && N < 1792 && !gate && !rms;
+        }
         // What the library runs on it by itself, from measurements against the kernels that served these products before.  33 .. 64 rows:
         // everything that fits (against the tile GEMM: N = K = 4096 at 48 rows 13.8 -> 9.0 us, 12288 x 4096 21.0 -> 15.0, 4096 x 11008 20.5 -> 16.6,
         // RMSNorm and SiLU-gate at 11008 x 4096 35.2 -> 22.4; against the row-streaming kernel up to K = 2048 1.2 - 1.9 x).  17 .. 32 rows: all but more
@@ -1163,7 +1170,7 @@ namespace nnf
             const bool fixed_k = w4a16_mrows_fixed_k(M, K);
             // (17 .. 32 rows: N = 320 .. 600 at K = 1024 takes 3.3 us there, 3.5 here; N = 256 .. 2400 at K = 11776 .. 12288 0.92 - 0.97 x, 4480 and more
             // 1.06 - 1.16)
-            if (M < 2 || M > 1024 || (M > 16 && M <= 32 && (K <= 1024 || (K > 11264 && N < 4096))))
+            if (M < 2 || M > 1024 || (M > 16 && M <= 32 && (K <= 1024 || (K > 11264 && N < 4096))) || kstream_behind_mrows(M, N, K, gate, rms))
                 return best;
             // 2 .. 16 rows, against the row-streaming kernel and the MFMA GEMV (time there / here, 1320 products).  K that is a compile-time constant
             // of the row-streaming kernel stays there (SiLU-gate 0.85 - 1.08, others 0.91 - 1.25, most within 8 %); with any other K RMSNorm and SiLU-gate,
@@ -1193,7 +1200,8 @@ namespace nnf
         inline KstreamPlan kstream_choice_q(int M, int N, int K, int qg, int num_cu, bool gate, bool rms)
         {
             KstreamPlan best;
-            if (M < 2 || M > 512 || qg < 5 || qg > 7 || (M > 64 && K > 6144))
+            if (M < 2 || M > 512 || qg < 5 || qg > 7 || (M > 64 && K > 6144) ||
+                (kstream_behind_mrows(M, N, K, gate, rms) && w4a16_mrows_q_fits(M, N, K, qg, true, num_cu)))
                 return best;
             const int fewest = (M + 63) / 64, most = M <= 32 ? 1 : fewest + 2;
             for (int row_blocks = fewest; row_blocks <= most; ++row_blocks)

@@ -1413,6 +1413,18 @@ int main(int argc, char** argv)
             EXPECT(own(ws::w8a8_kstream_choice(100, 8208, 1024, 256), 5, 4) && own(ws::w8a8_kstream_choice(128, 12288, 1152, 256), 6, 4) &&
                    own(ws::w8a8_kstream_choice(64, 24560, 1024, 256), 6, 4) && own(ws::w8a8_kstream_choice(16, 24560, 1152, 256), 6, 1) &&
                    own(ws::w8a8_kstream_choice(30, 20000, 1024, 256), 5, 2) && own(ws::w8a8_kstream_choice(33, 24576, 1024, 256), 6, 3));
+            // 17 .. 32 rows of K = 2048 in few tiles: the row-streaming kernels, but for groups of 128 with zero points, which they do not take there
+            for (int m : {16, 17, 32, 33})
+                for (int n : {256, 1776, 1792, 4096})
+                {
+                    const bool left = m > 16 && m <= 32 && n < 1792;
+                    EXPECT((ws::kstream_choice(m, n, 2048, 256, false, false, 0, 0).tiles == 0) == (left || m <= 16));
+                    EXPECT((ws::kstream_choice_q(m, n, 2048, 6, 256, false, false).tiles == 0) == (left || m <= 16));
+                    EXPECT(ws::kstream_choice(m, n, 2048, 256, false, true, 0, 0).tiles > 0 || m <= 16);
+                    EXPECT(ws::kstream_choice_q(m, n, 2048, 7, 256, false, false).tiles > 0 || m <= 16);
+                    EXPECT(!left || (ws::route_w4a16(m, n, 2048, false, false, false, 256).kind == ws::W4A16Route::MROWS &&
+                                     ws::w4a16_mrows_q_fits(m, n, 2048, 6, true, 256)));
+                }
             // tests of the tile GEMM with other block parameters: tiles shared between workgroups, not on the K-streaming kernel
             const int shared[][3] = {{600, 520, 2048}, {130, 1024, 8192}, {256, 1040, 7168}, {70, 300, 6400}, {520, 128, 1536}, {1000, 300, 4096}};
             for (const auto& s : shared)

@@ -148,8 +148,9 @@ typedef struct nnf_plan
      * workgroup a few rows before its first tile; no pass of its own), and the row-streaming kernel for a few
      * activation rows and K above 8192, which works on ranges of K, adds the ranges up itself (the last workgroup to
      * arrive at a group of columns, in the order of the ranges; no reduction pass).  Products of 17 .. 256 rows may run on the K-streaming
-     * kernel over ranges of K then, which they do not without (another order of sums: equal to rounding, not bit for bit).  W8A8 with 8 .. 32 rows and K from
-     * 8192 runs its row-streaming kernel over two ranges of K the same way (int32 sums: exact), given sync_flags and
+     * kernel over ranges of K then, which they do not without (another order of sums: equal to rounding, not bit for bit).  The row-streaming kernel of W8A8
+     * (NNF_W8A8_GEMV_ROWS; by itself the library takes the K-streaming kernel there, which needs neither words nor workspace) runs 8 .. 32 rows
+     * with K from 8192 over two ranges of K the same way (int32 sums: exact), given sync_flags and
      * nnf_w8a8_gemm_variant_workspace_bytes of workspace; without either, in one pass over K (same bits, ~1 us more).
      *   sync_flags: device memory, 16-byte aligned, ALL ZERO before the first call that uses it; every call leaves it
      *     all zero again, so it needs clearing once (when it is allocated), not per call.  It must not be scratch
@@ -192,8 +193,8 @@ NNF_API int nnf_w4a16_gemm_variant(nnf_stream_t stream,
  * combination (group 32 / 64 / 128, K a multiple of group) 4-bit weights run on the kernels of nnf_w4a16_gemm where
  * those apply: the K-streaming kernel for 2 .. 512 rows where it was measured ahead (no workspace; 8-bit weights too), else
  * the row-streaming kernels for M = 1 with K a multiple of 256 from 1024 to 16384 and for 2 <= M <= 16
- * with K a multiple of 256 from about 2560 on (2048 / 4096 also up to 32 rows; above K = 8192 over ranges of K with a
- * reduction pass), and the tile GEMM for the other shapes above 16 rows with K a multiple of 256 and zero_points
+ * with K a multiple of 256 from about 2560 on (2048 / 4096 also up to 32 rows, where the K-streaming kernel is not ahead or has no room for the
+ * columns; above K = 8192 over ranges of K with a reduction pass), and the tile GEMM for the other shapes above 16 rows with K a multiple of 256 and zero_points
  * 4-byte aligned.  The ranges of K and the tile GEMM want nnf_wna16_gemm_workspace_bytes of workspace; called with
  * less (or NULL) the product runs on a plain kernel instead, at about half the rate.
  * Everything else runs on plain kernels that need no workspace: a row-per-wavefront GEMV for M = 1, an MFMA kernel
@@ -263,7 +264,7 @@ enum nnf_activation
 };
 
 /* Same GEMM with prologue / epilogue in one call.  They run inside the kernel that serves the shape: the
- * K-streaming kernel (2 rows and more), the row-streaming kernels (M = 1; M <= 64) and the tile GEMM multiply gamma in on the way in, rstd[m] and the
+ * K-streaming kernel (2 .. 1024 rows), the row-streaming kernels (M = 1; M <= 64) and the tile GEMM multiply gamma in on the way in, rstd[m] and the
  * epilogue at their end.  The K-streaming kernel and the row-streaming kernels add up the squares of the activations they hold themselves
  * (row-streaming: K a multiple of 1024 up to 8192; M = 1: any K they take): one launch in all; the tile GEMM and the other
  * forms take rstd from a small pre-pass over A (fp32 [M] in `workspace`); a GEMV kernel over ranges of K

@@ -285,8 +285,9 @@ namespace nnfusion
                     std::string ws = "nullptr";
                     if (ws_bytes > 0)
                         ws = allocate_tensor(Shape{ws_bytes}, element::character)->get_name();
-                    // a few rows with a long K: the row-streaming kernel over two ranges of K, which meet at one word per
-                    // workgroup of a range
+                    // a few rows with a long K: words for the row-streaming kernel over two ranges of K, which meet at one word per
+                    // workgroup of a range (the library's own choice is the K-streaming kernel now, which leaves words and workspace untouched; a
+                    // program that names the row-streaming kernel finds both)
                     std::string plan;
                     if (nnf::workspace::w8a8_mrows_preferred((int)M, (int)N, (int)K, nnf::workspace::PLAN_CUS) &&
                         nnf::workspace::w8a8_mrows_ranges((int)M, (int)N, (int)K, nnf::workspace::PLAN_CUS) > 1)

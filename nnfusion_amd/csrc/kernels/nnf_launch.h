@@ -94,7 +94,8 @@ namespace nnf
     // a few rows (workspace::w4a16_mrows_fits): weights streamed through LDS rings, activations in registers
     // (N: outputs; gate / fusion.gate: from 2 N weight rows)
     // the same kernel for groups of 2^group_shift = 32 / 64 / 128 and a scalar zero point or (zero_points != null) one per
-    // (row, group): 2 <= M <= 16 (32 up to K = 4096), K = 2048 / 4096 / 8192.  fusion: gamma (normalised inside the kernel; no rstd; where
+    // (row, group): 2 <= M <= 16 (32 up to K = 4096), K = 2048 / 4096 / 8192.  (By the library's own choice 17 .. 32 rows run here for K = 2048 in few
+    // tiles and where there are more tiles than the K-streaming kernel holds, N above 24576.)  fusion: gamma (normalised inside the kernel; no rstd; where
     // workspace::mrows_q_norm_inside), bias / residual or gate, where w4a16_mrows_q_fused_supported
     hipError_t launch_w4a16_mrows_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                     int K, int group_shift, int zp, const void* zero_points, int num_cu,
@@ -132,8 +133,9 @@ namespace nnf
                                         int M, int N, int K, int zp, int num_cu, const void* gamma = nullptr, void* Y = nullptr,
                                         const GemvFusion* epilogue = nullptr, uint32_t* sync = nullptr);
 
-    // 33 .. 64 rows: the K-streaming kernel, as `plan` (workspace::kstream_plan) says.  fusion: gamma (rstd computed inside), bias /
-    // residual or gate; over ranges of K neither gamma nor gate, the ranges' sums in `partial` (plan.partial_bytes) and one zeroed
+    // 2 .. 1024 rows in blocks of up to 64: the K-streaming kernel, as `plan` (workspace::kstream_plan) says, which sees to it that K is a
+    // multiple of 128 from 1024 on, N at least 16 (even with an odd number of groups of 128) and that tiles and LDS fit.  The caller: tensors
+    // aligned to 16 bytes, Y not over A.  fusion: gamma (rstd computed inside), bias / residual (which may be Y) or gate; over ranges of K neither gamma nor gate, the ranges' sums in `partial` (plan.partial_bytes) and one zeroed
     // word per workgroup of a range in `sync` (zero again afterwards)
     hipError_t launch_w4a16_kstream(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* Wq, const void* S,
                                     void* Y, int M, int N, int K, int zp, const GemvFusion& fusion, float* partial, uint32_t* sync);
@@ -230,7 +232,8 @@ namespace nnf
     hipError_t launch_w8a8_mrows(hipStream_t stream, const void* A, const void* s_tok, const void* W, const void* s_ch,
                                  void* Y, void* acc, int M, int N, int K, int num_cu, void* partial_ws = nullptr,
                                  size_t partial_bytes = 0, uint32_t* sync = nullptr, size_t sync_bytes = 0);
-    // a few rows, or blocks of rows: the K-streaming kernel, as `plan` (workspace::w8a8_kstream_plan) says
+    // 2 .. 1024 rows in blocks of up to 64: the K-streaming kernel, as `plan` (workspace::w8a8_kstream_plan) says (K a multiple of 128 from 1024
+    // on, N at least 16); the caller: tensors aligned to 16 bytes, the output not over A
     hipError_t launch_w8a8_kstream(hipStream_t stream, const workspace::KstreamPlan& plan, const void* A, const void* s_tok, const void* W,
                                    const void* s_ch, void* Y, void* acc, int M, int N, int K);
     bool w8a8_mrows_supported(int M, int N, int K, int num_cu);

@@ -421,8 +421,10 @@ namespace
         // elsewhere; the callers refuse other tensors that do)
         if (!aligned16(A) || !aligned16(Y))
             return NNF_OK;
-        // (RMSNorm of a few rows inside that kernel where it is inside the row-streaming kernels as well or SiLU-gate follows; otherwise a
-        // launch ahead of it, so that the fused product stays the nodes' own arithmetic, bit for bit)
+        // RMSNorm of a few rows of 4-bit weights: inside that kernel where it is inside the row-streaming kernels as well or SiLU-gate follows,
+        // otherwise a launch ahead of it, although inside is faster (11 x 8064 x 1408 in groups of 32 7.0 us ahead, 5.4 inside; 25 x 768 x 3456
+        // 8.6, 7.2): the tests hold these products to the bits of the nodes' own kernels one after the other.  More rows, and 8 bits, had the
+        // nodes one by one before and no such test.
         if (q->bits == 4 && fusion.gamma && !fusion.gate && M <= 32 && !nnf::workspace::mrows_q_norm_inside(M, K))
         {
             if (nnf::workspace::kstream_choice_q(M, N, K, group_shift_of(q->group), num_cu, false, false).tiles > 0)

@@ -642,6 +642,7 @@ namespace nnf
         // the int32 sums of the ranges): every workgroup fetches all M x K activations ahead of its first MFMA, over two ranges
         // half of them.  Measured (8 .. 32 rows, N = 4096 .. 8192, K = 8192 and 14336) 0.8 - 1.3 us faster than one pass;
         // slower at K = 4096, with more than four tiles per workgroup (N = 16384: +3 us) and over four ranges.
+        // (A caller who names the row-streaming kernel; by itself the library runs these products on the K-streaming kernel: w8a8_kstream_choice.)
         inline int w8a8_mrows_ranges(int M, int N, int K, int num_cu)
         {
             const int per_range = num_cu / 2;

@@ -190,8 +190,8 @@ def _w8a8_variant(a, s_tok, w, s_ch, y, acc, variant, plan, workspace, sync=None
 
 def w8a8_gemm(a, s_tok, w, s_ch, out=None, workspace=None, variant="auto", plan=None, sync=None):
     """Y fp16 [M,N] = fp16((float)(A . W^T) * s_tok[m] * s_ch[n]) ; a i8 [M,K], w i8 [N,K].  A variant (a key of
-    W8A8_VARIANTS), a plan (tile_rows, k_parts) or `sync` (see sync_flags: a few rows with a long K then run over
-    two ranges of K in one launch) goes through nnf_w8a8_gemm_variant."""
+    W8A8_VARIANTS), a plan (tile_rows, k_parts) or `sync` (see sync_flags: with variant "gemv_rows" a few rows with a
+    long K then run over two ranges of K in one launch) goes through nnf_w8a8_gemm_variant."""
     if variant == "auto" and plan is None:
         return _native.w8a8_gemm(a, s_tok, w, s_ch, out, workspace, sync)
     assert a.dtype == torch.int8 and w.dtype == torch.int8

@@ -178,10 +178,11 @@ namespace nnf
         {
 #pragma unroll
             for (int e = 0; e < GQ; ++e)
-            {
-                const int u = min(wave * 64 + e * (WAVES * 64) + lane, a_units - 1);
-                gq[e] = reinterpret_cast<const uintx4*>(f.gamma)[u];
-            }
+                if (wave * 64 + e * (WAVES * 64) < a_units)
+                {
+                    const int u = min(wave * 64 + e * (WAVES * 64) + lane, a_units - 1);
+                    gq[e] = reinterpret_cast<const uintx4*>(f.gamma)[u];
+                }
         }
 
         // ---- this wavefront's K segment; its first D rows are fixed: widx, widx + gpw, ... ---------------------
@@ -234,6 +235,12 @@ namespace nnf
         // (two rows now; the rest of the ring after the activations are in registers: with everything asked for at
         // once the last wavefronts stall at issue -- a CU takes about 64 wavefront-wide loads -- and hold up the barrier)
         constexpr int D0 = D < 2 ? D : 2;
+        // (A CU's loads come back in the order they were issued in, whichever wavefront they belong to: with RMSNorm, whose weight makes
+        // the prologue's loads more, the last wavefronts' would queue up behind the first ones' weights, and the barrier below wait
+        // for those to come from memory.  N = K = 4096: that barrier opens 1.1 us after the start of the launch, 1.5 - 1.6 without this
+        // one, and the launch takes 4.28 us in a graph, 5.20 before; without RMSNorm this barrier costs 0.07 us and gives nothing.)
+        if (EPI != 0 && f.gamma)
+            asm volatile("s_barrier" ::: "memory");
 #pragma unroll
         for (int d = 0; d < D0; ++d)
             issue(widx + d * gpw, d);
@@ -261,34 +268,27 @@ namespace nnf
         // Only the weights asked for above may still be in flight afterwards: the scales have landed too.
         __builtin_amdgcn_s_waitcnt(rows_vmcnt(D0 * LPR));
         NNF_ROWS_STAMP(1); // activations and scales have arrived
+        // (Every instruction here is time between the activations' arrival and the first row: sums and sum of squares on
+        // v_dot2_f32_f16, 0.2 us less with RMSNorm than conversions, adds and a run-time choice among the gamma registers.)
+        float ss = 0.f;
         if (a_loader)
         {
-            const float ce = -(1024.0f + (QZT ? 0.f : (float)zp));
-            const float co = W8 ? ce : -(64.0f + (QZT ? 0.f : (float)zp));
-            float ss = 0.f;
-            int e = 0;
-            for (int u0 = wave * 64; u0 < a_units; u0 += WAVES * 64, ++e)
-            {
-                const int u = u0 + lane;
+            // -(1024 + zp) and -(64 + zp) twice, as bits (exact: ulps of 1 and 1/16)
+            const uint32_t z = QZT ? 0u : (uint32_t)zp;
+            const uint32_t ce_bits = (0xE400u | z) * 0x10001u, co_bits = W8 ? ce_bits : (0xD400u | (z << 4)) * 0x10001u;
+            const half2_t ce = as_half2(ce_bits), co = as_half2(co_bits), one = {(half_t)1.0f, (half_t)1.0f};
+            auto prepare = [&](int u, const uintx4& g) {
                 uintx4 raw = act[u];
-                if (own_rstd && u < a_units)
+                if (own_rstd)
                 {
                     // RMSNorm without a pass of its own: every unit of the row goes through exactly one lane here
-                    const uint32_t rr[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                    {
-                        const half2_t hh = as_half2(rr[i]);
-                        ss += (float)hh.x * (float)hh.x + (float)hh.y * (float)hh.y;
-                    }
+                    const float sq = dot2(as_half2(raw.x), as_half2(raw.x), dot2(as_half2(raw.y), as_half2(raw.y), 0.f)) +
+                                     dot2(as_half2(raw.z), as_half2(raw.z), dot2(as_half2(raw.w), as_half2(raw.w), 0.f));
+                    ss += u < a_units ? sq : 0.f;
                 }
                 if (EPI != 0 && f.gamma)
                 {
                     // fp16(a * gamma): the product of two fp16 values, rounded once
-                    uintx4 g = gq[0];
-#pragma unroll
-                    for (int i = 1; i < GQ; ++i)
-                        g = e == i ? gq[i] : g;
                     raw.x = as_u32(as_half2(raw.x) * as_half2(g.x));
                     raw.y = as_u32(as_half2(raw.y) * as_half2(g.y));
                     raw.z = as_u32(as_half2(raw.z) * as_half2(g.z));
@@ -296,24 +296,44 @@ namespace nnf
                 }
                 const uintx4 a = W8 ? raw : permute_a8(raw);
                 const half2_t x = as_half2(a.x), y = as_half2(a.y), z = as_half2(a.z), w = as_half2(a.w);
-                const float se = ((float)x.x + (float)x.y) + ((float)z.x + (float)z.y);
-                const float so = ((float)y.x + (float)y.y) + ((float)w.x + (float)w.y);
                 act[u] = a;
-                corr[u] = ce * se + co * so;
+                corr[u] = dot2(x, ce, dot2(z, ce, 0.f)) + dot2(y, co, dot2(w, co, 0.f));
                 if (QZT)
-                    asum_u[u] = se + so;
-            }
-            if (own_rstd)
-            {
-                ss = row16_sum(ss);
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x142, 0xA, 0xF, false));
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x143, 0xC, 0xF, false));
-                if (lane == 63)
-                    sum_sq[wave] = ss;
-            }
+                    asum_u[u] = dot2(x, one, dot2(z, one, 0.f)) + dot2(y, one, dot2(w, one, 0.f));
+            };
+            if constexpr (GQ > 1)
+                static_for<0, GQ>([&](auto ec) {
+                    constexpr int e = decltype(ec)::value;
+                    if (wave * 64 + e * (WAVES * 64) < a_units)
+                        prepare(wave * 64 + e * (WAVES * 64) + lane, gq[e]);
+                });
+            else
+                for (int u0 = wave * 64; u0 < a_units; u0 += WAVES * 64)
+                    prepare(u0 + lane, gq[0]);
+        }
+        if (own_rstd)
+        {
+            ss = row16_sum(ss);
+            ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x142, 0xA, 0xF, false));
+            ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x143, 0xC, 0xF, false));
+            if (lane == 63)
+                sum_sq[wave] = ss;
         }
         lds_barrier();
         NNF_ROWS_STAMP(2); // every wavefront has prepared its share of the activations
+        // (here, while the first weights are on their way, and not at the flush, where nothing hides it: 0.35 us)
+        float rs = 1.0f;
+        if (own_rstd)
+        {
+            float part[WAVES], total = 0.f;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w)
+                part[w] = sum_sq[w];
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w)
+                total += part[w];
+            rs = 1.0f / __builtin_sqrtf(total / (float)K + f.rms_eps);
+        }
         uintx4 areg[SEG][UPL];
         float ncorr[SEG], asum[SEG];
 #pragma unroll
@@ -474,14 +494,8 @@ namespace nnf
         // ---- outputs ------------------------------------------------------------------------------------
         lds_barrier();
         NNF_ROWS_STAMP(5); // ... and every wavefront's
-        float rs = (EPI != 0 && f.rstd) ? f.rstd[0] : 1.0f;
-        if (own_rstd)
-        {
-            float total = 0.f;
-            for (int w = 0; w * 64 < a_units && w < WAVES; ++w) // the wavefronts that fetched a share of the row
-                total += sum_sq[w];
-            rs = 1.0f / __builtin_sqrtf(total / (float)K + f.rms_eps);
-        }
+        if (EPI != 0 && f.rstd)
+            rs = f.rstd[0];
         for (int r = tid; r < n_out; r += WAVES * 64)
         {
             float y = 0.f;

@@ -146,44 +146,76 @@ namespace nnf
         }
     }
 
+    // im / M for 0 <= im < 2^13 and M <= 64, by multiplication (a division is forty instructions, at the end of the launch)
+    struct DivideByRows
+    {
+        uint32_t inverse;
+        __device__ __forceinline__ explicit DivideByRows(int M) : inverse((uint32_t)(1048576.0f / (float)M) + 1u) {}
+        __device__ __forceinline__ int operator()(int im) const { return (int)(((uint32_t)im * inverse) >> 20); }
+    };
+    // The residual of a thread's first two outputs, asked for in the prologue: at the flush the load took 0.3 - 0.7 us of a launch.
+    struct MrowsAhead
+    {
+        half_t residual[2];
+    };
+    // output `idx` of the workgroup (rows of 16 columns: output tile it, row m) -> column nn; false: a column that the tile before it owns
+    // (the last tile of an N that is not a multiple of 16 was moved back over those: written once, so that a residual that is
+    // the output buffer itself is added once)
+    __device__ __forceinline__ bool mrows_output(int idx, int t0, int M, int N, const DivideByRows& by_rows, int& it, int& m, int& nn)
+    {
+        const int im = idx >> 4;
+        it = by_rows(im);
+        m = im - it * M;
+        nn = min((t0 + it) * 16, N - 16) + (idx & 15);
+        return nn >= (t0 + it) * 16;
+    }
+    __device__ __forceinline__ void mrows_ask_ahead(MrowsAhead& x, const half_t* residual, int t0, int T_out, int M, int N, int tid)
+    {
+        const DivideByRows by_rows(M);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+        {
+            int it, m, nn;
+            mrows_output(min(tid + i * 512, T_out * M * 16 - 1), t0, M, N, by_rows, it, m, nn);
+            x.residual[i] = residual[(size_t)m * N + nn];
+        }
+    }
     // The workgroup's parked sums -> Y.  Plain: fp16 of the sum.  Fused (see GemvFusion in nnf_launch.h): the sums of
     // row m times rstd[m]; gate: tiles 2 i and 2 i + 1 of the workgroup are the gate and the up rows of its output tile
-    // i; bias and residual.  t0: the workgroup's first output tile, T_out of them; N: output columns.
-    // sum_sq ([8 wavefronts][MB x 16 rows], or null) and K: RMSNorm without a pass of its own (gamma, no rstd).
+    // i; bias and residual (that of a thread's first two outputs: `ahead`, unless null).  t0: the workgroup's first output tile, T_out of
+    // them; N: output columns.  own_rstd ([MB x 16 rows] of LDS, or null): RMSNorm without a pass of its own (gamma, no rstd).
     template <bool FUSED, int MB>
     __device__ __forceinline__ void mrows_flush(const float* parked, half_t* __restrict__ Y, int t0, int T_out, int M, int N,
-                                                int tid, const GemvFusionArgs& f, int gate, const float* sum_sq = nullptr, int K = 0)
+                                                int tid, const GemvFusionArgs& f, int gate, const float* own_rstd = nullptr,
+                                                const MrowsAhead* ahead = nullptr)
     {
-        for (int idx = tid; idx < T_out * M * 16; idx += 512)
-        {
-            const int n = idx & 15;
-            const int im = idx >> 4;
-            const int it = im / M, m = im - it * M;
-            const int nn = min((t0 + it) * 16, N - 16) + n;
-            // (the last tile of an N that is not a multiple of 16 was moved back over columns that the tile before it
-            // owns: written once, so that a residual that is the output buffer itself is added once)
-            if (nn < (t0 + it) * 16)
-                continue;
+        const DivideByRows by_rows(M);
+        auto finish = [&](int idx, const half_t* residual) {
+            int it, m, nn;
+            if (!mrows_output(idx, t0, M, N, by_rows, it, m, nn))
+                return;
             const size_t at = (size_t)m * N + nn;
             if (!FUSED)
                 Y[at] = (half_t)parked[idx];
             else
             {
-                float rs = f.rstd ? f.rstd[m] : 1.0f;
-                if (sum_sq)
-                {
-                    float total = 0.f;
-#pragma unroll
-                    for (int w = 0; w < MR_WAVES; ++w)
-                        total += sum_sq[w * (MB * 16) + m];
-                    rs = 1.0f / __builtin_sqrtf(total / (float)K + f.rms_eps);
-                }
+                const float rs = own_rstd ? own_rstd[m] : f.rstd ? f.rstd[m] : 1.0f;
                 if (gate)
-                    Y[at] = finish_silu_gate(parked[((2 * it) * M + m) * 16 + n] * rs, parked[((2 * it + 1) * M + m) * 16 + n] * rs);
+                    Y[at] = finish_silu_gate(parked[((2 * it) * M + m) * 16 + (idx & 15)] * rs, parked[((2 * it + 1) * M + m) * 16 + (idx & 15)] * rs);
                 else
-                    Y[at] = finish_bias_residual(parked[idx] * rs, f.bias, nn, f.residual, at);
+                    Y[at] = finish_bias_residual(parked[idx] * rs, f.bias, nn, residual ? residual : f.residual, residual ? 0 : at);
             }
+        };
+        const int total = T_out * M * 16;
+        if (FUSED && ahead)
+        {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (tid + i * 512 < total)
+                    finish(tid + i * 512, f.residual ? &ahead->residual[i] : nullptr);
         }
+        for (int idx = tid + (FUSED && ahead ? 1024 : 0); idx < total; idx += 512)
+            finish(idx, nullptr);
     }
 
     template <int MB, int GA>
@@ -298,16 +330,23 @@ namespace nnf
 
     // K = GW * STEPS * 1024; MB = blocks of 16 activation rows (1 or 2).
     // LDS (bytes): weights [8 wavefronts][2 slots][GW KiB] | scales [8][2][256] | partial tiles [2][8][MB KiB] |
-    //              parked sums [tiles of the workgroup][M][16] fp32
+    //              sums of squares [8][16 MB] fp32 | parked sums [tiles of the workgroup][M][16] fp32
+    //              (from the partial tiles on, while the kernel starts: activations [8][8 KiB] | RMSNorm weight [8][1 or 2 KiB])
     // pack = M | zp << 8 | gate << 16;  a workgroup's output tiles: tiles_q, one more for the first tiles_r workgroups.
     // FUSED: the prologue / epilogue of `f`; gate != 0: N outputs from 2 N weight rows, the workgroup walks the gate and
     // the up tile of each of its output tiles in turn (twice the tiles).
-    // STAGE: the activations through LDS as whole lines (row_block_fetch); otherwise straight into the registers
-    template <int GW, int STEPS, int MB, bool FUSED, bool STAGE>
+    // RL: loads per block of activations, of four rows each (M <= 4 RL with one block of rows)
+    // tiles = tiles_q | tiles_r << 16.  The pointers that the prologue needs come first: fourteen dwords of arguments arrive in
+    // scalar registers with the wavefront, the rest (Y, f) is loaded from memory.
+    // FUSE: 0 plain, 1 the epilogue of `f` (and gate), 2 RMSNorm as well.  (An instantiation of its own: with a branch on gamma in every
+    // block of activations the prologue took 0.3 us longer, RMSNorm or not.)
+    template <int GW, int STEPS, int MB, int FUSE, int RL>
     __global__ __launch_bounds__(512) void w4a16_mrows_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
-                                                              const half_t* __restrict__ S, half_t* __restrict__ Y, int N,
-                                                              int tiles_q, int tiles_r, int pack, GemvFusionArgs f)
+                                                              const half_t* __restrict__ S, const half_t* gamma, const half_t* residual,
+                                                              int N, int tiles, int pack, half_t* Y, GemvFusionArgs f)
     {
+        static_assert(RL == 4 || (MB == 1 && (RL == 1 || RL == 2)), "rows of a block");
+        constexpr bool FUSED = FUSE != 0, norm = FUSE == 2;
         static_assert(GW >= 1 && GW <= 8 && STEPS >= 1 && GW * STEPS <= 8, "K = GW * STEPS * 1024");
         static_assert(MB == 1 || (MB == 2 && GW * STEPS <= 4), "two blocks of rows: 32 VGPRs per group");
         constexpr int K = GW * STEPS * 1024, G = K / 128;
@@ -334,6 +373,7 @@ namespace nnf
         // (gate rides in `pack`, among the arguments that arrive in scalar registers with the wavefront: as an argument of
         // its own behind `f` it was loaded from memory and waited for ahead of the first weight load)
         const int M = pack & 0xff, zp = (pack >> 8) & 0xff, gate = (pack >> 16) & 1;
+        const int tiles_q = tiles & 0xffff, tiles_r = (int)((unsigned)tiles >> 16);
         const int b = blockIdx.x;
         const int t0 = b * tiles_q + min(b, tiles_r);
         const int T_out = tiles_q + (b < tiles_r ? 1 : 0);
@@ -386,119 +426,112 @@ namespace nnf
                                              (mr_lds_ptr_t)(sc_ring + slot * 256), 4, 0, 0);
         };
 
-        // ---- the first two tiles, then the activations: straight into the MFMA operand registers -----------------
-        // (the activations are requested last: vector-memory operations complete in order and the compiler waits
-        // for them where they are used, which then also covers the two tiles -- requested first, those tiles'
-        // loads are not held back by anything)
+        // ---- the prologue's loads: RMSNorm weight, residual, activations, the first two steps of weights ----------------------
+        // A CU's loads come back in the order they were issued in, whichever wavefront they belong to and wherever they come
+        // from.  Activations asked for behind the weights therefore wait for those to come from memory (1.4 us), and
+        // everything that is done to them starts only then; weights behind all activations are asked for late (a CU has
+        // about 64 loads in flight).  So: as many blocks of activations as LDS has room for, the weights, the rest.
+        // Measured (us a launch in a graph, weights from memory, N = K = 4096 plain / with RMSNorm / with a residual): 6 rows 5.00 / 7.46 /
+        // 5.95 with the weights first and RMSNorm's weight last, 4.42 / 5.32 / 4.75 now; 16 rows 5.46 / 6.88 / 6.00, now 5.43 / 6.08 /
+        // 5.46.  (Three blocks of 16 rows in flight 0.1 slower, one block ahead of the weights and the others behind 0.2 at 6 rows, a
+        // barrier between activations and weights 0 - 0.3.)
+        // The RMSNorm weight of the wavefront's k positions (GA x 256 bytes) comes through LDS as well, one load per four groups.
+        uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
+        const uint8_t* gamma_block = red + MR_WAVES * (2 * ROW_BLOCK_BYTES) + wave * (GAMMA_LOADS * 1024);
+        if constexpr (norm)
+        {
+#pragma unroll
+            for (int i = 0; i < GAMMA_LOADS; ++i)
+            {
+                const int g = min(4 * i + (lane >> 4), GA - 1);
+                const uint8_t* src = reinterpret_cast<const uint8_t*>(gamma) + wave * (GW * 256) + (g / GW) * (SPAN * 4) + (g % GW) * 256 + (lane & 15) * 16;
+                __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(gamma_block + i * 1024), 16, 0, 0);
+            }
+        }
+        constexpr int NP = MB * GA;                                                        // blocks of 4 RL rows x 256 bytes
+        constexpr int ROOM = 2 * ROW_BLOCK_BYTES / 1024 / RL, NF = ROOM < NP ? ROOM : NP; // ... in flight, at the places p % NF
+        auto fetch = [&](auto p_c) {
+            constexpr int p = decltype(p_c)::value, mb = p / GA, g = p % GA;
+#pragma unroll
+            for (int c = 0; c < RL; ++c)
+            {
+                const int r = c * 4 + (lane >> 4);
+                const uint8_t* src = reinterpret_cast<const uint8_t*>(A) + (size_t)min(mb * 16 + r, M - 1) * (K * 2) +
+                                     ((g / GW) * (SPAN * 4) + wave * (GW * 256) + (g % GW) * 256 + ((lane & 15) ^ r) * 16);
+                __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(stage + (p % NF) * (RL * 1024) + c * 1024), 16, 0, 0);
+            }
+        };
+        unroll_for<0, NF>([&](auto p_c) { fetch(p_c); });
         issue(0, 0, 0);
         issue(min(1 / STEPS, T - 1), 1 % STEPS, 1);
-        // (through LDS as whole lines, see row_block_fetch: two blocks per wavefront, over what holds the partial tiles
-        // and the parked sums later -- hence the barrier behind the last block)
-        // (a few rows: a load touches few lines as it is -- the lanes of the rows that do not exist ask for the last row
-        // again -- and the detour costs 0.3 - 0.5 us: straight into the registers)
+        // ---- the activations, block by block: MFMA operand registers in the pair order of the nibble trick, the constant part
+        // of each group's sum; RMSNorm: gamma onto them (fp16 products, rounded once) and the wavefront's share of sum a^2 of
+        // every row
         uintx4 areg[MB][GA][4];
-        if constexpr (!STAGE)
-        {
-            const uint8_t* a_bytes = reinterpret_cast<const uint8_t*>(A);
-            const uint32_t a_off = (uint32_t)min(col, M - 1) * (uint32_t)(K * 2) + (uint32_t)wave * (GW * 256) + (uint32_t)kq * 64u;
-#pragma unroll
-            for (int g = 0; g < GA; ++g)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    areg[0][g][j] = *reinterpret_cast<const uintx4*>(a_bytes + (size_t)(a_off + (g / GW) * (SPAN * 4) + (g % GW) * 256 + j * 16));
-        }
-        else
-        {
-            uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
-            constexpr int NP = MB * GA;
-            auto fetch = [&](int p) {
-                const int mb = p / GA, g = p % GA;
-                row_block_fetch(reinterpret_cast<const uint8_t*>(A), (size_t)K * 2, mb * 16, M - 1,
-                                (size_t)((g / GW) * (SPAN * 4) + wave * (GW * 256) + (g % GW) * 256), stage + (p & 1) * ROW_BLOCK_BYTES, lane);
-            };
-            fetch(0);
-#pragma unroll
-            for (int p = 0; p < NP; ++p)
-            {
-                if (p + 1 < NP)
-                {
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // block p-1 has been read out of the half that is filled next
-                    fetch(p + 1);
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
-                }
-                else if (FUSED && f.gamma)
-                {
-                    // The RMSNorm weight of the wavefront's k positions (GA x 256 bytes) follows the last block into the
-                    // free half, one load per four groups: as sixteen 16-byte loads per lane straight into registers --
-                    // the sixteen lanes of a column asking for the same bytes -- it took the load pipeline a microsecond
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-                    for (int i = 0; i < GAMMA_LOADS; ++i)
-                    {
-                        const int g = min(4 * i + (lane >> 4), GA - 1);
-                        const uint8_t* src = reinterpret_cast<const uint8_t*>(f.gamma) + wave * (GW * 256) + (g / GW) * (SPAN * 4) +
-                                             (g % GW) * 256 + (lane & 15) * 16;
-                        __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(stage + (NP & 1) * ROW_BLOCK_BYTES + i * 1024),
-                                                         16, 0, 0);
-                    }
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(GAMMA_LOADS));
-                }
-                else
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    areg[p / GA][p % GA][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
-            }
-        }
-        // RMSNorm without a pass of its own: the wavefront's share of sum a^2 of every row, from the registers
-        const bool own_rstd = FUSED && f.gamma && !f.rstd;
-        float ss[MB];
-        if (own_rstd)
-        {
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-            {
-                ss[mb] = 0.f;
-#pragma unroll
-                for (int g = 0; g < GA; ++g)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                    {
-                        // (v_dot2_f32_f16: one instruction per pair; with conversions and multiplies of its own the sum took
-                        // more than a microsecond of a SIMD's vector unit at 16 rows x 4096)
-                        const uint32_t rr[4] = {areg[mb][g][j].x, areg[mb][g][j].y, areg[mb][g][j].z, areg[mb][g][j].w};
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            ss[mb] = dot2(as_half2(rr[i]), as_half2(rr[i]), ss[mb]);
-                    }
-                ss[mb] += __shfl_xor(ss[mb], 16, 64);
-                ss[mb] += __shfl_xor(ss[mb], 32, 64);
-            }
-        }
-        if constexpr (STAGE)
-        {
-            if (FUSED && f.gamma)
-            {
-                const uint8_t* gamma_block = red + wave * (2 * ROW_BLOCK_BYTES) + ((MB * GA) & 1) * ROW_BLOCK_BYTES;
-                __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-                mrows_scale_a<MB, GA>(areg, [&](int g) { return gamma_block + g * 256 + kq * 64; });
-            }
-            // (the blocks lay over what holds the partial tiles, the sums of squares and the parked sums from here on)
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __syncthreads();
-        }
-        else if (FUSED && f.gamma)
-            mrows_scale_a<MB, GA>(areg, [&](int g) {
-                return reinterpret_cast<const uint8_t*>(f.gamma) + wave * (GW * 256) + kq * 64 + (g / GW) * (SPAN * 4) + (g % GW) * 256;
-            });
-        if (own_rstd && kq == 0)
-        {
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-                sum_sq[wave * (MB * 16) + mb * 16 + col] = ss[mb];
-        }
         floatx4 ncorr[MB][GA];
-        mrows_prepare_a<MB, GA>(areg, ncorr, zp);
+        floatx4 sq[MB]; // A . A^T: the sums of squares are its diagonal (the matrix cores have nothing else to do here)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            sq[mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+        // -(1024 + zp), -(64 + zp) twice each, as bits (exact)
+        const uint32_t ce2 = (0xE400u | (uint32_t)zp) * 0x10001u, co2 = (0xD400u | ((uint32_t)zp << 4)) * 0x10001u;
+        const half8_t cvec = __builtin_bit_cast(half8_t, uintx4{ce2, co2, ce2, co2});
+        unroll_for<0, NP>([&](auto p_c) {
+            constexpr int p = decltype(p_c)::value, mb = p / GA, g = p % GA;
+            // what has been asked for behind this block
+            constexpr int LATER = RL * ((NF + p < NP ? NF + p : NP) - 1 - p) + (p < NF ? 2 * LT : 0);
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(LATER));
+            const int row = col & (4 * RL - 1);
+            uintx4 a[4], gm[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                a[j] = *reinterpret_cast<const uintx4*>(stage + (p % NF) * (RL * 1024) + row * 256 + (((kq * 4 + j) ^ row) << 4));
+            if constexpr (norm)
+            {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    gm[j] = *reinterpret_cast<const uintx4*>(gamma_block + g * 256 + kq * 64 + j * 16);
+            }
+            if constexpr (p + NF < NP)
+            {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the block has been read out of the place that is filled next
+                fetch(std::integral_constant<int, (p + NF < NP ? p + NF : 0)>{});
+            }
+            floatx4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                if constexpr (norm)
+                {
+                    sq[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[j]), __builtin_bit_cast(half8_t, a[j]), sq[mb], 0, 0, 0);
+                    a[j].x = as_u32(as_half2(a[j].x) * as_half2(gm[j].x));
+                    a[j].y = as_u32(as_half2(a[j].y) * as_half2(gm[j].y));
+                    a[j].z = as_u32(as_half2(a[j].z) * as_half2(gm[j].z));
+                    a[j].w = as_u32(as_half2(a[j].w) * as_half2(gm[j].w));
+                }
+                areg[mb][g][j] = permute_a8(a[j]);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[mb][g][j]), cvec, t, 0, 0, 0);
+            }
+            ncorr[mb][g] = t;
+        });
+        // (behind the weights: the tile loop's counted waits then wait for two of the second step's loads as well)
+        MrowsAhead ahead;
+        if (FUSED && residual)
+            mrows_ask_ahead(ahead, residual, t0, T_out, M, N, tid);
+        // (the blocks lay over what holds the partial tiles, the sums of squares and the parked sums from here on)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (norm)
+        {
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+            {
+                // row m of D in element m % 4 of the lanes with kq = m / 4
+                const float lower = (col & 1) ? sq[mb].y : sq[mb].x, upper = (col & 1) ? sq[mb].w : sq[mb].z;
+                const float sum = (col & 2) ? upper : lower;
+                if (kq == (col >> 2)) // (by hand: ahead of an LDS write that it can see, the compiler waits for every LDS-bound load in flight)
+                    asm volatile("ds_write_b32 %0, %1" ::"v"(lds_address(sum_sq + wave * (MB * 16) + mb * 16 + col)), "v"(sum) : "memory");
+            }
+        }
 
         // ---- tile loop ---------------------------------------------------------------------------------------
         // operand reads of a slot: lane (n = col, kq), group g: piece g*4 + kq of row n
@@ -540,11 +573,25 @@ namespace nnf
                     mrows_group<MB, GA>(acc, areg, ncorr, st * GW + g, wv[g], sv[g], MAGIC, MAGIC_HI, MASK_LO, MASK_HI);
             }
             mrows_reduce_park<MB>(acc, red, red_addr, parked_addr, it & 1, it, M, tid);
+            if (norm && it == 0 && tid < MB * 16)
+            {
+                // rstd of row `tid`, in place of its first share (the sums were visible with the tile's barrier; at the flush this
+                // took 0.4 us, a row's share at a time for every output)
+                float part[MR_WAVES], total = 0.f;
+#pragma unroll
+                for (int w = 0; w < MR_WAVES; ++w)
+                    part[w] = sum_sq[w * (MB * 16) + tid];
+#pragma unroll
+                for (int w = 0; w < MR_WAVES; ++w)
+                    total += part[w];
+                const float rs = 1.0f / __builtin_sqrtf(total / (float)K + f.rms_eps);
+                asm volatile("ds_write_b32 %0, %1" ::"v"(lds_address(sum_sq + tid)), "v"(rs) : "memory");
+            }
         }
         __builtin_amdgcn_s_waitcnt(mr_vmcnt(0)); // the reloads past the end, before the LDS goes away
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         // ---- flush: parked sums -> Y -----------------------------------------------------------------------------
-        mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate, own_rstd ? sum_sq : nullptr, K);
+        mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate, norm ? sum_sq : nullptr, FUSED && !f.bias ? &ahead : nullptr);
     }
 
     // ---- other block parameters ------------------------------------------------------------------------------------
@@ -1581,7 +1628,7 @@ namespace nnf
         }
 
         // N: output columns (fusion.gate: from 2 N weight rows)
-        template <int GW, int STEPS, int MB, bool FUSED, bool STAGE = true>
+        template <int GW, int STEPS, int MB, int FUSE, int RL>
         hipError_t launch_mrows_mb(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
                                    int num_cu, const GemvFusion& fusion)
         {
@@ -1592,7 +1639,7 @@ namespace nnf
                 workspace::w4a16_mrows_lds_bytes(GW * STEPS * 1024, M, (fusion.gate ? 2 : 1) * (tiles_q + (tiles_r ? 1 : 0)));
             if (lds > MAX_LDS_BYTES)
                 return hipErrorInvalidValue;
-            auto kernel = &w4a16_mrows_kernel<GW, STEPS, MB, FUSED, STAGE>;
+            auto kernel = &w4a16_mrows_kernel<GW, STEPS, MB, FUSE, RL>;
             if (lds > 64 * 1024)
             {
                 static LdsGrant granted;
@@ -1600,26 +1647,34 @@ namespace nnf
                 if (e != hipSuccess)
                     return e;
             }
+            if (tiles_q > 0xffff)
+                return hipErrorInvalidValue;
             hipLaunchKernelGGL(kernel, dim3(grid), dim3(MR_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
-                               (const half_t*)S, (half_t*)Y, N, tiles_q, tiles_r, M | (zp << 8) | (fusion.gate ? 1 << 16 : 0),
-                               fusion_args(fusion));
+                               (const half_t*)S, (const half_t*)fusion.gamma, (const half_t*)fusion.residual, N, tiles_q | (tiles_r << 16),
+                               M | (zp << 8) | (fusion.gate ? 1 << 16 : 0), (half_t*)Y, fusion_args(fusion));
             return hipGetLastError();
         }
 
+        template <int GW, int STEPS, int MB, int RL>
+        hipError_t launch_mrows_rl(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
+                                   int num_cu, const GemvFusion& fusion)
+        {
+            return fusion.gamma   ? launch_mrows_mb<GW, STEPS, MB, 2, RL>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion)
+                   : fusion.any() ? launch_mrows_mb<GW, STEPS, MB, 1, RL>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion)
+                                  : launch_mrows_mb<GW, STEPS, MB, 0, RL>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion);
+        }
+        // (blocks of 4, 8 or 16 rows of activations: with M rows in blocks of 16, up to four times the bytes, most of them of
+        // the last row again, would pass through the memory pipeline)
         template <int GW, int STEPS>
         hipError_t launch_mrows(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
                                 int num_cu, const GemvFusion& fusion)
         {
-            const bool fused = fusion.any();
-            if (M <= 16 && !workspace::mrows_stages_activations(M, GW * STEPS * 1024))
-                return fused ? launch_mrows_mb<GW, STEPS, 1, true, false>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion)
-                             : launch_mrows_mb<GW, STEPS, 1, false, false>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion);
             if (M <= 16)
-                return fused ? launch_mrows_mb<GW, STEPS, 1, true>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion)
-                             : launch_mrows_mb<GW, STEPS, 1, false>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion);
+                return M <= 4   ? launch_mrows_rl<GW, STEPS, 1, 1>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion)
+                       : M <= 8 ? launch_mrows_rl<GW, STEPS, 1, 2>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion)
+                                : launch_mrows_rl<GW, STEPS, 1, 4>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion);
             if constexpr (GW * STEPS <= 4)
-                return fused ? launch_mrows_mb<GW, STEPS, 2, true>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion)
-                             : launch_mrows_mb<GW, STEPS, 2, false>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion);
+                return launch_mrows_rl<GW, STEPS, 2, 4>(stream, A, Wq, S, Y, M, N, zp, num_cu, fusion);
             return hipErrorInvalidValue;
         }
     } // namespace

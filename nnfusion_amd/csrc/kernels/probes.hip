@@ -348,19 +348,19 @@ extern "C" int nnf_probe_gemm_timeline(void* stream, const void* A, const void* 
     p.trace = trace;
     if (plan.tile_weight_rows == 128)
     {
-        using T = gemm_sk::Tile<4, 1>;
-        auto kernel = &w4a16_gemm_sk_kernel<4, 1, false, false, false, false>;
+        using T = gemm_sk::TileOf<128, 128>;
+        auto kernel = &w4a16_gemm_sk_kernel<T::TM, T::TN, T::NW, T::KH, false, false, false, false>;
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES) != hipSuccess)
             return -1;
-        launch_sk_kernel(kernel, plan.grid, T::LDS_BYTES, (hipStream_t)stream, p);
+        launch_sk_kernel<T>(kernel, plan.grid, (hipStream_t)stream, p);
     }
     else
     {
-        using T = gemm_sk::Tile<4, 2>;
-        auto kernel = &w4a16_gemm_sk_kernel<4, 2, false, false, false, false>;
+        using T = gemm_sk::TileOf<128, 256>;
+        auto kernel = &w4a16_gemm_sk_kernel<T::TM, T::TN, T::NW, T::KH, false, false, false, false>;
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES) != hipSuccess)
             return -1;
-        launch_sk_kernel(kernel, plan.grid, T::LDS_BYTES, (hipStream_t)stream, p);
+        launch_sk_kernel<T>(kernel, plan.grid, (hipStream_t)stream, p);
     }
     return hipGetLastError() == hipSuccess ? plan.grid : -1;
 }

@@ -116,30 +116,74 @@ namespace nnf
     namespace gemm_sk
     {
         constexpr int BK = 64;
-        constexpr int WAVES = 4;
-        constexpr int THREADS = WAVES * 64;
         constexpr int STAGES = 3;
 
-        template <int TM, int TN>
+        // TM_ x TN_ MFMA tiles of 32 x 32 a wavefront; NW_ wavefronts side by side along N, KH_ such rows of wavefronts
+        // that take turns with the supersteps of a tile
+        template <int TM_, int TN_, int NW_, int KH_>
         struct Tile
         {
+            static constexpr int TM = TM_, TN = TN_, NW = NW_, KH = KH_;
+            static constexpr int WAVES = NW * KH;
+            static constexpr int THREADS = WAVES * 64;
+            static constexpr int STRIP_THREADS = NW * 64; // of one row of wavefronts
+            static constexpr int OWN = TM / KH;           // blocks of 32 rows a wavefront finishes
+            static constexpr int ROUND = OWN >= 2 ? 2 : 1; // ... at a time
+            static constexpr int A_LOADS = TM * 4 / NW;   // activation loads of 8 rows a wavefront and K step
             static constexpr int BM = TM * 32;
-            static constexpr int BN = WAVES * TN * 32; // weight rows per tile (GATE: half gate, half up rows)
+            static constexpr int BN = NW * TN * 32; // weight rows per tile (GATE: half gate, half up rows)
             static constexpr int A_TILE_BYTES = BM * BK * 2;
             // per wavefront 256 bytes: (RMS) the step's 64 gamma values twice over
-            static constexpr int CONST_BYTES = WAVES * 256;
+            static constexpr int CONST_BYTES = NW * 256;
             static constexpr int STAGE_BYTES = A_TILE_BYTES + CONST_BYTES;
-            // the epilogue turns the results through a private piece of the ring per wavefront
-            static constexpr int EPILOGUE_BYTES = WAVES * (TM >= 2 ? 2 : 1) * 32 * (TN * 64 + 16);
+            static constexpr int RING_BYTES = STAGES * STAGE_BYTES; // of one row of wavefronts
+            // the epilogue turns the results through a private piece of the rings per wavefront
+            static constexpr int EPILOGUE_BYTES = WAVES * ROUND * 32 * (TN * 64 + 16);
+            // KH = 2: what a wavefront hands to the one that holds the other half of its sums
+            static constexpr int EXCHANGE_BYTES = KH > 1 ? OWN * TN * 4096 : 0;
             // Weights through LDS (see the kernel): every tile but the largest, whose K step is long enough for the loads
             // it has and which has the least LDS bandwidth to spare (M = 4096, N = K = 8192: 2 % slower that way;
             // M = 1024 on 256 x 128 tiles: 3 % faster; 128-row tiles: 3 - 7 % faster).  Behind the ring: per wavefront
             // and column tile the 32 x 128 bytes of the next superstep
             static constexpr bool W_VIA_LDS = !(TM == 8 && TN >= 2);
-            static constexpr int W_LDS_OFFSET = STAGES * STAGE_BYTES > EPILOGUE_BYTES ? STAGES * STAGE_BYTES : EPILOGUE_BYTES;
+            static constexpr int W_LDS_OFFSET = KH * RING_BYTES > EPILOGUE_BYTES ? KH * RING_BYTES : EPILOGUE_BYTES;
             static constexpr int W_LDS_BYTES = W_VIA_LDS ? WAVES * TN * 4096 : 0;
             static constexpr int LDS_BYTES = W_LDS_OFFSET + W_LDS_BYTES;
+            static_assert(WAVES * EXCHANGE_BYTES <= LDS_BYTES && LDS_BYTES <= 160 * 1024 - 64, "LDS of a CU");
+            static_assert(TM % KH == 0 && OWN % ROUND == 0 && A_LOADS * NW == TM * 4, "whole blocks and loads a wavefront");
             static constexpr size_t SLOT_FLOATS = (size_t)BM * BN;
+        };
+
+        // rows x columns (weight rows) of a tile -> the wavefronts that work on it
+        template <int ROWS, int COLS>
+        struct TileOf;
+        template <>
+        struct TileOf<32, 256> : Tile<1, 2, 4, 1>
+        {
+        };
+        template <>
+        struct TileOf<64, 128> : Tile<2, 1, 4, 2>
+        {
+        };
+        template <>
+        struct TileOf<64, 256> : Tile<2, 1, 8, 1>
+        {
+        };
+        template <>
+        struct TileOf<128, 128> : Tile<4, 1, 4, 2>
+        {
+        };
+        template <>
+        struct TileOf<128, 256> : Tile<4, 1, 8, 1>
+        {
+        };
+        template <>
+        struct TileOf<256, 128> : Tile<8, 1, 4, 1>
+        {
+        };
+        template <>
+        struct TileOf<256, 256> : Tile<8, 2, 4, 1>
+        {
         };
 
         // s_waitcnt with only the vector-memory counter set (gfx9 encoding: vmcnt = bits 3:0 and 15:14)
@@ -167,24 +211,24 @@ namespace nnf
 
         // Which loads a wavefront issues where.  A K step has four quarters of TM x TN MFMAs; step kt is of type
         // T = kt mod 4 (its place in the superstep).
-        //   * The TM activation loads (+ gamma with RMS) for step kt+3 go out in four positions: position 0 in
+        //   * The AL activation loads (+ gamma with RMS) for step kt+3 go out in four positions: position 0 in
         //     quarter 3 of step kt (right behind the barrier that frees the stage), positions 1 .. 3 in quarters
         //     0 .. 2 of step kt+1.
         //   * The NW loads (four of weights, the others scales and zero points) per column tile for the next superstep
         //     go out in quarters 0 .. 2 of step T = w_step(tile), ahead of that quarter's activation loads.
         //     (NW: loads per column tile and superstep, weights and scales)
-        template <int TM, int TN, bool RMS, int NW>
+        template <int AL, int TN, bool RMS, int NW>
         struct Sched
         {
-            static constexpr int a_pos(int i) { return (i * 4) / TM; }
+            static constexpr int a_pos(int i) { return (i * 4) / AL; }
             static constexpr int a_loads_at(int pos)
             {
                 int n = (RMS && pos == 0) ? 1 : 0;
-                for (int i = 0; i < TM; ++i)
+                for (int i = 0; i < AL; ++i)
                     n += a_pos(i) == pos ? 1 : 0;
                 return n;
             }
-            static constexpr int a_loads_total() { return TM + (RMS ? 1 : 0); }
+            static constexpr int a_loads_total() { return AL + (RMS ? 1 : 0); }
             // two tiles in the first step where there are four: everything has been asked for by the end of step 2
             static constexpr int w_step(int j) { return TN <= 3 ? j : (j < 2 ? 0 : j - 1); }
             static constexpr int w_loads_in_step(int T)
@@ -219,7 +263,7 @@ namespace nnf
             static constexpr int later(int T)
             {
                 const int Tp = (T + 3) & 3;
-                const int lp = a_pos(TM - 1); // 0: the last one went out in quarter 3 of step kt-2, p: in quarter p-1 of step kt-1
+                const int lp = a_pos(AL - 1); // 0: the last one went out in quarter 3 of step kt-2, p: in quarter p-1 of step kt-1
                 int n = 0;
                 for (int Q = lp; Q < 3; ++Q)
                     n += loads_at(Tp, Q);
@@ -297,22 +341,25 @@ namespace nnf
     // (8 columns) per lane: bias, residual, store.  Rounding as the unfused graph would: the GEMM result to fp16 first,
     // then the element-wise operation in fp32, then fp16 again.
     // bytes of LDS sk_finish_round uses per wavefront
-    template <int TM, int TN, bool GATE>
+    template <int ROUND_TM, int TN, bool GATE>
     constexpr int sk_region_bytes()
     {
-        return (TM >= 2 ? 2 : 1) * 32 * ((GATE ? TN / 2 : TN) * 64 + 16);
+        return ROUND_TM * 32 * ((GATE ? TN * 32 : TN * 64) + 16);
     }
 
-    template <int TM, int TN, bool GATE, bool BIAS, bool RESID, bool RMS>
-    __device__ __forceinline__ void sk_finish_round(const SkGemmParams& p, const floatx16 (&c)[TM >= 2 ? 2 : 1][TN], int r, int m0, int n0,
+    template <int ROUND_TM, int TN, bool GATE, bool BIAS, bool RESID, bool RMS>
+    __device__ __forceinline__ void sk_finish_round(const SkGemmParams& p, const floatx16 (&c)[ROUND_TM][TN], int r, int m0, int n0,
                                                     uint8_t* region, int wave, int lane)
     {
-        constexpr int OUT_TN = GATE ? TN / 2 : TN;
-        constexpr int ROUND_TM = TM >= 2 ? 2 : 1;
-        constexpr int PITCH = OUT_TN * 64 + 16; // bytes per staged row (padding spreads the banks)
-        constexpr int LANES_PER_ROW = OUT_TN * 4, ROWS_PER_READ = 64 / LANES_PER_ROW;
+        constexpr int OUT_COLS = GATE ? TN * 16 : TN * 32; // of the wavefront's strip
+        constexpr int PITCH = OUT_COLS * 2 + 16; // bytes per staged row (padding spreads the banks)
+        constexpr int LANES_PER_ROW = OUT_COLS / 8, ROWS_PER_READ = 64 / LANES_PER_ROW;
+        // a gate value's element and its up value's: in the same place of the column tile TN / 2 further, or (one column
+        // tile, 16 gate and 16 up rows) eight elements further
+        constexpr int OUT_TN = GATE ? (TN + 1) / 2 : TN, OUT_GROUPS = GATE && TN == 1 ? 2 : 4;
+        constexpr int UP_J = GATE ? TN / 2 : 0, UP_E = GATE && TN == 1 ? 8 : 0;
         const int l32 = lane & 31, h = lane >> 5;
-        const int n_wave = n0 + wave * (OUT_TN * 32);
+        const int n_wave = n0 + wave * OUT_COLS;
         const int piece = lane % LANES_PER_ROW;
         const int n_lane = n_wave + piece * 8; // first of this lane's 8 columns in the row phase
         bool vec = ((p.N & 7) == 0) && ((p.ldy & 7) == 0) && ((reinterpret_cast<uintptr_t>(p.Y) & 15) == 0);
@@ -335,7 +382,7 @@ namespace nnf
 #pragma unroll
             for (int j = 0; j < OUT_TN; ++j)
 #pragma unroll
-                for (int g = 0; g < 4; ++g)
+                for (int g = 0; g < OUT_GROUPS; ++g)
                 {
                     half4_t y;
 #pragma unroll
@@ -344,8 +391,7 @@ namespace nnf
                         if (GATE)
                         {
                             const float gt = (float)(half_t)(RMS ? c[ii][j][4 * g + k] * rs : c[ii][j][4 * g + k]);
-                            const float up =
-                                (float)(half_t)(RMS ? c[ii][j + TN / 2][4 * g + k] * rs : c[ii][j + TN / 2][4 * g + k]);
+                            const float up = (float)(half_t)(RMS ? c[ii][j + UP_J][UP_E + 4 * g + k] * rs : c[ii][j + UP_J][UP_E + 4 * g + k]);
                             y[k] = (half_t)(gt * (1.0f / (1.0f + __expf(-gt))) * up);
                         }
                         else
@@ -404,26 +450,27 @@ namespace nnf
     };
     // Parts of a block kept in flight at once (16 TN registers each).  SAME_LAUNCH: inside the GEMM kernel, with its
     // accumulation registers still set aside, and (sk_loads_ahead) two blocks' worth of them in flight.
-    template <int TM, int TN>
+    template <class T>
     constexpr bool sk_loads_ahead()
     {
-        return TM * TN <= 8;
+        return T::TM * T::TN <= 8;
     }
-    template <int TM, int TN, bool SAME_LAUNCH>
+    template <class T, bool SAME_LAUNCH>
     struct SkPartsInFlight
     {
-        static constexpr int D = !SAME_LAUNCH ? 8 : (sk_loads_ahead<TM, TN>() && TN >= 2) ? 3 : 4;
-        floatx4 v[D][TN][4]; // [part][column tile][quarter of its 16 elements]
+        static constexpr int D = !SAME_LAUNCH ? 8 : (sk_loads_ahead<T>() && T::TN >= 2) ? 3 : 4;
+        floatx4 v[D][T::TN][4]; // [part][column tile][quarter of its 16 elements]
     };
     // Asks for parts sg0 .. sg0 + D - 1 (clamped to the last) of block `r` (32 rows) of strip `wave` of a shared tile.
     // SAME_LAUNCH: the parts were parked by other workgroups of the launch that is still running (device-scope loads).
-    template <int TM, int TN, bool SAME_LAUNCH>
-    __device__ __forceinline__ void sk_request_parts(SkPartsInFlight<TM, TN, SAME_LAUNCH>& x, const SkGemmParams& p,
+    // tid: of the threads of a row of wavefronts
+    template <class T, bool SAME_LAUNCH>
+    __device__ __forceinline__ void sk_request_parts(SkPartsInFlight<T, SAME_LAUNCH>& x, const SkGemmParams& p,
                                                      int gemm_grid, const SkSharedTile& t, int r, int sg0, int tid)
     {
         using namespace gemm_sk;
-        using T = Tile<TM, TN>;
-        constexpr int D = SkPartsInFlight<TM, TN, SAME_LAUNCH>::D;
+        constexpr int TN = T::TN;
+        constexpr int D = SkPartsInFlight<T, SAME_LAUNCH>::D;
         buffer_t parked;
         if constexpr (SAME_LAUNCH)
             parked = parked_buffer(p.partial, p.partial_bytes);
@@ -438,7 +485,7 @@ namespace nnf
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                 {
-                    const size_t at = first_float + (size_t)(((r * TN + j) * 4 + q) * THREADS * 4);
+                    const size_t at = first_float + (size_t)(((r * TN + j) * 4 + q) * T::STRIP_THREADS * 4);
                     if constexpr (SAME_LAUNCH)
                         x.v[d][j][q] = load_device_scope(parked, (uint32_t)(at * sizeof(float)));
                     else
@@ -450,14 +497,14 @@ namespace nnf
     // `gemm_grid` worked on: adds their parked parts in K order -- the first ones have been asked for into `x` -- and
     // finishes the block (epilogue, stores).  Used by the second launch and, with SkGemmParams::sync, by the GEMM's own
     // workgroups: same order, same bits.
-    template <int TM, int TN, bool GATE, bool BIAS, bool RESID, bool RMS, bool SAME_LAUNCH>
-    __device__ __forceinline__ void sk_finish_block(SkPartsInFlight<TM, TN, SAME_LAUNCH>& x, const SkGemmParams& p,
+    template <class T, bool GATE, bool BIAS, bool RESID, bool RMS, bool SAME_LAUNCH>
+    __device__ __forceinline__ void sk_finish_block(SkPartsInFlight<T, SAME_LAUNCH>& x, const SkGemmParams& p,
                                                     int gemm_grid, const SkSharedTile& t, int r, uint8_t* stage, int wave, int lane)
     {
         using namespace gemm_sk;
-        using T = Tile<TM, TN>;
+        constexpr int TN = T::TN;
         constexpr int BN_OUT = GATE ? T::BN / 2 : T::BN;
-        constexpr int D = SkPartsInFlight<TM, TN, SAME_LAUNCH>::D;
+        constexpr int D = SkPartsInFlight<T, SAME_LAUNCH>::D;
         int tm, tn;
         {
             constexpr int GM = 4;
@@ -479,7 +526,7 @@ namespace nnf
         for (int sg0 = 0; sg0 < t.n_seg; sg0 += D)
         {
             if (sg0 > 0)
-                sk_request_parts<TM, TN, SAME_LAUNCH>(x, p, gemm_grid, t, r, sg0, wave * 64 + lane);
+                sk_request_parts<T, SAME_LAUNCH>(x, p, gemm_grid, t, r, sg0, wave * 64 + lane);
 #pragma unroll
             for (int d = 0; d < D; ++d)
                 if (sg0 + d < t.n_seg)
@@ -499,34 +546,43 @@ namespace nnf
         sk_finish_round<1, TN, GATE, BIAS, RESID, RMS>(p, c, r, m0, n0, stage, wave, lane);
     }
 
-    // rstd[m] = rsqrt(mean_k(A[m, k]^2) + eps) for rows first, first + step, ... < end by the 256 threads of a workgroup
+    // rstd[m] = rsqrt(mean_k(A[m, k]^2) + eps) for rows first, first + step, ... < end, a row by 256 threads of a workgroup
     // (the summation order of the pre-pass kernel, rms_rstd_kernel: same bits), stored at device scope; complete for
-    // every thread of the workgroup on return.  part: four floats of LDS.
+    // every thread of the workgroup on return.  part: a float of LDS per wavefront.
+    template <int THREADS>
     __device__ __forceinline__ void sk_rstd_rows(const SkGemmParams& p, int first, int end, int step, float* part, int tid)
     {
+        constexpr int ROWS = THREADS / 256; // at a time
         const int units = p.K >> 3;
-        for (int m = first; m < end; m += step)
+        for (int m0 = first; m0 < end; m0 += ROWS * step)
         {
-            const uintx4* row = reinterpret_cast<const uintx4*>(p.A + (size_t)m * p.K);
-            float ss = 0.f;
-            for (int i = tid; i < units; i += gemm_sk::THREADS)
+            const int m = m0 + (tid >> 8) * step;
+            if (m < end)
             {
-                const uintx4 v = row[i];
-                const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
+                const uintx4* row = reinterpret_cast<const uintx4*>(p.A + (size_t)m * p.K);
+                float ss = 0.f;
+                for (int i = tid & 255; i < units; i += 256)
                 {
-                    const half2_t hh = as_half2(vv[j]);
-                    ss += (float)hh.x * (float)hh.x + (float)hh.y * (float)hh.y;
+                    const uintx4 v = row[i];
+                    const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                    {
+                        const half2_t hh = as_half2(vv[j]);
+                        ss += (float)hh.x * (float)hh.x + (float)hh.y * (float)hh.y;
+                    }
                 }
+                ss = wave_sum(ss);
+                if ((tid & 63) == 0)
+                    part[tid >> 6] = ss;
             }
-            ss = wave_sum(ss);
-            if ((tid & 63) == 0)
-                part[tid >> 6] = ss;
             __syncthreads();
-            if (tid == 0)
-                __hip_atomic_store(p.rstd_out + m, 1.0f / __builtin_sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)p.K + p.rms_eps),
+            if ((tid & 255) == 0 && m < end)
+            {
+                const float* four = part + (tid >> 6);
+                __hip_atomic_store(p.rstd_out + m, 1.0f / __builtin_sqrtf(((four[0] + four[1]) + (four[2] + four[3])) / (float)p.K + p.rms_eps),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
             __syncthreads();
         }
         gemm_sk::wait_vector_memory();
@@ -567,8 +623,8 @@ namespace nnf
     // tile and superstep it fetches the 256 / group scales of its row in one load (4, 8 or 16 bytes) and the byte(s) that
     // hold their zero points in another (1, 2 or 4 bytes; without p.zps: the scales again, unused) -- six loads per
     // column tile as for QG = 0, on the same schedule -- and keeps a scale and the pair -(1024 + z), -(64 + z) per K step.
-    template <int TM, int TN, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0>
-    __global__ __launch_bounds__(256, 1) void w4a16_gemm_sk_kernel(const half_t* __restrict__ A_first,
+    template <int TM, int TN, int NW, int KH, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0>
+    __global__ __launch_bounds__(NW * KH * 64, 1) void w4a16_gemm_sk_kernel(const half_t* __restrict__ A_first,
                                                                    const uint8_t* __restrict__ Wq_first,
                                                                    const half_t* __restrict__ S_first, long long units_first,
                                                                    int M_first, int N_first, int K_first, int tiles_n_first,
@@ -588,14 +644,14 @@ namespace nnf
         p.tiles_n = tiles_n_first;
         p.supersteps = supersteps_first;
         using namespace gemm_sk;
-        using T = Tile<TM, TN>;
+        using T = Tile<TM, TN, NW, KH>;
         // loads per column tile and superstep: four of weights; two of scales and zero points, or (the specialised kernel)
         // three of scales, see load_w
-        constexpr int NW = QG != 0 ? 6 : 7;
-        using SCH = Sched<TM, TN, RMS, NW>;
+        constexpr int WL = QG != 0 ? 6 : 7;
+        constexpr int AL = T::A_LOADS;
+        using SCH = Sched<AL, TN, RMS, WL>;
         static_assert(!(GATE && (BIAS || RESID)), "SiLU-gate is not combined with bias or residual");
         static_assert(TN == 1 || TN == 2 || TN == 4, "column tiles per wavefront");
-        static_assert(!GATE || TN >= 2, "gate and up rows are the two halves of a wavefront's column tiles");
         static_assert(QG == 0 || (QG >= 5 && QG <= 7), "groups of 32, 64 or 128");
         constexpr bool QZ = QG != 0;
         constexpr int GSH = QZ ? QG : 7;                    // log2 of the group size
@@ -619,12 +675,15 @@ namespace nnf
         const int lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int l32 = lane & 31, h = lane >> 5;
+        // this wavefront's strip of columns; which of the KH rows of wavefronts it belongs to
+        const int strip = KH > 1 ? wave % NW : wave, kh = KH > 1 ? wave / NW : 0;
         const int K = p.K;
         const int G = K >> GSH;
         const bool g_even = !(G & 1);
         const int SS = p.supersteps;
         const int grid = grid_first; // = gridDim.x
         const uint32_t lds0 = lds_address(smem);
+        const uint32_t ring0 = (uint32_t)(kh * T::RING_BYTES); // the ring of this row of wavefronts
 
         // workgroup ids are dealt round-robin to the 8 XCDs: number the workgroups so that an XCD (own L2) holds a
         // contiguous run of them, i.e. of units, i.e. of tiles
@@ -641,7 +700,7 @@ namespace nnf
 
         // ---- (rstd_out) RMSNorm's rstd[] inside this launch: this workgroup's rows now, counted in once they are
         // visible to every CU; an epilogue looks at the count before it reads rstd[] (ensure_rstd) ------------------
-        __shared__ float rstd_part[4];
+        __shared__ float rstd_part[T::WAVES];
         __shared__ uint32_t rstd_note;
         bool rstd_ok = true; // (uniform) rstd[] is known to be complete
         if constexpr (RMS)
@@ -649,7 +708,7 @@ namespace nnf
             if (p.rstd_out)
             {
                 rstd_ok = false;
-                sk_rstd_rows(p, v, p.M, grid, rstd_part, tid);
+                sk_rstd_rows<T::THREADS>(p, v, p.M, grid, rstd_part, tid);
                 if (tid == 0)
                     atomicAdd(p.rstd_sync, 1u);
             }
@@ -677,7 +736,7 @@ namespace nnf
                 rstd_ok = rstd_note != 0u;
                 __syncthreads();
                 if (!rstd_ok)
-                    sk_rstd_rows(p, m_first, min(m_end, p.M), 1, rstd_part, tid);
+                    sk_rstd_rows<T::THREADS>(p, m_first, min(m_end, p.M), 1, rstd_part, tid);
             }
         };
 
@@ -688,12 +747,12 @@ namespace nnf
         uint32_t a_rd[4]; // quarter s: piece (4h + s) ^ swizzle of row l32
 #pragma unroll
         for (int s = 0; s < 4; ++s)
-            a_rd[s] = lds0 + (uint32_t)(l32 * 128 + ((((h << 2) + s) ^ ((l32 >> 1) & 7)) << 4));
+            a_rd[s] = lds0 + ring0 + (uint32_t)(l32 * 128 + ((((h << 2) + s) ^ ((l32 >> 1) & 7)) << 4));
         // gamma of quarter s: the 8 values at k = 32h + 8s of the wavefront's private copy
-        const uint32_t g_rd = lds0 + (uint32_t)(A_TILE_BYTES + wave * 256 + h * 64);
+        const uint32_t g_rd = lds0 + ring0 + (uint32_t)(A_TILE_BYTES + strip * 256 + h * 64);
         // LDS destinations of this wavefront's loads within a stage
-        const uint32_t lds_a = (uint32_t)(wave * TM * 1024);
-        const uint32_t lds_g = (uint32_t)(A_TILE_BYTES + wave * 256);
+        const uint32_t lds_a = ring0 + (uint32_t)(strip * AL * 1024);
+        const uint32_t lds_g = ring0 + (uint32_t)(A_TILE_BYTES + strip * 256);
         // the wavefront's weights of the next superstep; a lane's piece for K step x: piece 2 x + h of row l32
         const uint32_t lds_w = (uint32_t)(T::W_LDS_OFFSET + wave * TN * 4096);
         uint32_t w_rd[4];
@@ -733,16 +792,21 @@ namespace nnf
             const int k_begin = ss_begin * 256;
             const int KT = 4 * NSS;                             // K steps of this segment (the last two may lie past K)
             const int kt_max = min(KT, (K - k_begin) >> 6) - 1; // last K step inside K
+            // The rows of wavefronts take turns with the supersteps of the segment: a wavefront's superstep s is the
+            // segment's KH s + kh, its K step kt likewise (clamped to the last ones inside the segment)
+            const int my_ss = KH > 1 ? (NSS - kh + KH - 1) / KH : NSS;
+            auto segment_ss = [&](int s) { return min(KH * s + kh, NSS - 1); };
+            auto segment_kt = [&](int kt) { return min(KH > 1 ? 4 * (KH * (kt >> 2) + kh) + (kt & 3) : kt, kt_max); };
 
             // ---- activations: direct-load map ------------------------------------------------------------------
             // chunk c fills LDS rows c*8 .. +7; lane l lands at (row = c*8 + l/8, slot = l%8) and therefore
-            // fetches piece  slot ^ ((row >> 1) & 7)  of that row.  Wavefront w fetches chunks w*TM .. +TM-1.
+            // fetches piece  slot ^ ((row >> 1) & 7)  of that row.  Strip w fetches chunks w*AL .. +AL-1.
             // (byte offsets from the operand's base: the matrices are below 4 GiB, checked by the launcher)
-            uint32_t a_off[TM];
+            uint32_t a_off[AL];
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < AL; ++i)
             {
-                const int row = (wave * TM + i) * 8 + (lane >> 3);
+                const int row = (strip * AL + i) * 8 + (lane >> 3);
                 const int piece = (lane & 7) ^ ((row >> 1) & 7);
                 a_off[i] = (uint32_t)(((size_t)min(m0 + row, p.M - 1) * K + k_begin + piece * 8) * 2);
             }
@@ -751,8 +815,8 @@ namespace nnf
             const uint32_t g_off = (uint32_t)(lane & 31) * 4u;
             // scalar base of K step kt (clamped to the last inside K: past it a valid tile goes to a free stage, or is
             // multiplied by weights of zero)
-            auto a_base_of = [&](int kt) { return scalar_base(a_bytes + (size_t)min(kt, kt_max) * (BK * 2)); };
-            auto g_base_of = [&](int kt) { return scalar_base(g_bytes + (size_t)min(kt, kt_max) * (BK * 2)); };
+            auto a_base_of = [&](int kt) { return scalar_base(a_bytes + (size_t)segment_kt(kt) * (BK * 2)); };
+            auto g_base_of = [&](int kt) { return scalar_base(g_bytes + (size_t)segment_kt(kt) * (BK * 2)); };
             // activation load i of a K step -> stage
             auto load_a = [&](auto i_c, const uint8_t* a_base, uint32_t stage_off) {
                 constexpr int i = decltype(i_c)::value;
@@ -773,10 +837,12 @@ namespace nnf
             // when the superstep begins.
             // the row of the wavefront's column tile j that sits at place r (0 .. 31)
             auto weight_row = [&](int j, int r) {
+                if (GATE && TN == 1) // rows 0 .. 15: gate rows, the others: the up rows that pair with them
+                    return min((r >= 16 ? p.up_row_offset - 16 : 0) + n0 + strip * 16 + r, p.up_row_offset + p.N - 1);
                 if (GATE) // column tiles 0 .. TN/2-1: gate rows, the others: the up rows that pair with them
-                    return min((j >= TN / 2 ? p.up_row_offset + n0 + (j - TN / 2) * 32 : n0 + j * 32) + wave * (TN / 2) * 32 + r,
+                    return min((j >= TN / 2 ? p.up_row_offset + n0 + (j - TN / 2) * 32 : n0 + j * 32) + strip * (TN / 2) * 32 + r,
                                p.up_row_offset + p.N - 1);
-                return min(n0 + wave * (TN * 32) + j * 32 + r, p.N - 1);
+                return min(n0 + strip * (TN * 32) + j * 32 + r, p.N - 1);
             };
             constexpr bool W_LDS = T::W_VIA_LDS;
             constexpr int WSETS = W_LDS ? 1 : 2; // register sets of weights: without the detour the next superstep's as well
@@ -823,7 +889,7 @@ namespace nnf
                 uint32_t repeat; // 64: the second 64 bytes of the superstep do not exist
             };
             auto w_base_of = [&](int s) {
-                s = min(s, NSS - 1);
+                s = segment_ss(s);
                 WBase b;
                 if constexpr (QZ)
                 {
@@ -924,7 +990,7 @@ namespace nnf
                         }
                     return;
                 }
-                s = min(s, NSS - 1);
+                s = segment_ss(s);
                 const bool second_valid = 2 * (ss_begin + s) + 1 < G;
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
@@ -1114,7 +1180,7 @@ namespace nnf
                             {
                                 // the (L - N_W)-th activation load of this position
                                 constexpr int POS = Q == 3 ? 0 : Q + 1;
-                                constexpr int FIRST = (POS * TM + 3) / 4; // smallest i with a_pos(i) == POS
+                                constexpr int FIRST = (POS * AL + 3) / 4; // smallest i with a_pos(i) == POS
                                 static_assert(SCH::a_pos(FIRST + L - N_W) == POS, "activation loads of a position are consecutive");
                                 load_a(std::integral_constant<int, FIRST + L - N_W>{}, Q == 3 ? a_next : a_late, Q == 3 ? stage_off : prev_off);
                             }
@@ -1142,14 +1208,14 @@ namespace nnf
                 // steps 0 and 1 and superstep 0 in full, of step 2 what quarter 3 of a step before the first would
                 // have asked for
                 const WBase w0 = w_base_of(0);
-                unroll_for<0, TM>([&](auto i_c) { load_a(i_c, a_base_of(0), 0u); });
-                unroll_for<0, TN>([&](auto j_c) { unroll_for<0, NW>([&](auto x_c) { load_w(I0{}, j_c, x_c, w0); }); });
+                unroll_for<0, AL>([&](auto i_c) { load_a(i_c, a_base_of(0), 0u); });
+                unroll_for<0, TN>([&](auto j_c) { unroll_for<0, WL>([&](auto x_c) { load_w(I0{}, j_c, x_c, w0); }); });
                 if constexpr (RMS)
                     load_gamma(g_base_of(0), 0u);
-                unroll_for<0, TM>([&](auto i_c) { load_a(i_c, a_base_of(1), (uint32_t)STAGE_BYTES); });
+                unroll_for<0, AL>([&](auto i_c) { load_a(i_c, a_base_of(1), (uint32_t)STAGE_BYTES); });
                 if constexpr (RMS)
                     load_gamma(g_base_of(1), (uint32_t)STAGE_BYTES);
-                unroll_for<0, TM>([&](auto i_c) {
+                unroll_for<0, AL>([&](auto i_c) {
                     if constexpr (SCH::a_pos(decltype(i_c)::value) == 0)
                         load_a(i_c, a_base_of(2), (uint32_t)(2 * STAGE_BYTES));
                 });
@@ -1197,13 +1263,13 @@ namespace nnf
             __builtin_amdgcn_sched_barrier(0);
             // No LDS read other than the fragments of quarter 0 is in flight at the top of a K step.
             {
-                constexpr uint32_t RING = (uint32_t)(STAGES * STAGE_BYTES);
+                constexpr uint32_t RING = (uint32_t)T::RING_BYTES;
                 auto next_of = [](uint32_t o) { return o + STAGE_BYTES == RING ? 0u : o + (uint32_t)STAGE_BYTES; };
                 uint32_t pv = RING - (uint32_t)STAGE_BYTES, st = 0;
                 // one loop body: the superstep works on register set 0 and fills set 1, which moves to set 0 at its end
                 // (a few dozen register moves per 256 MFMAs; two bodies that swap the roles of the sets instead measured the
                 // same at every M, and spilled registers under the 256 x 256 tile)
-                for (int s = 0; s < NSS; ++s)
+                for (int s = 0; s < my_ss; ++s)
                 {
                     k_step(I0{}, s, pv, st, next_of(st));
                     pv = st, st = next_of(st);
@@ -1236,30 +1302,76 @@ namespace nnf
                     }
                 }
             }
+            if constexpr (KH > 1)
+            {
+                // an odd number of supersteps: the barriers of the last one, which only the other wavefronts have
+                if (my_ss < (NSS + KH - 1) / KH)
+                    for (int i = 0; i < 4; ++i)
+                        workgroup_barrier();
+            }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the fragments read ahead for a step that does not exist
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));          // nothing may land in LDS or in registers any more ...
             __syncthreads();                                   // ... from any wavefront: the ring is free
+            // ---- KH = 2: the two wavefronts of a strip trade sums through LDS: each finishes OWN blocks of 32 rows, the
+            // first the first ones (acc[0 .. OWN - 1] from here on: the blocks kh OWN ...)
+            if constexpr (KH > 1)
+            {
+                static_assert(KH <= 2, "two rows of wavefronts at most");
+                floatx4* mine = reinterpret_cast<floatx4*>(smem + wave * T::EXCHANGE_BYTES) + lane;
+                const floatx4* theirs = reinterpret_cast<const floatx4*>(smem + (wave ^ NW) * T::EXCHANGE_BYTES) + lane;
+#pragma unroll
+                for (int i = 0; i < T::OWN; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                        {
+                            floatx4 x;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                            {
+                                const float lower = acc[i][j][4 * q + e], upper = acc[T::OWN + i][j][4 * q + e];
+                                x[e] = kh ? lower : upper;
+                                acc[i][j][4 * q + e] = kh ? upper : lower;
+                            }
+                            mine[((i * TN + j) * 4 + q) * 64] = x;
+                        }
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < T::OWN; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                        {
+                            const floatx4 x = theirs[((i * TN + j) * 4 + q) * 64];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                acc[i][j][4 * q + e] += x[e];
+                        }
+                __syncthreads(); // the epilogue's staging regions are free
+            }
             if (u >= u_end)
                 NNF_SK_STAMP(2); // the K loop of the last segment is over
             else if (first_of_mine)
                 NNF_SK_STAMP(10); // ... of the first segment, when it is not the last
 
             // ---- a tile shared with other workgroups: park the sums in register order (element block q of MFMA tile
-            // (i, j) of all 256 threads is one contiguous 4 KiB); w4a16_gemm_sk_fixup_kernel adds the parts and finishes
+            // (i, j) of all threads of a row of wavefronts is contiguous); w4a16_gemm_sk_fixup_kernel adds the parts and finishes
             if (!whole)
             {
-                const size_t first_float = ((size_t)v + (first_of_mine ? 0 : (size_t)grid)) * T::SLOT_FLOATS + (size_t)tid * 4;
+                const size_t first_float = ((size_t)v + (first_of_mine ? 0 : (size_t)grid)) * T::SLOT_FLOATS + (size_t)(strip * 64 + lane) * 4;
                 float* mine = p.partial + first_float;
                 const bool same_launch = p.sync != nullptr;
                 const buffer_t parked = parked_buffer(p.partial, p.partial_bytes);
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+                for (int i = 0; i < T::OWN; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
 #pragma unroll
                         for (int q = 0; q < 4; ++q)
                         {
-                            const size_t at = (size_t)(((i * TN + j) * 4 + q) * THREADS * 4);
+                            const size_t at = (size_t)((((kh * T::OWN + i) * TN + j) * 4 + q) * T::STRIP_THREADS * 4);
                             const floatx4 part = floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
                             if (same_launch)
                                 store_device_scope(parked, (uint32_t)((first_float + at) * sizeof(float)), part);
@@ -1290,10 +1402,10 @@ namespace nnf
             else
             {
                 // ---- epilogue: two blocks of 32 rows at a time ------------------------------------------------------
-                constexpr int ROUND_TM = TM >= 2 ? 2 : 1;
+                constexpr int ROUND_TM = T::ROUND;
                 ensure_rstd(m0, m0 + BM);
 #pragma unroll
-                for (int r = 0; r < TM / ROUND_TM; ++r)
+                for (int r = 0; r < T::OWN / ROUND_TM; ++r)
                 {
                     floatx16 c[ROUND_TM][TN];
 #pragma unroll
@@ -1301,7 +1413,8 @@ namespace nnf
 #pragma unroll
                         for (int j = 0; j < TN; ++j)
                             c[ii][j] = acc[r * ROUND_TM + ii][j];
-                    sk_finish_round<TM, TN, GATE, BIAS, RESID, RMS>(p, c, r, m0, n0, smem + wave * sk_region_bytes<TM, TN, GATE>(), wave, lane);
+                    sk_finish_round<ROUND_TM, TN, GATE, BIAS, RESID, RMS>(p, c, kh * (T::OWN / ROUND_TM) + r, m0, n0,
+                                                                          smem + wave * sk_region_bytes<ROUND_TM, TN, GATE>(), strip, lane);
                     __builtin_amdgcn_sched_barrier(0); // (one round at a time: few registers)
                 }
             }
@@ -1359,8 +1472,17 @@ namespace nnf
             // device scope, and so are the parts)
             // The blocks to finish, those of the first tile in bits 0 .. 7, of the second in bits 8 .. 15, one after the
             // other; where the registers allow it the parts of the next block are asked for ahead of this block's sums.
-            constexpr bool AHEAD = sk_loads_ahead<TM, TN>();
+            constexpr bool AHEAD = sk_loads_ahead<T>();
             uint32_t todo = blocks[0] | (blocks[1] << 8);
+            if constexpr (KH > 1)
+            {
+                // each row of wavefronts takes every second one
+                uint32_t rest = todo;
+                for (int n = 0; rest; ++n, rest &= rest - 1)
+                    if ((n & 1) != kh)
+                        todo &= ~(rest & -rest);
+            }
+            const int strip_tid = strip * 64 + lane;
             // (selected field by field: an array indexed at run time would live in private memory)
             auto tile_of = [&](int task) {
                 const bool second = task >= 8;
@@ -1373,35 +1495,35 @@ namespace nnf
             };
             if constexpr (AHEAD)
             {
-                SkPartsInFlight<TM, TN, true> x0, x1;
+                SkPartsInFlight<T, true> x0, x1;
                 int cur = todo ? __builtin_ctz(todo) : -1;
                 if (cur >= 0)
-                    sk_request_parts<TM, TN, true>(x0, p, grid, tile_of(cur), cur & 7, 0, tid);
+                    sk_request_parts<T, true>(x0, p, grid, tile_of(cur), cur & 7, 0, strip_tid);
                 while (cur >= 0)
                 {
                     todo &= todo - 1;
                     int nxt = todo ? __builtin_ctz(todo) : -1;
                     if (nxt >= 0)
-                        sk_request_parts<TM, TN, true>(x1, p, grid, tile_of(nxt), nxt & 7, 0, tid);
-                    sk_finish_block<TM, TN, GATE, BIAS, RESID, RMS, true>(x0, p, grid, tile_of(cur), cur & 7, stage, wave, lane);
+                        sk_request_parts<T, true>(x1, p, grid, tile_of(nxt), nxt & 7, 0, strip_tid);
+                    sk_finish_block<T, GATE, BIAS, RESID, RMS, true>(x0, p, grid, tile_of(cur), cur & 7, stage, strip, lane);
                     if (nxt < 0)
                         break;
                     todo &= todo - 1;
                     cur = todo ? __builtin_ctz(todo) : -1;
                     if (cur >= 0)
-                        sk_request_parts<TM, TN, true>(x0, p, grid, tile_of(cur), cur & 7, 0, tid);
-                    sk_finish_block<TM, TN, GATE, BIAS, RESID, RMS, true>(x1, p, grid, tile_of(nxt), nxt & 7, stage, wave, lane);
+                        sk_request_parts<T, true>(x0, p, grid, tile_of(cur), cur & 7, 0, strip_tid);
+                    sk_finish_block<T, GATE, BIAS, RESID, RMS, true>(x1, p, grid, tile_of(nxt), nxt & 7, stage, strip, lane);
                 }
             }
             else
             {
-                SkPartsInFlight<TM, TN, true> x;
+                SkPartsInFlight<T, true> x;
                 while (todo)
                 {
                     const int cur = __builtin_ctz(todo);
                     todo &= todo - 1;
-                    sk_request_parts<TM, TN, true>(x, p, grid, tile_of(cur), cur & 7, 0, tid);
-                    sk_finish_block<TM, TN, GATE, BIAS, RESID, RMS, true>(x, p, grid, tile_of(cur), cur & 7, stage, wave, lane);
+                    sk_request_parts<T, true>(x, p, grid, tile_of(cur), cur & 7, 0, strip_tid);
+                    sk_finish_block<T, GATE, BIAS, RESID, RMS, true>(x, p, grid, tile_of(cur), cur & 7, stage, strip, lane);
                 }
             }
             __syncthreads(); // every wavefront's strips are finished
@@ -1436,10 +1558,10 @@ namespace nnf
     }
 
     // launches w4a16_gemm_sk_kernel<...> on `grid` workgroups
-    template <class Kernel>
-    inline void launch_sk_kernel(Kernel kernel, int grid, size_t lds_bytes, hipStream_t stream, const SkGemmParams& p)
+    template <class T, class Kernel>
+    inline void launch_sk_kernel(Kernel kernel, int grid, hipStream_t stream, const SkGemmParams& p)
     {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(gemm_sk::THREADS), lds_bytes, stream, p.A, p.Wq, p.S, p.units, p.M, p.N, p.K,
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(T::THREADS), T::LDS_BYTES, stream, p.A, p.Wq, p.S, p.units, p.M, p.N, p.K,
                            p.tiles_n, p.supersteps, grid, p);
     }
 
@@ -1448,15 +1570,15 @@ namespace nnf
     // another here: one workgroup of a single wavefront per tile, block of 32 rows and strip (a few dozen tiles
     // then still spread over all CUs); one whose tile had a single owner has nothing to do.  `gemm_grid`: workgroups of
     // the GEMM launch.
-    template <int TM, int TN, bool GATE, bool BIAS, bool RESID, bool RMS>
+    template <class T, bool GATE, bool BIAS, bool RESID, bool RMS>
     __global__ __launch_bounds__(64) void w4a16_gemm_sk_fixup_kernel(SkGemmParams p, int gemm_grid)
     {
         using namespace gemm_sk;
-        constexpr int ROUND_TM = 1, ROUNDS = TM; // (the epilogue routine of a tile one block high)
-        __shared__ __attribute__((aligned(16))) uint8_t stage[ROUND_TM * 32 * (TN * 64 + 16)];
+        constexpr int ROUNDS = T::TM; // (the epilogue routine of a tile one block high)
+        __shared__ __attribute__((aligned(16))) uint8_t stage[sk_region_bytes<1, T::TN, GATE>()];
         const int lane = threadIdx.x;
-        const int wave = (int)blockIdx.x % WAVES; // the strip: what wavefront `wave` of the GEMM's workgroup parked
-        const int tile = (int)blockIdx.x / (WAVES * ROUNDS), r = ((int)blockIdx.x / WAVES) % ROUNDS;
+        const int wave = (int)blockIdx.x % T::NW; // the strip
+        const int tile = (int)blockIdx.x / (T::NW * ROUNDS), r = ((int)blockIdx.x / T::NW) % ROUNDS;
         const int SS = p.supersteps;
         const long long t0 = (long long)tile * SS;
         const int v_first = owner_of_unit(t0, p.units, gemm_grid);
@@ -1467,8 +1589,8 @@ namespace nnf
         const bool first_is_second_slot = first_unit_of(v_first, p.units, gemm_grid) < t0;
         SkSharedTile t;
         t.tile = tile, t.v_first = v_first, t.n_seg = n_seg, t.first_is_second_slot = first_is_second_slot;
-        SkPartsInFlight<TM, TN, false> x;
-        sk_request_parts<TM, TN, false>(x, p, gemm_grid, t, r, 0, wave * 64 + lane);
-        sk_finish_block<TM, TN, GATE, BIAS, RESID, RMS, false>(x, p, gemm_grid, t, r, stage, wave, lane);
+        SkPartsInFlight<T, false> x;
+        sk_request_parts<T, false>(x, p, gemm_grid, t, r, 0, wave * 64 + lane);
+        sk_finish_block<T, GATE, BIAS, RESID, RMS, false>(x, p, gemm_grid, t, r, stage, wave, lane);
     }
 } // namespace nnf

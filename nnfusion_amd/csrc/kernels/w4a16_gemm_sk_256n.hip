@@ -5,6 +5,6 @@ namespace nnf
 {
     hipError_t launch_gemm_sk_256_narrow(hipStream_t stream, const SkGemmParams& p, int grid)
     {
-        return gemm_sk::launch_tile_height_plain<8, 1>(stream, p, grid);
+        return gemm_sk::launch_tile_height_plain<gemm_sk::TileOf<256, 128>>(stream, p, grid);
     }
 } // namespace nnf

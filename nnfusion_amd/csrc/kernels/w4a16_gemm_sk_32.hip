@@ -5,6 +5,6 @@ namespace nnf
 {
     hipError_t launch_gemm_sk_32(hipStream_t stream, const SkGemmParams& p, int grid, bool gate)
     {
-        return gemm_sk::launch_tile_height<1, 2>(stream, p, grid, gate);
+        return gemm_sk::launch_tile_height<gemm_sk::TileOf<32, 256>>(stream, p, grid, gate);
     }
 } // namespace nnf

@@ -5,6 +5,6 @@ namespace nnf
 {
     hipError_t launch_gemm_sk_64_narrow(hipStream_t stream, const SkGemmParams& p, int grid)
     {
-        return gemm_sk::launch_tile_height_plain<2, 1>(stream, p, grid);
+        return gemm_sk::launch_tile_height_plain<gemm_sk::TileOf<64, 128>>(stream, p, grid);
     }
 } // namespace nnf

@@ -9,11 +9,10 @@ namespace nnf
 {
     namespace gemm_sk
     {
-        template <int TM, int TN, bool GATE, bool BIAS, bool RESID, bool RMS>
+        template <class T, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0>
         hipError_t launch_instance(hipStream_t stream, const SkGemmParams& p, int grid)
         {
-            using T = Tile<TM, TN>;
-            auto kernel = &w4a16_gemm_sk_kernel<TM, TN, GATE, BIAS, RESID, RMS>;
+            auto kernel = &w4a16_gemm_sk_kernel<T::TM, T::TN, T::NW, T::KH, GATE, BIAS, RESID, RMS, QG>;
             if (T::LDS_BYTES > 48 * 1024)
             {
                 static LdsGrant granted;
@@ -21,88 +20,69 @@ namespace nnf
                 if (e != hipSuccess)
                     return e;
             }
-            launch_sk_kernel(kernel, grid, T::LDS_BYTES, stream, p);
+            launch_sk_kernel<T>(kernel, grid, stream, p);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess || !p.partial || p.sync)
                 return e;
             // tiles shared by several workgroups: their parts are added and finished by a second launch (unless the
-            // workgroups did it themselves: p.sync)
-            constexpr int ROUNDS = TM; // blocks of 32 rows
-            hipLaunchKernelGGL((w4a16_gemm_sk_fixup_kernel<TM, TN, GATE, BIAS, RESID, RMS>), dim3(p.tiles_m * p.tiles_n * ROUNDS * WAVES),
+            // workgroups did it themselves: p.sync); it does not depend on the block parameters
+            using Parts = Tile<T::TM, T::TN, T::NW, T::KH>;
+            constexpr int ROUNDS = T::TM; // blocks of 32 rows
+            hipLaunchKernelGGL((w4a16_gemm_sk_fixup_kernel<Parts, GATE, BIAS, RESID, RMS>), dim3(p.tiles_m * p.tiles_n * ROUNDS * T::NW),
                                dim3(64), 0, stream, p, grid);
             return hipGetLastError();
         }
 
-        template <int TM, int TN>
+        template <class T>
         hipError_t launch_tile_height(hipStream_t stream, const SkGemmParams& p, int grid, bool gate)
         {
             const bool hb = p.bias != nullptr, hr = p.residual != nullptr, rms = p.gamma != nullptr;
             if (gate)
-                return rms ? launch_instance<TM, TN, true, false, false, true>(stream, p, grid)
-                           : launch_instance<TM, TN, true, false, false, false>(stream, p, grid);
+                return rms ? launch_instance<T, true, false, false, true>(stream, p, grid)
+                           : launch_instance<T, true, false, false, false>(stream, p, grid);
             if (hb && hr)
-                return rms ? launch_instance<TM, TN, false, true, true, true>(stream, p, grid)
-                           : launch_instance<TM, TN, false, true, true, false>(stream, p, grid);
+                return rms ? launch_instance<T, false, true, true, true>(stream, p, grid)
+                           : launch_instance<T, false, true, true, false>(stream, p, grid);
             if (hb)
-                return rms ? launch_instance<TM, TN, false, true, false, true>(stream, p, grid)
-                           : launch_instance<TM, TN, false, true, false, false>(stream, p, grid);
+                return rms ? launch_instance<T, false, true, false, true>(stream, p, grid)
+                           : launch_instance<T, false, true, false, false>(stream, p, grid);
             if (hr)
-                return rms ? launch_instance<TM, TN, false, false, true, true>(stream, p, grid)
-                           : launch_instance<TM, TN, false, false, true, false>(stream, p, grid);
-            return rms ? launch_instance<TM, TN, false, false, false, true>(stream, p, grid)
-                       : launch_instance<TM, TN, false, false, false, false>(stream, p, grid);
+                return rms ? launch_instance<T, false, false, true, true>(stream, p, grid)
+                           : launch_instance<T, false, false, true, false>(stream, p, grid);
+            return rms ? launch_instance<T, false, false, false, true>(stream, p, grid)
+                       : launch_instance<T, false, false, false, false>(stream, p, grid);
         }
         // the forms without SiLU-gate (tiles one column tile per wavefront wide have no gate | up pairs)
-        template <int TM, int TN>
+        template <class T>
         hipError_t launch_tile_height_plain(hipStream_t stream, const SkGemmParams& p, int grid)
         {
             const bool hb = p.bias != nullptr, hr = p.residual != nullptr, rms = p.gamma != nullptr;
             if (hb && hr)
-                return rms ? launch_instance<TM, TN, false, true, true, true>(stream, p, grid)
-                           : launch_instance<TM, TN, false, true, true, false>(stream, p, grid);
+                return rms ? launch_instance<T, false, true, true, true>(stream, p, grid)
+                           : launch_instance<T, false, true, true, false>(stream, p, grid);
             if (hb)
-                return rms ? launch_instance<TM, TN, false, true, false, true>(stream, p, grid)
-                           : launch_instance<TM, TN, false, true, false, false>(stream, p, grid);
+                return rms ? launch_instance<T, false, true, false, true>(stream, p, grid)
+                           : launch_instance<T, false, true, false, false>(stream, p, grid);
             if (hr)
-                return rms ? launch_instance<TM, TN, false, false, true, true>(stream, p, grid)
-                           : launch_instance<TM, TN, false, false, true, false>(stream, p, grid);
-            return rms ? launch_instance<TM, TN, false, false, false, true>(stream, p, grid)
-                       : launch_instance<TM, TN, false, false, false, false>(stream, p, grid);
+                return rms ? launch_instance<T, false, false, true, true>(stream, p, grid)
+                           : launch_instance<T, false, false, true, false>(stream, p, grid);
+            return rms ? launch_instance<T, false, false, false, true>(stream, p, grid)
+                       : launch_instance<T, false, false, false, false>(stream, p, grid);
         }
         // other block parameters (QG = log2 of the group size; zero points per (row, group) when p.zps is set): the
-        // plain product; the second launch does not depend on them
-        template <int TM, int TN, int QG>
-        hipError_t launch_instance_q(hipStream_t stream, const SkGemmParams& p, int grid)
-        {
-            using T = Tile<TM, TN>;
-            auto kernel = &w4a16_gemm_sk_kernel<TM, TN, false, false, false, false, QG>;
-            if (T::LDS_BYTES > 48 * 1024)
-            {
-                static LdsGrant granted;
-                const hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), granted, T::LDS_BYTES);
-                if (e != hipSuccess)
-                    return e;
-            }
-            launch_sk_kernel(kernel, grid, T::LDS_BYTES, stream, p);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess || !p.partial || p.sync)
-                return e;
-            hipLaunchKernelGGL((w4a16_gemm_sk_fixup_kernel<TM, TN, false, false, false, false>), dim3(p.tiles_m * p.tiles_n * TM * WAVES),
-                               dim3(64), 0, stream, p, grid);
-            return hipGetLastError();
-        }
+        // plain product
         // tile_rows x tile_cols as sk_tile_shape chooses them for a plain product
         template <int QG>
         hipError_t launch_tiles_q(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols)
         {
             if (tile_cols == 128)
-                return tile_rows == 256   ? launch_instance_q<8, 1, QG>(stream, p, grid)
-                       : tile_rows == 128 ? launch_instance_q<4, 1, QG>(stream, p, grid)
-                       : tile_rows == 64  ? launch_instance_q<2, 1, QG>(stream, p, grid)
+                return tile_rows == 256   ? launch_instance<TileOf<256, 128>, false, false, false, false, QG>(stream, p, grid)
+                       : tile_rows == 128 ? launch_instance<TileOf<128, 128>, false, false, false, false, QG>(stream, p, grid)
+                       : tile_rows == 64  ? launch_instance<TileOf<64, 128>, false, false, false, false, QG>(stream, p, grid)
                                           : hipErrorInvalidValue;
-            return tile_rows == 256   ? launch_instance_q<8, 2, QG>(stream, p, grid)
-                   : tile_rows == 128 ? launch_instance_q<4, 2, QG>(stream, p, grid)
-                   : tile_rows == 32  ? launch_instance_q<1, 2, QG>(stream, p, grid)
+            return tile_rows == 256   ? launch_instance<TileOf<256, 256>, false, false, false, false, QG>(stream, p, grid)
+                   : tile_rows == 128 ? launch_instance<TileOf<128, 256>, false, false, false, false, QG>(stream, p, grid)
+                   : tile_rows == 32  ? launch_instance<TileOf<32, 256>, false, false, false, false, QG>(stream, p, grid)
                                       : hipErrorInvalidValue;
         }
     } // namespace gemm_sk

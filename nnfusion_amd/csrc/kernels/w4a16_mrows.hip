@@ -46,22 +46,24 @@ namespace nnf
     } // namespace
 
     // ---- pieces shared by the two forms of the kernel ----------------------------------------------------------------
-    // The activations of a wavefront as loaded -> the MFMA operand order of the nibble trick (pairs (a0,a4) (a1,a5)
-    // (a2,a6) (a3,a7)), and per group the constant part of its sum (an MFMA against a
-    // constant operand), negative, as the initial accumulator of the group.
-    // areg[.][g][.] *= the RMSNorm weight of the same k (fp16 products, rounded once); gsrc: the lane's 64 bytes of
-    // gamma for group g start at gsrc(g)
+    // areg[.][g][.] *= the RMSNorm weight of the same k (fp16 products, rounded once; gsrc: the lane's 64 bytes of gamma for group
+    // g start at gsrc(g)): activations in the pair order of the nibble trick, with the constant parts of their sums anew
     template <int MB, int GA, class F>
-    __device__ __forceinline__ void mrows_scale_a(uintx4 (&areg)[MB][GA][4], F&& gsrc)
+    __device__ __forceinline__ void mrows_scale_taken(uintx4 (&areg)[MB][GA][4], floatx4 (&ncorr)[MB][GA], int zp, F&& gsrc)
     {
+        const uint32_t ce2 = (0xE400u | (uint32_t)zp) * 0x10001u, co2 = (0xD400u | ((uint32_t)zp << 4)) * 0x10001u;
+        const half8_t cvec = __builtin_bit_cast(half8_t, uintx4{ce2, co2, ce2, co2});
 #pragma unroll
         for (int g = 0; g < GA; ++g)
         {
             const uintx4* gp = reinterpret_cast<const uintx4*>(gsrc(g));
 #pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+                ncorr[mb][g] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
             for (int j = 0; j < 4; ++j)
             {
-                const uintx4 gm = gp[j];
+                const uintx4 gm = permute_a8(gp[j]);
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
                 {
@@ -71,6 +73,7 @@ namespace nnf
                     a.z = as_u32(as_half2(a.z) * as_half2(gm.z));
                     a.w = as_u32(as_half2(a.w) * as_half2(gm.w));
                     areg[mb][g][j] = a;
+                    ncorr[mb][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), cvec, ncorr[mb][g], 0, 0, 0);
                 }
             }
         }
@@ -218,28 +221,77 @@ namespace nnf
             finish(idx, nullptr);
     }
 
-    template <int MB, int GA>
-    __device__ __forceinline__ void mrows_prepare_a(uintx4 (&areg)[MB][GA][4], floatx4 (&ncorr)[MB][GA], int zp)
+    // ---- the activations in blocks of 4 RL rows x 256 bytes (a group of 128), brought in through LDS as whole lines (see
+    // row_block_fetch), NF of them in flight at the places p % NF of a wavefront's 8 KiB: block p is group p % GA of the
+    // 16-row block p / GA.
+    constexpr int mrows_blocks_in_flight(int blocks, int RL) { return 8 / RL < blocks ? 8 / RL : blocks; }
+    // the loads of a block: row r of it (clamped to row M - 1), bytes [byte0, byte0 + 256), its 16 pieces XORed with r
+    template <int RL>
+    __device__ __forceinline__ void mrows_block_fetch(const uint8_t* A, size_t row_bytes, int first_row, int M, size_t byte0, uint8_t* block, int lane)
     {
-        const half_t ceh = (half_t)(-(1024.0f + (float)zp)), coh = (half_t)(-(64.0f + (float)zp)); // exact
-        const uint32_t ce2 = as_u32(half2_t{ceh, ceh}), co2 = as_u32(half2_t{coh, coh});
-        const uintx4 cvec = {ce2, co2, ce2, co2};
+#pragma unroll
+        for (int c = 0; c < RL; ++c)
+        {
+            const int r = c * 4 + (lane >> 4);
+            const uint8_t* src = A + (size_t)min(first_row + r, M - 1) * row_bytes + byte0 + ((lane & 15) ^ r) * 16;
+            __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(block + c * 1024), 16, 0, 0);
+        }
+    }
+    // Takes the blocks as they come: MFMA operand registers in the pair order of the nibble trick, the constant part of each
+    // group's sum (an MFMA against a constant operand, negative, the initial accumulator of the group); NORM: gamma onto them
+    // (fp16 products, rounded once) and the wavefront's share of sum a^2 of every row, the diagonal of A . A^T (the matrix
+    // cores have nothing else to do here).  fetch(integral_constant p): asks for block p; the first NF have been asked for, BEHIND
+    // other loads after them.  gamma_block: the group's 256 bytes of gamma one after the other, in LDS, asked for ahead of the blocks.
+    template <int MB, int GA, int RL, bool NORM, int BEHIND, class F>
+    __device__ __forceinline__ void mrows_take_blocks(uintx4 (&areg)[MB][GA][4], floatx4 (&ncorr)[MB][GA], floatx4 (&sq)[MB], const uint8_t* stage,
+                                                      const uint8_t* gamma_block, int zp, int col, int kq, F&& fetch)
+    {
+        constexpr int NP = MB * GA, NF = mrows_blocks_in_flight(NP, RL);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
+            sq[mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+        // -(1024 + zp), -(64 + zp) twice each, as bits (exact)
+        const uint32_t ce2 = (0xE400u | (uint32_t)zp) * 0x10001u, co2 = (0xD400u | ((uint32_t)zp << 4)) * 0x10001u;
+        const half8_t cvec = __builtin_bit_cast(half8_t, uintx4{ce2, co2, ce2, co2});
+        const int row = col & (4 * RL - 1);
+        unroll_for<0, NP>([&](auto p_c) {
+            constexpr int p = decltype(p_c)::value, mb = p / GA, g = p % GA;
+            // what has been asked for behind this block (vector-memory operations complete in order)
+            constexpr int LATER = RL * ((NF + p < NP ? NF + p : NP) - 1 - p) + (p < NF ? BEHIND : 0);
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(LATER));
+            const uint8_t* block = stage + (p % NF) * (RL * 1024) + row * 256;
+            uintx4 a[4], gm[4];
 #pragma unroll
-            for (int g = 0; g < GA; ++g)
+            for (int j = 0; j < 4; ++j)
+                a[j] = *reinterpret_cast<const uintx4*>(block + (((kq * 4 + j) ^ row) << 4));
+            if constexpr (NORM)
             {
-                floatx4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                {
-                    const uintx4 a = permute_a8(areg[mb][g][j]);
-                    areg[mb][g][j] = a;
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, cvec), t,
-                                                               0, 0, 0);
-                }
-                ncorr[mb][g] = t;
+                    gm[j] = *reinterpret_cast<const uintx4*>(gamma_block + g * 256 + kq * 64 + j * 16);
             }
+            if constexpr (p + NF < NP)
+            {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the block has been read out of the place that is filled next
+                fetch(std::integral_constant<int, (p + NF < NP ? p + NF : 0)>{});
+            }
+            floatx4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                if constexpr (NORM)
+                {
+                    sq[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[j]), __builtin_bit_cast(half8_t, a[j]), sq[mb], 0, 0, 0);
+                    a[j].x = as_u32(as_half2(a[j].x) * as_half2(gm[j].x));
+                    a[j].y = as_u32(as_half2(a[j].y) * as_half2(gm[j].y));
+                    a[j].z = as_u32(as_half2(a[j].z) * as_half2(gm[j].z));
+                    a[j].w = as_u32(as_half2(a[j].w) * as_half2(gm[j].w));
+                }
+                areg[mb][g][j] = permute_a8(a[j]);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[mb][g][j]), cvec, t, 0, 0, 0);
+            }
+            ncorr[mb][g] = t;
+        });
     }
 
     // One group of 128 along K: the lane's 16 bytes of weights (32 nibbles) against group ga of the activations,
@@ -448,72 +500,18 @@ namespace nnf
                 __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(gamma_block + i * 1024), 16, 0, 0);
             }
         }
-        constexpr int NP = MB * GA;                                                        // blocks of 4 RL rows x 256 bytes
-        constexpr int ROOM = 2 * ROW_BLOCK_BYTES / 1024 / RL, NF = ROOM < NP ? ROOM : NP; // ... in flight, at the places p % NF
+        constexpr int NF = mrows_blocks_in_flight(MB * GA, RL);
         auto fetch = [&](auto p_c) {
-            constexpr int p = decltype(p_c)::value, mb = p / GA, g = p % GA;
-#pragma unroll
-            for (int c = 0; c < RL; ++c)
-            {
-                const int r = c * 4 + (lane >> 4);
-                const uint8_t* src = reinterpret_cast<const uint8_t*>(A) + (size_t)min(mb * 16 + r, M - 1) * (K * 2) +
-                                     ((g / GW) * (SPAN * 4) + wave * (GW * 256) + (g % GW) * 256 + ((lane & 15) ^ r) * 16);
-                __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(stage + (p % NF) * (RL * 1024) + c * 1024), 16, 0, 0);
-            }
+            constexpr int p = decltype(p_c)::value, g = p % GA;
+            mrows_block_fetch<RL>(reinterpret_cast<const uint8_t*>(A), (size_t)K * 2, (p / GA) * 16, M,
+                                  (size_t)((g / GW) * (SPAN * 4) + wave * (GW * 256) + (g % GW) * 256), stage + (p % NF) * (RL * 1024), lane);
         };
         unroll_for<0, NF>([&](auto p_c) { fetch(p_c); });
         issue(0, 0, 0);
         issue(min(1 / STEPS, T - 1), 1 % STEPS, 1);
-        // ---- the activations, block by block: MFMA operand registers in the pair order of the nibble trick, the constant part
-        // of each group's sum; RMSNorm: gamma onto them (fp16 products, rounded once) and the wavefront's share of sum a^2 of
-        // every row
         uintx4 areg[MB][GA][4];
-        floatx4 ncorr[MB][GA];
-        floatx4 sq[MB]; // A . A^T: the sums of squares are its diagonal (the matrix cores have nothing else to do here)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-            sq[mb] = floatx4{0.f, 0.f, 0.f, 0.f};
-        // -(1024 + zp), -(64 + zp) twice each, as bits (exact)
-        const uint32_t ce2 = (0xE400u | (uint32_t)zp) * 0x10001u, co2 = (0xD400u | ((uint32_t)zp << 4)) * 0x10001u;
-        const half8_t cvec = __builtin_bit_cast(half8_t, uintx4{ce2, co2, ce2, co2});
-        unroll_for<0, NP>([&](auto p_c) {
-            constexpr int p = decltype(p_c)::value, mb = p / GA, g = p % GA;
-            // what has been asked for behind this block
-            constexpr int LATER = RL * ((NF + p < NP ? NF + p : NP) - 1 - p) + (p < NF ? 2 * LT : 0);
-            __builtin_amdgcn_s_waitcnt(vmcnt_only(LATER));
-            const int row = col & (4 * RL - 1);
-            uintx4 a[4], gm[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                a[j] = *reinterpret_cast<const uintx4*>(stage + (p % NF) * (RL * 1024) + row * 256 + (((kq * 4 + j) ^ row) << 4));
-            if constexpr (norm)
-            {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    gm[j] = *reinterpret_cast<const uintx4*>(gamma_block + g * 256 + kq * 64 + j * 16);
-            }
-            if constexpr (p + NF < NP)
-            {
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the block has been read out of the place that is filled next
-                fetch(std::integral_constant<int, (p + NF < NP ? p + NF : 0)>{});
-            }
-            floatx4 t = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-            {
-                if constexpr (norm)
-                {
-                    sq[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[j]), __builtin_bit_cast(half8_t, a[j]), sq[mb], 0, 0, 0);
-                    a[j].x = as_u32(as_half2(a[j].x) * as_half2(gm[j].x));
-                    a[j].y = as_u32(as_half2(a[j].y) * as_half2(gm[j].y));
-                    a[j].z = as_u32(as_half2(a[j].z) * as_half2(gm[j].z));
-                    a[j].w = as_u32(as_half2(a[j].w) * as_half2(gm[j].w));
-                }
-                areg[mb][g][j] = permute_a8(a[j]);
-                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[mb][g][j]), cvec, t, 0, 0, 0);
-            }
-            ncorr[mb][g] = t;
-        });
+        floatx4 ncorr[MB][GA], sq[MB];
+        mrows_take_blocks<MB, GA, RL, norm, 2 * LT>(areg, ncorr, sq, stage, gamma_block, zp, col, kq, fetch);
         // (behind the weights: the tile loop's counted waits then wait for two of the second step's loads as well)
         MrowsAhead ahead;
         if (FUSED && residual)
@@ -1349,13 +1347,14 @@ namespace nnf
     // pack = M | zp << 8.
     // FUSED: as in w4a16_mrows_kernel; over ranges of K only the RMSNorm weight applies here (the sums of a range go to
     // `partial` as they are: rstd and the rest of the epilogue belong to the reduction pass).
-    template <int GW, int STEPS, int MB, bool FUSED, bool STAGE>
+    template <int GW, int STEPS, int MB, bool FUSED, int RL>
     __global__ __launch_bounds__(512) void w4a16_mrows_any_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                                   const half_t* __restrict__ S, half_t* __restrict__ Y,
                                                                   float* __restrict__ partial, int N, int K, int tiles,
                                                                   int pack, GemvFusionArgs f, uint32_t* sync)
     {
         static_assert(GW >= 1 && GW <= 7 && STEPS >= 1 && GW * STEPS <= 8, "groups per wavefront");
+        static_assert(RL == 4 || (MB == 1 && (RL == 1 || RL == 2)), "rows of a block");
         static_assert(MB == 1 || (MB == 2 && GW * STEPS <= 4) || (MB == 4 && GW * STEPS <= 2), "16 VGPRs per group and block of rows");
         constexpr int GA = GW * STEPS;         // groups of a wavefront
         constexpr int SLICE = GW * 64;         // a wavefront's bytes of a weight row per step
@@ -1430,6 +1429,15 @@ namespace nnf
             __builtin_amdgcn_global_load_lds((mr_global_ptr_t)(reinterpret_cast<const uint8_t*>(S) + s_word * 4u),
                                              (mr_lds_ptr_t)(sc_ring + slot * 256), 4, 0, 0);
         };
+        // ---- the activations ahead of the weights, as in w4a16_mrows_kernel
+        uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
+        constexpr int NF = mrows_blocks_in_flight(MB * GA, RL);
+        auto fetch = [&](auto p_c) {
+            constexpr int p = decltype(p_c)::value, ga = p % GA;
+            mrows_block_fetch<RL>(reinterpret_cast<const uint8_t*>(A), (size_t)K * 2, (p / GA) * 16, M,
+                                  (size_t)(fetch_group(ga / GW) + ga % GW) * 256, stage + (p % NF) * (RL * 1024), lane);
+        };
+        unroll_for<0, NF>([&](auto p_c) { fetch(p_c); });
         issue(0, 0, 0);
         issue(min(1 / STEPS, T - 1), 1 % STEPS, 1);
 
@@ -1438,56 +1446,21 @@ namespace nnf
         const uint32_t red_addr = lds_address(red) + (uint32_t)(wave * (MB * 1024) + lane * 16);
         const uint32_t parked_addr = lds_address(parked);
         int slot = 0;
+        MrowsAhead ahead;
         {
-            // ---- the activations: into the MFMA operand registers, through LDS as whole lines (see row_block_fetch: two
-            // blocks per wavefront, over what holds the partial tiles and the parked sums later -- hence the barrier)
-            // (a few rows: straight into the registers, as in the kernel above)
             uintx4 areg[MB][GA][4];
-            floatx4 ncorr[MB][GA];
-            if constexpr (!STAGE)
-            {
-                const uint8_t* a_row = reinterpret_cast<const uint8_t*>(A) + (size_t)min(col, M - 1) * (size_t)(K * 2) + kq * 64;
-#pragma unroll
-                for (int ga = 0; ga < GA; ++ga)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        areg[0][ga][j] = *reinterpret_cast<const uintx4*>(a_row + (size_t)(fetch_group(ga / GW) + ga % GW) * 256 + j * 16);
-            }
-            else
-            {
-                uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
-                constexpr int NP = MB * GA;
-                auto fetch = [&](int p) {
-                    const int mb = p / GA, ga = p % GA;
-                    row_block_fetch(reinterpret_cast<const uint8_t*>(A), (size_t)K * 2, mb * 16, M - 1,
-                                    (size_t)(fetch_group(ga / GW) + ga % GW) * 256, stage + (p & 1) * ROW_BLOCK_BYTES, lane);
-                };
-                fetch(0);
-#pragma unroll
-                for (int p = 0; p < NP; ++p)
-                {
-                    if (p + 1 < NP)
-                    {
-                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // block p-1 has been read out of the half that is filled next
-                        fetch(p + 1);
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
-                    }
-                    else
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        areg[p / GA][p % GA][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
-                }
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                __syncthreads();
-            }
+            floatx4 ncorr[MB][GA], unused[MB];
+            mrows_take_blocks<MB, GA, RL, false, 2 * LT>(areg, ncorr, unused, stage, nullptr, zp, col, kq, fetch);
+            if (FUSED && f.residual && !partial)
+                mrows_ask_ahead(ahead, f.residual, t0, T_out, M, N, tid);
+            // (the blocks lay over what holds the partial tiles and the parked sums from here on)
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             // (RMSNorm: gamma here, rstd from a pass of its own.  The sum of squares and gamma inside the kernel -- spills at eight
             // groups or two blocks of rows, gamma straight from memory -- took longer than that pass: 7168 / 12 rows 0.7 x)
             if (FUSED && f.gamma)
-                mrows_scale_a<MB, GA>(areg, [&](int g) {
+                mrows_scale_taken<MB, GA>(areg, ncorr, zp, [&](int g) {
                     return reinterpret_cast<const uint8_t*>(f.gamma) + kq * 64 + (size_t)fetch_group(g / GW) * 256 + (g % GW) * 256;
                 });
-            mrows_prepare_a<MB, GA>(areg, ncorr, zp);
             for (int it = 0; it < T; ++it)
             {
                 floatx4 acc[MB];
@@ -1528,13 +1501,14 @@ namespace nnf
         }
         __builtin_amdgcn_s_waitcnt(mr_vmcnt(0)); // the reloads past the end, before the LDS goes away
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const DivideByRows by_rows(M);
         if (partial && !sync)
         {
             for (int idx = tid; idx < T * M * 16; idx += 512)
             {
                 const int n = idx & 15;
                 const int im = idx >> 4;
-                const int it = im / M, m = im - it * M;
+                const int it = by_rows(im), m = im - it * M;
                 partial[(size_t)blockIdx.y * M * N + (size_t)m * N + min((t0 + it) * 16, N - 16) + n] = parked[idx];
             }
         }
@@ -1549,7 +1523,7 @@ namespace nnf
             {
                 const int n = idx & 15;
                 const int im = idx >> 4;
-                const int it = im / M, m = im - it * M;
+                const int it = by_rows(im), m = im - it * M;
                 __hip_atomic_store(partial + (size_t)blockIdx.y * M * N + (size_t)m * N + min((t0 + it) * 16, N - 16) + n, parked[idx],
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -1567,7 +1541,7 @@ namespace nnf
                 {
                     const int n = idx & 15;
                     const int im = idx >> 4;
-                    const int it = im / M, m = im - it * M;
+                    const int it = by_rows(im), m = im - it * M;
                     const int nn = min((t0 + it) * 16, N - 16) + n;
                     if (nn < (t0 + it) * 16) // (a last tile moved back: these columns belong to the tile before it)
                         continue;
@@ -1616,7 +1590,7 @@ namespace nnf
             }
         }
         else
-            mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate);
+            mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate, nullptr, FUSED ? &ahead : nullptr);
     }
 
     namespace
@@ -1682,7 +1656,7 @@ namespace nnf
     namespace
     {
         // ranges == 1: the whole of K, fp16 results to Y; otherwise ranges of range_groups groups, fp32 sums to partial
-        template <int GW, int STEPS, int MB, bool FUSED, bool STAGE = true>
+        template <int GW, int STEPS, int MB, bool FUSED, int RL = 4>
         hipError_t launch_mrows_any_mb(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
                                        int zp, int num_cu, float* partial, int ranges, int range_groups, const GemvFusion& fusion,
                                        uint32_t* sync)
@@ -1695,7 +1669,7 @@ namespace nnf
             // over ranges of K the epilogue belongs to whoever adds the ranges up: the reduction pass, or (sync) the launch itself
             if (lds > MAX_LDS_BYTES || (ranges > 1 && (fusion.gate || (!sync && (fusion.bias || fusion.residual || fusion.rstd)))))
                 return hipErrorInvalidValue;
-            auto kernel = &w4a16_mrows_any_kernel<GW, STEPS, MB, FUSED, STAGE>;
+            auto kernel = &w4a16_mrows_any_kernel<GW, STEPS, MB, FUSED, RL>;
             if (lds > 64 * 1024)
             {
                 static LdsGrant granted;
@@ -1717,9 +1691,12 @@ namespace nnf
                                       int zp, int num_cu, float* partial, int ranges, int range_groups, const GemvFusion& fusion,
                                       uint32_t* sync)
         {
-            if (M <= 16 && !workspace::mrows_stages_activations(M, K))
-                return launch_mrows_any_mb<GW, STEPS, 1, FUSED, false>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, partial, ranges,
-                                                                       range_groups, fusion, sync);
+            if (M <= 4)
+                return launch_mrows_any_mb<GW, STEPS, 1, FUSED, 1>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, partial, ranges, range_groups,
+                                                                   fusion, sync);
+            if (M <= 8)
+                return launch_mrows_any_mb<GW, STEPS, 1, FUSED, 2>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, partial, ranges, range_groups,
+                                                                   fusion, sync);
             if (M <= 16)
                 return launch_mrows_any_mb<GW, STEPS, 1, FUSED>(stream, A, Wq, S, Y, M, N, K, zp, num_cu, partial, ranges, range_groups,
                                                                 fusion, sync);

@@ -149,6 +149,21 @@ namespace nnf
         }
     }
 
+    // v of this lane + v of the lane 16 (32) away, the same in both, without the LDS unit: the compiler waits for every LDS-bound
+    // load in flight ahead of a ds_bpermute.  (The builtin's two results, given the same operand twice, come out as one.)
+    __device__ __forceinline__ float row_pair_sum(float v)
+    {
+        float other = v;
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(other));
+        return v + other;
+    }
+    __device__ __forceinline__ float half_pair_sum(float v)
+    {
+        float other = v;
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(v), "+v"(other));
+        return v + other;
+    }
+
     // im / M for 0 <= im < 2^13 and M <= 64, by multiplication (a division is forty instructions, at the end of the launch)
     struct DivideByRows
     {
@@ -239,17 +254,18 @@ namespace nnf
     }
     // Takes the blocks as they come: MFMA operand registers in the pair order of the nibble trick, the constant part of each
     // group's sum (an MFMA against a constant operand, negative, the initial accumulator of the group); NORM: gamma onto them
-    // (fp16 products, rounded once) and the wavefront's share of sum a^2 of every row, the diagonal of A . A^T (the matrix
-    // cores have nothing else to do here).  fetch(integral_constant p): asks for block p; the first NF have been asked for, BEHIND
+    // (fp16 products, rounded once) and the lane's share of sum a^2 of its row.  fetch(integral_constant p): asks for block p; the first NF have been asked for, BEHIND
     // other loads after them.  gamma_block: the group's 256 bytes of gamma one after the other, in LDS, asked for ahead of the blocks.
+    // (v_dot2_f32_f16 in one chain, in the order of k.  On the matrix cores, as the diagonal of A . A^T, the squares cost
+    // nothing and the sum is no worse, but rounds otherwise; no difference in time at 6 and 16 rows x 4096.)
     template <int MB, int GA, int RL, bool NORM, int BEHIND, class F>
-    __device__ __forceinline__ void mrows_take_blocks(uintx4 (&areg)[MB][GA][4], floatx4 (&ncorr)[MB][GA], floatx4 (&sq)[MB], const uint8_t* stage,
+    __device__ __forceinline__ void mrows_take_blocks(uintx4 (&areg)[MB][GA][4], floatx4 (&ncorr)[MB][GA], float (&sq)[MB], const uint8_t* stage,
                                                       const uint8_t* gamma_block, int zp, int col, int kq, F&& fetch)
     {
         constexpr int NP = MB * GA, NF = mrows_blocks_in_flight(NP, RL);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
-            sq[mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+            sq[mb] = 0.f;
         // -(1024 + zp), -(64 + zp) twice each, as bits (exact)
         const uint32_t ce2 = (0xE400u | (uint32_t)zp) * 0x10001u, co2 = (0xD400u | ((uint32_t)zp << 4)) * 0x10001u;
         const half8_t cvec = __builtin_bit_cast(half8_t, uintx4{ce2, co2, ce2, co2});
@@ -281,7 +297,10 @@ namespace nnf
             {
                 if constexpr (NORM)
                 {
-                    sq[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[j]), __builtin_bit_cast(half8_t, a[j]), sq[mb], 0, 0, 0);
+                    sq[mb] = dot2(as_half2(a[j].x), as_half2(a[j].x), sq[mb]);
+                    sq[mb] = dot2(as_half2(a[j].y), as_half2(a[j].y), sq[mb]);
+                    sq[mb] = dot2(as_half2(a[j].z), as_half2(a[j].z), sq[mb]);
+                    sq[mb] = dot2(as_half2(a[j].w), as_half2(a[j].w), sq[mb]);
                     a[j].x = as_u32(as_half2(a[j].x) * as_half2(gm[j].x));
                     a[j].y = as_u32(as_half2(a[j].y) * as_half2(gm[j].y));
                     a[j].z = as_u32(as_half2(a[j].z) * as_half2(gm[j].z));
@@ -510,7 +529,8 @@ namespace nnf
         issue(0, 0, 0);
         issue(min(1 / STEPS, T - 1), 1 % STEPS, 1);
         uintx4 areg[MB][GA][4];
-        floatx4 ncorr[MB][GA], sq[MB];
+        floatx4 ncorr[MB][GA];
+        float sq[MB];
         mrows_take_blocks<MB, GA, RL, norm, 2 * LT>(areg, ncorr, sq, stage, gamma_block, zp, col, kq, fetch);
         // (behind the weights: the tile loop's counted waits then wait for two of the second step's loads as well)
         MrowsAhead ahead;
@@ -523,10 +543,8 @@ namespace nnf
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
             {
-                // row m of D in element m % 4 of the lanes with kq = m / 4
-                const float lower = (col & 1) ? sq[mb].y : sq[mb].x, upper = (col & 1) ? sq[mb].w : sq[mb].z;
-                const float sum = (col & 2) ? upper : lower;
-                if (kq == (col >> 2)) // (by hand: ahead of an LDS write that it can see, the compiler waits for every LDS-bound load in flight)
+                const float pair = row_pair_sum(sq[mb]), sum = half_pair_sum(pair);
+                if (kq == 0) // (by hand: ahead of an LDS write that it can see, the compiler waits for every LDS-bound load in flight)
                     asm volatile("ds_write_b32 %0, %1" ::"v"(lds_address(sum_sq + wave * (MB * 16) + mb * 16 + col)), "v"(sum) : "memory");
             }
         }
@@ -1449,7 +1467,8 @@ namespace nnf
         MrowsAhead ahead;
         {
             uintx4 areg[MB][GA][4];
-            floatx4 ncorr[MB][GA], unused[MB];
+            floatx4 ncorr[MB][GA];
+            float unused[MB];
             mrows_take_blocks<MB, GA, RL, false, 2 * LT>(areg, ncorr, unused, stage, nullptr, zp, col, kq, fetch);
             if (FUSED && f.residual && !partial)
                 mrows_ask_ahead(ahead, f.residual, t0, T_out, M, N, tid);

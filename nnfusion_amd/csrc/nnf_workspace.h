@@ -1022,15 +1022,15 @@ namespace nnf
                 return false;
             if (w4a16_mrows_fixed_k(M, K))
                 return true;
+            // Up to seven rows, even numbers of groups, against the MFMA GEMV, whatever part of what is fetched counts (N = 1024 / 4096 / 12288): K = 1280 ..
+            // 1920 1.0 - 1.2 x, 2304 .. 5888 1.0 - 1.1, 6144 .. 7936 1.04 - 1.4 (4096 x 7168 9.7 -> 7.7 us at seven rows), 1024 and 1152 0.86 - 1.0.
+            // (Before the activations came first, in blocks of four or eight rows, these were level or slower.)  Odd numbers of groups keep the GEMV and
+            // with it the order of their sums, 1.0 - 1.2 x here.
+            if (M < 8)
+                return !(K & 128) && K >= 1280;
             const int gw = w4a16_mrows_step_groups(M, K);
-            if (gw == 4 && M < 8) // K = 6400 .. 7936: N = K = 7168 takes 10.7 us at M = 2 against 9.0 (level from M = 6 on)
-                return false;
-            // Odd numbers of groups, and up to sixteen of them (one group per wavefront and step), from eight rows on (N = 1152 /
-            // 4096 / 12288 against the MFMA GEMV, 2 / 6 rows: 0.91 - 1.1 x; 12 / 16 rows: K = 3200 1.15 - 1.4 x, 5504 1.6 - 1.75,
-            // 8064 1.2 - 1.45, 1920 1.1 - 1.25).  17 .. 32 rows, whose other kernel is the tile GEMM, whatever part of what is fetched
-            // counts (K = 1664 .. 1920 1.8 - 2.9 x, 3200 1.7 - 2.5, 3968 1.8 - 2.2).
-            if (((K & 128) || gw == 1) && M < 8)
-                return false;
+            // 8 .. 16 rows (K = 3200 1.15 - 1.4 x, 5504 1.6 - 1.75, 8064 1.2 - 1.45, 1920 1.1 - 1.25); 17 .. 32 rows, whose other kernel is the
+            // tile GEMM, whatever part of what is fetched counts (K = 1664 .. 1920 1.8 - 2.9 x, 3200 1.7 - 2.5, 3968 1.8 - 2.2).
             // 33 .. 64 rows (the library's own choice is the K-streaming kernel there, 1.2 - 1.9 x; scratch sizes follow this rule), up to
             // sixteen groups: four blocks of rows against the tile GEMM, 1152 / 4096 / 12288 / 22016 weight rows: K = 1280
             // 1.45 / 1.3 / 0.9 - 1.0 / 0.7 x, 1664 .. 2048 1.5 / 1.4 / 1.1 - 1.3 / 0.8 - 1.0; RMSNorm and SiLU-gate 1.5 / 1.5 / 1.2 - 1.4 / 1.0 - 1.3
@@ -1408,7 +1408,7 @@ namespace nnf
                 // the reduction would have to pair, nor with RMSNorm, which the single launch folds in without a pre-pass)
                 const bool two_ranges = !gate && !rms && K == 8192 && M >= 8 && M <= 16 && w4a16_mrows_split(M, n_rows, K, num_cu).ranges > 1;
                 // (the products that once ran elsewhere: gamma times the activations alone may leave the range of fp16)
-                const bool taken_over = rms && !w4a16_mrows_fixed_k(M, K) && ((K & 128) || M > 32 || 4 * (K >> 7) < 3 * 16 * (K <= 4096 ? 2 : 3));
+                const bool taken_over = rms && !w4a16_mrows_fixed_k(M, K) && ((K & 128) || M > 32 || 4 * (K >> 7) < 3 * 16 * (K <= 4096 ? 2 : 3) || (M < 8 && K > 6144));
                 const bool gemv_ahead = any && !gate && !in_place_residual && w4a16_skinny_ahead_of_mrows(M, n_rows, K);
                 if (rows_family && M > 1 && !two_ranges && !gemv_ahead && !(any && taken_over && !room_for_copy) &&
                     (any ? w4a16_mrows_preferred(M, N, K, num_cu, gate) : w4a16_mrows_fits(M, N, K, num_cu, gate)))

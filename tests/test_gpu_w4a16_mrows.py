@@ -1,7 +1,7 @@
 """The row-streaming MFMA kernel with K a compile-time constant (w4a16_mrows.hip): activations in blocks of 4, 8 and 16 rows.
 
 Rows on both sides of a block's size, every number of blocks a wavefront brings in (1 .. 8, of which two, four or eight are in
-flight), a last tile that is moved back, and -- 22016 columns and more -- more outputs a thread than the two whose residual is asked
+flight), the ends of the run-time K that two to seven rows take to it (1280, 1792, 6400, 7936), a last tile that is moved back, and -- 22016 columns and more -- more outputs a thread than the two whose residual is asked
 for ahead.  Tolerance, of the result's RMS: the output's rounding, 2^-11 of up to 5.5 RMS, 2.7e-3, and a residual's once more; with RMSNorm
 activations times gamma rounded to eleven bits, 2^-11 / sqrt(3) in the 2-norm at most and 5.5 of that, 1.6e-3: 5e-3 (SiLU-gate: two
 rounded products multiplied, values up to some ten RMS, 2e-2).
@@ -26,7 +26,7 @@ def _check(y, ref, tol=TOL):
 
 
 @pytest.mark.parametrize("m,n,k", [(4, 40, 1024), (5, 300, 2048), (8, 1000, 3072), (9, 520, 4096), (2, 4104, 6144), (4, 300, 8192), (8, 72, 8192),
-                                   (16, 300, 8192), (7, 24584, 1024), (16, 22016, 2048), (17, 300, 1024)])
+                                   (16, 300, 8192), (3, 520, 1280), (7, 300, 1792), (2, 1000, 6400), (7, 300, 7936), (7, 24584, 1024), (16, 22016, 2048), (17, 300, 1024)])
 @pytest.mark.parametrize("form", ["plain", "residual", "rms", "rms-residual", "rms-gate"])
 def test_blocks_of_activations(gpu, form, m, n, k):
     import torch

@@ -484,15 +484,16 @@ namespace nnf
             p.rstd_sync = (uint32_t*)choice.sync_flags;
             p.rms_eps = rms_eps;
         }
+        const bool eight = workspace::sk_eight_wavefronts(plan, gate, rms, num_cu);
         if (plan.tile_weight_rows == 128)
             return plan.tile_rows == 256 ? launch_gemm_sk_256_narrow(stream, p, plan.grid)
-                   : plan.tile_rows == 128 ? launch_gemm_sk_128_narrow(stream, p, plan.grid)
-                                           : launch_gemm_sk_64_narrow(stream, p, plan.grid);
+                   : plan.tile_rows == 128 ? launch_gemm_sk_128_narrow(stream, p, plan.grid, eight)
+                                           : launch_gemm_sk_64_narrow(stream, p, plan.grid, eight);
         switch (plan.tile_rows)
         {
         case 256: return launch_gemm_sk_256(stream, p, plan.grid, gate);
-        case 128: return launch_gemm_sk_128(stream, p, plan.grid, gate);
-        case 64: return launch_gemm_sk_64(stream, p, plan.grid, gate);
+        case 128: return launch_gemm_sk_128(stream, p, plan.grid, gate, eight);
+        case 64: return launch_gemm_sk_64(stream, p, plan.grid, gate, eight);
         default: return launch_gemm_sk_32(stream, p, plan.grid, gate);
         }
     }
@@ -579,11 +580,12 @@ namespace nnf
         p.units = plan.units;
         p.zps = (const uint8_t*)zero_points;
         set_sync(p, plan, choice, num_cu);
+        const bool eight = workspace::sk_eight_wavefronts(plan, false, false, num_cu);
         switch (group_shift)
         {
-        case 5: return launch_gemm_sk_q5(stream, p, plan.grid, plan.tile_rows, plan.tile_weight_rows);
-        case 6: return launch_gemm_sk_q6(stream, p, plan.grid, plan.tile_rows, plan.tile_weight_rows);
-        default: return launch_gemm_sk_q7(stream, p, plan.grid, plan.tile_rows, plan.tile_weight_rows);
+        case 5: return launch_gemm_sk_q5(stream, p, plan.grid, plan.tile_rows, plan.tile_weight_rows, eight);
+        case 6: return launch_gemm_sk_q6(stream, p, plan.grid, plan.tile_rows, plan.tile_weight_rows, eight);
+        default: return launch_gemm_sk_q7(stream, p, plan.grid, plan.tile_rows, plan.tile_weight_rows, eight);
         }
     }
 } // namespace nnf

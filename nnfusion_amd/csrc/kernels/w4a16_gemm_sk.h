@@ -1,4 +1,4 @@
-// fp16 x int4 (g128) MFMA tile GEMM for gfx950: four wavefronts side by side along N, tiles cut into
+// fp16 x int4 (g128) MFMA tile GEMM for gfx950: four or eight wavefronts a workgroup, tiles cut into
 // equal parts of K, or the work of all tiles split evenly over the CUs.
 //
 //   Y[M,N] = epilogue( prologue(A)[M,K] . ((Wq - zp) * S)^T )
@@ -14,9 +14,9 @@
 // accumulators of a 256 x 256 tile in registers there is one wavefront per SIMD, whose vector, LDS and
 // memory instructions are issued between its own MFMAs and not under them.  The structure therefore
 // minimises traffic and instructions per MFMA:
-//   * One workgroup = four wavefronts (one per SIMD, up to 512 registers each) over a (TM*32) x (TN*128)
-//     tile, each wavefront owning all TM*32 rows of a strip of TN*32 columns (TM x TN MFMA tiles of
-//     32x32x16).  A weight belongs to exactly one wavefront: it is unpacked once per workgroup (16 VALU
+//   * One workgroup = four wavefronts (one per SIMD, up to 512 registers each; two of up to 256 where
+//     gemm_sk::TileOf says so) over a tile, each wavefront owning all TM*32 rows of a strip of TN*32 columns
+//     (TM x TN MFMA tiles of 32x32x16).  A weight belongs to exactly one wavefront: it is unpacked once per workgroup (16 VALU
 //     operations per 8 weights, feeding TM MFMAs each), not once per wavefront row.
 //   * A lane owns one weight row of each of its column tiles and one half of every 64-wide K step, and holds the
 //     weights of one "superstep" of 256 k (two quantization groups, four K steps) in registers at a time: 4 x 16
@@ -154,27 +154,49 @@ namespace nnf
             static constexpr size_t SLOT_FLOATS = (size_t)BM * BN;
         };
 
-        // rows x columns (weight rows) of a tile -> the wavefronts that work on it
-        template <int ROWS, int COLS>
+        // Rows x columns (weight rows) of a tile -> the wavefronts that work on it.  EIGHT: two a SIMD instead of one (64- and
+        // 128-row tiles; workspace::sk_eight_wavefronts chooses): while one waits for its operands or unpacks, the other's MFMAs
+        // run.  256 wide: eight strips of 32 columns instead of four of 64, each fragment of the activations read eight times
+        // instead of four.  128 wide, where strips of 16 columns would be left: two rows of four wavefronts, each with a ring of
+        // its own, every second superstep each, their sums added up at the end.  The two rings leave no room for a second
+        // workgroup on the CU.  (N = 12288, K = 4096: M = 256 on 128 x 128 tiles 33.3 -> 30.4 us, with RMSNorm 41.8 -> 37.0;
+        // M = 384 on 128 x 256 51.5 -> 47.7; 4096 x 11008 at M = 384 on 128 x 128 72.5 -> 57.8.)
+        template <int ROWS, int COLS, bool EIGHT = false>
         struct TileOf;
         template <>
         struct TileOf<32, 256> : Tile<1, 2, 4, 1>
         {
         };
         template <>
-        struct TileOf<64, 128> : Tile<2, 1, 4, 2>
+        struct TileOf<64, 128> : Tile<2, 1, 4, 1>
         {
         };
         template <>
-        struct TileOf<64, 256> : Tile<2, 1, 8, 1>
+        struct TileOf<64, 128, true> : Tile<2, 1, 4, 2>
         {
         };
         template <>
-        struct TileOf<128, 128> : Tile<4, 1, 4, 2>
+        struct TileOf<64, 256> : Tile<2, 2, 4, 1>
         {
         };
         template <>
-        struct TileOf<128, 256> : Tile<4, 1, 8, 1>
+        struct TileOf<64, 256, true> : Tile<2, 1, 8, 1>
+        {
+        };
+        template <>
+        struct TileOf<128, 128> : Tile<4, 1, 4, 1>
+        {
+        };
+        template <>
+        struct TileOf<128, 128, true> : Tile<4, 1, 4, 2>
+        {
+        };
+        template <>
+        struct TileOf<128, 256> : Tile<4, 2, 4, 1>
+        {
+        };
+        template <>
+        struct TileOf<128, 256, true> : Tile<4, 1, 8, 1>
         {
         };
         template <>
@@ -556,12 +578,12 @@ namespace nnf
         const int units = p.K >> 3;
         for (int m0 = first; m0 < end; m0 += ROWS * step)
         {
-            const int m = m0 + (tid >> 8) * step;
+            const int m = m0 + (ROWS > 1 ? tid >> 8 : 0) * step;
             if (m < end)
             {
                 const uintx4* row = reinterpret_cast<const uintx4*>(p.A + (size_t)m * p.K);
                 float ss = 0.f;
-                for (int i = tid & 255; i < units; i += 256)
+                for (int i = ROWS > 1 ? tid & 255 : tid; i < units; i += 256)
                 {
                     const uintx4 v = row[i];
                     const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
@@ -577,9 +599,9 @@ namespace nnf
                     part[tid >> 6] = ss;
             }
             __syncthreads();
-            if ((tid & 255) == 0 && m < end)
+            if ((ROWS > 1 ? tid & 255 : tid) == 0 && m < end)
             {
-                const float* four = part + (tid >> 6);
+                const float* four = part + (ROWS > 1 ? tid >> 6 : 0);
                 __hip_atomic_store(p.rstd_out + m, 1.0f / __builtin_sqrtf(((four[0] + four[1]) + (four[2] + four[3])) / (float)p.K + p.rms_eps),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -677,6 +699,7 @@ namespace nnf
         const int l32 = lane & 31, h = lane >> 5;
         // this wavefront's strip of columns; which of the KH rows of wavefronts it belongs to
         const int strip = KH > 1 ? wave % NW : wave, kh = KH > 1 ? wave / NW : 0;
+        const int strip_tid = KH > 1 ? strip * 64 + lane : tid;
         const int K = p.K;
         const int G = K >> GSH;
         const bool g_even = !(G & 1);
@@ -1360,7 +1383,7 @@ namespace nnf
             // (i, j) of all threads of a row of wavefronts is contiguous); w4a16_gemm_sk_fixup_kernel adds the parts and finishes
             if (!whole)
             {
-                const size_t first_float = ((size_t)v + (first_of_mine ? 0 : (size_t)grid)) * T::SLOT_FLOATS + (size_t)(strip * 64 + lane) * 4;
+                const size_t first_float = ((size_t)v + (first_of_mine ? 0 : (size_t)grid)) * T::SLOT_FLOATS + (size_t)strip_tid * 4;
                 float* mine = p.partial + first_float;
                 const bool same_launch = p.sync != nullptr;
                 const buffer_t parked = parked_buffer(p.partial, p.partial_bytes);
@@ -1482,7 +1505,6 @@ namespace nnf
                     if ((n & 1) != kh)
                         todo &= ~(rest & -rest);
             }
-            const int strip_tid = strip * 64 + lane;
             // (selected field by field: an array indexed at run time would live in private memory)
             auto tile_of = [&](int task) {
                 const bool second = task >= 8;

@@ -3,8 +3,9 @@
 
 namespace nnf
 {
-    hipError_t launch_gemm_sk_64(hipStream_t stream, const SkGemmParams& p, int grid, bool gate)
+    hipError_t launch_gemm_sk_64(hipStream_t stream, const SkGemmParams& p, int grid, bool gate, bool eight)
     {
-        return gemm_sk::launch_tile_height<gemm_sk::TileOf<64, 256>>(stream, p, grid, gate);
+        return eight ? gemm_sk::launch_tile_height<gemm_sk::TileOf<64, 256, true>>(stream, p, grid, gate)
+                     : gemm_sk::launch_tile_height<gemm_sk::TileOf<64, 256>>(stream, p, grid, gate);
     }
 } // namespace nnf

@@ -52,7 +52,7 @@ namespace nnf
             return rms ? launch_instance<T, false, false, false, true>(stream, p, grid)
                        : launch_instance<T, false, false, false, false>(stream, p, grid);
         }
-        // the forms without SiLU-gate (tiles one column tile per wavefront wide have no gate | up pairs)
+        // the forms without SiLU-gate (128-wide tiles have none)
         template <class T>
         hipError_t launch_tile_height_plain(hipStream_t stream, const SkGemmParams& p, int grid)
         {
@@ -70,33 +70,41 @@ namespace nnf
                        : launch_instance<T, false, false, false, false>(stream, p, grid);
         }
         // other block parameters (QG = log2 of the group size; zero points per (row, group) when p.zps is set): the
-        // plain product
-        // tile_rows x tile_cols as sk_tile_shape chooses them for a plain product
-        template <int QG>
-        hipError_t launch_tiles_q(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols)
+        // plain product; tile_rows x tile_cols as sk_tile_shape chooses them for it
+        template <int QG, bool EIGHT>
+        hipError_t launch_low_tiles_q(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols)
         {
             if (tile_cols == 128)
-                return tile_rows == 256   ? launch_instance<TileOf<256, 128>, false, false, false, false, QG>(stream, p, grid)
-                       : tile_rows == 128 ? launch_instance<TileOf<128, 128>, false, false, false, false, QG>(stream, p, grid)
-                       : tile_rows == 64  ? launch_instance<TileOf<64, 128>, false, false, false, false, QG>(stream, p, grid)
-                                          : hipErrorInvalidValue;
-            return tile_rows == 256   ? launch_instance<TileOf<256, 256>, false, false, false, false, QG>(stream, p, grid)
-                   : tile_rows == 128 ? launch_instance<TileOf<128, 256>, false, false, false, false, QG>(stream, p, grid)
-                   : tile_rows == 32  ? launch_instance<TileOf<32, 256>, false, false, false, false, QG>(stream, p, grid)
-                                      : hipErrorInvalidValue;
+                return tile_rows == 128 ? launch_instance<TileOf<128, 128, EIGHT>, false, false, false, false, QG>(stream, p, grid)
+                                        : launch_instance<TileOf<64, 128, EIGHT>, false, false, false, false, QG>(stream, p, grid);
+            return tile_rows == 128 ? launch_instance<TileOf<128, 256, EIGHT>, false, false, false, false, QG>(stream, p, grid)
+                                    : hipErrorInvalidValue; // (64 x 256: SiLU-gate only)
+        }
+        template <int QG>
+        hipError_t launch_tiles_q(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols, bool eight)
+        {
+            if (tile_rows == 64 || tile_rows == 128)
+                return eight ? launch_low_tiles_q<QG, true>(stream, p, grid, tile_rows, tile_cols)
+                             : launch_low_tiles_q<QG, false>(stream, p, grid, tile_rows, tile_cols);
+            if (tile_rows == 256)
+                return tile_cols == 128 ? launch_instance<TileOf<256, 128>, false, false, false, false, QG>(stream, p, grid)
+                                        : launch_instance<TileOf<256, 256>, false, false, false, false, QG>(stream, p, grid);
+            return tile_rows == 32 && tile_cols == 256 ? launch_instance<TileOf<32, 256>, false, false, false, false, QG>(stream, p, grid)
+                                                       : hipErrorInvalidValue;
         }
     } // namespace gemm_sk
 
     // groups of 32 / 64 / 128 with p.zps or p.zp (w4a16_gemm_sk_q5.hip ... _q7.hip)
-    hipError_t launch_gemm_sk_q5(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols);
-    hipError_t launch_gemm_sk_q6(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols);
-    hipError_t launch_gemm_sk_q7(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols);
-    // one per tile height (w4a16_gemm_sk_32.hip ... _256.hip); narrow: 128 x 128 tiles, plain product, bias, residual, RMSNorm
-    hipError_t launch_gemm_sk_64_narrow(hipStream_t stream, const SkGemmParams& p, int grid);
-    hipError_t launch_gemm_sk_128_narrow(hipStream_t stream, const SkGemmParams& p, int grid);
+    hipError_t launch_gemm_sk_q5(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols, bool eight);
+    hipError_t launch_gemm_sk_q6(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols, bool eight);
+    hipError_t launch_gemm_sk_q7(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols, bool eight);
+    // one per tile height (w4a16_gemm_sk_32.hip ... _256.hip); narrow: tiles 128 wide, plain product, bias, residual, RMSNorm;
+    // eight: on eight wavefronts
+    hipError_t launch_gemm_sk_64_narrow(hipStream_t stream, const SkGemmParams& p, int grid, bool eight);
+    hipError_t launch_gemm_sk_128_narrow(hipStream_t stream, const SkGemmParams& p, int grid, bool eight);
     hipError_t launch_gemm_sk_256_narrow(hipStream_t stream, const SkGemmParams& p, int grid);
     hipError_t launch_gemm_sk_32(hipStream_t stream, const SkGemmParams& p, int grid, bool gate);
-    hipError_t launch_gemm_sk_64(hipStream_t stream, const SkGemmParams& p, int grid, bool gate);
-    hipError_t launch_gemm_sk_128(hipStream_t stream, const SkGemmParams& p, int grid, bool gate);
+    hipError_t launch_gemm_sk_64(hipStream_t stream, const SkGemmParams& p, int grid, bool gate, bool eight);
+    hipError_t launch_gemm_sk_128(hipStream_t stream, const SkGemmParams& p, int grid, bool gate, bool eight);
     hipError_t launch_gemm_sk_256(hipStream_t stream, const SkGemmParams& p, int grid, bool gate);
 } // namespace nnf

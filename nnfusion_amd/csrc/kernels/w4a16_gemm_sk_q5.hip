@@ -4,8 +4,8 @@
 
 namespace nnf
 {
-    hipError_t launch_gemm_sk_q5(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols)
+    hipError_t launch_gemm_sk_q5(hipStream_t stream, const SkGemmParams& p, int grid, int tile_rows, int tile_cols, bool eight)
     {
-        return gemm_sk::launch_tiles_q<5>(stream, p, grid, tile_rows, tile_cols);
+        return gemm_sk::launch_tiles_q<5>(stream, p, grid, tile_rows, tile_cols, eight);
     }
 } // namespace nnf

@@ -383,6 +383,40 @@ namespace nnf
             }
             return best_grid ? plan_w4a16_sk(M, N, K, gate, num_cu, rows, best_grid, cols) : even;
         }
+        // Eight wavefronts on a tile of 64 or 128 rows instead of four (gemm_sk::TileOf).  A wavefront's own share of the work is halved, what
+        // comes before and behind the K loop is not, so it takes a long enough share; a second workgroup on the CU, which hides the
+        // waits as well, has no room beside the two rings of the 128-wide tiles; and near the full chip the activations' way out of LDS,
+        // read twice as often by the 256-wide ones, costs more than it hides.  3000 products on every tile and number of parts, start /
+        // this in the geometric mean: 128 x 128 tiles, one a CU, shares of 2 / 4 / 8 / 16 / 32 supersteps 0.93 / 1.02 / 1.11 / 1.17 / 1.23 (with
+        // RMSNorm 1.31 on few CUs, where rstd[] of many rows a workgroup takes half as long), more tiles than CUs 0.75 - 0.94; parts of
+        // 1 / 2 / 4 / 8 / 16: 0.92 / 0.95 / 1.02 / 1.09 / 1.16 up to half of the CUs, 0.92 / 0.89 / 0.90 / 0.98 / 1.05 above three quarters; 128 x 256
+        // one a CU 1.2 (few, short) .. 0.99 (220 and more, from 32 on), parts 1.10 .. 1.02, from three quarters of the CUs on 0.96 - 1.0.
+        inline bool sk_eight_wavefronts(const SkPlan& p, bool gate, bool rms, int num_cu)
+        {
+            if ((p.tile_rows != 64 && p.tile_rows != 128) || p.grid < 1)
+                return false;
+            const long long tiles = (long long)p.tiles_m * p.tiles_n, share = p.units / p.grid;
+            const bool one_each = p.grid == tiles, parts = p.grid > tiles && p.grid % tiles == 0;
+            if (rms && p.grid <= num_cu && (long long)p.tiles_m * p.tile_rows >= 4ll * p.grid && (one_each || parts))
+                return true;
+            if (p.tile_weight_rows == 128)
+            {
+                // (128 rows on more than three quarters of the CUs: 3 - 5 % faster by itself, but the chip's power goes with it: 1000 x 4096 x
+                // 11008 in groups of 32 behind two products of 1000 x 11008 x 4096 100.2 -> 96.7 us, and those 98.7 -> 103.3 each)
+                if (one_each && p.tile_rows == 128 && !rms && 4ll * p.grid > 3ll * num_cu)
+                    return false;
+                if (one_each)
+                    return p.grid <= num_cu && (share >= 8 || (share >= 4 && 8ll * p.grid <= 5ll * num_cu));
+                if (parts)
+                    return share >= 16 || (rms ? share >= 4 && 4ll * p.grid <= 3ll * num_cu : share >= 8 && 8ll * p.grid <= 5ll * num_cu);
+                return tiles > p.grid && p.supersteps >= 8;
+            }
+            if (one_each)
+                return share <= 16 || (share < 32 && p.grid <= num_cu && !gate) || 2ll * p.grid <= num_cu;
+            if (parts)
+                return 8ll * p.grid <= 5ll * num_cu && share < 32;
+            return (!gate && p.supersteps < 8) || (rms && share < 16);
+        }
         inline SkPlan plan_w4a16_tiles(int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = SIZE_MAX)
         {
             return plan_w4a16_tiles(plan_w4a16_sk(M, N, K, gate, num_cu), M, N, K, gate, rms, num_cu, sync_bytes);

@@ -563,3 +563,47 @@ def test_scratch_memory_sized_for_the_tile_gemm_is_accepted(gpu, m, n, k):
         y = ops.w4a16_gemm_fused(ta, tw, ts, rms_gamma=tg, rms_eps=1e-6, residual=tr, workspace=buf[:256], variant="gemv_rows")
         _check(y.cpu().numpy(), ref)
         assert bool((buf[need:] == 0x5A).all())
+
+
+# Tiles of 64 and 128 rows on four wavefronts and on eight: one a CU over odd and even numbers of supersteps, the last one of a
+# single group; parts of few and of many supersteps; more tiles than CUs one by one and in the even split (plan without parts:
+# tiles that workgroups share in the middle); ragged rows and columns
+@pytest.mark.parametrize("m,n,k,rows,parts,cols", [
+    (130, 520, 2176, 128, 1, 128), (65, 130, 2048, 128, 1, 128), (200, 300, 512, 128, 1, 128), (100, 384, 4480, 128, 2, 128),
+    (256, 1000, 1280, 128, 4, 128), (1000, 5000, 512, 128, 1, 128), (1100, 4700, 2176, 128, 0, 128), (40, 3000, 11136, 128, 0, 128),
+    (33, 257, 2432, 64, 1, 128), (64, 640, 2048, 64, 1, 128), (190, 500, 640, 64, 1, 128), (100, 520, 4480, 64, 2, 128),
+    (256, 9000, 2176, 64, 0, 128), (256, 9000, 640, 64, 1, 128), (130, 520, 2176, 128, 1, 256), (100, 1000, 4480, 128, 2, 256),
+    (100, 2700, 2432, 128, 12, 256), (1100, 9000, 1408, 128, 0, 256), (33, 1000, 2176, 64, 1, 256), (64, 3000, 4480, 64, 12, 256),
+    (1, 300, 2176, 128, 1, 128), (1, 300, 2176, 64, 1, 256)])
+def test_four_and_eight_wavefronts(gpu, m, n, k, rows, parts, cols):
+    """Against float32 products of the same values: rounding the weights (times gamma) and the result to fp16 gives 2-norm errors
+    of about 2^-11.5 each, SiLU-gate three such results (1e-3, 2e-3); one and two launches bit for bit."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case M={m} N={n} K={k} tile={rows}x{cols} parts={parts}", flush=True)
+    a, wq, s = datagen.w4a16_case(m + n + k, m, 2 * n, k)
+    gamma = datagen.normal_f16(m, datagen.S_GAMMA, (k,), 1.0, 0.1)
+    res = datagen.normal_f16(m, datagen.S_RES, (m, n))
+    bias = datagen.normal_f16(m, datagen.S_BIAS, (n,))
+    a, wq, s, gamma, res, bias = _t(gpu, a, wq, s, gamma, res, bias)
+    q = torch.stack((wq & 15, wq >> 4), dim=2).reshape(2 * n, k).float() - 8
+    w = q * s.float().repeat_interleave(128, dim=1)
+    x = a.float()
+    xn = x * torch.rsqrt(x.pow(2).mean(dim=1, keepdim=True) + 1e-6) * gamma.float()
+    w1, s1 = wq[:n].contiguous(), s[:n].contiguous()
+    gate, up = (xn @ w.t()).split(n, dim=1)
+    forms = [(wq, s, dict(act=1, rms_gamma=gamma), torch.nn.functional.silu(gate) * up, 2e-3)]
+    if not (rows == 64 and cols == 256):
+        forms += [(w1, s1, {}, x @ w[:n].t(), 1e-3), (w1, s1, dict(rms_gamma=gamma, residual=res), xn @ w[:n].t() + res.float(), 1e-3),
+                  (w1, s1, dict(bias=bias, residual=res), x @ w[:n].t() + bias.float() + res.float(), 1e-3)]
+    sync = ops.sync_flags(gpu)
+    for w_, s_, kw, ref, tol in forms:
+        plan = (rows, parts, 256 if "act" in kw else cols)
+        one = ops.w4a16_gemm_fused(a, w_, s_, variant="gemm_mfma", plan=plan, sync=sync, **kw)
+        two = ops.w4a16_gemm_fused(a, w_, s_, variant="gemm_mfma", plan=plan, **kw)
+        assert torch.equal(one, two)
+        assert float((one.float() - ref).norm() / ref.norm()) <= tol
+        assert float((one.float() - ref).abs().max() / ref.pow(2).mean().sqrt()) <= (2e-2 if "act" in kw else TOL)
+        assert not sync.any()

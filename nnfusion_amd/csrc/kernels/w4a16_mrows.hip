@@ -79,42 +79,28 @@ namespace nnf
         }
     }
 
-    // RMSNorm of the activations in registers as rms_norm_kernel computes it: fp16(x * rstd * gamma), in fp32, one rounding.
-    // Lane (m = col, kq) holds 64 bytes of each of its wavefront's GA groups; gsrc(g): the 64 bytes of gamma that pair with
-    // group g.  sum_sq: [8 wavefronts][MB x 16 rows] of LDS of its own.  (Unlike mrows_scale_a, where rstd joins the sums at the end:
-    // these kernels have no per-group sums to scale, and x * gamma alone may leave the range of fp16.)
-    template <int MB, int GA, class F>
-    __device__ __forceinline__ void mrows_rms_norm(uintx4 (&areg)[MB][GA][4], float* sum_sq, int K, float eps, int wave, int col, int kq,
-                                                   F&& gsrc)
+    // sum a^2 of a lane's 32 values of a group, in fp32, in the order of k
+    __device__ __forceinline__ float sum_of_squares(const uintx4 (&a)[4])
     {
+        float sg = 0.f;
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
+        for (int j = 0; j < 4; ++j)
         {
-            float ss = 0.f;
+            const uint32_t rr[4] = {a[j].x, a[j].y, a[j].z, a[j].w};
 #pragma unroll
-            for (int g = 0; g < GA; ++g)
+            for (int i = 0; i < 4; ++i)
             {
-                float sg = 0.f;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                {
-                    const uint32_t rr[4] = {areg[mb][g][j].x, areg[mb][g][j].y, areg[mb][g][j].z, areg[mb][g][j].w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                    {
-                        const half2_t h = as_half2(rr[i]);
-                        sg = __builtin_fmaf((float)h.x, (float)h.x, sg);
-                        sg = __builtin_fmaf((float)h.y, (float)h.y, sg);
-                    }
-                }
-                ss += sg;
+                const half2_t h = as_half2(rr[i]);
+                sg = __builtin_fmaf((float)h.x, (float)h.x, sg);
+                sg = __builtin_fmaf((float)h.y, (float)h.y, sg);
             }
-            ss += __shfl_xor(ss, 16, 64);
-            ss += __shfl_xor(ss, 32, 64);
-            if (kq == 0)
-                sum_sq[wave * (MB * 16) + mb * 16 + col] = ss;
         }
-        __syncthreads();
+        return sg;
+    }
+    // The second half of mrows_rms_norm: the wavefronts' shares of the rows' sums are in sum_sq.
+    template <int MB, int GA, class F>
+    __device__ __forceinline__ void mrows_normalise(uintx4 (&areg)[MB][GA][4], const float* sum_sq, int K, float eps, int col, F&& gsrc)
+    {
         float rs[MB];
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -147,6 +133,29 @@ namespace nnf
                 }
             }
         }
+    }
+    // RMSNorm of the activations in registers as rms_norm_kernel computes it: fp16(x * rstd * gamma), in fp32, one rounding.
+    // Lane (m = col, kq) holds 64 bytes of each of its wavefront's GA groups; gsrc(g): the 64 bytes of gamma that pair with
+    // group g.  sum_sq: [8 wavefronts][MB x 16 rows] of LDS of its own.  (Unlike mrows_scale_a, where rstd joins the sums at the end:
+    // these kernels have no per-group sums to scale, and x * gamma alone may leave the range of fp16.)
+    template <int MB, int GA, class F>
+    __device__ __forceinline__ void mrows_rms_norm(uintx4 (&areg)[MB][GA][4], float* sum_sq, int K, float eps, int wave, int col, int kq,
+                                                   F&& gsrc)
+    {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+        {
+            float ss = 0.f;
+#pragma unroll
+            for (int g = 0; g < GA; ++g)
+                ss += sum_of_squares(areg[mb][g]);
+            ss += __shfl_xor(ss, 16, 64);
+            ss += __shfl_xor(ss, 32, 64);
+            if (kq == 0)
+                sum_sq[wave * (MB * 16) + mb * 16 + col] = ss;
+        }
+        __syncthreads();
+        mrows_normalise<MB, GA>(areg, sum_sq, K, eps, col, gsrc);
     }
 
     // v of this lane + v of the lane 16 (32) away, the same in both, without the LDS unit: the compiler waits for every LDS-bound
@@ -310,6 +319,38 @@ namespace nnf
                 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[mb][g][j]), cvec, t, 0, 0, 0);
             }
             ncorr[mb][g] = t;
+        });
+    }
+
+    // The same blocks for the kernels of other block parameters: operand registers as they are in memory (NORM) or in the pair order of the
+    // nibble trick; NORM: the lane's share of sum a^2 of its row, in the order in which mrows_rms_norm adds it up.
+    template <int MB, int GA, int RL, bool NORM, int BEHIND, class F>
+    __device__ __forceinline__ void mrows_take_blocks_q(uintx4 (&areg)[MB][GA][4], float& sq, const uint8_t* stage, int col, int kq, F&& fetch)
+    {
+        static_assert(MB == 1 || !NORM, "");
+        constexpr int NP = MB * GA, NF = mrows_blocks_in_flight(NP, RL);
+        const int row = col & (4 * RL - 1);
+        sq = 0.f;
+        unroll_for<0, NP>([&](auto p_c) {
+            constexpr int p = decltype(p_c)::value, mb = p / GA, g = p % GA;
+            // what has been asked for behind this block (vector-memory operations complete in order)
+            constexpr int LATER = RL * ((NF + p < NP ? NF + p : NP) - 1 - p) + (p < NF ? BEHIND : 0);
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(LATER));
+            const uint8_t* block = stage + (p % NF) * (RL * 1024) + row * 256;
+            uintx4 a[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                a[j] = *reinterpret_cast<const uintx4*>(block + (((kq * 4 + j) ^ row) << 4));
+            if constexpr (p + NF < NP)
+            {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the block has been read out of the place that is filled next
+                fetch(std::integral_constant<int, (p + NF < NP ? p + NF : 0)>{});
+            }
+            if constexpr (NORM)
+                sq += sum_of_squares(a);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                areg[mb][g][j] = NORM ? a[j] : permute_a8(a[j]);
         });
     }
 
@@ -622,26 +663,29 @@ namespace nnf
     // loads, NSL of them) and, ZPT, their zero points (one byte per lane, NZL loads; a byte load lands in a lane's four
     // bytes of LDS).
     // LDS (bytes): weights [8 wavefronts][2 slots][GW KiB] | scales and zero points [8][2][(NSL + NZL) x 256] |
-    //              (FUSED where RMSNorm may be inside: sums of squares [8][16] fp32) | partial tiles [2][8][MB KiB] |
+    //              (FUSE == 2: sums of squares [8][16] fp32) | partial tiles [2][8][MB KiB] |
     //              parked sums [tiles of the workgroup][M][16] fp32
-    // pack = M | zp << 8 | gate << 16.
-    // FUSED: RMSNorm ahead of the product (f.gamma), bias / residual or SiLU-gate behind it, as the nodes of their own
+    //              (from the partial tiles on, while the kernel starts: activations [8][8 KiB] | RMSNorm weight [8][1 KiB])
+    // pack = M | zp << 8 | gate << 16; tiles, RL: as in w4a16_mrows_kernel.
+    // FUSE: 0 plain, 1 with the epilogue of `f`, 2 with RMSNorm as well.  RMSNorm ahead of the product (f.gamma), bias / residual or SiLU-gate behind it, as the nodes of their own
     // would compute them.  They were launches of their own (2 - 4 us each at 8 rows, 19 of the 56 us of a decoder layer
     // with groups of 64 and zero points); inside, the prologue runs while the first weights are on their way.  RMSNorm only
     // where workspace::mrows_q_norm_inside says so (every workgroup normalises all the rows for itself: with more groups per
     // wavefront that takes longer than the pass of its own).
-    template <int GW, int GSHIFT, bool ZPT, int MB, bool FUSED>
+    template <int GW, int GSHIFT, bool ZPT, int MB, int FUSE, int RL>
     __global__ __launch_bounds__(512) void w4a16_mrows_q_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
-                                                                const half_t* __restrict__ S, half_t* __restrict__ Y,
-                                                                const uint8_t* __restrict__ zps, int N, int tiles_q,
-                                                                int tiles_r, int pack, GemvFusionArgs f)
+                                                                const half_t* __restrict__ S, const uint8_t* __restrict__ zps,
+                                                                const half_t* gamma, int N, int tiles, int pack, half_t* Y, GemvFusionArgs f)
     {
+        static_assert(RL == 4 || (MB == 1 && RL == 2), "rows of a block");
+        constexpr bool FUSED = FUSE != 0, NORM = FUSE == 2;
+        static_assert(!NORM || (MB == 1 && GW <= 2), "RMSNorm inside");
+        constexpr bool ACTIVATIONS_FIRST = GW < 4 || RL < 4;
         static_assert(GW == 1 || GW == 2 || GW == 4, "K = 2048, 4096, 8192");
         static_assert(GSHIFT >= 5 && GSHIFT <= 7 && ((GW << (7 - GSHIFT)) & 1) == 0, "whole words of scales, whole bytes of zero points");
         static_assert(MB == 1 || (MB == 2 && GW <= 2), "two blocks of rows: 32 VGPRs per group");
         constexpr int STEPS = 2;
         constexpr int K = GW * STEPS * 1024, G = K >> GSHIFT;
-        constexpr bool NORM = FUSED && MB == 1 && GW <= 2;
         constexpr int GA = GW * STEPS;         // groups of 128 of a wavefront
         constexpr int GAMMA_LOADS = (GA + 3) / 4; // of the RMSNorm weight into LDS: 1 KiB, four groups, each
         constexpr int ROW_BYTES = K / 2;       // a weight row
@@ -667,6 +711,7 @@ namespace nnf
         const int col = lane & 15; // n within the tile (B operand / D column), m for the A operand
         const int kq = lane >> 4;  // K quarter of the MFMA operands, row quad of D
         const int M = pack & 0xff, zp = (pack >> 8) & 0xff, gate = FUSED ? (pack >> 16) & 1 : 0;
+        const int tiles_q = tiles & 0xffff, tiles_r = (int)((unsigned)tiles >> 16);
         const int b = blockIdx.x;
         const int t0 = b * tiles_q + min(b, tiles_r);
         const int T_out = tiles_q + (b < tiles_r ? 1 : 0);
@@ -727,81 +772,63 @@ namespace nnf
             }
         };
 
-        issue(0, 0, 0);
-        issue(0, 1, 1);
-        // activations: into the MFMA operand registers (through LDS as whole lines from a few rows on, see
-        // workspace::mrows_stages_activations), then in the pair order of the nibble trick
+        // RMSNorm weight, as many blocks of activations as there is room for, the weights, the rest, in this order: as in w4a16_mrows_kernel.
+        // Nine rows and more of K = 8192, four times as many blocks as there is room for: the weights first (3 % faster).
+        // (With the activations behind the weights, and RMSNorm's weight behind those, groups of 64 with zero points, N = K = 4096: 4 / 8
+        // rows 5.82 / 6.21 us, with a residual 6.18 / 6.31, RMSNorm and SiLU-gate at N = 11008 8 rows 17.2; now 5.09 / 5.40, 5.34 / 5.54, 16.3.)
+        uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
+        const uint8_t* gamma_block = red + MR_WAVES * (2 * ROW_BLOCK_BYTES) + wave * (GAMMA_LOADS * 1024);
+        if constexpr (NORM)
+        {
+#pragma unroll
+            for (int i = 0; i < GAMMA_LOADS; ++i)
+            {
+                const int g = min(4 * i + (lane >> 4), GA - 1);
+                const uint8_t* src = reinterpret_cast<const uint8_t*>(gamma) + wave * (GW * 256) + (g / GW) * (SPAN * 4) + (g % GW) * 256 + (lane & 15) * 16;
+                __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(gamma_block + i * 1024), 16, 0, 0);
+            }
+        }
+        constexpr int NF = mrows_blocks_in_flight(MB * GA, RL);
+        auto fetch = [&](auto p_c) {
+            constexpr int p = decltype(p_c)::value, g = p % GA;
+            mrows_block_fetch<RL>(reinterpret_cast<const uint8_t*>(A), (size_t)K * 2, (p / GA) * 16, M,
+                                  (size_t)((g / GW) * (SPAN * 4) + wave * (GW * 256) + (g % GW) * 256), stage + (p % NF) * (RL * 1024), lane);
+        };
+        if constexpr (!ACTIVATIONS_FIRST)
+        {
+            issue(0, 0, 0);
+            issue(0, 1, 1);
+        }
+        unroll_for<0, NF>([&](auto p_c) { fetch(p_c); });
+        if constexpr (ACTIVATIONS_FIRST)
+        {
+            issue(0, 0, 0);
+            issue(0, 1, 1);
+        }
         uintx4 areg[MB][GA][4];
-        if (MB == 1 && !workspace::mrows_stages_activations(M, K))
+        float sq;
+        mrows_take_blocks_q<MB, GA, RL, NORM, ACTIVATIONS_FIRST ? 2 * LT : 0>(areg, sq, stage, col, kq, fetch);
+        MrowsAhead ahead;
+        if (FUSED && f.residual)
+            mrows_ask_ahead(ahead, f.residual, t0, T_out, M, N, tid);
+        if constexpr (NORM)
         {
-            const uint8_t* a_bytes = reinterpret_cast<const uint8_t*>(A);
-            const uint32_t a_off = (uint32_t)min(col, M - 1) * (uint32_t)(K * 2) + (uint32_t)wave * (GW * 256) + (uint32_t)kq * 64u;
+            const float pair = row_pair_sum(sq), sum = half_pair_sum(pair);
+            if (kq == 0) // (by hand: ahead of an LDS write that it can see, the compiler waits for every LDS-bound load in flight)
+                asm volatile("ds_write_b32 %0, %1" ::"v"(lds_address(sum_sq + wave * 16 + col)), "v"(sum) : "memory");
+        }
+        // (the blocks lay over what holds the partial tiles and the parked sums from here on; the RMSNorm weight over parked sums alone, which are
+        // written behind the first tile's barrier)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (NORM)
+        {
+            mrows_normalise<MB, GA>(areg, sum_sq, K, f.rms_eps, col, [&](int g) { return gamma_block + g * 256 + kq * 64; });
 #pragma unroll
             for (int g = 0; g < GA; ++g)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    areg[0][g][j] = *reinterpret_cast<const uintx4*>(a_bytes + (size_t)(a_off + (g / GW) * (SPAN * 4) + (g % GW) * 256 + j * 16));
-            if (NORM && f.gamma)
-                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [&](int g) {
-                    return reinterpret_cast<const uint8_t*>(f.gamma) + wave * (GW * 256) + kq * 64 + (g / GW) * (SPAN * 4) + (g % GW) * 256;
-                });
+                    areg[0][g][j] = permute_a8(areg[0][g][j]);
         }
-        else
-        {
-            uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
-            constexpr int NP = MB * GA;
-            auto fetch = [&](int p) {
-                const int mb = p / GA, g = p % GA;
-                row_block_fetch(reinterpret_cast<const uint8_t*>(A), (size_t)K * 2, mb * 16, M - 1,
-                                (size_t)((g / GW) * (SPAN * 4) + wave * (GW * 256) + (g % GW) * 256), stage + (p & 1) * ROW_BLOCK_BYTES, lane);
-            };
-            fetch(0);
-#pragma unroll
-            for (int p = 0; p < NP; ++p)
-            {
-                if (p + 1 < NP)
-                {
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // block p-1 has been read out of the half that is filled next
-                    fetch(p + 1);
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
-                }
-                else if (NORM && f.gamma)
-                {
-                    // gamma of the wavefront's k positions into the free half, as in w4a16_mrows_kernel
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-                    for (int i = 0; i < GAMMA_LOADS; ++i)
-                    {
-                        const int g = min(4 * i + (lane >> 4), GA - 1);
-                        const uint8_t* src = reinterpret_cast<const uint8_t*>(f.gamma) + wave * (GW * 256) + (g / GW) * (SPAN * 4) +
-                                             (g % GW) * 256 + (lane & 15) * 16;
-                        __builtin_amdgcn_global_load_lds((mr_global_ptr_t)src, (mr_lds_ptr_t)(stage + (NP & 1) * ROW_BLOCK_BYTES + i * 1024),
-                                                         16, 0, 0);
-                    }
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(GAMMA_LOADS));
-                }
-                else
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    areg[p / GA][p % GA][j] = row_block_piece(stage + (p & 1) * ROW_BLOCK_BYTES, col, kq * 4 + j);
-            }
-            if (NORM && f.gamma)
-            {
-                const uint8_t* gamma_block = stage + (NP & 1) * ROW_BLOCK_BYTES;
-                __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-                mrows_rms_norm<MB, GA>(areg, sum_sq, K, f.rms_eps, wave, col, kq, [&](int g) { return gamma_block + g * 256 + kq * 64; });
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __syncthreads();
-        }
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int g = 0; g < GA; ++g)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    areg[mb][g][j] = permute_a8(areg[mb][g][j]);
 
         // ---- tile loop ---------------------------------------------------------------------------------------
         const uint32_t rd_base = (uint32_t)col * SLICE;
@@ -881,7 +908,7 @@ namespace nnf
         }
         __builtin_amdgcn_s_waitcnt(mr_vmcnt(0)); // the reloads past the end, before the LDS goes away
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate);
+        mrows_flush<FUSED, MB>(parked, Y, t0, T_out, M, N, tid, f, gate, nullptr, FUSED && !f.bias ? &ahead : nullptr);
     }
 
     // ---- 8-bit weights -------------------------------------------------------------------------------------------------
@@ -1783,11 +1810,11 @@ namespace nnf
 
     namespace
     {
-        template <int GW, int GSHIFT, bool ZPT, int MB, bool FUSED>
+        template <int GW, int GSHIFT, bool ZPT, int MB, int FUSE, int RL = 4>
         hipError_t launch_mrows_q_mb(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
                                      const void* zps, int num_cu, const GemvFusion& fusion)
         {
-            if constexpr (((GW << (7 - GSHIFT)) & 1) != 0 || (MB == 2 && GW > 2))
+            if constexpr (((GW << (7 - GSHIFT)) & 1) != 0 || (MB == 2 && GW > 2) || (FUSE == 2 && GW > 2))
                 return hipErrorInvalidValue;
             else
             {
@@ -1795,10 +1822,10 @@ namespace nnf
                 const int grid = n_tiles < num_cu ? n_tiles : num_cu;
                 const int tiles_q = n_tiles / grid, tiles_r = n_tiles % grid;
                 const size_t lds = workspace::w4a16_mrows_q_lds_bytes(GW * 2048, M, (tiles_q + (tiles_r ? 1 : 0)) * (fusion.gate ? 2 : 1),
-                                                                      GSHIFT, ZPT, FUSED);
-                if (lds > MAX_LDS_BYTES)
+                                                                      GSHIFT, ZPT, FUSE != 0);
+                if (lds > MAX_LDS_BYTES || tiles_q > 0xffff || tiles_r > 0xffff)
                     return hipErrorInvalidValue;
-                auto kernel = &w4a16_mrows_q_kernel<GW, GSHIFT, ZPT, MB, FUSED>;
+                auto kernel = &w4a16_mrows_q_kernel<GW, GSHIFT, ZPT, MB, FUSE, RL>;
                 if (lds > 64 * 1024)
                 {
                     static LdsGrant granted;
@@ -1807,20 +1834,30 @@ namespace nnf
                         return e;
                 }
                 hipLaunchKernelGGL(kernel, dim3(grid), dim3(MR_WAVES * 64), lds, stream, (const half_t*)A, (const uint8_t*)Wq,
-                                   (const half_t*)S, (half_t*)Y, (const uint8_t*)zps, N, tiles_q, tiles_r,
-                                   M | (zp << 8) | ((fusion.gate ? 1 : 0) << 16), fusion_args(fusion));
+                                   (const half_t*)S, (const uint8_t*)zps, (const half_t*)fusion.gamma, N, tiles_q | (tiles_r << 16),
+                                   M | (zp << 8) | ((fusion.gate ? 1 : 0) << 16), (half_t*)Y, fusion_args(fusion));
                 return hipGetLastError();
             }
+        }
+        template <int GW, int GSHIFT, bool ZPT, int FUSE>
+        hipError_t launch_mrows_q_rows(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
+                                       const void* zps, int num_cu, const GemvFusion& f)
+        {
+            if (M <= 8)
+                return launch_mrows_q_mb<GW, GSHIFT, ZPT, 1, FUSE, 2>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            if (M <= 16)
+                return launch_mrows_q_mb<GW, GSHIFT, ZPT, 1, FUSE>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            if constexpr (FUSE != 2) // (RMSNorm inside: up to 16 rows)
+                return launch_mrows_q_mb<GW, GSHIFT, ZPT, 2, FUSE>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            return hipErrorInvalidValue;
         }
         template <int GW, int GSHIFT, bool ZPT>
         hipError_t launch_mrows_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int zp,
                                   const void* zps, int num_cu, const GemvFusion& f)
         {
-            if (f.any())
-                return M <= 16 ? launch_mrows_q_mb<GW, GSHIFT, ZPT, 1, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f)
-                               : launch_mrows_q_mb<GW, GSHIFT, ZPT, 2, true>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
-            return M <= 16 ? launch_mrows_q_mb<GW, GSHIFT, ZPT, 1, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f)
-                           : launch_mrows_q_mb<GW, GSHIFT, ZPT, 2, false>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
+            return f.gamma   ? launch_mrows_q_rows<GW, GSHIFT, ZPT, 2>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f)
+                   : f.any() ? launch_mrows_q_rows<GW, GSHIFT, ZPT, 1>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f)
+                             : launch_mrows_q_rows<GW, GSHIFT, ZPT, 0>(stream, A, Wq, S, Y, M, N, zp, zps, num_cu, f);
         }
         template <int GW>
         hipError_t launch_mrows_q_gw(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,

@@ -768,7 +768,10 @@ namespace nnf
             const int loads = (16 * words + 63) / 64;
             const size_t aux = (size_t)(zero_points ? 2 : 1) * loads * 256;
             const size_t mb = M <= 16 ? 1 : 2; // blocks of 16 rows
-            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (fused && M <= 16 && K <= 4096 ? 8 * 64 : 0) + mrows_tail_bytes((size_t)2 * 8 * mb * 1024 + (size_t)tiles * M * 64);
+            // (RMSNorm inside: the wavefronts' sums of squares per row, and 1 KiB of its weight behind the activations while the kernel starts)
+            const bool norm = fused && M <= 16 && K <= 4096;
+            const size_t tail = mrows_tail_bytes((size_t)2 * 8 * mb * 1024 + (size_t)tiles * M * 64), staging = (size_t)8 * (2 * 4096 + 1024);
+            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (norm ? 8 * 64 + (tail > staging ? tail : staging) : tail);
         }
         // (17 .. 32 rows: two blocks of rows in registers, up to K = 4096)
         // fused, gate: with the nodes around the product inside the kernel, N outputs from 2 N weight rows
@@ -1248,7 +1251,9 @@ namespace nnf
                 if (M <= 16)
                 {
                     const bool fixed_k = K == 2048 || K == 4096 || K == 8192;
-                    if (fixed_k ? !rms || (gate && p.tiles > (K == 2048 ? 6 : 4)) : K > 8192 && (N < 4096 || p.tiles > 2))
+                    // (K = 2048: where the row-streaming kernel takes these parameters, five and six tiles take 8 - 16 % less time there; up to four level or more)
+                    const bool few = K != 2048 || w4a16_mrows_q_fits(M, N, K, qg, true, num_cu, true, gate);
+                    if (fixed_k ? !rms || (gate && p.tiles > (few ? 4 : 6)) : K > 8192 && (N < 4096 || p.tiles > 2))
                         continue;
                 }
                 else if (M <= 64)

@@ -316,6 +316,15 @@ def test_fused_rows_equal_the_nodes(gpu, m, n, k, group, zp_tensor):
     close(ops.wna16_gemm_fused(x, t[1], t[2], zero_points=tz, rms_gamma=gamma, rms_eps=1e-5, act=1, **q), gated(normed), 2e-2)
 
 
+# blocks of eight rows and of sixteen on either side of their line, weights ahead of the activations (K = 8192) and behind them; five and
+# six tiles a workgroup with SiLU-gate at K = 2048
+@pytest.mark.parametrize("m,n,k", [(8, 24, 2048), (9, 24, 2048), (8, 520, 4096), (9, 4111, 4096), (8, 520, 8192), (9, 520, 8192), (8, 8224, 2048),
+                                   (15, 12288, 2048)])
+@pytest.mark.parametrize("group,zp_tensor", [(32, True), (64, False), (128, True)])
+def test_fused_rows_in_blocks_of_eight_and_sixteen(gpu, m, n, k, group, zp_tensor):
+    test_fused_rows_equal_the_nodes(gpu, m, n, k, group, zp_tensor)
+
+
 # both sides of the line between RMSNorm ahead of the row-streaming kernels and inside them: rows at K = 4096 (8 and up
 # inside) and at K = 2048 (17 and up ahead); every other K ahead
 @pytest.mark.parametrize("m,n,k", [(7, 1000, 4096), (17, 520, 4096), (32, 4111, 4096), (17, 520, 2048), (2, 1000, 8192), (16, 4111, 8192),

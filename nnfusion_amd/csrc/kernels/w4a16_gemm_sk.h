@@ -319,6 +319,11 @@ namespace nnf
             return off;
         }
         typedef const void __attribute__((address_space(1))) * global_ptr;
+        // (rows of an odd number of groups of 128 begin anywhere: the alignment their scales and zero points have)
+        typedef uintx4 __attribute__((aligned(8))) uintx4_at8;
+        typedef uintx2 __attribute__((aligned(4))) uintx2_at4;
+        typedef uint32_t __attribute__((aligned(2))) uint32_at2;
+        typedef uint16_t __attribute__((aligned(1))) uint16_at1;
         typedef void __attribute__((address_space(3))) * lds_ptr;
         __device__ __forceinline__ void workgroup_barrier()
         {
@@ -641,7 +646,7 @@ namespace nnf
     }
 
     // QG = 0: groups of 128, the zero point p.zp.  QG = 5, 6, 7: groups of 2^QG and, with p.zps, a zero point per
-    // (row, group); K a multiple of 256.  A lane's 32 weights of a K step lie in one group whatever its size: per column
+    // (row, group).  A lane's 32 weights of a K step lie in one group whatever its size: per column
     // tile and superstep it fetches the 256 / group scales of its row in one load (4, 8 or 16 bytes) and the byte(s) that
     // hold their zero points in another (1, 2 or 4 bytes; without p.zps: the scales again, unused) -- six loads per
     // column tile as for QG = 0, on the same schedule -- and keeps a scale and the pair -(1024 + z), -(64 + z) per K step.
@@ -890,7 +895,7 @@ namespace nnf
                 {
                     // the scales of the row's groups of this superstep; their zero points, or (no tensor) the scales again
                     s_off[j] = (uint32_t)(((size_t)gn * G + (size_t)(256 >> GSH) * ss_begin) * 2);
-                    z_off[j] = p.zps ? (uint32_t)((size_t)gn * (G >> 1) + (size_t)(128 >> GSH) * ss_begin) : s_off[j];
+                    z_off[j] = p.zps ? (uint32_t)((size_t)gn * ((G + 1) >> 1) + (size_t)(128 >> GSH) * ss_begin) : s_off[j];
                 }
                 else
                     s_off[j] = (uint32_t)(((size_t)gn * G + 2 * ss_begin) * 2);
@@ -911,16 +916,20 @@ namespace nnf
                 const uint8_t *w, *s_lo, *s_hi;
                 uint32_t repeat; // 64: the second 64 bytes of the superstep do not exist
             };
+            auto superstep_is_whole = [&](int s) { return (ss_begin + s) * 256 + 128 < K; };
             auto w_base_of = [&](int s) {
                 s = segment_ss(s);
                 WBase b;
                 if constexpr (QZ)
                 {
-                    // (K is a multiple of 256)  s_lo: the scales; s_hi: the zero points, or the scales again
+                    // s_lo: the scales; s_hi: the zero points, or the scales again.  A superstep of 128 k: from half a superstep before
+                    // (groups of 128: the byte holds its zero point all the same), so that nothing is read past the end of a row
+                    const bool whole = superstep_is_whole(s);
                     b.w = scalar_base(p.Wq + (size_t)s * 128);
-                    b.repeat = 0u;
-                    b.s_lo = scalar_base(s_bytes + (size_t)s * (512 >> GSH));
-                    b.s_hi = p.zps ? scalar_base(p.zps + (size_t)s * (128 >> GSH)) : b.s_lo;
+                    b.repeat = whole ? 0u : 64u;
+                    const int k0 = min((ss_begin + s) * 256, K - 256) - ss_begin * 256; // (a select by `whole` instead does not compile)
+                    b.s_lo = scalar_base(s_bytes + (ptrdiff_t)(k0 >> GSH) * 2);
+                    b.s_hi = p.zps ? scalar_base(p.zps + (QG == 7 ? (ptrdiff_t)s : (ptrdiff_t)(k0 >> (GSH + 1)))) : b.s_lo;
                     return b;
                 }
                 const bool second_valid = 2 * (ss_begin + s) + 1 < G;
@@ -962,23 +971,23 @@ namespace nnf
                 {
                     if constexpr (QG == 5)
                     {
-                        const uintx4 v = *(const uintx4 __attribute__((address_space(1)))*)(b.s_lo + here(s_off[j]));
+                        const uintx4 v = *(const uintx4_at8 __attribute__((address_space(1)))*)(b.s_lo + here(s_off[j]));
                         sraw[set][j][0] = v.x, sraw[set][j][1] = v.y, sraw[set][j][2] = v.z, sraw[set][j][3] = v.w;
                     }
                     else if constexpr (QG == 6)
                     {
-                        const uintx2 v = *(const uintx2 __attribute__((address_space(1)))*)(b.s_lo + here(s_off[j]));
+                        const uintx2 v = *(const uintx2_at4 __attribute__((address_space(1)))*)(b.s_lo + here(s_off[j]));
                         sraw[set][j][0] = v.x, sraw[set][j][1] = v.y;
                     }
                     else
-                        sraw[set][j][0] = *(const uint32_t __attribute__((address_space(1)))*)(b.s_lo + here(s_off[j]));
+                        sraw[set][j][0] = *(const uint32_at2 __attribute__((address_space(1)))*)(b.s_lo + here(s_off[j]));
                 }
                 else
                 {
                     if constexpr (QG == 5)
-                        zraw[set][j] = *(const uint32_t __attribute__((address_space(1)))*)(b.s_hi + here(z_off[j]));
+                        zraw[set][j] = *(const uint32_at2 __attribute__((address_space(1)))*)(b.s_hi + here(z_off[j]));
                     else if constexpr (QG == 6)
-                        zraw[set][j] = *(const uint16_t __attribute__((address_space(1)))*)(b.s_hi + here(z_off[j]));
+                        zraw[set][j] = *(const uint16_at1 __attribute__((address_space(1)))*)(b.s_hi + here(z_off[j]));
                     else
                         zraw[set][j] = *(const uint8_t __attribute__((address_space(1)))*)(b.s_hi + here(z_off[j]));
                 }
@@ -991,26 +1000,39 @@ namespace nnf
                 constexpr int set = decltype(set_c)::value;
                 if constexpr (QZ)
                 {
+                    // (half a superstep: its scales and zero points are the second half of what was loaded, and zero follows)
+                    const bool whole = superstep_is_whole(segment_ss(s));
+                    constexpr int REGS = SW;
+                    const uint32_t keep = whole ? 0xffffffffu : 0u, s_shift = whole ? 0u : 16u, z_shift = whole ? 0u : QG == 5 ? 16u : 8u;
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
+                    {
+                        uint32_t words[REGS];
+#pragma unroll
+                        for (int i = 0; i < REGS; ++i)
+                            words[i] = REGS == 1       ? sraw[set][j][0] >> s_shift
+                                       : i < REGS / 2 ? (sraw[set][j][i] & keep) | (sraw[set][j][i + REGS / 2] & ~keep)
+                                                      : sraw[set][j][i] & keep;
+                        const uint32_t zeros = QG == 7 ? zraw[set][j] : zraw[set][j] >> z_shift;
 #pragma unroll
                         for (int i = 0; i < NSC; ++i)
                         {
                             uint32_t sv, z;
                             if constexpr (QG == 5)
                             {
-                                sv = __builtin_amdgcn_perm(sraw[set][j][i], sraw[set][j][i], h_sel);
-                                z = zraw[set][j] >> (uint32_t)(8 * i + 4 * h);
+                                sv = __builtin_amdgcn_perm(words[i], words[i], h_sel);
+                                z = zeros >> (uint32_t)(8 * i + 4 * h);
                             }
                             else
                             {
-                                sv = __builtin_amdgcn_perm(sraw[set][j][i >> 1], sraw[set][j][i >> 1], (i & 1) ? 0x03020302u : 0x01000100u);
-                                z = zraw[set][j] >> (uint32_t)(4 * i);
+                                sv = __builtin_amdgcn_perm(words[i >> 1], words[i >> 1], (i & 1) ? 0x03020302u : 0x01000100u);
+                                z = zeros >> (uint32_t)(4 * i);
                             }
                             z = (z & z_and) | z_or;
                             sc[set][j][i] = as_half2(sv);
                             dq[set][j][i] = as_half2((z | (z << 20)) | 0xD400E400u);
                         }
+                    }
                     return;
                 }
                 s = segment_ss(s);

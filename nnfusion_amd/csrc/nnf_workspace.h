@@ -853,10 +853,15 @@ namespace nnf
             return p;
         }
         // The tile GEMM with other block parameters (groups of 32 / 64 / 128, zero points per (row, group)): above 16 rows,
-        // K a multiple of 256 (the kernel addresses its operands with 32-bit byte offsets); the plain product, same plan
+        // K a multiple of 128 (the kernel addresses its operands with 32-bit byte offsets); the plain product, same plan.
+        // Odd multiples, whose last superstep of 256 is half work for nothing, where it is ahead of the plain tile kernel (900 products, time there / here):
+        // K = 384 0.87, 640 0.95, 896 1.04, from 1152 on 1.1 - 1.5 (1000 x 4096 x 4224 in groups of 32 56.2 -> 40.5 us, 2000 rows 92.5 -> 67.4),
+        // but above 1600 rows 0.92 at 1152 / 1408, 1.03 up to 1920; few columns 0.8 - 0.97 at short K, and with few rows too at long (185 x 320 x 15232).
         inline bool w4a16_gemm_q_fits(int M, int N, int K, int group_shift)
         {
-            return M > 16 && N >= 1 && K >= 256 && !(K & 255) && group_shift >= 5 && group_shift <= 7 &&
+            if ((K & 128) && (K < (M > 1600 || N < 768 ? 2176 : 1152) || (N < 512 && M <= 256)))
+                return false;
+            return M > 16 && N >= 1 && K >= 256 && !(K & 127) && group_shift >= 5 && group_shift <= 7 &&
                    (size_t)M * K * 2 + 8192 < ((size_t)1 << 32) && (size_t)N * (K >> 1) < ((size_t)1 << 32);
         }
         // ---- the plain tile kernel (wna16_generic.hip): tile shape and ranges of K ------------------------------------------

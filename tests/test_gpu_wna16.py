@@ -212,6 +212,34 @@ def test_products_beyond_the_k_streaming_kernel(gpu, m, n, k, bits, group, zp_te
     _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
 
 
+# the tile GEMM on odd multiples of 128: a last superstep of half the weights, whose scales and zero points end with the row (the last
+# row: with the tensor); every height of its tiles, parts of K that end with it, the shortest K; two that stay on the plain kernel
+@pytest.mark.parametrize("m,n,k", [(1000, 1030, 1152), (520, 300, 2176), (530, 700, 4224), (130, 520, 11136), (40, 9000, 8320), (70, 513, 8320),
+                                   (1700, 2048, 2176), (2600, 2500, 2176), (900, 767, 1152), (256, 300, 6272)])
+@pytest.mark.parametrize("group,zp_tensor", [(32, True), (64, True), (128, True), (32, False), (64, False)])
+def test_tile_gemm_on_odd_multiples_of_128(gpu, m, n, k, group, zp_tensor):
+    """Against float32 products of the dequantised weights; 2-norm of the roundings of weights and result to fp16 about 4e-4 (1e-3)."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case M={m} N={n} K={k} group={group} zero points={zp_tensor}", flush=True)
+    a, wq, s, zps = _case(m + n + k + group, m, n, k, 4, group, zp_tensor)
+    a, wq, s = [torch.from_numpy(x).to(gpu) for x in (a, wq, s)]
+    q = torch.stack((wq & 15, wq >> 4), dim=2).reshape(n, k).float()
+    z = 5.0
+    if zp_tensor:
+        zt = torch.from_numpy(zps).to(gpu)
+        z = torch.stack((zt & 15, zt >> 4), dim=2).reshape(n, -1)[:, :k // group].float().repeat_interleave(group, dim=1)
+    ref = a.float() @ ((q - z) * s.float().repeat_interleave(group, dim=1)).t()
+    sync = ops.sync_flags(gpu)
+    par = dict(bits=4, group=group, zp=5, zero_points=zt if zp_tensor else None)
+    for y in (ops.wna16_gemm(a, wq, s, **par), ops.wna16_gemm(a, wq, s, sync=sync, **par)):
+        assert float((y.float() - ref).norm() / ref.norm()) <= 1e-3
+        assert float((y.float() - ref).abs().max() / ref.pow(2).mean().sqrt()) <= 1e-2
+    assert not sync.any()
+
+
 def test_default_parameters_are_the_specialised_kernels(gpu):
     import torch
 

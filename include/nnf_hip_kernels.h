@@ -194,9 +194,10 @@ NNF_API int nnf_w4a16_gemm_variant(nnf_stream_t stream,
  * those apply: the K-streaming kernel for 2 .. 512 rows where it was measured ahead (no workspace; 8-bit weights too), else
  * the row-streaming kernels for M = 1 with K a multiple of 256 from 1024 to 16384 and for 2 <= M <= 16
  * with K a multiple of 256 from about 2560 on (2048 / 4096 also up to 32 rows, where the K-streaming kernel is not ahead or has no room for the
- * columns; above K = 8192 over ranges of K with a reduction pass), and the tile GEMM for the other shapes above 16 rows with K a multiple of 256 (of 128 from about 1152 on) and zero_points
+ * columns; above K = 8192 over ranges of K with a reduction pass), and the tile GEMM for the other shapes above 16 rows with K a multiple of 256 and zero_points
  * 4-byte aligned.  The ranges of K and the tile GEMM want nnf_wna16_gemm_workspace_bytes of workspace; called with
  * less (or NULL) the product runs on a plain kernel instead, at about half the rate.
+ * Odd multiples of 128 from about 1152 on run on the tile GEMM as well, given nnf_wna16_gemm_preferred_workspace_bytes.
  * Everything else runs on plain kernels that need no workspace: a row-per-wavefront GEMV for M = 1, an MFMA kernel
  * with the operands fetched straight into registers for 2 <= M <= 16, MFMA tiles through LDS above (over ranges of K where
  * nnf_wna16_gemm_preferred_workspace_bytes says so and the caller brings them). */
@@ -211,8 +212,9 @@ typedef struct nnf_quant
 NNF_API int nnf_wna16_supported(int M, int N, int K, const nnf_quant* q);
 NNF_API size_t nnf_wna16_gemm_workspace_bytes(int M, int N, int K, const nnf_quant* q);
 /* At least that: the bytes with which nnf_wna16_gemm runs fastest.  More where the tile kernel behind products without a
- * specialised one (8-bit weights, K no multiple of 128 or a short odd one; above 16 rows) leaves CUs idle and can work on ranges of K instead,
- * whose fp32 sums it keeps there; given less it runs as many ranges as fit, or one. */
+ * specialised one (8-bit weights, K no multiple of 256; above 16 rows) leaves CUs idle and can work on ranges of K instead,
+ * whose fp32 sums it keeps there; given less it runs as many ranges as fit, or one.  And where the tile GEMM takes 4-bit weights on an
+ * odd multiple of 128: its parked tiles. */
 NNF_API size_t nnf_wna16_gemm_preferred_workspace_bytes(int M, int N, int K, const nnf_quant* q);
 NNF_API int nnf_wna16_gemm(nnf_stream_t stream,
                    const void* A, const void* Wq, const void* scales, void* Y,

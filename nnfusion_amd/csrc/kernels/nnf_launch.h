@@ -168,7 +168,7 @@ namespace nnf
                                          int M, int N, int K, int zp, int ksplits, int num_cu);
 
     // the tile GEMM for groups of 2^group_shift = 32 / 64 / 128 and a scalar zero point or (zero_points != null) one per
-    // (row, group): M > 16, workspace::w4a16_gemm_q_fits; partial_ws: workspace::wna16_gemm bytes (0: not needed)
+    // (row, group): M > 16, workspace::w4a16_gemm_q_fits or _odd_fits; partial_ws: workspace::plan_w4a16_sk bytes (0: not needed)
     bool w4a16_gemm_q_supported(int M, int N, int K, int group_shift);
     hipError_t launch_w4a16_gemm_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                    int K, int group_shift, int zp, const void* zero_points, void* partial_ws, int num_cu,

@@ -548,7 +548,10 @@ namespace nnf
     }
 
     // ---- the tile GEMM with other block parameters ----------------------------------------------------------------------
-    bool w4a16_gemm_q_supported(int M, int N, int K, int group_shift) { return workspace::w4a16_gemm_q_fits(M, N, K, group_shift); }
+    bool w4a16_gemm_q_supported(int M, int N, int K, int group_shift) 
+    {
+        return workspace::w4a16_gemm_q_fits(M, N, K, group_shift) || workspace::w4a16_gemm_q_odd_fits(M, N, K, group_shift);
+    }
     hipError_t launch_w4a16_gemm_q(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N,
                                    int K, int group_shift, int zp, const void* zero_points, void* partial_ws, int num_cu,
                                    const LaunchChoice& choice)

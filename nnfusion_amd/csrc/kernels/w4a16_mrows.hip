@@ -1822,7 +1822,7 @@ namespace nnf
                 const int grid = n_tiles < num_cu ? n_tiles : num_cu;
                 const int tiles_q = n_tiles / grid, tiles_r = n_tiles % grid;
                 const size_t lds = workspace::w4a16_mrows_q_lds_bytes(GW * 2048, M, (tiles_q + (tiles_r ? 1 : 0)) * (fusion.gate ? 2 : 1),
-                                                                      GSHIFT, ZPT, FUSE != 0);
+                                                                      GSHIFT, ZPT, FUSE != 0, FUSE == 2);
                 if (lds > MAX_LDS_BYTES || tiles_q > 0xffff || tiles_r > 0xffff)
                     return hipErrorInvalidValue;
                 auto kernel = &w4a16_mrows_q_kernel<GW, GSHIFT, ZPT, MB, FUSE, RL>;

@@ -361,7 +361,8 @@ int nnf_wna16_gemm_planned(nnf_stream_t stream, const void* A, const void* Wq, c
         !nnf::w4a16_mrows_q_supported(M, N, K, group_shift_of(q->group), q->zero_points != nullptr, dev.num_cu) &&
         (reinterpret_cast<uintptr_t>(q->zero_points) & 3) == 0)
     {
-        const size_t need = nnf::workspace::wna16_gemm(M, N, K, q->bits, q->group, dev.num_cu);
+        const size_t need = (K & 255) ? nnf::workspace::plan_w4a16_sk(M, N, K, false, dev.num_cu).bytes()
+                                      : nnf::workspace::wna16_gemm(M, N, K, q->bits, q->group, dev.num_cu);
         if (need == 0 || (workspace && aligned16(workspace) && workspace_bytes >= need))
             return (int)nnf::launch_w4a16_gemm_q((hipStream_t)stream, A, Wq, scales, Y, M, N, K, group_shift_of(q->group),
                                                  q->zero_point, q->zero_points, workspace, dev.num_cu, choice);

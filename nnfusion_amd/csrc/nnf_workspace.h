@@ -761,17 +761,16 @@ namespace nnf
         // K = 3072 / 3584 0.88 - 1.00, 0.92 - 1.01; K = 4608 / 5120 0.76 - 0.96, 0.80 - 0.97; K = 8192 0.70 - 0.91, 0.78 - 0.95.
         constexpr bool mrows_q_norm_inside(int M, int K) { return M <= 16 && (K == 2048 || (K == 4096 && mrows_stages_activations(M, K))); }
         // (fused: with room for the wavefronts' sums of squares per row, at the sizes that may have RMSNorm inside)
-        inline size_t w4a16_mrows_q_lds_bytes(int K, int M, int tiles, int group_shift, bool zero_points, bool fused = false)
+        // norm: with RMSNorm inside, 1 KiB of its weight per wavefront behind the activations while the kernel starts (at most 72 KiB beside 41: always room)
+        inline size_t w4a16_mrows_q_lds_bytes(int K, int M, int tiles, int group_shift, bool zero_points, bool fused = false, bool norm = false)
         {
             const int gw = K >> 11;
             const int words = (gw << (7 - group_shift)) / 2; // of scales per row, step and wavefront
             const int loads = (16 * words + 63) / 64;
             const size_t aux = (size_t)(zero_points ? 2 : 1) * loads * 256;
             const size_t mb = M <= 16 ? 1 : 2; // blocks of 16 rows
-            // (RMSNorm inside: the wavefronts' sums of squares per row, and 1 KiB of its weight behind the activations while the kernel starts)
-            const bool norm = fused && M <= 16 && K <= 4096;
             const size_t tail = mrows_tail_bytes((size_t)2 * 8 * mb * 1024 + (size_t)tiles * M * 64), staging = (size_t)8 * (2 * 4096 + 1024);
-            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (norm ? 8 * 64 + (tail > staging ? tail : staging) : tail);
+            return (size_t)8 * 2 * gw * 1024 + 8 * 2 * aux + (fused && M <= 16 && K <= 4096 ? 8 * 64 : 0) + (norm && tail < staging ? staging : tail);
         }
         // (17 .. 32 rows: two blocks of rows in registers, up to K = 4096)
         // fused, gate: with the nodes around the product inside the kernel, N outputs from 2 N weight rows
@@ -853,16 +852,23 @@ namespace nnf
             return p;
         }
         // The tile GEMM with other block parameters (groups of 32 / 64 / 128, zero points per (row, group)): above 16 rows,
-        // K a multiple of 128 (the kernel addresses its operands with 32-bit byte offsets); the plain product, same plan.
-        // Odd multiples, whose last superstep of 256 is half work for nothing, where it is ahead of the plain tile kernel (900 products, time there / here):
-        // K = 384 0.87, 640 0.95, 896 1.04, from 1152 on 1.1 - 1.5 (1000 x 4096 x 4224 in groups of 32 56.2 -> 40.5 us, 2000 rows 92.5 -> 67.4),
-        // but above 1600 rows 0.92 at 1152 / 1408, 1.03 up to 1920; few columns 0.8 - 0.97 at short K, and with few rows too at long (185 x 320 x 15232).
+        // K a multiple of 256 (the kernel addresses its operands with 32-bit byte offsets); the plain product, same plan
+        inline bool w4a16_gemm_q_addressable(int M, int N, int K, int group_shift)
+        {
+            return M > 16 && N >= 1 && K >= 256 && group_shift >= 5 && group_shift <= 7 && (size_t)M * K * 2 + 8192 < ((size_t)1 << 32) &&
+                   (size_t)N * (K >> 1) < ((size_t)1 << 32);
+        }
         inline bool w4a16_gemm_q_fits(int M, int N, int K, int group_shift)
         {
-            if ((K & 128) && (K < (M > 1600 || N < 768 ? 2176 : 1152) || (N < 512 && M <= 256)))
-                return false;
-            return M > 16 && N >= 1 && K >= 256 && !(K & 127) && group_shift >= 5 && group_shift <= 7 &&
-                   (size_t)M * K * 2 + 8192 < ((size_t)1 << 32) && (size_t)N * (K >> 1) < ((size_t)1 << 32);
+            return !(K & 255) && w4a16_gemm_q_addressable(M, N, K, group_shift);
+        }
+        // ... and on odd multiples of 128, whose last superstep of 256 is half work for nothing, given scratch memory that is preferred and not needed
+        // (plan_w4a16_sk: what parked tiles may take), where it is ahead of the plain tile kernel.  900 products, time there / here:
+        // K = 384 0.87, 640 0.95, 896 1.04, from 1152 on 1.1 - 1.5 (1000 x 4096 x 4224 in groups of 32 56.2 -> 41 us, 2000 rows 92.5 -> 68),
+        // but above 1600 rows 0.92 at 1152 / 1408, 1.03 up to 1920; few columns 0.8 - 0.97 at short K, and with few rows too at long (185 x 320 x 15232).
+        inline bool w4a16_gemm_q_odd_fits(int M, int N, int K, int group_shift)
+        {
+            return (K & 255) == 128 && K >= (M > 1600 || N < 768 ? 2176 : 1152) && (N >= 512 || M > 256) && w4a16_gemm_q_addressable(M, N, K, group_shift);
         }
         // ---- the plain tile kernel (wna16_generic.hip): tile shape and ranges of K ------------------------------------------
         // One range: the tile shape with the lowest time of a K step of 64 on a busy chip: 256 x 256 (0) 2.0 us a round of
@@ -952,6 +958,11 @@ namespace nnf
         {
             const size_t needed = wna16_gemm(M, N, K, bits, group, num_cu);
             const int gs = group == 32 ? 5 : group == 64 ? 6 : group == 128 ? 7 : 0;
+            if (bits == 4 && w4a16_gemm_q_odd_fits(M, N, K, gs))
+            {
+                const size_t parked = plan_w4a16_sk(M, N, K, false, num_cu).bytes();
+                return parked > needed ? parked : needed;
+            }
             if (gs == 0 || (bits != 4 && bits != 8) || (bits == 4 && w4a16_gemm_q_fits(M, N, K, gs)) ||
                 !wna16_on_tile_kernel(M, N, K, bits, gs, num_cu))
                 return needed;

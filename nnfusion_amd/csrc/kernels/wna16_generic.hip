@@ -85,8 +85,9 @@ namespace nnf
     // grid: any; each wavefront walks blocks of R consecutive rows (R x its number, + R x the number of wavefronts, ...);
     // a lane takes 16 bytes of each of the R rows per pass over K (32 or 16 weights, inside one group): the sum of
     // a x (q - z) over them (v_dot2_f32_f16 on exact operands) times the group's scale is added to the lane's fp32 sums.
-    // The activations a lane meets are fetched once per pass for all R rows.  MB: upper bound of M.
-    template <int BITS, int R, int MB>
+    // The activations a lane meets are fetched once per pass for all R rows.  MB: upper bound of M.  AHEAD: a pass is asked for
+    // while the one before it is added up: without, every pass is a wait for its zero points, scales and weights.
+    template <int BITS, int R, int MB, bool AHEAD>
     __global__ __launch_bounds__(256) void wna16_gemv_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                              const half_t* __restrict__ S, half_t* __restrict__ Y, int M, int N,
                                                              int K, QuantArgs qa)
@@ -108,19 +109,37 @@ namespace nnf
                 for (int m = 0; m < MB; ++m)
                     acc[m][r] = 0.f;
             }
-            for (int k = lane * WPL; k < K; k += 64 * WPL)
+            // what a pass needs, as it arrives
+            struct Operands
             {
-                const int g = k >> qa.group_shift;
-                uintx4 w[R];
-                float sc[R];
+                uintx4 w[R], a[MB][WPL / 8];
+                half_t s[R];
                 int z[R];
+            };
+            auto fetch = [&](int k, Operands& o) {
+                const int g = k >> qa.group_shift;
 #pragma unroll
                 for (int r = 0; r < R; ++r)
                 {
-                    w[r] = *reinterpret_cast<const uintx4*>(Wq + (size_t)row[r] * row_bytes + (size_t)k * BITS / 8);
-                    z[r] = zero_point_of<BITS>(qa, row[r], g);
-                    sc[r] = (float)S[(size_t)row[r] * G + g];
+                    o.w[r] = *reinterpret_cast<const uintx4*>(Wq + (size_t)row[r] * row_bytes + (size_t)k * BITS / 8);
+                    o.z[r] = zero_point_of<BITS>(qa, row[r], g);
+                    o.s[r] = S[(size_t)row[r] * G + g];
                 }
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int p = 0; p < WPL / 8; ++p)
+                        o.a[m][p] = *reinterpret_cast<const uintx4*>(A + (size_t)min(m, M - 1) * K + k + 8 * p);
+            };
+            Operands cur, nxt;
+            if (AHEAD && lane * WPL < K)
+                fetch(lane * WPL, cur);
+            for (int k = lane * WPL; k < K; k += 64 * WPL)
+            {
+                if constexpr (!AHEAD)
+                    fetch(k, cur);
+                else if (k + 64 * WPL < K)
+                    fetch(k + 64 * WPL, nxt);
                 float part[MB][R];
 #pragma unroll
                 for (int m = 0; m < MB; ++m)
@@ -134,17 +153,17 @@ namespace nnf
 #pragma unroll
                     for (int r = 0; r < R; ++r)
                     {
-                        const ExactWeights<BITS> exact(z[r]);
+                        const ExactWeights<BITS> exact(cur.z[r]);
                         if constexpr (BITS == 4)
-                            exact(w[r][p], 0u, v[r]);
+                            exact(cur.w[r][p], 0u, v[r]);
                         else
-                            exact(w[r][2 * p], w[r][2 * p + 1], v[r]);
+                            exact(cur.w[r][2 * p], cur.w[r][2 * p + 1], v[r]);
                     }
 #pragma unroll
                     for (int m = 0; m < MB; ++m)
                         if (m < M)
                         {
-                            uintx4 a = *reinterpret_cast<const uintx4*>(A + (size_t)m * K + k + 8 * p);
+                            uintx4 a = cur.a[m][p];
                             if constexpr (BITS == 4)
                                 a = permute_a8(a);
 #pragma unroll
@@ -158,7 +177,9 @@ namespace nnf
                 for (int m = 0; m < MB; ++m)
 #pragma unroll
                     for (int r = 0; r < R; ++r)
-                        acc[m][r] = __builtin_fmaf(part[m][r], sc[r], acc[m][r]);
+                        acc[m][r] = __builtin_fmaf(part[m][r], (float)cur.s[r], acc[m][r]);
+                if constexpr (AHEAD)
+                    cur = nxt;
             }
 #pragma unroll
             for (int m = 0; m < MB; ++m)
@@ -175,13 +196,13 @@ namespace nnf
         }
     }
 
-    template <int BITS, int R, int MB>
+    template <int BITS, int R, int MB, bool AHEAD>
     void launch_wna16_gemv(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
                            const QuantArgs& qa, int num_cu)
     {
         // enough wavefronts to cover the blocks of rows once, at most eight workgroups of four per CU
         const int want = (N + 4 * R - 1) / (4 * R), cap = num_cu * 8;
-        hipLaunchKernelGGL((wna16_gemv_kernel<BITS, R, MB>), dim3((unsigned)(want < cap ? want : cap)), dim3(256), 0, stream,
+        hipLaunchKernelGGL((wna16_gemv_kernel<BITS, R, MB, AHEAD>), dim3((unsigned)(want < cap ? want : cap)), dim3(256), 0, stream,
                            (const half_t*)A, (const uint8_t*)Wq, (const half_t*)S, (half_t*)Y, M, N, K, qa);
     }
 
@@ -678,10 +699,15 @@ namespace nnf
                 // rows the row-streaming kernel can walk: that kernel
                 if (w4a16_gemv_rows_q_supported(1, N, K, qa.group_shift, zero_points != nullptr, num_cu, bits))
                     return launch_w4a16_gemv_rows_q(stream, A, Wq, S, Y, N, K, qa.group_shift, zp, zero_points, num_cu, bits);
-                if (bits == 4)
-                    launch_wna16_gemv<4, 4, 1>(stream, A, Wq, S, Y, M, N, K, qa, num_cu);
+                // Fewer than 32 rows a CU: one a wavefront, so that all SIMDs have some, and a pass ahead; four, which share their activations,
+                // otherwise.  N = 4096 with groups of 32 and zero points, K = 4224 / 8320 / 11136 9.1 / 16.3 / 22.3 -> 7.4 / 10.7 / 12.6 us,
+                // 1024 x 1152 4.6 -> 2.9; two rows and a pass ahead 0.88 x at 11008 x 2176, four 0.76 at 16384.
+                if (N < 32 * num_cu)
+                    bits == 4 ? launch_wna16_gemv<4, 1, 1, true>(stream, A, Wq, S, Y, M, N, K, qa, num_cu)
+                              : launch_wna16_gemv<8, 1, 1, true>(stream, A, Wq, S, Y, M, N, K, qa, num_cu);
                 else
-                    launch_wna16_gemv<8, 4, 1>(stream, A, Wq, S, Y, M, N, K, qa, num_cu);
+                    bits == 4 ? launch_wna16_gemv<4, 4, 1, false>(stream, A, Wq, S, Y, M, N, K, qa, num_cu)
+                              : launch_wna16_gemv<8, 4, 1, false>(stream, A, Wq, S, Y, M, N, K, qa, num_cu);
                 return hipGetLastError();
             }
             // blocks of two tiles of 16 rows, at most four workgroups per CU

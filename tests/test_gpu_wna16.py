@@ -212,6 +212,15 @@ def test_products_beyond_the_k_streaming_kernel(gpu, m, n, k, bits, group, zp_te
     _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
 
 
+# one row on the plain GEMV: fewer rows than wavefronts, either side of 32 a CU, a pass of a few lanes, one pass and many
+@pytest.mark.parametrize("n,k", [(1, 128), (33, 384), (1000, 1152), (4096, 2176), (8191, 640), (8192, 640), (300, 16512)])
+@pytest.mark.parametrize("bits,group,zp_tensor", [(4, 32, True), (4, 64, False), (8, 32, True), (8, 128, False)])
+def test_one_row_on_the_plain_kernel(gpu, n, k, bits, group, zp_tensor):
+    a, wq, s, zps = _case(n + k + bits + group, 1, n, k, bits, group, zp_tensor)
+    zp = 7 if bits == 4 else 131
+    _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
+
+
 # the tile GEMM on odd multiples of 128: a last superstep of half the weights, whose scales and zero points end with the row (the last
 # row: with the tensor); every height of its tiles, parts of K that end with it, the shortest K; two that stay on the plain kernel
 @pytest.mark.parametrize("m,n,k", [(1000, 1030, 1152), (520, 300, 2176), (530, 700, 4224), (130, 520, 11136), (40, 9000, 8320), (70, 513, 8320),

@@ -268,23 +268,28 @@ namespace nnf
         // Only the weights asked for above may still be in flight afterwards: the scales have landed too.
         __builtin_amdgcn_s_waitcnt(rows_vmcnt(D0 * LPR));
         NNF_ROWS_STAMP(1); // activations and scales have arrived
-        // (Every instruction here is time between the activations' arrival and the first row: sums and sum of squares on
-        // v_dot2_f32_f16, 0.2 us less with RMSNorm than conversions, adds and a run-time choice among the gamma registers.)
+        // (Sums and squares in fp32 additions, each rounded once: v_dot2_f32_f16 loses low bits of the smaller of its two products -- one
+        // in twelve sums of two squares is an ulp off -- and takes no less time, 16 launches of a decoder stack 109.4 us against 109.7.)
         float ss = 0.f;
         if (a_loader)
         {
-            // -(1024 + zp) and -(64 + zp) twice, as bits (exact: ulps of 1 and 1/16)
-            const uint32_t z = QZT ? 0u : (uint32_t)zp;
-            const uint32_t ce_bits = (0xE400u | z) * 0x10001u, co_bits = W8 ? ce_bits : (0xD400u | (z << 4)) * 0x10001u;
-            const half2_t ce = as_half2(ce_bits), co = as_half2(co_bits), one = {(half_t)1.0f, (half_t)1.0f};
+            const float ce = -(1024.0f + (QZT ? 0.f : (float)zp));
+            const float co = W8 ? ce : -(64.0f + (QZT ? 0.f : (float)zp));
             auto prepare = [&](int u, const uintx4& g) {
                 uintx4 raw = act[u];
                 if (own_rstd)
                 {
                     // RMSNorm without a pass of its own: every unit of the row goes through exactly one lane here
-                    const float sq = dot2(as_half2(raw.x), as_half2(raw.x), dot2(as_half2(raw.y), as_half2(raw.y), 0.f)) +
-                                     dot2(as_half2(raw.z), as_half2(raw.z), dot2(as_half2(raw.w), as_half2(raw.w), 0.f));
-                    ss += u < a_units ? sq : 0.f;
+                    if (u < a_units)
+                    {
+                        const uint32_t rr[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                        {
+                            const half2_t hh = as_half2(rr[i]);
+                            ss += (float)hh.x * (float)hh.x + (float)hh.y * (float)hh.y;
+                        }
+                    }
                 }
                 if (EPI != 0 && f.gamma)
                 {
@@ -296,10 +301,12 @@ namespace nnf
                 }
                 const uintx4 a = W8 ? raw : permute_a8(raw);
                 const half2_t x = as_half2(a.x), y = as_half2(a.y), z = as_half2(a.z), w = as_half2(a.w);
+                const float se = ((float)x.x + (float)x.y) + ((float)z.x + (float)z.y);
+                const float so = ((float)y.x + (float)y.y) + ((float)w.x + (float)w.y);
                 act[u] = a;
-                corr[u] = dot2(x, ce, dot2(z, ce, 0.f)) + dot2(y, co, dot2(w, co, 0.f));
+                corr[u] = ce * se + co * so;
                 if (QZT)
-                    asum_u[u] = dot2(x, one, dot2(z, one, 0.f)) + dot2(y, one, dot2(w, one, 0.f));
+                    asum_u[u] = se + so;
             };
             if constexpr (GQ > 1)
                 static_for<0, GQ>([&](auto ec) {

@@ -208,3 +208,48 @@ def test_mfma_gemv_adds_bias_and_residual_as_the_nodes_do(gpu, m, n, k):
     y = res.clone()
     ops.w4a16_gemm_fused(*t, residual=y, out=y)
     assert torch.equal(y, ops.elementwise("add", plain, res))
+
+
+def test_one_row_constants_of_cancelling_activations_cancel(gpu):
+    """Weights of 0 with a zero point of 15, a unit of eight activations of which b + c - b - c remains: 0.  The products with 1024 + 0
+    are exact, so that only the rounding of the unit's constant, -(1024 + 15) x (its even activations), could be left over."""
+    k, n = 4096, 128
+    rng = np.random.default_rng(5)
+    a = np.zeros((1, k), np.float16)
+    for u in range(0, k // 8, 4):
+        b, c = np.float16(rng.uniform(1, 2)), np.float16(rng.uniform(1, 2) * 2.0 ** -int(rng.integers(8, 13)))
+        a[0, 8 * u:8 * u + 8] = [b, 0, -b, 0, c, 0, -c, 0]
+        if u % 8:
+            a[0, 8 * u:8 * u + 8] = [0, b, 0, -b, 0, c, 0, -c]
+    wq = np.zeros((n, k // 2), np.uint8)
+    s = np.ones((n, k // 128), np.float16)
+    assert not _run(gpu, a, wq, s, zp=15, path="rows_gemv").any()
+
+
+@pytest.mark.parametrize("seed", range(24))
+def test_one_row_rms_norm_adds_squares_in_fp32(gpu, seed):
+    """The sum of squares of eight activations: one pair after the other added to it, each sum rounded once to fp32.  An epsilon that leaves 256
+    ulps of the mean shows its last bit: a bit off is 2e-3 of the results, whose rounding to fp16 is 5e-4 (1 / sqrt and a scale in fp32 beside it:
+    5.1e-4 allowed).  RMSNorm's weight picks out eight other activations, of 1 / 32: whole numbers times a scale, without rounding."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    k, n = 1024, 256
+    rng = np.random.default_rng(seed)
+    unit = (rng.uniform(1, 2, 8) * 2.0 ** rng.integers(-6, 5, 8)).astype(np.float16)
+    at, ones = 8 * rng.permutation(k // 8)[:2]
+    a, gamma = np.zeros((1, k), np.float16), np.zeros(k, np.float16)
+    a[0, at:at + 8], a[0, ones:ones + 8], gamma[ones:ones + 8] = unit, 1 / 32, 1
+    total = np.float32(0)
+    for x, y in unit.astype(np.float32).reshape(4, 2):
+        total = total + (x * x + y * y)  # (both squares are exact)
+    mean = (total + np.float32(8 / 1024)) / np.float32(k)
+    left = 256 * np.spacing(mean)
+    wq = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    s = rng.uniform(0.005, 0.02, (n, k // 128)).astype(np.float16)
+    q = wq[:, ones // 2:ones // 2 + 4]
+    ref = ((q & 15) + (q >> 4)).sum(axis=1) / 32 * s[:, ones // 128].astype(np.float64) / np.sqrt(float(left))
+    t = [torch.from_numpy(x).to(gpu) for x in (a, wq, s, gamma)]
+    y = ops.w4a16_gemm_fused(*t[:3], zp=0, rms_gamma=t[3], rms_eps=float(left - mean), variant="gemv_rows").cpu().numpy()
+    assert (np.abs(y[0] - ref) <= 5.1e-4 * ref).all()

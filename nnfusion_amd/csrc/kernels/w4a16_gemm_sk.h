@@ -330,6 +330,9 @@ namespace nnf
             asm volatile("s_barrier" ::: "memory");
         }
 
+        // what stands in for activations and RMSNorm weights past K (a lane reads sixteen or four bytes of it)
+        static __device__ const uint8_t sk_zeros[16] __attribute__((aligned(16))) = {};
+
         // regions per quarter and fragments per region
         constexpr int regions_of(int TM) { return TM < 4 ? TM : 4; }
 
@@ -648,9 +651,11 @@ namespace nnf
     // QG = 0: groups of 128, the zero point p.zp.  QG = 5, 6, 7: groups of 2^QG and, with p.zps, a zero point per
     // (row, group).  A lane's 32 weights of a K step lie in one group whatever its size: per column
     // tile and superstep it fetches the 256 / group scales of its row in one load (4, 8 or 16 bytes) and the byte(s) that
-    // hold their zero points in another (1, 2 or 4 bytes; without p.zps: the scales again, unused) -- six loads per
-    // column tile as for QG = 0, on the same schedule -- and keeps a scale and the pair -(1024 + z), -(64 + z) per K step.
-    template <int TM, int TN, int NW, int KH, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0>
+    // hold their zero points in another (1, 2 or 4 bytes; without p.zps: the scales again, masked out) and keeps a scale
+    // and the pair -(1024 + z), -(64 + z) per K step.
+    // ODD: K is an odd multiple of 128, whose last superstep has half the weights.  An instantiation of its own: with what that takes
+    // inside every kernel, 200 products on even multiples took 1.0 - 2.0 % longer (4096 x 8192 x 8192 446.7 us against 441.4).
+    template <int TM, int TN, int NW, int KH, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0, bool ODD = false>
     __global__ __launch_bounds__(NW * KH * 64, 1) void w4a16_gemm_sk_kernel(const half_t* __restrict__ A_first,
                                                                    const uint8_t* __restrict__ Wq_first,
                                                                    const half_t* __restrict__ S_first, long long units_first,
@@ -672,9 +677,9 @@ namespace nnf
         p.supersteps = supersteps_first;
         using namespace gemm_sk;
         using T = Tile<TM, TN, NW, KH>;
-        // loads per column tile and superstep: four of weights; two of scales and zero points, or (the specialised kernel)
-        // three of scales, see load_w
-        constexpr int WL = QG != 0 ? 6 : 7;
+        // loads per column tile and superstep, every one of them used (the wait counts rely on it): four of weights; two of scales and
+        // zero points, or (groups of 128, a scalar zero point) one of both scales, ODD two of one each, see load_w
+        constexpr int WL = QG != 0 || ODD ? 6 : 5;
         constexpr int AL = T::A_LOADS;
         using SCH = Sched<AL, TN, RMS, WL>;
         static_assert(!(GATE && (BIAS || RESID)), "SiLU-gate is not combined with bias or residual");
@@ -683,7 +688,7 @@ namespace nnf
         constexpr bool QZ = QG != 0;
         constexpr int GSH = QZ ? QG : 7;                    // log2 of the group size
         constexpr int NSC = QZ ? (QG == 7 ? 2 : 4) : 2;     // scales a lane keeps per column tile and superstep
-        constexpr int SW = QZ ? (QG == 5 ? 4 : QG == 6 ? 2 : 1) : 3; // registers of scales as loaded
+        constexpr int SW = QG == 5 ? 4 : QG == 6 || (QG == 0 && ODD) ? 2 : 1; // registers of scales as loaded
         constexpr int BM = T::BM, BN = T::BN;
         constexpr int A_TILE_BYTES = T::A_TILE_BYTES, STAGE_BYTES = T::STAGE_BYTES;
         constexpr int BN_OUT = GATE ? BN / 2 : BN;
@@ -707,7 +712,6 @@ namespace nnf
         const int strip_tid = KH > 1 ? strip * 64 + lane : tid;
         const int K = p.K;
         const int G = K >> GSH;
-        const bool g_even = !(G & 1);
         const int SS = p.supersteps;
         const int grid = grid_first; // = gridDim.x
         const uint32_t lds0 = lds_address(smem);
@@ -824,7 +828,8 @@ namespace nnf
             // segment's KH s + kh, its K step kt likewise (clamped to the last ones inside the segment)
             const int my_ss = KH > 1 ? (NSS - kh + KH - 1) / KH : NSS;
             auto segment_ss = [&](int s) { return min(KH * s + kh, NSS - 1); };
-            auto segment_kt = [&](int kt) { return min(KH > 1 ? 4 * (KH * (kt >> 2) + kh) + (kt & 3) : kt, kt_max); };
+            auto unclamped_kt = [&](int kt) { return KH > 1 ? 4 * (KH * (kt >> 2) + kh) + (kt & 3) : kt; };
+            auto segment_kt = [&](int kt) { return min(unclamped_kt(kt), kt_max); };
 
             // ---- activations: direct-load map ------------------------------------------------------------------
             // chunk c fills LDS rows c*8 .. +7; lane l lands at (row = c*8 + l/8, slot = l%8) and therefore
@@ -841,17 +846,35 @@ namespace nnf
             const uint8_t* a_bytes = reinterpret_cast<const uint8_t*>(p.A);
             const uint8_t* g_bytes = reinterpret_cast<const uint8_t*>(p.gamma) + (size_t)k_begin * 2;
             const uint32_t g_off = (uint32_t)(lane & 31) * 4u;
-            // scalar base of K step kt (clamped to the last inside K: past it a valid tile goes to a free stage, or is
-            // multiplied by weights of zero)
-            auto a_base_of = [&](int kt) { return scalar_base(a_bytes + (size_t)segment_kt(kt) * (BK * 2)); };
-            auto g_base_of = [&](int kt) { return scalar_base(g_bytes + (size_t)segment_kt(kt) * (BK * 2)); };
-            // activation load i of a K step -> stage
-            auto load_a = [&](auto i_c, const uint8_t* a_base, uint32_t stage_off) {
-                constexpr int i = decltype(i_c)::value;
-                __builtin_amdgcn_global_load_lds((global_ptr)(a_base + here(a_off[i])), (lds_ptr)(smem + stage_off + lds_a + i * 1024), 16, 0, 0);
+            // Scalar base of K step kt (clamped to the last inside K: past it a valid tile goes to a free stage) and which bits of the lanes'
+            // offsets count.  ODD: steps 2 and 3 of a superstep may lie past K and are worked on all the same, with weights of zero: zeros for
+            // them, since an infinity in their place would make NaN: 0.6 % of 190 products' time.  (Loop left in the middle instead: 2 KiB of
+            // registers spilled under the 256 x 256 tile.)
+            struct KBase
+            {
+                const uint8_t* at;
+                uint32_t lanes;
             };
-            auto load_gamma = [&](const uint8_t* g_base, uint32_t stage_off) {
-                __builtin_amdgcn_global_load_lds((global_ptr)(g_base + here(g_off)), (lds_ptr)(smem + stage_off + lds_g), 4, 0, 0);
+            auto base_of = [&](const uint8_t* bytes, auto type_c, int kt) {
+                const uint8_t* in_k = bytes + (size_t)segment_kt(kt) * (BK * 2);
+                if constexpr (!ODD || decltype(type_c)::value < 2)
+                    return KBase{scalar_base(in_k), ~0u};
+                else
+                {
+                    const bool inside = unclamped_kt(kt) <= kt_max;
+                    return KBase{scalar_base(inside ? in_k : sk_zeros), inside ? ~0u : 0u};
+                }
+            };
+            // type_c: the step's place in its superstep
+            auto a_base_of = [&](auto type_c, int kt) { return base_of(a_bytes, type_c, kt); };
+            auto g_base_of = [&](auto type_c, int kt) { return base_of(g_bytes, type_c, kt); };
+            // activation load i of a K step -> stage
+            auto load_a = [&](auto i_c, const KBase& b, uint32_t stage_off) {
+                constexpr int i = decltype(i_c)::value;
+                __builtin_amdgcn_global_load_lds((global_ptr)(b.at + (here(a_off[i]) & b.lanes)), (lds_ptr)(smem + stage_off + lds_a + i * 1024), 16, 0, 0);
+            };
+            auto load_gamma = [&](const KBase& b, uint32_t stage_off) {
+                __builtin_amdgcn_global_load_lds((global_ptr)(b.at + (here(g_off) & b.lanes)), (lds_ptr)(smem + stage_off + lds_g), 4, 0, 0);
             };
 
             // ---- weights and scales ----------------------------------------------------------------------------------
@@ -916,7 +939,7 @@ namespace nnf
                 const uint8_t *w, *s_lo, *s_hi;
                 uint32_t repeat; // 64: the second 64 bytes of the superstep do not exist
             };
-            auto superstep_is_whole = [&](int s) { return (ss_begin + s) * 256 + 128 < K; };
+            auto superstep_is_whole = [&](int s) { return !ODD || (ss_begin + s) * 256 + 128 < K; };
             auto w_base_of = [&](int s) {
                 s = segment_ss(s);
                 WBase b;
@@ -927,12 +950,12 @@ namespace nnf
                     const bool whole = superstep_is_whole(s);
                     b.w = scalar_base(p.Wq + (size_t)s * 128);
                     b.repeat = whole ? 0u : 64u;
-                    const int k0 = min((ss_begin + s) * 256, K - 256) - ss_begin * 256; // (a select by `whole` instead does not compile)
+                    const int k0 = ODD ? min((ss_begin + s) * 256, K - 256) - ss_begin * 256 : s * 256; // (a select by `whole` instead does not compile)
                     b.s_lo = scalar_base(s_bytes + (ptrdiff_t)(k0 >> GSH) * 2);
                     b.s_hi = p.zps ? scalar_base(p.zps + (QG == 7 ? (ptrdiff_t)s : (ptrdiff_t)(k0 >> (GSH + 1)))) : b.s_lo;
                     return b;
                 }
-                const bool second_valid = 2 * (ss_begin + s) + 1 < G;
+                const bool second_valid = superstep_is_whole(s);
                 b.w = scalar_base(p.Wq + (size_t)s * 128);
                 b.repeat = second_valid ? 0u : 64u;
                 b.s_lo = scalar_base(s_bytes + (size_t)s * 4);
@@ -940,7 +963,7 @@ namespace nnf
                 return b;
             };
             // load x of column tile j.  0 .. 3: rows 8 x .. 8 x + 7 of its weights -> the wavefront's area in LDS;
-            // 4 .. 5: scales -> register set
+            // 4, 5: scales and zero points -> register set
             auto load_w = [&](auto set_c, auto j_c, auto x_c, const WBase& b) {
                 constexpr int set = decltype(set_c)::value, j = decltype(j_c)::value, x = decltype(x_c)::value;
                 if constexpr (x < 4 && W_LDS)
@@ -953,19 +976,13 @@ namespace nnf
                     wbuf[set][j][x] = *(const uintx4 __attribute__((address_space(1)))*)(b.w + (x * 32 - (x >= 2 ? b.repeat : 0u)) + here(w_off[j][0]));
                 else if constexpr (!QZ)
                 {
-                    // Loads 4 .. 6, the superstep's two scales of the lane's row.  A load costs by the lines it touches
-                    // (32 rows here).  An even number of groups per row (K a multiple of 256): the two are one aligned
-                    // word, load 4 brings it and loads 5 and 6 ask for the same two bytes in every lane (one line).
-                    // An odd number: load 4 is the one that asks for one line, loads 5 and 6 bring a scale each.
-                    // (One sequence of instructions for both: a branch around a load made the compiler drain every
-                    // load in flight.)
+                    // The superstep's two scales of the lane's row.  A load costs by the lines it touches (32 rows here): one aligned word
+                    // where rows have an even number of them, otherwise loads 4 and 5 bring a scale each.
                     const uint32_t mine = here(s_off[j]);
-                    if constexpr (x == 4)
-                        sraw[set][j][2] = *(const uint32_t __attribute__((address_space(1)))*)(b.s_lo + (g_even ? mine : 0u));
-                    else if constexpr (x == 5)
-                        sraw[set][j][0] = *(const uint16_t __attribute__((address_space(1)))*)(b.s_lo + (g_even ? 0u : mine));
+                    if constexpr (!ODD)
+                        sraw[set][j][0] = *(const uint32_t __attribute__((address_space(1)))*)(b.s_lo + mine);
                     else
-                        sraw[set][j][1] = *(const uint16_t __attribute__((address_space(1)))*)((g_even ? b.s_lo : b.s_hi) + (g_even ? 0u : mine));
+                        sraw[set][j][x - 4] = *(const uint16_t __attribute__((address_space(1)))*)((x == 4 ? b.s_lo : b.s_hi) + mine);
                 }
                 else if constexpr (x == 4)
                 {
@@ -1036,14 +1053,13 @@ namespace nnf
                     return;
                 }
                 s = segment_ss(s);
-                const bool second_valid = 2 * (ss_begin + s) + 1 < G;
+                const bool second_valid = superstep_is_whole(s);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
                 {
-                    const uint32_t first = g_even ? sraw[set][j][2] : sraw[set][j][0];
-                    const uint32_t second = g_even ? sraw[set][j][2] : sraw[set][j][1];
+                    const uint32_t first = sraw[set][j][0], second = sraw[set][j][ODD ? 1 : 0];
                     sc[set][j][0] = as_half2(__builtin_amdgcn_perm(first, first, 0x01000100u));
-                    sc[set][j][1] = as_half2(second_valid ? __builtin_amdgcn_perm(second, second, g_even ? 0x03020302u : 0x01000100u) : 0u);
+                    sc[set][j][1] = as_half2(second_valid ? __builtin_amdgcn_perm(second, second, ODD ? 0x01000100u : 0x03020302u) : 0u);
                 }
             };
 
@@ -1093,9 +1109,9 @@ namespace nnf
                 const int kt = 4 * s + T_;
                 // loads of this step: positions 1 .. 3 of the activations of step kt+2 (-> the stage of step kt-1),
                 // position 0 of step kt+3 (-> this step's stage), weights of superstep s+1
-                const uint8_t* a_late = a_base_of(kt + 2);
-                const uint8_t* a_next = a_base_of(kt + 3);
-                const uint8_t* g_next = RMS ? g_base_of(kt + 3) : nullptr;
+                const KBase a_late = a_base_of(std::integral_constant<int, (T_ + 2) & 3>{}, kt + 2);
+                const KBase a_next = a_base_of(std::integral_constant<int, (T_ + 3) & 3>{}, kt + 3);
+                const KBase g_next = RMS ? g_base_of(std::integral_constant<int, (T_ + 3) & 3>{}, kt + 3) : KBase{nullptr, 0u};
                 const WBase w_next = w_base_of(s + 1);
                 unroll_for<0, 4>([&](auto q_c) {
                     constexpr int Q = decltype(q_c)::value;
@@ -1253,19 +1269,19 @@ namespace nnf
                 // steps 0 and 1 and superstep 0 in full, of step 2 what quarter 3 of a step before the first would
                 // have asked for
                 const WBase w0 = w_base_of(0);
-                unroll_for<0, AL>([&](auto i_c) { load_a(i_c, a_base_of(0), 0u); });
+                unroll_for<0, AL>([&](auto i_c) { load_a(i_c, a_base_of(I0{}, 0), 0u); });
                 unroll_for<0, TN>([&](auto j_c) { unroll_for<0, WL>([&](auto x_c) { load_w(I0{}, j_c, x_c, w0); }); });
                 if constexpr (RMS)
-                    load_gamma(g_base_of(0), 0u);
-                unroll_for<0, AL>([&](auto i_c) { load_a(i_c, a_base_of(1), (uint32_t)STAGE_BYTES); });
+                    load_gamma(g_base_of(I0{}, 0), 0u);
+                unroll_for<0, AL>([&](auto i_c) { load_a(i_c, a_base_of(I1{}, 1), (uint32_t)STAGE_BYTES); });
                 if constexpr (RMS)
-                    load_gamma(g_base_of(1), (uint32_t)STAGE_BYTES);
+                    load_gamma(g_base_of(I1{}, 1), (uint32_t)STAGE_BYTES);
                 unroll_for<0, AL>([&](auto i_c) {
                     if constexpr (SCH::a_pos(decltype(i_c)::value) == 0)
-                        load_a(i_c, a_base_of(2), (uint32_t)(2 * STAGE_BYTES));
+                        load_a(i_c, a_base_of(I2{}, 2), (uint32_t)(2 * STAGE_BYTES));
                 });
                 if constexpr (RMS)
-                    load_gamma(g_base_of(2), (uint32_t)(2 * STAGE_BYTES));
+                    load_gamma(g_base_of(I2{}, 2), (uint32_t)(2 * STAGE_BYTES));
             }
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(SCH::a_loads_total() + SCH::a_loads_at(0))); // step 0 and superstep 0 have landed
             workgroup_barrier();

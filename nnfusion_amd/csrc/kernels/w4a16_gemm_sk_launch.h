@@ -9,10 +9,10 @@ namespace nnf
 {
     namespace gemm_sk
     {
-        template <class T, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0>
-        hipError_t launch_instance(hipStream_t stream, const SkGemmParams& p, int grid)
+        template <class T, bool GATE, bool BIAS, bool RESID, bool RMS, int QG, bool ODD>
+        hipError_t launch_product(hipStream_t stream, const SkGemmParams& p, int grid)
         {
-            auto kernel = &w4a16_gemm_sk_kernel<T::TM, T::TN, T::NW, T::KH, GATE, BIAS, RESID, RMS, QG>;
+            auto kernel = &w4a16_gemm_sk_kernel<T::TM, T::TN, T::NW, T::KH, GATE, BIAS, RESID, RMS, QG, ODD>;
             if (T::LDS_BYTES > 48 * 1024)
             {
                 static LdsGrant granted;
@@ -21,7 +21,14 @@ namespace nnf
                     return e;
             }
             launch_sk_kernel<T>(kernel, grid, stream, p);
-            hipError_t e = hipGetLastError();
+            return hipGetLastError();
+        }
+
+        template <class T, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0>
+        hipError_t launch_instance(hipStream_t stream, const SkGemmParams& p, int grid)
+        {
+            const hipError_t e = (p.K & 128) ? launch_product<T, GATE, BIAS, RESID, RMS, QG, true>(stream, p, grid)
+                                             : launch_product<T, GATE, BIAS, RESID, RMS, QG, false>(stream, p, grid);
             if (e != hipSuccess || !p.partial || p.sync)
                 return e;
             // tiles shared by several workgroups: their parts are added and finished by a second launch (unless the

@@ -249,6 +249,48 @@ def test_tile_gemm_on_odd_multiples_of_128(gpu, m, n, k, group, zp_tensor):
     assert not sync.any()
 
 
+# (128, False): the kernel of groups of 128 with a scalar zero point, by name
+@pytest.mark.parametrize("m,n,k", [(1000, 1030, 1152), (520, 300, 2176), (17, 12479, 8320), (99, 8405, 1152), (260, 11121, 1152), (387, 8291, 1152),
+                                   (523, 13487, 1152)])
+@pytest.mark.parametrize("group,zp_tensor", [(32, True), (64, False), (128, True), (128, False)])
+def test_infinities_at_the_end_of_odd_multiples_of_128(gpu, m, n, k, group, zp_tensor):
+    """Infinite activations in the last K step of the tile GEMM: infinities of the sign that the sum over K has, NaN where a weight is 0 or
+    two of them cancel; other rows as without them.  So with an infinity in RMSNorm's weight, in every row."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case infinities M={m} N={n} K={k} group={group} zero points={zp_tensor}", flush=True)
+    a, wq, s, zps = _case(m + n + k + group, m, n, k, 4, group, zp_tensor)
+    bad = a.copy()
+    bad[1, k - 1], bad[2, k - 64], bad[m - 1, k - 1], bad[m - 1, k - 2] = np.inf, -np.inf, np.inf, -np.inf
+    ta, tb, tw, ts = [torch.from_numpy(x).to(gpu) for x in (a, bad, wq, s)]
+    q = torch.stack((tw & 15, tw >> 4), dim=2).reshape(n, k)
+    tz = torch.from_numpy(zps).to(gpu) if zp_tensor else None
+    z = 5 if tz is None else torch.stack((tz & 15, tz >> 4), dim=2).reshape(n, -1)[:, :k // group].repeat_interleave(group, dim=1).int()
+    sign = (q.int() - z).sign().float()
+
+    def same(y, ref):
+        assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isposinf(), ref.isposinf()) and torch.equal(y.isneginf(), ref.isneginf())
+
+    forms = [dict(), dict(sync=ops.sync_flags(gpu))]
+    for kw in forms:
+        if (group, zp_tensor) == (128, False):
+            run = lambda x, **more: ops.w4a16_gemm_fused(x, tw, ts, zp=5, variant="gemm_mfma", **kw, **more)
+        else:
+            run = lambda x: ops.wna16_gemm(x, tw, ts, bits=4, group=group, zp=5, zero_points=tz, **kw)
+        y, clean = run(tb), run(ta)
+        rows = [r for r in range(m) if r not in (1, 2, m - 1)]
+        assert torch.equal(y[rows], clean[rows]) and bool(clean.isfinite().all())
+        same(y[1], float("inf") * sign[:, k - 1])
+        same(y[2], -float("inf") * sign[:, k - 64])
+        same(y[m - 1], float("inf") * sign[:, k - 1] - float("inf") * sign[:, k - 2])
+        if (group, zp_tensor) == (128, False):
+            gamma = torch.ones(k, dtype=torch.float16, device=gpu)
+            gamma[k - 1] = float("inf")
+            same(run(ta, rms_gamma=gamma), float("inf") * ta[:, k - 1:].sign().float() * sign[:, k - 1])
+
+
 def test_default_parameters_are_the_specialised_kernels(gpu):
     import torch
 

@@ -389,8 +389,12 @@ namespace nnf
         // read twice as often by the 256-wide ones, costs more than it hides.  3000 products on every tile and number of parts, start /
         // this in the geometric mean: 128 x 128 tiles, one a CU, shares of 2 / 4 / 8 / 16 / 32 supersteps 0.93 / 1.02 / 1.11 / 1.17 / 1.23 (with
         // RMSNorm 1.31 on few CUs, where rstd[] of many rows a workgroup takes half as long), more tiles than CUs 0.75 - 0.94; parts of
-        // 1 / 2 / 4 / 8 / 16: 0.92 / 0.95 / 1.02 / 1.09 / 1.16 up to half of the CUs, 0.92 / 0.89 / 0.90 / 0.98 / 1.05 above three quarters; 128 x 256
+        // 1 / 2 / 4 / 8 / 16: 0.92 / 0.95 / 1.02 / 1.09 / 1.16 up to half of the CUs, 0.92 / 0.89 / 0.90 / 0.98 / 1.05 above three quarters; the even
+        // split of more tiles than workgroups 0.94 / 0.97 / 1.02 / 1.03 / 1.03 (of fewer tiles 0.87 - 1.0, left on four); 128 x 256
         // one a CU 1.2 (few, short) .. 0.99 (220 and more, from 32 on), parts 1.10 .. 1.02, from three quarters of the CUs on 0.96 - 1.0.
+        // The faster kernel takes power from its neighbours.  70 products of 128 x 128 tiles on 193 .. 255 CUs from eight supersteps on, by themselves
+        // 1.047, with pauses 1.039, behind 64 x 4096 x 4096 1.039, behind the product that leads back to their K 1.035, each for the whole
+        // sequence; behind two of M x 11008 x 4096 0.997 (0.93 .. 1.05).
         inline bool sk_eight_wavefronts(const SkPlan& p, bool gate, bool rms, int num_cu)
         {
             if ((p.tile_rows != 64 && p.tile_rows != 128) || p.grid < 1)
@@ -401,10 +405,6 @@ namespace nnf
                 return true;
             if (p.tile_weight_rows == 128)
             {
-                // (128 rows on more than three quarters of the CUs: 3 - 5 % faster by itself, but the chip's power goes with it: 1000 x 4096 x
-                // 11008 in groups of 32 behind two products of 1000 x 11008 x 4096 100.2 -> 96.7 us, and those 98.7 -> 103.3 each)
-                if (one_each && p.tile_rows == 128 && !rms && 4ll * p.grid > 3ll * num_cu)
-                    return false;
                 if (one_each)
                     return p.grid <= num_cu && (share >= 8 || (share >= 4 && 8ll * p.grid <= 5ll * num_cu));
                 if (parts)

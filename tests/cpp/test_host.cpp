@@ -1439,6 +1439,14 @@ int main(int argc, char** argv)
                 EXPECT(ws::w4a16_mrows_q_fits(s[0], s[1], s[2], 5, true, 256) == (s[0] <= 32 && s[2] >= 2048));
                 EXPECT((s[0] == 70) == (ws::kstream_choice_b8(s[0], s[1], s[2], 5, 256, false, false, false, true).tiles > 0));
             }
+            // eight wavefronts on whole 128 x 128 tiles near the full chip too
+            const int nearly_full[][3] = {{1000, 4096, 11008}, {1744, 1792, 3072}, {256, 15488, 4096}};
+            for (const auto& s : nearly_full)
+            {
+                const ws::SkPlan p = ws::plan_w4a16_tiles_q(s[0], s[1], s[2], 256, 0);
+                EXPECT(p.tile_rows == 128 && p.tile_weight_rows == 128 && p.grid > 192 && p.grid == p.tiles_m * p.tiles_n);
+                EXPECT(ws::sk_eight_wavefronts(p, false, false, 256));
+            }
             // by itself the library runs no W8A8 product over two ranges of K on the row-streaming kernel: the K-streaming kernel takes them all
             for (int m = 2; m <= 32; ++m)
                 for (int k = 8192; k <= 16384; k += 512)

@@ -1447,6 +1447,28 @@ int main(int argc, char** argv)
                 EXPECT(p.tile_rows == 128 && p.tile_weight_rows == 128 && p.grid > 192 && p.grid == p.tiles_m * p.tiles_n);
                 EXPECT(ws::sk_eight_wavefronts(p, false, false, 256));
             }
+            // the test of its odd multiples of 128: tile, wavefronts and split of every case, with and without synchronisation words
+            enum { WHOLE, PARTS, EVEN };
+            const int odd[][7] = {{17, 12479, 8320, 32, 256, 0, PARTS}, {18, 12368, 10368, 32, 256, 0, EVEN},
+                                  {34, 8407, 12160, 64, 128, 1, PARTS}, {99, 8405, 1152, 64, 128, 1, WHOLE},
+                                  {65, 528, 6272, 64, 128, 0, PARTS}, {37, 8202, 8832, 64, 128, 0, EVEN},
+                                  {65, 11910, 8320, 128, 128, 1, PARTS}, {526, 803, 1152, 128, 128, 1, WHOLE},
+                                  {65, 512, 7040, 128, 128, 0, PARTS}, {132, 10994, 1152, 128, 128, 0, WHOLE},
+                                  {1287, 12013, 1152, 128, 256, 1, EVEN}, {260, 11121, 1152, 128, 256, 1, WHOLE},
+                                  {65, 11184, 6784, 128, 256, 0, PARTS}, {261, 3746, 11392, 128, 256, 0, EVEN},
+                                  {387, 8291, 1152, 256, 128, 0, WHOLE}, {2060, 269, 2176, 256, 128, 0, PARTS},
+                                  {523, 13487, 1152, 256, 256, 0, WHOLE}, {135, 11914, 11136, 256, 256, 0, PARTS},
+                                  {1566, 10194, 2432, 256, 256, 0, EVEN}};
+            for (const auto& s : odd)
+                for (int gs = 5; gs <= 7; ++gs)
+                    for (size_t sync : {(size_t)0, (size_t)64 << 10})
+                    {
+                        const ws::SkPlan p = ws::plan_w4a16_tiles_q(s[0], s[1], s[2], 256, sync);
+                        const int tiles = p.tiles_m * p.tiles_n, split = p.grid == tiles ? WHOLE : p.grid > tiles && p.grid % tiles == 0 ? PARTS : EVEN;
+                        EXPECT(ws::w4a16_gemm_q_odd_fits(s[0], s[1], s[2], gs) && ws::kstream_choice_q(s[0], s[1], s[2], gs, 256, false, false).tiles == 0);
+                        EXPECT(p.tile_rows == s[3] && p.tile_weight_rows == s[4] && split == s[6]);
+                        EXPECT(ws::sk_eight_wavefronts(p, false, false, 256) == (s[5] != 0));
+                    }
             // by itself the library runs no W8A8 product over two ranges of K on the row-streaming kernel: the K-streaming kernel takes them all
             for (int m = 2; m <= 32; ++m)
                 for (int k = 8192; k <= 16384; k += 512)

@@ -222,7 +222,7 @@ def test_one_row_on_the_plain_kernel(gpu, n, k, bits, group, zp_tensor):
 
 
 # the tile GEMM on odd multiples of 128: a last superstep of half the weights, whose scales and zero points end with the row (the last
-# row: with the tensor); every height of its tiles, parts of K that end with it, the shortest K; two that stay on the plain kernel
+# row: with the tensor); tiles of 128 x 128, 64 x 128 and 256 x 128, parts of K that end with it, the shortest K; two that stay on the plain kernel
 @pytest.mark.parametrize("m,n,k", [(1000, 1030, 1152), (520, 300, 2176), (530, 700, 4224), (130, 520, 11136), (40, 9000, 8320), (70, 513, 8320),
                                    (1700, 2048, 2176), (2600, 2500, 2176), (900, 767, 1152), (256, 300, 6272)])
 @pytest.mark.parametrize("group,zp_tensor", [(32, True), (64, True), (128, True), (32, False), (64, False)])
@@ -247,6 +247,17 @@ def test_tile_gemm_on_odd_multiples_of_128(gpu, m, n, k, group, zp_tensor):
         assert float((y.float() - ref).norm() / ref.norm()) <= 1e-3
         assert float((y.float() - ref).abs().max() / ref.pow(2).mean().sqrt()) <= 1e-2
     assert not sync.any()
+
+
+# ... every shape of its tiles, on four wavefronts and on eight, whole, in parts of K and in the even split (tests/cpp/test_host.cpp holds the plan to that)
+@pytest.mark.parametrize("m,n,k", [(17, 12479, 8320), (18, 12368, 10368), (34, 8407, 12160), (99, 8405, 1152), (65, 528, 6272),
+                                  (37, 8202, 8832), (65, 11910, 8320), (526, 803, 1152), (65, 512, 7040), (132, 10994, 1152),
+                                  (1287, 12013, 1152), (260, 11121, 1152), (65, 11184, 6784), (261, 3746, 11392),
+                                  (387, 8291, 1152), (2060, 269, 2176), (523, 13487, 1152), (135, 11914, 11136),
+                                  (1566, 10194, 2432)])
+@pytest.mark.parametrize("group,zp_tensor", [(32, True), (64, False), (128, True)])
+def test_every_tile_on_odd_multiples_of_128(gpu, m, n, k, group, zp_tensor):
+    test_tile_gemm_on_odd_multiples_of_128(gpu, m, n, k, group, zp_tensor)
 
 
 # (128, False): the kernel of groups of 128 with a scalar zero point, by name

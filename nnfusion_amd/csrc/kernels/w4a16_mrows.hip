@@ -18,10 +18,10 @@
 //     no barrier on the load path.  Two steps per tile (one tile in flight per wavefront) measured fastest.
 //     The 16-byte pieces of a row are XOR-swizzled with the row number on the way (each lane chooses which
 //     piece it fetches), so the 128-bit operand reads are conflict free.
-//   * The activations never touch LDS: lane (m, kq) loads the 64 bytes of row m that its MFMA operand holds of
-//     each of the wavefront's groups, once, and keeps them (16 VGPRs per group; hence K <= 8192), in the pair
-//     order of the nibble trick; the constant part of a group sum is an MFMA against a
-//     constant operand and becomes the (negative) initial accumulator of the group (see w4a16_skinny.hip).
+//   * The activations pass through LDS once, while the kernel starts, as whole lines and ahead of the weights: lane
+//     (m, kq) then keeps the 64 bytes of row m that its MFMA operand holds of each of the wavefront's groups (16 VGPRs
+//     per group; hence K <= 8192), in the pair order of the nibble trick; the constant part of a group sum is an MFMA against
+//     a constant operand and becomes the (negative) initial accumulator of the group (see w4a16_skinny.hip).
 //   * Per step: GW x 4 MFMAs (v_mfma_f32_16x16x32_f16, weights as the B operand) per wavefront, the group sum
 //     times the group scale in fp32; per tile the eight partial 16 x 16 tiles meet in LDS (one LDS-only barrier,
 //     two alternating buffers), 256 threads add them and park the sums in LDS; Y is written after the
@@ -97,7 +97,11 @@ namespace nnf
         }
         return sg;
     }
-    // The second half of mrows_rms_norm: the wavefronts' shares of the rows' sums are in sum_sq.
+    // RMSNorm of the activations in registers as rms_norm_kernel computes it: fp16(x * rstd * gamma), in fp32, one rounding.
+    // (Not x * gamma with rstd on the sums at the end, as in w4a16_mrows_kernel: the kernels of other block parameters have no
+    // per-group sums to scale, and x * gamma alone may leave the range of fp16.)  Lane (m = col, kq) holds 64 bytes of each of its
+    // wavefront's GA groups; gsrc(g): the 64 bytes of gamma that pair with group g.  sum_sq: [8 wavefronts][MB x 16 rows] of LDS,
+    // the wavefronts' shares of the rows' sums of squares: per lane group after group (sum_of_squares), then over the four kq.
     template <int MB, int GA, class F>
     __device__ __forceinline__ void mrows_normalise(uintx4 (&areg)[MB][GA][4], const float* sum_sq, int K, float eps, int col, F&& gsrc)
     {
@@ -133,29 +137,6 @@ namespace nnf
                 }
             }
         }
-    }
-    // RMSNorm of the activations in registers as rms_norm_kernel computes it: fp16(x * rstd * gamma), in fp32, one rounding.
-    // Lane (m = col, kq) holds 64 bytes of each of its wavefront's GA groups; gsrc(g): the 64 bytes of gamma that pair with
-    // group g.  sum_sq: [8 wavefronts][MB x 16 rows] of LDS of its own.  (Unlike mrows_scale_a, where rstd joins the sums at the end:
-    // these kernels have no per-group sums to scale, and x * gamma alone may leave the range of fp16.)
-    template <int MB, int GA, class F>
-    __device__ __forceinline__ void mrows_rms_norm(uintx4 (&areg)[MB][GA][4], float* sum_sq, int K, float eps, int wave, int col, int kq,
-                                                   F&& gsrc)
-    {
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-        {
-            float ss = 0.f;
-#pragma unroll
-            for (int g = 0; g < GA; ++g)
-                ss += sum_of_squares(areg[mb][g]);
-            ss += __shfl_xor(ss, 16, 64);
-            ss += __shfl_xor(ss, 32, 64);
-            if (kq == 0)
-                sum_sq[wave * (MB * 16) + mb * 16 + col] = ss;
-        }
-        __syncthreads();
-        mrows_normalise<MB, GA>(areg, sum_sq, K, eps, col, gsrc);
     }
 
     // v of this lane + v of the lane 16 (32) away, the same in both, without the LDS unit: the compiler waits for every LDS-bound
@@ -264,8 +245,9 @@ namespace nnf
     }
     // Takes the blocks as they come: MFMA operand registers in the pair order of the nibble trick, the constant part of each
     // group's sum (an MFMA against a constant operand, negative, the initial accumulator of the group); NORM: gamma onto them
-    // (fp16 products, rounded once) and the lane's share of sum a^2 of its row.  fetch(integral_constant p): asks for block p; the first NF have been asked for, BEHIND
-    // other loads after them.  gamma_block: the group's 256 bytes of gamma one after the other, in LDS, asked for ahead of the blocks.
+    // (fp16 products, rounded once) and the lane's share of sum a^2 of its row.  fetch(integral_constant p): asks for block p;
+    // the first NF have been asked for, BEHIND other loads after them.  gamma_block: the group's 256 bytes of gamma one after the
+    // other, in LDS, asked for ahead of the blocks.
     // (v_dot2_f32_f16 in one chain, in the order of k.  On the matrix cores, as the diagonal of A . A^T, the squares cost
     // nothing and the sum is no worse, but rounds otherwise; no difference in time at 6 and 16 rows x 4096.)
     template <int MB, int GA, int RL, bool NORM, int BEHIND, class F>
@@ -323,8 +305,8 @@ namespace nnf
         });
     }
 
-    // The same blocks for the kernels of other block parameters: operand registers as they are in memory (NORM) or in the pair order of the
-    // nibble trick; NORM: the lane's share of sum a^2 of its row, in the order in which mrows_rms_norm adds it up.
+    // The same blocks for the kernel of other block parameters: operand registers as they are in memory (NORM) or in the pair
+    // order of the nibble trick; NORM: the lane's share of sum a^2 of its row, group after group.
     template <int MB, int GA, int RL, bool NORM, int BEHIND, class F>
     __device__ __forceinline__ void mrows_take_blocks_q(uintx4 (&areg)[MB][GA][4], float& sq, const uint8_t* stage, int col, int kq, F&& fetch)
     {
@@ -668,11 +650,11 @@ namespace nnf
     //              parked sums [tiles of the workgroup][M][16] fp32
     //              (from the partial tiles on, while the kernel starts: activations [8][8 KiB] | RMSNorm weight [8][1 KiB])
     // pack = M | zp << 8 | gate << 16; tiles, RL: as in w4a16_mrows_kernel.
-    // FUSE: 0 plain, 1 with the epilogue of `f`, 2 with RMSNorm as well.  RMSNorm ahead of the product (f.gamma), bias / residual or SiLU-gate behind it, as the nodes of their own
-    // would compute them.  They were launches of their own (2 - 4 us each at 8 rows, 19 of the 56 us of a decoder layer
-    // with groups of 64 and zero points); inside, the prologue runs while the first weights are on their way.  RMSNorm only
-    // where workspace::mrows_q_norm_inside says so (every workgroup normalises all the rows for itself: with more groups per
-    // wavefront that takes longer than the pass of its own).
+    // FUSE: 0 plain, 1 with the epilogue of `f`, 2 with RMSNorm as well.  RMSNorm ahead of the product (f.gamma), bias / residual
+    // or SiLU-gate behind it, as the nodes of their own would compute them.  They were launches of their own (2 - 4 us each at 8
+    // rows, 19 of the 56 us of a decoder layer with groups of 64 and zero points); inside, the prologue runs while the first
+    // weights are on their way.  RMSNorm only where workspace::mrows_q_norm_inside says so (every workgroup normalises all the
+    // rows for itself: with more groups per wavefront that takes longer than the pass of its own).
     template <int GW, int GSHIFT, bool ZPT, int MB, int FUSE, int RL>
     __global__ __launch_bounds__(512) void w4a16_mrows_q_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                                 const half_t* __restrict__ S, const uint8_t* __restrict__ zps,
@@ -775,8 +757,9 @@ namespace nnf
 
         // RMSNorm weight, as many blocks of activations as there is room for, the weights, the rest, in this order: as in w4a16_mrows_kernel.
         // Nine rows and more of K = 8192, four times as many blocks as there is room for: the weights first (3 % faster).
-        // (With the activations behind the weights, and RMSNorm's weight behind those, groups of 64 with zero points, N = K = 4096: 4 / 8
-        // rows 5.82 / 6.21 us, with a residual 6.18 / 6.31, RMSNorm and SiLU-gate at N = 11008 8 rows 17.2; now 5.09 / 5.40, 5.34 / 5.54, 16.3.)
+        // (With the activations behind the weights, and RMSNorm's weight behind those, groups of 64 with zero points, N = K =
+        // 4096: 4 / 8 rows 5.82 / 6.21 us, with a residual 6.18 / 6.31, RMSNorm and SiLU-gate at N = 11008 8 rows 17.2; now 5.09
+        // / 5.40, 5.34 / 5.54, 16.3.)
         uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
         const uint8_t* gamma_block = red + MR_WAVES * (2 * ROW_BLOCK_BYTES) + wave * (GAMMA_LOADS * 1024);
         if constexpr (NORM)
@@ -818,8 +801,8 @@ namespace nnf
             if (kq == 0) // (by hand: ahead of an LDS write that it can see, the compiler waits for every LDS-bound load in flight)
                 asm volatile("ds_write_b32 %0, %1" ::"v"(lds_address(sum_sq + wave * 16 + col)), "v"(sum) : "memory");
         }
-        // (the blocks lay over what holds the partial tiles and the parked sums from here on; the RMSNorm weight over parked sums alone, which are
-        // written behind the first tile's barrier)
+        // (the blocks lay over what holds the partial tiles and the parked sums from here on; the RMSNorm weight over parked sums
+        // alone, which are written behind the first tile's barrier)
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if constexpr (NORM)
         {

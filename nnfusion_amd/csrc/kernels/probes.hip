@@ -317,7 +317,7 @@ extern "C" int nnf_probe_mfma(int kind, int mode, int iters, int num_cu, double*
 
 // ---- where a launch of the tile GEMM spends its time ------------------------------------------------------------------
 // The product's own kernel (w4a16_gemm_sk.h), compiled here once more with time stamps (NNF_SK_TRACE): the plain product
-// on 128-row tiles of 128 or 256 columns, in its one-launch form.  trace: 16 x grid 64-bit stamps of the 100 MHz clock
+// on 128-row tiles of 128 or 256 columns, on four or eight wavefronts as the library chooses, in its one-launch form.  trace: 16 x grid 64-bit stamps of the 100 MHz clock
 // (0 start, 1 first operands arrived, 2 K loop of the last segment over, 3 its part parked, 4 counted in, 5 waits for the
 // other workgroups of its shared tiles over, 6 its share of those tiles finished, 9 end; for a workgroup with two segments
 // also 10 K loop of the first over, 11 its part parked and counted in, 12 first operands of the last arrived).
@@ -346,22 +346,20 @@ extern "C" int nnf_probe_gemm_timeline(void* stream, const void* A, const void* 
     p.sync = plan.slots ? (uint32_t*)sync : nullptr;
     p.spin_limit = 1 << 13;
     p.trace = trace;
-    if (plan.tile_weight_rows == 128)
-    {
-        using T = gemm_sk::TileOf<128, 128>;
+    auto launch = [&](auto tile) {
+        using T = decltype(tile);
         auto kernel = &w4a16_gemm_sk_kernel<T::TM, T::TN, T::NW, T::KH, false, false, false, false>;
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES) != hipSuccess)
-            return -1;
+            return false;
         launch_sk_kernel<T>(kernel, plan.grid, (hipStream_t)stream, p);
-    }
-    else
-    {
-        using T = gemm_sk::TileOf<128, 256>;
-        auto kernel = &w4a16_gemm_sk_kernel<T::TM, T::TN, T::NW, T::KH, false, false, false, false>;
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES) != hipSuccess)
-            return -1;
-        launch_sk_kernel<T>(kernel, plan.grid, (hipStream_t)stream, p);
-    }
+        return true;
+    };
+    using namespace gemm_sk;
+    const bool eight = workspace::sk_eight_wavefronts(plan, false, false, num_cu);
+    const bool launched = plan.tile_weight_rows == 128 ? (eight ? launch(TileOf<128, 128, true>{}) : launch(TileOf<128, 128>{}))
+                                                       : (eight ? launch(TileOf<128, 256, true>{}) : launch(TileOf<128, 256>{}));
+    if (!launched)
+        return -1;
     return hipGetLastError() == hipSuccess ? plan.grid : -1;
 }
 

@@ -8,8 +8,8 @@
 // the scale); the kernels in w4a16_*.hip serve the one combination the benchmark uses (4 bits, groups of 128, a
 // scalar zero point) as fast as the hardware allows, these serve every other one correctly and simply:
 //   * wna16_gemv_kernel (M = 1 where K is not a multiple of 256; the others run on the row-streaming kernel of
-//     w4a16_gemv_rows.hip, 4- and 8-bit weights alike): a wavefront per block of four weight rows; a lane turns 16
-//     bytes of weights of each into the exact integers q - z in fp16, multiplies them with the activations
+//     w4a16_gemv_rows.hip, 4- and 8-bit weights alike): a wavefront per block of four weight rows, or per row where
+//     there are up to 24 (28, 31 of 8-bit weights) a CU; a lane turns 16 bytes of weights of each into the exact integers q - z in fp16, multiplies them with the activations
 //     (v_dot2_f32_f16, fp32 sums) and applies the group's scale to the sum over its piece of the group;
 //   * wna16_skinny_kernel (2 <= M <= 16): v_mfma_f32_16x16x32_f16, activations and weights fetched straight into the
 //     operand registers, eight wavefronts share the K range of two tiles of 16 weight rows;
@@ -699,10 +699,14 @@ namespace nnf
                 // rows the row-streaming kernel can walk: that kernel
                 if (w4a16_gemv_rows_q_supported(1, N, K, qa.group_shift, zero_points != nullptr, num_cu, bits))
                     return launch_w4a16_gemv_rows_q(stream, A, Wq, S, Y, N, K, qa.group_shift, zp, zero_points, num_cu, bits);
-                // Fewer than 32 rows a CU: one a wavefront, so that all SIMDs have some, and a pass ahead; four, which share their activations,
-                // otherwise.  N = 4096 with groups of 32 and zero points, K = 4224 / 8320 / 11136 9.1 / 16.3 / 22.3 -> 7.4 / 10.7 / 12.6 us,
-                // 1024 x 1152 4.6 -> 2.9; two rows and a pass ahead 0.88 x at 11008 x 2176, four 0.76 at 16384.
-                if (N < 32 * num_cu)
+                // One row a wavefront, so that all SIMDs have some, and a pass ahead, while they fit on the CUs at once (4-bit weights:
+                // six a SIMD by their registers); four, which share their activations, otherwise.  N = 4096 with groups of 32 and
+                // zero points, K = 4224 / 8320 / 11136 9.1 / 16.3 / 22.3 -> 7.4 / 10.7 / 12.6 us, 1024 x 1152 4.6 -> 2.9.  One row /
+                // four around the line, K = 384 .. 11136: 4 bits 1.03 - 1.13 x at 24 rows a CU, 0.87 - 0.98 just above, 0.83 - 0.94
+                // at 31; 8 bits 1.00 - 1.11 at 28, above that 0.98 - 1.08 up to K = 2176, 0.95 - 0.99 from 4224 on.  Two rows and a
+                // pass ahead 0.88 x at 11008 x 2176, four 0.76 at 16384.
+                const int rows_a_cu = bits == 4 ? 24 : K < 4096 ? 31 : 28;
+                if (N <= rows_a_cu * num_cu)
                     bits == 4 ? launch_wna16_gemv<4, 1, 1, true>(stream, A, Wq, S, Y, M, N, K, qa, num_cu)
                               : launch_wna16_gemv<8, 1, 1, true>(stream, A, Wq, S, Y, M, N, K, qa, num_cu);
                 else

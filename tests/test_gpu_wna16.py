@@ -212,8 +212,9 @@ def test_products_beyond_the_k_streaming_kernel(gpu, m, n, k, bits, group, zp_te
     _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
 
 
-# one row on the plain GEMV: fewer rows than wavefronts, either side of 32 a CU, a pass of a few lanes, one pass and many
-@pytest.mark.parametrize("n,k", [(1, 128), (33, 384), (1000, 1152), (4096, 2176), (8191, 640), (8192, 640), (300, 16512)])
+# one row on the plain GEMV: fewer rows than wavefronts, either side of 24, 28 and 31 a CU, a pass of a few lanes, one pass and many
+@pytest.mark.parametrize("n,k", [(1, 128), (33, 384), (1000, 1152), (4096, 2176), (6144, 640), (6145, 384), (7168, 4224),
+                                 (7169, 4224), (7936, 640), (7937, 640), (8191, 640), (8192, 640), (300, 16512)])
 @pytest.mark.parametrize("bits,group,zp_tensor", [(4, 32, True), (4, 64, False), (8, 32, True), (8, 128, False)])
 def test_one_row_on_the_plain_kernel(gpu, n, k, bits, group, zp_tensor):
     a, wq, s, zps = _case(n + k + bits + group, 1, n, k, bits, group, zp_tensor)

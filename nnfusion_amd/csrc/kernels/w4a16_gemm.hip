@@ -548,7 +548,7 @@ namespace nnf
     }
 
     // ---- the tile GEMM with other block parameters ----------------------------------------------------------------------
-    bool w4a16_gemm_q_supported(int M, int N, int K, int group_shift) 
+    bool w4a16_gemm_q_supported(int M, int N, int K, int group_shift)
     {
         return workspace::w4a16_gemm_q_fits(M, N, K, group_shift) || workspace::w4a16_gemm_q_odd_fits(M, N, K, group_shift);
     }

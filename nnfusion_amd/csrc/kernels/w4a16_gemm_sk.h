@@ -846,10 +846,10 @@ namespace nnf
             const uint8_t* a_bytes = reinterpret_cast<const uint8_t*>(p.A);
             const uint8_t* g_bytes = reinterpret_cast<const uint8_t*>(p.gamma) + (size_t)k_begin * 2;
             const uint32_t g_off = (uint32_t)(lane & 31) * 4u;
-            // Scalar base of K step kt (clamped to the last inside K: past it a valid tile goes to a free stage) and which bits of the lanes'
-            // offsets count.  ODD: steps 2 and 3 of a superstep may lie past K and are worked on all the same, with weights of zero: zeros for
-            // them, since an infinity in their place would make NaN: 0.6 % of 190 products' time.  (Loop left in the middle instead: 2 KiB of
-            // registers spilled under the 256 x 256 tile.)
+            // Scalar base of K step kt (clamped to the last inside K: past it a valid tile goes to a free stage) and which bits
+            // of the lanes' offsets count.  ODD: steps 2 and 3 of a superstep may lie past K and are worked on all the same, with
+            // weights of zero: zeros for them, since an infinity in their place would make NaN: 0.6 % of 190 products' time.
+            // (Loop left in the middle instead: 2 KiB of registers spilled under the 256 x 256 tile.)
             struct KBase
             {
                 const uint8_t* at;

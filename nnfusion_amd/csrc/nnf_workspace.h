@@ -383,18 +383,19 @@ namespace nnf
             }
             return best_grid ? plan_w4a16_sk(M, N, K, gate, num_cu, rows, best_grid, cols) : even;
         }
-        // Eight wavefronts on a tile of 64 or 128 rows instead of four (gemm_sk::TileOf).  A wavefront's own share of the work is halved, what
-        // comes before and behind the K loop is not, so it takes a long enough share; a second workgroup on the CU, which hides the
-        // waits as well, has no room beside the two rings of the 128-wide tiles; and near the full chip the activations' way out of LDS,
-        // read twice as often by the 256-wide ones, costs more than it hides.  3000 products on every tile and number of parts, start /
-        // this in the geometric mean: 128 x 128 tiles, one a CU, shares of 2 / 4 / 8 / 16 / 32 supersteps 0.93 / 1.02 / 1.11 / 1.17 / 1.23 (with
-        // RMSNorm 1.31 on few CUs, where rstd[] of many rows a workgroup takes half as long), more tiles than CUs 0.75 - 0.94; parts of
-        // 1 / 2 / 4 / 8 / 16: 0.92 / 0.95 / 1.02 / 1.09 / 1.16 up to half of the CUs, 0.92 / 0.89 / 0.90 / 0.98 / 1.05 above three quarters; the even
-        // split of more tiles than workgroups 0.94 / 0.97 / 1.02 / 1.03 / 1.03 (of fewer tiles 0.87 - 1.0, left on four); 128 x 256
-        // one a CU 1.2 (few, short) .. 0.99 (220 and more, from 32 on), parts 1.10 .. 1.02, from three quarters of the CUs on 0.96 - 1.0.
-        // The faster kernel takes power from its neighbours.  70 products of 128 x 128 tiles on 193 .. 255 CUs from eight supersteps on, by themselves
-        // 1.047, with pauses 1.039, behind 64 x 4096 x 4096 1.039, behind the product that leads back to their K 1.035, each for the whole
-        // sequence; behind two of M x 11008 x 4096 0.997 (0.93 .. 1.05).
+        // Eight wavefronts on a tile of 64 or 128 rows instead of four (gemm_sk::TileOf).  A wavefront's own share of the work is
+        // halved, what comes before and behind the K loop is not, so it takes a long enough share; a second workgroup on the CU,
+        // which hides the waits as well, has no room beside the two rings of the 128-wide tiles; and near the full chip the
+        // activations' way out of LDS, read twice as often by the 256-wide ones, costs more than it hides.  3000 products on
+        // every tile and number of parts, start / this in the geometric mean: 128 x 128 tiles, one a CU, shares of 2 / 4 / 8 / 16
+        // / 32 supersteps 0.93 / 1.02 / 1.11 / 1.17 / 1.23 (with RMSNorm 1.31 on few CUs, where rstd[] of many rows a workgroup
+        // takes half as long), more tiles than CUs 0.75 - 0.94; parts of 1 / 2 / 4 / 8 / 16: 0.92 / 0.95 / 1.02 / 1.09 / 1.16 up
+        // to half of the CUs, 0.92 / 0.89 / 0.90 / 0.98 / 1.05 above three quarters; the even split of more tiles than workgroups
+        // 0.94 / 0.97 / 1.02 / 1.03 / 1.03 (of fewer tiles 0.87 - 1.0, left on four); 128 x 256 one a CU 1.2 (few, short) .. 0.99
+        // (220 and more, from 32 on), parts 1.10 .. 1.02, from three quarters of the CUs on 0.96 - 1.0.
+        // The faster kernel takes power from its neighbours.  70 products of 128 x 128 tiles on 193 .. 255 CUs from eight
+        // supersteps on, by themselves 1.047, with pauses 1.039, behind 64 x 4096 x 4096 1.039, behind the product that leads
+        // back to their K 1.035, each for the whole sequence; behind two of M x 11008 x 4096 0.997 (0.93 .. 1.05).
         inline bool sk_eight_wavefronts(const SkPlan& p, bool gate, bool rms, int num_cu)
         {
             if ((p.tile_rows != 64 && p.tile_rows != 128) || p.grid < 1)
@@ -699,7 +700,7 @@ namespace nnf
         // their scales, two sets of eight partial tiles (one or two blocks of 16 rows), and the workgroup's finished
         // tiles parked until the end.
         // Two forms.  K / 1024 = 1, 2, 3, 4, 6, 8: K is a compile-time constant of the kernel.  Any other multiple of
-        // 256 up to 8192 (M <= 16): K is a run-time value, two steps of 8 * GW groups with the smallest GW (2, 3, 4)
+        // 128 up to 8192 (M <= 16): K is a run-time value, two steps of 8 * GW groups with the smallest GW (1 .. 4)
         // that covers K; wavefronts past the end of K fetch groups that another one already covers and discard them.
         inline bool w4a16_mrows_fixed_k(int M, int K)
         {
@@ -713,11 +714,13 @@ namespace nnf
                 return (kw & 1) ? kw : kw / 2; // even K / 1024: two steps per tile
             return G <= 16 ? 1 : G <= 32 ? 2 : G <= 48 ? 3 : 4;
         }
-        // Whether the kernel brings its activations in through LDS as whole lines or straight into the registers.  Straight
-        // in, a load touches two lines of every row for 32 bytes each, four times over; through LDS every line is touched
-        // once, but the blocks come one behind the other (0.3 - 0.5 us).  Measured, K = 4096: 2 / 4 / 6 rows 4.84 / 5.07 /
-        // 5.20 us straight against 5.19 / 5.27 / 5.29, 8 / 12 / 16 rows 5.63 / 6.52 / 7.3 against 5.30 / 5.40 / 5.55;
-        // K = 8192: 4 / 6 rows 12.05 / 12.45 against 11.58 / 11.70; 32 rows at N = K = 4096: 10.8 against 7.1.
+        // Whether the kernels of 8-bit weights and of a run-time K with other block parameters, which ask for their activations
+        // behind the weights and in blocks of 16 rows, bring them in through LDS as whole lines or straight into the registers.
+        // (The others always go through LDS, in blocks of 4, 8 or 16 rows ahead of the weights.)  Straight in, a load touches two
+        // lines of every row for 32 bytes each, four times over; through LDS every line is touched once, but the blocks come one
+        // behind the other (0.3 - 0.5 us).  Measured with 4-bit weights in groups of 128 loaded that way, K = 4096: 2 / 4 / 6 rows
+        // 4.84 / 5.07 / 5.20 us straight against 5.19 / 5.27 / 5.29, 8 / 12 / 16 rows 5.63 / 6.52 / 7.3 against 5.30 / 5.40 /
+        // 5.55; K = 8192: 4 / 6 rows 12.05 / 12.45 against 11.58 / 11.70; 32 rows at N = K = 4096: 10.8 against 7.1.
         constexpr bool mrows_stages_activations(int M, int K) { return (long long)M * K >= 32768; }
         // the room for that: two blocks of 16 rows x 256 bytes per wavefront, where the partial tiles and parked sums go later
         constexpr size_t mrows_tail_bytes(size_t tail) { return tail > (size_t)8 * 2 * 4096 ? tail : (size_t)8 * 2 * 4096; }
@@ -759,9 +762,13 @@ namespace nnf
         // 17 .. 32 rows 0.93 - 0.98, 0.97 - 1.02; K = 4096, 2 .. 7 rows 0.87 - 0.93, 0.92 - 0.99 (8 rows and up bring their
         // activations in as whole lines), 8 .. 16 rows 0.95 - 1.02, 0.97 - 1.03, 17 .. 32 rows 0.82 - 0.89, 0.83 - 0.93;
         // K = 3072 / 3584 0.88 - 1.00, 0.92 - 1.01; K = 4608 / 5120 0.76 - 0.96, 0.80 - 0.97; K = 8192 0.70 - 0.91, 0.78 - 0.95.
+        // Those are times with the activations behind the weights.  Ahead of them, K = 4096 and 2 .. 7 rows (with the pass / inside):
+        // alone 1.05 - 1.13 at 2304 and 4096 columns, 0.92 - 1.01 at 11008; with SiLU-gate 0.93 - 1.06.  The pass stays there: the
+        // tests hold these products to the bits of the nodes one after the other.
         constexpr bool mrows_q_norm_inside(int M, int K) { return M <= 16 && (K == 2048 || (K == 4096 && mrows_stages_activations(M, K))); }
         // (fused: with room for the wavefronts' sums of squares per row, at the sizes that may have RMSNorm inside)
-        // norm: with RMSNorm inside, 1 KiB of its weight per wavefront behind the activations while the kernel starts (at most 72 KiB beside 41: always room)
+        // norm: with RMSNorm inside, 1 KiB of its weight per wavefront behind the activations while the kernel starts (at most
+        // 72 KiB beside 41: always room)
         inline size_t w4a16_mrows_q_lds_bytes(int K, int M, int tiles, int group_shift, bool zero_points, bool fused = false, bool norm = false)
         {
             const int gw = K >> 11;
@@ -863,9 +870,10 @@ namespace nnf
             return !(K & 255) && w4a16_gemm_q_addressable(M, N, K, group_shift);
         }
         // ... and on odd multiples of 128, whose last superstep of 256 is half work for nothing, given scratch memory that is preferred and not needed
-        // (plan_w4a16_sk: what parked tiles may take), where it is ahead of the plain tile kernel.  900 products, time there / here:
-        // K = 384 0.87, 640 0.95, 896 1.04, from 1152 on 1.1 - 1.5 (1000 x 4096 x 4224 in groups of 32 56.2 -> 41 us, 2000 rows 92.5 -> 68),
-        // but above 1600 rows 0.92 at 1152 / 1408, 1.03 up to 1920; few columns 0.8 - 0.97 at short K, and with few rows too at long (185 x 320 x 15232).
+        // (plan_w4a16_sk: what parked tiles may take), where it is ahead of the plain tile kernel.  900 products, time there /
+        // here: K = 384 0.87, 640 0.95, 896 1.04, from 1152 on 1.1 - 1.5 (1000 x 4096 x 4224 in groups of 32 56.2 -> 41 us, 2000
+        // rows 92.5 -> 68), but above 1600 rows 0.92 at 1152 / 1408, 1.03 up to 1920; few columns 0.8 - 0.97 at short K, and with
+        // few rows too at long (185 x 320 x 15232).
         inline bool w4a16_gemm_q_odd_fits(int M, int N, int K, int group_shift)
         {
             return (K & 255) == 128 && K >= (M > 1600 || N < 768 ? 2176 : 1152) && (N >= 512 || M > 256) && w4a16_gemm_q_addressable(M, N, K, group_shift);
@@ -1066,27 +1074,30 @@ namespace nnf
         }
         // Where the library picks it by itself, from measurements against the split-K MFMA GEMV on cold weights
         // (M = 2 / 16): K = 2048, 4096, 6144, 8192: 0-15 % / 15-30 % faster;  K = 1024, 3072: 5-35 % faster;
-        // run-time K: 0-5 % / 15-35 % faster at K = 3584, 5120, 7168 (but up to 19 % slower below eight rows at K = 7168), level
-        // at K = 2560, slower at K = 1536 and 2304, where most of what the wavefronts fetch is discarded: taken when at
-        // least three quarters of the fetched groups count.
+        // run-time K from eight rows on: 15-35 % faster at K = 3584, 5120, 7168, level at K = 2560, slower at K = 1536 and 2304,
+        // where most of what the wavefronts fetch is discarded: taken when at least three quarters of the fetched groups count.
         inline bool w4a16_mrows_preferred(int M, int N, int K, int num_cu, bool gate = false)
         {
             if (!w4a16_mrows_fits(M, N, K, num_cu, gate, true))
                 return false;
             if (w4a16_mrows_fixed_k(M, K))
                 return true;
-            // Up to seven rows, even numbers of groups, against the MFMA GEMV, whatever part of what is fetched counts (N = 1024 / 4096 / 12288): K = 1280 ..
-            // 1920 1.0 - 1.2 x, 2304 .. 5888 1.0 - 1.1, 6144 .. 7936 1.04 - 1.4 (4096 x 7168 9.7 -> 7.7 us at seven rows), 1024 and 1152 0.86 - 1.0.
-            // (Before the activations came first, in blocks of four or eight rows, these were level or slower.)  Odd numbers of groups keep the GEMV and
-            // with it the order of their sums, 1.0 - 1.2 x here.
+            // Up to seven rows, even numbers of groups, against the MFMA GEMV, whatever part of what is fetched counts (N = 1024
+            // / 4096 / 12288): K = 1280 .. 1920 1.0 - 1.2 x, 2304 .. 5888 1.0 - 1.1, 6144 .. 7936 1.04 - 1.4 (4096 x 7168 9.7 ->
+            // 7.7 us at seven rows), 1024 and 1152 0.86 - 1.0.
+            // (Before the activations came first, in blocks of four or eight rows, these were level or slower.)  Odd numbers of
+            // groups keep the GEMV: 4 and 7 rows 1.0 - 1.3 x here from K = 1408 on, 2 and 6 rows 0.95 - 1.25 (K = 1152, 4224
+            // and 6272 0.92 - 1.13); RMSNorm, whose pass goes ahead either way, level.
             if (M < 8)
                 return !(K & 128) && K >= 1280;
             const int gw = w4a16_mrows_step_groups(M, K);
-            // 8 .. 16 rows (K = 3200 1.15 - 1.4 x, 5504 1.6 - 1.75, 8064 1.2 - 1.45, 1920 1.1 - 1.25); 17 .. 32 rows, whose other kernel is the
-            // tile GEMM, whatever part of what is fetched counts (K = 1664 .. 1920 1.8 - 2.9 x, 3200 1.7 - 2.5, 3968 1.8 - 2.2).
-            // 33 .. 64 rows (the library's own choice is the K-streaming kernel there, 1.2 - 1.9 x; scratch sizes follow this rule), up to
-            // sixteen groups: four blocks of rows against the tile GEMM, 1152 / 4096 / 12288 / 22016 weight rows: K = 1280
-            // 1.45 / 1.3 / 0.9 - 1.0 / 0.7 x, 1664 .. 2048 1.5 / 1.4 / 1.1 - 1.3 / 0.8 - 1.0; RMSNorm and SiLU-gate 1.5 / 1.5 / 1.2 - 1.4 / 1.0 - 1.3
+            // 8 .. 16 rows (K = 3200 1.15 - 1.4 x, 5504 1.6 - 1.75, 8064 1.2 - 1.45, 1920 1.1 - 1.25); 17 .. 32 rows, whose other
+            // kernel is the tile GEMM, whatever part of what is fetched counts (K = 1664 .. 1920 1.8 - 2.9 x, 3200 1.7 - 2.5,
+            // 3968 1.8 - 2.2).
+            // 33 .. 64 rows (the library's own choice is the K-streaming kernel there, 1.2 - 1.9 x; scratch sizes follow this
+            // rule), up to sixteen groups: four blocks of rows against the tile GEMM, 1152 / 4096 / 12288 / 22016 weight rows:
+            // K = 1280 1.45 / 1.3 / 0.9 - 1.0 / 0.7 x, 1664 .. 2048 1.5 / 1.4 / 1.1 - 1.3 / 0.8 - 1.0; RMSNorm and SiLU-gate
+            // 1.5 / 1.5 / 1.2 - 1.4 / 1.0 - 1.3
             if (M > 32)
                 return gate ? 2 * N <= (K >= 1280 ? 22016 : 12288) : N <= (K >= 1408 ? 12288 : 8192);
             // (up to 16 rows K = 1536 on one group per wavefront is level: left where it was)
@@ -1098,6 +1109,8 @@ namespace nnf
         // RMSNorm: K = 3200, 8 .. 10 rows 0.94 - 0.98 (4096 columns at 8 rows 5.7 / 6.0 us), 3456, 8 and 9 rows 0.96 - 1.01, 1664, 8 rows
         // 0.94 - 0.97; with 9152 columns 0.98 - 1.06; K = 3712, 3968, 1792, and 1664 at nine rows: 0.98 - 1.2.
         // (Not with SiLU-gate, 1.05 - 1.2 x here, nor with the residual in place, for which that route asks for scratch memory.)
+        // What the library runs by itself is the K-streaming kernel at these sizes (4096 columns at 8 rows of K = 3200 4.8 us);
+        // scratch sizes, and devices that kernel does not fit, follow this rule.
         inline bool w4a16_skinny_ahead_of_mrows(int M, int N, int K)
         {
             const int gw = w4a16_mrows_step_groups(M, K);
@@ -1267,7 +1280,8 @@ namespace nnf
                 if (M <= 16)
                 {
                     const bool fixed_k = K == 2048 || K == 4096 || K == 8192;
-                    // (K = 2048: where the row-streaming kernel takes these parameters, five and six tiles take 8 - 16 % less time there; up to four level or more)
+                    // (K = 2048: where the row-streaming kernel takes these parameters, five and six tiles take 8 - 16 % less
+                    // time there; up to four level or more)
                     const bool few = K != 2048 || w4a16_mrows_q_fits(M, N, K, qg, true, num_cu, true, gate);
                     if (fixed_k ? !rms || (gate && p.tiles > (few ? 4 : 6)) : K > 8192 && (N < 4096 || p.tiles > 2))
                         continue;

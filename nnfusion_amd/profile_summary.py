@@ -35,7 +35,7 @@ def demangle(name):
     return re.sub(r"\(.*\)$", "", name)
 
 
-def short(name, width=64):
+def short(name, width=80):
     """nnf::gemm_sk::kernel<4, 2, ...>(args) -> kernel<4, 2, ...>, cut to `width`."""
     name = demangle(name)
     name = re.sub(r"\b(nnf|gemm_sk)::", "", name)
@@ -147,18 +147,18 @@ def counters(directory, log, prefixes):
     segs, _ = segments(csv_rows(directory, "counter_collection.csv"), probe)
     names = sorted({k for _, ds in segs for d in ds for k in d if k not in ("kernel", "us")})
     out = ["counters per dispatch (means over the row's launches; summed over the chip): " + " ".join(names), "",
-           f"{'row':<30} {'kernel':<46} {'us':>7} " + " ".join(f"{n[-14:]:>14}" for n in names)]
+           f"{'row':<30} {'kernel':<72} {'us':>7} " + " ".join(f"{n[-14:]:>14}" for n in names)]
     derived = []
     for row, ds in segs:
         if prefixes and not any(row["row"].startswith(p) for p in prefixes):
             continue
         by_kernel = collections.OrderedDict()
         for d in ds:
-            by_kernel.setdefault(short(d["kernel"], 46), []).append(d)
+            by_kernel.setdefault(short(d["kernel"], 72), []).append(d)
         for k, group in by_kernel.items():
             mean = {n: sum(d.get(n, 0.0) for d in group) / len(group) for n in names}
             us = sum(d.get("us", 0.0) for d in group) / len(group)
-            out.append(f"{row['row'][:30]:<30} {k:<46} {us:>7.1f} " + " ".join(f"{mean[n]:>14.0f}" for n in names))
+            out.append(f"{row['row'][:30]:<30} {k:<72} {us:>7.1f} " + " ".join(f"{mean[n]:>14.0f}" for n in names))
             extra = []
             if mean.get("TCC_REQ_sum") and "TCC_HIT_sum" in mean:
                 extra.append(f"L2 hit {100 * mean['TCC_HIT_sum'] / mean['TCC_REQ_sum']:.1f} %")
@@ -175,7 +175,7 @@ def counters(directory, log, prefixes):
                     if n in mean:
                         extra.append(f"{label} {100 * mean[n] / mean['SQ_WAVE_CYCLES']:.1f} %")
             if extra:
-                derived.append(f"{row['row'][:30]:<30} {k:<46} " + ", ".join(extra))
+                derived.append(f"{row['row'][:30]:<30} {k:<72} " + ", ".join(extra))
     return out + ["", "derived:"] + derived
 
 
@@ -190,7 +190,7 @@ def kernels(directory, last, parts):
             d["us"] = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
     groups = collections.OrderedDict()
     for d in by_dispatch.values():
-        name = short(d["kernel"], 60)
+        name = short(d["kernel"], 78)
         if not parts or any(p in name for p in parts):
             groups.setdefault(name, []).append(d)
     names = sorted({k for g in groups.values() for d in g for k in d if k not in ("kernel", "us")})

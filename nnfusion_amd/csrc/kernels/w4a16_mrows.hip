@@ -302,6 +302,10 @@ namespace nnf
                 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, areg[mb][g][j]), cvec, t, 0, 0, 0);
             }
             ncorr[mb][g] = t;
+            // (pinned: its only use is behind a branch, where the compiler moved the whole chain, every block as it was with it: 65
+            // registers spilled at K = 8192)
+            if constexpr (NORM)
+                asm volatile("" : "+v"(sq[mb]));
         });
     }
 

@@ -874,9 +874,16 @@ namespace nnf
         // here: K = 384 0.87, 640 0.95, 896 1.04, from 1152 on 1.1 - 1.5 (1000 x 4096 x 4224 in groups of 32 56.2 -> 41 us, 2000
         // rows 92.5 -> 68), but above 1600 rows 0.92 at 1152 / 1408, 1.03 up to 1920; few columns 0.8 - 0.97 at short K, and with
         // few rows too at long (185 x 320 x 15232).
+        // Below 512 columns, where a few dozen tiles or their parts are all there is (192 .. 448 columns, 258 .. 2048 rows): K = 2176 / 2688
+        // 0.76 - 0.97 up to 300 000 outputs, 1.0 - 1.57 from 320 000 on; K = 6272 0.90 - 0.96 up to 102 000, 0.99 - 1.6 above, from 8576
+        // on 0.96 - 1.17 there as well.
         inline bool w4a16_gemm_q_odd_fits(int M, int N, int K, int group_shift)
         {
-            return (K & 255) == 128 && K >= (M > 1600 || N < 768 ? 2176 : 1152) && (N >= 512 || M > 256) && w4a16_gemm_q_addressable(M, N, K, group_shift);
+            if ((K & 255) != 128 || !w4a16_gemm_q_addressable(M, N, K, group_shift))
+                return false;
+            if (N >= 512)
+                return K >= (M > 1600 || N < 768 ? 2176 : 1152);
+            return M > 256 && K >= 2176 && (long long)M * N >= (K < 3456 ? 320000 : K < 8192 ? 110000 : 0);
         }
         // ---- the plain tile kernel (wna16_generic.hip): tile shape and ranges of K ------------------------------------------
         // One range: the tile shape with the lowest time of a K step of 64 on a busy chip: 256 x 256 (0) 2.0 us a round of

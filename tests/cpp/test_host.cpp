@@ -1469,6 +1469,11 @@ int main(int argc, char** argv)
                         EXPECT(p.tile_rows == s[3] && p.tile_weight_rows == s[4] && split == s[6]);
                         EXPECT(ws::sk_eight_wavefronts(p, false, false, 256) == (s[5] != 0));
                     }
+            // ... few columns stay on the plain kernel where a few dozen tiles are all there is
+            const int few[][4] = {{650, 192, 2688, 0}, {1318, 192, 2176, 0}, {1000, 256, 2176, 0}, {400, 256, 6272, 0}, {257, 320, 3456, 0}, {256, 511, 16256, 0},
+                                  {1318, 256, 2176, 1}, {1000, 320, 2688, 1}, {650, 192, 3456, 1}, {400, 320, 6272, 1}, {257, 192, 8320, 1}, {150, 512, 8576, 1}};
+            for (const auto& s : few)
+                EXPECT(ws::w4a16_gemm_q_odd_fits(s[0], s[1], s[2], 6) == (s[3] != 0));
             // by itself the library runs no W8A8 product over two ranges of K on the row-streaming kernel: the K-streaming kernel takes them all
             for (int m = 2; m <= 32; ++m)
                 for (int k = 8192; k <= 16384; k += 512)

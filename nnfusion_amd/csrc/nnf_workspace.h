@@ -876,11 +876,18 @@ namespace nnf
         // few rows too at long (185 x 320 x 15232).
         // Below 512 columns, where a few dozen tiles or their parts are all there is (192 .. 448 columns, 258 .. 2048 rows): K = 2176 / 2688
         // 0.76 - 0.97 up to 300 000 outputs, 1.0 - 1.57 from 320 000 on; K = 6272 0.90 - 0.96 up to 102 000, 0.99 - 1.6 above, from 8576
-        // on 0.96 - 1.17 there as well.
+        // on 0.96 - 1.17 there as well.  Up to 128 rows and 1024 columns, where the plan is an even split whose shares of two
+        // supersteps straddle tiles: 153 products 0.93 (0.80 .. 1.18); with equal parts of tiles 165 products 1.08 (0.94 .. 1.34).
         inline bool w4a16_gemm_q_odd_fits(int M, int N, int K, int group_shift)
         {
             if ((K & 255) != 128 || !w4a16_gemm_q_addressable(M, N, K, group_shift))
                 return false;
+            if (M <= 128 && N <= 1024)
+            {
+                const SkPlan p = plan_w4a16_tiles_q(M, N, K, PLAN_CUS);
+                if (p.grid % (p.tiles_m * p.tiles_n))
+                    return false;
+            }
             if (N >= 512)
                 return K >= (M > 1600 || N < 768 ? 2176 : 1152);
             return M > 256 && K >= 2176 && (long long)M * N >= (K < 3456 ? 320000 : K < 8192 ? 110000 : 0);

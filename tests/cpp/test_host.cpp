@@ -1471,7 +1471,8 @@ int main(int argc, char** argv)
                     }
             // ... few columns stay on the plain kernel where a few dozen tiles are all there is
             const int few[][4] = {{650, 192, 2688, 0}, {1318, 192, 2176, 0}, {1000, 256, 2176, 0}, {400, 256, 6272, 0}, {257, 320, 3456, 0}, {256, 511, 16256, 0},
-                                  {1318, 256, 2176, 1}, {1000, 320, 2688, 1}, {650, 192, 3456, 1}, {400, 320, 6272, 1}, {257, 192, 8320, 1}, {150, 512, 8576, 1}};
+                                  {1318, 256, 2176, 1}, {1000, 320, 2688, 1}, {650, 192, 3456, 1}, {400, 320, 6272, 1}, {257, 192, 8320, 1}, {150, 512, 8576, 1}, {65, 512, 6272, 0},
+                                  {128, 768, 6784, 0}, {128, 640, 8320, 1}, {128, 1025, 6272, 1}};
             for (const auto& s : few)
                 EXPECT(ws::w4a16_gemm_q_odd_fits(s[0], s[1], s[2], 6) == (s[3] != 0));
             // by itself the library runs no W8A8 product over two ranges of K on the row-streaming kernel: the K-streaming kernel takes them all

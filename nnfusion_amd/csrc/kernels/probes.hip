@@ -355,7 +355,7 @@ extern "C" int nnf_probe_gemm_timeline(void* stream, const void* A, const void* 
         return true;
     };
     using namespace gemm_sk;
-    const bool eight = workspace::sk_eight_wavefronts(plan, false, false, num_cu);
+    const bool eight = workspace::sk_eight_wavefronts(plan, false, false, num_cu, (N & 7) != 0);
     const bool launched = plan.tile_weight_rows == 128 ? (eight ? launch(TileOf<128, 128, true>{}) : launch(TileOf<128, 128>{}))
                                                        : (eight ? launch(TileOf<128, 256, true>{}) : launch(TileOf<128, 256>{}));
     if (!launched)

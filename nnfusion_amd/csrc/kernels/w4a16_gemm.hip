@@ -484,7 +484,7 @@ namespace nnf
             p.rstd_sync = (uint32_t*)choice.sync_flags;
             p.rms_eps = rms_eps;
         }
-        const bool eight = workspace::sk_eight_wavefronts(plan, gate, rms, num_cu);
+        const bool eight = workspace::sk_eight_wavefronts(plan, gate, rms, num_cu, (N & 7) != 0);
         if (plan.tile_weight_rows == 128)
             return plan.tile_rows == 256 ? launch_gemm_sk_256_narrow(stream, p, plan.grid)
                    : plan.tile_rows == 128 ? launch_gemm_sk_128_narrow(stream, p, plan.grid, eight)
@@ -583,7 +583,7 @@ namespace nnf
         p.units = plan.units;
         p.zps = (const uint8_t*)zero_points;
         set_sync(p, plan, choice, num_cu);
-        const bool eight = workspace::sk_eight_wavefronts(plan, false, false, num_cu);
+        const bool eight = workspace::sk_eight_wavefronts(plan, false, false, num_cu, (N & 7) != 0);
         switch (group_shift)
         {
         case 5: return launch_gemm_sk_q5(stream, p, plan.grid, plan.tile_rows, plan.tile_weight_rows, eight);

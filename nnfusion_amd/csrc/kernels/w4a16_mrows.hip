@@ -531,9 +531,10 @@ namespace nnf
         // everything that is done to them starts only then; weights behind all activations are asked for late (a CU has
         // about 64 loads in flight).  So: as many blocks of activations as LDS has room for, the weights, the rest.
         // Measured (us a launch in a graph, weights from memory, N = K = 4096 plain / with RMSNorm / with a residual): 6 rows 5.00 / 7.46 /
-        // 5.95 with the weights first and RMSNorm's weight last, 4.42 / 5.32 / 4.75 now; 16 rows 5.46 / 6.88 / 6.00, now 5.43 / 6.08 /
-        // 5.46.  (Three blocks of 16 rows in flight 0.1 slower, one block ahead of the weights and the others behind 0.2 at 6 rows, a
-        // barrier between activations and weights 0 - 0.3.)
+        // 5.95 with the weights first and RMSNorm's weight last, 4.42 / 5.32 / 4.75 now; 16 rows 5.60 / 6.96 / 6.22, now 5.82 / 6.50 /
+        // 6.00: nine rows and more of a plain product at K = 4096 lose 2 - 6 % (16 x 256 4.10 -> 4.35), of K = 3072 up to 4 %; with
+        // the weights first they do so as well, so it is not the order.  (Three blocks of 16 rows in flight 0.1 slower, one block
+        // ahead of the weights and the others behind 0.2 at 6 rows, a barrier between activations and weights 0 - 0.3.)
         // The RMSNorm weight of the wavefront's k positions (GA x 256 bytes) comes through LDS as well, one load per four groups.
         uint8_t* stage = red + wave * (2 * ROW_BLOCK_BYTES);
         const uint8_t* gamma_block = red + MR_WAVES * (2 * ROW_BLOCK_BYTES) + wave * (GAMMA_LOADS * 1024);

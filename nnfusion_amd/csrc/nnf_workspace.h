@@ -396,9 +396,14 @@ namespace nnf
         // The faster kernel takes power from its neighbours.  70 products of 128 x 128 tiles on 193 .. 255 CUs from eight
         // supersteps on, by themselves 1.047, with pauses 1.039, behind 64 x 4096 x 4096 1.039, behind the product that leads
         // back to their K 1.035, each for the whole sequence; behind two of M x 11008 x 4096 0.997 (0.93 .. 1.05).
-        inline bool sk_eight_wavefronts(const SkPlan& p, bool gate, bool rms, int num_cu)
+        // ragged: columns that are no multiple of eight, whose rows are written an element at a time: from strips of 32 columns that takes
+        // longer than from strips of 64 (tiles 256 wide on more than half of the CUs, K = 1024 .. 4096: 0.84 - 1.0, 1029 x 16190 x 1024 in
+        // groups of 64 0.84, 300 x 16190 x 4096 0.93).
+        inline bool sk_eight_wavefronts(const SkPlan& p, bool gate, bool rms, int num_cu, bool ragged = false)
         {
             if ((p.tile_rows != 64 && p.tile_rows != 128) || p.grid < 1)
+                return false;
+            if (ragged && !gate && p.tile_weight_rows == 256 && 2ll * p.grid > num_cu)
                 return false;
             const long long tiles = (long long)p.tiles_m * p.tiles_n, share = p.units / p.grid;
             const bool one_each = p.grid == tiles, parts = p.grid > tiles && p.grid % tiles == 0;

@@ -1446,6 +1446,10 @@ int main(int argc, char** argv)
                 const ws::SkPlan p = ws::plan_w4a16_tiles_q(s[0], s[1], s[2], 256, 0);
                 EXPECT(p.tile_rows == 128 && p.tile_weight_rows == 128 && p.grid > 192 && p.grid == p.tiles_m * p.tiles_n);
                 EXPECT(ws::sk_eight_wavefronts(p, false, false, 256));
+                // ... not on 128 x 256 with columns that are no multiple of eight
+                const ws::SkPlan r = ws::plan_w4a16_tiles_q(1029, 5698, 4096, 256);
+                EXPECT(r.tile_rows == 128 && r.tile_weight_rows == 256 && r.grid == 207);
+                EXPECT(ws::sk_eight_wavefronts(r, false, false, 256) && !ws::sk_eight_wavefronts(r, false, false, 256, true));
             }
             // the test of its odd multiples of 128: tile, wavefronts and split of every case, with and without synchronisation words
             enum { WHOLE, PARTS, EVEN };

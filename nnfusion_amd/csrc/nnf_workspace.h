@@ -883,9 +883,11 @@ namespace nnf
         // 0.76 - 0.97 up to 300 000 outputs, 1.0 - 1.57 from 320 000 on; K = 6272 0.90 - 0.96 up to 102 000, 0.99 - 1.6 above, from 8576
         // on 0.96 - 1.17 there as well.  Up to 128 rows and 1024 columns, where the plan is an even split whose shares of two
         // supersteps straddle tiles: 153 products 0.93 (0.80 .. 1.18); with equal parts of tiles 165 products 1.08 (0.94 .. 1.34).
+        // Columns that are no multiple of eight, which this kernel writes an element at a time (2050 .. 16190 columns, 300 .. 1500 rows):
+        // K = 1152 0.67 - 0.88, 1408 0.71 - 0.93, 2176 0.82 - 1.15 (0.95 in the mean), 2688 0.89 - 1.33 (1.03), 4224 1.0 - 1.4.
         inline bool w4a16_gemm_q_odd_fits(int M, int N, int K, int group_shift)
         {
-            if ((K & 255) != 128 || !w4a16_gemm_q_addressable(M, N, K, group_shift))
+            if ((K & 255) != 128 || ((N & 7) && K < 2688) || !w4a16_gemm_q_addressable(M, N, K, group_shift))
                 return false;
             if (M <= 128 && N <= 1024)
             {

@@ -1454,15 +1454,15 @@ int main(int argc, char** argv)
             // the test of its odd multiples of 128: tile, wavefronts and split of every case, with and without synchronisation words
             enum { WHOLE, PARTS, EVEN };
             const int odd[][7] = {{17, 12479, 8320, 32, 256, 0, PARTS}, {18, 12368, 10368, 32, 256, 0, EVEN},
-                                  {34, 8407, 12160, 64, 128, 1, PARTS}, {99, 8405, 1152, 64, 128, 1, WHOLE},
+                                  {34, 8407, 12160, 64, 128, 1, PARTS}, {99, 8408, 1152, 64, 128, 1, WHOLE},
                                   {65, 528, 6272, 64, 128, 0, PARTS}, {37, 8202, 8832, 64, 128, 0, EVEN},
-                                  {65, 11910, 8320, 128, 128, 1, PARTS}, {526, 803, 1152, 128, 128, 1, WHOLE},
-                                  {65, 512, 7040, 128, 128, 0, PARTS}, {132, 10994, 1152, 128, 128, 0, WHOLE},
-                                  {1287, 12013, 1152, 128, 256, 1, EVEN}, {260, 11121, 1152, 128, 256, 1, WHOLE},
+                                  {65, 11910, 8320, 128, 128, 1, PARTS}, {526, 808, 1152, 128, 128, 1, WHOLE},
+                                  {65, 512, 7040, 128, 128, 0, PARTS}, {132, 11000, 1152, 128, 128, 0, WHOLE},
+                                  {1287, 12016, 1152, 128, 256, 1, EVEN}, {260, 11128, 1152, 128, 256, 1, WHOLE},
                                   {65, 11184, 6784, 128, 256, 0, PARTS}, {261, 3746, 11392, 128, 256, 0, EVEN},
-                                  {387, 8291, 1152, 256, 128, 0, WHOLE}, {2060, 269, 2176, 256, 128, 0, PARTS},
-                                  {523, 13487, 1152, 256, 256, 0, WHOLE}, {135, 11914, 11136, 256, 256, 0, PARTS},
-                                  {1566, 10194, 2432, 256, 256, 0, EVEN}};
+                                  {387, 8296, 1152, 256, 128, 0, WHOLE}, {2060, 272, 2176, 256, 128, 0, PARTS},
+                                  {523, 13488, 1152, 256, 256, 0, WHOLE}, {135, 11914, 11136, 256, 256, 0, PARTS},
+                                  {1566, 10200, 2432, 256, 256, 0, EVEN}};
             for (const auto& s : odd)
                 for (int gs = 5; gs <= 7; ++gs)
                     for (size_t sync : {(size_t)0, (size_t)64 << 10})
@@ -1473,10 +1473,11 @@ int main(int argc, char** argv)
                         EXPECT(p.tile_rows == s[3] && p.tile_weight_rows == s[4] && split == s[6]);
                         EXPECT(ws::sk_eight_wavefronts(p, false, false, 256) == (s[5] != 0));
                     }
-            // ... few columns stay on the plain kernel where a few dozen tiles are all there is
+            // ... few columns stay on the plain kernel where a few dozen tiles are all there is, and so do columns that are no multiple of eight of short K
             const int few[][4] = {{650, 192, 2688, 0}, {1318, 192, 2176, 0}, {1000, 256, 2176, 0}, {400, 256, 6272, 0}, {257, 320, 3456, 0}, {256, 511, 16256, 0},
                                   {1318, 256, 2176, 1}, {1000, 320, 2688, 1}, {650, 192, 3456, 1}, {400, 320, 6272, 1}, {257, 192, 8320, 1}, {150, 512, 8576, 1}, {65, 512, 6272, 0},
-                                  {128, 768, 6784, 0}, {128, 640, 8320, 1}, {128, 1025, 6272, 1}};
+                                  {128, 768, 6784, 0}, {128, 640, 8320, 1}, {128, 1025, 6272, 1}, {861, 16190, 1152, 0}, {861, 16192, 1152, 1}, {520, 4100, 2432, 0},
+                                  {520, 4097, 2688, 1}};
             for (const auto& s : few)
                 EXPECT(ws::w4a16_gemm_q_odd_fits(s[0], s[1], s[2], 6) == (s[3] != 0));
             // by itself the library runs no W8A8 product over two ranges of K on the row-streaming kernel: the K-streaming kernel takes them all

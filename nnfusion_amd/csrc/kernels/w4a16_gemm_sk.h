@@ -576,45 +576,80 @@ namespace nnf
         sk_finish_round<1, TN, GATE, BIAS, RESID, RMS>(p, c, r, m0, n0, stage, wave, lane);
     }
 
-    // rstd[m] = rsqrt(mean_k(A[m, k]^2) + eps) for rows first, first + step, ... < end, a row by 256 threads of a workgroup
-    // (the summation order of the pre-pass kernel, rms_rstd_kernel: same bits), stored at device scope; complete for
-    // every thread of the workgroup on return.  part: a float of LDS per wavefront.
-    template <int THREADS>
+    // rstd[m] = rsqrt(mean_k(A[m, k]^2) + eps) for rows first, first + step, ... < end, stored at device scope; complete for
+    // every thread of the workgroup on return.  The summation order is that of the pre-pass kernel (rms_rstd_kernel: a row by
+    // four wavefronts): same bits.  A row or two: four wavefronts each, their sums through `part`, a float of LDS per wavefront.
+    // More of them: a row by every wavefront, which keeps the four partial sums side by side and knows no barrier, where four
+    // wavefronts took 0.7 us a row whatever its length (64-row tiles of few columns, with SiLU-gate: 593 x 324 x 512 33.3 -> 22.8 us,
+    // 756 x 704 x 768 26.4 -> 20.2; 887 x 512 x 14848 without 44.8 -> 42.2; one row a workgroup 3 - 4 % slower that way, two of
+    // more than the 8192 values a wavefront has in flight 5 %: 346 x 1164 x 9472 36.1 / 38.1 us).
+    __device__ __forceinline__ void sk_square_sum(float& ss, const uintx4& v)
+    {
+        const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            const half2_t hh = as_half2(vv[j]);
+            ss += (float)hh.x * (float)hh.x + (float)hh.y * (float)hh.y;
+        }
+    }
+    // (ACC: the workgroup's sums are in registers: four wavefronts a row whatever there is to do, which takes fewer of them -- 128 x 128
+    // tiles run two workgroups a CU by their registers.)
+    template <int THREADS, bool ACC>
     __device__ __forceinline__ void sk_rstd_rows(const SkGemmParams& p, int first, int end, int step, float* part, int tid)
     {
-        constexpr int ROWS = THREADS / 256; // at a time
-        const int units = p.K >> 3;
-        for (int m0 = first; m0 < end; m0 += ROWS * step)
+        constexpr int WAVES = THREADS / 64, ROWS = THREADS / 256; // ROWS: by four wavefronts each at a time
+        const int units = p.K >> 3, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const auto store = [&](int m, float s0, float s1, float s2, float s3) {
+            __hip_atomic_store(p.rstd_out + m, 1.0f / __builtin_sqrtf(((s0 + s1) + (s2 + s3)) / (float)p.K + p.rms_eps), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        };
+        if (ACC || first + (units <= 1024 ? ROWS : 2 * ROWS) * step >= end)
         {
-            const int m = m0 + (ROWS > 1 ? tid >> 8 : 0) * step;
-            if (m < end)
+            for (int m0 = first; m0 < end; m0 += ROWS * step)
+            {
+                const int m = m0 + (ROWS > 1 ? wave >> 2 : 0) * step;
+                if (m < end)
+                {
+                    const uintx4* row = reinterpret_cast<const uintx4*>(p.A + (size_t)m * p.K);
+                    float ss = 0.f;
+                    for (int i = ROWS > 1 ? tid & 255 : tid; i < units; i += 256)
+                        sk_square_sum(ss, row[i]);
+                    ss = wave_sum(ss);
+                    if (lane == 0)
+                        part[wave] = ss;
+                }
+                __syncthreads();
+                if ((ROWS > 1 ? tid & 255 : tid) == 0 && m < end)
+                    store(m, part[wave], part[wave + 1], part[wave + 2], part[wave + 3]);
+                __syncthreads(); // (`part` has been read)
+            }
+        }
+        else
+            for (int m = first + wave * step; m < end; m += WAVES * step)
             {
                 const uintx4* row = reinterpret_cast<const uintx4*>(p.A + (size_t)m * p.K);
-                float ss = 0.f;
-                for (int i = ROWS > 1 ? tid & 255 : tid; i < units; i += 256)
+                float ss[4] = {0.f, 0.f, 0.f, 0.f};
+                for (int i0 = 0; i0 < units; i0 += 1024)
                 {
-                    const uintx4 v = row[i];
-                    const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
+                    uintx4 v[16];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                    {
-                        const half2_t hh = as_half2(vv[j]);
-                        ss += (float)hh.x * (float)hh.x + (float)hh.y * (float)hh.y;
-                    }
+                    for (int w = 0; w < 16; ++w)
+                        v[w] = row[min(i0 + w * 64 + lane, units - 1)];
+#pragma unroll
+                    for (int w = 0; w < 16; ++w)
+                        if (i0 + w * 64 < units) // (uniform)
+                        {
+                            const uint32_t in_k = i0 + w * 64 + lane < units ? ~0u : 0u;
+                            sk_square_sum(ss[w & 3], uintx4{v[w].x & in_k, v[w].y & in_k, v[w].z & in_k, v[w].w & in_k});
+                        }
                 }
-                ss = wave_sum(ss);
-                if ((tid & 63) == 0)
-                    part[tid >> 6] = ss;
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    ss[w] = wave_sum(ss[w]);
+                if (lane == 0)
+                    store(m, ss[0], ss[1], ss[2], ss[3]);
             }
-            __syncthreads();
-            if ((ROWS > 1 ? tid & 255 : tid) == 0 && m < end)
-            {
-                const float* four = part + (ROWS > 1 ? tid >> 6 : 0);
-                __hip_atomic_store(p.rstd_out + m, 1.0f / __builtin_sqrtf(((four[0] + four[1]) + (four[2] + four[3])) / (float)p.K + p.rms_eps),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __syncthreads();
-        }
         gemm_sk::wait_vector_memory();
         __syncthreads();
     }
@@ -740,7 +775,7 @@ namespace nnf
             if (p.rstd_out)
             {
                 rstd_ok = false;
-                sk_rstd_rows<T::THREADS>(p, v, p.M, grid, rstd_part, tid);
+                sk_rstd_rows<T::THREADS, false>(p, v, p.M, grid, rstd_part, tid);
                 if (tid == 0)
                     atomicAdd(p.rstd_sync, 1u);
             }
@@ -768,7 +803,7 @@ namespace nnf
                 rstd_ok = rstd_note != 0u;
                 __syncthreads();
                 if (!rstd_ok)
-                    sk_rstd_rows<T::THREADS>(p, m_first, min(m_end, p.M), 1, rstd_part, tid);
+                    sk_rstd_rows<T::THREADS, true>(p, m_first, min(m_end, p.M), 1, rstd_part, tid);
             }
         };
 

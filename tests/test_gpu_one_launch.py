@@ -112,6 +112,30 @@ def test_one_launch_fused_forms(gpu, fused, spin_limit):
         _check(one.cpu().numpy(), ref, 2e-2)
 
 
+# rows a workgroup between one and many, rows shorter and longer than one and two sweeps of a wavefront's 2048 values, the last
+# sweep of 128
+@pytest.mark.parametrize("m,n,k", [(65, 64, 128), (77, 290, 640), (130, 2000, 2048), (131, 1100, 2176), (300, 130, 4096), (513, 600, 4224),
+                                   (700, 96, 384)])
+def test_rstd_of_many_rows_a_workgroup_bit_for_bit(gpu, m, n, k):
+    """Rows by one wavefront each: the bits of the pre-pass, in every form, on tiles of four and eight wavefronts."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    a, wq, s = datagen.w4a16_case(m + k, m, 2 * n, k)
+    gamma = (1.0 + 0.1 * np.random.default_rng(m).standard_normal(k)).astype(np.float16)
+    ta, tw, ts, tg = _t(gpu, a, wq, s, gamma)
+    sync = ops.sync_flags(gpu)
+    for act, plan in ((0, (64, 1, 128)), (0, (128, 1, 128)), (0, (128, 0, 256)), (1, (64, 1)), (1, (128, 1)), (0, (256, 1, 256))):
+        w_, s_ = (tw, ts) if act else (tw[:n].contiguous(), ts[:n].contiguous())
+        kw = dict(rms_gamma=tg, act=act, variant="gemm_mfma", plan=plan)
+        two = ops.w4a16_gemm_fused(ta, w_, s_, **kw)
+        for spin_limit in (0, -1):
+            one = ops.w4a16_gemm_fused(ta, w_, s_, sync=sync, spin_limit=spin_limit, **kw)
+            assert torch.equal(one, two)
+            assert not sync.any()
+
+
 @pytest.mark.parametrize("m,k", [(300, 1024), (1000, 4096)])
 def test_rstd_inside_the_launch_with_more_rows_than_workgroups(gpu, m, k):
     """More activation rows than the launch has workgroups: each adds up the squares of several rows."""

@@ -374,10 +374,12 @@ namespace nnf
         // (the row-streaming kernels add up the squares of the activations they hold themselves: no pre-pass; the form
         // with a run-time K keeps it)
         const bool normalised_copy = route.normalised_copy;
-        const workspace::SkPlan plan = route.kind == W4A16Route::TILE
+        workspace::SkPlan plan = route.kind == W4A16Route::TILE
                                            ? workspace::w4a16_launch_plan(route, M, N, K, gate, rms, num_cu,
                                                                           choice.sync_flags ? choice.sync_bytes : 0)
                                            : workspace::SkPlan();
+        if (route.kind == W4A16Route::TILE && route.own_plan)
+            plan = workspace::plan_w4a16_192(plan, M, N, K, gate, num_cu);
         const bool rstd_in_tile_gemm = rms && route.kind == W4A16Route::TILE && rstd_inside_tile_gemm(plan, choice, num_cu);
         const bool rstd_in_kernel = route.kind == W4A16Route::ROWS ||
                                     (route.kind == W4A16Route::MROWS && workspace::w4a16_mrows_fixed_k(M, K)) || rstd_in_tile_gemm;
@@ -485,6 +487,8 @@ namespace nnf
             p.rms_eps = rms_eps;
         }
         const bool eight = workspace::sk_eight_wavefronts(plan, gate, rms, num_cu, (N & 7) != 0);
+        if (plan.tile_weight_rows == 192)
+            return launch_gemm_sk_192(stream, p, plan.grid, gate);
         if (plan.tile_weight_rows == 128)
             return plan.tile_rows == 256 ? launch_gemm_sk_256_narrow(stream, p, plan.grid)
                    : plan.tile_rows == 128 ? launch_gemm_sk_128_narrow(stream, p, plan.grid, eight)

@@ -152,6 +152,7 @@ namespace nnf
             static_assert(WAVES * EXCHANGE_BYTES <= LDS_BYTES && LDS_BYTES <= 160 * 1024 - 64, "LDS of a CU");
             static_assert(TM % KH == 0 && OWN % ROUND == 0 && A_LOADS * NW == TM * 4, "whole blocks and loads a wavefront");
             static constexpr size_t SLOT_FLOATS = (size_t)BM * BN;
+            static constexpr bool SHARED = TN != 3; // its tiles may belong to several workgroups
         };
 
         // Rows x columns (weight rows) of a tile -> the wavefronts that work on it.  EIGHT: two a SIMD instead of one (64- and
@@ -197,6 +198,10 @@ namespace nnf
         };
         template <>
         struct TileOf<128, 256, true> : Tile<4, 1, 8, 1>
+        {
+        };
+        template <>
+        struct TileOf<128, 192> : Tile<4, 3, 2, 2>
         {
         };
         template <>
@@ -383,11 +388,12 @@ namespace nnf
     {
         constexpr int OUT_COLS = GATE ? TN * 16 : TN * 32; // of the wavefront's strip
         constexpr int PITCH = OUT_COLS * 2 + 16; // bytes per staged row (padding spreads the banks)
-        constexpr int LANES_PER_ROW = OUT_COLS / 8, ROWS_PER_READ = 64 / LANES_PER_ROW;
-        // a gate value's element and its up value's: in the same place of the column tile TN / 2 further, or (one column
-        // tile, 16 gate and 16 up rows) eight elements further
-        constexpr int OUT_TN = GATE ? (TN + 1) / 2 : TN, OUT_GROUPS = GATE && TN == 1 ? 2 : 4;
-        constexpr int UP_J = GATE ? TN / 2 : 0, UP_E = GATE && TN == 1 ? 8 : 0;
+        constexpr int LANES_PER_ROW = OUT_COLS / 8, ROWS_PER_READ = 64 / LANES_PER_ROW; // (TN = 3: the last four lanes have none)
+        // a gate value's element and its up value's: in the same place of the column tile TN / 2 further, or (an odd number of column
+        // tiles, of 16 gate and 16 up rows each) eight elements further
+        constexpr bool HALVES = GATE && (TN & 1);
+        constexpr int OUT_TN = GATE && !HALVES ? TN / 2 : TN, OUT_GROUPS = HALVES ? 2 : 4, OUT_TILE = HALVES ? 16 : 32;
+        constexpr int UP_J = GATE && !HALVES ? TN / 2 : 0, UP_E = HALVES ? 8 : 0;
         const int l32 = lane & 31, h = lane >> 5;
         const int n_wave = n0 + wave * OUT_COLS;
         const int piece = lane % LANES_PER_ROW;
@@ -429,14 +435,16 @@ namespace nnf
                             y[k] = (half_t)(RMS ? c[ii][j][4 * g + k] * rs : c[ii][j][4 * g + k]);
                         }
                     }
-                    *reinterpret_cast<half4_t*>(region + (ii * 32 + l32) * PITCH + (j * 32 + 8 * g + 4 * h) * 2) = y;
+                    *reinterpret_cast<half4_t*>(region + (ii * 32 + l32) * PITCH + (j * OUT_TILE + 8 * g + 4 * h) * 2) = y;
                 }
         }
         // LDS operations of one wavefront execute in order: no barrier around the private region
 #pragma unroll
-        for (int it = 0; it < ROUND_TM * 32 / ROWS_PER_READ; ++it)
+        for (int it = 0; it < (ROUND_TM * 32 + ROWS_PER_READ - 1) / ROWS_PER_READ; ++it)
         {
             const int row = it * ROWS_PER_READ + lane / LANES_PER_ROW;
+            if (ROWS_PER_READ * LANES_PER_ROW < 64 && (lane >= ROWS_PER_READ * LANES_PER_ROW || row >= ROUND_TM * 32))
+                continue;
             half8_t o = *reinterpret_cast<const half8_t*>(region + row * PITCH + piece * 16);
             const int m = m0 + r * (ROUND_TM * 32) + row;
             if (m >= p.M || n_lane >= p.N)
@@ -718,7 +726,7 @@ namespace nnf
         constexpr int AL = T::A_LOADS;
         using SCH = Sched<AL, TN, RMS, WL>;
         static_assert(!(GATE && (BIAS || RESID)), "SiLU-gate is not combined with bias or residual");
-        static_assert(TN == 1 || TN == 2 || TN == 4, "column tiles per wavefront");
+        static_assert(TN >= 1 && TN <= 4, "column tiles per wavefront");
         static_assert(QG == 0 || (QG >= 5 && QG <= 7), "groups of 32, 64 or 128");
         constexpr bool QZ = QG != 0;
         constexpr int GSH = QZ ? QG : 7;                    // log2 of the group size
@@ -840,7 +848,7 @@ namespace nnf
             const int ss_begin = (int)(u - (long long)tile * SS);
             const int ss_end = (int)min((long long)SS, ss_begin + (u_end - u));
             const int NSS = ss_end - ss_begin;
-            const bool whole = NSS == SS;
+            const bool whole = !T::SHARED || NSS == SS;
             const bool first_of_mine = u == u_begin;
             u += NSS;
             int tm, tn;
@@ -923,8 +931,8 @@ namespace nnf
             // when the superstep begins.
             // the row of the wavefront's column tile j that sits at place r (0 .. 31)
             auto weight_row = [&](int j, int r) {
-                if (GATE && TN == 1) // rows 0 .. 15: gate rows, the others: the up rows that pair with them
-                    return min((r >= 16 ? p.up_row_offset - 16 : 0) + n0 + strip * 16 + r, p.up_row_offset + p.N - 1);
+                if (GATE && (TN & 1)) // rows 0 .. 15: gate rows, the others: the up rows that pair with them
+                    return min((r >= 16 ? p.up_row_offset - 16 : 0) + n0 + (strip * TN + j) * 16 + r, p.up_row_offset + p.N - 1);
                 if (GATE) // column tiles 0 .. TN/2-1: gate rows, the others: the up rows that pair with them
                     return min((j >= TN / 2 ? p.up_row_offset + n0 + (j - TN / 2) * 32 : n0 + j * 32) + strip * (TN / 2) * 32 + r,
                                p.up_row_offset + p.N - 1);
@@ -1523,7 +1531,7 @@ namespace nnf
         // Every workgroup has counted itself in at all its tiles before it waits here, so the waits cannot form a
         // cycle; they are bounded all the same (workgroups of a grid that is not resident as a whole): a workgroup
         // whose wait runs out marks its blocks for the last arriver, who never waits.
-        if (p.sync && (pend_tile[0] >= 0 || pend_tile[1] >= 0))
+        if (T::SHARED && p.sync && (pend_tile[0] >= 0 || pend_tile[1] >= 0))
         {
             __syncthreads(); // the epilogue's staging regions are free
             uint8_t* stage = smem + wave * sk_region_bytes<1, TN, GATE>();

@@ -27,17 +27,22 @@ namespace nnf
         template <class T, bool GATE, bool BIAS, bool RESID, bool RMS, int QG = 0>
         hipError_t launch_instance(hipStream_t stream, const SkGemmParams& p, int grid)
         {
-            const hipError_t e = (p.K & 128) ? launch_product<T, GATE, BIAS, RESID, RMS, QG, true>(stream, p, grid)
-                                             : launch_product<T, GATE, BIAS, RESID, RMS, QG, false>(stream, p, grid);
-            if (e != hipSuccess || !p.partial || p.sync)
-                return e;
-            // tiles shared by several workgroups: their parts are added and finished by a second launch (unless the
-            // workgroups did it themselves: p.sync); it does not depend on the block parameters
-            using Parts = Tile<T::TM, T::TN, T::NW, T::KH>;
-            constexpr int ROUNDS = T::TM; // blocks of 32 rows
-            hipLaunchKernelGGL((w4a16_gemm_sk_fixup_kernel<Parts, GATE, BIAS, RESID, RMS>), dim3(p.tiles_m * p.tiles_n * ROUNDS * T::NW),
-                               dim3(64), 0, stream, p, grid);
-            return hipGetLastError();
+            if constexpr (!T::SHARED) // (even multiples of 128 only, too)
+                return launch_product<T, GATE, BIAS, RESID, RMS, QG, false>(stream, p, grid);
+            else
+            {
+                const hipError_t e = (p.K & 128) ? launch_product<T, GATE, BIAS, RESID, RMS, QG, true>(stream, p, grid)
+                                                 : launch_product<T, GATE, BIAS, RESID, RMS, QG, false>(stream, p, grid);
+                if (e != hipSuccess || !p.partial || p.sync)
+                    return e;
+                // tiles shared by several workgroups: their parts are added and finished by a second launch (unless the
+                // workgroups did it themselves: p.sync); it does not depend on the block parameters
+                using Parts = Tile<T::TM, T::TN, T::NW, T::KH>;
+                constexpr int ROUNDS = T::TM; // blocks of 32 rows
+                hipLaunchKernelGGL((w4a16_gemm_sk_fixup_kernel<Parts, GATE, BIAS, RESID, RMS>), dim3(p.tiles_m * p.tiles_n * ROUNDS * T::NW),
+                                   dim3(64), 0, stream, p, grid);
+                return hipGetLastError();
+            }
         }
 
         template <class T>
@@ -114,4 +119,6 @@ namespace nnf
     hipError_t launch_gemm_sk_64(hipStream_t stream, const SkGemmParams& p, int grid, bool gate, bool eight);
     hipError_t launch_gemm_sk_128(hipStream_t stream, const SkGemmParams& p, int grid, bool gate, bool eight);
     hipError_t launch_gemm_sk_256(hipStream_t stream, const SkGemmParams& p, int grid, bool gate);
+    // tiles of 128 x 192, whole ones (w4a16_gemm_sk_192.hip)
+    hipError_t launch_gemm_sk_192(hipStream_t stream, const SkGemmParams& p, int grid, bool gate);
 } // namespace nnf

@@ -423,6 +423,29 @@ namespace nnf
                 return 8ll * p.grid <= 5ll * num_cu && share < 32;
             return (!gate && p.supersteps < 8) || (rms && share < 16);
         }
+        // Whole tiles of 128 x 192 (gemm_sk::TileOf<128, 192>: half of what a K step reads from LDS a weight, every wavefront three strips of
+        // 32 columns over half of K) in place of the plan `other`, where they fill more than two thirds of the CUs and no more than all:
+        // tiles of 128 x 256 leave a third idle there, those of 128 x 128 are too many for one round.  450 products of 100 .. 1600
+        // rows: 1.05 - 1.17 x from there to the full chip (256 x 22016 x 4096 with RMSNorm and SiLU-gate 59.6 -> 54.4 us on 230 tiles), 0.6 - 0.9 on
+        // fewer tiles and 0.6 - 0.8 on a few more than CUs; two rounds of them 0.93 - 1.04.  Below ten supersteps the sums that the halves of
+        // K trade behind the loop cost more (0.91 - 1.06); above 40 and below three quarters of the CUs ranges of K are
+        // ahead (0.96); and so are 64-row tiles where they are the plan's, of 129 .. 192 rows (0.91 - 0.98).
+        inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu)
+        {
+            SkPlan p;
+            p.tile_rows = 128;
+            p.tile_weight_rows = 192;
+            p.tiles_m = ceil_div(M, 128);
+            p.tiles_n = ceil_div(N, gate ? 96 : 192);
+            p.supersteps = K / 256;
+            p.units = (long long)p.tiles_m * p.tiles_n * p.supersteps;
+            const long long tiles = (long long)p.tiles_m * p.tiles_n;
+            if (other.grid < 1 || (K & 255) || other.tile_rows == 64 || p.supersteps < 10 || tiles > num_cu || 3 * tiles <= 2ll * num_cu ||
+                (p.supersteps > 40 && 4 * tiles < 3ll * num_cu))
+                return other;
+            p.grid = (int)tiles;
+            return p;
+        }
         inline SkPlan plan_w4a16_tiles(int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = SIZE_MAX)
         {
             return plan_w4a16_tiles(plan_w4a16_sk(M, N, K, gate, num_cu), M, N, K, gate, rms, num_cu, sync_bytes);

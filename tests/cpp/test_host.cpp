@@ -1561,6 +1561,25 @@ int main(int argc, char** argv)
                 EXPECT(ws::plan_w4a16_tiles(1000, 16384, k, false, false, 256).tile_weight_rows == 128);
             EXPECT(ws::plan_w4a16_tiles(1000, 16384, 7168, false, false, 256).tile_weight_rows == 256);
             EXPECT(ws::plan_w4a16_tiles(1300, 128, 896, true, false, 256).slots > 0 && ws::plan_w4a16_tiles(1300, 128, 640, true, false, 256).slots == 0);
+            // whole tiles of 128 x 192 take a plan's place where they nearly fill the CUs (the shapes of the GPU test, plain / SiLU-gate)
+            const auto wide = [](int m, int n, int k, bool gate, int cus) {
+                const auto other = ws::plan_w4a16_tiles(m, n, k, gate, true, cus);
+                const auto p = ws::plan_w4a16_192(other, m, n, k, gate, cus);
+                const long long tiles = (long long)ws::ceil_div(m, 128) * ws::ceil_div(gate ? 2 * n : n, 192);
+                if (p.tile_weight_rows == 192)
+                    EXPECT(p.tile_rows == 128 && p.slots == 0 && p.grid == tiles && p.grid <= cus && k % 256 == 0 && p.supersteps * 256 == k);
+                else
+                    EXPECT(p.grid == other.grid && p.tile_rows == other.tile_rows && p.tile_weight_rows == other.tile_weight_rows);
+                return p.tile_weight_rows == 192;
+            };
+            const int wide_shapes[][4] = {{300, 11300, 5601, 2560}, {257, 11523, 5555, 2816}, {700, 6200, 3000, 3072}, {513, 9216, 4608, 2560},
+                                          {1000, 4608, 2310, 4096}, {201, 24500, 12199, 2816}};
+            for (const auto& s : wide_shapes)
+                EXPECT(wide(s[0], s[1], s[3], false, 256) && wide(s[0], s[2], s[3], true, 256) && !wide(s[0], s[1], s[3] + 128, false, 256) &&
+                       !wide(s[0], s[1] / 2, s[3], false, 256) && !wide(s[0], s[1], 2304, false, 256));
+            EXPECT(wide(256, 11008, 4096, true, 256) && !wide(256, 12288, 4096, false, 256) && !wide(183, 8192, 11264, true, 256));
+            for (int i = 0; i < 2000; ++i)
+                wide(65 + draw(0, 2000), draw(1, 1 << draw(8, 14)), 128 * draw(1, 100), draw(0, 1) != 0, i % 5 == 0 ? draw(1, 304) : 256);
             // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
             const auto walk_slots = [](const ws::SkPlan& p) {
                 const long long G = p.supersteps;

@@ -607,3 +607,41 @@ def test_four_and_eight_wavefronts(gpu, m, n, k, rows, parts, cols):
         assert float((one.float() - ref).norm() / ref.norm()) <= tol
         assert float((one.float() - ref).abs().max() / ref.pow(2).mean().sqrt()) <= (2e-2 if "act" in kw else TOL)
         assert not sync.any()
+
+
+# Whole tiles of 128 x 192: even and odd numbers of supersteps, the last tile of rows and columns ragged (columns no multiple of eight
+# too: stored an element at a time), N = the plain form's and the SiLU-gate form's outputs, both within the rule
+@pytest.mark.parametrize("m,n_plain,n_gate,k", [(300, 11300, 5601, 2560), (257, 11523, 5555, 2816), (700, 6200, 3000, 3072), (513, 9216, 4608, 2560),
+                                                (1000, 4608, 2310, 4096), (201, 24500, 12199, 2816)])
+def test_tiles_of_192_columns(gpu, m, n_plain, n_gate, k):
+    """Against float32 products of the same values, bounds as for the other tiles (test_four_and_eight_wavefronts); with and without
+    synchronisation words bit for bit."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case M={m} N={n_plain}/{n_gate} K={k}", flush=True)
+    n = max(n_plain, 2 * n_gate)
+    a, wq, s = datagen.w4a16_case(m + n + k, m, n, k)
+    gamma = datagen.normal_f16(m, datagen.S_GAMMA, (k,), 1.0, 0.1)
+    res = datagen.normal_f16(m, datagen.S_RES, (m, n_plain))
+    bias = datagen.normal_f16(m, datagen.S_BIAS, (n_plain,))
+    a, wq, s, gamma, res, bias = _t(gpu, a, wq, s, gamma, res, bias)
+    q = torch.stack((wq & 15, wq >> 4), dim=2).reshape(n, k).float() - 8
+    w = q * s.float().repeat_interleave(128, dim=1)
+    x = a.float()
+    xn = x * torch.rsqrt(x.pow(2).mean(dim=1, keepdim=True) + 1e-6) * gamma.float()
+    wp, sp, wg, sg = (t[:c].contiguous() for c in (n_plain, 2 * n_gate) for t in (wq, s))
+    gate, up = (xn @ w[:2 * n_gate].t()).split(n_gate, dim=1)
+    plain, normed = x @ w[:n_plain].t(), xn @ w[:n_plain].t()
+    sync = ops.sync_flags(gpu)
+    for w_, s_, kw, ref, tol in ((wg, sg, dict(act=1, rms_gamma=gamma), torch.nn.functional.silu(gate) * up, 2e-3), (wp, sp, {}, plain, 1e-3),
+                                 (wp, sp, dict(rms_gamma=gamma, residual=res), normed + res.float(), 1e-3),
+                                 (wp, sp, dict(bias=bias, residual=res), plain + bias.float() + res.float(), 1e-3),
+                                 (wp, sp, dict(rms_gamma=gamma, bias=bias), normed + bias.float(), 1e-3)):
+        one = ops.w4a16_gemm_fused(a, w_, s_, variant="gemm_mfma", plan=(0, 0, 0), sync=sync, **kw)
+        two = ops.w4a16_gemm_fused(a, w_, s_, variant="gemm_mfma", plan=(0, 0, 0), **kw)
+        assert torch.equal(one, two)
+        assert float((one.float() - ref).norm() / ref.norm()) <= tol
+        assert float((one.float() - ref).abs().max() / ref.pow(2).mean().sqrt()) <= (2e-2 if "act" in kw else TOL)
+        assert not sync.any()

@@ -234,4 +234,22 @@ namespace nnf
             v += __shfl_xor(v, off, WAVE);
         return v;
     }
+    // A wavefront's priority counts down over its last four steps (3 ahead of the first, `left` steps behind this one, LAST: none).  Of
+    // two wavefronts of a SIMD the hardware issues the older first, which runs ahead of the other by a step and more and leaves it alone
+    // at the end, with nothing to issue while it waits; this way whichever is behind goes first and both end together.  (Four levels for
+    // all steps: the same with four, half of it with eight.  For the loads of a step alone: nothing.  A chain of compares ahead of every
+    // step took 0.1 us of a launch of 4.)
+    template <bool LAST>
+    __device__ __forceinline__ void count_down_priority(int left)
+    {
+        if constexpr (LAST)
+            __builtin_amdgcn_s_setprio(0);
+        else if (left <= 2)
+        {
+            if (left == 1)
+                __builtin_amdgcn_s_setprio(1);
+            else
+                __builtin_amdgcn_s_setprio(2);
+        }
+    }
 } // namespace nnf

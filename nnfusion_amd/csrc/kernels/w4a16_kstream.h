@@ -284,6 +284,7 @@ namespace nnf
             constexpr int AHEAD = decltype(ahead)::value;
             constexpr bool FULL = AHEAD == D;
             constexpr int LATER = FULL ? (D - 1) * L : AHEAD * L; // of later chunks, asked for before this one began
+            count_down_priority<AHEAD == 0>(chunks - 1 - c);
             const int g = group_of(c), gn = group_of(c + D);
             const uint8_t* slot = at_slot;
             uintx4 gm[4];
@@ -516,6 +517,7 @@ namespace nnf
             if constexpr (D > 1)
                 at_slot = at_slot == ring + (D - 1) * SLOT ? ring : at_slot + SLOT;
         };
+        __builtin_amdgcn_s_setprio(3);
         int c = 0;
         for (; c < chunks - D; ++c)
             chunk(c, std::integral_constant<int, D>());

@@ -112,7 +112,6 @@ namespace nnf
             // where their place has just been read; the wait counts are the loads that follow the one waited for (LAST: no next chunk).
             auto chunk = [&](int c, auto last) {
                 constexpr bool LAST = decltype(last)::value;
-                count_down_priority<LAST>(chunks - 1 - c);
                 const int next = unit_of(c + 1);
                 intx4 areg[MB][J];
                 unroll_for<0, MB>([&](auto mb_c) {
@@ -153,7 +152,6 @@ namespace nnf
                             acc[t][mb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(areg[mb][j], wv[j], acc[t][mb], 0, 0, 0);
                 });
             };
-            __builtin_amdgcn_s_setprio(3);
             for (int c = 0; c < chunks - 1; ++c)
                 chunk(c, std::false_type());
             if (chunks > 0)

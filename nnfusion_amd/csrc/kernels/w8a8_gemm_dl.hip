@@ -56,11 +56,11 @@ namespace nnf
             static constexpr int STAGE_BYTES = A_TILE_BYTES + W_TILE_BYTES;
             static constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
             // a wavefront-wide load covers 16 rows of 64 bytes or 8 of 128; every wavefront issues the same number of loads
-            // (with fewer chunks than wavefronts two wavefronts fetch the same chunk into the same place)
+            // (where the chunks are no multiple of the wavefronts two of them fetch the same chunk into the same place)
             static constexpr int A_CHUNKS = BM / ROWS_PER_LOAD;
             static constexpr int W_CHUNKS = BN / ROWS_PER_LOAD;
-            static constexpr int A_LOADS = A_CHUNKS >= WAVES ? A_CHUNKS / WAVES : 1;
-            static constexpr int W_LOADS = W_CHUNKS >= WAVES ? W_CHUNKS / WAVES : 1;
+            static constexpr int A_LOADS = (A_CHUNKS + WAVES - 1) / WAVES;
+            static constexpr int W_LOADS = (W_CHUNKS + WAVES - 1) / WAVES;
             static constexpr int TILE_LOADS = A_LOADS + W_LOADS;
         };
 
@@ -399,7 +399,7 @@ namespace nnf
         // per group of four elements.  They are scaled in registers, turned through a private piece of LDS
         // (the ring is free after the barrier) and written as whole rows of the wavefront's sub-tile, 16
         // bytes per lane.
-        constexpr int ROUND_TM = TM >= 2 ? 2 : 1;  // 32-row blocks per pass through LDS
+        constexpr int ROUND_TM = TM % 2 == 0 ? 2 : 1; // 32-row blocks per pass through LDS
         constexpr int PITCH = TN * 64 + 16;        // bytes per staged row (padding spreads the banks)
         constexpr int REGION = ROUND_TM * 32 * PITCH;
         static_assert(T::WAVES * REGION <= T::LDS_BYTES, "the staging regions reuse the ring");
@@ -445,10 +445,12 @@ namespace nnf
             }
             // LDS operations of one wavefront execute in order: no barrier around the private region
 #pragma unroll
-            for (int it = 0; it < ROUND_TM * 32 / ROWS_PER_READ; ++it)
+            for (int it = 0; it < (ROUND_TM * 32 + ROWS_PER_READ - 1) / ROWS_PER_READ; ++it)
             {
                 const int row = it * ROWS_PER_READ + lane / LANES_PER_ROW;
                 const int piece = lane % LANES_PER_ROW;
+                if (ROWS_PER_READ * LANES_PER_ROW < 64 && (lane >= ROWS_PER_READ * LANES_PER_ROW || row >= ROUND_TM * 32))
+                    continue;
                 const uintx4 v = *reinterpret_cast<const uintx4*>(region + row * PITCH + piece * 16);
                 const int m = m_wave + r * (ROUND_TM * 32) + row;
                 const int n = n_wave + piece * 8;
@@ -565,11 +567,20 @@ namespace nnf
                     return launch_tile<2, 4, 4, 2, 4, RAW, false, 2>(stream, p);
                 e = launch_tile<2, 4, 4, 2, 4, RAW, true, 2>(stream, p);
                 break;
-            case workspace::GEMM_TILE_TALL: // 256 x 128, three stages of 128, one workgroup per CU
+            // 256 x 128, three stages of 128, one workgroup per CU.  Wavefronts of 64 x 64 read four fragments for four MFMAs, of 128 x 32
+            // five, and LDS is what bounds them: 520 products 1.03 x in the geometric mean (0.97 .. 1.25; 3000 x 6144 x 5504 141 -> 136 us)
+            case workspace::GEMM_TILE_TALL:
                 if (!plan.reduce_pass)
-                    return launch_tile<2, 4, 4, 1, 3, RAW, false, 2, 128>(stream, p);
-                e = launch_tile<2, 4, 4, 1, 3, RAW, true, 2, 128>(stream, p);
+                    return launch_tile<4, 2, 2, 2, 3, RAW, false, 2, 128>(stream, p);
+                e = launch_tile<4, 2, 2, 2, 3, RAW, true, 2, 128>(stream, p);
                 break;
+            // whole tiles only; stages of 128, as many as LDS holds.  (256 x 192 with four stages of 64 113 us where two of 128 take 108, on
+            // four wavefronts 115: 2000 x 12288 x 4096.  128 x 192 on four wavefronts is 9 % ahead of eight in part of a round, level in one.)
+            case workspace::GEMM_TILE_256_192: return launch_tile<4, 2, 2, 3, 2, RAW, false, 2, 128>(stream, p);
+            case workspace::GEMM_TILE_192_256: return launch_tile<2, 4, 3, 2, 2, RAW, false, 2, 128>(stream, p);
+            case workspace::GEMM_TILE_128_256: return launch_tile<2, 4, 2, 2, 3, RAW, false, 2, 128>(stream, p);
+            case workspace::GEMM_TILE_192_128: return launch_tile<2, 4, 3, 1, 3, RAW, false, 2, 128>(stream, p);
+            case workspace::GEMM_TILE_128_192: return launch_tile<2, 2, 2, 3, 4, RAW, false, 1, 128>(stream, p);
             case workspace::GEMM_TILE_MID: // 128 x 128: four stages of 128, one workgroup per CU; or three of 64, two per CU
                 if (long_k)
                 {

@@ -23,6 +23,12 @@ namespace nnf
             GEMM_TILE_SMALL = 2, //  64 x 256
             GEMM_TILE_TINY = 3,  //  32 x 256 (not built for W8A8)
             GEMM_TILE_TALL = 4,  // 256 x 128 (W8A8 only: fills the chip where 256 x 256 tiles leave CUs idle)
+            // whole tiles of W8A8 that only the launch chooses (w8a8_whole_tile)
+            GEMM_TILE_256_192 = 5,
+            GEMM_TILE_192_256 = 6,
+            GEMM_TILE_128_256 = 7,
+            GEMM_TILE_192_128 = 8,
+            GEMM_TILE_128_192 = 9,
         };
         struct GemmPlan
         {
@@ -101,7 +107,52 @@ namespace nnf
         {
             return plan_gemm(M, N, K, false, true, forced_tile, forced_splits);
         }
-        // What the launch runs: that plan, but for 64 x 256 tiles, which write their results themselves where K is in one range
+        // More than 128 rows of W8A8: whole tiles of another shape in place of `planned`, where the estimates say they are more than 2 %
+        // faster.  Tiles of 256 x 128 and 128 x 128 alone leave up to half of the CUs idle in the last round: 3000 x 6144 x 5504 is 576 of
+        // 256 x 128, 2.25 rounds in the time of three, and 768 of 128 x 192, three rounds of half the work.  Microseconds, fitted to 520
+        // products of 129 .. 4096 rows (N = 256 .. 16384, K = 512 .. 16384, weights from memory, every shape timed; 10 % rms): rounds of
+        // tiles x start, and per 128 of K a step a round and up to `load` with the CUs busy.  Over ranges of K: the plan's own estimate, which is
+        // a tenth too long.  161 of the 520 are on another tile by it, 1.16 x in the geometric mean, the slowest of them 0.98; the fastest shape of
+        // each would gain all of them 1.048, this gains 1.046.  Of 416 others, short K among them, five are more than 2 % slower (1549 x 9984 x
+        // 1152 32.9 -> 35.0 us, from 128 x 128 tiles two a CU, which the estimate of one a CU places too late).  (192 x 192, on
+        // four wavefronts, is the fastest for three.)
+        inline int w8a8_whole_tile(int M, int N, int K, const GemmPlan& planned)
+        {
+            struct Cost
+            {
+                int tile, rows, cols;
+                double start, step, load;
+            };
+            static const Cost costs[] = {
+                {GEMM_TILE_BIG, 256, 256, 9.77, 1.109, 0.749},     {GEMM_TILE_TALL, 256, 128, 6.50, 0.738, 0.303},
+                {GEMM_TILE_MID, 128, 128, 4.48, 0.359, 0.186},     {GEMM_TILE_256_192, 256, 192, 7.72, 1.036, 0.493},
+                {GEMM_TILE_192_256, 192, 256, 7.80, 1.036, 0.438}, {GEMM_TILE_128_256, 128, 256, 6.61, 0.737, 0.299},
+                {GEMM_TILE_192_128, 192, 128, 5.62, 0.595, 0.207}, {GEMM_TILE_128_192, 128, 192, 7.99, 0.459, 0.247},
+            };
+            if (M <= 128 || K < 512 || planned.tile == GEMM_TILE_SMALL || planned.tile == GEMM_TILE_TINY)
+                return planned.tile;
+            const double steps = K / 128;
+            double best = planned.splits > 1 ? 0.9e6 * estimate_gemm(M, N, K, false, planned.tile, planned.splits, true) : -1.0;
+            const auto estimate = [&](const Cost& c) {
+                const long long tiles = (long long)ceil_div(M, c.rows) * ceil_div(N, c.cols), rounds = (tiles + PLAN_CUS - 1) / PLAN_CUS;
+                const double last = (double)(tiles - (rounds - 1) * PLAN_CUS) / PLAN_CUS;
+                return rounds * (c.start + steps * c.step) + (rounds - 1 + last) * steps * c.load;
+            };
+            for (const Cost& c : costs)
+                if (best < 0.0 && c.tile == planned.tile)
+                    best = estimate(c);
+            best *= 0.98;
+            int tile = planned.tile;
+            for (const Cost& c : costs)
+                if (c.tile >= GEMM_TILE_256_192)
+                {
+                    const double t = estimate(c);
+                    if (t < best)
+                        best = t, tile = c.tile;
+                }
+            return tile;
+        }
+        // What the launch runs: that plan, but for other whole tiles (above) where the caller fixed nothing, and for 64 x 256 tiles, which write their results themselves where K is in one range
         // and whose ranges (never more than the plan's, whose scratch memory is what callers bring) follow a fit of measured
         // times: per round of tiles 3.6 us, per 128 of K 0.47 and up to 0.64 with the CUs busy; ranges 2 us, 0.28 each and their
         // sums at 10 TB/s (1482 timings, 17 .. 64 rows, 64 %: within 3 %).  33 .. 64 rows: 7 % faster in the geometric mean of
@@ -110,7 +161,12 @@ namespace nnf
         {
             GemmPlan p = plan_w8a8_gemm(M, N, K, forced_tile, forced_splits);
             if (p.tile != GEMM_TILE_SMALL)
+            {
+                const int tile = forced_tile == -1 && forced_splits <= 0 ? w8a8_whole_tile(M, N, K, p) : p.tile;
+                if (tile != p.tile)
+                    p.tile = tile, p.splits = 1, p.reduce_pass = false;
                 return p;
+            }
             static const int split_options[] = {1, 2, 3, 4, 6, 8, 12, 16};
             double best = -1.0;
             const int planned = p.splits;

@@ -1487,6 +1487,29 @@ int main(int argc, char** argv)
                         if (ws::w8a8_mrows_preferred(m, n, k, 256) && ws::w8a8_mrows_ranges(m, n, k, 256) > 1)
                             EXPECT(ws::w8a8_kstream_choice(m, n, k, 256).tiles > 0);
         }
+        // W8A8 tile GEMM: whole tiles of other shapes where the estimates put them ahead (the GPU test's products), never what a caller fixed,
+        // nor more scratch memory than the queries ask for
+        {
+            const int tiles[][4] = {{1012, 8412, 512, ws::GEMM_TILE_256_192}, {964, 9008, 1152, ws::GEMM_TILE_256_192}, {531, 13308, 512, ws::GEMM_TILE_192_256},
+                                    {1411, 5400, 640, ws::GEMM_TILE_192_256}, {538, 11108, 512, ws::GEMM_TILE_128_256}, {590, 9984, 1152, ws::GEMM_TILE_128_256},
+                                    {262, 12544, 512, ws::GEMM_TILE_192_128}, {455, 8247, 640, ws::GEMM_TILE_192_128}, {396, 11112, 896, ws::GEMM_TILE_128_192},
+                                    {595, 8476, 896, ws::GEMM_TILE_128_192}, {1354, 4170, 896, ws::GEMM_TILE_128_192}, {2000, 12288, 4096, ws::GEMM_TILE_256_192}};
+            for (const auto& t : tiles)
+            {
+                const ws::GemmPlan p = ws::plan_w8a8_launch(t[0], t[1], t[2], -1, 0);
+                EXPECT(p.tile == t[3] && p.splits == 1 && !p.reduce_pass && ws::w8a8_kstream_choice(t[0], t[1], t[2], 256).tiles == 0);
+                for (int forced : {(int)ws::GEMM_TILE_BIG, (int)ws::GEMM_TILE_TALL, (int)ws::GEMM_TILE_MID})
+                    EXPECT(ws::plan_w8a8_launch(t[0], t[1], t[2], forced, 0).tile == forced);
+                EXPECT(ws::plan_w8a8_launch(t[0], t[1], t[2], -1, 2).tile <= ws::GEMM_TILE_TALL && ws::plan_w8a8_launch(t[0], t[1], t[2], -2, 0).tile <= ws::GEMM_TILE_TALL);
+            }
+            for (int m = 100; m < 3000; m += 37)
+                for (int n = 256; n < 12000; n += 333)
+                    for (int k : {128, 384, 512, 2048, 8192})
+                    {
+                        const ws::GemmPlan p = ws::plan_w8a8_launch(m, n, k, -1, 0), q = ws::plan_w8a8_gemm(m, n, k);
+                        EXPECT(p.tile == q.tile ? p.splits <= q.splits : p.splits == 1 && !p.reduce_pass && m > 128 && k >= 512);
+                    }
+        }
         // fp16 x int4 tile GEMM: the (tile, superstep) units are split evenly over at most one workgroup per CU; a
         // workgroup parks at most two partial tiles; whole tiles need no workspace
         {

@@ -177,3 +177,25 @@ def test_64_row_tiles_at_ragged_columns(gpu, m, n, k):
         torch.cuda.synchronize()
         assert np.array_equal(out[:m * n].cpu().numpy().reshape(m, n), want)
         assert bool((out[m * n:] == 77).all()) and bool((ws[need:] == 0x5A).all())
+
+
+# Whole tiles of 256 x 192, 192 x 256, 128 x 256, 192 x 128 and 128 x 192 (tests/cpp/test_host.cpp holds the plan to that): the last tile of
+# rows and of columns ragged, columns no multiple of eight (rows stored an element at a time), one round of tiles and more
+@pytest.mark.parametrize("m,n,k", [(1012, 8412, 512), (964, 9008, 1152), (531, 13308, 512), (1411, 5400, 640), (538, 11108, 512), (590, 9984, 1152),
+                                   (262, 12544, 512), (455, 8247, 640), (396, 11112, 896), (595, 8476, 896), (1354, 4170, 896)])
+def test_tiles_of_192_rows_or_columns(gpu, m, n, k):
+    """Accumulators against products in float64 (exact: below 2^53), the fp16 results bit for bit."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case M={m} N={n} K={k}", flush=True)
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(m + n + k)
+    a, w = (torch.randint(-127, 128, s, generator=gen, device=gpu, dtype=torch.int8) for s in ((m, k), (n, k)))
+    s_tok, s_ch = (torch.rand(s, generator=gen, device=gpu) * 0.009 + 0.001 for s in (m, n))
+    ref = (a.double() @ w.double().t()).to(torch.int32)
+    assert torch.equal(ops.w8a8_gemm_acc(a, w), ref)
+    # ((float)acc * s_tok) * s_ch, rounded to fp32 each time, then to fp16
+    y = (ref.float() * s_tok[:, None] * s_ch[None, :]).half()
+    assert torch.equal(ops.w8a8_gemm(a, s_tok, w, s_ch), y)

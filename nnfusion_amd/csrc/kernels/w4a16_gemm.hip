@@ -35,18 +35,24 @@ namespace nnf
     };
 
     // one row per workgroup of four wavefronts: Xn[m, :] = fp16( x * rsqrt(mean_k(x^2) + eps) * gamma ).
-    // The row is read once: a thread keeps its 16-byte units in registers between the two passes (up to K = 16384;
-    // the units beyond that are read again).
+    // The row is read once: a thread keeps its KEEP 16-byte units in registers between the two passes (8: up to K = 16384;
+    // the units beyond that are read again).  Bound by the way to memory and back: load, sum over the workgroup, store.  So
+    // a row takes no more units than it has (of 0 where it has fewer than KEEP * 256), and gamma is asked for along with it,
+    // not behind the sum: rows x K 16 x 4096 2.71 -> 2.33 us, 256 x 4096 3.01 -> 2.63, 1000 x 4096 5.59 -> 4.74 (a copy of them
+    // 3.8), 2000 x 640 5.60 -> 3.31, 1000 x 11008 9.40 -> 8.69.  KEEP = 8 leaves too few registers: with gamma early 1062 x
+    // 14080 takes 15.0 us, behind the sum 13.9.
+    template <int KEEP>
     __global__ __launch_bounds__(256) void rms_norm_kernel(const half_t* __restrict__ X, const half_t* __restrict__ gamma,
                                                            half_t* __restrict__ Xn, int M, int K, float eps)
     {
-        constexpr int KEEP = 8; // units per thread kept in registers
+        constexpr bool EARLY = KEEP <= 6;
         __shared__ float part[4];
         const int tid = threadIdx.x;
         const int m = blockIdx.x;
         const int units = K >> 3;
         const uintx4* row = reinterpret_cast<const uintx4*>(X + (size_t)m * K);
-        uintx4 kept[KEEP];
+        const uintx4* grow = reinterpret_cast<const uintx4*>(gamma);
+        uintx4 kept[KEEP], kept_gamma[EARLY ? KEEP : 1];
         float ss = 0.f;
         auto sq = [&](const uintx4& v) {
             const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
@@ -63,6 +69,13 @@ namespace nnf
             const int i = tid + e * 256;
             kept[e] = i < units ? row[i] : uintx4{0u, 0u, 0u, 0u};
         }
+        if constexpr (EARLY)
+#pragma unroll
+            for (int e = 0; e < KEEP; ++e)
+            {
+                const int i = tid + e * 256;
+                kept_gamma[e] = i < units ? grow[i] : uintx4{0u, 0u, 0u, 0u};
+            }
 #pragma unroll
         for (int e = 0; e < KEEP; ++e)
             sq(kept[e]);
@@ -74,7 +87,6 @@ namespace nnf
         __syncthreads();
         ss = (part[0] + part[1]) + (part[2] + part[3]);
         const float rstd = 1.0f / __builtin_sqrtf(ss / (float)K + eps);
-        const uintx4* grow = reinterpret_cast<const uintx4*>(gamma);
         uintx4* out = reinterpret_cast<uintx4*>(Xn + (size_t)m * K);
         auto norm = [&](const uintx4& v, const uintx4& g) {
             const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
@@ -95,7 +107,7 @@ namespace nnf
         {
             const int i = tid + e * 256;
             if (i < units)
-                out[i] = norm(kept[e], grow[i]);
+                out[i] = norm(kept[e], EARLY ? kept_gamma[EARLY ? e : 0] : grow[i]);
         }
         for (int i = tid + KEEP * 256; i < units; i += 256)
             out[i] = norm(row[i], grow[i]);
@@ -387,15 +399,18 @@ namespace nnf
         {
             if (normalised_copy)
             {
-                hipLaunchKernelGGL(rms_norm_kernel, dim3(M), dim3(256), 0, stream, (const half_t*)A, (const half_t*)rms_gamma,
-                                   (half_t*)rms_ws, M, K, rms_eps);
+                const hipError_t e = launch_rms_norm(stream, A, rms_gamma, rms_ws, M, K, rms_eps);
+                if (e != hipSuccess)
+                    return e;
                 A = rms_ws;
             }
             else
+            {
                 hipLaunchKernelGGL(rms_rstd_kernel, dim3(M), dim3(256), 0, stream, (const half_t*)A, (float*)rms_ws, M, K, rms_eps);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess)
-                return e;
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess)
+                    return e;
+            }
         }
         const float* rstd = (rms && !normalised_copy && !rstd_in_kernel) ? (const float*)rms_ws : nullptr;
         // ---- the row-streaming kernels (one row; up to 32 rows): prologue and epilogue inside the one launch ------
@@ -504,7 +519,9 @@ namespace nnf
 
     hipError_t launch_rms_norm(hipStream_t stream, const void* X, const void* gamma, void* Xn, int M, int K, float eps)
     {
-        hipLaunchKernelGGL(rms_norm_kernel, dim3(M), dim3(256), 0, stream, (const half_t*)X, (const half_t*)gamma, (half_t*)Xn, M, K, eps);
+        const int keep = (K + 2047) / 2048; // units a thread
+        const auto kernel = keep <= 1 ? rms_norm_kernel<1> : keep <= 2 ? rms_norm_kernel<2> : keep <= 4 ? rms_norm_kernel<4> : keep <= 6 ? rms_norm_kernel<6> : rms_norm_kernel<8>;
+        hipLaunchKernelGGL(kernel, dim3(M), dim3(256), 0, stream, (const half_t*)X, (const half_t*)gamma, (half_t*)Xn, M, K, eps);
         return hipGetLastError();
     }
     namespace

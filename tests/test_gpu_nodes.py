@@ -89,6 +89,21 @@ def test_rms_norm_node(gpu, m, k):
     assert _ulps(ops.rms_norm(tc, tg, 0.0).cpu().numpy(), np.broadcast_to(-gamma, (2, k)).copy()) <= 1
 
 
+@pytest.mark.parametrize("k", [8, 2040, 2048, 2056, 4096, 4104, 8192, 8200, 12288, 12296, 16384, 16392])
+@pytest.mark.parametrize("m", [1, 3])
+def test_rms_norm_units_per_thread(gpu, m, k):
+    """Rows that just fit the 16-byte units of 256 threads a kernel keeps, and one more, in place too.  One ulp: another order of the sum."""
+    from nnfusion_amd import ops
+
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    gamma = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float16)
+    tx, tg = _t(gpu, x, gamma)
+    y = ops.rms_norm(tx, tg, 1e-6)
+    assert _ulps(y.cpu().numpy(), oracle.rmsnorm_f16(x, gamma, 1e-6)) <= 1
+    assert ops.rms_norm(tx, tg, 1e-6, out=tx).equal(y)
+
+
 @pytest.mark.parametrize("bits,group,zpt", [(4, 128, False), (4, 32, True), (4, 64, False), (8, 64, True), (8, 128, False)])
 @pytest.mark.parametrize("n,k", [(16, 256), (100, 1024), (4096, 4096)])
 def test_dequantize_node_is_exact(gpu, bits, group, zpt, n, k):

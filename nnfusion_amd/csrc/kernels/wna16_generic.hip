@@ -331,35 +331,43 @@ namespace nnf
     // for every load in flight at the top of the loop.  Tiles are numbered in groups of four tile rows, tile row fastest,
     // and dealt to the eight XCDs in contiguous runs, so that the workgroups in flight together share activations and
     // weights in one L2 (groups of 2, 8 or 16 tile rows measure the same).
+    // KH = 2: steps of 128, a pair of wavefronts on each sub-tile, half of a step each, whose sums meet behind the loop.  LDS bounds the
+    // tiles: 192 x 128 on eight wavefronts of 96 x 32 reads 128 KiB of fragments for 64 of K, 160 x 96 on four pairs of 80 x 48 (5 x 3
+    // MFMAs of 16 x 16 x 32) half of that, 128 x 128 on four pairs of 64 x 64 what four wavefronts read, with two wavefronts a SIMD.
+    // For 64 of K on a full chip 160 x 96 takes 0.68 us, 128 x 128 0.66 and 128 x 96 0.59 (192 x 128 0.95, 128 x 128 on four wavefronts
+    // 0.9): 300 x 11008 x 4096, 8 bits, 57.5 -> 47.6 us with the weights from memory.  (One wavefront of a pair storing its pieces
+    // ahead of its MFMAs, so that the two are out of step: 5 - 10 % slower.)
     // Ranges of K (blockIdx.y; range_k values each, a multiple of 256, the last range what is left): fp32 sums of a range to
     // partial[range][M][N], added up by the reduction pass.  (An instantiation of its own: the choice at run time
     // cost the product of one range 2 %.)  For products whose
     // tiles leave CUs idle: 249 x 256 x 15232 with 8-bit weights took 80 us on 16 workgroups.
-    template <int BITS, int WM, int WN, bool TAIL, int WAVES_M, int WAVES_N, bool RANGES>
-    __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void wna16_tile_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
+    template <int BITS, int WM, int WN, bool TAIL, int WAVES_M, int WAVES_N, bool RANGES, int MF, int KH>
+    __global__ __launch_bounds__(64 * WAVES_M * WAVES_N * KH) void wna16_tile_kernel(const half_t* __restrict__ A, const uint8_t* __restrict__ Wq,
                                                              const half_t* __restrict__ S, half_t* __restrict__ Y, int M, int N,
                                                              int K_row, int tiles_m, int tiles_n, QuantArgs qa,
                                                              float* __restrict__ partial, int range_k)
     {
-        constexpr int NW = WAVES_M * WAVES_N, THREADS = 64 * NW; // wavefronts: WAVES_M x WAVES_N
-        constexpr int TM = 32 * WAVES_M * WM, TN = 32 * WAVES_N * WN; // rows and columns of the output tile
-        constexpr int A_ROWS = THREADS / 8;                   // rows of activations the workgroup fetches per pass
-        constexpr int KS = 64;            // values of K per step
-        constexpr int PITCH = KS + 8;     // halves per staged row (144 bytes: 16-byte pieces stay aligned)
+        constexpr int NW = WAVES_M * WAVES_N * KH, THREADS = 64 * NW; // wavefronts: WAVES_M x WAVES_N x KH
+        constexpr int TM = MF * WAVES_M * WM, TN = MF * WAVES_N * WN; // rows and columns of the output tile
+        constexpr int KS = 64 * KH;       // values of K per step
+        constexpr int KM = MF == 32 ? 16 : 32; // values of K per MFMA
+        constexpr int PARTS = 64 / KM;    // of a wavefront's step
+        constexpr int A_PPR = KS / 8, A_ROWS = THREADS / A_PPR; // pieces of a row of activations; rows the workgroup fetches per pass
+        constexpr int PITCH = KS + 8;     // halves per staged row (144 or 272 bytes: 16-byte pieces stay aligned)
         constexpr int A_OPERAND = TM * PITCH, W_OPERAND = TN * PITCH; // halves of the staged operands
         constexpr int BUFFER = A_OPERAND + W_OPERAND;
         constexpr int WPP = 128 / BITS;   // weights of a 16-byte piece (inside one group)
         constexpr int PPR = KS / WPP;     // pieces per weight row and step
-        constexpr int A_PER = TM / A_ROWS; // pieces of activations per thread and step: piece tid % 8 of rows tid / 8 + 32 i
+        constexpr int A_PER = TM / A_ROWS; // pieces of activations per thread and step: piece tid % A_PPR of rows tid / A_PPR + A_ROWS i
         constexpr int W_PIECES = TN * PPR;
         // the activations (L2 hits) are fetched one step ahead where a step is long (256-row tiles: a microsecond and
         // more), two steps ahead like the weights otherwise
-        constexpr int A_AHEAD = WM >= 4 ? 1 : 2;
+        constexpr int A_AHEAD = WM * MF >= 128 ? 1 : 2;
         // The barrier of a step stands behind its third quarter where the registers allow it (CARRY: the first fragments
         // of the next step are read during the fourth quarter and carried into the next step; the 256 x 256 tile, whose
         // sums take all 256 accumulation registers, has no room for that and keeps its barrier at the end of the step)
-        constexpr bool CARRY = WM * WN < 16 && NW != 8;
-        constexpr int SLICES = CARRY ? 3 : 4; // quarters that store pieces of the next step
+        constexpr bool CARRY = KH > 1 || (WM * WN < 16 && NW != 8);
+        constexpr int SLICES = CARRY ? PARTS - 1 : PARTS; // quarters that store pieces of the next step
         constexpr int W_PER = (W_PIECES + THREADS - 1) / THREADS; // pieces of weights per thread and step: piece p % PPR of row p / PPR, p = tid + THREADS j
         extern __shared__ __attribute__((aligned(16))) half_t lds[]; // [buffer][A: TM rows, W: TN rows][PITCH]
         const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -393,10 +401,11 @@ namespace nnf
                 qa.zps += ((k_first >> qa.group_shift) * BITS) >> 3;
         }
         const int steps = (K + KS - 1) / KS;
-        const int a_row = tid >> 3, a_k = (tid & 7) * 8;
-        // fragments: wavefront (wm, wn) owns rows [32 WM wm, +32 WM) x columns [32 WN wn, +32 WN)
-        const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-        const int f_row = lane & 31, f_k = (lane >> 5) * 8;
+        const int a_row = tid / A_PPR, a_k = (tid % A_PPR) * 8;
+        // fragments: wavefront (wm, wn, kh) owns rows [MF WM wm, +MF WM) x columns [MF WN wn, +MF WN) of part kh of every step
+        const int kh = KH > 1 ? wave / (WAVES_M * WAVES_N) : 0, wave_mn = wave - kh * (WAVES_M * WAVES_N);
+        const int wm = wave_mn / WAVES_N, wn = wave_mn % WAVES_N;
+        const int f_row = lane % MF, f_k = kh * 64 + (lane / MF) * 8;
 
         // what a thread fetches per step, as it arrives: anything computed from it here would be waited for here
         struct Staged
@@ -506,13 +515,15 @@ namespace nnf
                 if (q < 0 || (3 * W_PER + i) * SLICES / UNITS == q)
                     stage_a(step, ra, i);
         };
-        floatx16 acc[WM][WN];
+        constexpr int ELEMS = MF * MF / 64; // of a lane's
+        typedef float acc_t __attribute__((ext_vector_type(ELEMS)));
+        acc_t acc[WM][WN];
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
             for (int j = 0; j < WN; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
+                for (int e = 0; e < ELEMS; ++e)
                     acc[i][j][e] = 0.f;
         // step s: the loads of step s + 2 into the set step s was stored from; then in quarters (16 values of K): the
         // next quarter's fragments, this quarter's MFMAs and, between them, a slice of the next step's pieces on their way
@@ -526,10 +537,10 @@ namespace nnf
             const half_t* w_s = a_s + A_OPERAND;
 #pragma unroll
             for (int i = 0; i < WM; ++i)
-                fa[kk & 1][i] = *reinterpret_cast<const half8_t*>(a_s + ((wm * WM + i) * 32 + f_row) * PITCH + kk * 16 + f_k);
+                fa[kk & 1][i] = *reinterpret_cast<const half8_t*>(a_s + ((wm * WM + i) * MF + f_row) * PITCH + kk * KM + f_k);
 #pragma unroll
             for (int j = 0; j < WN; ++j)
-                fw[kk & 1][j] = *reinterpret_cast<const half8_t*>(w_s + ((wn * WN + j) * 32 + f_row) * PITCH + kk * 16 + f_k);
+                fw[kk & 1][j] = *reinterpret_cast<const half8_t*>(w_s + ((wn * WN + j) * MF + f_row) * PITCH + kk * KM + f_k);
         };
         auto step = [&](int s, Staged& refill, const Staged& ready) {
             if constexpr (A_AHEAD == 1)
@@ -546,9 +557,9 @@ namespace nnf
             if constexpr (!CARRY)
                 read_frags(s, 0, fa, fw);
 #pragma unroll
-            for (int kk = 0; kk < KS / 16; ++kk)
+            for (int kk = 0; kk < PARTS; ++kk)
             {
-                if (kk + 1 < KS / 16)
+                if (kk + 1 < PARTS)
                     read_frags(s, kk + 1, fa, fw);
                 else if constexpr (CARRY)
                     read_frags(s + 1, 0, fa, fw);
@@ -556,7 +567,10 @@ namespace nnf
                 for (int i = 0; i < WM; ++i)
 #pragma unroll
                     for (int j = 0; j < WN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kk & 1][i], fw[kk & 1][j], acc[i][j], 0, 0, 0);
+                        if constexpr (MF == 32)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kk & 1][i], fw[kk & 1][j], acc[i][j], 0, 0, 0);
+                        else
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[kk & 1][i], fw[kk & 1][j], acc[i][j], 0, 0, 0);
                 if (kk < SLICES)
                     stage(s + 1, A_AHEAD == 1 ? refill : ready, ready, kk);
                 __builtin_amdgcn_sched_barrier(0);
@@ -582,17 +596,16 @@ namespace nnf
             step(s, r0, r1);
             step(s + 1, r1, r0);
         }
-        // D[m][n]: lane l holds column l % 32; element e is row 8 (e / 4) + 4 (l / 32) + e % 4
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
+        // D[m][n]: lane l holds column l % MF; element e is row 8 (e / 4) + 4 (l / MF) + e % 4
+        const auto store = [&](int i) {
 #pragma unroll
             for (int j = 0; j < WN; ++j)
             {
-                const int n = n0 + (wn * WN + j) * 32 + (lane & 31);
+                const int n = n0 + (wn * WN + j) * MF + lane % MF;
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
+                for (int e = 0; e < ELEMS; ++e)
                 {
-                    const int m = m0 + (wm * WM + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+                    const int m = m0 + (wm * WM + i) * MF + 8 * (e >> 2) + 4 * (lane / MF) + (e & 3);
                     if (m < M && n < N)
                     {
                         if constexpr (RANGES)
@@ -602,21 +615,53 @@ namespace nnf
                     }
                 }
             }
+        };
+        if constexpr (KH == 1)
+        {
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+                store(i);
+        }
+        else
+        {
+            // the two halves of K: each wavefront hands the other one's rows over and finishes its own (kh = 0: the first HALF
+            // blocks, 1: the others), through LDS
+            constexpr int HALF = (WM + 1) / 2;
+            acc_t* const given = reinterpret_cast<acc_t*>(lds) + (size_t)wave_mn * (WM * WN * 64) + lane;
+            static_assert(KH == 2 && WAVES_M * WAVES_N * WM * WN * 64 * sizeof(acc_t) <= 2 * BUFFER * sizeof(half_t), "fits the buffers");
+            __syncthreads(); // the last fragments have been read
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+                if ((i < HALF) != (kh == 0))
+#pragma unroll
+                    for (int j = 0; j < WN; ++j)
+                        given[(i * WN + j) * 64] = acc[i][j];
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+                if ((i < HALF) == (kh == 0))
+                {
+#pragma unroll
+                    for (int j = 0; j < WN; ++j)
+                        acc[i][j] += given[(i * WN + j) * 64];
+                    store(i);
+                }
+        }
     }
 
     namespace
     {
-        template <int BITS, int WM, int WN, bool TAIL, int WAVES_M, int WAVES_N, bool RANGES>
+        template <int BITS, int WM, int WN, bool TAIL, int WAVES_M, int WAVES_N, bool RANGES, int MF, int KH>
         hipError_t launch_wna16_tile_k(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
                                      const QuantArgs& qa, float* partial, int range_k)
         {
-            constexpr int NW = WAVES_M * WAVES_N;
-            constexpr int TM = 32 * WAVES_M * WM, TN = 32 * WAVES_N * WN;
-            constexpr int LDS = 2 * (TM + TN) * (64 + 8) * (int)sizeof(half_t);
+            constexpr int NW = WAVES_M * WAVES_N * KH;
+            constexpr int TM = MF * WAVES_M * WM, TN = MF * WAVES_N * WN;
+            constexpr int LDS = 2 * (TM + TN) * (64 * KH + 8) * (int)sizeof(half_t);
             const int tiles_m = (M + TM - 1) / TM, tiles_n = (N + TN - 1) / TN;
             if ((long long)tiles_m * tiles_n > 0x7fffff00ll)
                 return hipErrorInvalidValue;
-            auto kernel = &wna16_tile_kernel<BITS, WM, WN, TAIL, WAVES_M, WAVES_N, RANGES>;
+            auto kernel = &wna16_tile_kernel<BITS, WM, WN, TAIL, WAVES_M, WAVES_N, RANGES, MF, KH>;
             if (LDS > 64 * 1024)
             {
                 static LdsGrant granted;
@@ -634,16 +679,24 @@ namespace nnf
 
     namespace
     {
-        // (K is a multiple of 32; the kernel walks K in pairs of steps of 64)
+        // (K is a multiple of 32; the kernel walks K in pairs of steps)
         template <int BITS, int WM, int WN, int WAVES_M, int WAVES_N>
         hipError_t launch_wna16_tile(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
                                      const QuantArgs& qa, float* partial, int range_k)
         {
             if (partial)
-                return K % 128 ? launch_wna16_tile_k<BITS, WM, WN, true, WAVES_M, WAVES_N, true>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k)
-                               : launch_wna16_tile_k<BITS, WM, WN, false, WAVES_M, WAVES_N, true>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k);
-            return K % 128 ? launch_wna16_tile_k<BITS, WM, WN, true, WAVES_M, WAVES_N, false>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k)
-                           : launch_wna16_tile_k<BITS, WM, WN, false, WAVES_M, WAVES_N, false>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k);
+                return K % 128 ? launch_wna16_tile_k<BITS, WM, WN, true, WAVES_M, WAVES_N, true, 32, 1>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k)
+                               : launch_wna16_tile_k<BITS, WM, WN, false, WAVES_M, WAVES_N, true, 32, 1>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k);
+            return K % 128 ? launch_wna16_tile_k<BITS, WM, WN, true, WAVES_M, WAVES_N, false, 32, 1>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k)
+                           : launch_wna16_tile_k<BITS, WM, WN, false, WAVES_M, WAVES_N, false, 32, 1>(stream, A, Wq, S, Y, M, N, K, qa, partial, range_k);
+        }
+        // 2 x 2 wavefronts by two halves of every step of 128; one range
+        template <int BITS, int WM, int WN, int MF>
+        hipError_t launch_wna16_tile_whole(hipStream_t stream, const void* A, const void* Wq, const void* S, void* Y, int M, int N, int K,
+                                           const QuantArgs& qa)
+        {
+            return K % 256 ? launch_wna16_tile_k<BITS, WM, WN, true, 2, 2, false, MF, 2>(stream, A, Wq, S, Y, M, N, K, qa, nullptr, K)
+                           : launch_wna16_tile_k<BITS, WM, WN, false, 2, 2, false, MF, 2>(stream, A, Wq, S, Y, M, N, K, qa, nullptr, K);
         }
     } // namespace
 
@@ -727,7 +780,8 @@ namespace nnf
         }
         // 256 x 256 (eight wavefronts, 2 x 4, of 128 x 64), 256 x 128 (eight, 4 x 2, of 64 x 64), 192 x 128 (eight, 2 x 4, of
         // 96 x 32), 128 x 128 or 64 x 64
-        // tiles (four wavefronts), over as many ranges of K as the plan says and the workspace holds
+        // tiles (four wavefronts), over as many ranges of K as the plan says and the workspace holds; 160 x 96, 128 x 128 or
+        // 128 x 96 (four pairs of wavefronts) over all of K
         const workspace::Wna16TilePlan plan =
             workspace::plan_wna16_tile(M, N, K, num_cu, ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 ? ws_bytes : 0);
         float* partial = plan.ranges > 1 ? (float*)ws : nullptr;
@@ -749,6 +803,18 @@ namespace nnf
         case 4:
             e = bits == 4 ? launch_wna16_tile<4, 3, 1, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
                           : launch_wna16_tile<8, 3, 1, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
+            break;
+        case 5:
+            e = bits == 4 ? launch_wna16_tile_whole<4, 5, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa)
+                          : launch_wna16_tile_whole<8, 5, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa);
+            break;
+        case 6:
+            e = bits == 4 ? launch_wna16_tile_whole<4, 2, 2, 32>(stream, A, Wq, S, Y, M, N, K, qa)
+                          : launch_wna16_tile_whole<8, 2, 2, 32>(stream, A, Wq, S, Y, M, N, K, qa);
+            break;
+        case 7:
+            e = bits == 4 ? launch_wna16_tile_whole<4, 4, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa)
+                          : launch_wna16_tile_whole<8, 4, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa);
             break;
         default:
             e = bits == 4 ? launch_wna16_tile<4, 1, 1, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)

@@ -1487,6 +1487,23 @@ int main(int argc, char** argv)
                         if (ws::w8a8_mrows_preferred(m, n, k, 256) && ws::w8a8_mrows_ranges(m, n, k, 256) > 1)
                             EXPECT(ws::w8a8_kstream_choice(m, n, k, 256).tiles > 0);
         }
+        // plain tile kernel: tiles on pairs of wavefronts (the GPU test's products), one round of them and no scratch memory
+        {
+            const int pairs[][4] = {{300, 10900, 1280, 5}, {300, 10900, 1152, 5}, {301, 10983, 1184, 5}, {158, 21500, 1248, 5}, {1150, 2690, 1280, 6},
+                                    {1120, 3100, 1056, 6}, {1150, 2690, 1152, 6}, {1130, 2900, 1056, 6}, {1005, 2560, 1024, 7}, {1130, 2562, 1152, 7},
+                                    {470, 5800, 1120, 7}, {505, 5801, 1184, 7}, {300, 11008, 4096, 5}};
+            for (const auto& t : pairs)
+                EXPECT(ws::plan_wna16_tile(t[0], t[1], t[2], 256, 0).tile == t[3]);
+            for (int m = 17; m < 3000; m += 61)
+                for (int n = 64; n < 16000; n += 509)
+                    for (int k : {96, 992, 1024, 1120, 4096, 13056})
+                    {
+                        const auto p = ws::plan_wna16_tile(m, n, k, 256, (size_t)64 << 20);
+                        if (p.tile >= 5)
+                            EXPECT(p.tile <= 7 && k >= 1024 && p.ranges == 1 && p.range_k == k && p.bytes == 0 &&
+                                   ws::ceil_div(m, p.tile == 5 ? 160 : 128) * ws::ceil_div(n, p.tile == 6 ? 128 : 96) <= 256);
+                    }
+        }
         // W8A8 tile GEMM: whole tiles of other shapes where the estimates put them ahead (the GPU test's products), never what a caller fixed,
         // nor more scratch memory than the queries ask for
         {

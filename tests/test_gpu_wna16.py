@@ -212,6 +212,25 @@ def test_products_beyond_the_k_streaming_kernel(gpu, m, n, k, bits, group, zp_te
     _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
 
 
+# 160 x 96, 128 x 128 and 128 x 96 tiles on pairs of wavefronts (tests/cpp/test_host.cpp holds the plan to that): ragged rows and columns, an even and
+# an odd number of steps of 128, a last one of 32, 64 and 96 values
+@pytest.mark.parametrize("bits,m,n,k", [(8, 300, 10900, 1280), (8, 300, 10900, 1152), (8, 301, 10983, 1184), (4, 158, 21500, 1248),
+                                        (8, 1150, 2690, 1280), (8, 1120, 3100, 1056), (8, 1150, 2690, 1152), (4, 1130, 2900, 1056),
+                                        (8, 1005, 2560, 1024), (8, 1130, 2562, 1152), (4, 470, 5800, 1120), (4, 505, 5801, 1184)])
+def test_tiles_on_pairs_of_wavefronts(gpu, bits, m, n, k):
+    print(f"case pairs of wavefronts bits={bits} M={m} N={n} K={k}", flush=True)
+    group = 32 if k % 64 else 64
+    a, wq, s, zps = _case(m + n + k, m, n, k, bits, group, bits == 8)
+    zp = 7 if bits == 4 else 131
+    _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
+    # one-hot rows: the dequantised weights bit for bit, each k from the half of a step that holds it
+    a[:] = 0
+    ks = [(37 * r) % k for r in range(m)]
+    a[np.arange(m), ks] = 1.0
+    wd = oracle.dequantize_wn(wq, s, bits, group, zp=zp, zero_points=zps).astype(np.float16)
+    np.testing.assert_array_equal(_run(gpu, a, wq, s, bits, group, zp, zps), wd[:, ks].T)
+
+
 # one row on the plain GEMV: fewer rows than wavefronts, either side of 24, 28 and 31 a CU, a pass of a few lanes, one pass and many
 @pytest.mark.parametrize("n,k", [(1, 128), (33, 384), (1000, 1152), (4096, 2176), (6144, 640), (6145, 384), (7168, 4224),
                                  (7169, 4224), (7936, 640), (7937, 640), (8191, 640), (8192, 640), (300, 16512)])

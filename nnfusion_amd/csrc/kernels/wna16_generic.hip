@@ -401,11 +401,13 @@ namespace nnf
                 qa.zps += ((k_first >> qa.group_shift) * BITS) >> 3;
         }
         const int steps = (K + KS - 1) / KS;
-        const int a_row = tid / A_PPR, a_k = (tid % A_PPR) * 8;
+        const int a_row = tid >> (KH + 2), a_k = (tid & (A_PPR - 1)) * 8;
+        // (shifts and masks: with / and % by MF and A_PPR the 256 x 256 tile spilled 22 registers, 1 this way; 4096 x 8192 x 8192,
+        // 8 bits, 661 -> 528 us)
         // fragments: wavefront (wm, wn, kh) owns rows [MF WM wm, +MF WM) x columns [MF WN wn, +MF WN) of part kh of every step
         const int kh = KH > 1 ? wave / (WAVES_M * WAVES_N) : 0, wave_mn = wave - kh * (WAVES_M * WAVES_N);
         const int wm = wave_mn / WAVES_N, wn = wave_mn % WAVES_N;
-        const int f_row = lane % MF, f_k = kh * 64 + (lane / MF) * 8;
+        const int f_row = lane & (MF - 1), f_k = kh * 64 + (lane >> (MF == 32 ? 5 : 4)) * 8;
 
         // what a thread fetches per step, as it arrives: anything computed from it here would be waited for here
         struct Staged
@@ -601,11 +603,11 @@ namespace nnf
 #pragma unroll
             for (int j = 0; j < WN; ++j)
             {
-                const int n = n0 + (wn * WN + j) * MF + lane % MF;
+                const int n = n0 + (wn * WN + j) * MF + f_row;
 #pragma unroll
                 for (int e = 0; e < ELEMS; ++e)
                 {
-                    const int m = m0 + (wm * WM + i) * MF + 8 * (e >> 2) + 4 * (lane / MF) + (e & 3);
+                    const int m = m0 + (wm * WM + i) * MF + 8 * (e >> 2) + 4 * (lane >> (MF == 32 ? 5 : 4)) + (e & 3);
                     if (m < M && n < N)
                     {
                         if constexpr (RANGES)

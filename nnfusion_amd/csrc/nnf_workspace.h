@@ -485,7 +485,8 @@ namespace nnf
         // rows: 1.05 - 1.17 x from there to the full chip (256 x 22016 x 4096 with RMSNorm and SiLU-gate 59.6 -> 54.4 us on 230 tiles), 0.6 - 0.9 on
         // fewer tiles and 0.6 - 0.8 on a few more than CUs; two rounds of them 0.93 - 1.04.  Below ten supersteps the sums that the halves of
         // K trade behind the loop cost more (0.91 - 1.06); above 40 and below three quarters of the CUs ranges of K are
-        // ahead (0.96); and so are 64-row tiles where they are the plan's, of 129 .. 192 rows (0.91 - 0.98).
+        // ahead (0.96); and so are 64-row tiles where they are the plan's, of 129 .. 192 rows (0.91 - 0.98), and 32-row ones of up to
+        // 64 rows, of which these tiles pad three quarters and half (16 SiLU-gate products 0.90 - 0.98: 41 x 16356 x 3328 40.8 us, 45.4 on them).
         inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu)
         {
             SkPlan p;
@@ -496,7 +497,7 @@ namespace nnf
             p.supersteps = K / 256;
             p.units = (long long)p.tiles_m * p.tiles_n * p.supersteps;
             const long long tiles = (long long)p.tiles_m * p.tiles_n;
-            if (other.grid < 1 || (K & 255) || other.tile_rows == 64 || p.supersteps < 10 || tiles > num_cu || 3 * tiles <= 2ll * num_cu ||
+            if (other.grid < 1 || (K & 255) || other.tile_rows <= 64 || p.supersteps < 10 || tiles > num_cu || 3 * tiles <= 2ll * num_cu ||
                 (p.supersteps > 40 && 4 * tiles < 3ll * num_cu))
                 return other;
             p.grid = (int)tiles;

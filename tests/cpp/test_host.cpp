@@ -1620,6 +1620,25 @@ int main(int argc, char** argv)
             EXPECT(wide(256, 11008, 4096, true, 256) && !wide(256, 12288, 4096, false, 256) && !wide(183, 8192, 11264, true, 256));
             for (int i = 0; i < 2000; ++i)
                 wide(65 + draw(0, 2000), draw(1, 1 << draw(8, 14)), 128 * draw(1, 100), draw(0, 1) != 0, i % 5 == 0 ? draw(1, 304) : 256);
+            // ... but not of up to 64 rows: what the launch runs there, route and K-streaming kernel included, are tiles of 32 or 64
+            unsigned long long lot_state = 20;
+            const auto lot = [&](int low, int high) {
+                lot_state = lot_state * 6364136223846793005ull + 1442695040888963407ull;
+                return low + (int)((lot_state >> 33) % (unsigned)(high - low + 1));
+            };
+            const int few_rows[][3] = {{64, 16384, 4096}, {36, 16384, 5120}, {43, 16384, 2560}, {50, 16384, 5120}, {41, 16356, 3328}};
+            for (const auto& s : few_rows)
+                EXPECT(ws::plan_w4a16_192(ws::plan_w4a16_tiles(s[0], s[1], s[2], true, true, 256), s[0], s[1], s[2], true, 256).tile_rows == 32);
+            for (int i = 0; i < 20000; ++i)
+            {
+                const int m = lot(1, 64), n = lot(1, 1 << lot(8, 16)), k = 256 * lot(10, 64);
+                const bool gate = lot(0, 1) != 0, rms = lot(0, 1) != 0;
+                const auto r = ws::route_w4a16(m, n, k, gate, rms, false, 256);
+                if (r.kind != ws::W4A16Route::TILE || ws::w4a16_launch_kstream(r, m, n, k, gate, rms, 256, 65536).tiles > 0)
+                    continue;
+                const auto other = ws::w4a16_launch_plan(r, m, n, k, gate, rms, 256, 65536);
+                EXPECT(other.tile_rows > 64 || ws::plan_w4a16_192(other, m, n, k, gate, 256).tile_rows == other.tile_rows);
+            }
             // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
             const auto walk_slots = [](const ws::SkPlan& p) {
                 const long long G = p.supersteps;

@@ -487,6 +487,8 @@ namespace nnf
         // K trade behind the loop cost more (0.91 - 1.06); above 40 and below three quarters of the CUs ranges of K are
         // ahead (0.96); and so are 64-row tiles where they are the plan's, of 129 .. 192 rows (0.91 - 0.98), and 32-row ones of up to
         // 64 rows, of which these tiles pad three quarters and half (16 SiLU-gate products 0.90 - 0.98: 41 x 16356 x 3328 40.8 us, 45.4 on them).
+        // One round of whole 128 x 128 tiles, two thirds of the work a workgroup, is ahead as well: 37 products 0.72 - 0.93
+        // (1024 x 4096 x 4096 39.1 us, 52.7 on 176 of these tiles; 148 x 16365 x 7936 with RMSNorm 78.7 / 92.5).
         inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu)
         {
             SkPlan p;
@@ -497,7 +499,8 @@ namespace nnf
             p.supersteps = K / 256;
             p.units = (long long)p.tiles_m * p.tiles_n * p.supersteps;
             const long long tiles = (long long)p.tiles_m * p.tiles_n;
-            if (other.grid < 1 || (K & 255) || other.tile_rows <= 64 || p.supersteps < 10 || tiles > num_cu || 3 * tiles <= 2ll * num_cu ||
+            const bool one_round = other.tile_rows == 128 && other.tile_weight_rows == 128 && !other.slots && other.grid <= num_cu;
+            if (other.grid < 1 || one_round || (K & 255) || other.tile_rows <= 64 || p.supersteps < 10 || tiles > num_cu || 3 * tiles <= 2ll * num_cu ||
                 (p.supersteps > 40 && 4 * tiles < 3ll * num_cu))
                 return other;
             p.grid = (int)tiles;

@@ -1639,6 +1639,22 @@ int main(int argc, char** argv)
                 const auto other = ws::w4a16_launch_plan(r, m, n, k, gate, rms, 256, 65536);
                 EXPECT(other.tile_rows > 64 || ws::plan_w4a16_192(other, m, n, k, gate, 256).tile_rows == other.tile_rows);
             }
+            // ... nor in place of 128 x 128 tiles that fit one round, one workgroup each
+            const int one_round[][3] = {{1024, 4096, 4096}, {1000, 4096, 4096}, {2048, 2048, 4096}, {400, 8192, 4096}, {512, 8192, 4096}, {939, 4096, 2816}, {148, 16365, 7936}};
+            for (const auto& s : one_round)
+                for (bool rms : {false, true})
+                {
+                    const auto p = ws::plan_w4a16_192(ws::plan_w4a16_tiles(s[0], s[1], s[2], false, rms, 256), s[0], s[1], s[2], false, 256);
+                    EXPECT(p.tile_rows == 128 && p.tile_weight_rows == 128 && p.grid == ws::ceil_div(s[0], 128) * ws::ceil_div(s[1], 128) && p.slots == 0);
+                }
+            for (int i = 0; i < 20000; ++i)
+            {
+                const int m = lot(65, 4096), n = lot(1, 1 << lot(8, 15)), k = 256 * lot(10, 64);
+                const bool rms = lot(0, 1) != 0;
+                const auto other = ws::plan_w4a16_tiles(m, n, k, false, rms, 256);
+                EXPECT(!(other.tile_rows == 128 && other.tile_weight_rows == 128 && !other.slots && other.grid == other.tiles_m * other.tiles_n && other.grid <= 256) ||
+                       ws::plan_w4a16_192(other, m, n, k, false, 256).tile_weight_rows == 128);
+            }
             // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
             const auto walk_slots = [](const ws::SkPlan& p) {
                 const long long G = p.supersteps;

@@ -391,7 +391,7 @@ namespace nnf
                                                                           choice.sync_flags ? choice.sync_bytes : 0)
                                            : workspace::SkPlan();
         if (route.kind == W4A16Route::TILE && route.own_plan)
-            plan = workspace::plan_w4a16_192(plan, M, N, K, gate, num_cu);
+            plan = workspace::plan_w4a16_192(plan, M, N, K, gate, num_cu, rms);
         const bool rstd_in_tile_gemm = rms && route.kind == W4A16Route::TILE && rstd_inside_tile_gemm(plan, choice, num_cu);
         const bool rstd_in_kernel = route.kind == W4A16Route::ROWS ||
                                     (route.kind == W4A16Route::MROWS && workspace::w4a16_mrows_fixed_k(M, K)) || rstd_in_tile_gemm;

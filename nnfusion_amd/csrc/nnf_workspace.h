@@ -489,7 +489,12 @@ namespace nnf
         // 64 rows, of which these tiles pad three quarters and half (16 SiLU-gate products 0.90 - 0.98: 41 x 16356 x 3328 40.8 us, 45.4 on them).
         // One round of whole 128 x 128 tiles, two thirds of the work a workgroup, is ahead as well: 37 products 0.72 - 0.93
         // (1024 x 4096 x 4096 39.1 us, 52.7 on 176 of these tiles; 148 x 16365 x 7936 with RMSNorm 78.7 / 92.5).
-        inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu)
+        // So are equal parts of 256-row tiles with less work a workgroup: halves of 256 x 128 and quarters of 256 x 256, two thirds of it
+        // (26 products 0.80 - 1.06 on these tiles, 0.925 in the geometric mean: 4085 x 1024 x 6656 60.6 us, 65.9 on them; with RMSNorm, whose sums
+        // of squares more workgroups share, 19 products 0.95 - 2.1), and thirds of 256 x 256, eight ninths, of long K: of 293 products those of
+        // up to 35 supersteps 1.12 on these tiles, from 48 on 0.98; between them 1.07 for more than 256 rows with RMSNorm or with less
+        // to pad on these tiles, 0.99 for the others.  (Up to 256 rows, one row of tiles there and two here, 0.94 from 36 on.)
+        inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu, bool rms = true)
         {
             SkPlan p;
             p.tile_rows = 128;
@@ -503,6 +508,14 @@ namespace nnf
             if (other.grid < 1 || one_round || (K & 255) || other.tile_rows <= 64 || p.supersteps < 10 || tiles > num_cu || 3 * tiles <= 2ll * num_cu ||
                 (p.supersteps > 40 && 4 * tiles < 3ll * num_cu))
                 return other;
+            const long long other_tiles = (long long)other.tiles_m * other.tiles_n, area = (long long)other.tile_rows * other.tile_weight_rows;
+            if (other.slots && other.tile_rows == 256 && other.grid % other_tiles == 0)
+            {
+                const long long of_a_workgroup = area * other_tiles / other.grid;
+                const bool later = M > 256 && (rms || tiles * 128 * 192 < other_tiles * area);
+                if (of_a_workgroup <= 128 * 128 ? !rms : (of_a_workgroup < 128 * 192 && p.supersteps >= (later ? 48 : 36)))
+                    return other;
+            }
             p.grid = (int)tiles;
             return p;
         }

@@ -1655,6 +1655,21 @@ int main(int argc, char** argv)
                 EXPECT(!(other.tile_rows == 128 && other.tile_weight_rows == 128 && !other.slots && other.grid == other.tiles_m * other.tiles_n && other.grid <= 256) ||
                        ws::plan_w4a16_192(other, m, n, k, false, 256).tile_weight_rows == 128);
             }
+            // ... nor of equal parts of 256-row tiles whose workgroups have less work: two thirds of it (halves of 256 x 128, quarters of 256 x 256:
+            // but with RMSNorm), or eight ninths (thirds of 256 x 256) from a K on that depends on RMSNorm
+            const auto parts_kept = [](int m, int n, int k, bool gate, bool rms) {
+                const auto other = ws::plan_w4a16_tiles(m, n, k, gate, rms, 256), p = ws::plan_w4a16_192(other, m, n, k, gate, 256, rms);
+                EXPECT(other.tile_rows == 256 && other.slots && other.grid % (other.tiles_m * other.tiles_n) == 0);
+                return p.tile_rows == 256 && p.grid == other.grid;
+            };
+            const int less_work[][3] = {{3646, 1024, 9216}, {1959, 1984, 9472}, {4085, 1024, 6656}, {1006, 4096, 9728}, {4096, 1024, 4096}, {16384, 256, 4096}};
+            for (const auto& s : less_work)
+                EXPECT(parts_kept(s[0], s[1], s[2], false, false));
+            EXPECT(!parts_kept(3863, 1007, 6144, false, true) && !parts_kept(2212, 896, 4352, true, true));
+            EXPECT(parts_kept(3517, 1216, 13568, false, false) && parts_kept(471, 10240, 15616, false, false) && parts_kept(3556, 1161, 9984, false, false));
+            EXPECT(parts_kept(993, 2304, 16384, true, true) && parts_kept(159, 9740, 13056, true, true) && parts_kept(252, 9920, 11264, true, true));
+            EXPECT(!parts_kept(2429, 1657, 6656, false, true) && !parts_kept(2996, 1664, 7168, false, false) && !parts_kept(3887, 1156, 7680, false, false));
+            EXPECT(!parts_kept(2661, 1792, 5888, false, true) && !parts_kept(2944, 832, 11008, true, true) && !parts_kept(1119, 3968, 9728, false, false));
             // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
             const auto walk_slots = [](const ws::SkPlan& p) {
                 const long long G = p.supersteps;

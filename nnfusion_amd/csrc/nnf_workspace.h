@@ -494,6 +494,9 @@ namespace nnf
         // of squares more workgroups share, 19 products 0.95 - 2.1), and thirds of 256 x 256, eight ninths, of long K: of 293 products those of
         // up to 35 supersteps 1.12 on these tiles, from 48 on 0.98; between them 1.07 for more than 256 rows with RMSNorm or with less
         // to pad on these tiles, 0.99 for the others.  (Up to 256 rows, one row of tiles there and two here, 0.94 from 36 on.)
+        // And so is a plan of four fifths of these tiles' whole area, padding included: few columns and a second tile for some of them (30827 x 128
+        // x 2816 32.2 / 38.9 us, 16133 x 233 x 2560 0.94; a fifth more to compute is level).  With RMSNorm the sums of squares of so many
+        // rows make 2.3 - 2.9 x of it.
         inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu, bool rms = true)
         {
             SkPlan p;
@@ -509,6 +512,8 @@ namespace nnf
                 (p.supersteps > 40 && 4 * tiles < 3ll * num_cu))
                 return other;
             const long long other_tiles = (long long)other.tiles_m * other.tiles_n, area = (long long)other.tile_rows * other.tile_weight_rows;
+            if (!rms && 4 * tiles * 128 * 192 > 5 * other_tiles * area)
+                return other;
             if (other.slots && other.tile_rows == 256 && other.grid % other_tiles == 0)
             {
                 const long long of_a_workgroup = area * other_tiles / other.grid;

@@ -1670,6 +1670,12 @@ int main(int argc, char** argv)
             EXPECT(parts_kept(993, 2304, 16384, true, true) && parts_kept(159, 9740, 13056, true, true) && parts_kept(252, 9920, 11264, true, true));
             EXPECT(!parts_kept(2429, 1657, 6656, false, true) && !parts_kept(2996, 1664, 7168, false, false) && !parts_kept(3887, 1156, 7680, false, false));
             EXPECT(!parts_kept(2661, 1792, 5888, false, true) && !parts_kept(2944, 832, 11008, true, true) && !parts_kept(1119, 3968, 9728, false, false));
+            // ... nor where they compute columns that are not there, a second tile for a few of them, unless RMSNorm's sums of squares are to be shared
+            const int padded[][3] = {{30827, 128, 2816}, {32755, 112, 3840}, {16133, 233, 2560}, {15565, 213, 2560}, {32000, 97, 3072}};
+            for (const auto& s : padded)
+                for (bool rms : {false, true})
+                    EXPECT((ws::plan_w4a16_192(ws::plan_w4a16_tiles(s[0], s[1], s[2], false, rms, 256), s[0], s[1], s[2], false, 256, rms).tile_weight_rows == 192) == rms);
+            EXPECT(ws::plan_w4a16_192(ws::plan_w4a16_tiles(27712, 192, 2560, false, false, 256), 27712, 192, 2560, false, 256, false).tile_weight_rows == 192);
             // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
             const auto walk_slots = [](const ws::SkPlan& p) {
                 const long long G = p.supersteps;

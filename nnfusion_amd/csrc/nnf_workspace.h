@@ -113,9 +113,13 @@ namespace nnf
         // products of 129 .. 4096 rows (N = 256 .. 16384, K = 512 .. 16384, weights from memory, every shape timed; 10 % rms): rounds of
         // tiles x start, and per 128 of K a step a round and up to `load` with the CUs busy.  Over ranges of K: the plan's own estimate, which is
         // a tenth too long.  161 of the 520 are on another tile by it, 1.16 x in the geometric mean, the slowest of them 0.98; the fastest shape of
-        // each would gain all of them 1.048, this gains 1.046.  Of 416 others, short K among them, five are more than 2 % slower (1549 x 9984 x
-        // 1152 32.9 -> 35.0 us, from 128 x 128 tiles two a CU, which the estimate of one a CU places too late).  (192 x 192, on
+        // each would gain all of them 1.048, this gains 1.046.  (192 x 192, on
         // four wavefronts, is the fastest for three.)
+        // The row of 128 x 128 is of stages of 128, one workgroup a CU; below K = 2560 the launch takes stages of 64 and two a CU, whose short
+        // loops cover for each other.  There 128 x 256 tiles are estimated ahead a little too soon: 160 products whose columns are a multiple of
+        // eight: in one round of them 0.995 at K = 512 and 640, 1.04 at 768 and 896, 1.03 - 1.12 above; in two 0.95, 0.98, 0.99 at 1024, 1.01 at
+        // 1152 and 1.07 above (2143 x 7352 x 512 20.3 / 21.7 us, 1549 x 9984 x 1152 32.0 / 30.7).  Other columns are stored an element at a
+        // time, with which fewer, larger tiles get along better: 1.11 - 1.17 at every K.
         inline int w8a8_whole_tile(int M, int N, int K, const GemmPlan& planned)
         {
             struct Cost
@@ -130,6 +134,9 @@ namespace nnf
                 {GEMM_TILE_192_128, 192, 128, 5.62, 0.595, 0.207}, {GEMM_TILE_128_192, 128, 192, 7.99, 0.459, 0.247},
             };
             if (M <= 128 || K < 512 || planned.tile == GEMM_TILE_SMALL || planned.tile == GEMM_TILE_TINY)
+                return planned.tile;
+            const long long mids = (long long)ceil_div(M, 128) * ceil_div(N, 128);
+            if (planned.tile == GEMM_TILE_MID && planned.splits == 1 && (N & 7) == 0 && K < (mids > 2 * PLAN_CUS ? 1152 : 768))
                 return planned.tile;
             const double steps = K / 128;
             double best = planned.splits > 1 ? 0.9e6 * estimate_gemm(M, N, K, false, planned.tile, planned.splits, true) : -1.0;

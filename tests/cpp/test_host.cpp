@@ -1527,6 +1527,19 @@ int main(int argc, char** argv)
                         EXPECT(p.tile == q.tile ? p.splits <= q.splits : p.splits == 1 && !p.reduce_pass && m > 128 && k >= 512);
                     }
         }
+        // ... and not in place of 128 x 128 tiles two a CU of so short a K that they are ahead: below K = 768 in one round of them, 1152 in two
+        {
+            const int kept[][3] = {{518, 11520, 512}, {845, 8320, 512}, {1102, 7040, 512}, {620, 12160, 512}, {1115, 14144, 512}, {1080, 13440, 512}, {2143, 7352, 512},
+                                   {2137, 7616, 640}, {1378, 10944, 640}, {2922, 5504, 768}, {2160, 7424, 896}, {2360, 6592, 1024}};
+            for (const auto& t : kept)
+            {
+                const ws::GemmPlan p = ws::plan_w8a8_launch(t[0], t[1], t[2], -1, 0), q = ws::plan_w8a8_gemm(t[0], t[1], t[2]);
+                EXPECT(q.tile == ws::GEMM_TILE_MID && p.tile == q.tile && p.splits == q.splits && p.reduce_pass == q.reduce_pass);
+            }
+            const int moved[][3] = {{531, 11456, 768}, {1852, 8448, 1152}, {1549, 9984, 1152}, {1106, 6665, 2048}, {558, 12043, 512}, {1115, 14145, 512}};
+            for (const auto& t : moved)
+                EXPECT(ws::plan_w8a8_launch(t[0], t[1], t[2], -1, 0).tile == ws::GEMM_TILE_128_256);
+        }
         // fp16 x int4 tile GEMM: the (tile, superstep) units are split evenly over at most one workgroup per CU; a
         // workgroup parks at most two partial tiles; whole tiles need no workspace
         {

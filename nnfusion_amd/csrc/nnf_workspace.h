@@ -1063,13 +1063,17 @@ namespace nnf
                 }
             // Pairs of wavefronts, all of K in one round of 160 x 96 (5), 128 x 128 (6) or 128 x 96 (7) tiles: 3.7 us and 0.68 / 0.66 / 0.59
             // a step, walked in fours, where that is 5 % below the estimate of the others.  Of 2568 products of 18 .. 4000 rows, 8 bits and
-            // 4, it moves 116: 1.11 x in the geometric mean (613 x 6272 x 10752 194 -> 137 us, 249 x 10368 x 4864 71 -> 56), three of them
-            // 4 - 9 % slower (898 x 4032 x 9600 on all CUs 110 -> 121).  Two rounds and more 0.85 - 1.08, K below 1024 0.87 - 0.98 with 4
-            // bits and 1.04 with 8.
+            // 4, it moves 116 (before the exception below): 1.11 x in the geometric mean (613 x 6272 x 10752 194 -> 137 us, 249 x 10368 x 4864 71 -> 56).  Two rounds and more 0.85 -
+            // 1.08, K below 1024 0.87 - 0.98 with 4 bits and 1.04 with 8.  Ranges of K whose workgroups have no more work than a 128 x 128
+            // tile, halves of 256 x 128 and quarters of 256 x 256 tiles, pay for their sums, less and less of it with K: 73 products with
+            // such a plan 1.05 on 128 x 128 tiles up to K = 7000, 1.00 up to 7500, 0.97 (0.91 - 1.09) above (898 x 4032 x 9600 105 us, 112 on them).
             double other = 0.95 * estimate(best.tile, best.ranges, best.range_k);
+            const bool same_work = K >= 7500 && best.tile <= 1 && rows[best.tile] * cols[best.tile] <= 128 * 128 * best.ranges;
             if (K >= 1024)
                 for (int pair = 5; pair < 8; ++pair)
                 {
+                    if (pair == 6 && same_work)
+                        continue;
                     const long long grid = (long long)ceil_div(M, pair == 5 ? 160 : 128) * ceil_div(N, pair == 6 ? 128 : 96);
                     const double t = 3.7 + (pair == 5 ? 0.68 : pair == 6 ? 0.66 : 0.59) * 4 * ceil_div(K, 256);
                     if (grid <= num_cu && t < other)

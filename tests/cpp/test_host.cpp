@@ -1504,6 +1504,19 @@ int main(int argc, char** argv)
                                    ws::ceil_div(m, p.tile == 5 ? 160 : 128) * ws::ceil_div(n, p.tile == 6 ? 128 : 96) <= 256);
                     }
         }
+        // ... and not of 128 x 128 in place of ranges of K of 256-row tiles with no more work a workgroup, at long K; without the scratch memory
+        // for ranges they are what is left
+        {
+            const int ranges[][3] = {{898, 4032, 9600}, {511, 8128, 9856}, {448, 7808, 9472}, {450, 7808, 9344}, {503, 8192, 8448}, {753, 5184, 8064}, {1784, 2304, 10752}, {227, 15808, 7808}};
+            for (const auto& s : ranges)
+            {
+                const auto p = ws::plan_wna16_tile(s[0], s[1], s[2], 256, (size_t)64 << 20);
+                EXPECT(p.tile <= 1 && p.ranges == (p.tile ? 2 : 4) && ws::plan_wna16_tile(s[0], s[1], s[2], 256, 0).tile == 6);
+            }
+            const int pairs[][3] = {{681, 5248, 6656}, {1191, 3200, 7168}, {1171, 3200, 7168}, {503, 8192, 4096}};
+            for (const auto& s : pairs)
+                EXPECT(ws::plan_wna16_tile(s[0], s[1], s[2], 256, (size_t)64 << 20).tile == 6);
+        }
         // W8A8 tile GEMM: whole tiles of other shapes where the estimates put them ahead (the GPU test's products), never what a caller fixed,
         // nor more scratch memory than the queries ask for
         {

@@ -112,8 +112,8 @@ def test_one_launch_fused_forms(gpu, fused, spin_limit):
         _check(one.cpu().numpy(), ref, 2e-2)
 
 
-# rows a workgroup between one and many, rows shorter and longer than one and two sweeps of a wavefront's 2048 values, the last
-# sweep of 128
+# rows a workgroup between one and many, rows of one sweep of a wavefront's 8192 values, shorter and longer than the 2048 that four wavefronts
+# read at a time, the last 128 by themselves
 @pytest.mark.parametrize("m,n,k", [(65, 64, 128), (77, 290, 640), (130, 2000, 2048), (131, 1100, 2176), (300, 130, 4096), (513, 600, 4224),
                                    (700, 96, 384)])
 def test_rstd_of_many_rows_a_workgroup_bit_for_bit(gpu, m, n, k):
@@ -127,6 +127,30 @@ def test_rstd_of_many_rows_a_workgroup_bit_for_bit(gpu, m, n, k):
     ta, tw, ts, tg = _t(gpu, a, wq, s, gamma)
     sync = ops.sync_flags(gpu)
     for act, plan in ((0, (64, 1, 128)), (0, (128, 1, 128)), (0, (128, 0, 256)), (1, (64, 1)), (1, (128, 1)), (0, (256, 1, 256))):
+        w_, s_ = (tw, ts) if act else (tw[:n].contiguous(), ts[:n].contiguous())
+        kw = dict(rms_gamma=tg, act=act, variant="gemm_mfma", plan=plan)
+        two = ops.w4a16_gemm_fused(ta, w_, s_, **kw)
+        for spin_limit in (0, -1):
+            one = ops.w4a16_gemm_fused(ta, w_, s_, sync=sync, spin_limit=spin_limit, **kw)
+            assert torch.equal(one, two)
+            assert not sync.any()
+
+
+# A sweep of a wavefront is 8192 values of its row: rows just below, at and above one sweep, two sweeps, one and two groups of 128 in the last one
+@pytest.mark.parametrize("m,n,k", [(700, 96, 8064), (700, 96, 8192), (513, 130, 8320), (300, 64, 8448), (700, 96, 16384), (259, 64, 16512)])
+def test_rstd_of_rows_of_several_sweeps_bit_for_bit(gpu, m, n, k):
+    """Few columns and many rows: from eight to 64 rows a workgroup, each by one wavefront in one, two or three sweeps: the bits of the
+    pre-pass, and of four wavefronts a row where the wait for the other workgroups runs out."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case rows of several sweeps M={m} N={n} K={k}", flush=True)
+    a, wq, s = datagen.w4a16_case(m + k, m, 2 * n, k)
+    gamma = (1.0 + 0.1 * np.random.default_rng(m).standard_normal(k)).astype(np.float16)
+    ta, tw, ts, tg = _t(gpu, a, wq, s, gamma)
+    sync = ops.sync_flags(gpu)
+    for act, plan in ((0, (64, 1, 128)), (0, (128, 1, 128)), (1, (64, 1)), (1, (128, 1)), (0, (256, 1, 256))):
         w_, s_ = (tw, ts) if act else (tw[:n].contiguous(), ts[:n].contiguous())
         kw = dict(rms_gamma=tg, act=act, variant="gemm_mfma", plan=plan)
         two = ops.w4a16_gemm_fused(ta, w_, s_, **kw)

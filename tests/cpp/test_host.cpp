@@ -1504,6 +1504,15 @@ int main(int argc, char** argv)
                                    ws::ceil_div(m, p.tile == 5 ? 160 : 128) * ws::ceil_div(n, p.tile == 6 ? 128 : 96) <= 256);
                     }
         }
+        {
+            // (the products of the GPU test of their block parameters; 4-bit ones of a K or columns that the tile GEMM does not take)
+            const int forms[][5] = {{300, 10900, 1280, 0, 5}, {300, 10900, 1152, 0, 5}, {301, 10983, 1184, 0, 5}, {284, 10894, 1920, 5, 5}, {1150, 2690, 1152, 0, 6}, {1120, 3100, 1056, 0, 6},
+                                    {834, 4526, 1152, 6, 6}, {834, 4526, 1152, 7, 6}, {1005, 2560, 1024, 0, 7}, {1130, 2562, 1152, 0, 7}, {515, 4250, 2176, 7, 7}, {470, 5800, 1120, 5, 7}};
+            for (const auto& t : forms)
+                EXPECT(ws::plan_wna16_tile(t[0], t[1], t[2], 256, 0).tile == t[4] && ws::plan_wna16_tile(t[0], t[1], t[2], 256, (size_t)64 << 20).tile == t[4] &&
+                       (t[3] == 0 || (!ws::w4a16_gemm_q_fits(t[0], t[1], t[2], t[3]) && !ws::w4a16_gemm_q_odd_fits(t[0], t[1], t[2], t[3]) &&
+                                      ws::wna16_on_tile_kernel(t[0], t[1], t[2], 4, t[3], 256))));
+        }
         // ... and not of 128 x 128 in place of ranges of K of 256-row tiles with no more work a workgroup, at long K; without the scratch memory
         // for ranges they are what is left
         {
@@ -1646,6 +1655,8 @@ int main(int argc, char** argv)
             EXPECT(wide(256, 11008, 4096, true, 256) && !wide(256, 12288, 4096, false, 256) && !wide(183, 8192, 11264, true, 256));
             for (int i = 0; i < 2000; ++i)
                 wide(65 + draw(0, 2000), draw(1, 1 << draw(8, 14)), 128 * draw(1, 100), draw(0, 1) != 0, i % 5 == 0 ? draw(1, 304) : 256);
+            for (const auto& s : wide_shapes)
+                EXPECT(ws::plan_w4a16_192(ws::plan_w4a16_tiles(s[0], s[1], s[3], false, false, 256), s[0], s[1], s[3], false, 256, false).tile_weight_rows == 192);
             // ... but not of up to 64 rows: what the launch runs there, route and K-streaming kernel included, are tiles of 32 or 64
             unsigned long long lot_state = 20;
             const auto lot = [&](int low, int high) {

@@ -645,3 +645,27 @@ def test_tiles_of_192_columns(gpu, m, n_plain, n_gate, k):
         assert float((one.float() - ref).norm() / ref.norm()) <= tol
         assert float((one.float() - ref).abs().max() / ref.pow(2).mean().sqrt()) <= (2e-2 if "act" in kw else TOL)
         assert not sync.any()
+
+
+@pytest.mark.parametrize("m,n_plain,n_gate,k", [(300, 11300, 5601, 2560), (257, 11523, 5555, 2816), (700, 6200, 3000, 3072), (1000, 4608, 2310, 4096)])
+def test_tiles_of_192_columns_where_the_wait_runs_out(gpu, m, n_plain, n_gate, k):
+    """RMSNorm inside the launch: rows that a workgroup computes itself, its wait for the others being over at once, have the same bits."""
+    import torch
+
+    from nnfusion_amd import ops
+
+    print(f"case M={m} N={n_plain}/{n_gate} K={k}", flush=True)
+    n = max(n_plain, 2 * n_gate)
+    a, wq, s = datagen.w4a16_case(m + n + k, m, n, k)
+    gamma = datagen.normal_f16(m, datagen.S_GAMMA, (k,), 1.0, 0.1)
+    res = datagen.normal_f16(m, datagen.S_RES, (m, n_plain))
+    bias = datagen.normal_f16(m, datagen.S_BIAS, (n_plain,))
+    a, wq, s, gamma, res, bias = _t(gpu, a, wq, s, gamma, res, bias)
+    wp, sp, wg, sg = (t[:c].contiguous() for c in (n_plain, 2 * n_gate) for t in (wq, s))
+    sync = ops.sync_flags(gpu)
+    for w_, s_, kw in ((wg, sg, dict(act=1)), (wp, sp, {}), (wp, sp, dict(residual=res)), (wp, sp, dict(bias=bias)), (wp, sp, dict(bias=bias, residual=res))):
+        kw = dict(kw, rms_gamma=gamma, variant="gemm_mfma", plan=(0, 0, 0))
+        two = ops.w4a16_gemm_fused(a, w_, s_, **kw)
+        for spin_limit in (0, -1):
+            assert torch.equal(ops.w4a16_gemm_fused(a, w_, s_, sync=sync, spin_limit=spin_limit, **kw), two)
+            assert not sync.any()

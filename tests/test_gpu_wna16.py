@@ -231,6 +231,25 @@ def test_tiles_on_pairs_of_wavefronts(gpu, bits, m, n, k):
     np.testing.assert_array_equal(_run(gpu, a, wq, s, bits, group, zp, zps), wd[:, ks].T)
 
 
+# ... with every form of their block parameters: groups as long as a step, a scalar zero point with 8 bits, zero points two a byte, an odd number of
+# them a row
+@pytest.mark.parametrize("bits,m,n,k,group,zp_tensor",
+                         [(8, 300, 10900, 1280, 128, False), (8, 300, 10900, 1152, 128, True), (8, 301, 10983, 1184, 32, False), (4, 284, 10894, 1920, 32, True),
+                          (8, 1150, 2690, 1152, 128, False), (8, 1120, 3100, 1056, 32, False), (4, 834, 4526, 1152, 64, True), (4, 834, 4526, 1152, 128, True),
+                          (8, 1005, 2560, 1024, 128, False), (8, 1130, 2562, 1152, 128, True), (4, 515, 4250, 2176, 128, True), (4, 470, 5800, 1120, 32, True)])
+def test_block_parameters_of_tiles_on_pairs_of_wavefronts(gpu, bits, m, n, k, group, zp_tensor):
+    """Bounds as for the other tiles (test_tiles_on_pairs_of_wavefronts)."""
+    print(f"case pairs of wavefronts bits={bits} M={m} N={n} K={k} group={group} zero_points={zp_tensor}", flush=True)
+    a, wq, s, zps = _case(m + n + k + group, m, n, k, bits, group, zp_tensor)
+    zp = 7 if bits == 4 else 131
+    _check(_run(gpu, a, wq, s, bits, group, zp, zps), oracle.wna16_gemm(a, wq, s, bits, group, zp=zp, zero_points=zps, f32_out=True))
+    a[:] = 0
+    ks = [(37 * r) % k for r in range(m)]
+    a[np.arange(m), ks] = 1.0
+    wd = oracle.dequantize_wn(wq, s, bits, group, zp=zp, zero_points=zps).astype(np.float16)
+    np.testing.assert_array_equal(_run(gpu, a, wq, s, bits, group, zp, zps), wd[:, ks].T)
+
+
 # one row on the plain GEMV: fewer rows than wavefronts, either side of 24, 28 and 31 a CU, a pass of a few lanes, one pass and many
 @pytest.mark.parametrize("n,k", [(1, 128), (33, 384), (1000, 1152), (4096, 2176), (6144, 640), (6145, 384), (7168, 4224),
                                  (7169, 4224), (7936, 640), (7937, 640), (8191, 640), (8192, 640), (300, 16512)])

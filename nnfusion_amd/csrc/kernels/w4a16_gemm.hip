@@ -10,7 +10,7 @@
 //     the unfused graph, at most 64 rows of it).
 //   * epilogues: bias, residual add, SiLU(gate) * up with the gate and up projections as two halves of
 //     the N tile -- inside the kernels, in the reduction pass, or (SiLU-gate of the MFMA GEMV) in an element-wise kernel.
-//   * tile height and split of the work over the CUs follow nnf::workspace::plan_w4a16_tiles.
+//   * tiles and split of the work over the CUs follow nnf::workspace::w4a16_launch_tiles.
 #include "w4a16_gemm_sk_launch.h"
 
 #include "../nnf_workspace.h"
@@ -386,12 +386,10 @@ namespace nnf
         // (the row-streaming kernels add up the squares of the activations they hold themselves: no pre-pass; the form
         // with a run-time K keeps it)
         const bool normalised_copy = route.normalised_copy;
-        workspace::SkPlan plan = route.kind == W4A16Route::TILE
-                                           ? workspace::w4a16_launch_plan(route, M, N, K, gate, rms, num_cu,
-                                                                          choice.sync_flags ? choice.sync_bytes : 0)
+        const workspace::SkPlan plan = route.kind == W4A16Route::TILE
+                                           ? workspace::w4a16_launch_tiles(route, M, N, K, gate, rms, num_cu,
+                                                                           choice.sync_flags ? choice.sync_bytes : 0)
                                            : workspace::SkPlan();
-        if (route.kind == W4A16Route::TILE && route.own_plan)
-            plan = workspace::plan_w4a16_192(plan, M, N, K, gate, num_cu, rms);
         const bool rstd_in_tile_gemm = rms && route.kind == W4A16Route::TILE && rstd_inside_tile_gemm(plan, choice, num_cu);
         const bool rstd_in_kernel = route.kind == W4A16Route::ROWS ||
                                     (route.kind == W4A16Route::MROWS && workspace::w4a16_mrows_fixed_k(M, K)) || rstd_in_tile_gemm;

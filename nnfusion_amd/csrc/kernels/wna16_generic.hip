@@ -348,6 +348,7 @@ namespace nnf
                                                              float* __restrict__ partial, int range_k)
     {
         constexpr int NW = WAVES_M * WAVES_N * KH, THREADS = 64 * NW; // wavefronts: WAVES_M x WAVES_N x KH
+        static_assert(KH == 1 || KH == 2, "halves of a step at most"); // (a_row, the exchange behind the loop)
         constexpr int TM = MF * WAVES_M * WM, TN = MF * WAVES_N * WN; // rows and columns of the output tile
         constexpr int KS = 64 * KH;       // values of K per step
         constexpr int KM = MF == 32 ? 16 : 32; // values of K per MFMA
@@ -790,31 +791,31 @@ namespace nnf
         hipError_t e;
         switch (plan.tile)
         {
-        case 0:
+        case workspace::WNA16_256_256:
             e = bits == 4 ? launch_wna16_tile<4, 4, 2, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
                           : launch_wna16_tile<8, 4, 2, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
             break;
-        case 1:
+        case workspace::WNA16_256_128:
             e = bits == 4 ? launch_wna16_tile<4, 2, 2, 4, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
                           : launch_wna16_tile<8, 2, 2, 4, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
             break;
-        case 2:
+        case workspace::WNA16_128_128:
             e = bits == 4 ? launch_wna16_tile<4, 2, 2, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
                           : launch_wna16_tile<8, 2, 2, 2, 2>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
             break;
-        case 4:
+        case workspace::WNA16_192_128:
             e = bits == 4 ? launch_wna16_tile<4, 3, 1, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k)
                           : launch_wna16_tile<8, 3, 1, 2, 4>(stream, A, Wq, S, Y, M, N, K, qa, partial, plan.range_k);
             break;
-        case 5:
+        case workspace::WNA16_PAIRS_160_96:
             e = bits == 4 ? launch_wna16_tile_whole<4, 5, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa)
                           : launch_wna16_tile_whole<8, 5, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa);
             break;
-        case 6:
+        case workspace::WNA16_PAIRS_128_128:
             e = bits == 4 ? launch_wna16_tile_whole<4, 2, 2, 32>(stream, A, Wq, S, Y, M, N, K, qa)
                           : launch_wna16_tile_whole<8, 2, 2, 32>(stream, A, Wq, S, Y, M, N, K, qa);
             break;
-        case 7:
+        case workspace::WNA16_PAIRS_128_96:
             e = bits == 4 ? launch_wna16_tile_whole<4, 4, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa)
                           : launch_wna16_tile_whole<8, 4, 3, 16>(stream, A, Wq, S, Y, M, N, K, qa);
             break;

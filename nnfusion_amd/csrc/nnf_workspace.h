@@ -215,7 +215,7 @@ namespace nnf
         struct SkPlan
         {
             int tile_rows = 0; // 32, 64, 128 or 256
-            int tile_weight_rows = 256; // weight rows of a tile: 256, or 128 (narrow tiles: plain product only)
+            int tile_weight_rows = 256; // weight rows of a tile: 256, 128 (narrow tiles: plain product only) or 192 (whole tiles of 128 rows: plan_w4a16_192)
             int tiles_m = 0, tiles_n = 0;
             int supersteps = 0; // per tile: ceil(K / 256)
             long long units = 0;
@@ -1016,9 +1016,21 @@ namespace nnf
         // workgroups costs 2.5 us, the reduction pass 3 us, 0.3 a range and its sums at 2.5 TB/s; taken where the estimate is 7 % lower and
         // ws_bytes hold the sums.  Sixty products of 17 .. 2500 rows, one range -> the plan's: 21 x 512 x 16256 81 -> 16 us,
         // 249 x 256 x 15232 80 -> 20, 126 x 1472 x 11648 86 -> 25, 1707 x 896 x 15872 156 -> 82, 261 x 3840 x 8320 88 -> 53.
+        enum Wna16Tile
+        {
+            WNA16_256_256 = 0,
+            WNA16_256_128 = 1,
+            WNA16_128_128 = 2,
+            WNA16_64_64 = 3,
+            WNA16_192_128 = 4,
+            // on pairs of wavefronts: all of K in one range
+            WNA16_PAIRS_160_96 = 5,
+            WNA16_PAIRS_128_128 = 6,
+            WNA16_PAIRS_128_96 = 7,
+        };
         struct Wna16TilePlan
         {
-            int tile = 3, ranges = 1, range_k = 0;
+            int tile = WNA16_64_64, ranges = 1, range_k = 0;
             size_t bytes = 0; // of fp32 sums [ranges][M][N]
         };
         inline Wna16TilePlan plan_wna16_tile(int M, int N, int K, int num_cu, size_t ws_bytes)
@@ -1068,14 +1080,15 @@ namespace nnf
             // tile, halves of 256 x 128 and quarters of 256 x 256 tiles, pay for their sums, less and less of it with K: 73 products with
             // such a plan 1.05 on 128 x 128 tiles up to K = 7000, 1.00 up to 7500, 0.97 (0.91 - 1.09) above (898 x 4032 x 9600 105 us, 112 on them).
             double other = 0.95 * estimate(best.tile, best.ranges, best.range_k);
-            const bool same_work = K >= 7500 && best.tile <= 1 && rows[best.tile] * cols[best.tile] <= 128 * 128 * best.ranges;
+            const bool same_work = K >= 7500 && best.tile <= WNA16_256_128 && rows[best.tile] * cols[best.tile] <= 128 * 128 * best.ranges;
             if (K >= 1024)
-                for (int pair = 5; pair < 8; ++pair)
+                for (int pair = WNA16_PAIRS_160_96; pair <= WNA16_PAIRS_128_96; ++pair)
                 {
-                    if (pair == 6 && same_work)
+                    if (pair == WNA16_PAIRS_128_128 && same_work)
                         continue;
-                    const long long grid = (long long)ceil_div(M, pair == 5 ? 160 : 128) * ceil_div(N, pair == 6 ? 128 : 96);
-                    const double t = 3.7 + (pair == 5 ? 0.68 : pair == 6 ? 0.66 : 0.59) * 4 * ceil_div(K, 256);
+                    const long long grid = (long long)ceil_div(M, pair == WNA16_PAIRS_160_96 ? 160 : 128) * ceil_div(N, pair == WNA16_PAIRS_128_128 ? 128 : 96);
+                    const double step = pair == WNA16_PAIRS_160_96 ? 0.68 : pair == WNA16_PAIRS_128_128 ? 0.66 : 0.59;
+                    const double t = 3.7 + step * 4 * ceil_div(K, 256);
                     if (grid <= num_cu && t < other)
                     {
                         other = t;
@@ -1600,7 +1613,7 @@ namespace nnf
             // residual in place, which the kernel adds itself now: the scratch memory is still asked for, not written.
             bool via_scratch = false;
             SkPlan plan;              // TILE: what the caller fixed, or (own_plan) the even split, in whose scratch memory the launch fits
-            bool own_plan = false;    // TILE: the launch follows plan_w4a16_tiles (w4a16_launch_plan)
+            bool own_plan = false;    // TILE: the launch follows plan_w4a16_tiles and plan_w4a16_192 (w4a16_launch_tiles)
             size_t partial_bytes = 0; // partial sums / parked tiles / the products ahead of SiLU-gate
             size_t rms_bytes = 0;     // RMSNorm prologue: rstd, fp32 [M] (the kernels multiply the RMSNorm weight in
                                       // themselves), or for the MFMA GEMV kernel the normalised activations, fp16 [M, K]
@@ -1707,11 +1720,17 @@ namespace nnf
             return route_w4a16(M, N, K, gate, rms, in_place_residual, num_cu, path, tile_rows, k_parts, tile_cols, false);
         }
 
-        // the tiles a TILE route's launch runs: the estimates are compared once, there, and not by the size queries and checks.
-        // sync_bytes: of synchronisation words (0: none)
+        // The plan of a TILE route's launch by the estimates, which are compared once, there, and not by the size queries and checks.  Its
+        // synchronisation words are what a generated program reserves.  sync_bytes: of synchronisation words (0: none)
         inline SkPlan w4a16_launch_plan(const W4A16Route& r, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes = SIZE_MAX)
         {
             return r.own_plan ? plan_w4a16_tiles(r.plan, M, N, K, gate, rms, num_cu, sync_bytes) : r.plan;
+        }
+        // ... and the tiles it runs: that plan, or whole tiles of 128 x 192, which need no scratch memory and no words but RMSNorm's two
+        inline SkPlan w4a16_launch_tiles(const W4A16Route& r, int M, int N, int K, bool gate, bool rms, int num_cu, size_t sync_bytes)
+        {
+            const SkPlan p = w4a16_launch_plan(r, M, N, K, gate, rms, num_cu, sync_bytes);
+            return r.own_plan ? plan_w4a16_192(p, M, N, K, gate, num_cu, rms) : p;
         }
 
         inline bool w4a16_variant_fits(int M, int N, int K, int variant, int num_cu)

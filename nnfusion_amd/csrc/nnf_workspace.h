@@ -500,13 +500,13 @@ namespace nnf
         // (26 products 0.80 - 1.06 on these tiles, 0.925 in the geometric mean: 4085 x 1024 x 6656 60.6 us, 65.9 on them; with RMSNorm, whose sums
         // of squares more workgroups share, 19 products 0.95 - 2.1), and thirds of 256 x 256, eight ninths, of long K: of 293 products those of
         // up to 35 supersteps 1.11 on these tiles, from 48 on 0.98; between them 1.06 for more than 256 rows with RMSNorm or with less to
-        // compute on these tiles, else 1.02 up to 41 and 0.99 above, 0.97 with SiLU-gate or columns that are no multiple of eight.  (Up to 256 rows, one row of tiles there
-        // and two here, 0.95 from 36 on.)
-        // And so is a plan with less to compute by a seventh and more, padding included: few columns, a second tile for some of them (30827 x 128 x
-        // 2816 32.2 / 38.9 us, 7633 x 640 x 3328 39.6 / 43.2; columns that are no multiple of eight level up to a fifth).  With RMSNorm the
-        // sums of squares of so many rows make 1.4 - 2.9 x of it.
-        // 816 products of 17 .. 34000 rows that the rule without these exceptions took: 1.095 x in the geometric mean, 134 of them more than 3 %
-        // slower; 617 are still on these tiles, 1.15 x, three of them more than 3 % slower (3998 x 1024 x 12288 with RMSNorm 0.96).
+        // compute on these tiles, else 1.02 up to 41 and 0.99 above, 0.97 with SiLU-gate or columns that are no multiple of
+        // eight.  (Up to 256 rows, one row of tiles there and two here, 0.95 from 36 on.)
+        // And so is a plan with less to compute by a seventh and more, padding included, or a fifth where columns are no multiple of eight: few
+        // columns, a second tile for some of them (30827 x 128 x 2816 32.2 / 38.9 us, 7633 x 640 x 3328 39.6 / 43.2; but 6014 x 602 x 2560, 1.18
+        // times the work, 37.2 / 34.1).  With RMSNorm the sums of squares of so many rows make 1.4 - 2.9 x of it.
+        // 816 products of 17 .. 34000 rows that the rule without these exceptions took: 1.10 x in the geometric mean, 131 of them more than 3 %
+        // slower; 627 are still on these tiles, 1.15 x, three of them more than 3 % slower (3998 x 1024 x 12288 with RMSNorm 0.96).
         inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu, bool rms = true)
         {
             SkPlan p;
@@ -522,7 +522,7 @@ namespace nnf
                 (p.supersteps > 40 && 4 * tiles < 3ll * num_cu))
                 return other;
             const long long other_tiles = (long long)other.tiles_m * other.tiles_n, area = (long long)other.tile_rows * other.tile_weight_rows;
-            if (!rms && 20 * tiles * 128 * 192 > 23 * other_tiles * area)
+            if (!rms && 20 * tiles * 128 * 192 > ((N & 7) ? 25 : 23) * other_tiles * area)
                 return other;
             if (other.slots && other.tile_rows == 256 && other.grid % other_tiles == 0)
             {

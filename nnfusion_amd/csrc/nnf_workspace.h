@@ -496,17 +496,24 @@ namespace nnf
         // 64 rows, of which these tiles pad three quarters and half (16 SiLU-gate products 0.90 - 0.98: 41 x 16356 x 3328 40.8 us, 45.4 on them).
         // One round of whole 128 x 128 tiles, two thirds of the work a workgroup, is ahead as well: 37 products 0.72 - 0.93
         // (1024 x 4096 x 4096 39.1 us, 52.7 on 176 of these tiles; 148 x 16365 x 7936 with RMSNorm 78.7 / 92.5).
-        // So are equal parts of 256-row tiles with less work a workgroup: halves of 256 x 128 and quarters of 256 x 256, two thirds of it
-        // (26 products 0.80 - 1.06 on these tiles, 0.925 in the geometric mean: 4085 x 1024 x 6656 60.6 us, 65.9 on them; with RMSNorm, whose sums
-        // of squares more workgroups share, 19 products 0.95 - 2.1), and thirds of 256 x 256, eight ninths, of long K: of 293 products those of
-        // up to 35 supersteps 1.11 on these tiles, from 48 on 0.98; between them 1.06 for more than 256 rows with RMSNorm or with less to
-        // compute on these tiles, else 1.02 up to 41 and 0.99 above, 0.97 with SiLU-gate or columns that are no multiple of
-        // eight.  (Up to 256 rows, one row of tiles there and two here, 0.95 from 36 on.)
-        // And so is a plan with less to compute by a seventh and more, padding included, or a fifth where columns are no multiple of eight: few
-        // columns, a second tile for some of them (30827 x 128 x 2816 32.2 / 38.9 us, 7633 x 640 x 3328 39.6 / 43.2; but 6014 x 602 x 2560, 1.18
-        // times the work, 37.2 / 34.1).  With RMSNorm the sums of squares of so many rows make 1.4 - 2.9 x of it.
-        // 816 products of 17 .. 34000 rows that the rule without these exceptions took: 1.10 x in the geometric mean, 131 of them more than 3 %
-        // slower; 627 are still on these tiles, 1.15 x, three of them more than 3 % slower (3998 x 1024 x 12288 with RMSNorm 0.96).
+        // The rest is a matter of `work`, tiles x their size x supersteps, padding included, against the plan's.  The two rows of wavefronts of
+        // these tiles take the supersteps in turn, so an odd number of them costs one more: whole tiles, no RMSNorm, columns a multiple of eight,
+        // 1.00 x with ten supersteps, 0.97 with eleven, 1.02 with twelve, 0.99 with thirteen.  Of such products with up to 1.07 times the work
+        // 948 gain 1.046, one is more than 3 % slower; above that 196 0.973 (4965 x 1024 x 3840 43.9 us, 47.2 on these tiles; 30827 x 128 x 2816
+        // 32.2 / 38.9).  Columns that are no multiple of eight are stored an element at a time, with which fewer, larger tiles are behind: 121
+        // products with up to 1.25 times the work 1.08, none below 1.02.  With RMSNorm more workgroups share the sums of squares: 777 products
+        // 1.19, 0.98 .. 2.9.
+        // Equal parts of tiles have less work a workgroup, and lose their lead with K, as their sums cost less of it:
+        //  - halves of 256 x 128 and 128 x 256 and quarters of 256 x 256, two thirds of it, stay: 103 halves 0.95 on these tiles (4085 x 1024 x
+        //    6656 60.6 us, 65.9; 1111 x 1792 x 9472 with SiLU-gate 79.5 / 85.0), 21 quarters from 20 supersteps on 0.91, below it 16 1.13.  With
+        //    RMSNorm 77 1.33, but from 32 supersteps on and up to 4096 rows five 0.93;
+        //  - thirds of 256 x 256, eight ninths of it, up to 35 supersteps: 261 1.12, but 20 of a little more work the shorter K is 1.00; up to 47:
+        //    115 with up to 1.03 times the work 1.04, 26 others 0.97, with RMSNorm 270 1.17; above: 63 with less work 1.035, others 73 0.97,
+        //    but with RMSNorm and more than 2048 rows 1.17.  Up to 256 rows, one row of tiles there and two here, 23 1.04 up to 41 supersteps,
+        //    15 above 0.97.
+        // 3777 products of 65 .. 34000 rows that the rule without these exceptions takes: 1.10 x in the geometric mean, 283 of them more than 3 %
+        // slower; 3276 are on these tiles, 1.125 x, 13 of them more than 3 % slower (662 x 6912 x 12032 0.95), and of the 501 others ten would
+        // gain more than 6 %.
         inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu, bool rms = true)
         {
             SkPlan p;
@@ -522,13 +529,20 @@ namespace nnf
                 (p.supersteps > 40 && 4 * tiles < 3ll * num_cu))
                 return other;
             const long long other_tiles = (long long)other.tiles_m * other.tiles_n, area = (long long)other.tile_rows * other.tile_weight_rows;
-            if (!rms && 20 * tiles * 128 * 192 > ((N & 7) ? 25 : 23) * other_tiles * area)
+            const long long work = tiles * 128 * 192 * (p.supersteps + (p.supersteps & 1)), others = other_tiles * area * p.supersteps;
+            if (!rms && !other.slots && 100 * work > ((N & 7) ? 125 : 107) * others)
                 return other;
-            if (other.slots && other.tile_rows == 256 && other.grid % other_tiles == 0)
+            if (other.slots && other.grid % other_tiles == 0)
             {
                 const long long of_a_workgroup = area * other_tiles / other.grid;
-                const int from = M <= 256 ? 36 : rms || tiles * 128 * 192 < other_tiles * area ? 48 : gate || (N & 7) ? 36 : 42;
-                if (of_a_workgroup <= 128 * 128 ? !rms : (of_a_workgroup < 128 * 192 && p.supersteps >= from))
+                bool stays = false;
+                if (of_a_workgroup <= 128 * 128)
+                    stays = rms ? p.supersteps >= 32 && M <= 4096 : area < 256 * 256 || p.supersteps >= 20;
+                else if (of_a_workgroup < 128 * 192)
+                    stays = M <= 256             ? p.supersteps >= 42
+                            : p.supersteps >= 48 ? work >= others && !(rms && M > 2048)
+                                                 : !rms && 100 * work > (p.supersteps >= 36 ? 103 : 139 - p.supersteps) * others;
+                if (stays)
                     return other;
             }
             p.grid = (int)tiles;

@@ -1713,6 +1713,15 @@ int main(int argc, char** argv)
                 for (bool rms : {false, true})
                     EXPECT((ws::plan_w4a16_192(ws::plan_w4a16_tiles(s[0], s[1], s[2], false, rms, 256), s[0], s[1], s[2], false, 256, rms).tile_weight_rows == 192) == rms);
             EXPECT(ws::plan_w4a16_192(ws::plan_w4a16_tiles(27712, 192, 2560, false, false, 256), 27712, 192, 2560, false, 256, false).tile_weight_rows == 192);
+            // ... nor for more work, the supersteps counted in twos: an odd number costs the halves of K one more; parts of tiles: with K, and fewer rows
+            const auto on_192 = [](int m, int n, int k, bool gate, bool rms) {
+                return ws::plan_w4a16_192(ws::plan_w4a16_tiles(m, n, k, gate, rms, 256), m, n, k, gate, 256, rms).tile_weight_rows == 192;
+            };
+            EXPECT(!on_192(4965, 1024, 3840, false, false) && !on_192(1432, 1792, 2816, true, false) && !on_192(788, 2816, 2816, true, false));
+            EXPECT(on_192(788, 2816, 2560, true, false) && on_192(788, 2816, 3072, true, false) && on_192(788, 2816, 2816, true, true));
+            EXPECT(on_192(257, 11523, 2816, false, false) && on_192(1040, 4096, 5632, false, false) && on_192(6014, 602, 2560, false, false));
+            EXPECT(!on_192(1111, 1792, 9472, true, false) && !on_192(662, 6912, 14080, false, false) && !on_192(1962, 1024, 8960, true, true));
+            EXPECT(on_192(2200, 896, 3072, true, false) && on_192(8809, 424, 15360, false, true) && !on_192(657, 7168, 15872, false, true));
             // parked tiles of a plan, counted share by share: what the closed form of plan_sk has to say for any number of workgroups
             const auto walk_slots = [](const ws::SkPlan& p) {
                 const long long G = p.supersteps;

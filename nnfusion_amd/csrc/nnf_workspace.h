@@ -511,6 +511,8 @@ namespace nnf
         //    115 with up to 1.03 times the work 1.04, 26 others 0.97, with RMSNorm 270 1.17; above: 63 with less work 1.035, others 73 0.97,
         //    but with RMSNorm and more than 2048 rows 1.17.  Up to 256 rows, one row of tiles there and two here, 23 1.04 up to 41 supersteps,
         //    15 above 0.97.
+        // (Without synchronisation words RMSNorm's sums of squares are a pass of their own and nothing is shared: 362 products 1.08, 12 of them more
+        // than 3 % slower, 2291 x 1792 x 9728 0.88.  The tiles are the same all the same: words don't change a product's bits here.)
         // 3777 products of 65 .. 34000 rows that the rule without these exceptions takes: 1.10 x in the geometric mean, 283 of them more than 3 %
         // slower; 3276 are on these tiles, 1.125 x, 13 of them more than 3 % slower (662 x 6912 x 12032 0.95), and of the 501 others ten would
         // gain more than 6 %.

@@ -786,7 +786,7 @@ namespace nnf
         // tiles (four wavefronts), over as many ranges of K as the plan says and the workspace holds; 160 x 96, 128 x 128 or
         // 128 x 96 (four pairs of wavefronts) over all of K
         const workspace::Wna16TilePlan plan =
-            workspace::plan_wna16_tile(M, N, K, num_cu, ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 ? ws_bytes : 0);
+            workspace::plan_wna16_tile(M, N, K, num_cu, ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 ? ws_bytes : 0, bits);
         float* partial = plan.ranges > 1 ? (float*)ws : nullptr;
         hipError_t e;
         switch (plan.tile)

@@ -1052,7 +1052,7 @@ namespace nnf
             int tile = WNA16_64_64, ranges = 1, range_k = 0;
             size_t bytes = 0; // of fp32 sums [ranges][M][N]
         };
-        inline Wna16TilePlan plan_wna16_tile(int M, int N, int K, int num_cu, size_t ws_bytes)
+        inline Wna16TilePlan plan_wna16_tile(int M, int N, int K, int num_cu, size_t ws_bytes, int bits = 8)
         {
             static const int rows[] = {256, 256, 128, 64, 192}, cols[] = {256, 128, 128, 64, 128};
             static const int ranges_tried[] = {2, 3, 4, 6, 8, 12, 16, 24};
@@ -1096,10 +1096,13 @@ namespace nnf
             // a step, walked in fours, where that is 5 % below the estimate of the others.  Of 2568 products of 18 .. 4000 rows, 8 bits and
             // 4, it moves 116 (before the exception below): 1.11 x in the geometric mean (613 x 6272 x 10752 194 -> 137 us, 249 x 10368 x 4864 71 -> 56).  Two rounds and more 0.85 -
             // 1.08, K below 1024 0.87 - 0.98 with 4 bits and 1.04 with 8.  Ranges of K whose workgroups have no more work than a 128 x 128
-            // tile, halves of 256 x 128 and quarters of 256 x 256 tiles, pay for their sums, less and less of it with K: 73 products with
-            // such a plan 1.05 on 128 x 128 tiles up to K = 7000, 1.00 up to 7500, 0.97 (0.91 - 1.09) above (898 x 4032 x 9600 105 us, 112 on them).
+            // tile, halves of 256 x 128 and quarters of 256 x 256 tiles, pay for their sums, less and less of it with K: 8 bits, 216 products with
+            // such a plan 1.035 on 128 x 128 tiles up to K = 7500, above that 103 halves 0.99 and 31 quarters 0.96 (898 x 4032 x 9600 105 us, 112
+            // on them).  Not so with 4 bits, whose steps take longer on the 256-row tiles: 284 halves 1.12, 1.10 above K = 7500, 31 quarters 1.02,
+            // 0.97 from 10000 on; nor with columns that are no multiple of eight: 72 1.11.
             double other = 0.95 * estimate(best.tile, best.ranges, best.range_k);
-            const bool same_work = K >= 7500 && best.tile <= WNA16_256_128 && rows[best.tile] * cols[best.tile] <= 128 * 128 * best.ranges;
+            const bool same_work = !(N & 7) && best.tile <= WNA16_256_128 && rows[best.tile] * cols[best.tile] <= 128 * 128 * best.ranges &&
+                                   (bits == 8 ? K >= 7500 : K >= 10000 && best.tile == WNA16_256_256);
             if (K >= 1024)
                 for (int pair = WNA16_PAIRS_160_96; pair <= WNA16_PAIRS_128_96; ++pair)
                 {
@@ -1158,7 +1161,7 @@ namespace nnf
             if (gs == 0 || (bits != 4 && bits != 8) || (bits == 4 && w4a16_gemm_q_fits(M, N, K, gs)) ||
                 !wna16_on_tile_kernel(M, N, K, bits, gs, num_cu))
                 return needed;
-            return align256(plan_wna16_tile(M, N, K, num_cu, (size_t)64 << 20).bytes);
+            return align256(plan_wna16_tile(M, N, K, num_cu, (size_t)64 << 20, bits).bytes);
         }
         // ---- the fused product / MLP block for block parameters that run the nodes one after the other ----------------------
         inline size_t w4a16_gemm(int M, int N, int K, int, int num_cu = PLAN_CUS);

@@ -1526,6 +1526,19 @@ int main(int argc, char** argv)
             for (const auto& s : pairs)
                 EXPECT(ws::plan_wna16_tile(s[0], s[1], s[2], 256, (size_t)64 << 20).tile == 6);
         }
+        // ... but with 4 bits or columns that are no multiple of eight; the scratch memory asked for is that of the plan
+        {
+            const int products[][3] = {{667, 5120, 8224}, {1133, 3008, 9376}, {459, 7808, 8800}, {753, 5184, 8032}};
+            for (const auto& s : products)
+            {
+                const size_t room = (size_t)64 << 20;
+                const auto p = ws::plan_wna16_tile(s[0], s[1], s[2], 256, room, 8);
+                EXPECT(p.tile <= 1 && p.bytes > 0 && ws::plan_wna16_tile(s[0], s[1], s[2], 256, room, 4).tile == 6 &&
+                       ws::plan_wna16_tile(s[0], s[1] - 3, s[2], 256, room, 8).tile == 6 && ws::plan_wna16_tile(s[0], s[1] - 3, s[2], 256, room, 4).tile == 6);
+                EXPECT(ws::wna16_gemm_preferred(s[0], s[1], s[2], 8, 32) == ws::align256(p.bytes) && ws::wna16_gemm_preferred(s[0], s[1], s[2], 4, 32) == 0);
+            }
+            EXPECT(ws::plan_wna16_tile(492, 8128, 10784, 256, (size_t)64 << 20, 4).tile == 0);
+        }
         // W8A8 tile GEMM: whole tiles of other shapes where the estimates put them ahead (the GPU test's products), never what a caller fixed,
         // nor more scratch memory than the queries ask for
         {

@@ -1099,14 +1099,16 @@ namespace nnf
             // tile, halves of 256 x 128 and quarters of 256 x 256 tiles, pay for their sums, less and less of it with K: 8 bits, 216 products with
             // such a plan 1.035 on 128 x 128 tiles up to K = 7500, above that 103 halves 0.99 and 31 quarters 0.96 (898 x 4032 x 9600 105 us, 112
             // on them).  Not so with 4 bits, whose steps take longer on the 256-row tiles: 284 halves 1.12, 1.10 above K = 7500, 31 quarters 1.02,
-            // 0.97 from 10000 on; nor with columns that are no multiple of eight: 72 1.11.
+            // 0.97 from 10000 on; nor with columns that are no multiple of eight: 72 1.11.  (160 x 96 tiles, next in the estimate where they fit
+            // as well, are 2 - 8 % behind 128 x 128: 423 x 8128 x 9344 104 us over ranges, 114 on them.  128 x 96, three quarters of the work:
+            // 44 products of 8 bits from K = 7500 on 1.055.)
             double other = 0.95 * estimate(best.tile, best.ranges, best.range_k);
             const bool same_work = !(N & 7) && best.tile <= WNA16_256_128 && rows[best.tile] * cols[best.tile] <= 128 * 128 * best.ranges &&
                                    (bits == 8 ? K >= 7500 : K >= 10000 && best.tile == WNA16_256_256);
             if (K >= 1024)
                 for (int pair = WNA16_PAIRS_160_96; pair <= WNA16_PAIRS_128_96; ++pair)
                 {
-                    if (pair == WNA16_PAIRS_128_128 && same_work)
+                    if (pair != WNA16_PAIRS_128_96 && same_work)
                         continue;
                     const long long grid = (long long)ceil_div(M, pair == WNA16_PAIRS_160_96 ? 160 : 128) * ceil_div(N, pair == WNA16_PAIRS_128_128 ? 128 : 96);
                     const double step = pair == WNA16_PAIRS_160_96 ? 0.68 : pair == WNA16_PAIRS_128_128 ? 0.66 : 0.59;

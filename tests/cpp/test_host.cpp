@@ -1538,6 +1538,10 @@ int main(int argc, char** argv)
                 EXPECT(ws::wna16_gemm_preferred(s[0], s[1], s[2], 8, 32) == ws::align256(p.bytes) && ws::wna16_gemm_preferred(s[0], s[1], s[2], 4, 32) == 0);
             }
             EXPECT(ws::plan_wna16_tile(492, 8128, 10784, 256, (size_t)64 << 20, 4).tile == 0);
+            // (nor 160 x 96 tiles, where they fit one round too)
+            const int ranges[][3] = {{423, 8128, 9344}, {475, 8128, 9344}, {3897, 960, 8576}, {428, 8064, 8320}, {2496, 1536, 7808}};
+            for (const auto& s : ranges)
+                EXPECT(ws::plan_wna16_tile(s[0], s[1], s[2], 256, (size_t)64 << 20).tile <= 1);
         }
         // W8A8 tile GEMM: whole tiles of other shapes where the estimates put them ahead (the GPU test's products), never what a caller fixed,
         // nor more scratch memory than the queries ask for

@@ -116,10 +116,10 @@ namespace nnf
         // each would gain all of them 1.048, this gains 1.046.  (192 x 192, on
         // four wavefronts, is the fastest for three.)
         // The row of 128 x 128 is of stages of 128, one workgroup a CU; below K = 2560 the launch takes stages of 64 and two a CU, whose short
-        // loops cover for each other.  There 128 x 256 tiles are estimated ahead a little too soon: 160 products whose columns are a multiple of
-        // eight: in one round of them 0.995 at K = 512 and 640, 1.04 at 768 and 896, 1.03 - 1.12 above; in two 0.95, 0.98, 0.99 at 1024, 1.01 at
-        // 1152 and 1.07 above (2143 x 7352 x 512 20.3 / 21.7 us, 1549 x 9984 x 1152 32.0 / 30.7).  Other columns are stored an element at a
-        // time, with which fewer, larger tiles get along better: 1.11 - 1.17 at every K.
+        // loops cover for each other.  There 128 x 256 tiles are estimated ahead a little too soon: 300 products whose columns are a multiple of
+        // eight: in one round of them 0.98 at K = 512, 1.00 - 1.02 at 640, 1.05 at 768, 1.04 at 896, 1.06 - 1.11 above; in two 0.92 at 512, 0.95,
+        // 0.98, 0.97 and 0.96 at 640 .. 1024, 1.00 at 1152, 1.03 at 1280 and up to 1.06 above (2143 x 7352 x 512 19.2 / 20.6 us, 1549 x 9984 x
+        // 1152 31.3 / 31.8).  Other columns are stored an element at a time, with which fewer, larger tiles get along better: 1.11 - 1.17 at every K.
         inline int w8a8_whole_tile(int M, int N, int K, const GemmPlan& planned)
         {
             struct Cost
@@ -513,8 +513,8 @@ namespace nnf
         //    15 above 0.97.
         // (Without synchronisation words RMSNorm's sums of squares are a pass of their own and nothing is shared: 362 products 1.08, 12 of them more
         // than 3 % slower, 2291 x 1792 x 9728 0.88.  The tiles are the same all the same: words don't change a product's bits here.)
-        // 3777 products of 65 .. 34000 rows that the rule without these exceptions takes: 1.10 x in the geometric mean, 283 of them more than 3 %
-        // slower; 3276 are on these tiles, 1.125 x, 13 of them more than 3 % slower (662 x 6912 x 12032 0.95), and of the 501 others ten would
+        // 4477 products of 65 .. 34000 rows that the rule without these exceptions takes: 1.10 x in the geometric mean, 331 of them more than 3 %
+        // slower; 3886 are on these tiles, 1.12 x, 16 of them more than 3 % slower (662 x 6912 x 12032 0.95), and of the 591 others 13 would
         // gain more than 6 %.
         inline SkPlan plan_w4a16_192(const SkPlan& other, int M, int N, int K, bool gate, int num_cu, bool rms = true)
         {
